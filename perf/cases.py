@@ -1,0 +1,632 @@
+"""Steps of the served models: the work that users of this framework have it do, over the range of a server's batches.
+
+A case is ONE step of a decoder stack of four layers through ModelRunner: decode batches replay a captured graph, steps
+with prompts in them run eagerly, as the engine drives them.  Three stacks, in the two sizes of the throughput options of
+bench.py: "llama" (4-bit AWQ / GPTQ linears, grouped-query attention), "dagupel" (latent attention) and "vebusun" (three
+delta-rule layers and one with windowed and lightning attention side by side).  Fields of a case:
+
+  model, size, dtype     the stack and what it computes in (float16: llama only)
+  quant                  checkpoint format of llama's linears, groups of 128
+  block                  tokens per cache block
+  singles, context       sequences that bring one token, and the longest context among them
+  verify, draft          sequences that bring `draft` + 1 tokens (verification of drafted tokens), at the same contexts
+  prompts, prompt        sequences that bring a prompt or a part of one, and the longest part
+  cached                 tokens that the prompts' sequences have in the cache already
+  ragged                 lengths spread over [1/2, 1] of the longest instead of all alike
+
+Weights are random with the spread that keeps a residual stream level, the cache holds normal random rows.  exact() is the
+same step in double precision, written out with plain torch operations.
+"""
+import dataclasses
+import math
+
+import numpy as np
+import torch
+
+from scalellm_amd.checkpoint import Checkpoint
+from scalellm_amd.dagupel import DagupelStep
+from scalellm_amd.decode import LlamaDecodeStep, LlamaShape
+from scalellm_amd.layers import InputParameters, Portion
+from scalellm_amd.model_runner import ModelRunner, ModelRunnerOptions
+from scalellm_amd.registry import ModelLimits
+from scalellm_amd.vebusun import VebusunStep
+
+DEV = "cuda"
+LAYERS, VOCAB, HEAD, MAX_POSITIONS, GRAPH_LENGTH = 4, 32768, 128, 8192, 4096
+GROUP = 128                                           # rows per scale of the 4-bit linears
+ROT, RANK, LIMIT = 64, 512, 7.0                       # dagupel: rotated width, latent width, clamp of the GLU
+TAPS, LOW, CAP, KEEP, MULT, SCALES = 4, 128, 30.0, 16, 0.5, (0.7, 0.6)   # vebusun
+EPS = 1e-5
+# width, heads, key heads, feed-forward, window of the windowed stacks
+SIZES = {"2b": (2048, 16, 8, 8192, 4096), "8b": (4096, 32, 8, 14336, 4096)}
+YARN = {"factor": 4.0, "original": 4096, "fast": 32.0, "slow": 1.0}
+DTYPES = {"bfloat16": torch.bfloat16, "float16": torch.float16}
+
+
+def _case(name, model, size, **more):
+    case = dict(name=name, model=model, size=size, dtype="bfloat16", quant="awq" if model == "llama" else "none",
+                block=16 if model == "llama" else 64, singles=0, context=0, verify=0, draft=0, prompts=0, prompt=0, cached=0, ragged=False)
+    case.update(more)
+    return case
+
+
+def listed():
+    return [
+        # one user at a terminal
+        _case("llama 8b, 1 sequence", "llama", "8b", singles=1, context=4096),
+        # a small server with users at different places of their conversations, on a GPTQ checkpoint in float16
+        _case("llama 8b, 32 ragged", "llama", "8b", dtype="float16", quant="gptq", singles=32, context=4000, ragged=True),
+        # a full server: the batch of the default benchmark
+        _case("llama 8b, 256 sequences", "llama", "8b", singles=256, context=4096),
+        # chunked prompts, verification of four drafted tokens and plain decoding in one step
+        _case("llama 8b, mixed", "llama", "8b", singles=8, context=3000, verify=120, draft=4, prompts=8, prompt=256, cached=1024, ragged=True),
+        _case("dagupel 8b, 1 sequence", "dagupel", "8b", singles=1, context=4096),
+        _case("dagupel 2b, 32 ragged", "dagupel", "2b", singles=32, context=4001, ragged=True),
+        _case("dagupel 8b, 128 sequences", "dagupel", "8b", singles=128, context=4096),
+        # new conversations that arrive together, of no particular length
+        _case("dagupel 8b, 4 prompts", "dagupel", "8b", prompts=4, prompt=2048, ragged=True),
+        _case("vebusun 8b, 32 ragged", "vebusun", "8b", singles=32, context=4001, ragged=True),
+        _case("vebusun 2b, 128 sequences", "vebusun", "2b", singles=128, context=4096),
+        # one long document
+        _case("vebusun 2b, 1 prompt", "vebusun", "2b", prompts=1, prompt=4096),
+        # long prompts in parts beside sequences that are being answered
+        _case("vebusun 8b, mixed", "vebusun", "8b", singles=24, context=2000, prompts=8, prompt=512, cached=3072, ragged=True),
+    ]
+
+
+def draw(rng):
+    def spread(a, b):
+        return int(round(math.exp(rng.uniform(math.log(a), math.log(b)))))
+    model = rng.choice(("llama", "dagupel", "vebusun"))
+    more = {"ragged": rng.random() < 0.6}
+    if model == "llama":
+        more.update(dtype=rng.choice(("bfloat16", "float16")), quant=rng.choice(("awq", "gptq")))
+    kind = rng.choice(("decode", "decode", "decode", "prompts", "mixed"))
+    if kind != "prompts":
+        more.update(singles=spread(1, (256 if model == "llama" else 128) if kind == "decode" else 64), context=spread(128, 4096))
+    if kind != "decode":
+        n = spread(1, 8)
+        more.update(prompts=n, prompt=spread(64, min(4096, (5120 if kind == "prompts" else 2048) // n)), cached=rng.choice((0, spread(64, 3584))))
+    if kind == "mixed" and model == "llama":
+        more.update(verify=spread(1, 128), draft=rng.randint(1, 4))
+    return {k: v for k, v in _case("", model, rng.choice(("2b", "8b")), **more).items() if k != "name"}
+
+
+# ------------------------------------------------------------------------------------------------------------------------
+# what a step brings
+# ------------------------------------------------------------------------------------------------------------------------
+def _lengths(case):
+    """(new tokens, tokens in the cache after the step) of every sequence: single tokens first, prompts last."""
+    rng = np.random.default_rng(11)
+
+    def of(longest, n):
+        return [int(x) for x in rng.integers((longest + 1) // 2, longest + 1, n)] if case["ragged"] else [longest] * n
+    q = [1] * case["singles"] + [case["draft"] + 1] * case["verify"]
+    kv = [max(a, b) for a, b in zip(of(case["context"], len(q)), q)]
+    new = of(case["prompt"], case["prompts"])
+    old = of(case["cached"], case["prompts"])
+    return q + new, kv + [a + b for a, b in zip(new, old)]
+
+
+def _generator(seed, what):
+    return torch.Generator(device=DEV).manual_seed(int(seed) * 64 + what)
+
+
+def _batch(case, seed):
+    """Inputs of the step on the host: blocks of the cache in random order, block 0 unused."""
+    q, kv = _lengths(case)
+    B, rng = case["block"], np.random.default_rng([int(seed), 5])
+    count = [(k + B - 1) // B for k in kv]
+    order = (rng.permutation(sum(count)) + 1).astype(np.int32) * B
+    starts = np.concatenate([[0], np.cumsum(count)]).astype(np.int32)
+    blocks = [order[starts[i]:starts[i + 1]] for i in range(len(q))]
+    pos = [np.arange(k - n, k, dtype=np.int32) for n, k in zip(q, kv)]
+    return {"q": q, "kv": kv, "blocks": blocks, "table": order, "starts": starts, "n_blocks": sum(count) + 1, "pos": pos,
+            "tokens": [rng.integers(0, VOCAB, n).astype(np.int32) for n in q],
+            "slots": [b[p // B] + p % B for b, p in zip(blocks, pos)]}
+
+
+def _shape(case):
+    width, heads, kv_heads, ff, window = SIZES[case["size"]]
+    return width, heads, kv_heads, ff, window
+
+
+def _normal(g, *shape, std=1.0, mean=0.0, dtype=torch.bfloat16):
+    return (torch.randn(shape, device=DEV, generator=g) * std + mean).to(dtype)
+
+
+# ------------------------------------------------------------------------------------------------------------------------
+# configurations and checkpoints
+# ------------------------------------------------------------------------------------------------------------------------
+def _llama_linears(case):
+    width, heads, kv_heads, ff, _ = _shape(case)
+    return {"qkv": (width, (heads + 2 * kv_heads) * HEAD), "o": (heads * HEAD, width), "gate_up": (width, 2 * ff), "down": (ff, width)}
+
+
+def _llama_weights(case, seed):
+    """Checkpoint tensors: random nibbles and zero points, scales that give weights of spread K^-1/2."""
+    g, dtype, width = _generator(seed, 1), DTYPES[case["dtype"]], _shape(case)[0]
+
+    def bits(*shape):
+        return torch.randint(-2 ** 31, 2 ** 31, shape, device=DEV, generator=g, dtype=torch.int64).to(torch.int32)
+
+    def linear(K, N):
+        qweight = bits(K, N // 8) if case["quant"] == "awq" else bits(K // 8, N)
+        scales = (torch.rand(K // GROUP, N, device=DEV, generator=g) + 0.5) * (K ** -0.5 / 6.5)
+        return {"qweight": qweight, "qzeros": bits(K // GROUP, N // 8), "scales": scales.to(dtype)}
+    w = {"layers": [], "embed": _normal(g, VOCAB, width, dtype=dtype), "head": _normal(g, width, VOCAB, std=width ** -0.5, dtype=dtype),
+         "norm": _normal(g, width, std=0.1, mean=1.0, dtype=dtype)}
+    for _ in range(LAYERS):
+        layer = {name: linear(*kn) for name, kn in _llama_linears(case).items()}
+        layer["in_norm"], layer["post_norm"] = (_normal(g, width, std=0.1, mean=1.0, dtype=dtype) for _ in range(2))
+        w["layers"].append(layer)
+    return w
+
+
+def _dagupel_config(case):
+    width, heads, _, ff, window = _shape(case)
+    layer = {"type": "latent_attention", "mlp": {"kind": "dense", "ff": ff, "limit": LIMIT},
+             "mixer": {"heads": heads, "dim": HEAD, "rot_dim": ROT, "vdim": HEAD, "kv_rank": RANK, "mask": {"size": window},
+                       "scale": (HEAD + ROT) ** -0.5, "rot": {"base": 10000.0, "dims": ROT, "scaling": YARN}}}
+    return {"architecture": "Dagupel", "vocab": VOCAB, "width": width, "max_positions": MAX_POSITIONS, "norm": {"eps": EPS}, "logit_scale": 1.0,
+            "layers": [layer] * LAYERS}
+
+
+def _dagupel_weights(case, seed):
+    g = _generator(seed, 1)
+    width, heads, _, ff, _ = _shape(case)
+    s = width ** -0.5
+    t = {"embed": _normal(g, VOCAB, width), "pos": _normal(g, MAX_POSITIONS, width, std=0.5), "final.norm": _normal(g, width, std=0.1, mean=s)}
+    for i in range(LAYERS):
+        p = f"l{i}."
+        t.update({p + "norm1": _normal(g, width, std=0.1, mean=1.0), p + "norm2": _normal(g, width, std=0.1, mean=1.0),
+                  p + "mix.q": _normal(g, heads * (HEAD + ROT), width, std=s), p + "mix.dkv": _normal(g, RANK + ROT, width, std=s),
+                  p + "mix.dkv.norm": _normal(g, RANK, std=0.1, mean=1.0), p + "mix.uk": _normal(g, heads * HEAD, RANK, std=RANK ** -0.5),
+                  p + "mix.uv": _normal(g, heads * HEAD, RANK, std=RANK ** -0.5), p + "mix.g": _normal(g, heads, width, std=s),
+                  p + "mix.o": _normal(g, width, heads * HEAD, std=2 * (heads * HEAD) ** -0.5),
+                  p + "mlp.gate": _normal(g, ff, width, std=s), p + "mlp.up": _normal(g, ff, width, std=s),
+                  p + "mlp.down": _normal(g, width, ff, std=ff ** -0.5)})
+    return t
+
+
+def _vebusun_config(case):
+    width, heads, kv_heads, ff, window = _shape(case)
+    mlp = {"kind": "dense", "ff": ff}
+    delta = {"type": "channel_delta", "mlp": mlp, "mixer": {"heads": heads, "kv_heads": heads, "dim": HEAD, "vdim": HEAD, "conv": TAPS}}
+    both = {"type": "parallel", "mlp": mlp, "mixer": {
+        "left_scale": SCALES[0], "right_scale": SCALES[1],
+        "left": {"heads": heads, "kv_heads": kv_heads, "dim": HEAD, "vdim": HEAD, "scale": HEAD ** -0.5, "softcap": CAP,
+                 "rot": {"base": 10000.0, "dims": HEAD}, "mask": {"size": window, "keep_first": KEEP}},
+        "right": {"heads": heads, "dim": HEAD, "vdim": HEAD, "decay": [1 - 2.0 ** -(3 + 4 * h / heads) for h in range(heads)]}}}
+    return {"architecture": "Vebusun", "vocab": VOCAB, "width": width, "norm": {"eps": EPS}, "embedding": {"scale": 1.0},
+            "residual_mult": MULT, "loop": None, "layers": [both if i % 4 == 3 else delta for i in range(LAYERS)]}
+
+
+def _vebusun_weights(case, seed):
+    g = _generator(seed, 1)
+    width, H, G, ff, _ = _shape(case)
+    s, D = width ** -0.5, HEAD
+    t = {"embed": _normal(g, VOCAB, width), "head": _normal(g, VOCAB, width, std=s)}
+
+    def norm(name):
+        t[name], t[name + ".b"], t[name + ".alpha"] = _normal(g, width, std=0.1, mean=1.0), _normal(g, width, std=0.1), torch.tensor(0.5)
+    norm("final.norm")
+    for i in range(LAYERS):
+        p = f"l{i}.mix."
+        norm(f"l{i}.norm1")
+        norm(f"l{i}.norm2")
+        if i % 4 != 3:
+            for n in "qkv":
+                t[p + n], t[p + n + ".conv"] = _normal(g, H * D, width, std=2 * s), _normal(g, H * D, TAPS, std=0.5)
+            t.update({p + "b": _normal(g, H, width, std=s), p + "A_log": _normal(g, H, std=0.3), p + "dt_bias": _normal(g, H * D, std=0.5, mean=-4.0),
+                      p + "a1": _normal(g, LOW, width, std=s), p + "a2": _normal(g, H * D, LOW, std=LOW ** -0.5), p + "g1": _normal(g, LOW, width, std=s),
+                      p + "g2": _normal(g, H * D, LOW, std=LOW ** -0.5), p + "norm": _normal(g, D, std=0.1, mean=1.0),
+                      p + "o": _normal(g, width, H * D, std=2 * (H * D) ** -0.5)})
+        else:
+            t.update({p + "left.q": _normal(g, H * D, width, std=s), p + "left.k": _normal(g, G * D, width, std=s),
+                      p + "left.v": _normal(g, G * D, width, std=s), p + "left.q.norm": _normal(g, D, std=0.1, mean=1.0),
+                      p + "left.k.norm": _normal(g, D, std=0.1, mean=1.0), p + "left.sink": _normal(g, H),
+                      p + "left.o": _normal(g, width, H * D, std=2 * (H * D) ** -0.5)})
+            t.update({p + "right." + n: _normal(g, H * D, width, std=s) for n in "qkvg"})
+            t.update({p + "right.norm": _normal(g, H * D, std=0.1, mean=1.0), p + "right.o": _normal(g, width, H * D, std=2 * (H * D) ** -0.5)})
+        p = f"l{i}.mlp."
+        t.update({p + "gate": _normal(g, ff, width, std=s), p + "up": _normal(g, ff, width, std=s), p + "down": _normal(g, width, ff, std=2 * ff ** -0.5)})
+    return t
+
+
+def _history(case, seed, shapes, dtype):
+    """What the caches hold: one tensor per (what, shape, type) given, drawn one after the other."""
+    g = _generator(seed, 2)
+    for shape, std, kind in shapes:
+        t = torch.empty(shape, device=DEV, dtype=kind or dtype)
+        yield t.normal_(0.0, std, generator=g)
+
+
+def _cache_shapes(case, n_slots):
+    """(shape, spread, type) of every cache and state of the stack, layer by layer."""
+    _, H, G, _, _ = _shape(case)
+    rows = (n_slots, G, HEAD)
+    if case["model"] == "llama":
+        return [(rows, 1.0, None)] * (2 * LAYERS)
+    if case["model"] == "dagupel":
+        return [((n_slots, RANK + ROT), 1.0, None)] * LAYERS
+    n = len(_lengths(case)[0])
+    state = ((n, H, HEAD, HEAD), 0.1, torch.float32)
+    out = []
+    for i in range(LAYERS):
+        out += [state, ((n, TAPS, 3 * H * HEAD), 1.0, None)] if i % 4 != 3 else [(rows, 1.0, None), (rows, 1.0, None), state]
+    return out
+
+
+def _buffers(case, model):
+    """The model's own caches and states, in the order of _cache_shapes()."""
+    if case["model"] == "llama":
+        return [t for L in model.layers for t in L["kv"].get_kv_cache()]
+    if case["model"] == "dagupel":
+        return [c.rows for c in model.caches]
+    out = []
+    for c in model.caches:
+        out += [*c[0].get_kv_cache(), c[1].state] if isinstance(c, tuple) else [c.state, c.ring]
+    return out
+
+
+# ------------------------------------------------------------------------------------------------------------------------
+# a server, ready for the step
+# ------------------------------------------------------------------------------------------------------------------------
+def _model(case, seed, rows, n_blocks, n_states):
+    dtype = DTYPES[case["dtype"]]
+    width, heads, kv_heads, ff, _ = _shape(case)
+    if case["model"] != "llama":
+        cls, config, weights = ((DagupelStep, _dagupel_config, _dagupel_weights) if case["model"] == "dagupel" else
+                                (VebusunStep, _vebusun_config, _vebusun_weights))
+        limits = ModelLimits(n_blocks, case["block"], dtype, DEV, n_states, max_positions=MAX_POSITIONS)
+        model = cls.from_checkpoint(config(case), Checkpoint(weights(case, seed)), limits)
+        model.reserve_workspaces(rows)
+        return model
+    shape = LlamaShape(hidden=width, n_heads=heads, n_kv_heads=kv_heads, head_dim=HEAD, intermediate=ff, n_layers=LAYERS, vocab=VOCAB,
+                       max_position=MAX_POSITIONS)
+    model = LlamaDecodeStep(shape, rows, n_blocks, case["block"], quant_method=case["quant"], group_size=GROUP, dtype=dtype, device=DEV)
+    w = _llama_weights(case, seed)
+    for L, layer in zip(model.layers, w["layers"]):
+        for name in ("qkv", "o", "gate_up", "down"):
+            L[name].load_state_dict(layer[name])
+            L[name].verify_loaded_weights()
+        L["in_norm"], L["post_norm"] = layer["in_norm"], layer["post_norm"]
+    model.embed, model.lm_head, model.final_norm = w["embed"], w["head"], w["norm"]
+    model.reserve_workspaces(rows, MAX_POSITIONS)
+    return model
+
+
+def prepare(case, seed):
+    b = _batch(case, seed)
+    n, rows = len(b["q"]), sum(b["q"])
+
+    def dev(a):
+        return torch.from_numpy(np.asarray(a, dtype=np.int32)).to(DEV)
+    model = _model(case, seed, rows, b["n_blocks"], n)
+    decode = max(b["q"]) == 1
+    runner = ModelRunner(model, DEV, ModelRunnerOptions(block_size=case["block"], cuda_graph_max_seq_len=GRAPH_LENGTH,
+                                                        cuda_graph_batch_sizes=[n] if decode else []), return_logits=True)
+    states = torch.arange(n, dtype=torch.int32, device=DEV) if case["model"] == "vebusun" else None
+    if decode:
+        runner.capture_cuda_graphs(n)
+    else:   # warm up with one token: weights are laid out at first use
+        one = InputParameters(dev([0, 1]), dev([0, 1]), dev([0]), dev([0]), dev([0, 1]), 1, 1, 1, state_slots=None if states is None else states[:1])
+        runner.forward(dev([0]), dev([0]), one)
+    buffers = _buffers(case, model)
+    for have, t in zip(buffers, _history(case, seed, _cache_shapes(case, b["n_blocks"] * case["block"]), DTYPES[case["dtype"]])):
+        have.copy_(t)
+    q_cu, kv_cu = np.concatenate([[0], np.cumsum(b["q"])]), np.concatenate([[0], np.cumsum(b["kv"])])
+    portions = [Portion(int(q_cu[i]), b["q"][i], b["kv"][i], b["blocks"][i]) for i in range(n - case["prompts"], n)]
+    params = InputParameters(dev(q_cu), dev(kv_cu), dev(np.concatenate(b["slots"])), dev(b["table"]), dev(b["starts"]), max(b["q"]), max(b["kv"]),
+                             int(kv_cu[-1]), portions=() if case["model"] == "llama" else portions, state_slots=states)
+    # what a step leaves behind for the next one: recurrent states always, cached rows where a step fills them by the hundred
+    if case["prompts"]:
+        kept = [t for t, (_, _, kind) in zip(buffers, _cache_shapes(case, 1)) if t.dim() != 3 or t.size(1) != TAPS]
+    else:
+        kept = [t for t in buffers if t.dtype == torch.float32]
+    return {"runner": runner, "tokens": dev(np.concatenate(b["tokens"])), "positions": dev(np.concatenate(b["pos"])), "params": params, "kept": kept}
+
+
+def run(state):
+    # (plans of a step's prompts are made for every step anew, as every step brings other sequences)
+    params = dataclasses.replace(state["params"], plans={})
+    return {"logits": state["runner"].forward(state["tokens"], state["positions"], params), "kept": state["kept"]}
+
+
+# ------------------------------------------------------------------------------------------------------------------------
+# what a step cannot do without
+# ------------------------------------------------------------------------------------------------------------------------
+def work(case):
+    width, H, G, ff, window = _shape(case)
+    q, kv = _lengths(case)
+    rows, n, D = sum(q), len(q), HEAD
+    pairs = keys = 0   # (query, key) pairs and cached rows that are read
+    for a, k in zip(q, kv):
+        p = np.arange(k - a, k) + 1
+        seen = np.minimum(p, window) if case["model"] != "llama" else p
+        pairs += int(seen.sum())
+        keys += min(k, window + a) if case["model"] != "llama" else k
+    head = VOCAB * width
+    nbytes, flops = 2 * head + 2 * n * VOCAB + 2 * rows * width, 2 * n * head
+    if case["model"] == "llama":
+        per = sum(K * N for K, N in _llama_linears(case).values())
+        nbytes += LAYERS * (per // 2 + per // GROUP * 5 // 2 + 2 * keys * G * D * 2)
+        flops += LAYERS * (2 * rows * per + 4 * pairs * H * D)
+        return {"bytes": nbytes, "flops": flops}
+    if case["model"] == "dagupel":
+        per = width * (H * (D + ROT) + RANK + ROT + H) + 2 * H * D * RANK + H * D * width + 3 * ff * width
+        nbytes += LAYERS * (2 * per + 2 * keys * (RANK + ROT))
+        absorbed, expanded = 2 * (2 * RANK + ROT), 2 * (2 * D + ROT)   # flops of a pair and head
+        flops += LAYERS * (2 * rows * per + pairs * H * (expanded if case["prompts"] else absorbed))
+        return {"bytes": nbytes, "flops": flops}
+    state = H * D * D
+    delta = width * (4 * H * D + H + 2 * LOW) + 2 * LOW * H * D + 3 * ff * width
+    both = width * ((H + 2 * G) * D + 4 * H * D + 2 * H * D) + 3 * ff * width
+    n_delta, n_both = LAYERS - LAYERS // 4, LAYERS // 4
+    nbytes += 2 * (n_delta * delta + n_both * both) + n_both * 2 * keys * G * D * 2 + LAYERS * n * state * 8 + n_delta * n * TAPS * 3 * H * D * 2
+    flops += 2 * rows * (n_delta * delta + n_both * both) + n_both * 4 * pairs * H * D + rows * state * (6 * n_delta + 4 * n_both)
+    return {"bytes": nbytes, "flops": flops}
+
+
+def tolerance(case):
+    # Four layers of 16-bit storage: what run() gives is 0.0004 - 0.001 (float16) and 0.003 - 0.009 (bfloat16) off exact().
+    # Another order of sums moves the roundings between layers, hence differences of that size between two right answers.
+    return {"rel": 0.004, "max": 0.06} if case["dtype"] == "float16" else {"rel": 0.02, "max": 0.3}
+
+
+# ------------------------------------------------------------------------------------------------------------------------
+# the step in double precision
+# ------------------------------------------------------------------------------------------------------------------------
+def _rms(x, w):
+    return x * torch.rsqrt(x.square().mean(-1, keepdim=True) + EPS) * w.double()
+
+
+def _turn(x, pos, freq, magnitude=1.0):
+    """Pairs (i, i + half) of the last dimension turned by position * frequency; x [tokens, heads, dims]."""
+    angle = torch.as_tensor(pos, device=DEV, dtype=torch.float64)[:, None, None] * freq
+    c, s, half = angle.cos() * magnitude, angle.sin() * magnitude, x.size(-1) // 2
+    u, v = x[..., :half], x[..., half:]
+    return torch.cat([u * c - v * s, v * c + u * s], -1)
+
+
+def _frequencies(base, dims):
+    return base ** (-2.0 * torch.arange(dims // 2, device=DEV, dtype=torch.float64) / dims)
+
+
+def _yarn():
+    def turns(t):
+        return ROT * math.log(YARN["original"] / (2 * math.pi * t)) / (2 * math.log(10000.0))
+    lo, hi = max(math.floor(turns(YARN["fast"])), 0), min(math.ceil(turns(YARN["slow"])), ROT - 1)
+    ramp = ((torch.arange(ROT // 2, device=DEV, dtype=torch.float64) - lo) / max(hi - lo, 0.001)).clamp(0, 1)
+    f = _frequencies(10000.0, ROT)
+    return f / YARN["factor"] * ramp + f * (1 - ramp), 0.1 * math.log(YARN["factor"]) + 1.0
+
+
+def _attend(q, k, v, scale, window=0, keep=0, cap=0.0, sink=None):
+    """q [n, H, D] of the last n positions, k [m, G, D], v [m, G, V]: causal attention, [n, H, V]."""
+    n, H, m, G = q.size(0), q.size(1), k.size(0), k.size(1)
+    at = torch.arange(m - n, m, device=DEV)[:, None]
+    j = torch.arange(m, device=DEV)[None]
+    hidden = j > at
+    if window:
+        hidden |= (at - j >= window) & (j >= keep)
+    out = torch.empty(n, H, v.size(2), device=DEV, dtype=torch.float64)
+    r = H // G
+    step = max(1, min(G, 400_000_000 // max(1, n * m * r)))
+    for g in range(0, G, step):
+        e = min(G, g + step)
+        s = torch.matmul(q[:, g * r:e * r].reshape(n, e - g, r, -1).permute(1, 2, 0, 3), k[:, g:e].permute(1, 2, 0).unsqueeze(1).contiguous()) * scale
+        if cap:
+            s = cap * torch.tanh(s / cap)
+        s = s.masked_fill(hidden, -math.inf)
+        top = s.amax(-1, keepdim=True)
+        extra = 0.0
+        if sink is not None:
+            b = sink[g * r:e * r].double().view(e - g, r, 1, 1)
+            top = torch.maximum(top, b)
+            extra = torch.exp(b - top)
+        p = torch.exp(s - top)
+        o = torch.matmul(p, v[:, g:e].transpose(0, 1).unsqueeze(1).contiguous()) / (p.sum(-1, keepdim=True) + extra)
+        out[:, g * r:e * r] = o.permute(2, 0, 1, 3).reshape(n, (e - g) * r, -1)
+    return out
+
+
+def _sequences(case, b):
+    """(rows of the step, positions, all slots, new slots) of every sequence."""
+    at = 0
+    for i, (n, k) in enumerate(zip(b["q"], b["kv"])):
+        p = np.arange(k)
+        slots = torch.from_numpy(b["blocks"][i][p // case["block"]] + p % case["block"]).to(DEV).long()
+        yield slice(at, at + n), b["pos"][i], slots, slots[k - n:]
+        at += n
+
+
+def _dequant(case, w, K, N):
+    """[K, N] of (nibble - zero) * scale."""
+    shift = torch.arange(8, device=DEV, dtype=torch.int32) * 4
+    lane = torch.tensor([0, 4, 1, 5, 2, 6, 3, 7], device=DEV)   # place of an AWQ word's column among its nibbles
+
+    def columns(t):
+        x = (t[:, :, None] >> shift) & 15
+        return (x[:, :, lane] if case["quant"] == "awq" else x).reshape(t.size(0), -1)
+    zero = columns(w["qzeros"])
+    if case["quant"] == "awq":
+        q = columns(w["qweight"])
+    else:
+        q = ((w["qweight"][:, None, :] >> shift[:, None]) & 15).reshape(K, N)
+        zero = zero + 1
+    return ((q.view(K // GROUP, GROUP, N) - zero[:, None]).double() * w["scales"].double()[:, None]).view(K, N)
+
+
+def _exact_llama(case, seed, b, history, tokens, keep):
+    _, H, G, ff, _ = _shape(case)
+    w = _llama_weights(case, seed)
+    x = w["embed"][tokens].double()
+    freq = _frequencies(500000.0, HEAD)
+    kept = []
+    for layer in w["layers"]:
+        weight = {name: _dequant(case, layer[name], *kn) for name, kn in _llama_linears(case).items()}
+        K, V = next(history), next(history)
+        if keep:
+            K, V = K.double(), V.double()
+        qkv = (_rms(x, layer["in_norm"]) @ weight["qkv"]).view(-1, H + 2 * G, HEAD)
+        out = torch.empty(x.size(0), H * HEAD, device=DEV, dtype=torch.float64)
+        for rows, pos, slots, new in _sequences(case, b):
+            q, k = _turn(qkv[rows, :H], pos, freq), _turn(qkv[rows, H:H + G], pos, freq)
+            ks, vs = K[slots].double(), V[slots].double()
+            ks[-len(pos):], vs[-len(pos):] = k, qkv[rows, H + G:]
+            if keep:
+                K[new], V[new] = k, qkv[rows, H + G:]
+            out[rows] = _attend(q, ks, vs, HEAD ** -0.5).reshape(len(pos), -1)
+        kept += [K, V] if keep else []
+        x = x + out @ weight["o"]
+        gate_up = _rms(x, layer["post_norm"]) @ weight["gate_up"]
+        x = x + (torch.nn.functional.silu(gate_up[:, :ff]) * gate_up[:, ff:]) @ weight["down"]
+    return lambda rows: _rms(x[rows], w["norm"]) @ w["head"].double(), kept
+
+
+def _exact_dagupel(case, seed, b, history, tokens, keep):
+    _, H, _, _, window = _shape(case)
+    w = _dagupel_weights(case, seed)
+    freq, magnitude = _yarn()
+    x = w["embed"][tokens].double() + w["pos"][torch.from_numpy(np.concatenate(b["pos"])).to(DEV).long()].double()
+    kept = []
+    for i in range(LAYERS):
+        t = {k[len(f"l{i}."):]: v.double() for k, v in w.items() if k.startswith(f"l{i}.")}
+        h = _rms(x, t["norm1"])
+        q, down = (h @ t["mix.q"].t()).view(-1, H, HEAD + ROT), h @ t["mix.dkv"].t()
+        gate = torch.sigmoid(h @ t["mix.g"].t())
+        latent = _rms(down[:, :RANK], t["mix.dkv.norm"])
+        cache = next(history)
+        cache = cache.double() if keep else cache
+        out = torch.empty(x.size(0), H * HEAD, device=DEV, dtype=torch.float64)
+        uk, uv = t["mix.uk"].view(H, HEAD, RANK), t["mix.uv"].view(H, HEAD, RANK)
+        for rows, pos, slots, new in _sequences(case, b):
+            row = torch.cat([latent[rows], _turn(down[rows, None, RANK:], pos, freq, magnitude)[:, 0]], -1)
+            c = cache[slots].double()
+            c[-len(pos):] = row
+            if keep:
+                cache[new] = row
+            # queries met with the cached rows themselves: one key head of RANK + ROT, values of RANK
+            qa = torch.cat([torch.matmul(q[rows, :, :HEAD].transpose(0, 1), uk).transpose(0, 1), _turn(q[rows, :, HEAD:], pos, freq, magnitude)], -1)
+            if len(pos) > 16:   # cheaper per head for prompts
+                k = torch.cat([(c[:, :RANK] @ t["mix.uk"].t()).view(-1, H, HEAD), c[:, None, RANK:].expand(-1, H, -1)], -1)
+                qq = torch.cat([q[rows, :, :HEAD], qa[..., RANK:]], -1)
+                o = _attend(qq, k, (c[:, :RANK] @ t["mix.uv"].t()).view(-1, H, HEAD), (HEAD + ROT) ** -0.5, window)
+            else:
+                o = _attend(qa, c[:, None], c[:, None, :RANK], (HEAD + ROT) ** -0.5, window)
+                o = torch.matmul(o.transpose(0, 1), uv.transpose(1, 2)).transpose(0, 1)
+            out[rows] = (o * gate[rows, :, None]).reshape(len(pos), -1)
+        kept += [cache] if keep else []
+        x = x + out @ t["mix.o"].t()
+        h = _rms(x, t["norm2"])
+        g, u = (h @ t["mlp.gate"].t()).clamp(max=LIMIT), (h @ t["mlp.up"].t()).clamp(-LIMIT, LIMIT)
+        x = x + (g * torch.sigmoid(1.702 * g) * (u + 1.0)) @ t["mlp.down"].t()
+    return lambda rows: _rms(x[rows], w["final.norm"]) @ w["embed"].double().t(), kept
+
+
+def _delta(t, h, state, ring, b, case):
+    H, D = state.size(1), HEAD
+    raw = torch.cat([h @ t[n].t() for n in "qkv"], -1)
+    taps = torch.cat([t[n + ".conv"] for n in "qkv"])
+    beta = torch.sigmoid(h @ t["b"].t())
+    decay = torch.exp(-torch.exp(t["A_log"])[:, None] * torch.nn.functional.softplus(h @ t["a1"].t() @ t["a2"].t() + t["dt_bias"]).view(-1, H, D))
+    gate = torch.sigmoid(h @ t["g1"].t() @ t["g2"].t()).view(-1, H, D)
+    out = torch.empty(h.size(0), H, D, device=DEV, dtype=torch.float64)
+    batch = [(i, rows, pos) for i, (rows, pos, _, _) in enumerate(_sequences(case, b))]
+    mixed = torch.empty_like(raw)
+    for i, rows, pos in batch:
+        before = [ring[i, p % TAPS].double() if p >= 0 else torch.zeros_like(raw[0]) for p in range(pos[0] - TAPS + 1, pos[0])]
+        padded = torch.cat([torch.stack(before), raw[rows]])
+        mixed[rows] = torch.nn.functional.silu(sum(padded[j:j + len(pos)] * taps[:, j] for j in range(TAPS)))
+    q, k, v = (u.reshape(-1, H, D) for u in mixed.split(H * D, -1))
+    q, k = (u * torch.rsqrt(u.square().sum(-1, keepdim=True) + 1e-6) for u in (q, k))
+    q = q * D ** -0.5
+    # sequences that bring equally many tokens go side by side
+    for n in sorted({len(pos) for _, _, pos in batch}):
+        some = [(i, rows) for i, rows, pos in batch if len(pos) == n]
+        index = torch.tensor([i for i, _ in some], device=DEV)
+        first = torch.tensor([rows.start for _, rows in some], device=DEV)
+        fresh = torch.tensor([b["pos"][i][0] == 0 for i, _ in some], device=DEV)
+        S = state[index].masked_fill(fresh[:, None, None, None], 0.0)
+        for s in range(n):
+            r = first + s
+            S = S * decay[r][..., None]
+            u = beta[r][..., None] * (v[r] - (k[r][..., None] * S).sum(2))
+            S = S + k[r][..., None] * u[:, :, None]
+            out[r] = (q[r][..., None] * S).sum(2)
+        state[index] = S
+    return (_rms(out, t["norm"]) * gate).reshape(h.size(0), -1) @ t["o"].t()
+
+
+def _lightning(t, h, state, decay, b, case):
+    H, D = state.size(1), HEAD
+    q, k, v = (torch.nn.functional.silu(h @ t[n].t()).view(-1, H, D) for n in "qkv")
+    out = torch.empty(h.size(0), H, D, device=DEV, dtype=torch.float64)
+    log = torch.log(decay)[None]
+    for i, (rows, pos, _, _) in enumerate(_sequences(case, b)):
+        S = state[i] if pos[0] else torch.zeros_like(state[i])
+        for at in range(rows.start, rows.stop, 128):   # 128 tokens at a time
+            r = slice(at, min(at + 128, rows.stop))
+            n = r.stop - r.start
+            j = torch.arange(n, device=DEV, dtype=torch.float64)
+            gap = (j[:, None] - j[None])[None]
+            inner = torch.exp(torch.where(gap >= 0, gap * log[..., None].transpose(0, 1).reshape(H, 1, 1), torch.full_like(gap, -math.inf)))
+            qs, ks, vs = (u[r].transpose(0, 1) for u in (q, k, v))
+            fall = torch.exp((j + 1)[None, :, None] * log.reshape(H, 1, 1))
+            o = torch.matmul(torch.matmul(qs, ks.transpose(1, 2).contiguous()) * inner, vs) + torch.matmul(qs * fall, S)
+            out[r] = o.transpose(0, 1)
+            rest = torch.exp((n - 1 - j)[None, :, None] * log.reshape(H, 1, 1))
+            S = torch.exp(n * log).reshape(H, 1, 1) * S + torch.matmul((ks * rest).transpose(1, 2).contiguous(), vs)
+        state[i] = S
+    return (_rms(out.reshape(h.size(0), -1), t["norm"]) * torch.sigmoid(h @ t["g"].t())) @ t["o"].t()
+
+
+def _exact_vebusun(case, seed, b, history, tokens, keep):
+    _, H, G, _, window = _shape(case)
+    w = _vebusun_weights(case, seed)
+    freq = _frequencies(10000.0, HEAD)
+    decay = torch.tensor(_vebusun_config(case)["layers"][3]["mixer"]["right"]["decay"], dtype=torch.float32, device=DEV).double()
+    x = w["embed"][tokens].double()
+
+    def norm(x, name):
+        return torch.tanh(w[name + ".alpha"].item() * x) * w[name].double() + w[name + ".b"].double()
+    kept = []
+    for i in range(LAYERS):
+        t = {k[len(f"l{i}.mix."):]: v.double() for k, v in w.items() if k.startswith(f"l{i}.mix.")}
+        h = norm(x, f"l{i}.norm1")
+        if i % 4 != 3:
+            state, ring = next(history).double(), next(history)
+            x = x + MULT * _delta(t, h, state, ring, b, case)
+            kept.append(state)
+        else:
+            K, V, state = next(history), next(history), next(history).double()
+            if keep:
+                K, V = K.double(), V.double()
+            left, right = ({k[len(p):]: v for k, v in t.items() if k.startswith(p)} for p in ("left.", "right."))
+            q, k, v = (h @ left[n].t() for n in "qkv")
+            q, k, v = _rms(q.view(-1, H, HEAD), left["q.norm"]), _rms(k.view(-1, G, HEAD), left["k.norm"]), v.view(-1, G, HEAD)
+            out = torch.empty(x.size(0), H * HEAD, device=DEV, dtype=torch.float64)
+            for rows, pos, slots, new in _sequences(case, b):
+                ks, vs = K[slots].double(), V[slots].double()
+                ks[-len(pos):], vs[-len(pos):] = _turn(k[rows], pos, freq), v[rows]
+                if keep:
+                    K[new], V[new] = ks[-len(pos):], vs[-len(pos):]
+                out[rows] = _attend(_turn(q[rows], pos, freq), ks, vs, HEAD ** -0.5, window, KEEP, CAP, left["sink"]).reshape(len(pos), -1)
+            x = x + MULT * (SCALES[0] * (out @ left["o"].t()) + SCALES[1] * _lightning(right, h, state, decay, b, case))
+            kept += [K, V, state] if keep else [state]
+        h = norm(x, f"l{i}.norm2")
+        gate, up, down = (w[f"l{i}.mlp.{n}"].double() for n in ("gate", "up", "down"))
+        x = x + MULT * (torch.nn.functional.silu(h @ gate.t()) * (h @ up.t())) @ down.t()
+    return lambda rows: norm(x[rows], "final.norm") @ w["head"].double().t(), kept
+
+
+def exact(case, seed):
+    b = _batch(case, seed)
+    history = _history(case, seed, _cache_shapes(case, b["n_blocks"] * case["block"]), DTYPES[case["dtype"]])
+    tokens = torch.from_numpy(np.concatenate(b["tokens"])).to(DEV).long()
+    steps = {"llama": _exact_llama, "dagupel": _exact_dagupel, "vebusun": _exact_vebusun}
+    logits, kept = steps[case["model"]](case, seed, b, history, tokens, case["prompts"] > 0)
+    last = torch.from_numpy(np.cumsum(b["q"]) - 1).to(DEV)
+    return {"logits": logits(last), "kept": kept}
