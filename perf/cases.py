@@ -53,24 +53,24 @@ def _case(name, model, size, **more):
 def listed():
     return [
         # one user at a terminal
-        _case("llama 8b, 1 sequence", "llama", "8b", singles=1, context=4096),
+        _case("llama 8b: 1 sequence", "llama", "8b", singles=1, context=4096),
         # a small server with users at different places of their conversations, on a GPTQ checkpoint in float16
-        _case("llama 8b, 32 ragged", "llama", "8b", dtype="float16", quant="gptq", singles=32, context=4000, ragged=True),
+        _case("llama 8b: 32 ragged", "llama", "8b", dtype="float16", quant="gptq", singles=32, context=4000, ragged=True),
         # a full server: the batch of the default benchmark
-        _case("llama 8b, 256 sequences", "llama", "8b", singles=256, context=4096),
+        _case("llama 8b: 256 sequences", "llama", "8b", singles=256, context=4096),
         # chunked prompts, verification of four drafted tokens and plain decoding in one step
-        _case("llama 8b, mixed", "llama", "8b", singles=8, context=3000, verify=120, draft=4, prompts=8, prompt=256, cached=1024, ragged=True),
-        _case("dagupel 8b, 1 sequence", "dagupel", "8b", singles=1, context=4096),
-        _case("dagupel 2b, 32 ragged", "dagupel", "2b", singles=32, context=4001, ragged=True),
-        _case("dagupel 8b, 128 sequences", "dagupel", "8b", singles=128, context=4096),
+        _case("llama 8b: mixed", "llama", "8b", singles=8, context=3000, verify=120, draft=4, prompts=8, prompt=256, cached=1024, ragged=True),
+        _case("dagupel 8b: 1 sequence", "dagupel", "8b", singles=1, context=4096),
+        _case("dagupel 2b: 32 ragged", "dagupel", "2b", singles=32, context=4001, ragged=True),
+        _case("dagupel 8b: 128 sequences", "dagupel", "8b", singles=128, context=4096),
         # new conversations that arrive together, of no particular length
-        _case("dagupel 8b, 4 prompts", "dagupel", "8b", prompts=4, prompt=2048, ragged=True),
-        _case("vebusun 8b, 32 ragged", "vebusun", "8b", singles=32, context=4001, ragged=True),
-        _case("vebusun 2b, 128 sequences", "vebusun", "2b", singles=128, context=4096),
+        _case("dagupel 8b: 4 prompts", "dagupel", "8b", prompts=4, prompt=2048, ragged=True),
+        _case("vebusun 8b: 32 ragged", "vebusun", "8b", singles=32, context=4001, ragged=True),
+        _case("vebusun 2b: 128 sequences", "vebusun", "2b", singles=128, context=4096),
         # one long document
-        _case("vebusun 2b, 1 prompt", "vebusun", "2b", prompts=1, prompt=4096),
+        _case("vebusun 2b: 1 prompt", "vebusun", "2b", prompts=1, prompt=4096),
         # long prompts in parts beside sequences that are being answered
-        _case("vebusun 8b, mixed", "vebusun", "8b", singles=24, context=2000, prompts=8, prompt=512, cached=3072, ragged=True),
+        _case("vebusun 8b: mixed", "vebusun", "8b", singles=24, context=2000, prompts=8, prompt=512, cached=3072, ragged=True),
     ]
 
 
