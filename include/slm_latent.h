@@ -62,6 +62,13 @@ typedef struct slm_linear_args {
 } slm_linear_args;
 enum { SLM_LIN_STORE = 0, SLM_LIN_F32 = 1, SLM_LIN_SLABS = 2, SLM_LIN_GLU = 3, SLM_LIN_GATE = 4 };
 SLM_API int slm_linear(const slm_linear_args* a, void* stream);
+/* The same for few rows in bf16, batch 1, without GATE, from weights in the order they are read in: w =  */
+/* [ceil(N / 64)][K / 64][4][2][64 lanes][8], columns past N zero; lane l of operand h of block c in step */
+/* s of panel p holds row 64 p + 16 c + l % 16, k = 64 s + 32 h + 8 (l / 16) .. + 7.  GLU: N % 64 == 0    */
+/* and the rows are taken 16 of the gate, the same 16 of the up half, in turn.  ldw is not read.          */
+SLM_API int slm_linear_stream(const slm_linear_args* a, void* stream);
+/* lays contiguous w [N, K] bf16 out so: out holds ceil(N / 64) * 64 * K elements                         */
+SLM_API int slm_stream_layout(void* out, const void* w, int64_t N, int64_t K, int32_t glu, void* stream);
 /* y = g sigmoid(alpha g) (u + shift), g = min(gate, limit), u = clamp(up, +-limit) (limit may be        */
 /* infinite: with alpha 1 and shift 0 the plain SiLU GLU); gu = [rows, 2 * half]                         */
 SLM_API int slm_clamped_glu(void* y, const void* gu, int64_t rows, int64_t half, int64_t ld_gu, int64_t ld_y,

@@ -101,6 +101,7 @@ class DagupelStep:
         # embedding and vocabulary projection are one table: zero padded to the product's tiles
         self.table = torch.zeros(round_up(c.vocab, 16), self.k_width, dtype=dt, device=dev)
         self.table[:c.vocab, :W] = ckpt.take("embed", (c.vocab, W)).to(device=dev, dtype=dt)
+        self.l_table = lk.stream_layout(self.table)
         self.pos_table = ckpt.take("pos", (c.max_positions, W)).to(device=dev, dtype=dt).contiguous()
         norm = lambda name: ckpt.take(name, (W,)).to(device=dev, dtype=torch.float32).contiguous()  # noqa: E731
         self.final_norm = norm("final.norm")
@@ -172,7 +173,7 @@ class DagupelStep:
         if rows.numel() == 0:
             return torch.empty(0, c.vocab, dtype=torch.float32, device=self.device)
         lk.residual_norm(resid, out, self.final_norm, c.eps, row_index=rows)
-        logits = lk.linear_f32(out, self.table, c.logit_scale)[:, :c.vocab]
+        logits = lk.linear_f32(out, self.table, c.logit_scale, self.l_table)[:, :c.vocab]
         if return_logits:
             return logits
         return torch.argmax(logits, dim=-1).to(torch.int32)

@@ -14,8 +14,10 @@ from . import _lib
 from ._lib import SLM_BF16, SLM_F32, SlmError, latent_check
 from .kernels import reserve_workspace
 
-# rows up to which the weight-streaming kernel serves a bf16 product; above it the vendor GEMM does
+# rows up to which a bf16 product of row-major weights is streamed; above it the vendor GEMM does it
 STREAM_MAX_ROWS = 32
+# the same of weights in the streamed layout (stream_layout()), where the product reduces or activates in its epilogue
+STREAM_LAYOUT_MAX_ROWS = 128
 # clamped GLU: y = g * sigmoid(alpha * g) * (u + shift)
 GLU_ALPHA, GLU_SHIFT = 1.702, 1.0
 
@@ -138,12 +140,56 @@ def streams_rows(x: torch.Tensor) -> bool:
     return x.dtype == torch.float32 or x.size(0) <= STREAM_MAX_ROWS
 
 
-def linear(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """x [M, K] W[N, K]^T -> [M, N] of the same dtype."""
+def stream_layout(w: torch.Tensor, glu: bool = False) -> Optional[torch.Tensor]:
+    """W [N, K] once more in the order slm_linear_stream reads it (include/slm_latent.h), made at load: what products of
+    few rows run on.  The row-major tensor stays for products of many.  glu: W = [gate | up].  None where that kernel has
+    no form (32-bit weights, gate halves that are no multiple of 32)."""
+    N, K = w.shape
+    if w.dtype != torch.bfloat16 or K % 64 or N % 16 or (glu and N % 64):
+        return None
+    _need(w.is_cuda and w.is_contiguous(), "stream_layout: contiguous weights on the GPU")
+    out = torch.empty((N + 63) // 64, K // 64, 4, 2, 64, 8, dtype=w.dtype, device=w.device)
+    latent_check(_lib.latent_lib().slm_stream_layout(_p(out), _p(w), N, K, int(glu), _stream()), "slm_stream_layout")
+    return out
+
+
+def slab_rows(layout: Optional[torch.Tensor]) -> int:
+    """Rows up to which a product with this streamed layout (None: row-major weights only) is left as slabs."""
+    return STREAM_MAX_ROWS if layout is None else STREAM_LAYOUT_MAX_ROWS
+
+
+def _stream_args(x, w, layout, M, N, K, rows) -> "Optional[_lib.LinearArgs]":
+    """Arguments of slm_linear_stream, or None where it does not serve the call."""
+    if layout is None or M > rows or x.stride(0) % 8 or x.data_ptr() % 16:
+        return None
+    _need(layout.is_contiguous() and layout.dtype == x.dtype and layout.numel() == (N + 63) // 64 * 64 * K, "linear: streamed layout of w")
+    a = _linear_args(x, w, M, N, K)
+    a.w, a.ldx, a.ldw = _p(layout), x.stride(0), K
+    return a
+
+
+def _run_stream(a) -> None:
+    latent_check(_lib.latent_lib().slm_linear_stream(C.byref(a), _stream()), "slm_linear_stream")
+
+
+def _store_rows(N: int) -> int:
+    """Rows up to which a product that is only stored is streamed.  Without slabs its workgroups are its columns': from 33
+    rows the vendor GEMM, which splits K for itself, is level or ahead under 8192 columns (6752 x 4096, 64 rows: 19.2 us
+    against 22.6), and above 64 rows always (16896 x 4096, 128 rows: 46.6 against 47.0; 64 rows: 44.0 against 38.5)."""
+    return 64 if N >= 8192 else STREAM_MAX_ROWS
+
+
+def linear(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None, layout: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """x [M, K] W[N, K]^T -> [M, N] of the same dtype.  layout: stream_layout(w)."""
     M, N, K = _check_xw(x, w)
     if out is None:
         out = torch.empty(M, N, dtype=x.dtype, device=x.device)
     _need(out.shape == (M, N) and out.stride(1) == 1 and out.dtype == x.dtype, "linear: out [M, N]")
+    a = _stream_args(x, w, layout, M, N, K, _store_rows(N))
+    if a is not None:
+        a.ldy, a.y, a.epilogue = out.stride(0), _p(out), _lib.LIN_STORE
+        _run_stream(a)
+        return out
     if not streams_rows(x):
         return torch.mm(x, w.t(), out=out)
     a = _linear_args(x, w, M, N, K)
@@ -152,14 +198,21 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None)
     return out
 
 
-def linear_f32(x: torch.Tensor, w: torch.Tensor, alpha: float = 1.0) -> torch.Tensor:
-    """alpha * x W^T as fp32 (logits)."""
+def linear_f32(x: torch.Tensor, w: torch.Tensor, alpha: float = 1.0, layout: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """alpha * x W^T as fp32 (logits).  layout: stream_layout(w)."""
     M, N, K = _check_xw(x, w)
     out = torch.empty(M, N, dtype=torch.float32, device=x.device)
-    a = _linear_args(x, w, M, N, K)
+    s = _stream_args(x, w, layout, M, N, K, M)
+    a = s if s is not None else _linear_args(x, w, M, N, K)
     a.ldx, a.ldw, a.ldy, a.y, a.epilogue, a.alpha = x.stride(0), K, N, _p(out), _lib.LIN_F32, float(alpha)
-    _run_linear(a)
+    (_run_linear if s is None else _run_stream)(a)
     return out
+
+
+def stream_split_count(n_out: int, k: int) -> int:
+    """Slabs of a streamed product: as many as give every CU a workgroup of 64 columns, at least 8 steps of 64 each (a slab
+    is written and read: 4096 columns, 128 rows, 4 against 8 slabs 34 us against 29, and 4 us less behind it)."""
+    return max(1, min(8, 256 // ((n_out + 63) // 64), k // 512))
 
 
 def split_count(rows: int, n_out: int, k: int) -> int:
@@ -169,29 +222,31 @@ def split_count(rows: int, n_out: int, k: int) -> int:
     return max(1, min(8, 768 // max(wgs, 1), k // 1024))
 
 
-def linear_slabs(x: torch.Tensor, w: torch.Tensor) -> Slabs:
-    """x W^T left as fp32 split-K partial sums for residual_norm()."""
+def linear_slabs(x: torch.Tensor, w: torch.Tensor, layout: Optional[torch.Tensor] = None) -> Slabs:
+    """x W^T left as fp32 split-K partial sums for residual_norm().  layout: stream_layout(w)."""
     M, N, K = _check_xw(x, w)
-    n = split_count(M, N, K)
+    s = _stream_args(x, w, layout, M, N, K, STREAM_LAYOUT_MAX_ROWS)
+    n = split_count(M, N, K) if s is None else stream_split_count(N, K)
     out = torch.empty(n, M, N, dtype=torch.float32, device=x.device)
-    a = _linear_args(x, w, M, N, K)
+    a = s if s is not None else _linear_args(x, w, M, N, K)
     a.ldx, a.ldw, a.ldy, a.y, a.epilogue, a.n_splits = x.stride(0), K, N, _p(out), _lib.LIN_SLABS, n
-    _run_linear(a)
+    (_run_linear if s is None else _run_stream)(a)
     return Slabs(out)
 
 
 def linear_glu(x: torch.Tensor, w_gate_up: torch.Tensor, out: torch.Tensor, limit: float, alpha: float = GLU_ALPHA,
-               shift: float = GLU_SHIFT) -> torch.Tensor:
-    """out = clamped GLU of the two halves of x [gate | up]^T: the activation is the product's epilogue where the
-    streaming kernel runs, one more launch behind the vendor GEMM otherwise."""
+               shift: float = GLU_SHIFT, layout: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """out = clamped GLU of the two halves of x [gate | up]^T: the activation is the product's epilogue where a
+    streaming kernel runs, one more launch behind the vendor GEMM otherwise.  layout: stream_layout(w_gate_up, glu=True)."""
     M, N, K = _check_xw(x, w_gate_up)
     half = N // 2
     _need(out.shape == (M, half) and out.stride(1) == 1 and out.dtype == x.dtype, "linear_glu: out [M, N / 2]")
-    if streams_rows(x):
-        a = _linear_args(x, w_gate_up, M, N, K)
+    s = _stream_args(x, w_gate_up, layout, M, N, K, STREAM_LAYOUT_MAX_ROWS)
+    if s is not None or streams_rows(x):
+        a = s if s is not None else _linear_args(x, w_gate_up, M, N, K)
         a.ldx, a.ldw, a.ldy, a.y, a.epilogue = x.stride(0), K, out.stride(0), _p(out), _lib.LIN_GLU
         a.limit, a.glu_alpha, a.glu_shift = float(limit), float(alpha), float(shift)
-        _run_linear(a)
+        (_run_linear if s is None else _run_stream)(a)
     else:
         gu = torch.mm(x, w_gate_up.t())
         clamped_glu(gu, out, limit, alpha, shift)

@@ -3,7 +3,8 @@ windowed latent attention with an output gate, and the clamped GLU feed-forward.
 
 Weights come as plain tensors in checkpoint layout ([out, in]) and are laid out once at load: projections that read
 the same input are merged into one product, heads are padded to the kernels' tile widths with zero rows, and W_uk is
-kept in both forms a key can be met in (absorbed into the query for single tokens, expanded for prompt portions).
+kept in both forms a key can be met in (absorbed into the query for single tokens, expanded for prompt portions).  Big bf16
+weights are kept twice: by rows for the products of prompts, in the streamed layout for those of decode batches.
 """
 from __future__ import annotations
 
@@ -190,6 +191,7 @@ class LatentAttention:
         self.o_k = round_up(H * self.v_pad, 64)
         self.w_o = z(round_up(width, 16), self.o_k)
         self.w_o[:width, :H * self.v_pad].view(width, H, self.v_pad)[:, :, :a.vdim] = g["o"].view(width, H, a.vdim)
+        self.l_in, self.l_o = lk.stream_layout(self.w_in), lk.stream_layout(self.w_o)
 
     def new_cache(self, n_blocks: int, block_size: int) -> LatentKVCache:
         return LatentKVCache(n_blocks, block_size, self.c_pad, self.r_pad, self.w_in.dtype, self.w_in.device)
@@ -197,7 +199,7 @@ class LatentAttention:
     def forward(self, h: torch.Tensor, positions: torch.Tensor, cache: LatentKVCache, params: InputParameters):
         """h [rows, padded width] -> what the residual stream receives (a tensor or split-K slabs)."""
         a, T = self.args, h.size(0)
-        proj = lk.linear(h, self.w_in)
+        proj = lk.linear(h, self.w_in, layout=self.l_in)
         portions = params.portions if self.portions_ok else ()
         n_tok = portions[0].row0 if portions else T
         q_abs = proj.new_empty(n_tok, a.heads, self.c_pad + self.r_pad)
@@ -223,8 +225,8 @@ class LatentAttention:
             kv = torch.mm(ctx[:, :self.c_pad], self.w_ukv.t())
             lk.latent_prefill(proj, ctx, kv, out, plan.tiles, heads=a.heads, q_dim=self.q_dim, c_pad=self.c_pad,
                               v_pad=self.v_pad, gate_off=self.off_g, window=a.window, scale=a.scale)
-        if T <= lk.STREAM_MAX_ROWS:
-            return lk.linear_slabs(out, self.w_o)
+        if T <= lk.slab_rows(self.l_o):
+            return lk.linear_slabs(out, self.w_o, self.l_o)
         return lk.linear(out, self.w_o)
 
 
@@ -244,10 +246,11 @@ class ClampedGLU:
         self.w_gate_up[f:f + ff, :width] = w["up"].to(device=device, dtype=dtype)
         self.w_down = torch.zeros(round_up(width, 16), f, dtype=dtype, device=device)
         self.w_down[:width, :ff] = w["down"].to(device=device, dtype=dtype)
+        self.l_gate_up, self.l_down = lk.stream_layout(self.w_gate_up, glu=True), lk.stream_layout(self.w_down)
 
     def forward(self, h: torch.Tensor):
         act = h.new_empty(h.size(0), self.w_down.size(1))
-        lk.linear_glu(h, self.w_gate_up, act, self.limit, self.alpha, self.shift)
-        if h.size(0) <= lk.STREAM_MAX_ROWS:
-            return lk.linear_slabs(act, self.w_down)
+        lk.linear_glu(h, self.w_gate_up, act, self.limit, self.alpha, self.shift, self.l_gate_up)
+        if h.size(0) <= lk.slab_rows(self.l_down):
+            return lk.linear_slabs(act, self.w_down, self.l_down)
         return lk.linear(act, self.w_down)

@@ -29,9 +29,9 @@ def single_rows(params: InputParameters, rows: int) -> int:
     return rows
 
 
-def out_product(x: torch.Tensor, w: torch.Tensor):
-    """What the residual stream receives: split-K slabs for few rows, a tensor otherwise."""
-    return lk.linear_slabs(x, w) if x.size(0) <= lk.STREAM_MAX_ROWS else lk.linear(x, w)
+def out_product(x: torch.Tensor, w: torch.Tensor, layout: Optional[torch.Tensor] = None):
+    """What the residual stream receives: split-K slabs for few rows, a tensor otherwise.  layout: lk.stream_layout(w)."""
+    return lk.linear_slabs(x, w, layout) if x.size(0) <= lk.slab_rows(layout) else lk.linear(x, w)
 
 
 def _rows_of(n: int, k: int, width: int, parts, dtype, device) -> torch.Tensor:
@@ -210,17 +210,18 @@ class ParallelMixer:
         self.w_o = torch.zeros(round_up(width, 16), self.o_k, dtype=left.dtype, device=self.w_in.device)
         self.w_o[:width, :left.out_width] = left.w_o
         self.w_o[:width, left.out_width:left.out_width + right.out_width] = right.w_o
+        self.l_in, self.l_o = lk.stream_layout(self.w_in), lk.stream_layout(self.w_o)
         left.w_in = right.w_in = left.w_o = right.w_o = None   # (laid out once)
 
     def new_cache(self, limits):
         return self.left.new_cache(limits), self.right.new_state(limits)
 
     def forward(self, h: torch.Tensor, positions: torch.Tensor, cache, params: InputParameters):
-        proj = lk.linear(h, self.w_in)
+        proj = lk.linear(h, self.w_in, layout=self.l_in)
         out = proj.new_empty(h.size(0), self.o_k)
         self.left.forward(proj[:, :self.split], positions, cache[0], params, out[:, :self.left.out_width])
         self.right.forward(proj[:, self.split:], positions, cache[1], params, out[:, self.left.out_width:])
-        return out_product(out, self.w_o)
+        return out_product(out, self.w_o, self.l_o)
 
 
 # ---------------------------------------------------------------------------------------
@@ -263,6 +264,7 @@ class ChannelDelta:
         self.o_k = round_up(vo, 64)
         self.w_o = torch.zeros(round_up(width, 16), self.o_k, dtype=dtype, device=device)
         self.w_o[:width, :vo] = w["o"].to(device=device, dtype=dtype)
+        self.l_in, self.l_o = lk.stream_layout(self.w_in), lk.stream_layout(self.w_o)
         f32 = lambda t: t.to(device=device, dtype=torch.float32).contiguous()  # noqa: E731
         self.spec = mk.RecurrentSpec(
             _lib.REC_DELTA, H, G, D, V, 0, qk, 2 * qk, eps, off_b=off_b, off_gate=self.low_n, q_scale=D ** -0.5, unit_eps=self.UNIT_EPS,
@@ -276,7 +278,7 @@ class ChannelDelta:
     def forward(self, h: torch.Tensor, positions: torch.Tensor, state: RecurrentState, params: InputParameters):
         s, T = self.spec, h.size(0)
         n = single_rows(params, T)
-        proj = lk.linear(h, self.w_in)
+        proj = lk.linear(h, self.w_in, layout=self.l_in)
         low_in = proj[:, self.off_a1:]
         low = proj.new_empty(T, 2 * self.low_n)
         if lk.streams_rows(h):
@@ -290,4 +292,4 @@ class ChannelDelta:
             mk.recurrent_step(*step, out=out[:n])
         if n < T:
             mk.gated_norm(mk.recurrent_portions(*step, mk.ChunkPlan.of(params, n, proj.device)), s.vdim, low[n:, self.low_n:], s.norm_weight, out[n:], eps=self.eps, per_head=True)
-        return out_product(out, self.w_o)
+        return out_product(out, self.w_o, self.l_o)

@@ -107,6 +107,7 @@ class VebusunStep:
         self.embed = ckpt.take("embed", (c.vocab, W)).to(device=dev, dtype=dt).contiguous()
         self.head = torch.zeros(round_up(c.vocab, 16), self.k_width, dtype=dt, device=dev)
         self.head[:c.vocab, :W] = ckpt.take("head", (c.vocab, W)).to(device=dev, dtype=dt)
+        self.l_head = lk.stream_layout(self.head)
         f32 = lambda name: ckpt.take(name, (W,)).to(device=dev, dtype=torch.float32).contiguous()  # noqa: E731
 
         def norm(name):
@@ -198,5 +199,5 @@ class VebusunStep:
             return torch.empty(0, c.vocab, dtype=torch.float32, device=self.device)
         out = torch.empty(rows.numel(), self.k_width, dtype=self.dtype, device=self.device)
         lk.residual_norm(resid, out, self.final_norm, c.eps, row_index=rows)
-        logits = lk.linear_f32(out, self.head)[:, :c.vocab]
+        logits = lk.linear_f32(out, self.head, layout=self.l_head)[:, :c.vocab]
         return logits if return_logits else torch.argmax(logits, dim=-1).to(torch.int32)

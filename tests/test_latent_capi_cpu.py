@@ -57,6 +57,13 @@ def test_invalid_arguments_come_back_as_status():
         setattr(a, field, bad)
         assert L.slm_linear(C.byref(a), None) == rc, field
         setattr(a, field, keep)
+    a.ldw = 0   # (not read by the streamed form)
+    for field, bad, rc in (("K", 63, -1), ("N", 15, -1), ("ldx", 32, -1), ("ldy", 8, -1), ("dtype", _lib.SLM_F32, -2), ("ldx", 68, -5),
+                           ("n_splits", 2, -1), ("batch", 2, -1), ("epilogue", _lib.LIN_GATE, -1), ("epilogue", _lib.LIN_GLU, -1), ("w", 4098, -5)):
+        keep = getattr(a, field)
+        setattr(a, field, bad)
+        assert L.slm_linear_stream(C.byref(a), None) == rc, field
+        setattr(a, field, keep)
     b = _lib.LatentAttnArgs()
     b.rows, b.batch, b.heads, b.c_pad, b.r_pad, b.block_size, b.dtype = 3, 1, 4, 64, 32, 16, _lib.SLM_BF16
     assert L.slm_latent_attn(C.byref(b), None) == -1          # null pointers
@@ -65,6 +72,9 @@ def test_invalid_arguments_come_back_as_status():
     b.block_size, b.dtype = 16, 0
     assert L.slm_latent_attn(C.byref(b), None) == -2
     assert L.slm_latent_gather(None, None, None, 1, 64, None) == -1
+    for args in ((None, 4096, 64, 64, 0), (4096, 4096, 72, 64, 0), (4096, 4096, 64, 72, 0), (4096, 4096, 96, 64, 1)):
+        assert L.slm_stream_layout(*args, None) == -1
+    assert L.slm_stream_layout(4096, 4104, 64, 64, 0, None) == -5
     assert L.slm_clamped_glu(4096, 4096, 1, 6, 12, 8, 1.0, 1.0, 1.0, _lib.SLM_BF16, None) == -1
     p = _lib.LatentPrefillArgs()
     assert L.slm_latent_prefill(C.byref(p), None) == -1

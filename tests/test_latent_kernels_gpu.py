@@ -98,6 +98,39 @@ def test_linear_epilogues(M, N, K, dtype):
         _close(out, ref.clamped_glu(want[:, :N // 2], want[:, N // 2:], 0.6), dtype, f32=1e-5, b16=2e-2)
 
 
+# row counts at the edges of every tile, columns that fill no panel of 64 and those that decide between tile widths, step
+# counts below, at and beyond a ring and a split.  fp32 sums of exact products of bf16: 1e-5 of the largest as above.
+@pytest.mark.parametrize("M", [1, 2, 16, 17, 32, 33, 64, 65, 127, 128, 140])
+@pytest.mark.parametrize("N,K", [(16, 64), (80, 192), (64, 576), (144, 1088), (192, 2112), (2048, 2048), (7168, 320), (16384, 128),
+                                 (16896, 64)])
+def test_streamed_products(M, N, K):
+    lk = _lk()
+    x = _rnd(1, M, K + 8, dtype=torch.bfloat16)[:, :K]
+    w = _rnd(2, N, K, dtype=torch.bfloat16, std=K ** -0.5)
+    want = _f64(x) @ _f64(w).T
+    layout = lk.stream_layout(w)
+    _close(lk.linear_f32(x, w, 0.25, layout), 0.25 * want, torch.float32, f32=1e-5)
+    _close(lk.linear(x, w, layout=layout), want, torch.bfloat16)
+    s = lk.linear_slabs(x, w, layout)
+    _close(s.t.sum(0), want, torch.float32, f32=1e-5)
+    if N % 64 == 0:
+        out = torch.zeros(M, N // 2, dtype=torch.bfloat16, device=DEV)
+        lk.linear_glu(x, w, out, 0.6, layout=lk.stream_layout(w, glu=True))
+        _close(out, ref.clamped_glu(want[:, :N // 2], want[:, N // 2:], 0.6), torch.bfloat16, b16=2e-2)
+
+
+def test_streamed_weight_layout():
+    lk, N, K = _lk(), 112, 192
+    w = torch.arange(N * K, device=DEV).remainder(251).to(torch.bfloat16).view(N, K)
+    p = torch.cat([w, w.new_zeros(16, K)])
+
+    def order(t):   # panels of 64 rows, steps of 64 k, blocks of 16 rows, halves of 32 k, lanes (k / 8, row)
+        return t.reshape(-1, 4, 16, K // 64, 2, 4, 8).permute(0, 3, 1, 4, 5, 2, 6).reshape(-1, K // 64, 4, 2, 64, 8)
+    assert torch.equal(lk.stream_layout(w), order(p))
+    assert torch.equal(lk.stream_layout(p, glu=True), order(p.view(2, 4, 16, K).transpose(0, 1)))
+    assert lk.stream_layout(w, glu=True) is None and lk.stream_layout(w.float()) is None
+
+
 def test_split_k_slabs_cover_k_once():
     lk = _lk()
     x, w = _rnd(1, 4, 8192, dtype=torch.bfloat16), _rnd(2, 64, 8192, dtype=torch.bfloat16, std=0.01)
