@@ -23,6 +23,8 @@
 //  * online softmax in base 2 (common/online_softmax.cuh:39-162 semantics), fp32 accumulate,
 //    exact conditional rescale (skipped when no running max moved in the wave).
 //  * split-KV partials (m, l, O) + combine kernel (math of attn_combine_kernel.cuh:14-21).
+#include <algorithm>
+
 #include "attn_common.h"
 #include "tuning.h"
 
@@ -661,6 +663,7 @@ struct AttnPlan {
   // balanced pure-decode partition (AttnKParams::bal): partial slots per (token, head) and the
   // piece-size floor that keeps a sequence's pieces within them
   int bal, part_slots, bal_qmin;
+  int small_splits;  // KV splits of the one-wave tile class of a mixed call whose other rows have one (else n_splits)
 };
 constexpr int ATTN_BAL_ALIGN = 64;
 
@@ -677,6 +680,25 @@ static bool decode_on_tile(const slm_attn_args* a) {
   // per-tile round trip dominates (8 pairs: 22 vs 13 us; 128 pairs: 48 vs 62 us; 256: 86 vs 128 us)
   return g_min > 0 && G >= g_min && G <= 32 && a->num_splits <= 0 && attn_tile_supported(a->head_dim) &&
          tune_get(TUNE_ATTN_TILE, 1) != 0 && (int64_t)a->batch_size * a->n_kv_heads >= 64;
+}
+
+// Sequences of different q_len in one call, on the tile kernel where they have more than one row
+static bool mixed_on_tile(const slm_attn_args* a) {
+  return a->max_q_len > 1 && (int64_t)a->batch_size * a->max_q_len != (int64_t)a->n_tokens && a->num_splits <= 0 &&
+         attn_tile_supported(a->head_dim) && tune_get(TUNE_ATTN_TILE, 1) != 0;
+}
+
+// The q_len = 1 sequences of a mixed call join the one-wave tiles.  The token kernel there has a workgroup per token of the
+// call, whatever the tokens are: eight single rows of 1.5 - 3 k context beside 120 verified sequences and 8 chunks took
+// it 223 us, one workgroup each, in front of the 192 us the tiles of the verified ones take; as eight more such tiles
+// they cost nothing that shows.  32 / 8 heads, n single rows of 4 k beside one prompt of 256, token -> tile: n = 1 358 -> 91 us,
+// 8 374 -> 94, 32 387 -> 139, 64 411 -> 235, 128 486 -> 410; of 512: 80 -> 47, 86 -> 51, 90 -> 61, 90 -> 68, 113 -> 95.  At 256
+// the token kernel has a workgroup on every CU and, with fewer than 8 heads on a KV head, the better rate (783 against
+// 814; 8 heads: 951 against 780).  SLM_ATTN_TILE_DECODE = 0: never.
+static bool singles_on_tile(const slm_attn_args* a) {
+  const int G = a->n_heads / a->n_kv_heads;
+  return decode_on_tile(a) || (mixed_on_tile(a) && G <= 32 && (G >= 8 || a->batch_size < 224) &&
+                               tune_get(TUNE_ATTN_TILE_DECODE, 8) > 0);
 }
 
 static int plan_attn(const slm_attn_args* a, AttnPlan* pl) {
@@ -868,6 +890,16 @@ static int plan_attn(const slm_attn_args* a, AttnPlan* pl) {
     pl->bal_qmin = (int)(qmin > 1 ? qmin : 1);
     if (pl->n_splits >= slots) pl->n_splits = slots - 1;  // P = n_tokens * n_splits workgroups per head group
   }
+  // A mixed call whose prompts need no split: the one-wave tiles have their own count, a wave for every SIMD as above, as
+  // far as its partials (a row for every token of the call) stay under 256 MB.
+  pl->small_splits = pl->n_splits;
+  if (pl->n_splits == 1 && mixed_on_tile(a) && tune_get(TUNE_ATTN_TILE_SPLITS, 0) <= 0) {
+    int64_t want = 1024 / ((int64_t)a->batch_size * a->n_kv_heads > 0 ? (int64_t)a->batch_size * a->n_kv_heads : 1);
+    const int64_t by_len = a->max_kv_len / 512, row = (int64_t)a->n_tokens * a->n_heads * (D + 2) * 4;
+    const int64_t by_size = row > 0 ? (256ll << 20) / row : 1;
+    want = std::min(std::min(want, (int64_t)16), std::min(by_len, by_size));
+    if (want > 1) pl->small_splits = (int)want;
+  }
   pl->u = tune_get(TUNE_ATTN_U, pl->w == 2 ? 2 : 4);  // (two chunks: the same bytes in flight with half the rows)
   if (pl->u != 2 && pl->u != 4) pl->u = 4;
   pl->nt = tune_get(TUNE_ATTN_NT, a->max_q_len <= 1 ? 1 : 0) != 0;
@@ -951,14 +983,15 @@ SLM_API int32_t slm_paged_kv_varlen_mha_auto_splits(const slm_attn_args* a) {
 SLM_API int32_t slm_paged_kv_varlen_mha_decode_kernel(const slm_attn_args* a) {
   AttnPlan pl;
   if (plan_attn(a, &pl) != SLM_OK) return -1;
-  return decode_on_tile(a) ? 1 : 0;
+  return singles_on_tile(a) ? 1 : 0;
 }
 
 SLM_API size_t slm_paged_kv_varlen_mha_workspace_bytes(const slm_attn_args* a) {
   AttnPlan pl;
   if (plan_attn(a, &pl) != SLM_OK) return 0;
-  if (pl.n_splits <= 1 && !pl.bal) return 0;
-  return (size_t)a->n_tokens * a->n_heads * pl.part_slots * (a->head_dim + 2) * sizeof(float);
+  const int slots = pl.bal || pl.n_splits > 1 ? pl.part_slots : pl.small_splits;
+  if (slots <= 1) return 0;
+  return (size_t)a->n_tokens * a->n_heads * slots * (a->head_dim + 2) * sizeof(float);
 }
 
 SLM_API int slm_paged_kv_varlen_mha(const slm_attn_args* a, void* stream) {
@@ -1019,15 +1052,17 @@ SLM_API int slm_paged_kv_varlen_mha(const slm_attn_args* a, void* stream) {
   kp.rows_hi = 0x7fffffff;
   kp.bal = pl.bal; kp.part_slots = pl.part_slots; kp.bal_qmin = pl.bal_qmin; kp.bal_align = ATTN_BAL_ALIGN;
   kp.prio = tune_get(TUNE_ATTN_PRIO, 1);  // measured on the two-lane bs 256 step: 25.08 -> 24.85 ms (2 x 2 runs)
-  if (pl.n_splits > 1 || pl.bal) {
+  const bool own_small = pl.small_splits > 1 && pl.n_splits == 1 && !pl.bal;  // only the one-wave tiles are split
+  if (pl.n_splits > 1 || pl.bal || own_small) {
+    const int slots = own_small ? pl.small_splits : pl.part_slots;
     const size_t need =
-        (size_t)a->n_tokens * a->n_heads * pl.part_slots * (a->head_dim + 2) * sizeof(float);
+        (size_t)a->n_tokens * a->n_heads * slots * (a->head_dim + 2) * sizeof(float);
     if (!a->workspace || a->workspace_bytes < need) return SLM_ERR_WORKSPACE;
     kp.o_part = reinterpret_cast<float*>(a->workspace);
-    kp.ml_part = kp.o_part + (size_t)a->n_tokens * a->n_heads * pl.part_slots * a->head_dim;
+    kp.ml_part = kp.o_part + (size_t)a->n_tokens * a->n_heads * slots * a->head_dim;
   }
   bool tile_used = false;
-  const bool dec_tile = decode_on_tile(a);
+  const bool dec_tile = singles_on_tile(a);
   const int first_tile_rows = dec_tile ? kp.group : kp.group + 1;  // smallest row count on the tile kernel
   // Every sequence brings exactly max_q_len tokens (the q lengths are bounded by max_q_len -- the grid contract
   // -- and add up to batch_size * max_q_len): ONE row class is populated, the launches of the others would only
@@ -1044,8 +1079,11 @@ SLM_API int slm_paged_kv_varlen_mha(const slm_attn_args* a, void* stream) {
     if (do_stream && first_tile_rows < 33 && !(uniform_q && max_rows > 32)) {  // (group >= 32: every multi-row sequence already has > 32 rows)
       tk.rows_lo = first_tile_rows;
       tk.rows_hi = 33;
+      if (own_small) tk.n_splits = tk.part_slots = pl.small_splits;
       rc = launch_attn_tile(tk, a->dtype, max_rows < 32 ? max_rows : 32, a->max_kv_len, st);
       if (rc != SLM_OK) return rc;
+      tk.n_splits = pl.n_splits;
+      tk.part_slots = pl.part_slots;
     }
     if (do_stream && max_rows > 32) {
       // rows <= group (q_len = 1) stay with the token-major kernel also when group > 32 (MQA)
@@ -1069,13 +1107,17 @@ SLM_API int slm_paged_kv_varlen_mha(const slm_attn_args* a, void* stream) {
     rc = hip_check_launch();
     if (rc != SLM_OK) return rc;
   }
-  if (do_combine && (pl.n_splits > 1 || pl.bal)) {
+  if (do_combine && (pl.n_splits > 1 || pl.bal || own_small)) {
     const int64_t items = (int64_t)a->n_tokens * a->n_heads;
     const dim3 g((unsigned)((items + 3) / 4)), blk(256);
     int lps_shift = 3;  // lanes per split: power of two >= head_dim / 4
     while ((4 << lps_shift) < a->head_dim) ++lps_shift;
     AttnKParams ck = kp;
-    if (tile_used) {  // every kernel of the call wrote partials: combine every row
+    if (own_small) {  // the one-wave tiles wrote partials
+      ck.rows_lo = first_tile_rows;
+      ck.rows_hi = 33;
+      ck.n_splits = ck.part_slots = pl.small_splits;
+    } else if (tile_used) {  // every kernel of the call wrote partials: combine every row
       ck.rows_lo = 0;
       ck.rows_hi = 0x7fffffff;
     }
