@@ -1,8 +1,12 @@
 // window_decode.hip -- windowed grouped-query attention of single rows over the paged cache on MFMA: kept first tokens,
 // capped scores, a sink.  Bound: the HBM stream of the visible keys and values.
 //
-// Work item: one workgroup = (row, kv head, block of 16 query heads, split of the visible keys); its four waves take tiles
-// of 32 keys in turn and never meet before the end.
+// Work item: one workgroup = (row, 1 / 2 / 4 neighbouring kv heads, block of 16 query heads, split of the visible keys); its four
+// waves are shared out over the kv heads, those of one head take tiles of 32 keys in turn, and none meet before the end.
+// What a cache row holds for neighbouring heads is neighbouring memory: read by one CU at about the same time it comes as
+// 512 or 1024 bytes a row instead of 256, past the caches (read once).  16 / 8 heads of 128, 128 rows of 4096 keys:
+// 398 us with a head to a workgroup (5.4 TB/s; 256 to 1024 workgroups, with non-temporal loads or without), 355 with two, 350
+// with four (6.1 TB/s); a barrier a tile between the heads 389.
 //   S[32 keys x 16 heads]      A = key rows straight from the cache (16 bytes per lane), B = the query heads in registers
 //   O^T[v x 16 heads]          P in registers: the C-fragment key order {4 g + e, 16 + 4 g + e} is the contraction order;
 //                              V^T out of a wave-private row-major LDS tile by the transpose read
@@ -21,6 +25,7 @@ struct WindowDecodeK {
   float* o_part;    // [rows, heads, splits, v_pad]
   float* ml_part;   // [rows, heads, splits, 2]
   int n_splits, head_blocks;
+  int hw_shift;     // log2 of the kv heads of a workgroup
 };
 
 __device__ __forceinline__ float over_groups(float v, bool take_max) {
@@ -48,8 +53,9 @@ __global__ void __launch_bounds__(256) window_decode_kernel(const WindowDecodeK 
   b /= p.n_splits;
   const int hb = b % p.head_blocks;
   b /= p.head_blocks;
-  const int kvh = b % a.kv_heads;
-  const int64_t row = b / a.kv_heads;
+  const int hw = 1 << p.hw_shift, phases = 4 >> p.hw_shift, phase = wave >> p.hw_shift;
+  const int kv0 = b % (a.kv_heads >> p.hw_shift) << p.hw_shift, kvh = kv0 + (wave & (hw - 1));
+  const int64_t row = b / (a.kv_heads >> p.hw_shift);
   const int seq = seq_of_row(a.q_cu, a.batch, (int)row);
   const int32_t* table = a.block_table + a.block_cu[seq];
   const VisibleKeys vis(a.positions[row], a.window, a.keep_first);
@@ -79,12 +85,12 @@ __global__ void __launch_bounds__(256) window_decode_kernel(const WindowDecodeK 
     for (int n = 0; n < 2; ++n) {
       const bf16* k = kc + (int64_t)__shfl(slot, 16 * n + l16, 64) * k_w;
 #pragma unroll
-      for (int s = 0; s < QS; ++s) kf[n][s] = *reinterpret_cast<const bf16x8_t*>(k + 32 * s);
+      for (int s = 0; s < QS; ++s) kf[n][s] = __builtin_bit_cast(bf16x8_t, __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(k + 32 * s)));
     }
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
       const int idx = lane + 64 * i;
-      vf[i] = *reinterpret_cast<const u32x4*>(vc + (int64_t)__shfl(slot, idx / VCH, 64) * v_w + 8 * (idx % VCH));
+      vf[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(vc + (int64_t)__shfl(slot, idx / VCH, 64) * v_w + 8 * (idx % VCH)));
     }
   };
   f32x4 o[NT];
@@ -96,13 +102,13 @@ __global__ void __launch_bounds__(256) window_decode_kernel(const WindowDecodeK 
   // transpose read: key 4 g + l16 / 4, columns 4 (l16 % 4)
   const uint32_t tr_base = (uint32_t)(uintptr_t)v_lds + (uint32_t)((4 * g + (l16 >> 2)) * VLS + (l16 & 3) * 8);
 
-  int t = split * per + wave;
+  int t = split * per + phase;
   int slot = 0;
   if (t < t1) {
     load_tile(slot_of(t));
-    slot = slot_of(min(t + 4, t1 - 1));
+    slot = slot_of(min(t + phases, t1 - 1));
   }
-  for (; t < t1; t += 4) {
+  for (; t < t1; t += phases) {
     f32x4 s[2];
 #pragma unroll
     for (int n = 0; n < 2; ++n) {
@@ -115,9 +121,9 @@ __global__ void __launch_bounds__(256) window_decode_kernel(const WindowDecodeK 
       const int idx = lane + 64 * i;
       *reinterpret_cast<u32x4*>(v_lds + idx / VCH * VLS + idx % VCH * 16) = vf[i];
     }
-    if (t + 4 < t1) {
+    if (t + phases < t1) {
       load_tile(slot);
-      slot = slot_of(min(t + 8, t1 - 1));
+      slot = slot_of(min(t + 2 * phases, t1 - 1));
     }
     // lane: head l16, keys 16 n + 4 g + e
     float mx = M_INIT_F;
@@ -170,10 +176,11 @@ __global__ void __launch_bounds__(256) window_decode_kernel(const WindowDecodeK 
 #pragma unroll
   for (int i = 0; i < NT; ++i) *reinterpret_cast<f32x4*>(ot + l16 * OS + 16 * i + 4 * g) = o[i];
   __syncthreads();
-  const int n_heads = min(16, group - 16 * hb);
-  for (int i = tid; i < n_heads * (VP / 4); i += 256) {
-    const int h = i / (VP / 4), c = i % (VP / 4) * 4, head = kvh * group + 16 * hb + h;
-    float top = fmaxf(fmaxf(sm[0][h], sm[1][h]), fmaxf(sm[2][h], sm[3][h])), sink2 = 0.f;
+  const int n_heads = min(16, group - 16 * hb), quads = n_heads * (VP / 4);
+  for (int i = tid; i < quads << p.hw_shift; i += 256) {
+    const int k = i / quads, h = i % quads / (VP / 4), c = i % (VP / 4) * 4, head = (kv0 + k) * group + 16 * hb + h;
+    float top = M_INIT_F, sink2 = 0.f;
+    for (int w = k; w < 4; w += hw) top = fmaxf(top, sm[w][h]);
     const bool whole = p.n_splits == 1;
     if (whole && a.sink) {
       sink2 = a.sink[head] * LOG2E_F;
@@ -181,8 +188,7 @@ __global__ void __launch_bounds__(256) window_decode_kernel(const WindowDecodeK 
     }
     float l = whole && a.sink ? fast_exp2(sink2 - top) : 0.f;
     f32x4 v = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
+    for (int w = k; w < 4; w += hw) {
       const float f = fast_exp2(sm[w][h] - top);
       l = __builtin_fmaf(f, sl[w][h], l);
       v += *reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(lds + w * WAVE_LDS) + h * OS + c) * f;
@@ -225,13 +231,19 @@ __global__ void __launch_bounds__(256) window_combine_kernel(const WindowDecodeK
 }
 
 static int head_blocks(const slm_window_attn_args& a) { return (a.heads / a.kv_heads + 15) / 16; }
-// splits: about four workgroups per CU, at least 128 keys (a tile per wave) each
+// kv heads of a workgroup: as many as leave enough rows to go round (2 / 4 heads against one, 4096 keys: 8 rows x 8 heads 36.4
+// us / 38.5 against 36.2, 1 row 17.6 / 23 against 14.7)
+static int hw_shift(const slm_window_attn_args& a) {
+  const int64_t pairs = a.rows * a.kv_heads;
+  return a.kv_heads % 4 == 0 && pairs >= 512 ? 2 : a.kv_heads % 2 == 0 && pairs >= 64 ? 1 : 0;
+}
+// splits: about two workgroups per CU, at least 128 keys (a tile per wave) each
 static int split_count(const slm_window_attn_args& a) {
   if (a.n_splits > 0) return a.n_splits < 64 ? a.n_splits : 64;
   int64_t keys = a.max_kv_len;
   if (a.window > 0 && keys > (int64_t)a.window + (a.keep_first > 0 ? a.keep_first : 0)) keys = (int64_t)a.window + (a.keep_first > 0 ? a.keep_first : 0);
-  const int64_t wgs = a.rows * a.kv_heads * head_blocks(a);
-  const int64_t want = (1024 + wgs - 1) / wgs, most = keys / 128;
+  const int64_t wgs = a.rows * (a.kv_heads >> hw_shift(a)) * head_blocks(a);
+  const int64_t want = (512 + wgs - 1) / wgs, most = keys / 128;
   const int64_t n = want < most ? want : most;
   return (int)(n < 1 ? 1 : n > 64 ? 64 : n);
 }
@@ -247,7 +259,7 @@ size_t window_decode_workspace(const slm_window_attn_args& a) {
 
 template <int DQ, int VP>
 static void wd_launch(const WindowDecodeK& p, hipStream_t st) {
-  const int64_t grid = p.a.rows * p.a.kv_heads * p.head_blocks * p.n_splits;
+  const int64_t grid = p.a.rows * (p.a.kv_heads >> p.hw_shift) * p.head_blocks * p.n_splits;
   window_decode_kernel<DQ, VP><<<dim3((unsigned)grid), dim3(256), 0, st>>>(p);
 }
 template <int DQ>
@@ -265,6 +277,7 @@ int window_decode(const slm_window_attn_args& a, hipStream_t st) {
   p.a = a;
   p.n_splits = split_count(a);
   p.head_blocks = head_blocks(a);
+  p.hw_shift = hw_shift(a);
   p.o_part = p.ml_part = nullptr;
   if (p.n_splits > 1) {
     if (!a.workspace || a.workspace_bytes < window_decode_workspace(a)) return SLM_ERR_WORKSPACE;

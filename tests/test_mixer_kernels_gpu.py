@@ -249,3 +249,38 @@ def test_silu_glu(rows, dtype):
     h, x = _hidden(rows, W, dtype, 8)
     layer = ClampedGLU(W, ff, float("inf"), w, dtype, DEV, 1.0, 0.0)
     _close(_total(layer.forward(x))[:, :W], ref.feed_forward(h, _f64(w)), dtype, 1e-5, 3e-2)
+
+
+# rows x kv heads below 64, to 512 and beyond: 1, 2 and 4 kv heads in a workgroup, 4, 2 and 1 of its waves on each; odd counts of
+# kv heads, more than 16 query heads on one, ranges of less than a tile, of splits that get no tile, windows with kept tokens
+@pytest.mark.parametrize("rows,heads,kv_heads,dim,vdim,longest,window,keep", [
+    (3, 6, 3, 64, 128, 900, 0, 0), (40, 8, 2, 128, 128, 300, 100, 7), (130, 16, 4, 96, 64, 200, 0, 0), (9, 160, 8, 128, 128, 700, 0, 0),
+    (130, 20, 5, 64, 64, 65, 33, 40), (64, 8, 8, 128, 128, 1500, 1000, 16), (1, 8, 8, 128, 128, 4000, 0, 0)])
+def test_window_attention_of_single_rows(rows, heads, kv_heads, dim, vdim, longest, window, keep):
+    from scalellm_amd import mixer_kernels as mk
+    from scalellm_amd.decode import make_batch_inputs
+    g = torch.Generator().manual_seed(rows)
+    lens = [1, longest] + torch.randint(1, longest + 1, (rows,), generator=g).tolist()
+    lens = lens[:rows] if rows > 1 else [longest]
+    _, positions, params, n_blocks = make_batch_inputs([1] * rows, lens, 16, DEV, seed=2)
+    rnd = lambda *shape: torch.randn(*shape, generator=g).to(torch.bfloat16).to(DEV)  # noqa: E731
+    q, k, v, sink = rnd(rows, heads * dim), rnd(n_blocks * 16, kv_heads, dim), rnd(n_blocks * 16, kv_heads, vdim), rnd(heads).float()
+    out = torch.zeros(rows, heads * vdim, dtype=torch.bfloat16, device=DEV)
+    mk.window_attention(q, k, v, out, sink, positions, params.q_cu_seq_lens, params.block_tables, params.cu_block_lens, block_size=16,
+                        max_kv_len=longest, heads=heads, window=window, keep_first=keep, scale=dim ** -0.5, softcap=20.0, out_scale=0.7)
+    table, starts, group = params.block_tables.long(), params.cu_block_lens.tolist(), heads // kv_heads
+    want = torch.empty(rows, heads, vdim, dtype=torch.float64, device=DEV)
+    for r, n in enumerate(lens):
+        pos = torch.arange(n, device=DEV)
+        if window:
+            pos = pos[(n - 1 - pos < window) | (pos < keep)]
+        slots = table[starts[r] + pos // 16] + pos % 16
+        ks, vs = k[slots].double(), v[slots].double()
+        for h in range(heads):
+            s = ks[:, h // group] @ q[r, h * dim:(h + 1) * dim].double() * dim ** -0.5
+            s = 20.0 * torch.tanh(s / 20.0)
+            e = torch.exp(s)
+            want[r, h] = 0.7 * (e @ vs[:, h // group]) / (e.sum() + torch.exp(sink[h].double()))
+    got = out.view(rows, heads, vdim).double()
+    # bf16 soft-max weights and results: 2^-9 each of a value, relative to the row
+    assert ((got - want).norm(dim=-1) / want.norm(dim=-1)).max() < 1e-2
