@@ -2,7 +2,9 @@
 // per key channel, and decayed linear attention.  Everything here is fp32 besides the projections it reads.
 //
 //   step     one row per sequence: convolution, activations, unit vectors, gates, the update and (delta) the output norm
-//            in one launch.  One workgroup per (row, head); the state is read and written once.  Bound: HBM (state).
+//            in one launch.  One workgroup per (row, head); the state is read and written once, past the caches.  Bound: HBM
+//            (state).  16 heads of 128 x 128, 128 rows: 74 us with ordinary loads and stores, 60 without, and 54 with the inputs'
+//            loads side by side; lightning 55 and 48 (5.6 TB/s).
 //   prepare  portions, cut into chunks of 16 tokens, every chunk at once: inputs activated and normed, decays summed, and
 //            what a chunk's tokens do to each other solved (a 16 x 16 triangular system).  Bound: VALU, HBM.
 //   scan     portions: chunk after chunk.  The columns of S are independent, so a workgroup owns 16 of them and keeps them
@@ -37,6 +39,25 @@ __device__ __forceinline__ float conv_input(const slm_recurrent_args& a, const E
     const float x = row - j >= row0 ? to_f32(src[(row - j) * a.ld_proj]) : to_f32(ring[(int64_t)((p - j) % a.taps) * ch + c]);
     acc = __builtin_fmaf(a.conv_w[(int64_t)(a.taps - 1 - j) * ch + c], x, acc);
   }
+  return silu_f32(acc);
+}
+// the same for the one row of a step, convolutions of at most 4 taps: every load at once
+template <typename E>
+__device__ __forceinline__ float conv_step4(const slm_recurrent_args& a, const E* ring, int64_t row, int p, int c) {
+  const int64_t ch = 2 * (int64_t)a.qk_heads * a.dim + (int64_t)a.heads * a.vdim;
+  const int qk = a.qk_heads * a.dim, most = min(a.taps - 1, p);
+  const int64_t col = c < qk ? a.off_q + c : c < 2 * qk ? a.off_k + (c - qk) : a.off_v + (c - 2 * qk);
+  float w[4], x[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {   // (taps there are not, and positions before 0: the last there is, times zero)
+    const int back = min(j, most);
+    w[j] = a.conv_w[(int64_t)(a.taps - 1 - back) * ch + c];
+    x[j] = j == 0 ? to_f32(reinterpret_cast<const E*>(a.proj)[row * a.ld_proj + col]) : to_f32(ring[(int64_t)((p - back) % a.taps) * ch + c]);
+  }
+  float acc = 0.f;
+#pragma unroll
+  for (int j = 3; j >= 0; --j)
+    if (j <= most) acc = __builtin_fmaf(w[j], x[j], acc);
   return silu_f32(acc);
 }
 // (raw projection of channel c, what the ring keeps)
@@ -100,7 +121,7 @@ __global__ void __launch_bounds__(1024) recurrent_step_kernel(const slm_recurren
   f32x4 s[NR];
 #pragma unroll
   for (int r = 0; r < NR; ++r)
-    s[r] = mine && p > 0 ? *reinterpret_cast<const f32x4*>(S + (int64_t)(rg + 16 * r) * a.v_pad) : f32x4{0.f, 0.f, 0.f, 0.f};
+    s[r] = mine && p > 0 ? __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(S + (int64_t)(rg + 16 * r) * a.v_pad)) : f32x4{0.f, 0.f, 0.f, 0.f};
 
   float beta = 0.f;
   if constexpr (DELTA_MODE(MODE)) {
@@ -110,30 +131,22 @@ __global__ void __launch_bounds__(1024) recurrent_step_kernel(const slm_recurren
     E* keep = ring + (int64_t)(p % a.taps) * ch;   // (no head reads this entry: the ring holds one more than the history)
     const bool first_of_group = head % (a.heads / a.qk_heads) == 0;
     float nq = 0.f, nk = 0.f;
-    for (int i = tid; i < DK; i += nthreads) {
-      float q = 0.f, k = 0.f, g = 0.f;
-      if (i < a.dim) {
-        const int c = qh * a.dim + i;
-        q = conv_input<E>(a, ring, row, row, p, c);
-        k = conv_input<E>(a, ring, row, row, p, qk + c);
-        g = expf(decay_exponent<E>(a, row, head, i));
-        if (first_of_group) {
-          keep[c] = raw_input<E>(a, row, c);
-          keep[qk + c] = raw_input<E>(a, row, qk + c);
-        }
+    // an input each: q, k, the decay, v (one after the other their loads are this kernel's length: 8.2 us for one row of 32 heads)
+    for (int i = tid; i < 3 * DK + a.v_pad; i += nthreads) {
+      const int kind = min(i / DK, 3), at = i - kind * DK;
+      if (kind == 2) {
+        sg[at] = at < a.dim ? expf(decay_exponent<E>(a, row, head, at)) : 0.f;
+        continue;
       }
-      nq = __builtin_fmaf(q, q, nq);
-      nk = __builtin_fmaf(k, k, nk);
-      sq[i] = q, sk[i] = k, sg[i] = g;
-    }
-    for (int i = nthreads - 1 - tid; i < a.v_pad; i += nthreads) {
-      float v = 0.f;
-      if (i < a.vdim) {
-        const int c = 2 * qk + head * a.vdim + i;
-        v = conv_input<E>(a, ring, row, row, p, c);
-        keep[c] = raw_input<E>(a, row, c);
+      float x = 0.f;
+      if (at < (kind == 3 ? a.vdim : a.dim)) {
+        const int c = kind == 3 ? 2 * qk + head * a.vdim + at : kind * qk + qh * a.dim + at;
+        x = a.taps <= 4 ? conv_step4<E>(a, ring, row, p, c) : conv_input<E>(a, ring, row, row, p, c);
+        if (kind == 3 || first_of_group) keep[c] = raw_input<E>(a, row, c);
       }
-      sv[i] = v;
+      if (kind == 0) nq = __builtin_fmaf(x, x, nq);
+      if (kind == 1) nk = __builtin_fmaf(x, x, nk);
+      (kind == 0 ? sq : kind == 1 ? sk : sv)[at] = x;
     }
     nq = wave_sum(nq), nk = wave_sum(nk);
     if (lane == 0) wred[0][wave] = nq, wred[1][wave] = nk;
@@ -179,7 +192,7 @@ __global__ void __launch_bounds__(1024) recurrent_step_kernel(const slm_recurren
     }
     if (mine)
 #pragma unroll
-      for (int r = 0; r < NR; ++r) *reinterpret_cast<f32x4*>(S + (int64_t)(rg + 16 * r) * a.v_pad) = s[r];
+      for (int r = 0; r < NR; ++r) __builtin_nontemporal_store(s[r], reinterpret_cast<f32x4*>(S + (int64_t)(rg + 16 * r) * a.v_pad));
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       o[j] += __shfl_xor(o[j], 16, 64);
@@ -228,7 +241,7 @@ __global__ void __launch_bounds__(1024) recurrent_step_kernel(const slm_recurren
         s[r][j] = __builtin_fmaf(k, v[j], s[r][j] * d);
         o[j] = __builtin_fmaf(q, s[r][j], o[j]);
       }
-      if (mine) *reinterpret_cast<f32x4*>(S + (int64_t)(rg + 16 * r) * a.v_pad) = s[r];
+      if (mine) __builtin_nontemporal_store(s[r], reinterpret_cast<f32x4*>(S + (int64_t)(rg + 16 * r) * a.v_pad));
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
