@@ -34,6 +34,8 @@ struct LatentAttnK {
   float* ml_part;  // [rows][heads][n_splits][2]
   float scale2;    // scale * log2(e)
   int block_shift, block_mask;
+  int mh;          // head blocks of 16 per workgroup
+  bool stream;     // the cache is read past the caches' replacement
 };
 
 typedef short tr_v4 __attribute__((ext_vector_type(4)));
@@ -145,13 +147,23 @@ __global__ void __launch_bounds__(512) latent_attn_kernel(const LatentAttnK p) {
       const int slot = tbl[(key >> p.block_shift) - blk0];
       src[i] = cache + (int64_t)(slot + (key & p.block_mask)) * (R * 2) + 16 * c;
     }
+    if (p.stream) {
 #pragma unroll
-    for (int i = 0; i < NHI; ++i)
-      if (i < NLO || wave < NTOT % 8)
-        asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
-                     :
-                     : "v"(src[i]), "s"(dst0 + (uint32_t)(wave + 8 * i) * 1024u)
-                     : "memory", "m0");
+      for (int i = 0; i < NHI; ++i)
+        if (i < NLO || wave < NTOT % 8)
+          asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt"
+                       :
+                       : "v"(src[i]), "s"(dst0 + (uint32_t)(wave + 8 * i) * 1024u)
+                       : "memory", "m0");
+    } else {
+#pragma unroll
+      for (int i = 0; i < NHI; ++i)
+        if (i < NLO || wave < NTOT % 8)
+          asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
+                       :
+                       : "v"(src[i]), "s"(dst0 + (uint32_t)(wave + 8 * i) * 1024u)
+                       : "memory", "m0");
+    }
   };
 
   f32x4 o[MH][NT];
@@ -441,19 +453,26 @@ __global__ void __launch_bounds__(256) latent_attn_any_kernel(const LatentAttnK 
   }
 }
 
-// head blocks of 16 per workgroup (the scores of four do not fit beside the tiles of the widest latent)
-static int la_mh(int heads, int c_pad) { return heads > 32 && c_pad < 512 ? 4 : heads > 16 ? 2 : 1; }
+// Head blocks of 16 per workgroup (the scores of four do not fit beside the tiles of the widest latent).  Few rows leave fewer
+// splits, and fewer partials behind them, with a block to a workgroup: the blocks of a split share an L2 (32 heads, 4096 keys: 1 row
+// 19.2 -> 16.1 us, 8 rows 26.9 -> 24.9; 32 rows, 2000 - 4001 keys 46 -> 50).
+static int la_mh(const slm_latent_attn_args& a) {
+  if (a.rows < 24 && a.heads <= 32) return 1;
+  return a.heads > 32 && a.c_pad < 512 ? 4 : a.heads > 16 ? 2 : 1;
+}
+static int64_t la_keys(const slm_latent_attn_args& a) {
+  const int64_t len = a.max_kv_len > 0 ? a.max_kv_len : 1;
+  return a.window > 0 && a.window < len ? a.window : len;
+}
 static bool la_mfma(int c_pad, int r_pad, int dtype) {
   return dtype == SLM_BF16 && (c_pad == 64 || c_pad == 128 || c_pad == 256 || c_pad == 512) && (r_pad == 32 || r_pad == 64);
 }
 static int la_splits(const slm_latent_attn_args& a) {
   if (!la_mfma(a.c_pad, a.r_pad, a.dtype) || a.generic) return 1;
   if (a.n_splits > 0) return a.n_splits < LA_MAX_SPLITS ? a.n_splits : LA_MAX_SPLITS;
-  const int mh = la_mh(a.heads, a.c_pad);
+  const int mh = la_mh(a);
   const int64_t wgs = a.rows * ((a.heads + 16 * mh - 1) / (16 * mh));
-  int64_t len = a.max_kv_len > 0 ? a.max_kv_len : 1;
-  if (a.window > 0 && a.window < len) len = a.window;
-  const int64_t tiles = (len + LA_KT - 1) / LA_KT;
+  const int64_t tiles = (la_keys(a) + LA_KT - 1) / LA_KT;
   // one round of workgroups: a ring of a wide latent fills a CU's LDS, narrow ones sit on a CU together
   const int per_cu = a.c_pad > 64 ? 1 : 2;
   int64_t n = 256 * per_cu / (wgs > 0 ? wgs : 1);
@@ -470,11 +489,10 @@ static void la_launch(const LatentAttnK& p, hipStream_t st) {
 }
 template <int KP, int RP>
 static void la_heads(const LatentAttnK& p, hipStream_t st) {
-  const int mh = la_mh(p.a.heads, KP);
-  if (mh == 1) la_launch<KP, RP, 1>(p, st);
-  else if (mh == 2) la_launch<KP, RP, 2>(p, st);
+  if (p.mh == 1) la_launch<KP, RP, 1>(p, st);
+  else if (p.mh == 2) la_launch<KP, RP, 2>(p, st);
   if constexpr (KP < 512) {
-    if (mh == 4) la_launch<KP, RP, 4>(p, st);
+    if (p.mh == 4) la_launch<KP, RP, 4>(p, st);
   }
 }
 template <int KP>
@@ -516,6 +534,10 @@ extern "C" SLM_API int slm_latent_attn(const slm_latent_attn_args* a, void* stre
   p.scale2 = a->scale * LOG2E_F;
   p.block_shift = ilog2(a->block_size);
   p.block_mask = a->block_size - 1;
+  p.mh = la_mh(*a);
+  // a stream far beyond the caches, each row of it read by one workgroup (128 rows x 4096: 16 heads 124 -> 111 us, 32 heads 134 -> 126;
+  // 8 rows, 38 MB: 26.9 -> 30)
+  p.stream = a->heads <= 16 * p.mh && a->rows * la_keys(*a) * (a->c_pad + a->r_pad) * 2 >= (100ll << 20);
   p.o_part = p.ml_part = nullptr;
   if (p.n_splits > 1) {
     if (!a->workspace || !aligned16(a->workspace) || a->workspace_bytes < slm_latent_attn_workspace_bytes(a)) return SLM_ERR_WORKSPACE;
