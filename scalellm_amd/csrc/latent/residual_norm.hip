@@ -8,10 +8,25 @@ namespace slm {
 constexpr int RN_THREADS = 256;
 constexpr int RN_STEPS = 16;  // register-resident chunks per thread
 
-// V: elements per chunk (4 when every row start is 4-element aligned, else 1)
-template <typename E, int MODE, int V>
-__global__ void __launch_bounds__(RN_THREADS) residual_norm_kernel(const slm_residual_norm_args a) {
-  __shared__ float red[4];
+// over a workgroup of T
+template <int T>
+__device__ __forceinline__ float row_sum(float v, float* red) {
+  v = wave_sum(v);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  float s = 0.f;
+#pragma unroll
+  for (int w = 0; w < T / 64; ++w) s += red[w];
+  return s;
+}
+
+// V: elements per chunk (4 when every row start is 4-element aligned, else 1).  T: threads of a row.  A row of a batch that fills
+// the chip takes 256; few rows are as long as a thread's chunks are many, so they get 1024 (below 256 rows, from 2048 columns;
+// 4096 columns, 4 slabs: 1 row 4.5 -> 3.0 us, 128 rows 5.1 -> 3.8; 2048 columns 3.3 -> 2.5, 3.7 -> 2.9).
+template <typename E, int MODE, int V, int T>
+__global__ void __launch_bounds__(T) residual_norm_kernel(const slm_residual_norm_args a) {
+  constexpr int RN_THREADS = T, RN_STEPS = slm::RN_STEPS * slm::RN_THREADS / T;
+  __shared__ float red[T / 64];
   const int tid = threadIdx.x;
   const int64_t row = blockIdx.x;
   const int width = (int)a.width;
@@ -77,7 +92,7 @@ __global__ void __launch_bounds__(RN_THREADS) residual_norm_kernel(const slm_res
   }
   if (!a.weight) return;  // (uniform: only the sum was asked for)
   const bool rms = a.norm == SLM_NORM_RMS;
-  const float rs = rms ? 1.0f / sqrtf(block_sum256(ss, red) / (float)width + a.eps) : 0.f;
+  const float rs = rms ? 1.0f / sqrtf(row_sum<T>(ss, red) / (float)width + a.eps) : 0.f;
   E* o = reinterpret_cast<E*>(a.out) + row * a.ld_out;
 #pragma unroll
   for (int s = 0; s < RN_STEPS; ++s) {
@@ -121,8 +136,10 @@ static int rn_launch(const slm_residual_norm_args& a, hipStream_t st) {
                   aligned16(a.embed) && aligned16(a.pos_table) && aligned16(a.weight) && aligned16(a.bias) && aligned16(a.out);
   if (a.width > (v4 ? 4 : 1) * RN_THREADS * RN_STEPS) return SLM_ERR_UNSUPPORTED;
   hip_clear_error();
-  if (v4) residual_norm_kernel<E, MODE, 4><<<dim3((unsigned)a.rows), dim3(RN_THREADS), 0, st>>>(a);
-  else residual_norm_kernel<E, MODE, 1><<<dim3((unsigned)a.rows), dim3(RN_THREADS), 0, st>>>(a);
+  const dim3 grid((unsigned)a.rows);
+  if (v4 && a.rows < 256 && a.width >= 2048) residual_norm_kernel<E, MODE, 4, 1024><<<grid, dim3(1024), 0, st>>>(a);
+  else if (v4) residual_norm_kernel<E, MODE, 4, RN_THREADS><<<grid, dim3(RN_THREADS), 0, st>>>(a);
+  else residual_norm_kernel<E, MODE, 1, RN_THREADS><<<grid, dim3(RN_THREADS), 0, st>>>(a);
   return hip_check_launch();
 }
 template <typename E>

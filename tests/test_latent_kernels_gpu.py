@@ -33,7 +33,7 @@ def _close(got, want, dtype, f32=3e-6, b16=1e-2):
 
 # ---- residual stream and norm ------------------------------------------------------------------
 @pytest.mark.parametrize("dtype", DTYPES)
-@pytest.mark.parametrize("rows,width", [(1, 64), (5, 77), (3, 4096), (130, 100), (2, 7168)])
+@pytest.mark.parametrize("rows,width", [(1, 64), (5, 77), (3, 4096), (130, 100), (2, 7168), (255, 2048), (256, 2048), (2, 2044), (3, 16384)])
 def test_residual_norm_modes(rows, width, dtype):
     lk, eps = _lk(), 1e-5
     pad = (width + 63) // 64 * 64
