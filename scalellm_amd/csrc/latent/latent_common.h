@@ -36,16 +36,26 @@ __device__ __forceinline__ void load_f32<4>(const float* p, float (&o)[4]) {
   const f32x4 t = *reinterpret_cast<const f32x4*>(p);
   o[0] = t.x; o[1] = t.y; o[2] = t.z; o[3] = t.w;
 }
+template <>
+__device__ __forceinline__ void load_f32<8>(const float* p, float (&o)[8]) {
+  const f32x4 t = *reinterpret_cast<const f32x4*>(p), u = *reinterpret_cast<const f32x4*>(p + 4);
+  o[0] = t.x; o[1] = t.y; o[2] = t.z; o[3] = t.w;
+  o[4] = u.x; o[5] = u.y; o[6] = u.z; o[7] = u.w;
+}
 template <int N>
 __device__ __forceinline__ void store_f32(float* p, const float (&o)[N]) {
-  if constexpr (N == 4) *reinterpret_cast<f32x4*>(p) = f32x4{o[0], o[1], o[2], o[3]};
-  else
+  if constexpr (N % 4 == 0) {
+#pragma unroll
+    for (int i = 0; i < N; i += 4) *reinterpret_cast<f32x4*>(p + i) = f32x4{o[i], o[i + 1], o[i + 2], o[i + 3]};
+  } else
 #pragma unroll
     for (int i = 0; i < N; ++i) p[i] = o[i];
 }
 template <int N>
 __device__ __forceinline__ void store_f32(bf16* p, const float (&o)[N]) {
   if constexpr (N == 4) *reinterpret_cast<u32x2*>(p) = u32x2{pack2<bf16_tag>(o[0], o[1]), pack2<bf16_tag>(o[2], o[3])};
+  else if constexpr (N == 8)
+    *reinterpret_cast<u32x4*>(p) = u32x4{pack2<bf16_tag>(o[0], o[1]), pack2<bf16_tag>(o[2], o[3]), pack2<bf16_tag>(o[4], o[5]), pack2<bf16_tag>(o[6], o[7])};
   else
 #pragma unroll
     for (int i = 0; i < N; ++i) p[i] = (bf16)o[i];

@@ -21,8 +21,9 @@ __device__ __forceinline__ float row_sum(float v, float* red) {
 }
 
 // V: elements per chunk (4 when every row start is 4-element aligned, else 1).  T: threads of a row.  A row of a batch that fills
-// the chip takes 256; few rows are as long as a thread's chunks are many, so they get 1024 (below 256 rows, from 2048 columns;
-// 4096 columns, 4 slabs: 1 row 4.5 -> 3.0 us, 128 rows 5.1 -> 3.8; 2048 columns 3.3 -> 2.5, 3.7 -> 2.9).
+// the chip hides its own latency; few rows are as long as a thread's chunks are many, so they get 1024 threads (below 256 rows, from
+// 2048 columns; 256 -> 1024 at 4096 columns, 4 slabs: 1 row 4.5 -> 3.0 us, 128 rows 5.1 -> 3.8; 2048 columns 3.3 -> 2.5, 3.7 -> 2.9)
+// and more rows 512 (256 / 512 / 1024: 300 x 4096 5.5 / 5.0 / 5.0, 4096 x 2048 18.5 / 17.3 / 19.3, 5692 x 4096 42.4 / 41.4 / 41.5).
 template <typename E, int MODE, int V, int T>
 __global__ void __launch_bounds__(T) residual_norm_kernel(const slm_residual_norm_args a) {
   constexpr int RN_THREADS = T, RN_STEPS = slm::RN_STEPS * slm::RN_THREADS / T;
@@ -114,19 +115,32 @@ __global__ void __launch_bounds__(T) residual_norm_kernel(const slm_residual_nor
   for (int i = width + tid; i < (int)a.ld_out; i += RN_THREADS) o[i] = (E)0.f;
 }
 
-template <typename E>
-__global__ void __launch_bounds__(256) clamped_glu_kernel(E* __restrict__ y, const E* __restrict__ gu, int64_t half4,
-                                                          int64_t n4, int64_t ld_gu, int64_t ld_y, float limit, float alpha,
-                                                          float shift) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= n4) return;
-  const int64_t row = i / half4, c = (i % half4) * 4;
-  float g[4], u[4], o[4];
-  load_f32<4>(gu + row * ld_gu + c, g);
-  load_f32<4>(gu + row * ld_gu + half4 * 4 + c, u);
+// V columns a thread: 8 where every row lies on 16 bytes, else 4.  5692 rows of 14336: 107 us -> 97 (490 MB; a 64-bit division a thread before).
+template <typename E, int V>
+__global__ void __launch_bounds__(256) clamped_glu_kernel(E* __restrict__ y, const E* __restrict__ gu, uint32_t steps, uint32_t n,
+                                                          int64_t ld_gu, int64_t ld_y, float limit, float alpha, float shift) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  const uint32_t row = i / steps, c = (i - row * steps) * V;
+  const E* src = gu + row * ld_gu + c;
+  float g[V], u[V], o[V];
+  load_f32<V>(src, g);
+  load_f32<V>(src + (int64_t)steps * V, u);
 #pragma unroll
-  for (int j = 0; j < 4; ++j) o[j] = clamped_glu_f32(g[j], u[j], limit, alpha, shift);
-  store_f32<4>(y + row * ld_y + c, o);
+  for (int j = 0; j < V; ++j) o[j] = clamped_glu_f32(g[j], u[j], limit, alpha, shift);
+  store_f32<V>(y + row * ld_y + c, o);
+}
+template <typename E>
+static int glu_launch(void* y, const void* gu, int64_t rows, int64_t half, int64_t ld_gu, int64_t ld_y, float limit, float alpha, float shift,
+                      hipStream_t st) {
+  const bool v8 = half % 8 == 0 && ld_gu % 8 == 0 && ld_y % 8 == 0;
+  const int64_t steps = half / (v8 ? 8 : 4), n = rows * steps;
+  if (n > 0xffffff00ll) return SLM_ERR_UNSUPPORTED;   // a launch has fewer than 2^32 threads
+  const dim3 grid((unsigned)((n + 255) / 256));
+  hip_clear_error();
+  if (v8) clamped_glu_kernel<E, 8><<<grid, dim3(256), 0, st>>>((E*)y, (const E*)gu, (uint32_t)steps, (uint32_t)n, ld_gu, ld_y, limit, alpha, shift);
+  else clamped_glu_kernel<E, 4><<<grid, dim3(256), 0, st>>>((E*)y, (const E*)gu, (uint32_t)steps, (uint32_t)n, ld_gu, ld_y, limit, alpha, shift);
+  return hip_check_launch();
 }
 
 template <typename E, int MODE>
@@ -138,6 +152,7 @@ static int rn_launch(const slm_residual_norm_args& a, hipStream_t st) {
   hip_clear_error();
   const dim3 grid((unsigned)a.rows);
   if (v4 && a.rows < 256 && a.width >= 2048) residual_norm_kernel<E, MODE, 4, 1024><<<grid, dim3(1024), 0, st>>>(a);
+  else if (v4 && a.width >= 2048) residual_norm_kernel<E, MODE, 4, 512><<<grid, dim3(512), 0, st>>>(a);
   else if (v4) residual_norm_kernel<E, MODE, 4, RN_THREADS><<<grid, dim3(RN_THREADS), 0, st>>>(a);
   else residual_norm_kernel<E, MODE, 1, RN_THREADS><<<grid, dim3(RN_THREADS), 0, st>>>(a);
   return hip_check_launch();
@@ -192,13 +207,7 @@ extern "C" SLM_API int slm_clamped_glu(void* y, const void* gu, int64_t rows, in
     return SLM_ERR_INVALID_ARG;
   if (!aligned16(y) || !aligned16(gu)) return SLM_ERR_ALIGNMENT;
   if (rows == 0) return SLM_OK;
-  const int64_t half4 = half / 4, n4 = rows * half4;
-  const dim3 grid((unsigned)((n4 + 255) / 256));
-  hip_clear_error();
-  if (dtype == SLM_BF16)
-    clamped_glu_kernel<bf16><<<grid, dim3(256), 0, (hipStream_t)stream>>>((bf16*)y, (const bf16*)gu, half4, n4, ld_gu, ld_y, limit, glu_alpha, glu_shift);
-  else if (dtype == SLM_F32)
-    clamped_glu_kernel<float><<<grid, dim3(256), 0, (hipStream_t)stream>>>((float*)y, (const float*)gu, half4, n4, ld_gu, ld_y, limit, glu_alpha, glu_shift);
-  else return SLM_ERR_UNSUPPORTED;
-  return hip_check_launch();
+  if (dtype == SLM_BF16) return glu_launch<bf16>(y, gu, rows, half, ld_gu, ld_y, limit, glu_alpha, glu_shift, (hipStream_t)stream);
+  if (dtype == SLM_F32) return glu_launch<float>(y, gu, rows, half, ld_gu, ld_y, limit, glu_alpha, glu_shift, (hipStream_t)stream);
+  return SLM_ERR_UNSUPPORTED;
 }

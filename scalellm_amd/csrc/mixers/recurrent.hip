@@ -666,6 +666,89 @@ __global__ void __launch_bounds__(256) gated_norm_kernel(const slm_gated_norm_ar
   }
 }
 
+// The same where values come in eights and lie on 16 bytes: 16-byte accesses, all loads before the sum.  PER_HEAD: VD / 8
+// lanes a head; else 256 threads a row of up to 8192.  4096 rows of 16 heads of 128:
+// per head 22.0 us -> 12.9, per row 19.9 -> 14; 32 rows of 32 heads 3.6 -> 3.2, 7.5 -> 4.0.
+template <typename E, int VD>
+__global__ void __launch_bounds__(256) gated_norm_heads_kernel(const slm_gated_norm_args a) {
+  constexpr int L = VD / 8;
+  const int tid = threadIdx.x, l = tid % L;
+  const int64_t item = (int64_t)blockIdx.x * (256 / L) + tid / L;
+  if (item >= a.rows * a.heads) return;
+  const int64_t row = item / a.heads;
+  const int h = (int)(item - row * a.heads);
+  float x[8], gl[8], w[8], ss = 0.f;
+  load_f32<8>(a.o + item * VD + 8 * l, x);
+  load_f32<8>(reinterpret_cast<const E*>(a.gate) + row * a.ld_gate + (int64_t)h * VD + 8 * l, gl);
+  load_f32<8>(a.weight + 8 * l, w);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) ss = __builtin_fmaf(x[j], x[j], ss);
+#pragma unroll
+  for (int d = 1; d < L; d <<= 1) ss += __shfl_xor(ss, d, 64);
+  const float rs = 1.0f / sqrtf(ss / (float)VD + a.eps);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) x[j] = a.scale * x[j] * rs * w[j] * sigmoid_f32(gl[j]);
+  E* out = reinterpret_cast<E*>(a.out) + row * a.ld_out;
+  store_f32<8>(out + h * VD + 8 * l, x);
+  if (h == a.heads - 1)
+    for (int64_t c = (int64_t)a.heads * VD + l; c < a.out_width; c += L) out[c] = (E)0.f;
+}
+template <typename E>
+__global__ void __launch_bounds__(256) gated_norm_row_kernel(const slm_gated_norm_args a) {
+  constexpr int NV = 4;
+  __shared__ float red[4];
+  const int tid = threadIdx.x;
+  const int64_t row = blockIdx.x;
+  const int n = a.heads * a.vdim;
+  const float* o = a.o + row * n;
+  const E* gate = reinterpret_cast<const E*>(a.gate) + row * a.ld_gate;
+  E* out = reinterpret_cast<E*>(a.out) + row * a.ld_out;
+  float x[NV][8], gl[NV][8], w[NV][8], ss = 0.f;
+#pragma unroll
+  for (int v = 0; v < NV; ++v) {
+    const int i = (tid + 256 * v) * 8;
+    if (i < n) {
+      load_f32<8>(o + i, x[v]);
+      load_f32<8>(gate + i, gl[v]);
+      load_f32<8>(a.weight + i, w[v]);
+    }
+  }
+#pragma unroll
+  for (int v = 0; v < NV; ++v)
+    if ((tid + 256 * v) * 8 < n)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) ss = __builtin_fmaf(x[v][j], x[v][j], ss);
+  const float rs = 1.0f / sqrtf(block_sum256(ss, red) / (float)n + a.eps);
+#pragma unroll
+  for (int v = 0; v < NV; ++v) {
+    const int i = (tid + 256 * v) * 8;
+    if (i < n) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) x[v][j] = a.scale * x[v][j] * rs * w[v][j] * sigmoid_f32(gl[v][j]);
+      store_f32<8>(out + i, x[v]);
+    }
+  }
+  for (int64_t i = n + tid; i < a.out_width; i += 256) out[i] = (E)0.f;
+}
+template <typename E>
+static bool gated_norm_eights(const slm_gated_norm_args& a, hipStream_t st) {
+  if (a.vdim != a.v_pad || a.vdim % 8 || a.ld_gate % 8 || a.ld_out % 8 || !aligned16(a.o) || !aligned16(a.gate) || !aligned16(a.weight) ||
+      !aligned16(a.out))
+    return false;
+  if (!a.per_head) {
+    if ((int64_t)a.heads * a.vdim > 8192) return false;
+    gated_norm_row_kernel<E><<<dim3((unsigned)a.rows), dim3(256), 0, st>>>(a);
+    return true;
+  }
+  const int64_t items = a.rows * a.heads;
+  auto grid = [&](int per) { return dim3((unsigned)((items + per - 1) / per)); };
+  if (a.vdim == 64) gated_norm_heads_kernel<E, 64><<<grid(32), dim3(256), 0, st>>>(a);
+  else if (a.vdim == 128) gated_norm_heads_kernel<E, 128><<<grid(16), dim3(256), 0, st>>>(a);
+  else if (a.vdim == 256) gated_norm_heads_kernel<E, 256><<<grid(8), dim3(256), 0, st>>>(a);
+  else return false;
+  return true;
+}
+
 constexpr int64_t NCT2_MIN = 512;   // column tiles from which a workgroup takes two
 static bool rec_sizes_ok(const slm_recurrent_args& a) {
   return a.heads > 0 && a.qk_heads > 0 && a.heads % a.qk_heads == 0 && a.dim > 0 && a.vdim > 0 && a.vdim <= a.v_pad &&
@@ -775,6 +858,7 @@ extern "C" SLM_API int slm_gated_norm(const slm_gated_norm_args* a, void* stream
   hipStream_t st = (hipStream_t)stream;
   const dim3 grid((unsigned)(a->per_head ? (a->rows * a->heads + 3) / 4 : a->rows)), block(256);
   hip_clear_error();
+  if (a->dtype == SLM_BF16 ? gated_norm_eights<bf16>(*a, st) : gated_norm_eights<float>(*a, st)) return hip_check_launch();
   if (a->dtype == SLM_BF16) {
     if (a->per_head) gated_norm_kernel<bf16, true><<<grid, block, 0, st>>>(*a);
     else gated_norm_kernel<bf16, false><<<grid, block, 0, st>>>(*a);

@@ -33,7 +33,7 @@ def _close(got, want, dtype, f32=3e-6, b16=1e-2):
 
 # ---- residual stream and norm ------------------------------------------------------------------
 @pytest.mark.parametrize("dtype", DTYPES)
-@pytest.mark.parametrize("rows,width", [(1, 64), (5, 77), (3, 4096), (130, 100), (2, 7168), (255, 2048), (256, 2048), (2, 2044), (3, 16384)])
+@pytest.mark.parametrize("rows,width", [(1, 64), (5, 77), (3, 4096), (130, 100), (2, 7168), (255, 2048), (256, 2048), (2, 2044), (3, 16384), (257, 2500)])
 def test_residual_norm_modes(rows, width, dtype):
     lk, eps = _lk(), 1e-5
     pad = (width + 63) // 64 * 64
@@ -166,6 +166,17 @@ def test_clamped_glu_bends_where_it_should(dtype):
     out = torch.empty(4, 28, dtype=dtype, device=DEV)
     lk.clamped_glu(gu, out, limit)
     _close(out, ref.clamped_glu(g.double().numpy(), u.double().numpy(), limit), dtype)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("rows,half,pad", [(1, 8, 0), (3, 4, 0), (7, 1000, 8), (5, 1004, 0), (3, 2056, 4), (300, 264, 16)])
+def test_clamped_glu_of_eights_and_fours(rows, half, pad, dtype):
+    lk = _lk()
+    gu = _rnd(11, rows, 2 * half + pad, dtype=dtype)
+    out = torch.full((rows, half + pad), 7.0, dtype=dtype, device=DEV)
+    lk.clamped_glu(gu[:, :2 * half], out[:, :half], 1.25)
+    _close(out[:, :half], ref.clamped_glu(_f64(gu)[:, :half], _f64(gu)[:, half:2 * half], 1.25), dtype)
+    assert (out[:, half:] == 7.0).all()
 
 
 # ---- rotation, latent norm, cache --------------------------------------------------------------

@@ -284,3 +284,65 @@ def test_window_attention_of_single_rows(rows, heads, kv_heads, dim, vdim, longe
     got = out.view(rows, heads, vdim).double()
     # bf16 soft-max weights and results: 2^-9 each of a value, relative to the row
     assert ((got - want).norm(dim=-1) / want.norm(dim=-1)).max() < 1e-2
+
+
+@pytest.mark.parametrize("dtype", BOTH)
+@pytest.mark.parametrize("per_head", [True, False])
+@pytest.mark.parametrize("rows,heads,vdim,shift", [(1, 1, 64, 0), (33, 3, 64, 0), (17, 5, 128, 0), (9, 32, 256, 0), (9, 33, 256, 0),
+                                                   (5, 4, 128, 4)])
+def test_gated_norm_of_eights(rows, heads, vdim, shift, per_head, dtype):
+    """Workgroups that end within a row, rows of 8192 (the most registers hold) and above, a gate off its 16 bytes in bf16."""
+    from scalellm_amd import mixer_kernels as mk
+    g = torch.Generator().manual_seed(7)
+    n = heads * vdim
+    o = torch.randn(rows, heads, vdim, generator=g) * 3
+    gate = torch.randn(rows, n + 8 + shift, generator=g).to(dtype).to(DEV)[:, shift:]
+    w = torch.randn(vdim if per_head else n, generator=g)
+    out = torch.full((rows, n + 40), float("nan"), dtype=dtype, device=DEV)
+    mk.gated_norm(o.to(DEV), vdim, gate, w.to(DEV), out, eps=1e-3, per_head=per_head, scale=0.3)
+    x = o.double().numpy() if per_head else o.double().numpy().reshape(rows, n)
+    want = 0.3 * ref.rms_norm(x, w.double().numpy(), 1e-3).reshape(rows, n) * ref.sigmoid(gate[:, :n].double().cpu().numpy())
+    # (one rounding to bf16, whose neighbours above 1 are 2^-7 apart: half of that, 2^-8 of the value at most)
+    got = out[:, :n].double().cpu().numpy()
+    np.testing.assert_allclose(got, want, rtol=1e-5 if dtype == torch.float32 else 2 ** -8 + 1e-5, atol=1e-6)
+    assert float(out[:, n:].abs().max()) == 0.0
+
+
+@pytest.mark.parametrize("dtype", BOTH)
+@pytest.mark.parametrize("heads,kv,dim,d_pad,rot,v_pad,shift", [(16, 8, 128, 128, 128, 128, 0), (3, 1, 64, 64, 32, 128, 0),
+                                                                (2, 2, 256, 256, 0, 64, 0), (6, 3, 112, 128, 48, 112, 0),
+                                                                (4, 2, 128, 128, 24, 128, 0), (4, 2, 64, 64, 64, 64, 4)])
+def test_window_append(heads, kv, dim, d_pad, rot, v_pad, shift, dtype):
+    """Queries in place and keys and values in their slots: every head width that columns in eights have, a rotation that ends or
+    whose halves end within a head, heads narrower than their columns, halves that are no eights, rows off their 16 bytes."""
+    from scalellm_amd import mixer_kernels as mk
+    g = torch.Generator().manual_seed(8)
+    rows, eps, off_k = 21, 1e-3, heads * d_pad
+    off_v = off_k + kv * d_pad
+    proj = torch.randn(rows, off_v + kv * v_pad + 8 + shift, generator=g).to(dtype)[:, shift:]
+    qw, kw, angle = torch.randn(dim, generator=g), torch.randn(dim, generator=g), torch.randn(50, rot // 2, generator=g)
+    cs = torch.cat([angle.cos(), angle.sin()], dim=1).contiguous()
+    pos, slots = torch.randperm(50, generator=g)[:rows].int(), torch.randperm(40, generator=g)[:rows].int()
+    keys = torch.full((40, kv, d_pad), 5.0, dtype=dtype, device=DEV)
+    values = torch.full((40, kv, v_pad), 5.0, dtype=dtype, device=DEV)
+    x = proj.to(DEV) if not shift else torch.nn.functional.pad(proj, (shift, 0)).to(DEV)[:, shift:]
+    mk.window_append(x, keys, values, qw.to(DEV), kw.to(DEV), cs.to(DEV), pos.to(DEV), slots.to(DEV), heads=heads, dim=dim, off_q=0,
+                     off_k=off_k, off_v=off_v, eps=eps)
+    src, c, s = proj.double().numpy(), np.cos(angle.double().numpy())[pos][:, None], np.sin(angle.double().numpy())[pos][:, None]
+
+    def check(got, v, w, n):
+        y = ref.rms_norm(v.reshape(rows, n, d_pad)[:, :, :dim], w.double().numpy(), eps)
+        lo, hi = y[:, :, :rot // 2].copy(), y[:, :, rot // 2:rot].copy()
+        size = np.abs(y).copy()
+        size[:, :, :rot // 2] = size[:, :, rot // 2:rot] = np.hypot(lo, hi)
+        y[:, :, :rot // 2], y[:, :, rot // 2:rot] = lo * c - hi * s, lo * s + hi * c
+        got = got.double().cpu().numpy().reshape(rows, n, d_pad)
+        # (one rounding to bf16, at most 2^-8 of the value; the rotation in 32 bits is off by some 1e-7 of the pair it turns)
+        assert (np.abs(got[:, :, :dim] - y) <= (0 if dtype == torch.float32 else 2 ** -8) * np.abs(y) + 2e-6 * size).all()
+        assert not got[:, :, dim:].any()
+    check(x[:, :off_k], src[:, :off_k], qw, heads)
+    check(keys[slots.long()], src[:, off_k:off_v], kw, kv)
+    assert torch.equal(values[slots.long()].cpu(), proj[:, off_v:off_v + kv * v_pad].reshape(rows, kv, v_pad))
+    assert torch.equal(x[:, off_k:].cpu(), proj[:, off_k:])
+    rest = [i for i in range(40) if i not in slots.tolist()]
+    assert (keys[rest] == 5.0).all() and (values[rest] == 5.0).all()
