@@ -15,10 +15,12 @@
 //             wave's soft-max has another tile's products to hide behind
 //   softmax   every wave reads the scores back in the B layout of the second product (column = head = lane % 16,
 //             8 consecutive keys) and does the row statistics itself: no second exchange, one scalar per lane
-//   O^T += C^T P^T   wave w owns an eighth of the latent columns; A = C^T out of the row-major tile by the transpose
+//   O^T += C^T P^T   a wave owns an eighth of the latent columns (several head blocks: a quarter of them for half of the blocks); A = C^T out of the row-major tile by the transpose
 //             read (ds_read_b64_tr_b16: 4 keys of one column per lane)
-// Bound: HBM (the cache stream) for 16 heads; the score exchange and the redundant soft-max are what a wide
-// head block costs.  Ranges that are split leave fp32 partials for latent_attn_combine_kernel.
+// Bound: HBM (the cache stream) for 16 heads, 128 rows of 4096 keys 5.5 TB/s; with 32 the soft-max every wave repeats, between two
+// barriers, is as long as the stream (the same with every tile out of the L2: 104 us).  32 heads, 128 rows of 4096 keys: 126 us with
+// the soft-max of both head blocks in every wave and a 64-bit address per lane and row, 110 with half of it and one address a tile;
+// 64 rows of 500 - 1000 keys 32.5 -> 30.6.  Ranges that are split leave fp32 partials for latent_attn_combine_kernel.
 //
 // latent_attn_any_kernel: any size, any dtype, VALU: the 32-bit path and sizes without an MFMA form.
 #include "latent_common.h"
@@ -74,7 +76,9 @@ __global__ void __launch_bounds__(512) latent_attn_kernel(const LatentAttnK p) {
   constexpr int QS = R / 32;                 // MFMA k-steps of the scores
   constexpr int KH = MH == 1 ? 2 : 1;        // waves that share a score block's contraction
   constexpr int QW = (QS + KH - 1) / KH;     // k-steps per wave
-  constexpr int NT = KP >= 128 ? KP / 128 : 1;  // 16-column blocks of the latent per wave
+  constexpr int HS = MH == 1 ? 1 : 2;        // groups of head blocks: a wave takes one, MG blocks,
+  constexpr int MG = MH / HS, CG = 8 / HS;   // and one of CG groups of the latent's columns,
+  constexpr int NT = KP >= 16 * CG ? KP / (16 * CG) : 1;  // NT blocks of 16
   constexpr int SS = KT + 4;                 // score row stride (floats)
   constexpr int SC = KH * 16 * MH * SS;      // floats of one tile's scores
   constexpr int FIT = (163840 - 8 * SC - 4 * LA_TBL) / TILE, NBUF = FIT > 8 ? 8 : FIT;  // tiles in the ring
@@ -121,55 +125,72 @@ __global__ void __launch_bounds__(512) latent_attn_kernel(const LatentAttnK p) {
   int lo = a.window > 0 ? max(0, pos - a.window + 1) : 0;
   int hi = pos + 1;
   if (p.n_splits > 1) {
-    const int tiles = (hi - lo + KT - 1) / KT;
+    const int first = lo & -KT, tiles = (hi - first + KT - 1) / KT;
     const int per = (tiles + p.n_splits - 1) / p.n_splits * KT;
-    lo = min(hi, lo + split * per);
-    hi = min(hi, lo + per);
+    lo = min(hi, max(lo, first + split * per));
+    hi = min(hi, first + (split + 1) * per);
   }
   // (the queries have arrived before the first DMA is issued: a wait for them later would drain the ring)
 #pragma unroll
   for (int s = 0; s < QW; ++s) asm volatile("" : "+v"(qf[s]));
 
-  // the segment of the range whose block-table entries are staged: keys [lo, hi)
+  // the segment of the range whose block-table entries are staged: keys [lo, hi), in tiles from the multiple of KT at or before lo
   const int range_hi = hi;
-  int blk0 = 0, n_tiles = 0;
+  int blk0 = 0, n_tiles = 0, base = 0;
   const uint32_t ring0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)ring;
   const char* cache = reinterpret_cast<const char*>(a.cache);
+  uint32_t from[NHI];   // where this lane's pieces lie in a tile of consecutive rows
+#pragma unroll
+  for (int i = 0; i < NHI; ++i) {
+    const int u = min(wave + 8 * i, NTOT - 1) * 64 + lane, r = u / CHP;
+    from[i] = (uint32_t)(r * (R * 2) + 16 * min((u % CHP) ^ ((r >> 1) & 7), CH - 1));
+  }
+  auto entry = [&](int t) { return tbl[(min(max(base + t * KT, lo), hi - 1) >> p.block_shift) - blk0]; };
+  // A whole tile within a block of the cache: one uniform address.  Else a row at a time (rows there are not re-read the first or the last
+  // there is; masked below).  (16 heads, every tile out of the L2: 95 us -> 82.)
   // (inline asm: through the builtin the compiler makes every read of the ring wait for the DMA into its other tiles)
-  auto issue = [&](int t) {
+  auto issue = [&](int t, int first_slot) {
     const uint32_t dst0 = ring0 + (uint32_t)(t % NBUF) * TILE;
-    const char* src[NHI];
+    const int k0 = base + t * KT;
+    if (p.block_shift >= 5 && k0 >= lo && k0 + KT <= hi) {
+      const char* src = cache + (int64_t)(__builtin_amdgcn_readfirstlane(first_slot) + (k0 & p.block_mask)) * (R * 2);
+      if (p.stream) {
+#pragma unroll
+        for (int i = 0; i < NHI; ++i)
+          if (i < NLO || wave < NTOT % 8)
+            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt"
+                         :
+                         : "v"(from[i]), "s"(src), "s"(dst0 + (uint32_t)(wave + 8 * i) * 1024u)
+                         : "memory", "m0");
+      } else {
+#pragma unroll
+        for (int i = 0; i < NHI; ++i)
+          if (i < NLO || wave < NTOT % 8)
+            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                         :
+                         : "v"(from[i]), "s"(src), "s"(dst0 + (uint32_t)(wave + 8 * i) * 1024u)
+                         : "memory", "m0");
+      }
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < NHI; ++i) {
-      const int u = min(wave + 8 * i, NTOT - 1) * 64 + lane;
-      const int r = u / CHP, c = min((u % CHP) ^ ((r >> 1) & 7), CH - 1);
-      const int key = min(lo + t * KT + r, hi - 1);  // rows past the end re-read the last one; masked below
+      const uint32_t r = from[i] / (R * 2), c = from[i] % (R * 2);
+      const int key = max(lo, min(k0 + (int)r, hi - 1));
       const int slot = tbl[(key >> p.block_shift) - blk0];
-      src[i] = cache + (int64_t)(slot + (key & p.block_mask)) * (R * 2) + 16 * c;
-    }
-    if (p.stream) {
-#pragma unroll
-      for (int i = 0; i < NHI; ++i)
-        if (i < NLO || wave < NTOT % 8)
-          asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt"
-                       :
-                       : "v"(src[i]), "s"(dst0 + (uint32_t)(wave + 8 * i) * 1024u)
-                       : "memory", "m0");
-    } else {
-#pragma unroll
-      for (int i = 0; i < NHI; ++i)
-        if (i < NLO || wave < NTOT % 8)
-          asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
-                       :
-                       : "v"(src[i]), "s"(dst0 + (uint32_t)(wave + 8 * i) * 1024u)
-                       : "memory", "m0");
+      const char* src = cache + (int64_t)(slot + (key & p.block_mask)) * (R * 2) + c;
+      if (i < NLO || wave < NTOT % 8)
+        asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
+                     :
+                     : "v"(src), "s"(dst0 + (uint32_t)(wave + 8 * i) * 1024u)
+                     : "memory", "m0");
     }
   };
 
-  f32x4 o[MH][NT];
-  float m_run[MH], l_run[MH];
+  f32x4 o[MG][NT];
+  float m_run[MG], l_run[MG];
 #pragma unroll
-  for (int m = 0; m < MH; ++m) {
+  for (int m = 0; m < MG; ++m) {
     m_run[m] = M_INIT_F;
     l_run[m] = 0.f;
 #pragma unroll
@@ -182,10 +203,11 @@ __global__ void __launch_bounds__(512) latent_attn_kernel(const LatentAttnK p) {
   const uint32_t tr_row = (uint32_t)(8 * g + (l16 >> 2)) * ROWB + (uint32_t)(l16 & 1) * 8u;
   const uint32_t tr_x0 = (uint32_t)((4 * g + (l16 >> 3)) & 7) ^ (uint32_t)((l16 >> 1) & 1);
   const uint32_t tr_x1 = (uint32_t)((4 * g + 2 + (l16 >> 3)) & 7) ^ (uint32_t)((l16 >> 1) & 1);
-  const uint32_t tr_c = (uint32_t)wave * (2 * NT);
-  const bool columns = KP >= 128 || wave < KP / 16;
+  const int hg = wave / CG, cg = wave % CG;
+  const uint32_t tr_c = (uint32_t)cg * (2 * NT);
+  const bool columns = cg < KP / (16 * NT);
 
-  constexpr int QC = QW > 10 ? (QW + 1) / 2 : QW;   // k-steps read ahead of the products (register budget)
+  constexpr int QC = QW > 10 ? (QW + 2) / 3 : QW;   // k-steps read ahead of the products (register budget)
   bf16x8_t kf[QC];
   auto read_rows = [&](int t, int first) {   // A fragments of tile t, k-steps from `first` of this wave's
     const uint32_t base = ring0 + (uint32_t)(t % NBUF) * TILE + (uint32_t)(16 * kb) * ROWB + k_row;
@@ -216,11 +238,13 @@ __global__ void __launch_bounds__(512) latent_attn_kernel(const LatentAttnK p) {
   for (; lo < range_hi; lo = hi) {
     blk0 = lo >> p.block_shift;
     hi = min(range_hi, (blk0 + LA_TBL) << p.block_shift);
-    n_tiles = (hi - lo + KT - 1) / KT;
+    base = lo & -KT;
+    n_tiles = (hi - base + KT - 1) / KT;
     for (int i = tid; i <= ((hi - 1) >> p.block_shift) - blk0; i += 512) tbl[i] = a.block_table[bcu + blk0 + i];
     __syncthreads();
 #pragma unroll 1
-    for (int t = 0; t < min(NBUF - 1, n_tiles); ++t) issue(t);
+    for (int t = 0; t < min(NBUF - 1, n_tiles); ++t) issue(t, entry(t));
+    int slot = entry(NBUF - 1);   // (of the tile issued next: read a tile ahead)
     arrived(min(NBUF - 2, n_tiles - 1));
     lds_barrier();
     if (scorer) {
@@ -228,10 +252,11 @@ __global__ void __launch_bounds__(512) latent_attn_kernel(const LatentAttnK p) {
       score(0);
     }
     for (int t = 0; t < n_tiles; ++t) {
-      const int k0 = lo + t * KT;
+      const int k0 = base + t * KT;
       if (t + 1 < n_tiles) arrived(min(NBUF - 3, n_tiles - 2 - t));
       lds_barrier();   // tile t + 1 and the scores of tile t are there, tile t - 1 is done with
-      if (t + NBUF - 1 < n_tiles) issue(t + NBUF - 1);
+      if (t + NBUF - 1 < n_tiles) issue(t + NBUF - 1, slot);
+      slot = entry(t + NBUF);
       const uint32_t tile = ring0 + (uint32_t)(t % NBUF) * TILE;
       const bool next = scorer && t + 1 < n_tiles;
       if (next) read_rows(t + 1, 0);
@@ -240,12 +265,12 @@ __global__ void __launch_bounds__(512) latent_attn_kernel(const LatentAttnK p) {
         continue;
       }
       // ---- scores back in the B layout of the second product, C^T fragments behind them (read under the soft-max)
-      f32x4 raw[MH][KH][2];
+      f32x4 raw[MG][KH][2];
 #pragma unroll
-      for (int m = 0; m < MH; ++m)
+      for (int m = 0; m < MG; ++m)
 #pragma unroll
         for (int k = 0; k < KH; ++k) {
-          const float* sp = &sc[t & 1][(16 * (MH * k + m) + l16) * SS + 8 * g];
+          const float* sp = &sc[t & 1][(16 * (MH * k + MG * hg + m) + l16) * SS + 8 * g];
           raw[m][k][0] = *reinterpret_cast<const f32x4*>(sp);
           raw[m][k][1] = *reinterpret_cast<const f32x4*>(sp + 4);
         }
@@ -261,9 +286,10 @@ __global__ void __launch_bounds__(512) latent_attn_kernel(const LatentAttnK p) {
       __builtin_amdgcn_sched_barrier(0);
       if (next) score(t + 1);
       // ---- soft-max
-      bf16x8_t pf[MH];
+      const bool cut = k0 < lo || k0 + KT > hi;
+      bf16x8_t pf[MG];
 #pragma unroll
-      for (int m = 0; m < MH; ++m) {
+      for (int m = 0; m < MG; ++m) {
         float v[8];
         float mx = M_INIT_F;
 #pragma unroll
@@ -271,9 +297,14 @@ __global__ void __launch_bounds__(512) latent_attn_kernel(const LatentAttnK p) {
           float x = raw[m][0][j >> 2][j & 3];
 #pragma unroll
           for (int k = 1; k < KH; ++k) x += raw[m][k][j >> 2][j & 3];
-          v[j] = k0 + 8 * g + j < hi ? x * p.scale2 : -INFINITY;
-          mx = fmaxf(mx, v[j]);
+          v[j] = x * p.scale2;
         }
+        if (cut)
+#pragma unroll
+          for (int j = 0; j < 8; ++j)
+            if (k0 + 8 * g + j < lo || k0 + 8 * g + j >= hi) v[j] = -INFINITY;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) mx = fmaxf(mx, v[j]);
         mx = max_over_groups(mx);
         const float m_new = fmaxf(m_run[m], mx);
         const float alpha = fast_exp2(m_run[m] - m_new);
@@ -297,29 +328,30 @@ __global__ void __launch_bounds__(512) latent_attn_kernel(const LatentAttnK p) {
 #pragma unroll
       for (int t2 = 0; t2 < NT; ++t2)
 #pragma unroll
-        for (int m = 0; m < MH; ++m)
+        for (int m = 0; m < MG; ++m)
           o[m][t2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, ct[t2]), pf[m], o[m][t2], 0, 0, 0);
     }
     lds_barrier();   // ring and table are free for the next segment
   }
 
-  // The accumulators (lane: head l16 of block m, latent columns 16 NT wave + 16 t + 4 g .. + 3) go through the ring, so
+  // The accumulators (lane: head l16 of a block, latent columns 16 NT cg + 16 t + 4 g .. + 3) go through the ring, so
   // that whole lines leave the chip: straight from the registers a store touches 64 bytes of 16 rows.
   constexpr int OS = KP + 4;   // row stride (floats)
   static_assert(16 * MH * OS * 4 <= NBUF * TILE, "the output tile fits the ring");
   float* ot = reinterpret_cast<float*>(ring);
 #pragma unroll
-  for (int m = 0; m < MH; ++m) {
+  for (int m = 0; m < MG; ++m) {
+    const int hr = 16 * (MG * hg + m) + l16;
     if (columns) {
 #pragma unroll
-      for (int t = 0; t < NT; ++t) *reinterpret_cast<f32x4*>(ot + (16 * m + l16) * OS + wave * (16 * NT) + 16 * t + 4 * g) = o[m][t];
+      for (int t = 0; t < NT; ++t) *reinterpret_cast<f32x4*>(ot + hr * OS + cg * (16 * NT) + 16 * t + 4 * g) = o[m][t];
     }
     float l = l_run[m];
     l += __shfl_xor(l, 16, 64);
     l += __shfl_xor(l, 32, 64);
-    if (wave == 0 && g == 0) {
-      sc[0][16 * m + l16] = m_run[m];
-      sc[1][16 * m + l16] = l;
+    if (cg == 0 && g == 0) {
+      sc[0][hr] = m_run[m];
+      sc[1][hr] = l;
     }
   }
   __syncthreads();
@@ -455,7 +487,8 @@ __global__ void __launch_bounds__(256) latent_attn_any_kernel(const LatentAttnK 
 
 // Head blocks of 16 per workgroup (the scores of four do not fit beside the tiles of the widest latent).  Few rows leave fewer
 // splits, and fewer partials behind them, with a block to a workgroup: the blocks of a split share an L2 (32 heads, 4096 keys: 1 row
-// 19.2 -> 16.1 us, 8 rows 26.9 -> 24.9; 32 rows, 2000 - 4001 keys 46 -> 50).
+// 19.2 -> 16.1 us, 8 rows 26.9 -> 24.9; 32 rows, 2000 - 4001 keys 46 -> 50, and two
+// blocks take 42 since their waves share the soft-max).
 static int la_mh(const slm_latent_attn_args& a) {
   if (a.rows < 24 && a.heads <= 32) return 1;
   return a.heads > 32 && a.c_pad < 512 ? 4 : a.heads > 16 ? 2 : 1;

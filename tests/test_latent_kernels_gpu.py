@@ -312,6 +312,29 @@ def test_latent_attention_of_more_blocks_than_are_staged_at_once(block, lens):
             _close(out, want, dt, b16=1.5e-2)
 
 
+@pytest.mark.parametrize("block", [16, 32, 128])
+@pytest.mark.parametrize("c_pad,heads", [(64, 32), (128, 64), (256, 40), (512, 16), (512, 32)])
+def test_latent_attention_of_whole_and_cut_tiles(c_pad, heads, block):
+    """Rows that see whole tiles of 32 keys of a block, and windows that cut the first and the last of them; what is in no sequence
+    is NaN and must not be read into a product."""
+    lk, r_pad, dt = _lk(), 64, torch.bfloat16
+    lens = [32, 63, 64, 95, 129, 300] * 4
+    pg = Paged(lens, block, c_pad, r_pad, dt, seed=block)
+    mine = torch.zeros(pg.cache.size(0), dtype=torch.bool)
+    for s, n in enumerate(lens):
+        mine[[pg.slot(s, p) for p in range(n)]] = True
+    pg.cache[~mine.to(DEV)] = float("nan")
+    q = _rnd(2, len(lens), heads, c_pad + r_pad, dtype=dt)
+    scale = (c_pad + r_pad) ** -0.5
+    for window in (0, 32, 97):
+        want = np.stack([_attn_ref(_f64(q[i]), pg.rows(i), n - 1, window, scale, c_pad) for i, n in enumerate(lens)])
+        for kw in (dict(), dict(n_splits=1), dict(n_splits=3)):
+            out = torch.full((len(lens), heads, c_pad), float("nan"), dtype=dt, device=DEV)
+            lk.latent_attention(q, pg.cache, out, pg.dev([n - 1 for n in lens]), pg.dev(range(len(lens) + 1)), pg.dev(pg.table),
+                                pg.dev(pg.cu), block_size=block, window=window, scale=scale, max_kv_len=300, **kw)
+            _close(out, want, dt, b16=1.5e-2)
+
+
 # ---- prompt portions ---------------------------------------------------------------------------
 @pytest.mark.parametrize("q_dim,r_pad,v_pad", [(32, 32, 32), (32, 64, 64), (64, 64, 128), (128, 32, 64), (128, 64, 128), (192, 64, 64)])
 @pytest.mark.parametrize("window", [0, 1, 40, 64, 129, 300])
