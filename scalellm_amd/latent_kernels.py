@@ -143,11 +143,11 @@ def streams_rows(x: torch.Tensor) -> bool:
 def stream_layout(w: torch.Tensor, glu: bool = False) -> Optional[torch.Tensor]:
     """W [N, K] once more in the order slm_linear_stream reads it (include/slm_latent.h), made at load: what products of
     few rows run on.  The row-major tensor stays for products of many.  glu: W = [gate | up].  None where that kernel has
-    no form (32-bit weights, gate halves that are no multiple of 32)."""
+    no form (32-bit weights, gate halves that are no multiple of 32) and for weights that no kernel reads yet (a model
+    loaded on the host)."""
     N, K = w.shape
-    if w.dtype != torch.bfloat16 or K % 64 or N % 16 or (glu and N % 64):
+    if w.dtype != torch.bfloat16 or K % 64 or N % 16 or (glu and N % 64) or not w.is_cuda or not w.is_contiguous() or w.data_ptr() % 16:
         return None
-    _need(w.is_cuda and w.is_contiguous(), "stream_layout: contiguous weights on the GPU")
     out = torch.empty((N + 63) // 64, K // 64, 4, 2, 64, 8, dtype=w.dtype, device=w.device)
     latent_check(_lib.latent_lib().slm_stream_layout(_p(out), _p(w), N, K, int(glu), _stream()), "slm_stream_layout")
     return out
