@@ -176,10 +176,10 @@ def main(argv=None):
                     nbytes, flops = bs * seen * R * 2, 2 * bs * seen * heads * (R + a0.c_pad)
                     h = torch.randn(bs, m.k_width, device=DEV).to(torch.bfloat16)
                     act = torch.randn(bs, ff, device=DEV).to(torch.bfloat16)
-                    lins = {"proj": lambda: [lk.linear(h, x.attn.w_in) for x in m.layers],
-                            "gate_up+act": lambda: [lk.linear_glu(h, x.mlp.w_gate_up, act, 7.0) for x in m.layers],
-                            "down": lambda: [x.mlp.w_down is not None and (lk.linear_slabs if bs <= lk.STREAM_MAX_ROWS else lk.linear)(act, x.mlp.w_down)
-                                             for x in m.layers]}
+                    lins = {"proj": lambda: [lk.linear(h, x.attn.w_in, layout=x.attn.l_in) for x in m.layers],
+                            "gate_up+act": lambda: [lk.linear_glu(h, x.mlp.w_gate_up, act, 7.0, layout=x.mlp.l_gate_up) for x in m.layers],
+                            "down": lambda: [x.mlp.w_down is not None and (lk.linear_slabs if bs <= lk.slab_rows(x.mlp.l_down) else lk.linear)(
+                                act, x.mlp.w_down, layout=x.mlp.l_down) for x in m.layers]}
                     wbytes = {"proj": a0.w_in.numel() * 2, "gate_up+act": m.layers[0].mlp.w_gate_up.numel() * 2,
                               "down": m.layers[0].mlp.w_down.numel() * 2}
                     wflops = {k: bs * v for k, v in wbytes.items()}
@@ -251,7 +251,7 @@ def main(argv=None):
                 if D:
                     h = torch.randn(T, m.k_width, device=DEV).to(torch.bfloat16)
                     act = torch.empty(T, ff, device=DEV, dtype=torch.bfloat16)
-                    t = timed(lambda: [lk.linear_glu(h, x.mlp.w_gate_up, act, 7.0) for x in m.layers]) / L
+                    t = timed(lambda: [lk.linear_glu(h, x.mlp.w_gate_up, act, 7.0, layout=x.mlp.l_gate_up) for x in m.layers]) / L
                 else:
                     h = torch.randn(T, width, device=DEV).to(torch.bfloat16)
                     t = timed(lambda: [x["gate_up"].forward(h, out=m.buf["act"][:T]) for x in m.layers]) / L

@@ -152,16 +152,16 @@ def main(argv=None):
                     block_size=BLOCK, window=window, keep_first=KEEP, scale=0.09, softcap=30.0, max_kv_len=context) for x, c in paras], len(paras),
                     nbytes=bs * seen * kv_heads * 512, flops=4 * bs * seen * heads * 128, bs=bs)
                 act = torch.randn(bs, ff, device=DEV).to(torch.bfloat16)
-                wide = bs > lk.STREAM_MAX_ROWS
+                wide = bs > lk.slab_rows(m.layers[0].mlp.l_down)
 
                 def mm(name, fn, w, n):
                     kernel(name, fn, n, nbytes=w.numel() * 2, flops=2 * bs * w.numel(), bs=bs)
-                mm("delta proj", lambda: [lk.linear(h, x.mixer.w_in) for x, _ in deltas], d0.w_in, len(deltas))
+                mm("delta proj", lambda: [lk.linear(h, x.mixer.w_in, layout=x.mixer.l_in) for x, _ in deltas], d0.w_in, len(deltas))
                 mm("low-rank", lambda: [lk.linear_heads(projd[:, d0.off_a1:], d0.low_k, x.mixer.w_low, low, d0.low_n) for x, _ in deltas], d0.w_low,
                    len(deltas))
-                mm("parallel proj", lambda: [lk.linear(h, x.mixer.w_in) for x, _ in paras], p0.w_in, len(paras))
-                mm("gate_up+act", lambda: [lk.linear_glu(h, x.mlp.w_gate_up, act, float("inf"), 1.0, 0.0) for x in m.layers], m.layers[0].mlp.w_gate_up, L)
-                mm("down", lambda: [(lk.linear if wide else lk.linear_slabs)(act, x.mlp.w_down) for x in m.layers], m.layers[0].mlp.w_down, L)
+                mm("parallel proj", lambda: [lk.linear(h, x.mixer.w_in, layout=x.mixer.l_in) for x, _ in paras], p0.w_in, len(paras))
+                mm("gate_up+act", lambda: [lk.linear_glu(h, x.mlp.w_gate_up, act, float("inf"), 1.0, 0.0, layout=x.mlp.l_gate_up) for x in m.layers], m.layers[0].mlp.w_gate_up, L)
+                mm("down", lambda: [(lk.linear if wide else lk.linear_slabs)(act, x.mlp.w_down, layout=x.mlp.l_down) for x in m.layers], m.layers[0].mlp.w_down, L)
             for name, q_lens, kv_lens in cases:
                 tokens, positions, params, _ = batch(q_lens, kv_lens, block, vocab, which != "llama")
                 T = tokens.numel()
@@ -199,7 +199,7 @@ def main(argv=None):
                        1, nbytes=T * 4 * (heads + 2 * kv_heads) * 128, batch=name)
                 h = torch.randn(T, m.k_width, device=DEV).to(torch.bfloat16)
                 act = torch.empty(T, ff, device=DEV, dtype=torch.bfloat16)
-                kernel("gate_up+act", lambda: [lk.linear_glu(h, z.mlp.w_gate_up, act, float("inf"), 1.0, 0.0) for z in m.layers], L, flops=4 * T * width * ff,
+                kernel("gate_up+act", lambda: [lk.linear_glu(h, z.mlp.w_gate_up, act, float("inf"), 1.0, 0.0, layout=z.mlp.l_gate_up) for z in m.layers], L, flops=4 * T * width * ff,
                        batch=name)
             del m
     return 0
