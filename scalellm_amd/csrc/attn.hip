@@ -542,13 +542,18 @@ __global__ void __launch_bounds__(256) attn_combine_kernel(const AttnKParams p, 
   // q_cu_lens[batch]: no kernel of the call wrote their partials) run on clamped / unwritten but
   // in-bounds data and only skip the final store, so the q_cu lookup overlaps the partial loads
   // instead of adding a round trip in front of them.
-  const int64_t n_items = (int64_t)p.n_tokens * p.n_heads;
+  const int64_t n_items = (p.part_rows > 0 ? (int64_t)p.batch * p.part_rows : (int64_t)p.n_tokens) * p.n_heads;
   const int64_t item_raw = (int64_t)blockIdx.x * 4 + wv;
   bool valid = item_raw < n_items;
   const int64_t item = valid ? item_raw : n_items - 1;
-  const int tok = (int)(item / p.n_heads), head = (int)(item % p.n_heads);
+  int tok = (int)(item / p.n_heads);
+  const int head = (int)(item % p.n_heads);
   const int q_end = p.q_cu[p.batch];
-  if (p.rows_hi != 0x7fffffff || p.rows_lo != 0) {
+  if (p.part_rows > 0) {  // partials of the short sequences only
+    const int b = tok / p.part_rows, i = tok % p.part_rows, q0 = p.q_cu[b], q_len = p.q_cu[b + 1] - q0;
+    if (i >= q_len || q_len * p.group < p.rows_lo || q_len * p.group >= p.rows_hi) return;
+    tok = q0 + i;
+  } else if (p.rows_hi != 0x7fffffff || p.rows_lo != 0) {
     // mixed call: only the rows the token-major kernel produced are combined
     int lo_b = 0, hi_b = p.batch;
     while (lo_b < hi_b) {
@@ -663,7 +668,9 @@ struct AttnPlan {
   // balanced pure-decode partition (AttnKParams::bal): partial slots per (token, head) and the
   // piece-size floor that keeps a sequence's pieces within them
   int bal, part_slots, bal_qmin;
-  int small_splits;  // KV splits of the one-wave tile class of a mixed call whose other rows have one (else n_splits)
+  // the one-wave tile class of a mixed call whose other rows are not split: its KV splits (1: none either) and its longest
+  // sequence, whose tokens have a row of partials each (AttnKParams::part_rows)
+  int small_splits, small_rows;
 };
 constexpr int ATTN_BAL_ALIGN = 64;
 
@@ -890,15 +897,18 @@ static int plan_attn(const slm_attn_args* a, AttnPlan* pl) {
     pl->bal_qmin = (int)(qmin > 1 ? qmin : 1);
     if (pl->n_splits >= slots) pl->n_splits = slots - 1;  // P = n_tokens * n_splits workgroups per head group
   }
-  // A mixed call whose prompts need no split: the one-wave tiles have their own count, a wave for every SIMD as above, as
-  // far as its partials (a row for every token of the call) stay under 256 MB.
-  pl->small_splits = pl->n_splits;
-  if (pl->n_splits == 1 && mixed_on_tile(a) && tune_get(TUNE_ATTN_TILE_SPLITS, 0) <= 0) {
-    int64_t want = 1024 / ((int64_t)a->batch_size * a->n_kv_heads > 0 ? (int64_t)a->batch_size * a->n_kv_heads : 1);
-    const int64_t by_len = a->max_kv_len / 512, row = (int64_t)a->n_tokens * a->n_heads * (D + 2) * 4;
-    const int64_t by_size = row > 0 ? (256ll << 20) / row : 1;
-    want = std::min(std::min(want, (int64_t)16), std::min(by_len, by_size));
-    if (want > 1) pl->small_splits = (int)want;
+  // A mixed call whose prompts need no split: the one-wave tiles have their own count, a wave for every SIMD as above.  Their
+  // partials lie by sequence (at most 32 / G tokens of each: 1024 waves of 32 rows, 17 MB at head_dim 128, whatever the
+  // prompts bring), and none are kept where the sizes leave room for no such sequence: all tokens but a short sequence's
+  // are more than the others can bring.
+  pl->small_splits = 1;
+  pl->small_rows = 32 / G;
+  const int64_t shortest = singles_on_tile(a) ? 1 : 2;
+  if (pl->n_splits == 1 && mixed_on_tile(a) && tune_get(TUNE_ATTN_TILE_SPLITS, 0) <= 0 && pl->small_rows >= shortest && a->batch_size > 0 &&
+      a->n_tokens <= (int64_t)(a->batch_size - 1) * a->max_q_len + pl->small_rows) {
+    const int64_t want = std::min<int64_t>(1024 / ((int64_t)a->batch_size * a->n_kv_heads), 16);
+    const int64_t by_len = a->max_kv_len / 512;
+    pl->small_splits = (int)std::max<int64_t>(std::min(want, by_len), 1);
   }
   pl->u = tune_get(TUNE_ATTN_U, pl->w == 2 ? 2 : 4);  // (two chunks: the same bytes in flight with half the rows)
   if (pl->u != 2 && pl->u != 4) pl->u = 4;
@@ -968,6 +978,16 @@ static void dispatch_lpr(const AttnKParams& kp, const AttnPlan& pl, int64_t grid
 #endif
 }
 
+// rows of partials the call leaves, and their scratch
+static int64_t part_rows_of(const slm_attn_args* a, const AttnPlan& pl) {
+  if (pl.bal || pl.n_splits > 1) return a->n_tokens;
+  return pl.small_splits > 1 ? (int64_t)a->batch_size * pl.small_rows : 0;
+}
+static size_t part_bytes(const slm_attn_args* a, const AttnPlan& pl) {
+  const int slots = pl.bal || pl.n_splits > 1 ? pl.part_slots : pl.small_splits;
+  return (size_t)part_rows_of(a, pl) * a->n_heads * slots * (a->head_dim + 2) * sizeof(float);
+}
+
 }  // namespace slm
 
 using namespace slm;
@@ -989,9 +1009,7 @@ SLM_API int32_t slm_paged_kv_varlen_mha_decode_kernel(const slm_attn_args* a) {
 SLM_API size_t slm_paged_kv_varlen_mha_workspace_bytes(const slm_attn_args* a) {
   AttnPlan pl;
   if (plan_attn(a, &pl) != SLM_OK) return 0;
-  const int slots = pl.bal || pl.n_splits > 1 ? pl.part_slots : pl.small_splits;
-  if (slots <= 1) return 0;
-  return (size_t)a->n_tokens * a->n_heads * slots * (a->head_dim + 2) * sizeof(float);
+  return part_bytes(a, pl);
 }
 
 SLM_API int slm_paged_kv_varlen_mha(const slm_attn_args* a, void* stream) {
@@ -1036,7 +1054,7 @@ SLM_API int slm_paged_kv_varlen_mha(const slm_attn_args* a, void* stream) {
   } else {
     kp.softcap = 0.f; kp.pre_scale = 0.f; kp.scale_log2 = a->sm_scale * LOG2E;
   }
-  kp.o_part = nullptr; kp.ml_part = nullptr;
+  kp.o_part = nullptr; kp.ml_part = nullptr; kp.part_rows = 0;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   // Many query rows per KV head (prefill, chunked prefill, speculative verify): MFMA tile kernel.
   // max_q_len is the same scheduling contract as the reference's grid (tile_scheduler.cuh:23-27).
@@ -1055,11 +1073,9 @@ SLM_API int slm_paged_kv_varlen_mha(const slm_attn_args* a, void* stream) {
   const bool own_small = pl.small_splits > 1 && pl.n_splits == 1 && !pl.bal;  // only the one-wave tiles are split
   if (pl.n_splits > 1 || pl.bal || own_small) {
     const int slots = own_small ? pl.small_splits : pl.part_slots;
-    const size_t need =
-        (size_t)a->n_tokens * a->n_heads * slots * (a->head_dim + 2) * sizeof(float);
-    if (!a->workspace || a->workspace_bytes < need) return SLM_ERR_WORKSPACE;
+    if (!a->workspace || a->workspace_bytes < part_bytes(a, pl)) return SLM_ERR_WORKSPACE;
     kp.o_part = reinterpret_cast<float*>(a->workspace);
-    kp.ml_part = kp.o_part + (size_t)a->n_tokens * a->n_heads * slots * a->head_dim;
+    kp.ml_part = kp.o_part + (size_t)part_rows_of(a, pl) * a->n_heads * slots * a->head_dim;
   }
   bool tile_used = false;
   const bool dec_tile = singles_on_tile(a);
@@ -1079,11 +1095,12 @@ SLM_API int slm_paged_kv_varlen_mha(const slm_attn_args* a, void* stream) {
     if (do_stream && first_tile_rows < 33 && !(uniform_q && max_rows > 32)) {  // (group >= 32: every multi-row sequence already has > 32 rows)
       tk.rows_lo = first_tile_rows;
       tk.rows_hi = 33;
-      if (own_small) tk.n_splits = tk.part_slots = pl.small_splits;
+      if (own_small) tk.n_splits = tk.part_slots = pl.small_splits, tk.part_rows = pl.small_rows;
       rc = launch_attn_tile(tk, a->dtype, max_rows < 32 ? max_rows : 32, a->max_kv_len, st);
       if (rc != SLM_OK) return rc;
       tk.n_splits = pl.n_splits;
       tk.part_slots = pl.part_slots;
+      tk.part_rows = 0;
     }
     if (do_stream && max_rows > 32) {
       // rows <= group (q_len = 1) stay with the token-major kernel also when group > 32 (MQA)
@@ -1108,7 +1125,7 @@ SLM_API int slm_paged_kv_varlen_mha(const slm_attn_args* a, void* stream) {
     if (rc != SLM_OK) return rc;
   }
   if (do_combine && (pl.n_splits > 1 || pl.bal || own_small)) {
-    const int64_t items = (int64_t)a->n_tokens * a->n_heads;
+    const int64_t items = part_rows_of(a, pl) * a->n_heads;
     const dim3 g((unsigned)((items + 3) / 4)), blk(256);
     int lps_shift = 3;  // lanes per split: power of two >= head_dim / 4
     while ((4 << lps_shift) < a->head_dim) ++lps_shift;
@@ -1117,6 +1134,7 @@ SLM_API int slm_paged_kv_varlen_mha(const slm_attn_args* a, void* stream) {
       ck.rows_lo = first_tile_rows;
       ck.rows_hi = 33;
       ck.n_splits = ck.part_slots = pl.small_splits;
+      ck.part_rows = pl.small_rows;
     } else if (tile_used) {  // every kernel of the call wrote partials: combine every row
       ck.rows_lo = 0;
       ck.rows_hi = 0x7fffffff;

@@ -19,8 +19,8 @@ struct AttnKParams {
   const int* bt;
   const int* bcu;
   const float* alibi;
-  float* o_part;   // [n_tokens, n_heads, part_slots, head_dim]
-  float* ml_part;  // [n_tokens, n_heads, part_slots, 2]
+  float* o_part;   // [n_tokens (part_rows > 0: batch * part_rows), n_heads, part_slots, head_dim]
+  float* ml_part;  // [the same, n_heads, part_slots, 2]
   int batch, n_tokens, n_heads, n_kv_heads, head_dim;
   int block_shift, block_mask;
   int group;      // q heads per kv head
@@ -45,6 +45,7 @@ struct AttnKParams {
   int bal_qmin;    // bounds the pieces of one sequence by part_slots
   int bal_align;
   int part_slots;  // partial slots per (token, head): n_splits (classic) or the piece bound (balanced)
+  int part_rows;   // > 0: partials lie by (sequence, its token), part_rows of them a sequence: only short sequences have any
   int prio;        // > 0: the token kernel raises its wave priority (attn.hip)
 };
 
