@@ -133,6 +133,9 @@ typedef struct slm_attn_args {
  * get_estimate_workspace_size / set_workspace, src/layers/attention/handler.h
  * :40-47 is the natural home).  Pass num_splits to query a forced split count.*/
 SLM_API size_t slm_paged_kv_varlen_mha_workspace_bytes(const slm_attn_args* a);
+/* The part of it without which the call comes back with SLM_ERR_WORKSPACE: 0 for a mixed call whose only
+ * partials are those of its short sequences (they are not split without scratch: slower), else all of it.    */
+SLM_API size_t slm_paged_kv_varlen_mha_workspace_required(const slm_attn_args* a);
 /* Split count the heuristic would pick for `a` (host-side sizes only).        */
 SLM_API int32_t slm_paged_kv_varlen_mha_auto_splits(const slm_attn_args* a);
 /* which kernel the plan gives the q_len = 1 (decode) rows of this call: 0 = attn_token_kernel (HBM

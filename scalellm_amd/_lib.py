@@ -116,6 +116,8 @@ def lib() -> C.CDLL:
     L.slm_paged_kv_varlen_mha.argtypes = [C.POINTER(AttnArgs), C.c_void_p]
     L.slm_paged_kv_varlen_mha_workspace_bytes.restype = C.c_size_t
     L.slm_paged_kv_varlen_mha_workspace_bytes.argtypes = [C.POINTER(AttnArgs)]
+    L.slm_paged_kv_varlen_mha_workspace_required.restype = C.c_size_t
+    L.slm_paged_kv_varlen_mha_workspace_required.argtypes = [C.POINTER(AttnArgs)]
     L.slm_paged_kv_varlen_mha_auto_splits.restype = C.c_int32
     L.slm_paged_kv_varlen_mha_auto_splits.argtypes = [C.POINTER(AttnArgs)]
     L.slm_paged_kv_varlen_mha_decode_kernel.restype = C.c_int32

@@ -1012,6 +1012,12 @@ SLM_API size_t slm_paged_kv_varlen_mha_workspace_bytes(const slm_attn_args* a) {
   return part_bytes(a, pl);
 }
 
+SLM_API size_t slm_paged_kv_varlen_mha_workspace_required(const slm_attn_args* a) {
+  AttnPlan pl;
+  if (plan_attn(a, &pl) != SLM_OK) return 0;
+  return pl.n_splits > 1 || pl.bal ? part_bytes(a, pl) : 0;
+}
+
 SLM_API int slm_paged_kv_varlen_mha(const slm_attn_args* a, void* stream) {
   AttnPlan pl;
   int rc = plan_attn(a, &pl);
@@ -1070,10 +1076,11 @@ SLM_API int slm_paged_kv_varlen_mha(const slm_attn_args* a, void* stream) {
   kp.rows_hi = 0x7fffffff;
   kp.bal = pl.bal; kp.part_slots = pl.part_slots; kp.bal_qmin = pl.bal_qmin; kp.bal_align = ATTN_BAL_ALIGN;
   kp.prio = tune_get(TUNE_ATTN_PRIO, 1);  // measured on the two-lane bs 256 step: 25.08 -> 24.85 ms (2 x 2 runs)
-  const bool own_small = pl.small_splits > 1 && pl.n_splits == 1 && !pl.bal;  // only the one-wave tiles are split
+  const bool scratch = a->workspace && a->workspace_bytes >= part_bytes(a, pl);
+  const bool own_small = pl.small_splits > 1 && scratch;  // only the one-wave tiles are split (without scratch: none)
   if (pl.n_splits > 1 || pl.bal || own_small) {
     const int slots = own_small ? pl.small_splits : pl.part_slots;
-    if (!a->workspace || a->workspace_bytes < part_bytes(a, pl)) return SLM_ERR_WORKSPACE;
+    if (!scratch) return SLM_ERR_WORKSPACE;
     kp.o_part = reinterpret_cast<float*>(a->workspace);
     kp.ml_part = kp.o_part + (size_t)part_rows_of(a, pl) * a->n_heads * slots * a->head_dim;
   }

@@ -370,7 +370,9 @@ void LlamaForCausalLMHip::attn(Lane& ln, size_t li, std::vector<KVCache>& kv, in
   a.phase = phase;  // (1 / 2: the two lanes hand the KV-stream token on between the stream kernel and the combine pass)
   if (a.n_tokens == 0 || a.batch_size == 0) return;
   const size_t need = slm_paged_kv_varlen_mha_workspace_bytes(&a);
-  if (need > 0) {
+  const bool at_hand = scratch_[ln.idx].defined() && static_cast<size_t>(scratch_[ln.idx].nbytes()) >= need;
+  // (being captured: scratch that is not there only where the call cannot do without, and scratch() says so then)
+  if (need > 0 && (at_hand || !capturing() || slm_paged_kv_varlen_mha_workspace_required(&a) > 0)) {
     const auto& ws = scratch(ln.idx, need);
     a.workspace = ws.mutable_data_ptr();
     a.workspace_bytes = ws.nbytes();

@@ -49,7 +49,8 @@ std::unordered_map<int, torch::Tensor> g_ws;       // device index -> current sc
 std::unordered_map<int, torch::Tensor> g_user_ws;  // device index -> caller-supplied scratch
 std::vector<torch::Tensor> g_retired;              // replaced buffers (earlier captures point here)
 
-torch::Tensor workspace_for(const torch::Tensor& like, size_t bytes) {
+// required: what the call cannot do without; where no more can be had (under capture), an undefined tensor if that is nothing
+torch::Tensor workspace_for(const torch::Tensor& like, size_t bytes, size_t required) {
   std::lock_guard<std::mutex> lk(g_ws_mu);
   const int dev = like.device().index();
   auto user = g_user_ws.find(dev);
@@ -58,6 +59,7 @@ torch::Tensor workspace_for(const torch::Tensor& like, size_t bytes) {
   auto& ws = g_ws[dev];
   if (!ws.defined() || static_cast<size_t>(ws.nbytes()) < bytes) {
     const auto capturing = c10::hip::currentStreamCaptureStatusMayInitCtx();
+    if (capturing != c10::hip::CaptureStatus::None && required == 0) return {};
     TORCH_CHECK(capturing == c10::hip::CaptureStatus::None,
                 "slm: the kernel workspace must be sized before graph capture (need ", bytes,
                 " bytes): warm the step up first or call paged_kv_varlen_mha_set_workspace()");
@@ -124,9 +126,9 @@ void paged_kv_varlen_mha(torch::Tensor& out, const torch::Tensor& query,
   const size_t need = slm_paged_kv_varlen_mha_workspace_bytes(&a);
   torch::Tensor ws;
   if (need > 0) {
-    ws = workspace_for(query, need);
-    a.workspace = ws.mutable_data_ptr();
-    a.workspace_bytes = ws.nbytes();
+    ws = workspace_for(query, need, slm_paged_kv_varlen_mha_workspace_required(&a));
+    a.workspace = ws.defined() ? ws.mutable_data_ptr() : nullptr;
+    a.workspace_bytes = ws.defined() ? ws.nbytes() : 0;
   }
   check(slm_paged_kv_varlen_mha(&a, current_stream(query)), "slm_paged_kv_varlen_mha");
 }
@@ -511,7 +513,7 @@ void gptq_gemm(const torch::Tensor& A, const torch::Tensor& B, torch::Tensor& C,
   const size_t need = slm_w4a16_gemm_workspace_bytes(&g);
   torch::Tensor ws;
   if (need > 0) {
-    ws = workspace_for(A, need);
+    ws = workspace_for(A, need, need);
     g.workspace = ws.mutable_data_ptr();
     g.workspace_bytes = ws.nbytes();
   }
@@ -670,7 +672,7 @@ torch::Tensor W4Linear::forward(const torch::Tensor& input, const std::optional<
   const size_t need = slm_w4a16_gemm_workspace_bytes(&g);
   torch::Tensor ws;
   if (need > 0) {
-    ws = workspace_for(a, need);
+    ws = workspace_for(a, need, need);
     g.workspace = ws.mutable_data_ptr();
     g.workspace_bytes = ws.nbytes();
   }

@@ -163,6 +163,12 @@ def reserve_workspace(nbytes: int, device: Optional[torch.device] = None,
     return _grow(_workspaces, nbytes, dev, "workspace")
 
 
+def _fits_or_grows(nbytes: int, dev: torch.device) -> bool:
+    """Does the scratch hold nbytes, or may it be grown now?"""
+    ws = _workspaces.get(_dev_key(dev))
+    return (ws is not None and ws.numel() >= nbytes) or not torch.cuda.is_current_stream_capturing()
+
+
 def retired_workspace_bytes() -> int:
     return sum(t.numel() for t in _retired)
 
@@ -280,6 +286,8 @@ def paged_kv_varlen_mha(
     if a.n_tokens == 0 or a.batch_size == 0:
         return
     need = L.slm_paged_kv_varlen_mha_workspace_bytes(C.byref(a))
+    if need and not _fits_or_grows(need, query.device):   # (being captured: only what the call cannot do without)
+        need = L.slm_paged_kv_varlen_mha_workspace_required(C.byref(a))
     if need:
         ws = reserve_workspace(need, query.device)
         a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
