@@ -907,7 +907,10 @@ static int plan_attn(const slm_attn_args* a, AttnPlan* pl) {
   if (pl->n_splits == 1 && mixed_on_tile(a) && tune_get(TUNE_ATTN_TILE_SPLITS, 0) <= 0 && pl->small_rows >= shortest && a->batch_size > 0 &&
       a->n_tokens <= (int64_t)(a->batch_size - 1) * a->max_q_len + pl->small_rows) {
     const int64_t want = std::min<int64_t>(1024 / ((int64_t)a->batch_size * a->n_kv_heads), 16);
-    const int64_t by_len = a->max_kv_len / 512;
+    // (of the keys such a sequence sees: all of them, or those in front of its first row that the window leaves and its own)
+    const int64_t seen = a->sliding_window < 0 ? a->max_kv_len
+                                               : std::min<int64_t>(a->max_kv_len, (int64_t)a->sliding_window + pl->small_rows);
+    const int64_t by_len = seen / 512;
     pl->small_splits = (int)std::max<int64_t>(std::min(want, by_len), 1);
   }
   pl->u = tune_get(TUNE_ATTN_U, pl->w == 2 ? 2 : 4);  // (two chunks: the same bytes in flight with half the rows)

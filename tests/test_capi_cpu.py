@@ -117,13 +117,19 @@ def test_scratch_of_mixed_calls_is_for_their_short_sequences():
     whatever the prompts bring, and none where the sizes leave no room for such a sequence."""
     L = _lib.lib()
     assert L.slm_tuning_clear(None) == 0
-    need = lambda a: L.slm_paged_kv_varlen_mha_workspace_bytes(C.byref(a))  # noqa: E731
+
+    def need(a, window=-1):
+        a.sliding_window = window
+        return L.slm_paged_kv_varlen_mha_workspace_bytes(C.byref(a))
     row = 32 * 130 * 4   # bytes of a row of partials: 32 heads, 128 + 2 floats
     assert need(_attn(4, 5948, max_q=2048, max_kv=2048)) == 4 * 8 * row * 4          # (2048, 1500, 1100, 1300: by length 4 splits)
     assert need(_attn(4, 1468, max_q=512, max_kv=1900)) == 4 * 8 * row * 3
     assert need(_attn(4, 7900, max_q=2048, max_kv=2048)) == 0                        # more than three of 2048 and eight
     assert need(_attn(9, 264, max_q=256, max_kv=1000)) == 0                          # (nothing to split)
     assert need(_attn(9, 1032, max_q=1024, max_kv=4000)) == 9 * 8 * row * 7
+    a = _attn(4, 5948, max_q=2048, max_kv=8000)
+    for window, splits in ((-1, 15), (0, 1), (503, 1), (1016, 2), (2040, 4), (100000, 15)):   # (of the keys that are seen: window + 8)
+        assert need(a, window) == (4 * 8 * row * splits if splits > 1 else 0), window
     for heads, kv_heads in ((32, 32), (32, 8), (64, 8), (64, 2)):
         for bs in (2, 3, 17, 64, 500):
             for max_q in (2, 33, 300, 4000):
