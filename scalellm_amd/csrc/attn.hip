@@ -701,11 +701,13 @@ static bool mixed_on_tile(const slm_attn_args* a) {
 // they cost nothing that shows.  32 / 8 heads, n single rows of 4 k beside one prompt of 256, token -> tile: n = 1 358 -> 91 us,
 // 8 374 -> 94, 32 387 -> 139, 64 411 -> 235, 128 486 -> 410; of 512: 80 -> 47, 86 -> 51, 90 -> 61, 90 -> 68, 113 -> 95.  At 256
 // the token kernel has a workgroup on every CU and, with fewer than 8 heads on a KV head, the better rate (783 against
-// 814; 8 heads: 951 against 780).  SLM_ATTN_TILE_DECODE = 0: never.
+// 814; 8 heads: 951 against 780).  SLM_ATTN_TILE_DECODE: minimum group size here too, 0 = never.
 static bool singles_on_tile(const slm_attn_args* a) {
   const int G = a->n_heads / a->n_kv_heads;
-  return decode_on_tile(a) || (mixed_on_tile(a) && G <= 32 && (G >= 8 || a->batch_size < 224) &&
-                               tune_get(TUNE_ATTN_TILE_DECODE, 8) > 0);
+  if (decode_on_tile(a)) return true;
+  if (!mixed_on_tile(a) || G > 32) return false;
+  if (tune_is_set(TUNE_ATTN_TILE_DECODE)) return tune_get(TUNE_ATTN_TILE_DECODE, 8) > 0 && G >= tune_get(TUNE_ATTN_TILE_DECODE, 8);
+  return G >= 8 || a->batch_size < 224;
 }
 
 static int plan_attn(const slm_attn_args* a, AttnPlan* pl) {

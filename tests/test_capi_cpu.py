@@ -136,6 +136,20 @@ def test_scratch_of_mixed_calls_is_for_their_short_sequences():
                 assert need(_attn(bs, bs * max_q - 1, heads, kv_heads, max_q=max_q, max_kv=max_q + 9)) <= 1024 * 32 * 130 * 4
 
 
+def test_single_rows_of_mixed_calls_obey_the_knobs():
+    L = _lib.lib()
+    assert L.slm_tuning_clear(None) == 0
+    kernel = lambda a: L.slm_paged_kv_varlen_mha_decode_kernel(C.byref(a))  # noqa: E731
+    a = _attn(4, 1468, max_q=512, max_kv=1900)   # 4 query heads on a KV head
+    assert kernel(a) == 1
+    try:
+        for least, want in ((0, 0), (1, 1), (4, 1), (5, 0), (8, 0)):   # the least group on the tiles, 0 = none
+            assert L.slm_tuning_set(b"SLM_ATTN_TILE_DECODE", least) == 0
+            assert kernel(a) == want, least
+    finally:
+        L.slm_tuning_clear(b"SLM_ATTN_TILE_DECODE")
+
+
 def test_split_kv_heuristic_host_side():
     L = _lib.lib()
     assert L.slm_tuning_clear(None) == 0  # heuristics only: no override knob set
