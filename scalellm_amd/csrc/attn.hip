@@ -906,7 +906,8 @@ static int plan_attn(const slm_attn_args* a, AttnPlan* pl) {
   pl->small_splits = 1;
   pl->small_rows = 32 / G;
   const int64_t shortest = singles_on_tile(a) ? 1 : 2;
-  if (pl->n_splits == 1 && mixed_on_tile(a) && tune_get(TUNE_ATTN_TILE_SPLITS, 0) <= 0 && pl->small_rows >= shortest && a->batch_size > 0 &&
+  if (pl->n_splits == 1 && mixed_on_tile(a) && forced_splits <= 0 && tune_get(TUNE_ATTN_TILE_SPLITS, 0) <= 0 &&
+      pl->small_rows >= shortest && a->batch_size > 0 &&
       a->n_tokens <= (int64_t)(a->batch_size - 1) * a->max_q_len + pl->small_rows) {
     const int64_t want = std::min<int64_t>(1024 / ((int64_t)a->batch_size * a->n_kv_heads), 16);
     // (of the keys such a sequence sees: all of them, or those in front of its first row that the window leaves and its own)

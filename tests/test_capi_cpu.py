@@ -148,6 +148,14 @@ def test_single_rows_of_mixed_calls_obey_the_knobs():
             assert kernel(a) == want, least
     finally:
         L.slm_tuning_clear(b"SLM_ATTN_TILE_DECODE")
+    need = lambda a: L.slm_paged_kv_varlen_mha_workspace_bytes(C.byref(a))  # noqa: E731
+    a.sliding_window = -1
+    assert need(a) > 0
+    try:
+        assert L.slm_tuning_set(b"SLM_ATTN_SPLITS", 1) == 0   # a forced count is for every class of the call
+        assert need(a) == 0
+    finally:
+        L.slm_tuning_clear(b"SLM_ATTN_SPLITS")
 
 
 def test_split_kv_heuristic_host_side():
