@@ -671,6 +671,7 @@ struct AttnPlan {
   // the one-wave tile class of a mixed call whose other rows are not split: its KV splits (1: none either) and its longest
   // sequence, whose tokens have a row of partials each (AttnKParams::part_rows)
   int small_splits, small_rows;
+  bool singles_on_tile;  // q_len = 1 sequences go to the one-wave tiles
 };
 constexpr int ATTN_BAL_ALIGN = 64;
 
@@ -695,19 +696,34 @@ static bool mixed_on_tile(const slm_attn_args* a) {
          attn_tile_supported(a->head_dim) && tune_get(TUNE_ATTN_TILE, 1) != 0;
 }
 
-// The q_len = 1 sequences of a mixed call join the one-wave tiles.  The token kernel there has a workgroup per token of the
-// call, whatever the tokens are: eight single rows of 1.5 - 3 k context beside 120 verified sequences and 8 chunks took
-// it 223 us, one workgroup each, in front of the 192 us the tiles of the verified ones take; as eight more such tiles
-// they cost nothing that shows.  32 / 8 heads, n single rows of 4 k beside one prompt of 256, token -> tile: n = 1 358 -> 91 us,
-// 8 374 -> 94, 32 387 -> 139, 64 411 -> 235, 128 486 -> 410; of 512: 80 -> 47, 86 -> 51, 90 -> 61, 90 -> 68, 113 -> 95.  At 256
-// the token kernel has a workgroup on every CU and, with fewer than 8 heads on a KV head, the better rate (783 against
-// 814; 8 heads: 951 against 780).  SLM_ATTN_TILE_DECODE: minimum group size here too, 0 = never.
-static bool singles_on_tile(const slm_attn_args* a) {
+// The q_len = 1 sequences of a mixed call join the one-wave tiles where that is the shorter way through their keys.  The token
+// kernel there has a workgroup per token of the call, whatever the tokens are, and one that streams all KV heads of a long
+// history is most of the call: eight single rows of 1.5 - 3 k context beside 120 verified sequences and 8 chunks took it
+// 223 us, one workgroup each, in front of the 192 us the tiles of the verified ones take; as eight more such tiles they cost
+// nothing that shows.  token -> tile in us, n single rows beside one prompt of 256:
+//   fewer waves than SIMDs.  A token workgroup takes 20 us per MB of its share (`heads` KV heads), a tile's wave 1.2 us per 32
+//   keys of its split and some 10 more: the tiles where the bytes are the 1700-fold of a wave's keys and 540 KB.  4096 keys, 32 / 8
+//   heads of 128: n = 1 139 -> 79, 8 140 -> 81, 32 361 -> 111, 64 371 -> 204; 12 / 12 of 64 (three workgroups a token) 1 25 -> 31, 8 44 ->
+//   73, 32 112 -> 90, 64 148 -> 154; 4 / 1 of 128 8 28 -> 35, 64 42 -> 71, 128 77 -> 65.  Where the prompts are split both have their
+//   count, and the token kernel short shares: 3000 bytes a key (4 / 4 of 128, 2048 a key, four prompts of 512 and 12 k: 115 -> 178;
+//   32 / 8, 4096 a key: 352 -> 52).  From 8 query heads a KV head on the token kernel is bound by its arithmetic: 16 / 2 47 -> 34 and
+//   112 -> 88 (12 k), 8 / 1 51 -> 54 and, 60 rows, 102 -> 139; 32 / 1 130 -> 173, but 32 rows 214 -> 181.
+//   more waves.  The tiles (32 / 8: n = 128 429 -> 368, 160 486 -> 452; 12 / 12 of 64: 128 293 -> 265; 16 / 16 of 128: 96 733 -> 609), but
+//   for heads of 128 where the token kernel's workgroup takes up to eight KV heads at its best rate, from 1.5 waves a SIMD on: n =
+//   192 566 -> 618, 224 659 -> 688, 256 724 -> 740 (12 k: 1980 -> 2124; heads of 64: within 2 %).
+// How many single rows there are the host does not know: as many prompts of max_q_len as the tokens allow, and of the rest
+// at least those that no further token can belong to; beside verified sequences that is none, and a few single rows must not
+// pay a launch of their own.  SLM_ATTN_TILE_DECODE: minimum group size here too, 0 = never.
+static bool mixed_singles_on_tile(const slm_attn_args* a, int64_t seen, int heads, int token_splits, int tile_splits) {
   const int G = a->n_heads / a->n_kv_heads;
-  if (decode_on_tile(a)) return true;
   if (!mixed_on_tile(a) || G > 32) return false;
   if (tune_is_set(TUNE_ATTN_TILE_DECODE)) return tune_get(TUNE_ATTN_TILE_DECODE, 8) > 0 && G >= tune_get(TUNE_ATTN_TILE_DECODE, 8);
-  return G >= 8 || a->batch_size < 224;
+  const int64_t more = (int64_t)a->n_tokens - a->batch_size, prompts = more / (a->max_q_len - 1), rest = more % (a->max_q_len - 1);
+  const int64_t waves = (a->batch_size - prompts - rest) * a->n_kv_heads;
+  if (waves >= 1024) return G >= 8 || a->head_dim != 128 || a->n_kv_heads > 8 || waves < 1480;
+  const int64_t key = (int64_t)heads * a->head_dim * 4 * (G >= 16 && a->batch_size >= 24 ? 20 : G >= 8 ? 10 : 1);
+  if (token_splits > 1) return key >= (G >= 8 ? 6000 : 3000);
+  return seen * key >= seen / tile_splits * 1700 + 540000;
 }
 
 static int plan_attn(const slm_attn_args* a, AttnPlan* pl) {
@@ -903,19 +919,20 @@ static int plan_attn(const slm_attn_args* a, AttnPlan* pl) {
   // partials lie by sequence (at most 32 / G tokens of each: 1024 waves of 32 rows, 17 MB at head_dim 128, whatever the
   // prompts bring), and none are kept where the sizes leave room for no such sequence: all tokens but a short sequence's
   // are more than the others can bring.
-  pl->small_splits = 1;
   pl->small_rows = 32 / G;
-  const int64_t shortest = singles_on_tile(a) ? 1 : 2;
-  if (pl->n_splits == 1 && mixed_on_tile(a) && forced_splits <= 0 && tune_get(TUNE_ATTN_TILE_SPLITS, 0) <= 0 &&
-      pl->small_rows >= shortest && a->batch_size > 0 &&
-      a->n_tokens <= (int64_t)(a->batch_size - 1) * a->max_q_len + pl->small_rows) {
+  // (the keys such a sequence sees: all of them, or those in front of its first row that the window leaves and its own)
+  const int64_t seen = a->sliding_window < 0 ? a->max_kv_len
+                                             : std::min<int64_t>(a->max_kv_len, (int64_t)a->sliding_window + pl->small_rows);
+  auto own_splits = [&](int shortest) -> int {  // where the shortest sequence on the tiles has so many tokens
+    if (pl->n_splits != 1 || !mixed_on_tile(a) || forced_splits > 0 || tune_get(TUNE_ATTN_TILE_SPLITS, 0) > 0 ||
+        pl->small_rows < shortest || a->batch_size <= 0 ||
+        a->n_tokens > (int64_t)(a->batch_size - 1) * a->max_q_len + pl->small_rows)
+      return 1;
     const int64_t want = std::min<int64_t>(1024 / ((int64_t)a->batch_size * a->n_kv_heads), 16);
-    // (of the keys such a sequence sees: all of them, or those in front of its first row that the window leaves and its own)
-    const int64_t seen = a->sliding_window < 0 ? a->max_kv_len
-                                               : std::min<int64_t>(a->max_kv_len, (int64_t)a->sliding_window + pl->small_rows);
-    const int64_t by_len = seen / 512;
-    pl->small_splits = (int)std::max<int64_t>(std::min(want, by_len), 1);
-  }
+    return (int)std::max<int64_t>(std::min(want, seen / 512), 1);
+  };
+  pl->singles_on_tile = decode_on_tile(a) || mixed_singles_on_tile(a, seen, hpw * hgw, pl->n_splits, std::max(pl->n_splits, own_splits(1)));
+  pl->small_splits = own_splits(pl->singles_on_tile ? 1 : 2);
   pl->u = tune_get(TUNE_ATTN_U, pl->w == 2 ? 2 : 4);  // (two chunks: the same bytes in flight with half the rows)
   if (pl->u != 2 && pl->u != 4) pl->u = 4;
   pl->nt = tune_get(TUNE_ATTN_NT, a->max_q_len <= 1 ? 1 : 0) != 0;
@@ -1009,7 +1026,7 @@ SLM_API int32_t slm_paged_kv_varlen_mha_auto_splits(const slm_attn_args* a) {
 SLM_API int32_t slm_paged_kv_varlen_mha_decode_kernel(const slm_attn_args* a) {
   AttnPlan pl;
   if (plan_attn(a, &pl) != SLM_OK) return -1;
-  return singles_on_tile(a) ? 1 : 0;
+  return pl.singles_on_tile ? 1 : 0;
 }
 
 SLM_API size_t slm_paged_kv_varlen_mha_workspace_bytes(const slm_attn_args* a) {
@@ -1091,7 +1108,7 @@ SLM_API int slm_paged_kv_varlen_mha(const slm_attn_args* a, void* stream) {
     kp.ml_part = kp.o_part + (size_t)part_rows_of(a, pl) * a->n_heads * slots * a->head_dim;
   }
   bool tile_used = false;
-  const bool dec_tile = singles_on_tile(a);
+  const bool dec_tile = pl.singles_on_tile;
   const int first_tile_rows = dec_tile ? kp.group : kp.group + 1;  // smallest row count on the tile kernel
   // Every sequence brings exactly max_q_len tokens (the q lengths are bounded by max_q_len -- the grid contract
   // -- and add up to batch_size * max_q_len): ONE row class is populated, the launches of the others would only

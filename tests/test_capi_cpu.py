@@ -141,6 +141,7 @@ def test_single_rows_of_mixed_calls_obey_the_knobs():
     assert L.slm_tuning_clear(None) == 0
     kernel = lambda a: L.slm_paged_kv_varlen_mha_decode_kernel(C.byref(a))  # noqa: E731
     a = _attn(4, 1468, max_q=512, max_kv=1900)   # 4 query heads on a KV head
+    a.sliding_window = -1
     assert kernel(a) == 1
     try:
         for least, want in ((0, 0), (1, 1), (4, 1), (5, 0), (8, 0)):   # the least group on the tiles, 0 = none
@@ -149,13 +150,30 @@ def test_single_rows_of_mixed_calls_obey_the_knobs():
     finally:
         L.slm_tuning_clear(b"SLM_ATTN_TILE_DECODE")
     need = lambda a: L.slm_paged_kv_varlen_mha_workspace_bytes(C.byref(a))  # noqa: E731
-    a.sliding_window = -1
     assert need(a) > 0
     try:
         assert L.slm_tuning_set(b"SLM_ATTN_SPLITS", 1) == 0   # a forced count is for every class of the call
         assert need(a) == 0
     finally:
         L.slm_tuning_clear(b"SLM_ATTN_SPLITS")
+
+
+# heads, KV heads, head_dim, single rows, (prompts, their length), verified sequences of 5, keys, kernel of the single rows (1: tiles)
+@pytest.mark.parametrize("heads,kv_heads,d,n,prompts,verified,keys,want", [
+    (32, 8, 128, 8, (1, 256), 0, 4096, 1), (32, 8, 128, 8, (8, 256), 120, 3000, 1), (32, 8, 128, 1, (1, 1024), 0, 512, 1),
+    (32, 8, 128, 180, (1, 256), 0, 4096, 1), (32, 8, 128, 192, (1, 256), 0, 4096, 0), (32, 8, 128, 256, (4, 512), 0, 4096, 0),
+    (32, 8, 128, 8, (4, 512), 230, 4096, 1),     # many verified sequences: they do not make the few single rows many
+    (32, 8, 64, 256, (1, 256), 0, 4096, 1), (32, 32, 128, 256, (1, 256), 0, 4096, 1), (16, 16, 128, 96, (1, 256), 0, 4096, 1),
+    (12, 12, 64, 8, (1, 256), 0, 4096, 0), (12, 12, 64, 32, (1, 256), 0, 4096, 1), (12, 12, 64, 64, (1, 256), 0, 4096, 0),
+    (12, 12, 64, 128, (1, 256), 0, 4096, 1), (4, 1, 128, 8, (1, 256), 0, 512, 0), (4, 1, 128, 128, (1, 256), 0, 4096, 1),
+    (4, 4, 128, 1, (4, 512), 0, 12000, 0), (16, 2, 128, 8, (1, 256), 0, 512, 1), (8, 1, 128, 32, (1, 256), 0, 12000, 0),
+    (64, 1, 128, 8, (1, 256), 0, 4096, 0)])
+def test_kernel_of_the_single_rows_of_mixed_calls(heads, kv_heads, d, n, prompts, verified, keys, want):
+    assert _lib.lib().slm_tuning_clear(None) == 0
+    count, length = prompts
+    a = _attn(n + count + verified, n + count * length + 5 * verified, heads, kv_heads, d, max_q=length, max_kv=max(keys, length))
+    a.sliding_window = -1
+    assert _lib.lib().slm_paged_kv_varlen_mha_decode_kernel(C.byref(a)) == want
 
 
 def test_split_kv_heuristic_host_side():
