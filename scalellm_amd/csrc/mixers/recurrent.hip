@@ -41,6 +41,20 @@ __device__ __forceinline__ float conv_input(const slm_recurrent_args& a, const E
   }
   return silu_f32(acc);
 }
+// The ring entry that the input j tokens back of position p lies in (a convolution of at most 4 taps), or -1: the step's own row.
+// Inputs there are not (older than the taps, or than the sequence) are the own row again and left out of the sum, so that no
+// load reads the entry another head of the launch may be writing.
+constexpr __host__ __device__ int step_entry(int j, int p, int taps) {
+  return j == 0 || j > taps - 1 || j > p ? -1 : (p - j) % taps;
+}
+constexpr bool step_reads_no_kept_entry() {
+  for (int taps = 1; taps <= 4; ++taps)
+    for (int p = 0; p < 12; ++p)
+      for (int j = 0; j < 4; ++j)
+        if (step_entry(j, p, taps) == p % taps) return false;
+  return true;
+}
+static_assert(step_reads_no_kept_entry(), "the entry of the step's own position is written while the others are read");
 // the same for the one row of a step, convolutions of at most 4 taps: every load at once
 template <typename E>
 __device__ __forceinline__ float conv_step4(const slm_recurrent_args& a, const E* ring, int64_t row, int p, int c) {
@@ -49,10 +63,11 @@ __device__ __forceinline__ float conv_step4(const slm_recurrent_args& a, const E
   const int64_t col = c < qk ? a.off_q + c : c < 2 * qk ? a.off_k + (c - qk) : a.off_v + (c - 2 * qk);
   float w[4], x[4];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {   // (taps there are not, and positions before 0: the last there is, times zero)
-    const int back = min(j, most);
-    w[j] = a.conv_w[(int64_t)(a.taps - 1 - back) * ch + c];
-    x[j] = j == 0 ? to_f32(reinterpret_cast<const E*>(a.proj)[row * a.ld_proj + col]) : to_f32(ring[(int64_t)((p - back) % a.taps) * ch + c]);
+  for (int j = 0; j < 4; ++j) {
+    const int entry = step_entry(j, p, a.taps);
+    const E* own = reinterpret_cast<const E*>(a.proj) + row * a.ld_proj + col;
+    w[j] = a.conv_w[(int64_t)(a.taps - 1 - min(j, most)) * ch + c];
+    x[j] = to_f32(*(entry < 0 ? own : ring + (int64_t)entry * ch + c));
   }
   float acc = 0.f;
 #pragma unroll
