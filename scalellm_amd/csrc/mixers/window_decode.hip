@@ -4,7 +4,7 @@
 // Work item: one workgroup = (row, 1 / 2 / 4 neighbouring kv heads, block of 16 query heads, split of the visible keys); its four
 // waves are shared out over the kv heads, those of one head take tiles of 32 keys in turn, and none meet before the end.
 // What a cache row holds for neighbouring heads is neighbouring memory: read by one CU at about the same time it comes as
-// 512 or 1024 bytes a row instead of 256, past the caches (read once).  16 / 8 heads of 128, 128 rows of 4096 keys:
+// 512 or 1024 bytes a row instead of 256, a large stream past the caches (read once).  16 / 8 heads of 128, 128 rows of 4096 keys:
 // 398 us with a head to a workgroup (5.4 TB/s; 256 to 1024 workgroups, with non-temporal loads or without), 355 with two, 350
 // with four (6.1 TB/s); a barrier a tile between the heads 389.
 //   S[32 keys x 16 heads]      A = key rows straight from the cache (16 bytes per lane), B = the query heads in registers
@@ -35,7 +35,15 @@ __device__ __forceinline__ float over_groups(float v, bool take_max) {
   return take_max ? fmaxf(v, y) : v + y;
 }
 
-template <int DQ, int VP>
+// 16 bytes of the cache; ONCE: past the caches' replacement
+template <bool ONCE>
+__device__ __forceinline__ u32x4 load_once(const bf16* p) {
+  const u32x4* q = reinterpret_cast<const u32x4*>(p);
+  if constexpr (ONCE) return __builtin_nontemporal_load(q);
+  else return *q;
+}
+
+template <int DQ, int VP, bool ONCE>
 __global__ void __launch_bounds__(256) window_decode_kernel(const WindowDecodeK p) {
   constexpr int KT = 32, QS = DQ / 32, NT = VP / 16;
   constexpr int VLS = VP * 2 + 16;                          // bytes of a value row in LDS
@@ -85,12 +93,12 @@ __global__ void __launch_bounds__(256) window_decode_kernel(const WindowDecodeK 
     for (int n = 0; n < 2; ++n) {
       const bf16* k = kc + (int64_t)__shfl(slot, 16 * n + l16, 64) * k_w;
 #pragma unroll
-      for (int s = 0; s < QS; ++s) kf[n][s] = __builtin_bit_cast(bf16x8_t, __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(k + 32 * s)));
+      for (int s = 0; s < QS; ++s) kf[n][s] = __builtin_bit_cast(bf16x8_t, load_once<ONCE>(k + 32 * s));
     }
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
       const int idx = lane + 64 * i;
-      vf[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(vc + (int64_t)__shfl(slot, idx / VCH, 64) * v_w + 8 * (idx % VCH)));
+      vf[i] = load_once<ONCE>(vc + (int64_t)__shfl(slot, idx / VCH, 64) * v_w + 8 * (idx % VCH));
     }
   };
   f32x4 o[NT];
@@ -237,11 +245,20 @@ static int hw_shift(const slm_window_attn_args& a) {
   const int64_t pairs = a.rows * a.kv_heads;
   return a.kv_heads % 4 == 0 && pairs >= 512 ? 2 : a.kv_heads % 2 == 0 && pairs >= 64 ? 1 : 0;
 }
+static int64_t visible_keys(const slm_window_attn_args& a) {
+  const int64_t seen = (int64_t)a.window + (a.keep_first > 0 ? a.keep_first : 0);
+  return a.window > 0 && a.max_kv_len > seen ? seen : a.max_kv_len;
+}
+// Past the caches' replacement where one workgroup reads a row and the stream is far beyond the L2s (with / without, us, 128 columns of
+// keys and of values: 16 / 8 heads, 8 rows x 1000 keys, 33 MB 18.9 / 17.8, x 2000 24.8 / 24.5, x 2500 25.7 / 27.9, x 4096 35.4 / 37.7; 32 x 4096
+// 96 / 104; several blocks of heads on a kv head, 128 / 1, 32 x 4096 90 / 59; 64 / 2, 128 x 4096 180 / 163).
+static bool reads_once(const slm_window_attn_args& a) {
+  return head_blocks(a) == 1 && a.rows * visible_keys(a) * a.kv_heads * (a.d_pad + a.v_pad) * 2 >= (64ll << 20);
+}
 // splits: about two workgroups per CU, at least 128 keys (a tile per wave) each
 static int split_count(const slm_window_attn_args& a) {
   if (a.n_splits > 0) return a.n_splits < 64 ? a.n_splits : 64;
-  int64_t keys = a.max_kv_len;
-  if (a.window > 0 && keys > (int64_t)a.window + (a.keep_first > 0 ? a.keep_first : 0)) keys = (int64_t)a.window + (a.keep_first > 0 ? a.keep_first : 0);
+  const int64_t keys = visible_keys(a);
   const int64_t wgs = a.rows * (a.kv_heads >> hw_shift(a)) * head_blocks(a);
   const int64_t want = (512 + wgs - 1) / wgs, most = keys / 128;
   const int64_t n = want < most ? want : most;
@@ -260,7 +277,8 @@ size_t window_decode_workspace(const slm_window_attn_args& a) {
 template <int DQ, int VP>
 static void wd_launch(const WindowDecodeK& p, hipStream_t st) {
   const int64_t grid = p.a.rows * (p.a.kv_heads >> p.hw_shift) * p.head_blocks * p.n_splits;
-  window_decode_kernel<DQ, VP><<<dim3((unsigned)grid), dim3(256), 0, st>>>(p);
+  if (reads_once(p.a)) window_decode_kernel<DQ, VP, true><<<dim3((unsigned)grid), dim3(256), 0, st>>>(p);
+  else window_decode_kernel<DQ, VP, false><<<dim3((unsigned)grid), dim3(256), 0, st>>>(p);
 }
 template <int DQ>
 static void wd_v(const WindowDecodeK& p, hipStream_t st) {
