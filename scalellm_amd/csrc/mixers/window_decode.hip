@@ -12,6 +12,7 @@
 //                              V^T out of a wave-private row-major LDS tile by the transpose read
 // A tile's keys and values are loaded while the tile before is consumed, its slots one tile further ahead.  The waves'
 // sums meet in LDS, splits in a second launch, where the sink enters.
+#include <algorithm>
 #include <type_traits>
 
 #include "window_common.h"
@@ -250,12 +251,6 @@ __global__ void __launch_bounds__(256) window_combine_kernel(const WindowDecodeK
 }
 
 static int head_blocks(const slm_window_attn_args& a) { return (a.heads / a.kv_heads + 15) / 16; }
-// kv heads of a workgroup: as many as leave enough rows to go round (2 / 4 heads against one, 4096 keys: 8 rows x 8 heads 36.4
-// us / 38.5 against 36.2, 1 row 17.6 / 23 against 14.7)
-static int hw_shift(const slm_window_attn_args& a) {
-  const int64_t pairs = a.rows * a.kv_heads;
-  return a.kv_heads % 4 == 0 && pairs >= 512 ? 2 : a.kv_heads % 2 == 0 && pairs >= 64 ? 1 : 0;
-}
 static int64_t visible_keys(const slm_window_attn_args& a) {
   const int64_t seen = (int64_t)a.window + (a.keep_first > 0 ? a.keep_first : 0);
   return a.window > 0 && a.max_kv_len > seen ? seen : a.max_kv_len;
@@ -265,6 +260,14 @@ static int64_t visible_keys(const slm_window_attn_args& a) {
 // 96 / 104; several blocks of heads on a kv head, 128 / 1, 32 x 4096 90 / 59; 64 / 2, 128 x 4096 180 / 163).
 static bool reads_once(const slm_window_attn_args& a) {
   return head_blocks(a) == 1 && a.rows * visible_keys(a) * a.kv_heads * (a.d_pad + a.v_pad) * 2 >= (64ll << 20);
+}
+// kv heads of a workgroup: as many as leave enough rows to go round (2 / 4 heads against one, 4096 keys: 8 rows x 8 heads 36.4
+// us / 38.5 against 36.2, 1 row 17.6 / 23 against 14.7; four where
+// splits of at least 128 keys leave under 400 workgroups: 64 rows x 500 keys 38.3 against 32.6 with two, 128 x 130 20.7 / 19.3, but 200 x
+// 250, 400 of them, 45.2 / 47.7)
+static int hw_shift(const slm_window_attn_args& a) {
+  const int64_t pairs = a.rows * a.kv_heads, most = std::max<int64_t>(visible_keys(a) / 128, 1);
+  return a.kv_heads % 4 == 0 && pairs >= 512 && pairs / 4 * most >= 400 ? 2 : a.kv_heads % 2 == 0 && pairs >= 64 ? 1 : 0;
 }
 // splits: about two workgroups per CU, at least 128 keys (a tile per wave) each
 static int split_count(const slm_window_attn_args& a) {

@@ -255,7 +255,8 @@ def test_silu_glu(rows, dtype):
 # kv heads, more than 16 query heads on one, ranges of less than a tile, of splits that get no tile, windows with kept tokens
 @pytest.mark.parametrize("rows,heads,kv_heads,dim,vdim,longest,window,keep", [
     (3, 6, 3, 64, 128, 900, 0, 0), (40, 8, 2, 128, 128, 300, 100, 7), (130, 16, 4, 96, 64, 200, 0, 0), (9, 160, 8, 128, 128, 700, 0, 0),
-    (130, 20, 5, 64, 64, 65, 33, 40), (64, 8, 8, 128, 128, 1500, 1000, 16), (1, 8, 8, 128, 128, 4000, 0, 0)])
+    (130, 20, 5, 64, 64, 65, 33, 40), (64, 8, 8, 128, 128, 1500, 1000, 16), (1, 8, 8, 128, 128, 4000, 0, 0),
+    (260, 8, 8, 64, 64, 200, 0, 0)])   # (four heads, one split)
 def test_window_attention_of_single_rows(rows, heads, kv_heads, dim, vdim, longest, window, keep):
     from scalellm_amd import mixer_kernels as mk
     from scalellm_amd.decode import make_batch_inputs
