@@ -485,17 +485,20 @@ __global__ void __launch_bounds__(256) latent_attn_any_kernel(const LatentAttnK 
   }
 }
 
-// Head blocks of 16 per workgroup (the scores of four do not fit beside the tiles of the widest latent).  Few rows leave fewer
-// splits, and fewer partials behind them, with a block to a workgroup: the blocks of a split share an L2 (32 heads, 4096 keys: 1 row
-// 19.2 -> 16.1 us, 8 rows 26.9 -> 24.9; 32 rows, 2000 - 4001 keys 46 -> 50, and two
-// blocks take 42 since their waves share the soft-max).
-static int la_mh(const slm_latent_attn_args& a) {
-  if (a.rows < 24 && a.heads <= 32) return 1;
-  return a.heads > 32 && a.c_pad < 512 ? 4 : a.heads > 16 ? 2 : 1;
-}
 static int64_t la_keys(const slm_latent_attn_args& a) {
   const int64_t len = a.max_kv_len > 0 ? a.max_kv_len : 1;
   return a.window > 0 && a.window < len ? a.window : len;
+}
+// Head blocks of 16 per workgroup (the scores of four do not fit beside the tiles of the widest latent).  Few rows leave fewer
+// splits, and fewer partials behind them, with a block to a workgroup: the blocks of a split share an L2.  It reads the keys once a
+// block, though, which shows from a number of keys on that the width sets (one block / two, us; latent 512, 32 heads: 1 row x 4096 16.2 /
+// 18.8, 8 x 4096 22.4 / 25.8, 20 x 4096 36.7 / 36.7, 16 x 12000 61 / 53, 23 x 32000 212 / 145; 256: 8 x 4096 19.3 / 19.7, 12 x 4096 23.4 / 22.2; 128,
+// 24 heads: 8 x 1500 11.0 / 12.1, 16 x 1500 14.1 / 12.9, 16 x 12000 47 / 31; 64: 12 x 4096 15.6 / 15.8, 16 x 12000 29.6 / 26; 32 rows, 2000 -
+// 4001 keys, latent 512: 50 / 42).
+static int la_mh(const slm_latent_attn_args& a) {
+  const int64_t few = a.c_pad >= 512 ? 90000 : a.c_pad == 256 ? 40000 : a.c_pad == 128 ? 18000 : 48000;
+  if (a.rows < 24 && a.heads <= 32 && a.rows * la_keys(a) <= few) return 1;
+  return a.heads > 32 && a.c_pad < 512 ? 4 : a.heads > 16 ? 2 : 1;
 }
 static bool la_mfma(int c_pad, int r_pad, int dtype) {
   return dtype == SLM_BF16 && (c_pad == 64 || c_pad == 128 || c_pad == 256 || c_pad == 512) && (r_pad == 32 || r_pad == 64);

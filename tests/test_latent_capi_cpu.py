@@ -94,3 +94,15 @@ def test_split_plan_sizes_its_workspace():
     assert L.slm_latent_attn_workspace_bytes(C.byref(b)) == 0
     b.rows, b.dtype = 2, _lib.SLM_F32
     assert L.slm_latent_attn_workspace_bytes(C.byref(b)) == 0
+
+
+@pytest.mark.parametrize("c_pad,rows,keys,blocks", [(512, 16, 4096, 1), (512, 16, 12000, 2), (512, 24, 500, 2), (512, 4, 12000, 1), (256, 8, 4096, 1),
+                                                    (256, 16, 4096, 2), (128, 8, 1500, 1), (128, 16, 1500, 2), (64, 8, 4096, 1), (64, 16, 12000, 2)])
+def test_head_blocks_of_few_rows_follow_the_keys(c_pad, rows, keys, blocks):
+    """32 heads as two workgroups of 16 or one of both, told from the splits: 256 workgroups (512 of the narrowest latent), a tile
+    of 32 keys at least each."""
+    b = _lib.LatentAttnArgs()
+    b.rows, b.batch, b.heads, b.c_pad, b.r_pad, b.block_size, b.dtype, b.max_kv_len = rows, rows, 32, c_pad, 64, 64, _lib.SLM_BF16, keys
+    got = _lib.latent_lib().slm_latent_attn_workspace_bytes(C.byref(b)) // (rows * 32 * (c_pad + 2) * 4)
+    splits = lambda n: (512 if c_pad == 64 else 256) // (rows * (2 // n))  # noqa: E731
+    assert splits(1) != splits(2) and got == min(splits(blocks), (keys + 31) // 32, 64), got

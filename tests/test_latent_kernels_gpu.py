@@ -335,6 +335,28 @@ def test_latent_attention_of_whole_and_cut_tiles(c_pad, heads, block):
             _close(out, want, dt, b16=1.5e-2)
 
 
+@pytest.mark.parametrize("heads,lens", [(16, [4096] * 20 + [4000, 33, 1, 4095, 4096]), (32, [4096] * 23 + [31, 2000]), (17, [4096] * 22 + [4064, 1])])
+def test_latent_attention_of_a_stream_past_the_caches(heads, lens):
+    """100 MB of keys and more that one workgroup reads: loads past the caches' replacement, with splits and without, whole tiles and
+    cut ones; 17 and 32 heads also as few rows of long histories, two blocks to a workgroup."""
+    from scalellm_amd.decode import make_batch_inputs
+    lk, c, r, block = _lk(), 512, 64, 64
+    _, positions, params, n_blocks = make_batch_inputs([1] * len(lens), lens, block, DEV, seed=3)
+    assert len(lens) * max(lens) * (c + r) * 2 >= 100 << 20
+    q, cache = _rnd(5, len(lens), heads, c + r, dtype=torch.bfloat16), _rnd(6, n_blocks * block, c + r, dtype=torch.bfloat16)
+    want = torch.empty(len(lens), heads, c, dtype=torch.float64, device=DEV)
+    for i, n in enumerate(lens):
+        pos = torch.arange(n, device=DEV)
+        rows = cache[params.block_tables.long()[int(params.cu_block_lens[i]) + pos // block] + pos % block].double()
+        want[i] = torch.softmax(q[i].double() @ rows.t() * (c + r) ** -0.5, -1) @ rows[:, :c]
+    for kw in (dict(), dict(n_splits=1), dict(n_splits=3)):
+        out = torch.full((len(lens), heads, c), float("nan"), dtype=torch.bfloat16, device=DEV)
+        lk.latent_attention(q, cache, out, positions, params.q_cu_seq_lens, params.block_tables, params.cu_block_lens, block_size=block,
+                            window=0, scale=(c + r) ** -0.5, max_kv_len=max(lens), **kw)
+        # (16-bit weights and results: 2^-9 of a value each; of a row's own norm, which 4096 averaged keys leave small)
+        assert ((out.double() - want).norm(dim=-1) / want.norm(dim=-1)).max() < 1.5e-2
+
+
 # ---- prompt portions ---------------------------------------------------------------------------
 @pytest.mark.parametrize("q_dim,r_pad,v_pad", [(32, 32, 32), (32, 64, 64), (64, 64, 128), (128, 32, 64), (128, 64, 128), (192, 64, 64)])
 @pytest.mark.parametrize("window", [0, 1, 40, 64, 129, 300])
