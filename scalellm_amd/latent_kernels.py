@@ -160,7 +160,7 @@ def slab_rows(layout: Optional[torch.Tensor]) -> int:
 
 def _stream_args(x, w, layout, M, N, K, rows) -> "Optional[_lib.LinearArgs]":
     """Arguments of slm_linear_stream, or None where it does not serve the call."""
-    if layout is None or M > rows or x.stride(0) % 8 or x.data_ptr() % 16:
+    if layout is None or M > rows or x.stride(0) < K or x.stride(0) % 8 or x.data_ptr() % 16:   # (rows that overlap: the vendor's)
         return None
     _need(layout.is_contiguous() and layout.dtype == x.dtype and layout.numel() == (N + 63) // 64 * 64 * K, "linear: streamed layout of w")
     a = _linear_args(x, w, M, N, K)

@@ -119,6 +119,20 @@ def test_streamed_products(M, N, K):
         _close(out, ref.clamped_glu(want[:, :N // 2], want[:, N // 2:], 0.6), torch.bfloat16, b16=2e-2)
 
 
+@pytest.mark.parametrize("M", [33, 64, 128])
+def test_products_of_one_row_many_times(M):
+    """Rows without a stride of their own (an expanded one), and rows that overlap: above 32 they are the vendor product's."""
+    lk, N, K = _lk(), 192, 128
+    w = _rnd(2, N, K, dtype=torch.bfloat16, std=K ** -0.5)
+    layout, glu = lk.stream_layout(w), lk.stream_layout(w, glu=True)
+    for x in (_rnd(1, 1, K, dtype=torch.bfloat16).expand(M, K), _rnd(1, 8 * M + K, dtype=torch.bfloat16).as_strided((M, K), (8, 1))):
+        want = _f64(x) @ _f64(w).T
+        _close(lk.linear(x, w, layout=layout), want, torch.bfloat16)
+        out = torch.zeros(M, N // 2, dtype=torch.bfloat16, device=DEV)
+        lk.linear_glu(x, w, out, 0.6, layout=glu)
+        _close(out, ref.clamped_glu(want[:, :N // 2], want[:, N // 2:], 0.6), torch.bfloat16, b16=2e-2)
+
+
 def test_streamed_weight_layout():
     lk, N, K = _lk(), 112, 192
     w = torch.arange(N * K, device=DEV).remainder(251).to(torch.bfloat16).view(N, K)
