@@ -149,7 +149,8 @@ def stream_layout(w: torch.Tensor, glu: bool = False) -> Optional[torch.Tensor]:
     if w.dtype != torch.bfloat16 or K % 64 or N % 16 or (glu and N % 64) or not w.is_cuda or not w.is_contiguous() or w.data_ptr() % 16:
         return None
     out = torch.empty((N + 63) // 64, K // 64, 4, 2, 64, 8, dtype=w.dtype, device=w.device)
-    latent_check(_lib.latent_lib().slm_stream_layout(_p(out), _p(w), N, K, int(glu), _stream()), "slm_stream_layout")
+    with torch.cuda.device(w.device):   # (a model may be built before its device is made the current one)
+        latent_check(_lib.latent_lib().slm_stream_layout(_p(out), _p(w), N, K, int(glu), _stream()), "slm_stream_layout")
     return out
 
 

@@ -106,3 +106,31 @@ def test_head_blocks_of_few_rows_follow_the_keys(c_pad, rows, keys, blocks):
     got = _lib.latent_lib().slm_latent_attn_workspace_bytes(C.byref(b)) // (rows * 32 * (c_pad + 2) * 4)
     splits = lambda n: (512 if c_pad == 64 else 256) // (rows * (2 // n))  # noqa: E731
     assert splits(1) != splits(2) and got == min(splits(blocks), (keys + 31) // 32, 64), got
+
+
+def test_streamed_layout_is_made_on_the_device_of_its_weight(monkeypatch):
+    """The current device may be another one while a model is built: launched there, the kernel would read foreign memory."""
+    import contextlib
+    import types
+    import torch
+    from scalellm_amd import latent_kernels as lk
+    current, made_on = ["cuda:0"], []
+
+    @contextlib.contextmanager
+    def device(d):
+        old, current[0] = current[0], str(d)
+        yield
+        current[0] = old
+
+    def layout(*args):
+        made_on.append(current[0])
+        return 0
+    monkeypatch.setattr(torch.cuda, "device", device)
+    monkeypatch.setattr(lk, "_stream", lambda: 0)
+    monkeypatch.setattr(lk, "_p", lambda t: 4096)
+    monkeypatch.setattr(lk._lib, "latent_lib", lambda: types.SimpleNamespace(slm_stream_layout=layout))
+    monkeypatch.setattr(torch, "empty", lambda *a, **k: object())
+    w = types.SimpleNamespace(shape=(64, 64), dtype=torch.bfloat16, is_cuda=True, is_contiguous=lambda: True, data_ptr=lambda: 4096,
+                              device="cuda:3")
+    lk.stream_layout(w)
+    assert made_on == ["cuda:3"]
