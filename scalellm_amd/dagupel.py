@@ -133,6 +133,8 @@ class DagupelStep:
             self.caches.append(weights[j].attn.new_cache(limits.n_blocks, limits.block_size))
         # portions go to their own kernels where every layer has them (the step's rows are ordered once)
         self.portion_min = LatentAttention.PORTION_MIN if all(L.attn.portions_ok for L in self.layers) else None
+        own = list({id(L): L for L in self.layers}.values())
+        self._copied = lk.copied_weights([self.l_table] + [t for L in own for t in (L.attn.l_in, L.attn.l_o) + ((L.mlp.l_gate_up, L.mlp.l_down) if L.mlp else ())])
         # called with (layer run, residual stream) after every layer, when set
         self.on_layer: Optional[Callable[[int, torch.Tensor], None]] = None
 
@@ -141,6 +143,10 @@ class DagupelStep:
         model = cls(DagupelConfig.parse(config), ckpt, limits)
         ckpt.finish()
         return model
+
+    def weights_version(self) -> int:
+        """Changes when a weight that products of few rows read a copy of is changed in place."""
+        return sum(w._version for w in self._copied)
 
     def reserve_workspaces(self, n_tokens: int) -> None:
         """Size the attention scratch for decode batches of up to n_tokens rows, before graphs are captured."""

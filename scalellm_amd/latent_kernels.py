@@ -6,7 +6,7 @@ there is no fallback: a missing library or a CPU tensor raises.
 from __future__ import annotations
 
 import ctypes as C
-from typing import Optional, Tuple
+from typing import List, Optional, Tuple
 
 import torch
 
@@ -144,14 +144,27 @@ def stream_layout(w: torch.Tensor, glu: bool = False) -> Optional[torch.Tensor]:
     """W [N, K] once more in the order slm_linear_stream reads it (include/slm_latent.h), made at load: what products of
     few rows run on.  The row-major tensor stays for products of many.  glu: W = [gate | up].  None where that kernel has
     no form (32-bit weights, gate halves that are no multiple of 32) and for weights that no kernel reads yet (a model
-    loaded on the host)."""
+    loaded on the host).  It is a copy of w as it is now: once w is changed in place (its version counter tells; inference
+    tensors have none and are not followed) products are w's own again, until a new layout is made."""
     N, K = w.shape
     if w.dtype != torch.bfloat16 or K % 64 or N % 16 or (glu and N % 64) or not w.is_cuda or not w.is_contiguous() or w.data_ptr() % 16:
         return None
     out = torch.empty((N + 63) // 64, K // 64, 4, 2, 64, 8, dtype=w.dtype, device=w.device)
     with torch.cuda.device(w.device):   # (a model may be built before its device is made the current one)
         latent_check(_lib.latent_lib().slm_stream_layout(_p(out), _p(w), N, K, int(glu), _stream()), "slm_stream_layout")
+    if not w.is_inference():
+        out.copy_of, out.copy_version = w, w._version
     return out
+
+
+def layout_is_current(layout: torch.Tensor, w: torch.Tensor) -> bool:
+    of = getattr(layout, "copy_of", None)
+    return of is None or (of.data_ptr() == w.data_ptr() and of._version == layout.copy_version)
+
+
+def copied_weights(layouts) -> List[torch.Tensor]:
+    """The weights behind layouts (None among them) that can be followed."""
+    return [t.copy_of for t in layouts if hasattr(t, "copy_of")]
 
 
 def slab_rows(layout: Optional[torch.Tensor]) -> int:
@@ -162,6 +175,8 @@ def slab_rows(layout: Optional[torch.Tensor]) -> int:
 def _stream_args(x, w, layout, M, N, K, rows) -> "Optional[_lib.LinearArgs]":
     """Arguments of slm_linear_stream, or None where it does not serve the call."""
     if layout is None or M > rows or x.stride(0) < K or x.stride(0) % 8 or x.data_ptr() % 16:   # (rows that overlap: the vendor's)
+        return None
+    if not layout_is_current(layout, w):
         return None
     _need(layout.is_contiguous() and layout.dtype == x.dtype and layout.numel() == (N + 63) // 64 * 64 * K, "linear: streamed layout of w")
     a = _linear_args(x, w, M, N, K)

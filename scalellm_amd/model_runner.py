@@ -69,6 +69,7 @@ class _Graph:
         # variant -> (graph, output); the key None is the reference's single graph
         self.variants: Dict[object, tuple] = {}
         self.last_variant = None
+        self.weights_version = None   # of the model when it was captured
 
     @property
     def graph(self) -> Optional[torch.cuda.CUDAGraph]:   # (the first captured variant: tests, tools)
@@ -85,6 +86,7 @@ class _Graph:
 
     def capture(self, fn: Callable) -> None:
         model = self.runner.model
+        self.weights_version = self.runner.weights_version()
         keys = [None]
         if all(hasattr(model, a) for a in ("graph_variants", "graph_variant_for", "graph_variant")):
             keys = list(model.graph_variants(self.n_tokens, self.batch_size, self.params.q_max_seq_len))
@@ -180,6 +182,11 @@ class ModelRunner:
             n_states = getattr(model, "n_states", 0)
             self.state_slots = torch.arange(mb, **i32) % n_states if n_states else None
 
+    def weights_version(self):
+        """Of a model that keeps copies of weights for its graphs' kernels (None: it keeps none)."""
+        version = getattr(self.model, "weights_version", None)
+        return version() if version is not None else None
+
     def _run(self, tokens, positions, params):
         return self.model.forward(tokens, positions, params, **self.forward_kwargs)
 
@@ -202,8 +209,9 @@ class ModelRunner:
         # (a graph gives the last row of every sequence: other rows are an eager step's)
         if g is not None and getattr(params, "logit_rows", None) is None:
             nd = self.options.num_decoding_tokens
+            # (weights changed in place since the capture: its kernels may read copies of them, so steps are eager)
             if (params.kv_max_seq_len <= self.options.cuda_graph_max_seq_len and
-                    params.q_max_seq_len == nd and tokens.numel() == bs * nd):
+                    params.q_max_seq_len == nd and tokens.numel() == bs * nd and g.weights_version == self.weights_version()):
                 self.num_graph_replayed += 1
                 return g.replay(tokens, positions, params)
         self.num_eager += 1

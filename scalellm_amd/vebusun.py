@@ -136,6 +136,7 @@ class VebusunStep:
             weights.append(L)
         self.layers = [weights[i] for i in c.runs]
         self.caches = [L.mixer.new_cache(limits) for L in self.layers]
+        self._copied = lk.copied_weights([self.l_head] + [t for L in weights for t in (L.mixer.l_in, L.mixer.l_o) + ((L.mlp.l_gate_up, L.mlp.l_down) if L.mlp else ())])
         # called with (layer run, residual stream) after every layer, when set
         self.on_layer: Optional[Callable[[int, torch.Tensor], None]] = None
 
@@ -167,6 +168,10 @@ class VebusunStep:
         model = cls(VebusunConfig.parse(config), ckpt, limits)
         ckpt.finish()
         return model
+
+    def weights_version(self) -> int:
+        """Changes when a weight that products of few rows read a copy of is changed in place."""
+        return sum(w._version for w in self._copied)
 
     def reserve_workspaces(self, n_tokens: int) -> None:
         """Size the attention scratch for decode batches of up to n_tokens rows, before graphs are captured."""

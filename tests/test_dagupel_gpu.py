@@ -257,6 +257,35 @@ def test_graph_replays_of_a_batch_the_vendor_products_serve():
     assert row_errors(outs[1], outs[0].astype(np.float64)).max() < 1e-2
 
 
+def test_steps_follow_weights_changed_in_place():
+    """Captured steps read copies of the weights: after a change they run eagerly, until the graph is captured again."""
+    cfg, t, tokens, _ = _model("wide")
+    rows = []
+    for graphs in ([], [1]):
+        engine = _engine(cfg, t, torch.bfloat16, n_blocks=40, block_size=16, graph_batch_sizes=graphs, graph_max_seq_len=256)
+        engine.capture_graphs()
+        s, got = _seq("a", tokens), []
+        _run(engine, [(s, 20)])
+
+        def step():
+            got.append(engine.run_entries([(s, 1)])[1].float().cpu().numpy())
+        step()
+        with torch.no_grad():
+            for L in engine.runner.model.layers:
+                L.attn.w_in.mul_(0.5)
+                if L.mlp:
+                    L.mlp.w_down.mul_(-1.0)
+        step()
+        step()
+        assert engine.runner.num_graph_replayed == (1 if graphs else 0)
+        rows.append(np.concatenate(got))
+    assert row_errors(rows[1], rows[0].astype(np.float64)).max() < 1e-2
+    assert row_errors(rows[0][1:2], rows[0][:1].astype(np.float64)).max() > 0.1   # (the change is seen)
+    engine.capture_graphs()
+    step()
+    assert engine.runner.num_graph_replayed == 2
+
+
 def test_preempted_sequences_start_over():
     cfg, t, _, _ = _model("tiny")
     from scalellm_amd.sampling import SamplingParams

@@ -131,6 +131,6 @@ def test_streamed_layout_is_made_on_the_device_of_its_weight(monkeypatch):
     monkeypatch.setattr(lk._lib, "latent_lib", lambda: types.SimpleNamespace(slm_stream_layout=layout))
     monkeypatch.setattr(torch, "empty", lambda *a, **k: object())
     w = types.SimpleNamespace(shape=(64, 64), dtype=torch.bfloat16, is_cuda=True, is_contiguous=lambda: True, data_ptr=lambda: 4096,
-                              device="cuda:3")
+                              device="cuda:3", is_inference=lambda: True)
     lk.stream_layout(w)
     assert made_on == ["cuda:3"]

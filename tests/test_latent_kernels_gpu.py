@@ -133,6 +133,27 @@ def test_products_of_one_row_many_times(M):
         _close(out, ref.clamped_glu(want[:, :N // 2], want[:, N // 2:], 0.6), torch.bfloat16, b16=2e-2)
 
 
+@pytest.mark.parametrize("M", [1, 20, 100])
+def test_products_follow_weights_changed_in_place(M):
+    lk, N, K = _lk(), 192, 128
+    x, w = _rnd(1, M, K, dtype=torch.bfloat16), _rnd(2, N, K, dtype=torch.bfloat16, std=K ** -0.5)
+    layout, glu = lk.stream_layout(w), lk.stream_layout(w, glu=True)
+
+    def check(layout, glu):
+        want, out = _f64(x) @ _f64(w).T, torch.zeros(M, N // 2, dtype=torch.bfloat16, device=DEV)
+        _close(lk.linear(x, w, layout=layout), want, torch.bfloat16)
+        _close(lk.linear_f32(x, w, 1.0, layout), want, torch.float32, f32=1e-5)
+        _close(lk.linear_slabs(x, w, layout).t.sum(0), want, torch.float32, f32=1e-5)
+        lk.linear_glu(x, w, out, 0.6, layout=glu)
+        _close(out, ref.clamped_glu(want[:, :N // 2], want[:, N // 2:], 0.6), torch.bfloat16, b16=2e-2)
+    check(layout, glu)
+    w[N // 2:].mul_(-2.0)
+    check(layout, glu)
+    check(lk.stream_layout(w), lk.stream_layout(w, glu=True))
+    w = w + 1.0   # (another tensor)
+    check(layout, glu)
+
+
 def test_streamed_weight_layout():
     lk, N, K = _lk(), 112, 192
     w = torch.arange(N * K, device=DEV).remainder(251).to(torch.bfloat16).view(N, K)
