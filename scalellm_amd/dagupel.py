@@ -86,6 +86,7 @@ class _LayerWeights:
 @register_model("Dagupel")
 class DagupelStep:
     libraries = ("latent",)
+    STREAMED = (("l_table", "table", False),)
 
     def __init__(self, config: DagupelConfig, ckpt: Checkpoint, limits: ModelLimits):
         c = self.config = config
@@ -101,7 +102,6 @@ class DagupelStep:
         # embedding and vocabulary projection are one table: zero padded to the product's tiles
         self.table = torch.zeros(round_up(c.vocab, 16), self.k_width, dtype=dt, device=dev)
         self.table[:c.vocab, :W] = ckpt.take("embed", (c.vocab, W)).to(device=dev, dtype=dt)
-        self.l_table = lk.stream_layout(self.table)
         self.pos_table = ckpt.take("pos", (c.max_positions, W)).to(device=dev, dtype=dt).contiguous()
         norm = lambda name: ckpt.take(name, (W,)).to(device=dev, dtype=torch.float32).contiguous()  # noqa: E731
         self.final_norm = norm("final.norm")
@@ -122,19 +122,21 @@ class DagupelStep:
                 if key not in tables:
                     tables[key] = rotary_table(m.rot_base, m.rot_dim, c.max_positions, m.rot_scaling, dev)
                 L.attn = LatentAttention(m, W, c.eps, {n: ckpt.take(p + "mix." + n, s) for n, s in shapes.items()}, tables[key],
-                                         dt, dev)
+                                         dt, dev, layouts=False)
                 L.norm1, L.norm2, L.mlp = norm(p + "norm1"), None, None
                 if mlp is not None:
                     L.norm2 = norm(p + "norm2")
                     L.mlp = ClampedGLU(W, mlp.ff, mlp.limit, {"gate": ckpt.take(p + "mlp.gate", (mlp.ff, W)),
                                                               "up": ckpt.take(p + "mlp.up", (mlp.ff, W)),
-                                                              "down": ckpt.take(p + "mlp.down", (W, mlp.ff))}, dt, dev)
+                                                              "down": ckpt.take(p + "mlp.down", (W, mlp.ff))}, dt, dev, layouts=False)
             self.layers.append(weights[j])
             self.caches.append(weights[j].attn.new_cache(limits.n_blocks, limits.block_size))
         # portions go to their own kernels where every layer has them (the step's rows are ordered once)
         self.portion_min = LatentAttention.PORTION_MIN if all(L.attn.portions_ok for L in self.layers) else None
-        own = list({id(L): L for L in self.layers}.values())
-        self._copied = lk.copied_weights([self.l_table] + [t for L in own for t in (L.attn.l_in, L.attn.l_o) + ((L.mlp.l_gate_up, L.mlp.l_down) if L.mlp else ())])
+        # (last: weights, cache and states come first)
+        own = [self] + [h for L in weights.values() for h in (L.attn, L.mlp) if h is not None]
+        lk.lay_out(own, lk.spare_memory(dev) if limits.stream_layouts else 0)
+        self._copied = lk.copied_weights(getattr(h, name) for h in own for name, _, _ in h.STREAMED)
         # called with (layer run, residual stream) after every layer, when set
         self.on_layer: Optional[Callable[[int, torch.Tensor], None]] = None
 

@@ -157,6 +157,32 @@ def stream_layout(w: torch.Tensor, glu: bool = False) -> Optional[torch.Tensor]:
     return out
 
 
+def spare_memory(device: torch.device) -> int:
+    """Half of what is left of the device's memory."""
+    if device.type != "cuda":
+        return 0
+    return (torch.cuda.mem_get_info(device)[0] + torch.cuda.memory_reserved(device) - torch.cuda.memory_allocated(device)) // 2
+
+
+def lay_out(holders, spare: Optional[int] = None) -> None:
+    """Makes the streamed layouts of holders' weights (STREAMED: attribute of the layout, of the weight, gate and up?), in their
+    order, as many as fit into `spare` bytes and can be had; products of the others run on the weights alone."""
+    for holder in holders:
+        for name, weight, glu in holder.STREAMED:
+            w = getattr(holder, weight)
+            size = (w.size(0) + 63) // 64 * 64 * w.size(1) * w.element_size()
+            setattr(holder, name, None)
+            if spare is not None and size > spare:
+                continue
+            try:
+                setattr(holder, name, stream_layout(w, glu))
+            except torch.OutOfMemoryError:
+                spare = 0
+                continue
+            if spare is not None and getattr(holder, name) is not None:
+                spare -= size
+
+
 def layout_is_current(layout: torch.Tensor, w: torch.Tensor) -> bool:
     of = getattr(layout, "copy_of", None)
     return of is None or (of.data_ptr() == w.data_ptr() and of._version == layout.copy_version)

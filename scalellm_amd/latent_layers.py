@@ -149,9 +149,10 @@ class LatentAttention:
     expanded by one product, multi-head attention over them.  32-bit: every row as a single token."""
 
     PORTION_MIN = 16
+    STREAMED = (("l_in", "w_in", False), ("l_o", "w_o", False))
 
     def __init__(self, args: LatentAttentionArgs, width: int, eps: float, w: Dict[str, torch.Tensor], cos_sin: torch.Tensor,
-                 dtype: torch.dtype, device):
+                 dtype: torch.dtype, device, layouts: bool = True):
         a = self.args = args
         self.eps, self.cos_sin = eps, cos_sin
         self.c_pad, self.r_pad = _pad_latent(a.kv_rank), round_up(a.rot_dim, 32)
@@ -191,7 +192,7 @@ class LatentAttention:
         self.o_k = round_up(H * self.v_pad, 64)
         self.w_o = z(round_up(width, 16), self.o_k)
         self.w_o[:width, :H * self.v_pad].view(width, H, self.v_pad)[:, :, :a.vdim] = g["o"].view(width, H, a.vdim)
-        self.l_in, self.l_o = lk.stream_layout(self.w_in), lk.stream_layout(self.w_o)
+        lk.lay_out([self], None if layouts else 0)
 
     def new_cache(self, n_blocks: int, block_size: int) -> LatentKVCache:
         return LatentKVCache(n_blocks, block_size, self.c_pad, self.r_pad, self.w_in.dtype, self.w_in.device)
@@ -237,8 +238,10 @@ class ClampedGLU:
     """W_down (g sigmoid(alpha g) (u + shift)), g = min(W_gate h, limit), u = clamp(W_up h, +-limit); without a limit, with
     alpha 1 and shift 0, the SiLU GLU."""
 
+    STREAMED = (("l_gate_up", "w_gate_up", True), ("l_down", "w_down", False))
+
     def __init__(self, width: int, ff: int, limit: float, w: Dict[str, torch.Tensor], dtype: torch.dtype, device,
-                 alpha: float = lk.GLU_ALPHA, shift: float = lk.GLU_SHIFT):
+                 alpha: float = lk.GLU_ALPHA, shift: float = lk.GLU_SHIFT, layouts: bool = True):
         self.limit, self.alpha, self.shift = float(limit), float(alpha), float(shift)
         k, f = round_up(width, 64), round_up(ff, 64)
         self.w_gate_up = torch.zeros(2 * f, k, dtype=dtype, device=device)
@@ -246,7 +249,7 @@ class ClampedGLU:
         self.w_gate_up[f:f + ff, :width] = w["up"].to(device=device, dtype=dtype)
         self.w_down = torch.zeros(round_up(width, 16), f, dtype=dtype, device=device)
         self.w_down[:width, :ff] = w["down"].to(device=device, dtype=dtype)
-        self.l_gate_up, self.l_down = lk.stream_layout(self.w_gate_up, glu=True), lk.stream_layout(self.w_down)
+        lk.lay_out([self], None if layouts else 0)
 
     def forward(self, h: torch.Tensor):
         act = h.new_empty(h.size(0), self.w_down.size(1))

@@ -202,7 +202,9 @@ class ParallelMixer:
     """Windowed attention and lightning attention on the same input: one product in front, one behind (the mixers' scales
     are applied to the heads' outputs)."""
 
-    def __init__(self, left: WindowAttention, right: LightningAttention, width: int):
+    STREAMED = (("l_in", "w_in", False), ("l_o", "w_o", False))
+
+    def __init__(self, left: WindowAttention, right: LightningAttention, width: int, layouts: bool = True):
         self.left, self.right = left, right
         self.split = left.w_in.size(0)
         self.w_in = torch.cat([left.w_in, right.w_in])
@@ -210,7 +212,7 @@ class ParallelMixer:
         self.w_o = torch.zeros(round_up(width, 16), self.o_k, dtype=left.dtype, device=self.w_in.device)
         self.w_o[:width, :left.out_width] = left.w_o
         self.w_o[:width, left.out_width:left.out_width + right.out_width] = right.w_o
-        self.l_in, self.l_o = lk.stream_layout(self.w_in), lk.stream_layout(self.w_o)
+        lk.lay_out([self], None if layouts else 0)
         left.w_in = right.w_in = left.w_o = right.w_o = None   # (laid out once)
 
     def new_cache(self, limits):
@@ -242,8 +244,9 @@ class ChannelDelta:
     o [width, heads vdim]."""
 
     UNIT_EPS = 1e-6
+    STREAMED = (("l_in", "w_in", False), ("l_o", "w_o", False))
 
-    def __init__(self, args: ChannelDeltaArgs, width: int, eps: float, w: Dict[str, torch.Tensor], dtype: torch.dtype, device):
+    def __init__(self, args: ChannelDeltaArgs, width: int, eps: float, w: Dict[str, torch.Tensor], dtype: torch.dtype, device, layouts: bool = True):
         a = self.args = args
         self.eps, self.dtype, self.device = eps, dtype, device
         H, G, D, V = a.heads, a.kv_heads, a.dim, a.vdim
@@ -264,7 +267,7 @@ class ChannelDelta:
         self.o_k = round_up(vo, 64)
         self.w_o = torch.zeros(round_up(width, 16), self.o_k, dtype=dtype, device=device)
         self.w_o[:width, :vo] = w["o"].to(device=device, dtype=dtype)
-        self.l_in, self.l_o = lk.stream_layout(self.w_in), lk.stream_layout(self.w_o)
+        lk.lay_out([self], None if layouts else 0)
         f32 = lambda t: t.to(device=device, dtype=torch.float32).contiguous()  # noqa: E731
         self.spec = mk.RecurrentSpec(
             _lib.REC_DELTA, H, G, D, V, 0, qk, 2 * qk, eps, off_b=off_b, off_gate=self.low_n, q_scale=D ** -0.5, unit_eps=self.UNIT_EPS,

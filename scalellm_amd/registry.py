@@ -34,6 +34,9 @@ class ModelLimits:
     device: str = "cuda"
     n_states: int = 64       # live sequences a recurrent model keeps state for
     max_positions: int = 0   # longest sequence of a model without a limit of its own; 0 = what the pool holds
+    # second copies of 16-bit weights in the order products of few rows read them, out of half of the memory that weights,
+    # cache and states leave (latent_kernels.lay_out); False: none, for what the program allocates later
+    stream_layouts: bool = True
 
 
 def register_model(name: str):

@@ -93,6 +93,7 @@ class _LayerWeights:
 @register_model("Vebusun")
 class VebusunStep:
     libraries = ("latent", "mixers")
+    STREAMED = (("l_head", "head", False),)
     portion_min = 2   # (a recurrence runs over whole portions)
 
     def __init__(self, config: VebusunConfig, ckpt: Checkpoint, limits: ModelLimits):
@@ -107,7 +108,6 @@ class VebusunStep:
         self.embed = ckpt.take("embed", (c.vocab, W)).to(device=dev, dtype=dt).contiguous()
         self.head = torch.zeros(round_up(c.vocab, 16), self.k_width, dtype=dt, device=dev)
         self.head[:c.vocab, :W] = ckpt.take("head", (c.vocab, W)).to(device=dev, dtype=dt)
-        self.l_head = lk.stream_layout(self.head)
         f32 = lambda name: ckpt.take(name, (W,)).to(device=dev, dtype=torch.float32).contiguous()  # noqa: E731
 
         def norm(name):
@@ -130,13 +130,16 @@ class VebusunStep:
                 L.norm2 = norm(p + "norm2")
                 L.mlp = ClampedGLU(W, layer.ff, math.inf, {"gate": ckpt.take(p + "mlp.gate", (layer.ff, W)),
                                                            "up": ckpt.take(p + "mlp.up", (layer.ff, W)),
-                                                           "down": ckpt.take(p + "mlp.down", (W, layer.ff))}, dt, dev, 1.0, 0.0)
+                                                           "down": ckpt.take(p + "mlp.down", (W, layer.ff))}, dt, dev, 1.0, 0.0, layouts=False)
             elif p + "norm2" in ckpt.names():   # (a norm nothing follows)
                 norm(p + "norm2")
             weights.append(L)
         self.layers = [weights[i] for i in c.runs]
         self.caches = [L.mixer.new_cache(limits) for L in self.layers]
-        self._copied = lk.copied_weights([self.l_head] + [t for L in weights for t in (L.mixer.l_in, L.mixer.l_o) + ((L.mlp.l_gate_up, L.mlp.l_down) if L.mlp else ())])
+        # (last: weights, cache and states come first)
+        own = [self] + [h for L in weights for h in (L.mixer, L.mlp) if h is not None]
+        lk.lay_out(own, lk.spare_memory(dev) if limits.stream_layouts else 0)
+        self._copied = lk.copied_weights(getattr(h, name) for h in own for name, _, _ in h.STREAMED)
         # called with (layer run, residual stream) after every layer, when set
         self.on_layer: Optional[Callable[[int, torch.Tensor], None]] = None
 
@@ -152,7 +155,7 @@ class VebusunStep:
                 if w[first].dim() != 2 or w[first].size(1) != W:
                     raise ValueError(f"{p}{first}: shape {tuple(w[first].shape)}")
                 w[second] = ckpt.take(p + second, (n, w[first].size(0)))
-            return ChannelDelta(m, W, c.eps, w, dt, dev)
+            return ChannelDelta(m, W, c.eps, w, dt, dev, layouts=False)
         a, b = m.left, m.right
         left = {"q": (a.heads * a.dim, W), "k": (a.kv_heads * a.dim, W), "v": (a.kv_heads * a.vdim, W), "q.norm": (a.dim,),
                 "k.norm": (a.dim,), "sink": (a.heads,), "o": (W, a.heads * a.vdim)}
@@ -161,7 +164,7 @@ class VebusunStep:
         left = {n: ckpt.take(f"{p}left.{n}", s) for n, s in left.items()}
         right = {n: ckpt.take(f"{p}right.{n}", s) for n, s in right.items()}
         return ParallelMixer(WindowAttention(a, W, c.eps, left, rotation(a), dt, dev, m.left_scale),
-                             LightningAttention(b, W, c.eps, right, dt, dev, m.right_scale), W)
+                             LightningAttention(b, W, c.eps, right, dt, dev, m.right_scale), W, layouts=False)
 
     @classmethod
     def from_checkpoint(cls, config: dict, ckpt: Checkpoint, limits: ModelLimits) -> "VebusunStep":

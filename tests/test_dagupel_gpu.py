@@ -347,3 +347,49 @@ def test_command_line_generates(tmp_path):
     assert p.returncode == 0, p.stderr[-2000:]
     got = [json.loads(ln)["tokens"] for ln in p.stdout.splitlines() if ln.startswith("{")]
     assert got == [_greedy(cfg, t, q, 5)[0] for q in ([1, 2, 3], [9, 8])]
+
+
+def test_second_copies_of_weights_come_out_of_spare_memory():
+    """The copies that decode products stream are made last, out of what weights and cache leave: a model that fills most of the
+    card loads without them, with some, or by ModelLimits without any, and gives the same."""
+    import gc
+    from tests import dagupel_common as dc
+    from scalellm_amd import latent_kernels as lk
+    from scalellm_amd.checkpoint import Checkpoint
+    from scalellm_amd.decode import make_batch_inputs
+    from scalellm_amd.registry import ModelLimits, model_class
+    cfg = dc.config(1024, [(dc.mixer(8, 64, 32, 64, 256, 40), 4096, 2.0), (dc.mixer(8, 64, 32, 64, 256, 40), 4096, 2.0)], vocab=8000)
+    t = weights(cfg, 3)
+    _, positions, params, _ = make_batch_inputs([1] * 3, [1] * 3, 16, "cuda", seed=1, vocab=8000)
+    tokens = torch.tensor([5, 17, 7999], dtype=torch.int32, device="cuda")
+
+    def build(**kw):
+        return model_class("Dagupel").from_checkpoint(cfg, Checkpoint(dict(t)), ModelLimits(8, 16, torch.bfloat16, "cuda", **kw))
+
+    def logits(m):
+        return m.forward(tokens, positions, params, return_logits=True).double()
+    full = build()
+    names = [(h, n) for L in full.layers for h, n in ((L.attn, "l_in"), (L.attn, "l_o"), (L.mlp, "l_gate_up"), (L.mlp, "l_down"))] + [(full, "l_table")]
+    assert all(getattr(h, n) is not None for h, n in names)
+    copies = sum(getattr(h, n).numel() * 2 for h, n in names)
+    want = logits(full)
+    none = build(stream_layouts=False)
+    assert none.l_table is None and none.layers[1].mlp.l_down is None and none.weights_version() == 0
+    assert (logits(none) - want).norm() / want.norm() < 1e-2   # (bf16 activations after sums in another order)
+
+    lk.lay_out([full] + [h for L in full.layers for h in (L.attn, L.mlp)], copies // 2)
+    kept = sum(getattr(h, n).numel() * 2 for h, n in names if getattr(h, n) is not None)
+    assert 0 < kept <= copies // 2 and (logits(full) - want).norm() / want.norm() < 1e-2
+
+    del full, none, names
+    gc.collect()
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total, held = torch.cuda.get_device_properties(0).total_memory, torch.cuda.memory_reserved()
+    try:   # room for the weights and what building takes, but not for the copies
+        torch.cuda.set_per_process_memory_fraction((held + copies + (40 << 20)) / total)
+        tight = build()
+        assert any(x is None for L in tight.layers for x in (L.attn.l_in, L.attn.l_o, L.mlp.l_gate_up, L.mlp.l_down))
+        assert (logits(tight) - want).norm() / want.norm() < 1e-2
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)

@@ -134,3 +134,30 @@ def test_streamed_layout_is_made_on_the_device_of_its_weight(monkeypatch):
                               device="cuda:3", is_inference=lambda: True)
     lk.stream_layout(w)
     assert made_on == ["cuda:3"]
+
+
+def test_layouts_fit_the_memory_that_is_left(monkeypatch):
+    import torch
+    from scalellm_amd import latent_kernels as lk
+
+    class Holder:
+        STREAMED = (("a", "wa", False), ("b", "wb", True), ("c", "wc", False))
+
+        def __init__(self):
+            self.wa, self.wb, self.wc = (torch.zeros(n, 64, dtype=torch.bfloat16) for n in (70, 640, 64))   # 16, 80 and 8 KB laid out
+    made = []
+    monkeypatch.setattr(lk, "stream_layout", lambda w, glu: made.append((w.size(0), glu)) or w)
+
+    def names(spare):
+        h, made[:] = Holder(), []
+        lk.lay_out([h], spare)
+        return "".join(n for n in "abc" if getattr(h, n) is not None)
+    assert names(None) == "abc" and made == [(70, False), (640, True), (64, False)]
+    assert [names(k << 10) for k in (0, 8, 16, 24, 96, 103, 104)] == ["", "c", "a", "ac", "ab", "ab", "abc"]
+
+    def full(w, glu):
+        if w.size(0) == 640:
+            raise torch.OutOfMemoryError
+        return w
+    monkeypatch.setattr(lk, "stream_layout", full)
+    assert names(None) == "a"   # (no more after a refusal)
