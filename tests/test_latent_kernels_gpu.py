@@ -99,11 +99,23 @@ def test_linear_epilogues(M, N, K, dtype):
 
 
 # row counts at the edges of every tile, columns that fill no panel of 64 and those that decide between tile widths, step
-# counts below, at and beyond a ring and a split.  fp32 sums of exact products of bf16: 1e-5 of the largest as above.
+# counts below and at a ring and a split.  fp32 sums of exact products of bf16: 1e-5 of the largest as above.
 @pytest.mark.parametrize("M", [1, 2, 16, 17, 32, 33, 64, 65, 127, 128, 140])
 @pytest.mark.parametrize("N,K", [(16, 64), (80, 192), (64, 576), (144, 1088), (192, 2112), (2048, 2048), (7168, 320), (16384, 128),
                                  (16896, 64)])
 def test_streamed_products(M, N, K):
+    _streamed_products(M, N, K)
+
+
+# Every tile shape of the dispatch with turns of its steady loop (several rings of steps a wave, or a split of it), in every epilogue that
+# it has, and step counts that leave waves, groups of waves and rings unequal tails.
+@pytest.mark.parametrize("M", [1, 16, 32, 63, 64, 100, 128, 140])
+@pytest.mark.parametrize("N,K", [(28672, 704), (16896, 1088), (16384, 2240), (7168, 1344), (6784, 2112), (1024, 16448), (64, 32832)])
+def test_streamed_products_of_many_steps(M, N, K):
+    _streamed_products(M, N, K)
+
+
+def _streamed_products(M, N, K):
     lk = _lk()
     x = _rnd(1, M, K + 8, dtype=torch.bfloat16)[:, :K]
     w = _rnd(2, N, K, dtype=torch.bfloat16, std=K ** -0.5)
