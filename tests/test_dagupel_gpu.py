@@ -236,14 +236,16 @@ def test_graph_replays_equal_eager_steps():
     assert row_errors(outs[1], outs[0].astype(np.float64)).max() < 1e-2
 
 
-def test_graph_replays_of_a_batch_the_vendor_products_serve():
-    """40 decode rows: the projections are library products inside the graph; every replay equals the eager step."""
+@pytest.mark.parametrize("batch", [40, 130])
+def test_graph_replays_of_a_batch_the_vendor_products_serve(batch):
+    """40 decode rows: the input projection is a library product inside the graph, the others are streamed; 130: every product is a
+    library one, with the activation's own launch.  Every replay equals the eager step."""
     cfg, t, _, _ = _model("wide")
     rng = np.random.default_rng(2)
-    prompts = [rng.integers(0, cfg["vocab"], 20 + k).tolist() for k in range(40)]
+    prompts = [rng.integers(0, cfg["vocab"], 20 + k % 40).tolist() for k in range(batch)]
     outs = []
-    for graphs in ([], [40]):
-        engine = _engine(cfg, t, torch.bfloat16, n_blocks=200, block_size=16, graph_batch_sizes=graphs, graph_max_seq_len=128)
+    for graphs in ([], [batch]):
+        engine = _engine(cfg, t, torch.bfloat16, n_blocks=5 * batch, block_size=16, graph_batch_sizes=graphs, graph_max_seq_len=128)
         engine.capture_graphs()
         seqs = [_seq(k, p) for k, p in enumerate(prompts)]
         _run(engine, [(s, len(s.tokens) - 9) for s in seqs])

@@ -196,15 +196,17 @@ def test_greedy_generation_through_the_scheduler(graphs):
     assert (engine.runner.num_graph_replayed > 0) == bool(graphs)
 
 
-@pytest.mark.parametrize("batch", [2, 40])
+@pytest.mark.parametrize("batch", [2, 40, 130])
 def test_graph_replays_equal_eager_steps(batch):
-    """bf16 decode batches through ModelRunner graphs, replays with eager steps between them (40 rows: vendor products)."""
+    """bf16 decode batches through ModelRunner graphs, replays with eager steps between them (40 rows: streamed products, but for
+    the input projections; 130: vendor products, with the activation's own launch)."""
     cfg, t, tokens, _ = _model("wide")
     rng = np.random.default_rng(2)
     prompts = [rng.integers(0, cfg["vocab"], 100 + k % 7).tolist() for k in range(batch)]
     steps, outs = 60 if batch == 2 else 8, []
     for graphs in ([], [batch]):
-        engine = _engine(cfg, t, torch.bfloat16, n_blocks=8 * batch + 8, block_size=16, graph_batch_sizes=graphs, graph_max_seq_len=256)
+        engine = _engine(cfg, t, torch.bfloat16, n_blocks=8 * batch + 8, block_size=16, n_states=max(64, batch + 1),
+                         graph_batch_sizes=graphs, graph_max_seq_len=256)
         engine.capture_graphs()
         seqs = [_seq(k, p) for k, p in enumerate(prompts)]
         rows = _run(engine, [(s, len(s.tokens) - steps) for s in seqs])
