@@ -41,21 +41,22 @@ __device__ __forceinline__ float conv_input(const slm_recurrent_args& a, const E
   }
   return silu_f32(acc);
 }
-// The ring entry that the input j tokens back of position p lies in (a convolution of at most 4 taps), or -1: the step's own row.
-// Inputs there are not (older than the taps, or than the sequence) are the own row again and left out of the sum, so that no
-// load reads the entry another head of the launch may be writing.
+// The ring entry that the input j > 0 tokens back of position p lies in, of a convolution of at least 2 taps.  Inputs there are not
+// (older than the taps, or than the sequence) are left out of the sum; their loads go to an entry that is there, and never to
+// that of p itself, which another head of the launch may be writing.
 constexpr __host__ __device__ int step_entry(int j, int p, int taps) {
-  return j == 0 || j > taps - 1 || j > p ? -1 : (p - j) % taps;
+  const int most = taps - 1 < p ? taps - 1 : p, back = j < most ? j : most;
+  return (p + taps - (back > 1 ? back : 1)) % taps;
 }
 constexpr bool step_reads_no_kept_entry() {
-  for (int taps = 1; taps <= 4; ++taps)
+  for (int taps = 2; taps <= 4; ++taps)
     for (int p = 0; p < 12; ++p)
-      for (int j = 0; j < 4; ++j)
-        if (step_entry(j, p, taps) == p % taps) return false;
+      for (int j = 1; j < 4; ++j)
+        if (step_entry(j, p, taps) == p % taps || (j <= p && j < taps && step_entry(j, p, taps) != (p - j) % taps)) return false;
   return true;
 }
 static_assert(step_reads_no_kept_entry(), "the entry of the step's own position is written while the others are read");
-// the same for the one row of a step, convolutions of at most 4 taps: every load at once
+// the same for the one row of a step, convolutions of 2 to 4 taps: every load at once
 template <typename E>
 __device__ __forceinline__ float conv_step4(const slm_recurrent_args& a, const E* ring, int64_t row, int p, int c) {
   const int64_t ch = 2 * (int64_t)a.qk_heads * a.dim + (int64_t)a.heads * a.vdim;
@@ -64,10 +65,8 @@ __device__ __forceinline__ float conv_step4(const slm_recurrent_args& a, const E
   float w[4], x[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    const int entry = step_entry(j, p, a.taps);
-    const E* own = reinterpret_cast<const E*>(a.proj) + row * a.ld_proj + col;
     w[j] = a.conv_w[(int64_t)(a.taps - 1 - min(j, most)) * ch + c];
-    x[j] = to_f32(*(entry < 0 ? own : ring + (int64_t)entry * ch + c));
+    x[j] = to_f32(j == 0 ? reinterpret_cast<const E*>(a.proj)[row * a.ld_proj + col] : ring[(int64_t)step_entry(j, p, a.taps) * ch + c]);
   }
   float acc = 0.f;
 #pragma unroll
@@ -156,7 +155,7 @@ __global__ void __launch_bounds__(1024) recurrent_step_kernel(const slm_recurren
       float x = 0.f;
       if (at < (kind == 3 ? a.vdim : a.dim)) {
         const int c = kind == 3 ? 2 * qk + head * a.vdim + at : kind * qk + qh * a.dim + at;
-        x = a.taps <= 4 ? conv_step4<E>(a, ring, row, p, c) : conv_input<E>(a, ring, row, row, p, c);
+        x = a.taps <= 4 && a.taps > 1 ? conv_step4<E>(a, ring, row, p, c) : conv_input<E>(a, ring, row, row, p, c);
         if (kind == 3 || first_of_group) keep[c] = raw_input<E>(a, row, c);
       }
       if (kind == 0) nq = __builtin_fmaf(x, x, nq);
