@@ -3,8 +3,9 @@
 //
 //   step     one row per sequence: convolution, activations, unit vectors, gates, the update and (delta) the output norm
 //            in one launch.  One workgroup per (row, head); the state is read and written once, past the caches.  Bound: HBM
-//            (state).  16 heads of 128 x 128, 128 rows: 74 us with ordinary loads and stores, 60 without, and 54 with the inputs'
-//            loads side by side; lightning 55 and 48 (5.6 TB/s).
+//            (state).  16 heads of 128 x 128: delta 128 rows 71 us with ordinary loads and stores and the inputs one after the
+//            other, 52 without (5.2 TB/s), 32 rows 18.4 and 14.1; lightning, the first alone, 128 rows 53 and 46 (5.8 TB/s), 32 rows
+//            14.4 and 12.7, 8 rows 6.0 and 5.5, 1 row 4.3 and 4.3.
 //   prepare  portions, cut into chunks of 16 tokens, every chunk at once: inputs activated and normed, decays summed, and
 //            what a chunk's tokens do to each other solved (a 16 x 16 triangular system).  Bound: VALU, HBM.
 //   scan     portions: chunk after chunk.  The columns of S are independent, so a workgroup owns 16 of them and keeps them

@@ -19,7 +19,7 @@ enum TuneKey : int {
   TUNE_ATTN_TILE_PF,      // SLM_ATTN_TILE_PF      tile kernel staging form: 0 = no prefetch, 2 = 32-row single-buffer tiles, 4 = register-staged 64-row tiles, 5 = LDS-DMA without the cross-tile pipeline (default 1: LDS-DMA + pipeline where they exist)
   TUNE_ATTN_U,            // SLM_ATTN_U            K/V register ring depth (2/4)
   TUNE_ATTN_NT,           // SLM_ATTN_NT           non-temporal KV loads on/off
-  TUNE_ATTN_TILE_DECODE,  // SLM_ATTN_TILE_DECODE  min GQA group at which q_len = 1 goes to the tile kernel (default 8, 0 = never)
+  TUNE_ATTN_TILE_DECODE,  // SLM_ATTN_TILE_DECODE  min GQA group at which q_len = 1 goes to the tile kernel (0 = never; default 8, in mixed calls the rule of attn.hip)
   TUNE_ATTN_BAL,          // SLM_ATTN_BAL          0 = classic per-sequence split-KV for pure decode (no balanced partition)
   TUNE_ATTN_W,            // SLM_ATTN_W            16-byte chunks of a K / V row per lane in the decode stream kernel: 1 / 2 force a form (default: by batch size and KV heads)
   TUNE_ATTN_PRIO,         // SLM_ATTN_PRIO         0 = the decode stream kernel does not raise its wave priority (default 1: s_setprio 3)

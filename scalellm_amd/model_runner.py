@@ -126,7 +126,8 @@ class _Graph:
                  (mine.block_tables[:given.block_tables.numel()], given.block_tables), (mine.cu_block_lens, given.cu_block_lens)]
         if mine.state_slots is not None:
             pairs.append((mine.state_slots, given.state_slots))
-        # (one launch: as copies of their own these are seven or eight, 3 us each in front of a step of a few hundred)
+        # (one launch: as copies of their own these are seven or eight, 3 us each in front of a step of a few hundred.  The first
+        # replay of a captured graph, whose upload separate copies would hide, pays 20 - 50 us for it, once)
         torch._foreach_copy_([d for d, _ in pairs], [s for _, s in pairs], non_blocking=True)
         key = None
         if None not in self.variants:   # the batch's own hints pick the variant (never the capture bound)
