@@ -178,7 +178,7 @@ __global__ void __launch_bounds__(64 * NW * (KV2 ? 2 : 1)) __attribute__((amdgpu
   const int tq = jvalid ? jrow / G : (rows_total - 1) / G;  // token index inside the sequence
   const int head = kvh * G + (jvalid ? jrow % G : 0);
   const int diag = kv_len - q_len + tq;  // last visible kv index of this row (causal)
-  const int64_t part_row = p.part_rows > 0 ? (int64_t)b * p.part_rows + tq : q_start + tq;  // where its partials go
+  auto part_row = [&]() -> int64_t { return p.part_rows > 0 ? (int64_t)b * p.part_rows + tq : q_start + tq; };  // where its partials go
   if (kv_len <= 0) {
     if (grp != 0) return;   // (workgroup-uniform condition: nobody reaches a barrier)
     // empty history (workgroup-uniform): this kernel owns the rows, so it publishes the empty
@@ -186,7 +186,7 @@ __global__ void __launch_bounds__(64 * NW * (KV2 ? 2 : 1)) __attribute__((amdgpu
     // whose loads are unconditional (an unwritten partial would be combined as garbage)
     if (!jvalid) return;
     if (p.n_splits > 1) {
-      const int64_t pi = (part_row * p.n_heads + head) * p.part_slots + split;
+      const int64_t pi = (part_row() * p.n_heads + head) * p.part_slots + split;
       float* opp = p.o_part + pi * HD;
       for (int d = 4 * hh; d < HD; d += 8) *reinterpret_cast<f32x4*>(opp + d) = f32x4{0.f, 0.f, 0.f, 0.f};
       if (hh == 0) {
@@ -809,7 +809,7 @@ __global__ void __launch_bounds__(64 * NW * (KV2 ? 2 : 1)) __attribute__((amdgpu
   if (p.n_splits > 1) {
     // split-KV partials in the token-major kernel's format (combined by attn_combine_kernel):
     // un-normalised O (fp32), running max (log2 domain) and sum of this KV share
-    const int64_t pi = (part_row * p.n_heads + head) * p.part_slots + split;
+    const int64_t pi = (part_row() * p.n_heads + head) * p.part_slots + split;
     float* opp = p.o_part + pi * HD;
 #pragma unroll
     for (int d = 0; d < DT; ++d)
