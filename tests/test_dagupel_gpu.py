@@ -387,8 +387,15 @@ def test_second_copies_of_weights_come_out_of_spare_memory():
     gc.collect()
     torch.cuda.synchronize()
     torch.cuda.empty_cache()
-    total, held = torch.cuda.get_device_properties(0).total_memory, torch.cuda.memory_reserved()
-    try:   # room for the weights and what building takes, but not for the copies
+    total, held, filler = torch.cuda.get_device_properties(0).total_memory, torch.cuda.memory_reserved(), []
+    try:   # room for the weights and what building takes, but not for the copies, nor in what earlier work left reserved
+        torch.cuda.set_per_process_memory_fraction(held / total)
+        for size in (1 << k for k in range(34, 19, -1)):
+            while torch.cuda.memory_allocated() + size <= held:
+                try:
+                    filler.append(torch.empty(size, dtype=torch.uint8, device="cuda"))
+                except torch.OutOfMemoryError:
+                    break
         torch.cuda.set_per_process_memory_fraction((held + copies + (40 << 20)) / total)
         tight = build()
         assert any(x is None for L in tight.layers for x in (L.attn.l_in, L.attn.l_o, L.mlp.l_gate_up, L.mlp.l_down))
