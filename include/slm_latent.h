@@ -73,6 +73,10 @@ SLM_API int slm_stream_layout(void* out, const void* w, int64_t N, int64_t K, in
 /* infinite: with alpha 1 and shift 0 the plain SiLU GLU); gu = [rows, 2 * half]                         */
 SLM_API int slm_clamped_glu(void* y, const void* gu, int64_t rows, int64_t half, int64_t ld_gu, int64_t ld_y,
                             float limit, float glu_alpha, float glu_shift, int32_t dtype, void* stream);
+/* The same in bf16 over the slabs [n_slabs][rows][2 * half] (n_slabs <= 8) that slm_linear_stream left of a product with  */
+/* a GLU layout: their columns come 16 of the gate, the same 16 of the up half in turn                   */
+SLM_API int slm_glu_slabs(void* y, const void* slabs, int64_t rows, int64_t half, int32_t n_slabs, int64_t ld_y,
+                          float limit, float glu_alpha, float glu_shift, void* stream);
 
 /* ---- 3. latent cache append: latent RMS norm, rotation of the shared key part and of the queries --- */
 typedef struct slm_latent_append_args {

@@ -282,6 +282,7 @@ def latent_lib() -> C.CDLL:
         ("slm_linear_stream", C.c_int, [P(LinearArgs), ptr]),
         ("slm_stream_layout", C.c_int, [ptr, ptr, i64, i64, i32, ptr]),
         ("slm_clamped_glu", C.c_int, [ptr, ptr, i64, i64, i64, i64, f32, f32, f32, i32, ptr]),
+        ("slm_glu_slabs", C.c_int, [ptr, ptr, i64, i64, i32, i64, f32, f32, f32, ptr]),
         ("slm_latent_append", C.c_int, [P(LatentAppendArgs), ptr]),
         ("slm_latent_attn_workspace_bytes", C.c_size_t, [P(LatentAttnArgs)]),
         ("slm_latent_attn", C.c_int, [P(LatentAttnArgs), ptr]),

@@ -1,6 +1,8 @@
 // residual_norm.hip -- the fp32 residual stream: what a sub-layer adds (or the embedding), and the norm (RMS, or
 // tanh(alpha x), which needs no statistics) in front of the next projection, in one launch.  One workgroup per row; the row stays in
 // registers between the sum of squares and the scaling.  Bound: HBM, trivial.
+#include <type_traits>
+
 #include "latent_common.h"
 
 namespace slm {
@@ -143,6 +145,28 @@ static int glu_launch(void* y, const void* gu, int64_t rows, int64_t half, int64
   return hip_check_launch();
 }
 
+// The GLU over NS slabs of a streamed product, whose columns come 16 of the gate, the same 16 of the up half in turn: four columns a
+// thread, all loads before the sums.  Bound: latency (4096 columns, 64 rows, 4 slabs: 4 MB out of the L2).
+template <int NS>
+__global__ void __launch_bounds__(256) glu_slabs_kernel(bf16* __restrict__ y, const float* __restrict__ slabs, uint32_t quads, uint32_t n,
+                                                        int64_t slab_stride, int64_t ld_y, float limit, float alpha, float shift) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  const uint32_t row = i / quads, c = (i - row * quads) * 4;
+  const float* src = slabs + (int64_t)row * (8 * (int64_t)quads) + 2 * (c & ~15u) + (c & 15u);
+  f32x4 g[NS], u[NS];
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+    g[s] = *reinterpret_cast<const f32x4*>(src + s * slab_stride);
+    u[s] = *reinterpret_cast<const f32x4*>(src + s * slab_stride + 16);
+  }
+#pragma unroll
+  for (int s = 1; s < NS; ++s) g[0] += g[s], u[0] += u[s];
+  bf16* o = y + row * ld_y + c;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) o[j] = (bf16)clamped_glu_f32(g[0][j], u[0][j], limit, alpha, shift);
+}
+
 template <typename E, int MODE>
 static int rn_launch(const slm_residual_norm_args& a, hipStream_t st) {
   const bool v4 = a.width % 4 == 0 && a.ld_delta % 4 == 0 && a.ld_embed % 4 == 0 && a.ld_out % 4 == 0 &&
@@ -210,4 +234,29 @@ extern "C" SLM_API int slm_clamped_glu(void* y, const void* gu, int64_t rows, in
   if (dtype == SLM_BF16) return glu_launch<bf16>(y, gu, rows, half, ld_gu, ld_y, limit, glu_alpha, glu_shift, (hipStream_t)stream);
   if (dtype == SLM_F32) return glu_launch<float>(y, gu, rows, half, ld_gu, ld_y, limit, glu_alpha, glu_shift, (hipStream_t)stream);
   return SLM_ERR_UNSUPPORTED;
+}
+
+extern "C" SLM_API int slm_glu_slabs(void* y, const void* slabs, int64_t rows, int64_t half, int32_t n_slabs, int64_t ld_y, float limit,
+                                     float glu_alpha, float glu_shift, void* stream) {
+  if (!y || !slabs || rows < 0 || half <= 0 || half % 16 || n_slabs < 1 || n_slabs > 8 || ld_y < half) return SLM_ERR_INVALID_ARG;
+  if (!aligned16(slabs)) return SLM_ERR_ALIGNMENT;
+  if (rows == 0) return SLM_OK;
+  const int64_t quads = half / 4, n = rows * quads;
+  if (n > 0xffffff00ll || rows > 0x7fffffff) return SLM_ERR_UNSUPPORTED;   // a launch has fewer than 2^32 threads
+  auto launch = [&](auto count) {
+    glu_slabs_kernel<decltype(count)::value><<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream>>>(
+        (bf16*)y, (const float*)slabs, (uint32_t)quads, (uint32_t)n, rows * 2 * half, ld_y, limit, glu_alpha, glu_shift);
+  };
+  hip_clear_error();
+  switch (n_slabs) {
+    case 1: launch(std::integral_constant<int, 1>{}); break;
+    case 2: launch(std::integral_constant<int, 2>{}); break;
+    case 3: launch(std::integral_constant<int, 3>{}); break;
+    case 4: launch(std::integral_constant<int, 4>{}); break;
+    case 5: launch(std::integral_constant<int, 5>{}); break;
+    case 6: launch(std::integral_constant<int, 6>{}); break;
+    case 7: launch(std::integral_constant<int, 7>{}); break;
+    default: launch(std::integral_constant<int, 8>{}); break;
+  }
+  return hip_check_launch();
 }

@@ -257,6 +257,21 @@ def stream_split_count(n_out: int, k: int) -> int:
     return max(1, min(8, 256 // ((n_out + 63) // 64), k // 512))
 
 
+def glu_split_count(n_out: int, k: int, rows: int) -> int:
+    """Slabs of a streamed product in front of the GLU; 1: the GLU is its epilogue.  A workgroup of that form walks all of K, 0.29 us a
+    step of 64 up to 64 rows and 0.53 above, however few columns there are; slabs share it out for one launch more (epilogue / slabs /
+    vendor product and GLU, us, 64 rows: 1024 x 1024 7.9 / 6.3 / 10.8, 1024 x 8192 39.0 / 10.9 / 15.9, 4096 x 4096 22.3 / 13.0 / 17.9, 8192 x 1024 8.6 / 9.9 /
+    14.8; 128 rows: 512 x 512 8.6 / 7.3 / 8.7, 4096 x 4096 36.3 / 19.1 / 27.0, 8192 x 8192 67.7 / 36.5 / 50.5, 14336 x 2048 21.8 / 26.7 / 21.4, 14336 x 8192
+    68.2 / 54.6 / 65.7).  Up to 32 rows the waves share K."""
+    if rows <= STREAM_MAX_ROWS or (k < 1536 and n_out > 4096):
+        return 1
+    panels = (n_out + 63) // 64
+    # (two workgroups a CU hide each other's waits where K is long: 11008 x 4096, 65 rows 35.7 -> 29.2, 8192 x 8192 39.9 -> 33.5)
+    wgs = 512 if rows > 64 and n_out > 4096 and k >= (8192 if n_out <= 8192 else 4096) else 256
+    step = 256 if (k < 2048 and n_out <= 2048) or (k < 1024 and n_out <= 4096) else 512
+    return max(1, min(8, wgs // panels, k // step))
+
+
 def split_count(rows: int, n_out: int, k: int) -> int:
     """Split-K slabs of a narrow product: enough workgroups for the chip, at least 4 steps of 64 per wave."""
     per = 16 if rows <= 16 else 32
@@ -284,6 +299,14 @@ def linear_glu(x: torch.Tensor, w_gate_up: torch.Tensor, out: torch.Tensor, limi
     half = N // 2
     _need(out.shape == (M, half) and out.stride(1) == 1 and out.dtype == x.dtype, "linear_glu: out [M, N / 2]")
     s = _stream_args(x, w_gate_up, layout, M, N, K, STREAM_LAYOUT_MAX_ROWS)
+    n = glu_split_count(N, K, M) if s is not None else 1
+    if n > 1:
+        slabs = torch.empty(n, M, N, dtype=torch.float32, device=x.device)
+        s.ldy, s.y, s.epilogue, s.n_splits = N, _p(slabs), _lib.LIN_SLABS, n
+        _run_stream(s)
+        latent_check(_lib.latent_lib().slm_glu_slabs(_p(out), _p(slabs), M, half, n, out.stride(0), float(limit), float(alpha), float(shift),
+                                                     _stream()), "slm_glu_slabs")
+        return out
     if s is not None or streams_rows(x):
         a = s if s is not None else _linear_args(x, w_gate_up, M, N, K)
         a.ldx, a.ldw, a.ldy, a.y, a.epilogue = x.stride(0), K, out.stride(0), _p(out), _lib.LIN_GLU

@@ -161,3 +161,33 @@ def test_layouts_fit_the_memory_that_is_left(monkeypatch):
         return w
     monkeypatch.setattr(lk, "stream_layout", full)
     assert names(None) == "a"   # (no more after a refusal)
+
+
+# one launch where K is short or the columns alone fill the chip, slabs and the GLU behind them where one workgroup would walk a long K
+@pytest.mark.parametrize("N,K,M,slabs", [
+    (4096, 4096, 32, 1), (512, 512, 33, 2), (1024, 1024, 64, 4), (1024, 8192, 64, 8), (4096, 768, 100, 3), (4096, 1024, 33, 2), (4096, 4096, 33, 4),
+    (4096, 14336, 128, 4), (5504, 1024, 100, 1), (8192, 1536, 64, 2), (8192, 8192, 64, 2), (8192, 8192, 65, 4), (11008, 4096, 64, 1),
+    (11008, 4096, 65, 2), (14336, 2048, 128, 1), (14336, 8192, 128, 2), (28672, 4096, 128, 1)])
+def test_glu_products_share_a_long_contraction(N, K, M, slabs, monkeypatch):
+    import types
+    import torch
+    from scalellm_amd import _lib as lib, latent_kernels as lk
+    ran, glu = [], []
+    monkeypatch.setattr(lk, "_p", lambda t: 4096)
+    monkeypatch.setattr(lk, "_stream", lambda: 0)
+    monkeypatch.setattr(lk, "_run_stream", lambda a: ran.append((a.epilogue, a.n_splits)))
+    monkeypatch.setattr(lk._lib, "latent_lib", lambda: types.SimpleNamespace(slm_glu_slabs=lambda *a: glu.append(a[2:6]) or 0))
+    t = lambda *shape: torch.empty(*shape, dtype=torch.bfloat16, device="meta")  # noqa: E731
+    lk.linear_glu(t(M, K), t(N, K), t(M, N // 2), 7.0, layout=t((N + 63) // 64, K // 64, 4, 2, 64, 8))
+    if slabs == 1:
+        assert ran == [(lib.LIN_GLU, 1)] and not glu
+    else:
+        assert ran == [(lib.LIN_SLABS, slabs)] and glu == [(M, N // 2, slabs, N // 2)]
+
+
+def test_glu_over_slabs_refuses_what_it_has_no_form_for():
+    f = _lib.latent_lib().slm_glu_slabs
+    args = lambda rows=1, half=32, n=2, ld=32, y=4096, s=4096: (y, s, rows, half, n, ld, 1.0, 1.0, 1.0, None)  # noqa: E731
+    assert f(*args(rows=0)) == 0
+    assert {f(*args(half=24)), f(*args(n=0)), f(*args(n=9)), f(*args(ld=31)), f(*args(y=None)), f(*args(rows=-1))} == {-1}
+    assert f(*args(s=4104)) == -5

@@ -131,6 +131,22 @@ def _streamed_products(M, N, K):
         _close(out, ref.clamped_glu(want[:, :N // 2], want[:, N // 2:], 0.6), torch.bfloat16, b16=2e-2)
 
 
+# every number of slabs, rows and columns that fill no workgroup, results at an odd address; one rounding to 16 bits
+@pytest.mark.parametrize("n", range(1, 9))
+@pytest.mark.parametrize("rows,half", [(1, 16), (33, 96), (128, 2752)])
+def test_glu_over_slabs(n, rows, half):
+    from scalellm_amd import _lib
+    lk = _lk()
+    slabs = _rnd(3, n, rows, 2 * half)
+    total = _f64(slabs).sum(0).reshape(rows, half // 16, 2, 16)
+    wide = torch.full((rows, half + 5), float("nan"), dtype=torch.bfloat16, device=DEV)
+    out = wide[:, 1:1 + half]
+    lk.latent_check(_lib.latent_lib().slm_glu_slabs(lk._p(out), lk._p(slabs), rows, half, n, wide.stride(0), 0.6, lk.GLU_ALPHA, lk.GLU_SHIFT,
+                                                    lk._stream()), "slm_glu_slabs")
+    _close(out, ref.clamped_glu(total[:, :, 0].reshape(rows, half), total[:, :, 1].reshape(rows, half), 0.6), torch.bfloat16)
+    assert wide[:, 0].isnan().all() and wide[:, 1 + half:].isnan().all()
+
+
 @pytest.mark.parametrize("M", [33, 64, 128])
 def test_products_of_one_row_many_times(M):
     """Rows without a stride of their own (an expanded one), and rows that overlap: above 32 they are the vendor product's."""
