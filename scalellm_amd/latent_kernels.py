@@ -251,10 +251,17 @@ def linear_f32(x: torch.Tensor, w: torch.Tensor, alpha: float = 1.0, layout: Opt
     return out
 
 
-def stream_split_count(n_out: int, k: int) -> int:
+def stream_split_count(n_out: int, k: int, rows: int) -> int:
     """Slabs of a streamed product: as many as give every CU a workgroup of 64 columns, at least 8 steps of 64 each (a slab
-    is written and read: 4096 columns, 128 rows, 4 against 8 slabs 34 us against 29, and 4 us less behind it)."""
-    return max(1, min(8, 256 // ((n_out + 63) // 64), k // 512))
+    is written and read: 4096 columns, 128 rows, 4 against 8 slabs 34 us against 29, and 4 us less behind it).  Above 32 rows a step is
+    0.3 to 0.5 us long, so short products of few columns take 4 steps each (with the norm behind them, 100 rows, before / after / vendor
+    product: 512 x 512 10.0 / 8.1 / 7.6, 2048 x 896 13.4 / 10.0 / 10.3, 1024 x 1536
+    10.7 / 9.5 / 10.1, 4096 x 768 13.2 / 11.4 / 10.9; more columns fill the chip: 5504 x 640 13.3 / 13.3 / 10.9), and large ones above 64 rows two workgroups a CU, which hide each other's
+    waits (8192 x 8192 43.5 / 37.0 / 41.8, 8192 x 14336 69.3 / 51.6 / 71.2)."""
+    panels = (n_out + 63) // 64
+    wgs = 512 if rows > 64 and n_out > 4096 and k >= (8192 if n_out <= 8192 else 4096) else 256
+    step = 256 if rows > STREAM_MAX_ROWS and ((k < 2048 and n_out <= 2048) or (k < 1024 and n_out <= 4096)) else 512
+    return max(1, min(8, wgs // panels, k // step))
 
 
 def glu_split_count(n_out: int, k: int, rows: int) -> int:
@@ -262,14 +269,10 @@ def glu_split_count(n_out: int, k: int, rows: int) -> int:
     step of 64 up to 64 rows and 0.53 above, however few columns there are; slabs share it out for one launch more (epilogue / slabs /
     vendor product and GLU, us, 64 rows: 1024 x 1024 7.9 / 6.3 / 10.8, 1024 x 8192 39.0 / 10.9 / 15.9, 4096 x 4096 22.3 / 13.0 / 17.9, 8192 x 1024 8.6 / 9.9 /
     14.8; 128 rows: 512 x 512 8.6 / 7.3 / 8.7, 4096 x 4096 36.3 / 19.1 / 27.0, 8192 x 8192 67.7 / 36.5 / 50.5, 14336 x 2048 21.8 / 26.7 / 21.4, 14336 x 8192
-    68.2 / 54.6 / 65.7).  Up to 32 rows the waves share K."""
+    68.2 / 54.6 / 65.7).  Up to 32 rows the epilogue is the faster form."""
     if rows <= STREAM_MAX_ROWS or (k < 1536 and n_out > 4096):
         return 1
-    panels = (n_out + 63) // 64
-    # (two workgroups a CU hide each other's waits where K is long: 11008 x 4096, 65 rows 35.7 -> 29.2, 8192 x 8192 39.9 -> 33.5)
-    wgs = 512 if rows > 64 and n_out > 4096 and k >= (8192 if n_out <= 8192 else 4096) else 256
-    step = 256 if (k < 2048 and n_out <= 2048) or (k < 1024 and n_out <= 4096) else 512
-    return max(1, min(8, wgs // panels, k // step))
+    return stream_split_count(n_out, k, rows)
 
 
 def split_count(rows: int, n_out: int, k: int) -> int:
@@ -283,7 +286,7 @@ def linear_slabs(x: torch.Tensor, w: torch.Tensor, layout: Optional[torch.Tensor
     """x W^T left as fp32 split-K partial sums for residual_norm().  layout: stream_layout(w)."""
     M, N, K = _check_xw(x, w)
     s = _stream_args(x, w, layout, M, N, K, STREAM_LAYOUT_MAX_ROWS)
-    n = split_count(M, N, K) if s is None else stream_split_count(N, K)
+    n = split_count(M, N, K) if s is None else stream_split_count(N, K, M)
     out = torch.empty(n, M, N, dtype=torch.float32, device=x.device)
     a = s if s is not None else _linear_args(x, w, M, N, K)
     a.ldx, a.ldw, a.ldy, a.y, a.epilogue, a.n_splits = x.stride(0), K, N, _p(out), _lib.LIN_SLABS, n

@@ -191,3 +191,12 @@ def test_glu_over_slabs_refuses_what_it_has_no_form_for():
     assert f(*args(rows=0)) == 0
     assert {f(*args(half=24)), f(*args(n=0)), f(*args(n=9)), f(*args(ld=31)), f(*args(y=None)), f(*args(rows=-1))} == {-1}
     assert f(*args(s=4104)) == -5
+
+
+@pytest.mark.parametrize("N,K,M,slabs", [
+    (512, 512, 32, 1), (512, 512, 33, 2), (512, 512, 128, 2), (2048, 896, 100, 3), (1024, 1536, 100, 6), (2048, 2048, 100, 4), (4096, 768, 65, 3),
+    (4096, 1024, 65, 2), (4096, 4096, 128, 4), (4096, 14336, 128, 4), (5504, 640, 100, 1), (8192, 8192, 64, 2), (8192, 8192, 65, 4), (8192, 14336, 128, 4),
+    (8192, 6144, 128, 2), (64, 32832, 1, 8)])
+def test_slabs_of_streamed_products(N, K, M, slabs):
+    from scalellm_amd import latent_kernels as lk
+    assert lk.stream_split_count(N, K, M) == slabs
