@@ -214,11 +214,13 @@ def _run_stream(a) -> None:
     latent_check(_lib.latent_lib().slm_linear_stream(C.byref(a), _stream()), "slm_linear_stream")
 
 
-def _store_rows(N: int) -> int:
+def _store_rows(N: int, K: int) -> int:
     """Rows up to which a product that is only stored is streamed.  Without slabs its workgroups are its columns': from 33
     rows the vendor GEMM, which splits K for itself, is level or ahead under 8192 columns (6752 x 4096, 64 rows: 19.2 us
-    against 22.6), and above 64 rows always (16896 x 4096, 128 rows: 46.6 against 47.0; 64 rows: 44.0 against 38.5)."""
-    return 64 if N >= 8192 else STREAM_MAX_ROWS
+    against 22.6) and a little above where K is long (vendor / streamed, 64 rows: 8192 x 2048 13.8 / 12.9, x 4096 19.1 / 22.3, x 8192
+    32.5 / 40.8; 9216 x 4096 26.4 / 22.9, x 8192 40.2 / 42.4; 12288 x 8192 44.0 / 43.3), and above 64 rows always (16896 x 4096, 128
+    rows: 46.6 against 47.0; 64 rows: 44.0 against 38.5)."""
+    return 64 if N >= 8192 and K <= 2048 + 5 * (N - 8192) // 2 else STREAM_MAX_ROWS
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None, layout: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -227,7 +229,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None,
     if out is None:
         out = torch.empty(M, N, dtype=x.dtype, device=x.device)
     _need(out.shape == (M, N) and out.stride(1) == 1 and out.dtype == x.dtype, "linear: out [M, N]")
-    a = _stream_args(x, w, layout, M, N, K, _store_rows(N))
+    a = _stream_args(x, w, layout, M, N, K, _store_rows(N, K))
     if a is not None:
         a.ldy, a.y, a.epilogue = out.stride(0), _p(out), _lib.LIN_STORE
         _run_stream(a)
@@ -256,8 +258,8 @@ def stream_split_count(n_out: int, k: int, rows: int) -> int:
     is written and read: 4096 columns, 128 rows, 4 against 8 slabs 34 us against 29, and 4 us less behind it).  Above 32 rows a step is
     0.3 to 0.5 us long, so short products of few columns take 4 steps each (with the norm behind them, 100 rows, before / after / vendor
     product: 512 x 512 10.0 / 8.1 / 7.6, 2048 x 896 13.4 / 10.0 / 10.3, 1024 x 1536
-    10.7 / 9.5 / 10.1, 4096 x 768 13.2 / 11.4 / 10.9; more columns fill the chip: 5504 x 640 13.3 / 13.3 / 10.9), and large ones above 64 rows two workgroups a CU, which hide each other's
-    waits (8192 x 8192 43.5 / 37.0 / 41.8, 8192 x 14336 69.3 / 51.6 / 71.2)."""
+    10.7 / 9.5 / 10.1, 4096 x 768 13.2 / 11.4 / 10.9; more columns leave no CUs for it: 5504 x 640 13.3 / 13.3 / 10.9), and large ones
+    above 64 rows two workgroups a CU, which hide each other's waits (8192 x 8192 43.5 / 37.0 / 41.8, 8192 x 14336 69.3 / 51.6 / 71.2)."""
     panels = (n_out + 63) // 64
     wgs = 512 if rows > 64 and n_out > 4096 and k >= (8192 if n_out <= 8192 else 4096) else 256
     step = 256 if rows > STREAM_MAX_ROWS and ((k < 2048 and n_out <= 2048) or (k < 1024 and n_out <= 4096)) else 512
@@ -269,7 +271,7 @@ def glu_split_count(n_out: int, k: int, rows: int) -> int:
     step of 64 up to 64 rows and 0.53 above, however few columns there are; slabs share it out for one launch more (epilogue / slabs /
     vendor product and GLU, us, 64 rows: 1024 x 1024 7.9 / 6.3 / 10.8, 1024 x 8192 39.0 / 10.9 / 15.9, 4096 x 4096 22.3 / 13.0 / 17.9, 8192 x 1024 8.6 / 9.9 /
     14.8; 128 rows: 512 x 512 8.6 / 7.3 / 8.7, 4096 x 4096 36.3 / 19.1 / 27.0, 8192 x 8192 67.7 / 36.5 / 50.5, 14336 x 2048 21.8 / 26.7 / 21.4, 14336 x 8192
-    68.2 / 54.6 / 65.7).  Up to 32 rows the epilogue is the faster form."""
+    68.2 / 54.6 / 65.7).  Up to 32 rows the epilogue is ahead of row-major weights at every size."""
     if rows <= STREAM_MAX_ROWS or (k < 1536 and n_out > 4096):
         return 1
     return stream_split_count(n_out, k, rows)

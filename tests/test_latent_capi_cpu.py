@@ -200,3 +200,25 @@ def test_glu_over_slabs_refuses_what_it_has_no_form_for():
 def test_slabs_of_streamed_products(N, K, M, slabs):
     from scalellm_amd import latent_kernels as lk
     assert lk.stream_split_count(N, K, M) == slabs
+
+
+def _route(monkeypatch, product, M, N, K):
+    """'stream', 'rows' or 'vendor': what serves an [M, K] x [N, K] product of weights with a streamed layout."""
+    import torch
+    from scalellm_amd import latent_kernels as lk
+    went = []
+    monkeypatch.setattr(lk, "_p", lambda t: 4096)
+    monkeypatch.setattr(lk, "_run_stream", lambda a: went.append("stream"))
+    monkeypatch.setattr(lk, "_run_linear", lambda a: went.append("rows"))
+    monkeypatch.setattr(lk, "clamped_glu", lambda *a: None)
+    monkeypatch.setattr(torch, "mm", lambda *a, **k: went.append("vendor"))
+    t = lambda *shape: torch.empty(*shape, dtype=torch.bfloat16, device="meta")  # noqa: E731
+    product(lk, t(M, K), t(N, K), t((N + 63) // 64, K // 64, 4, 2, 64, 8))
+    return went[0]
+
+
+@pytest.mark.parametrize("N,K,rows", [(6784, 4096, 32), (8128, 512, 32), (8192, 512, 64), (8192, 2048, 64), (8192, 4096, 32), (8192, 14336, 32),
+                                      (9216, 4096, 64), (9216, 8192, 32), (16896, 4096, 64), (28672, 8192, 64)])
+def test_stored_products_are_streamed_where_that_is_faster(N, K, rows, monkeypatch):
+    for M in (1, 32, 33, 64, 65):
+        assert _route(monkeypatch, lambda lk, x, w, layout: lk.linear(x, w, layout=layout), M, N, K) == ("stream" if M <= rows else "vendor"), M
