@@ -194,8 +194,10 @@ def copied_weights(layouts) -> List[torch.Tensor]:
 
 
 def slab_rows(layout: Optional[torch.Tensor]) -> int:
-    """Rows up to which a product with this streamed layout (None: row-major weights only) is left as slabs."""
-    return STREAM_MAX_ROWS if layout is None else STREAM_LAYOUT_MAX_ROWS
+    """Rows up to which a product with this streamed layout (None, or of a weight that has changed: row-major weights only) is left as slabs."""
+    if layout is None or not layout_is_current(layout, getattr(layout, "copy_of", None)):
+        return STREAM_MAX_ROWS
+    return STREAM_LAYOUT_MAX_ROWS
 
 
 def _stream_args(x, w, layout, M, N, K, rows) -> "Optional[_lib.LinearArgs]":

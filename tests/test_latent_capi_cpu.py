@@ -222,3 +222,14 @@ def _route(monkeypatch, product, M, N, K):
 def test_stored_products_are_streamed_where_that_is_faster(N, K, rows, monkeypatch):
     for M in (1, 32, 33, 64, 65):
         assert _route(monkeypatch, lambda lk, x, w, layout: lk.linear(x, w, layout=layout), M, N, K) == ("stream" if M <= rows else "vendor"), M
+
+
+def test_products_of_changed_weights_are_slabs_as_without_a_layout():
+    import torch
+    from scalellm_amd import latent_kernels as lk
+    layout = torch.empty(8, 64, 4, 2, 64, 8, dtype=torch.bfloat16, device="meta")
+    layout.copy_of = torch.zeros(1)
+    layout.copy_version = layout.copy_of._version
+    assert lk.slab_rows(layout) == 128
+    layout.copy_of.add_(1)
+    assert lk.slab_rows(layout) == lk.slab_rows(None) == 32
