@@ -683,7 +683,8 @@ __global__ void __launch_bounds__(256) gated_norm_kernel(const slm_gated_norm_ar
 
 // The same where values come in eights and lie on 16 bytes: 16-byte accesses, all loads before the sum.  PER_HEAD: VD / 8
 // lanes a head; else 256 threads a row of up to 8192.  4096 rows of 16 heads of 128:
-// per head 22.0 us -> 12.9, per row 19.9 -> 14; 32 rows of 32 heads 3.6 -> 3.2, 7.5 -> 4.0.
+// per head 22.0 us -> 12.9, per row 19.9 -> 14; 32 rows of 32 heads 3.6 -> 3.2, 7.5 -> 4.0.  Rows of fewer than 512 values leave most of its threads
+// idle and pay for registers they do not use (4096 rows: 128 values 8.2 us against 4.9 of a value a thread, 384 9.7 / 9.1): the general kernel's.
 template <typename E, int VD>
 __global__ void __launch_bounds__(256) gated_norm_heads_kernel(const slm_gated_norm_args a) {
   constexpr int L = VD / 8;
@@ -751,7 +752,7 @@ static bool gated_norm_eights(const slm_gated_norm_args& a, hipStream_t st) {
       !aligned16(a.out))
     return false;
   if (!a.per_head) {
-    if ((int64_t)a.heads * a.vdim > 8192) return false;
+    if ((int64_t)a.heads * a.vdim > 8192 || a.heads * a.vdim < 512) return false;
     gated_norm_row_kernel<E><<<dim3((unsigned)a.rows), dim3(256), 0, st>>>(a);
     return true;
   }

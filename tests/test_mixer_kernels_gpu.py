@@ -289,7 +289,7 @@ def test_window_attention_of_single_rows(rows, heads, kv_heads, dim, vdim, longe
 
 @pytest.mark.parametrize("dtype", BOTH)
 @pytest.mark.parametrize("per_head", [True, False])
-@pytest.mark.parametrize("rows,heads,vdim,shift", [(1, 1, 64, 0), (33, 3, 64, 0), (17, 5, 128, 0), (9, 32, 256, 0), (9, 33, 256, 0),
+@pytest.mark.parametrize("rows,heads,vdim,shift", [(1, 1, 64, 0), (33, 3, 64, 0), (70, 7, 64, 0), (70, 2, 256, 0), (17, 5, 128, 0), (9, 32, 256, 0), (9, 33, 256, 0),
                                                    (5, 4, 128, 4)])
 def test_gated_norm_of_eights(rows, heads, vdim, shift, per_head, dtype):
     """Workgroups that end within a row, rows of 8192 (the most registers hold) and above, a gate off its 16 bytes in bf16."""
