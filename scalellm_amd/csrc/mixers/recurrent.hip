@@ -2,7 +2,7 @@
 // per key channel, and decayed linear attention.  Everything here is fp32 besides the projections it reads.
 //
 //   step     one row per sequence: convolution, activations, unit vectors, gates, the update and (delta) the output norm
-//            in one launch.  One workgroup per (row, head); the state is read and written once, past the caches.  Bound: HBM
+//            in one launch.  One workgroup per (row, head); the state is read and written once, past the caches unless it is small.  Bound: HBM
 //            (state).  16 heads of 128 x 128: delta 128 rows 71 us with ordinary loads and stores and the inputs one after the
 //            other, 52 without (5.2 TB/s), 32 rows 18.4 and 14.1; lightning, the first alone, 128 rows 53 and 46 (5.8 TB/s), 32 rows
 //            14.4 and 12.7, 8 rows 6.0 and 5.5, 1 row 4.3 and 4.3.
@@ -114,10 +114,22 @@ __device__ __forceinline__ float decay_exponent(const slm_recurrent_args& a, int
   return a.neg_a[head] * softplus_f32(x + a.dt_bias[head * a.dim + c]);
 }
 
+// four columns of the state; ONCE: past the caches' replacement
+template <bool ONCE>
+__device__ __forceinline__ f32x4 load_state(const float* p) {
+  if constexpr (ONCE) return __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p));
+  else return *reinterpret_cast<const f32x4*>(p);
+}
+template <bool ONCE>
+__device__ __forceinline__ void store_state(float* p, f32x4 v) {
+  if constexpr (ONCE) __builtin_nontemporal_store(v, reinterpret_cast<f32x4*>(p));
+  else *reinterpret_cast<f32x4*>(p) = v;
+}
+
 // ---------------------------------------------------------------------------------------
 // step: threads = 256 per 64 columns; thread = (4 columns, row group of 16), NR rows of its group
 // ---------------------------------------------------------------------------------------
-template <typename E, int MODE, int NR>
+template <typename E, int MODE, int NR, bool ONCE>
 __global__ void __launch_bounds__(1024) recurrent_step_kernel(const slm_recurrent_args a) {
   constexpr int DK = 16 * NR;
   __shared__ float sq[DK], sk[DK], sg[DK], sv[256], red[16][64], wred[2][16];
@@ -136,7 +148,7 @@ __global__ void __launch_bounds__(1024) recurrent_step_kernel(const slm_recurren
   f32x4 s[NR];
 #pragma unroll
   for (int r = 0; r < NR; ++r)
-    s[r] = mine && p > 0 ? __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(S + (int64_t)(rg + 16 * r) * a.v_pad)) : f32x4{0.f, 0.f, 0.f, 0.f};
+    s[r] = mine && p > 0 ? load_state<ONCE>(S + (int64_t)(rg + 16 * r) * a.v_pad) : f32x4{0.f, 0.f, 0.f, 0.f};
 
   float beta = 0.f;
   if constexpr (DELTA_MODE(MODE)) {
@@ -207,7 +219,7 @@ __global__ void __launch_bounds__(1024) recurrent_step_kernel(const slm_recurren
     }
     if (mine)
 #pragma unroll
-      for (int r = 0; r < NR; ++r) __builtin_nontemporal_store(s[r], reinterpret_cast<f32x4*>(S + (int64_t)(rg + 16 * r) * a.v_pad));
+      for (int r = 0; r < NR; ++r) store_state<ONCE>(S + (int64_t)(rg + 16 * r) * a.v_pad, s[r]);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       o[j] += __shfl_xor(o[j], 16, 64);
@@ -256,7 +268,7 @@ __global__ void __launch_bounds__(1024) recurrent_step_kernel(const slm_recurren
         s[r][j] = __builtin_fmaf(k, v[j], s[r][j] * d);
         o[j] = __builtin_fmaf(q, s[r][j], o[j]);
       }
-      if (mine) __builtin_nontemporal_store(s[r], reinterpret_cast<f32x4*>(S + (int64_t)(rg + 16 * r) * a.v_pad));
+      if (mine) store_state<ONCE>(S + (int64_t)(rg + 16 * r) * a.v_pad, s[r]);
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -778,18 +790,31 @@ static bool rec_ptrs_ok(const slm_recurrent_args& a) {
   return a.low && a.conv_w && a.conv_ring && a.neg_a && a.dt_bias && a.taps >= 1;
 }
 
-template <typename E, int MODE>
-static int rec_step(const slm_recurrent_args& a, hipStream_t st) {
+// Past the caches' replacement from as many bytes of state on (past / through them, us, layers in turn over 32 MB and more; 128 x 128 heads:
+// lightning 64 KB 4.1 / 3.3, 4 MB 4.7 / 4.5, 8 MB 5.1 / 5.9; delta 256 KB 6.5 / 6.3, 1 MB 6.6 / 6.8, 4 MB 6.9 / 7.4; 256 x 256, whose registers hold
+// a wave's whole share: lightning 4 MB 9.3 / 7.7, 8 MB 9.7 / 9.0, 16 MB 10.4 / 13.2; delta 4 MB 13.1 / 12.4, 8 MB 13.4 / 15.4).
+static bool state_once(const slm_recurrent_args& a) {
+  const bool delta = DELTA_MODE(a.mode), wide = a.dim_pad == 256;
+  const int64_t least = delta ? (wide ? 8 : 0) : wide ? 16 : 8;
+  return (int64_t)a.n_single * a.heads * a.dim_pad * a.v_pad * 4 >= least << 20;
+}
+template <typename E, int MODE, bool ONCE>
+static int rec_step_of(const slm_recurrent_args& a, hipStream_t st) {
   const dim3 grid((unsigned)((int64_t)a.n_single * a.heads)), block(256 * ((a.v_pad + 63) / 64));
   hip_clear_error();
   switch (a.dim_pad / 16) {
-    case 2: recurrent_step_kernel<E, MODE, 2><<<grid, block, 0, st>>>(a); break;
-    case 4: recurrent_step_kernel<E, MODE, 4><<<grid, block, 0, st>>>(a); break;
-    case 8: recurrent_step_kernel<E, MODE, 8><<<grid, block, 0, st>>>(a); break;
-    case 12: recurrent_step_kernel<E, MODE, 12><<<grid, block, 0, st>>>(a); break;
-    default: recurrent_step_kernel<E, MODE, 16><<<grid, block, 0, st>>>(a);
+    case 2: recurrent_step_kernel<E, MODE, 2, ONCE><<<grid, block, 0, st>>>(a); break;
+    case 4: recurrent_step_kernel<E, MODE, 4, ONCE><<<grid, block, 0, st>>>(a); break;
+    case 8: recurrent_step_kernel<E, MODE, 8, ONCE><<<grid, block, 0, st>>>(a); break;
+    case 12: recurrent_step_kernel<E, MODE, 12, ONCE><<<grid, block, 0, st>>>(a); break;
+    default: recurrent_step_kernel<E, MODE, 16, ONCE><<<grid, block, 0, st>>>(a);
   }
   return hip_check_launch();
+}
+template <typename E, int MODE>
+static int rec_step(const slm_recurrent_args& a, hipStream_t st) {
+  if (state_once(a)) return rec_step_of<E, MODE, true>(a, st);
+  return rec_step_of<E, MODE, false>(a, st);
 }
 template <typename E, int MODE, int DK, int NCT>
 static void rec_scan_nct(const slm_recurrent_args& a, hipStream_t st) {
