@@ -117,6 +117,9 @@ static bool append_eights(const slm_window_append_args& a, hipStream_t st) {
     return false;
   const int64_t items = a.rows * (a.heads + 2 * (int64_t)a.kv_heads);
   if (items > (1ll << 32)) return false;
+  // (heads of 64: eight lanes a vector are a longer chain than a wave's 64, until rows fill the chip: 1 row of 1 / 1 heads 2.1 us against 2.8, 128 of 4 / 4 2.6
+  // / 3.0, 128 of 16 / 8 - 4096 vectors - 2.8 / 2.9, 128 of 32 / 8 3.1 / 2.9, 4096 of 16 / 8 23.2 / 9.0)
+  if (a.d_pad == 64 && items < 5000) return false;
   auto grid = [&](int per) { return dim3((unsigned)((items + per - 1) / per)); };
   if (a.d_pad == 64) window_append_eights_kernel<8><<<grid(32), dim3(256), 0, st>>>(a);
   else if (a.d_pad == 128) window_append_eights_kernel<16><<<grid(16), dim3(256), 0, st>>>(a);

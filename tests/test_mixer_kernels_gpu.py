@@ -347,3 +347,28 @@ def test_window_append(heads, kv, dim, d_pad, rot, v_pad, shift, dtype):
     assert torch.equal(x[:, off_k:].cpu(), proj[:, off_k:])
     rest = [i for i in range(40) if i not in slots.tolist()]
     assert (keys[rest] == 5.0).all() and (values[rest] == 5.0).all()
+
+
+@pytest.mark.parametrize("heads,kv,dim,rot,rows", [(3, 1, 64, 32, 999), (3, 1, 64, 32, 1001), (4, 4, 48, 16, 450), (16, 8, 64, 64, 700)])
+def test_window_append_of_many_narrow_heads(heads, kv, dim, rot, rows):
+    """Heads of 64 go eight columns a lane from some thousands of vectors on: the same as in smaller calls, to a rounding to bf16."""
+    from scalellm_amd import mixer_kernels as mk
+    g = torch.Generator(device=DEV).manual_seed(9)
+    rnd = lambda *shape: torch.randn(*shape, generator=g, device=DEV)  # noqa: E731
+    off_k = heads * 64
+    off_v = off_k + kv * 64
+    proj = rnd(rows, off_v + kv * 64).to(torch.bfloat16)
+    for t, n in ((proj[:, :off_k], heads), (proj[:, off_k:off_v], kv)):
+        t.view(rows, n, 64)[..., dim:] = 0.0
+    qw, kw, cs = rnd(dim), rnd(dim), rnd(50, rot)
+    pos, slots = torch.randint(0, 50, (rows,), generator=g, device=DEV).int(), torch.randperm(rows, generator=g, device=DEV).int()
+    got = []
+    for step in (rows, 100):
+        x, keys, values = proj.clone(), *(torch.full((rows, kv, 64), 5.0, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+        for r in range(0, rows, step):
+            mk.window_append(x[r:r + step], keys, values, qw, kw, cs, pos[r:r + step], slots[r:r + step], heads=heads, dim=dim, off_q=0,
+                             off_k=off_k, off_v=off_v, eps=1e-3)
+        got.append((x[:, :off_k].float(), keys.float(), values.float()))
+    assert torch.equal(got[0][2], got[1][2])
+    for a, b in zip(got[0][:2], got[1][:2]):   # (32-bit sums in another order: neighbouring bf16 values at most, 2^-7 of a value apart)
+        assert ((a - b).abs() <= 2 ** -7 * torch.maximum(a.abs(), b.abs()) + 1e-5).all() and (a - b).norm() <= 1e-3 * b.norm()
