@@ -262,21 +262,36 @@ static bool reads_once(const slm_window_attn_args& a) {
   return head_blocks(a) == 1 && a.rows * visible_keys(a) * a.kv_heads * (a.d_pad + a.v_pad) * 2 >= (64ll << 20);
 }
 // kv heads of a workgroup: as many as leave enough rows to go round (2 / 4 heads against one, 4096 keys: 8 rows x 8 heads 36.4
-// us / 38.5 against 36.2, 1 row 17.6 / 23 against 14.7; four where
-// splits of at least 128 keys leave under 400 workgroups: 64 rows x 500 keys 38.3 against 32.6 with two, 128 x 130 20.7 / 19.3, but 200 x
-// 250, 400 of them, 45.2 / 47.7)
+// us / 38.5 against 36.2, 1 row 17.6 / 23 against 14.7), and enough workgroups of splits of at least 128 keys.  Two where the chip is filled twice by
+// then, a little earlier for wide rows (16 / 8 heads of 128, one / two: 8 rows x 130 keys 7.1 / 9.9, 32 x 130 9.1 / 11.9, 8 x 500 12.9 / 16.5, 16 x 500
+// 16.6 / 18.0, 32 x 500 - 384 workgroups - 25.4 / 24.1, 128 x 130 23.1 / 19.3; 8 / 8 of 64: 32 x 500 15.3 / 17.2, 16 x 1000 16.3 / 17.7, 128 x 130 13.2 / 13.9).
+// Four from 400 on: 64 rows x 500 keys 38.3 against 32.6 with two, 128 x 130 20.7 / 19.3, but 200 x 250, 400 of them, 45.2 / 47.7.
 static int hw_shift(const slm_window_attn_args& a) {
   const int64_t pairs = a.rows * a.kv_heads, most = std::max<int64_t>(visible_keys(a) / 128, 1);
-  return a.kv_heads % 4 == 0 && pairs >= 512 && pairs / 4 * most >= 400 ? 2 : a.kv_heads % 2 == 0 && pairs >= 64 ? 1 : 0;
+  if (a.kv_heads % 4 == 0 && pairs >= 512 && pairs / 4 * most >= 400) return 2;
+  return a.kv_heads % 2 == 0 && pairs >= 64 && pairs / 2 * most >= (a.d_pad + a.v_pad >= 256 ? 384 : 512) ? 1 : 0;
 }
-// splits: about two workgroups per CU, at least 128 keys (a tile per wave) each
+// splits: two workgroups per CU, at least 128 keys (a tile per wave) each, in one round of the chip where their number allows it (24 / 3 heads, 96
+// columns of keys, 64 of values, 32 rows x 4096 keys: 5 splits, 480 workgroups, 33.7 us, 6 of them 38.0); more workgroups than CUs that
+// fill their last round badly are split further where that fills it better (100 rows x 4096, 300 workgroups: 2 splits 96 us, 4 81.8; 20 / 5
+// heads of 128, 128 x 4096: 1 250, 2 223).  Blocks of heads on one kv head read the same keys, n_splits workgroups apart: a multiple of four
+// puts them on one or two of the eight XCDs (64 / 1 heads of 128, 64 rows x 16000: 2 splits 301, 4 194; 48 x 4096 3 81.9, 4 56.3; 128 x 4096 1 157, 4
+// 122; short histories of many rows not: 256 x 1000 1 82, 4 91).
 static int split_count(const slm_window_attn_args& a) {
   if (a.n_splits > 0) return a.n_splits < 64 ? a.n_splits : 64;
-  const int64_t keys = visible_keys(a);
+  const int64_t keys = visible_keys(a), most = keys / 128;
   const int64_t wgs = a.rows * (a.kv_heads >> hw_shift(a)) * head_blocks(a);
-  const int64_t want = (512 + wgs - 1) / wgs, most = keys / 128;
-  const int64_t n = want < most ? want : most;
-  return (int)(n < 1 ? 1 : n > 64 ? 64 : n);
+  int64_t want = (512 + wgs - 1) / wgs;
+  if (head_blocks(a) > 1) {
+    if (wgs < 512 || keys >= 2048) want = (want + 3) / 4 * 4;
+  } else if (wgs <= 256) {
+    want = 512 / wgs;
+  } else {
+    const int64_t more = (1024 + wgs - 1) / wgs;
+    auto rounds = [&](int64_t n) { return (wgs * n + 511) / 512; };
+    if (10 * more * rounds(want) >= 13 * want * rounds(more)) want = more;   // (1.3 times as full)
+  }
+  return (int)std::max<int64_t>(std::min<int64_t>(std::min(want, most), 64), 1);
 }
 
 static bool wd_width(int w) { return w == 64 || w == 96 || w == 128 || w == 192 || w == 256; }

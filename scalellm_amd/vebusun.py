@@ -179,8 +179,8 @@ class VebusunStep:
     def reserve_workspaces(self, n_tokens: int) -> None:
         """Size the attention scratch for decode batches of up to n_tokens rows, before graphs are captured."""
         need = [L.mixer.left.args.heads * (L.mixer.left.v_pad + 2) * 4 for L in self.layers if isinstance(L.mixer, ParallelMixer)]
-        if need:   # (a split per spare workgroup: no more than about 1024 workgroups' worth of rows)
-            reserve_workspace(2 * max(n_tokens, 1024) * max(need), self.device)
+        if need:   # (two workgroups a CU, two rounds of them at most; four splits of a row where blocks of heads share their keys)
+            reserve_workspace(max(4 * n_tokens, 2048) * max(need), self.device)
 
     def forward(self, tokens: torch.Tensor, positions: torch.Tensor, params: InputParameters,
                 return_logits: bool = False) -> torch.Tensor:

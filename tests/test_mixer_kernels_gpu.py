@@ -251,12 +251,13 @@ def test_silu_glu(rows, dtype):
     _close(_total(layer.forward(x))[:, :W], ref.feed_forward(h, _f64(w)), dtype, 1e-5, 3e-2)
 
 
-# rows x kv heads below 64, to 512 and beyond: 1, 2 and 4 kv heads in a workgroup, 4, 2 and 1 of its waves on each; odd counts of
+# few workgroups, enough and many: 1, 2 and 4 kv heads in a workgroup, 4, 2 and 1 of its waves on each; odd counts of
 # kv heads, more than 16 query heads on one, ranges of less than a tile, of splits that get no tile, windows with kept tokens
 @pytest.mark.parametrize("rows,heads,kv_heads,dim,vdim,longest,window,keep", [
     (3, 6, 3, 64, 128, 900, 0, 0), (40, 8, 2, 128, 128, 300, 100, 7), (130, 16, 4, 96, 64, 200, 0, 0), (9, 160, 8, 128, 128, 700, 0, 0),
     (130, 20, 5, 64, 64, 65, 33, 40), (64, 8, 8, 128, 128, 1500, 1000, 16), (1, 8, 8, 128, 128, 4000, 0, 0),
-    (260, 8, 8, 64, 64, 200, 0, 0)])   # (four heads, one split)
+    (260, 8, 8, 64, 64, 200, 0, 0),    # (four heads, one split)
+    (130, 16, 8, 128, 128, 130, 0, 0), (40, 8, 2, 64, 64, 1700, 0, 0), (70, 64, 2, 64, 128, 1100, 0, 0)])   # (two heads: one split, several, blocks of heads)
 def test_window_attention_of_single_rows(rows, heads, kv_heads, dim, vdim, longest, window, keep):
     from scalellm_amd import mixer_kernels as mk
     from scalellm_amd.decode import make_batch_inputs

@@ -79,3 +79,31 @@ def test_split_plan_sizes_its_workspace():
     assert L.slm_window_attn_workspace_bytes(C.byref(b)) == 0
     b.window, b.dtype = 0, _lib.SLM_F32
     assert L.slm_window_attn_workspace_bytes(C.byref(b)) == 0
+
+
+# one round of two workgroups a CU; a better filled second one; blocks of heads on the same keys in fours
+@pytest.mark.parametrize("heads,kv_heads,d,v,rows,keys,splits", [
+    (16, 8, 128, 128, 128, 4096, 2), (16, 8, 128, 128, 32, 4096, 4), (24, 3, 96, 64, 32, 4096, 5), (24, 3, 96, 64, 8, 16000, 21), (24, 3, 96, 64, 100, 4096, 4),
+    (24, 3, 96, 64, 128, 4096, 2), (20, 5, 128, 128, 128, 4096, 2), (20, 5, 128, 128, 100, 4096, 2), (8, 1, 256, 256, 1, 300, 2), (64, 1, 128, 128, 32, 4096, 4),
+    (64, 1, 128, 128, 64, 16000, 4), (64, 1, 128, 128, 128, 4096, 4), (64, 1, 128, 128, 256, 1000, 1), (128, 2, 128, 128, 48, 4096, 4)])
+def test_splits_of_window_attention(heads, kv_heads, d, v, rows, keys, splits):
+    b = _lib.WindowAttnArgs()
+    for name in "q key_cache value_cache out positions q_cu block_table block_cu".split():
+        setattr(b, name, 4096)
+    b.rows, b.batch, b.heads, b.kv_heads, b.d_pad, b.v_pad, b.block_size, b.dtype, b.max_kv_len = rows, rows, heads, kv_heads, d, v, 64, _lib.SLM_BF16, keys
+    assert _lib.mixers_lib().slm_window_attn_workspace_bytes(C.byref(b)) == (rows * heads * splits * (v + 2) * 4 if splits > 1 else 0)
+
+
+def test_scratch_reserved_for_window_attention_holds_every_plan():
+    """VebusunStep.reserve_workspaces() before graphs of up to n rows: max(4 n, 2048) rows of partials of every head."""
+    b = _lib.WindowAttnArgs()
+    for name in "q key_cache value_cache out positions q_cu block_table block_cu".split():
+        setattr(b, name, 4096)
+    b.block_size, b.dtype = 64, _lib.SLM_BF16
+    for heads, kv_heads in ((1, 1), (16, 8), (24, 3), (20, 5), (32, 2), (64, 1), (128, 2), (160, 8)):
+        for keys in (100, 1000, 2048, 4096, 100000):
+            for rows in (1, 2, 7, 31, 64, 100, 129, 200, 256, 300, 400, 511, 512, 600, 700, 1024, 2000):
+                b.rows = b.batch = rows
+                b.heads, b.kv_heads, b.d_pad, b.v_pad, b.max_kv_len = heads, kv_heads, 128, 128, keys
+                need = _lib.mixers_lib().slm_window_attn_workspace_bytes(C.byref(b))
+                assert need <= max(4 * rows, 2048) * heads * 130 * 4, (heads, kv_heads, keys, rows)
