@@ -362,6 +362,15 @@ SLM_API int slm_rms_norm(void* out, const void* x, const void* weight, void* res
 SLM_API int slm_rms_norm_splitk(void* out, const float* partials /* [n_splits, n_tokens, dim] */,
                                 int32_t n_splits, const void* weight, void* residual,
                                 int64_t n_tokens, int64_t dim, float eps, int32_t dtype, void* stream);
+/* resid[t] = table[tokens[t]] (negative ids count from the table's end, ids outside it give NaN) and, where
+ * normed != NULL, normed = rms_norm(resid) * weight as slm_rms_norm gives it (EmbeddingImpl and the first
+ * input norm, src/models/meta/llama.h:204-216).  table [vocab, dim] T, contiguous rows everywhere. */
+SLM_API int slm_embed_norm(void* resid, void* normed, const void* table, const int32_t* tokens, const void* weight,
+                           int64_t n_tokens, int64_t dim, int64_t vocab, float eps, int32_t dtype, void* stream);
+/* out[i] = x[ends[i] - 1], 16-bit rows of dim: the last row of every sequence (ends = q_cu_seq_lens + 1);
+ * x has n_rows rows, an end outside 1 .. n_rows gives NaN */
+SLM_API int slm_last_rows(void* out, const void* x, const int32_t* ends, int64_t n, int64_t n_rows, int64_t dim,
+                          void* stream);
 /* LayerNorm with weight and optional bias (bias == NULL: none), fp32 statistics, one rounding:
  * out = T((x - mean) * rsqrt(var + eps) * weight + bias).  replaces kernel::layer_norm
  * (src/kernels/layernorm_kernels.cu:185-256; LayerNormImpl::forward src/layers/normalization.h:86-95)

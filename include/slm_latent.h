@@ -34,14 +34,14 @@ typedef struct slm_residual_norm_args {
   const int32_t* positions; /* EMBED with a position table: [rows]                                      */
   const void* embed;        /* EMBED: [vocab, ld_embed] of dtype                                        */
   const void* pos_table;    /* EMBED: [max_positions, width] of dtype, or NULL                          */
-  const int32_t* row_index; /* NULL, or [rows]: output row r is made of stream row row_index[r] (PLAIN) */
+  const int32_t* row_index; /* NULL, or [rows]: output row r is made of stream row row_index[r] + row_shift (PLAIN) */
   const float* weight;      /* [width] fp32; NULL: only the sum, no norm                                */
   const float* bias;        /* TANH: [width] fp32                                                       */
   void* out;                /* [rows, ld_out] of dtype; columns width .. ld_out-1 are zeroed            */
   int64_t rows, width, ld_delta, ld_embed, ld_out, slab_stride;
   float eps, norm_alpha;
   float delta_mult;         /* factor of what is added: the delta, or the embedding row                 */
-  int32_t n_slabs, mode, dtype, norm;
+  int32_t n_slabs, mode, dtype, norm, row_shift;
 } slm_residual_norm_args;
 enum { SLM_NORM_RMS = 0, SLM_NORM_TANH = 1 };
 enum { SLM_RN_EMBED = 0, SLM_RN_ADD = 1, SLM_RN_SLABS = 2, SLM_RN_PLAIN = 3 };

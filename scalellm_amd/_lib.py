@@ -162,6 +162,11 @@ def lib() -> C.CDLL:
         ("slm_rms_norm", C.c_int,
          [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int64, C.c_int64, C.c_float,
           C.c_int32, C.c_void_p]),
+        ("slm_embed_norm", C.c_int,
+         [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int64, C.c_int64, C.c_int64, C.c_float,
+          C.c_int32, C.c_void_p]),
+        ("slm_last_rows", C.c_int,
+         [C.c_void_p, C.c_void_p, C.c_void_p, C.c_int64, C.c_int64, C.c_int64, C.c_void_p]),
         ("slm_rope_kv_append", C.c_int,
          [C.c_void_p, C.c_int64, C.c_void_p, C.c_int64, C.c_void_p, C.c_int64, C.c_void_p,
           C.c_void_p, C.c_int32, C.c_int32, C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p,
@@ -219,7 +224,7 @@ class ResidualNormArgs(C.Structure):
     """slm_residual_norm_args."""
     _fields_ = _fields((C.c_void_p, "resid delta slabs tokens positions embed pos_table row_index weight bias out"),
                        (C.c_int64, "rows width ld_delta ld_embed ld_out slab_stride"),
-                       (C.c_float, "eps norm_alpha delta_mult"), (C.c_int32, "n_slabs mode dtype norm"))
+                       (C.c_float, "eps norm_alpha delta_mult"), (C.c_int32, "n_slabs mode dtype norm row_shift"))
 
 
 NORM_RMS, NORM_TANH = range(2)

@@ -15,6 +15,8 @@
 //  slm_gelu            <- kernel::gelu_new / gelu_fast and their *_with_mul forms
 //                         (src/kernels/activation_kernels.cu:20-40, 111-145; CPU path
 //                         src/layers/activation.cpp:24-34, 57-65).
+#include <type_traits>
+
 #include "common.h"
 
 namespace slm {
@@ -89,6 +91,66 @@ __global__ void __launch_bounds__(256) rms_norm_kernel(uint16_t* __restrict__ ou
       *reinterpret_cast<u32x4*>(out + tok * dim + vi * 8) = o;
     }
   }
+}
+
+// Rows of the embedding table by token id into the residual stream, and their RMSNorm (normed may be NULL: the stream
+// only) as rms_norm_kernel computes it.  One workgroup per token; bound: latency.  In front of a decode step torch's own form is
+// four launches (ids widened, gather, copy, norm).  Ids count from the end of the table where they are negative, as
+// torch's indexing has them; an id outside the table gives a row of NaN.
+template <typename T, int NV>
+__global__ void __launch_bounds__(256) embed_norm_kernel(uint16_t* __restrict__ resid, uint16_t* __restrict__ normed,
+                                                         const uint16_t* __restrict__ table, const int* __restrict__ tokens,
+                                                         const uint16_t* __restrict__ weight, int64_t dim, int64_t vocab, float eps) {
+  __shared__ float red[4];
+  const int64_t tok = blockIdx.x;
+  const int tid = threadIdx.x;
+  const int64_t nvec = dim / 8;
+  int64_t id = tokens[tok];
+  if (id < 0) id += vocab;
+  const bool known = id >= 0 && id < vocab;
+  if (!known) id = 0;
+  u32x4 a[NV], wv[NV];
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int64_t vic = min((int64_t)tid + 256 * i, nvec - 1);
+    if (normed) wv[i] = *reinterpret_cast<const u32x4*>(weight + vic * 8);
+    a[i] = *reinterpret_cast<const u32x4*>(table + id * dim + vic * 8);
+    if (!known) a[i] = u32x4{0x7fff7fffu, 0x7fff7fffu, 0x7fff7fffu, 0x7fff7fffu};
+  }
+  float v[NV][8];
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int64_t vi = tid + 256 * i;
+    const float f[8] = {lo_f32<T>(a[i].x), hi_f32<T>(a[i].x), lo_f32<T>(a[i].y), hi_f32<T>(a[i].y),
+                        lo_f32<T>(a[i].z), hi_f32<T>(a[i].z), lo_f32<T>(a[i].w), hi_f32<T>(a[i].w)};
+    if (vi < nvec) {
+      *reinterpret_cast<u32x4*>(resid + tok * dim + vi * 8) = a[i];
+      ss = rms_sumsq8(f, ss);
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[i][j] = f[j];
+  }
+  if (!normed) return;  // (uniform)
+  ss = wave_sum64(ss);
+  if ((tid & 63) == 0) red[tid >> 6] = ss;
+  __syncthreads();
+  const float rs = rsqrtf((red[0] + red[1] + red[2] + red[3]) / (float)dim + eps);
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int64_t vi = tid + 256 * i;
+    if (vi < nvec) *reinterpret_cast<u32x4*>(normed + tok * dim + vi * 8) = rms_apply8<T>(v[i], rs, wv[i]);
+  }
+}
+
+// out[i] = x[ends[i] - 1]: the last row of every sequence, whose bounds are `ends` (16 bits; torch: ends - 1, widened, gathered)
+__global__ void __launch_bounds__(256) last_rows_kernel(uint16_t* __restrict__ out, const uint16_t* __restrict__ x,
+                                                        const int* __restrict__ ends, int64_t n_rows, int64_t dim) {
+  const int64_t row = (int64_t)ends[blockIdx.x] - 1;
+  const bool known = row >= 0 && row < n_rows;
+  const u32x4* src = reinterpret_cast<const u32x4*>(x + (known ? row : 0) * dim);
+  u32x4* dst = reinterpret_cast<u32x4*>(out + (int64_t)blockIdx.x * dim);
+  for (int64_t i = threadIdx.x; i < dim / 8; i += 256) dst[i] = known ? src[i] : u32x4{0x7fff7fffu, 0x7fff7fffu, 0x7fff7fffu, 0x7fff7fffu};
 }
 
 // (a, b) rotated by (cos, sin): ONE spelling for every RoPE kernel (explicit fma, so the compiler's
@@ -469,6 +531,41 @@ SLM_API int slm_rms_norm_splitk(void* out, const float* partials, int32_t n_spli
   if (n_tokens != 0 && !partials) return SLM_ERR_INVALID_ARG;
   return rms_norm_launch(out, nullptr, partials, n_splits, weight, residual, n_tokens, dim, eps, dtype,
                          stream);
+}
+
+SLM_API int slm_embed_norm(void* resid, void* normed, const void* table, const int32_t* tokens, const void* weight,
+                           int64_t n_tokens, int64_t dim, int64_t vocab, float eps, int32_t dtype, void* stream) {
+  if (n_tokens == 0) return SLM_OK;
+  if (!resid || !table || !tokens || (normed && !weight) || n_tokens < 0 || vocab < 1) return SLM_ERR_INVALID_ARG;
+  if (dim <= 0 || dim % 8 || dim > 16384 || n_tokens > 0x7fffffff) return SLM_ERR_UNSUPPORTED;
+  if (!aligned16(resid) || !aligned16(normed) || !aligned16(table) || !aligned16(weight)) return SLM_ERR_ALIGNMENT;
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  hip_clear_error();
+  const int64_t per_thread = (dim / 8 + 255) / 256;
+  auto launch = [&](auto tag, auto nv) {
+    embed_norm_kernel<decltype(tag), decltype(nv)::value><<<dim3((unsigned)n_tokens), dim3(256), 0, st>>>(
+        (uint16_t*)resid, (uint16_t*)normed, (const uint16_t*)table, tokens, (const uint16_t*)weight, dim, vocab, eps);
+  };
+  auto by_width = [&](auto tag) {
+    if (per_thread <= 1) launch(tag, std::integral_constant<int, 1>{});
+    else if (per_thread <= 2) launch(tag, std::integral_constant<int, 2>{});
+    else if (per_thread <= 4) launch(tag, std::integral_constant<int, 4>{});
+    else launch(tag, std::integral_constant<int, 8>{});
+  };
+  if (dtype == SLM_BF16) by_width(bf16_tag{});
+  else if (dtype == SLM_F16) by_width(f16_tag{});
+  else return SLM_ERR_UNSUPPORTED;
+  return hip_check_launch();
+}
+
+SLM_API int slm_last_rows(void* out, const void* x, const int32_t* ends, int64_t n, int64_t n_rows, int64_t dim, void* stream) {
+  if (n == 0) return SLM_OK;
+  if (!out || !x || !ends || n < 0 || n_rows < 1) return SLM_ERR_INVALID_ARG;
+  if (dim <= 0 || dim % 8 || n > 0x7fffffff) return SLM_ERR_UNSUPPORTED;
+  if (!aligned16(out) || !aligned16(x)) return SLM_ERR_ALIGNMENT;
+  hip_clear_error();
+  last_rows_kernel<<<dim3((unsigned)n), dim3(256), 0, reinterpret_cast<hipStream_t>(stream)>>>((uint16_t*)out, (const uint16_t*)x, ends, n_rows, dim);
+  return hip_check_launch();
 }
 
 SLM_API int slm_rope_kv_append(void* q, int64_t q_token_stride, void* k, int64_t k_token_stride,

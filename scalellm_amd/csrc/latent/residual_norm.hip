@@ -33,7 +33,7 @@ __global__ void __launch_bounds__(T) residual_norm_kernel(const slm_residual_nor
   const int tid = threadIdx.x;
   const int64_t row = blockIdx.x;
   const int width = (int)a.width;
-  const int64_t src_row = (MODE == SLM_RN_PLAIN && a.row_index) ? a.row_index[row] : row;
+  const int64_t src_row = (MODE == SLM_RN_PLAIN && a.row_index) ? a.row_index[row] + a.row_shift : row;
   float* r = a.resid + src_row * a.width;
   const E* e0 = nullptr;
   const E* e1 = nullptr;

@@ -165,8 +165,9 @@ class DagupelStep:
         first = self.layers[0].norm1 if self.layers else None
         lk.residual_norm(resid, h, first, c.eps, embed=(tokens, self.table, positions, self.pos_table))
         n = len(self.layers)
+        rows = lk.wanted_rows(params, T if n else 0)   # (None: the last sum's launch norms them too)
         for i, L in enumerate(self.layers):
-            nxt = self.layers[i + 1].norm1 if i + 1 < n else None
+            nxt = self.layers[i + 1].norm1 if i + 1 < n else self.final_norm if rows is None else None
             delta = L.attn.forward(h, positions, self.caches[i], params)
             if L.mlp is not None:
                 lk.residual_norm(resid, h, L.norm2, c.eps, delta=delta)
@@ -174,13 +175,13 @@ class DagupelStep:
             lk.residual_norm(resid, h, nxt, c.eps, delta=delta)
             if self.on_layer is not None:
                 self.on_layer(i, resid)
-        rows = params.logit_rows
-        if rows is None:
-            rows = params.q_cu_seq_lens[1:] - 1
-        out = torch.empty(rows.numel(), self.k_width, dtype=self.dtype, device=self.device)
-        if rows.numel() == 0:
-            return torch.empty(0, c.vocab, dtype=torch.float32, device=self.device)
-        lk.residual_norm(resid, out, self.final_norm, c.eps, row_index=rows)
+        out = h
+        if rows is not None:
+            index, shift = rows
+            if index.numel() == 0:
+                return torch.empty(0, c.vocab, dtype=torch.float32, device=self.device)
+            out = torch.empty(index.numel(), self.k_width, dtype=self.dtype, device=self.device)
+            lk.residual_norm(resid, out, self.final_norm, c.eps, row_index=index, row_shift=shift)
         logits = lk.linear_f32(out, self.table, c.logit_scale, self.l_table)[:, :c.vocab]
         if return_logits:
             return logits

@@ -343,7 +343,7 @@ class LlamaDecodeStep:
     # ------------------------------------------------------------------------------------------
     class _Lane:
         __slots__ = ("idx", "r0", "r1", "T", "positions", "params", "resid", "alt", "normed", "qkv",
-                     "attn", "act", "gate_up", "o_buf", "down_buf", "pend", "fold", "stream", "q", "ar")
+                     "attn", "act", "gate_up", "o_buf", "down_buf", "pend", "fold", "stream", "q", "ar", "normed_in")
 
     def _tp_lanes_ok(self) -> bool:
         """May a tensor-parallel rank run its reductions on two streams at once?"""
@@ -593,6 +593,9 @@ class LlamaDecodeStep:
         ln.pend = self._reduce_add_norm(ln, 1, delta, nxt, L["down"].deferred if defer else None)
 
     def _first_norm(self, ln) -> None:
+        if ln.normed_in:   # (the embedding's launch did it)
+            ln.pend = None
+            return
         # A norm that has not run yet: (x, deferred slabs of x or None, residual or None, weight).
         # It either folds into the projection that consumes it (_norm_then) or runs on its own.
         ln.pend = (ln.resid, None, None, self.layers[0]["in_norm"])
@@ -645,11 +648,30 @@ class LlamaDecodeStep:
         join.record(side)
         main.wait_event(join)
 
-    def _run_layers(self, T: int, positions, params: InputParameters, o_buf, down_buf, ar) -> None:
-        """The decoder stack over rows [0, T) of the static buffers (residual stream in buf["resid"]): one lane
-        or two, final norm included -- everything of a step between the embedding and the lm_head."""
-        fold = self.fold_norm and self.pa.world_size == 1 and T <= 4
+    def _folds(self, T: int) -> bool:
+        """Do the norms of a step of T rows run in the prologues of the projections behind them?"""
+        return self.fold_norm and self.pa.world_size == 1 and T <= 4
+
+    def _embed(self, tokens: torch.Tensor, resid: torch.Tensor, normed: torch.Tensor) -> bool:
+        """resid = embed[tokens]; where the first norm does not fold into its projection, that too (True).  One launch on a
+        single rank; tables and ids that its kernel does not take go through torch."""
+        s, table = self.shape, self.embed
+        weight = self.layers[0]["in_norm"] if self.layers and not self._folds(tokens.numel()) else None
+        if (tokens.dtype != torch.int32 or not tokens.is_contiguous() or not table.is_contiguous() or table.dtype != resid.dtype or
+                table.shape != (s.vocab, s.hidden) or s.hidden % 8 or s.hidden > 16384 or table.data_ptr() % 16 or
+                (weight is not None and (weight.dtype != table.dtype or not weight.is_contiguous() or weight.data_ptr() % 16))):
+            resid.copy_(table[tokens.long()])
+            return False
+        kernels.embed_norm(resid, normed if weight is not None else None, table, tokens, weight, s.rms_eps)
+        return weight is not None
+
+    def _run_layers(self, T: int, positions, params: InputParameters, o_buf, down_buf, ar, normed_in: bool = False) -> None:
+        """The decoder stack over rows [0, T) of the static buffers (residual stream in buf["resid"], with normed_in its
+        first norm in buf["normed"]): one lane or two, final norm included -- everything of a step between the embedding and the lm_head."""
+        fold = self._folds(T)
         lanes = self._make_lanes(T, positions, params, o_buf, down_buf, ar, fold)
+        for ln in lanes:
+            ln.normed_in = normed_in
         self.last_lanes = len(lanes)
         if len(lanes) == 2:
             self._run_two_lanes(lanes[0], lanes[1])
@@ -678,7 +700,9 @@ class LlamaDecodeStep:
                 params = dataclasses.replace(params, kv_total_len=total)
         resid, normed = b["resid"][:T], b["normed"][:T]
         ar = self.custom_ar if pa.world_size > 1 else None
-        x = self.embed[tokens.long()]
+        normed_in = False
+        if pa.world_size > 1:
+            x = self.embed[tokens.long()]
         if ar is not None:
             # hidden-sharded embedding gather (embedding.h:74-81) as a SUM of disjoint column
             # slices through the fused all-reduce's plain mode: exact, and keeps the captured step
@@ -694,15 +718,22 @@ class LlamaDecodeStep:
         else:
             if pa.world_size > 1:
                 from .model_parallel import gather_from_model_parallel_region
-                x = gather_from_model_parallel_region(x, pa)
-            resid.copy_(x)
+                resid.copy_(gather_from_model_parallel_region(x, pa))
+            else:
+                normed_in = self._embed(tokens, resid, normed)
             o_buf, down_buf = b["o"][:T], b["down"][:T]
 
-        self._run_layers(T, positions, params, o_buf, down_buf, ar)
-        last = (params.q_cu_seq_lens[1:] - 1).long()
-        self.last_hidden = normed[last]  # final-norm output of each sequence's last token (tests)
+        self._run_layers(T, positions, params, o_buf, down_buf, ar, normed_in)
+        # final-norm output of each sequence's last token: all rows where every sequence brings one (what _lane_split relies on too)
+        q_cu = params.q_cu_seq_lens
+        if params.q_max_seq_len == 1 and T == q_cu.numel() - 1:
+            self.last_hidden = normed
+        elif q_cu.dtype == torch.int32 and q_cu.is_contiguous() and s.hidden % 8 == 0:
+            self.last_hidden = kernels.last_rows(normed, q_cu)
+        else:
+            self.last_hidden = normed[(q_cu[1:] - 1).long()]
         logits = self.last_hidden @ self.lm_head  # plain library GEMM (hipBLASLt): not on the graded path
-        if ar is not None and not return_logits and last.numel() <= ar.max_tokens \
+        if ar is not None and not return_logits and self.last_hidden.size(0) <= ar.max_tokens \
                 and 4 * pa.world_size <= s.hidden:
             return self._greedy_over_vocab_shards(logits, ar)
         if pa.world_size > 1:

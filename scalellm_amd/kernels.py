@@ -787,6 +787,38 @@ def rms_norm(out: torch.Tensor, x: torch.Tensor, weight: torch.Tensor, eps: floa
           "slm_rms_norm")
 
 
+def embed_norm(resid: torch.Tensor, normed: Optional[torch.Tensor], table: torch.Tensor, tokens: torch.Tensor,
+               weight: Optional[torch.Tensor], eps: float) -> None:
+    """resid = table[tokens] and, unless normed is None, normed = rms_norm(resid) * weight, in one launch."""
+    _require_gpu(resid, normed, table, tokens, weight)
+    n, dim = tokens.numel(), table.size(1)
+    for t in (resid, normed, table, tokens, weight):
+        if t is not None and not t.is_contiguous():
+            raise SlmError("embed_norm needs contiguous tensors")
+    if tokens.dtype != torch.int32 or resid.shape != (n, dim) or resid.dtype != table.dtype:
+        raise SlmError("embed_norm: int32 tokens [n], resid [n, dim] of the table's dtype")
+    if normed is not None and (normed.shape != resid.shape or normed.dtype != table.dtype or weight is None or
+                               weight.numel() != dim or weight.dtype != table.dtype):
+        raise SlmError("embed_norm: normed [n, dim] and weight [dim] of the table's dtype")
+    check(_lib.lib().slm_embed_norm(resid.data_ptr(), normed.data_ptr() if normed is not None else None, table.data_ptr(),
+                                    tokens.data_ptr(), weight.data_ptr() if weight is not None else None, n, dim,
+                                    table.size(0), float(eps), _dtype_code(table), _stream()), "slm_embed_norm")
+
+
+def last_rows(x: torch.Tensor, q_cu_seq_lens: torch.Tensor) -> torch.Tensor:
+    """x [rows, dim] (16-bit) at the last row of every sequence: x[q_cu_seq_lens[1:] - 1], in one launch."""
+    _require_gpu(x, q_cu_seq_lens)
+    _dtype_code(x)
+    n = q_cu_seq_lens.numel() - 1
+    if not x.is_contiguous() or q_cu_seq_lens.dtype != torch.int32 or not q_cu_seq_lens.is_contiguous():
+        raise SlmError("last_rows: contiguous rows, contiguous int32 q_cu_seq_lens")
+    out = torch.empty(n, x.size(1), dtype=x.dtype, device=x.device)
+    if n:
+        check(_lib.lib().slm_last_rows(out.data_ptr(), x.data_ptr(), q_cu_seq_lens.data_ptr() + 4, n, x.size(0), x.size(1),
+                                       _stream()), "slm_last_rows")
+    return out
+
+
 def layer_norm(out: torch.Tensor, x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor],
                eps: float) -> None:
     """kernel::layer_norm (layernorm_kernels.cu:231-256): out = T((x - mean) * rsqrt(var + eps) * weight

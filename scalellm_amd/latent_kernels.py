@@ -68,11 +68,12 @@ class Slabs:
 
 
 def residual_norm(resid: torch.Tensor, out: Optional[torch.Tensor], weight, eps: float,
-                  delta=None, embed=None, row_index: Optional[torch.Tensor] = None, mult: float = 1.0) -> None:
+                  delta=None, embed=None, row_index: Optional[torch.Tensor] = None, mult: float = 1.0,
+                  row_shift: int = 0) -> None:
     """resid (fp32 [rows, width]) += mult * delta (a [rows, >= width] tensor or Slabs), or
     resid = mult * (table[tokens] (+ pos[positions])) for embed = (tokens, table, positions, pos); then
     out = rms_norm(resid) * weight, or a TanhNorm given as weight, zero padded to out's width.  weight = None: the sum only.
-    row_index: out row r is the norm of stream row row_index[r]; nothing is added."""
+    row_index: out row r is the norm of stream row row_index[r] + row_shift; nothing is added."""
     a = _lib.ResidualNormArgs()
     rows, width = resid.shape
     _need(resid.dtype == torch.float32 and resid.is_contiguous(), "residual_norm: resid is contiguous fp32")
@@ -103,7 +104,7 @@ def residual_norm(resid: torch.Tensor, out: Optional[torch.Tensor], weight, eps:
             _need(out is not None, "residual_norm: row_index needs an output")
             rows = out.size(0)
             _i32(row_index, rows, "row_index")
-            a.row_index = _p(row_index)
+            a.row_index, a.row_shift = _p(row_index), row_shift
     a.rows = rows
     if isinstance(weight, TanhNorm):
         t, weight = weight, weight.weight
@@ -116,6 +117,17 @@ def residual_norm(resid: torch.Tensor, out: Optional[torch.Tensor], weight, eps:
         _need(out.stride(0) == out.size(1), "residual_norm: out rows are contiguous")
     a.dtype = _code(ref) if ref is not None else SLM_F32
     latent_check(_lib.latent_lib().slm_residual_norm(C.byref(a), _stream()), "slm_residual_norm")
+
+
+def wanted_rows(params, T: int):
+    """Which stream rows a step's logits are of: None for every row (each sequence brings one), else (index tensor, what to add to it):
+    params.logit_rows, by default the last row of every sequence."""
+    if params.logit_rows is not None:
+        return params.logit_rows, 0
+    q_cu = params.q_cu_seq_lens
+    if params.q_max_seq_len == 1 and T == q_cu.numel() - 1 > 0:
+        return None
+    return (q_cu[1:], -1) if q_cu.is_contiguous() else (q_cu[1:] - 1, 0)
 
 
 def _linear_args(x, w, M, N, K) -> "_lib.LinearArgs":

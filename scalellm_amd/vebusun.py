@@ -190,9 +190,10 @@ class VebusunStep:
         resid = torch.empty(T, c.width, dtype=torch.float32, device=self.device)
         h = torch.empty(T, self.k_width, dtype=self.dtype, device=self.device)
         n = len(self.layers)
+        rows = lk.wanted_rows(params, T if n else 0)   # (None: the last sum's launch norms them too)
         lk.residual_norm(resid, h, self.layers[0].norm1 if n else None, c.eps, embed=(tokens, self.embed, None, None), mult=c.embedding_scale)
         for i, L in enumerate(self.layers):
-            nxt = self.layers[i + 1].norm1 if i + 1 < n else None
+            nxt = self.layers[i + 1].norm1 if i + 1 < n else self.final_norm if rows is None else None
             delta = L.mixer.forward(h, positions, self.caches[i], params)
             if L.mlp is not None:
                 lk.residual_norm(resid, h, L.norm2, c.eps, delta=delta, mult=c.residual_mult)
@@ -200,12 +201,12 @@ class VebusunStep:
             lk.residual_norm(resid, h, nxt, c.eps, delta=delta, mult=c.residual_mult)
             if self.on_layer is not None:
                 self.on_layer(i, resid)
-        rows = params.logit_rows
-        if rows is None:
-            rows = params.q_cu_seq_lens[1:] - 1
-        if rows.numel() == 0:
-            return torch.empty(0, c.vocab, dtype=torch.float32, device=self.device)
-        out = torch.empty(rows.numel(), self.k_width, dtype=self.dtype, device=self.device)
-        lk.residual_norm(resid, out, self.final_norm, c.eps, row_index=rows)
+        out = h
+        if rows is not None:
+            index, shift = rows
+            if index.numel() == 0:
+                return torch.empty(0, c.vocab, dtype=torch.float32, device=self.device)
+            out = torch.empty(index.numel(), self.k_width, dtype=self.dtype, device=self.device)
+            lk.residual_norm(resid, out, self.final_norm, c.eps, row_index=index, row_shift=shift)
         logits = lk.linear_f32(out, self.head, layout=self.l_head)[:, :c.vocab]
         return logits if return_logits else torch.argmax(logits, dim=-1).to(torch.int32)

@@ -316,6 +316,23 @@ def test_llama_step_through_the_same_engine():
     assert [x[0] for x in outs[0]] == [x[0] for x in outs[1]]
 
 
+@pytest.mark.parametrize("design", ["dagupel", "vebusun"])
+def test_logits_of_last_rows_by_default(design):
+    """Steps that name no rows give the last row of every sequence, bit for bit what naming those rows gives: decode steps (whose
+    last sum norms every row), steps with portions in them, and both together."""
+    from .vebusun_common import CONFIGS as VEBUSUN
+    from .vebusun_common import weights as vebusun_weights
+    cfg = CONFIGS["wide"][0] if design == "dagupel" else VEBUSUN["wide"]
+    t = weights(cfg, 11, CONFIGS["wide"][1]) if design == "dagupel" else vebusun_weights(cfg, 11)
+    engines = [_engine(cfg, t, torch.bfloat16) for _ in range(2)]
+    tokens = np.random.default_rng(3).integers(0, cfg["vocab"], 60).tolist()
+    seqs = [[_seq(n, tokens[i:i + 50]) for i, n in enumerate("abc")] for _ in engines]
+    for lens in ((1, 5, 17), (1, 1, 1), (1, 1, 2), (1, 1, 1), (1, 1, 20)):
+        named = {i: [n - 1] for i, n in enumerate(lens)}
+        got = [e.run_entries(list(zip(s, lens)), rows)[1] for e, s, rows in zip(engines, seqs, (None, named))]
+        assert got[0].shape == (3, cfg["vocab"]) and torch.equal(*got), lens
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 def test_trace_replay_program(tmp_path, dtype):
     cfg, t, tokens, want = _model("odd")

@@ -238,3 +238,35 @@ def test_layer_norm_and_gelu_reject_what_they_do_not_cover():
         kernels.gelu_new(x)
     with pytest.raises(kernels.SlmError):
         kernels.layer_norm(torch.empty(4, 96, device=DEV, dtype=torch.bfloat16), x[:, :96], w[:96], None, 1e-5)  # not contiguous
+
+
+# widths at the edges of a workgroup's vectors (2048 columns each); ids from both ends of the table.  The stream is a copy and
+# the norm rms_norm's own arithmetic: bit for bit.
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("tokens,dim", [(1, 8), (3, 2048), (5, 2056), (130, 4096), (2, 8200), (1, 16384)])
+def test_embedding_and_first_norm(tokens, dim, dtype):
+    from scalellm_amd import kernels
+    g = torch.Generator(device=DEV).manual_seed(dim)
+    table = torch.randn(50, dim, device=DEV, dtype=dtype, generator=g)
+    w = (1 + 0.1 * torch.randn(dim, device=DEV, generator=g)).to(dtype)
+    ids = torch.randint(-50, 50, (tokens,), device=DEV, generator=g, dtype=torch.int32)
+    ids[0] = 49
+    want, normed_want = table[ids.long()], torch.empty(tokens, dim, device=DEV, dtype=dtype)
+    kernels.rms_norm(normed_want, want, w, 1e-5)
+    resid, normed = torch.zeros_like(want), torch.zeros_like(want)
+    kernels.embed_norm(resid, normed, table, ids, w, 1e-5)
+    assert torch.equal(resid, want) and torch.equal(normed, normed_want)
+    resid.zero_()
+    kernels.embed_norm(resid, None, table, ids, None, 1e-5)
+    assert torch.equal(resid, want)
+    ids[-1] = 50   # no row of the table
+    kernels.embed_norm(resid, normed, table, ids, w, 1e-5)
+    assert resid[-1].isnan().all() and normed[-1].isnan().all() and torch.equal(resid[:-1], want[:-1])
+
+
+@pytest.mark.parametrize("lens,dim", [([1], 8), ([3, 1, 7], 2048), ([1, 1, 1], 4104)])
+def test_last_rows(lens, dim):
+    from scalellm_amd import kernels
+    x = torch.randn(sum(lens), dim, device=DEV).to(torch.bfloat16)
+    q_cu = torch.tensor([0, *np.cumsum(lens)], dtype=torch.int32, device=DEV)
+    assert torch.equal(kernels.last_rows(x, q_cu), x[(q_cu[1:] - 1).long()])

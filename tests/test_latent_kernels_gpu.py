@@ -71,6 +71,16 @@ def test_residual_norm_modes(rows, width, dtype):
     _close(out[:, :width], ref.rms_norm(x[[rows - 1, 0, rows // 2]], _f64(w), eps), dtype)
 
 
+def test_residual_norm_of_rows_before_the_named_ones():
+    lk = _lk()
+    resid, w = _rnd(1, 9, 256), _rnd(2, 256)
+    picked, shifted = torch.empty(3, 256, device=DEV), torch.empty(3, 256, device=DEV)
+    ends = torch.tensor([0, 3, 4, 9], dtype=torch.int32, device=DEV)
+    lk.residual_norm(resid, picked, w, 1e-5, row_index=ends[1:] - 1)
+    lk.residual_norm(resid, shifted, w, 1e-5, row_index=ends[1:], row_shift=-1)
+    assert torch.equal(picked, shifted)
+
+
 def test_eps_is_inside_the_root():
     lk = _lk()
     x = torch.full((1, 64), 1e-3, device=DEV)
