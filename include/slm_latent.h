@@ -69,6 +69,11 @@ SLM_API int slm_linear(const slm_linear_args* a, void* stream);
 SLM_API int slm_linear_stream(const slm_linear_args* a, void* stream);
 /* lays contiguous w [N, K] bf16 out so: out holds ceil(N / 64) * 64 * K elements                         */
 SLM_API int slm_stream_layout(void* out, const void* w, int64_t N, int64_t K, int32_t glu, void* stream);
+/* The same for many rows in bf16, batch 1, STORE or GLU, rows of x, w and y on 16 bytes, x and w below 2 GB: tiles of  */
+/* up to 256 x 256.  tile: -1 or an index of the tiles (tests); slices: 0 as many as pay, n: the tiles of the   */
+/* last round are cut in K by n.  Without the workspace (optional, content does not matter) nothing is cut.     */
+SLM_API size_t slm_gemm_workspace_bytes(const slm_linear_args* a, int32_t tile, int32_t slices);
+SLM_API int slm_gemm(const slm_linear_args* a, void* workspace, size_t workspace_bytes, int32_t tile, int32_t slices, void* stream);
 /* y = g sigmoid(alpha g) (u + shift), g = min(gate, limit), u = clamp(up, +-limit) (limit may be        */
 /* infinite: with alpha 1 and shift 0 the plain SiLU GLU); gu = [rows, 2 * half]                         */
 SLM_API int slm_clamped_glu(void* y, const void* gu, int64_t rows, int64_t half, int64_t ld_gu, int64_t ld_y,

@@ -1,0 +1,351 @@
+// gemm.hip -- y = x W^T in bf16 for many rows (prompts, mixed steps), from row-major x and W, with the GLU as an epilogue.
+//
+// Four waves, one to a SIMD, hold a quarter of the tile each: 128 x 128 products of 16 x 16 x 32 in 256 accumulators read 0.5 KB
+// of LDS per 1024 matrix-pipe cycles and SIMD, where eight waves of 128 x 64 read 0.75 -- and what bounds a large product here is power
+// (8192^3: 582 us on zeros, 767 on normal numbers), which operand traffic is part of (32 x 32 x 16 products: 815).  The
+// accumulators are pinned to the second half of the register file by inline asm: left to itself the compiler spreads them over
+// both and copies 1000 registers a step.
+//
+// A step is 64 of k, 128 bytes a row, so that LDS-DMA moves whole lines; 16-byte chunk c of row r lies in slot c ^ (r & 7), which
+// the DMA does on its global side.  Each step's products come in two halves of 32 k: the first runs over the LDS reads of the
+// second, the second over those of the next step's first.  One barrier a step, between the halves: there this stage has been read
+// by all waves and the next one has landed.  x has three stages and its DMA runs half a step apart from that of w: all 16
+// instructions of a step at once back up in the address unit, and a wave alone on its SIMD stalls with them (582 us against
+// 665).  256 x 256: 160 KB of LDS.
+//
+// Tiles that do not fill the last round of the chip are cut in K (slices > 1): every slice leaves fp32 sums past the caches, the last one
+// to arrive (a counter per tile) adds them up in slice order and stores.  Nobody waits for anybody.
+//
+// us, vendor product (and the GLU's launch) / this, normal numbers: 5692 x 28672 x 4096 GLU 1093 / 997 (1.34 PFLOP/s), 5692 x 4096 x 14336 739 / 485,
+// 5692 x 4096 x 4096 149 / 147, 3226 x 28672 x 4096 GLU 712 / 571, 3226 x 16896 x 4096 443 / 349, 4096 x 16384 x 2048 GLU 227 / 216, 4096 x 8512 x 2048
+// 153 / 120, 1000 x 4096 x 14336 129 / 107, 600 x 28672 x 4096 GLU 148 / 134, 300 x 4096 x 14336 73 / 63, 200 x 16384 x 2048 GLU 31 / 23,
+// 8192^3 701 / 729; short and narrow 207 x 4096 x 4096 18.5 / 19.8, 178 x 3664 x 2048 10.6 / 14.6 (of up to 128 rows: the vendor's).
+#include "latent_common.h"
+
+namespace slm {
+
+struct GemmK {
+  const char* x;
+  const char* w;
+  bf16* y;
+  float* slabs;            // [tiles cut][slices][fragments][256] f32x4
+  uint32_t* arrived;       // [tiles cut], zero
+  int64_t M, N, K, ldy;
+  uint32_t ldx2, ldw2;     // bytes
+  int mb, nb, whole, cut, slices, group;   // tiles: `whole` by one workgroup each, `cut` by `slices` each
+  float limit, alpha, shift;
+};
+
+__device__ __forceinline__ void gemm_product(f32x4& c, const bf16x8_t& w, const bf16x8_t& x) {
+  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(w), "v"(x));
+}
+
+// A run of `n` items for each of the 8 XCDs, which workgroups go round: item of a workgroup, -1 for none
+__device__ __forceinline__ int xcd_run(int wg, int n) {
+  const int per = (n + 7) >> 3, i = wg >> 3, t = (wg & 7) * per + i;
+  return i < per && t < n ? t : -1;
+}
+
+template <int BM, int BN, int WS, bool GLU>
+__global__ void __launch_bounds__(256, 1) gemm_kernel(const GemmK a) {
+  constexpr int XS = 3;                              // stages of x; WS: of w
+  constexpr int XB = BM * 128, WB = BN * 128;        // bytes of a stage
+  constexpr int MT = BM / 32, NT = BN / 32;          // 16-row / 16-column tiles of a wave
+  constexpr int XD = BM / 32, WD = BN / 32, ND = XD + WD;   // DMA instructions of a wave and step (8 rows each)
+  constexpr int R = MT + NT, MM = MT * NT;           // LDS reads and products of a half step
+  constexpr int LATE = XD + (WS == 3 ? WD : 0);      // DMA under way that the next step does not need
+  constexpr int FRAGS = MM;
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r16 = lane & 15, g = lane >> 4, wm = wave & 1, wn = wave >> 1;
+
+  // (whole tiles: a multiple of 8 workgroups)
+  const int whole_wgs = (a.whole + 7) & ~7;
+  int t, slice = 0, own = -1;
+  if ((int)blockIdx.x < whole_wgs) {
+    t = xcd_run(blockIdx.x, a.whole);
+    if (t < 0) return;
+  } else {
+    const int u = xcd_run((int)blockIdx.x - whole_wgs, a.cut * a.slices);
+    if (u < 0) return;
+    own = u / a.slices;
+    slice = u - own * a.slices;
+    t = a.whole + own;
+  }
+  // `group` row blocks by columns: neighbours in a run share rows of x and of w in their L2
+  const int gsz = a.group * a.nb, gi = t / gsz, in = t - gi * gsz;
+  const int rows_in = min(a.group, a.mb - gi * a.group);
+  const int mb = gi * a.group + in % rows_in, nb = in / rows_in;
+  const int64_t half = a.N / 2;
+  const int64_t m0 = (int64_t)mb * BM, n0 = (int64_t)nb * (GLU ? BN / 2 : BN);
+
+  // instruction i of this wave brings 8 rows of 128 bytes (rows past the end: the last one, not stored)
+  uint32_t off[ND];
+#pragma unroll
+  for (int i = 0; i < ND; ++i) {
+    const int r = (i < XD ? (wave * XD + i) : (wave * WD + i - XD)) * 8 + (lane >> 3);
+    const uint32_t k = (uint32_t)(((lane & 7) ^ (i < XD ? r & 7 : (r & 3) | ((r >> 1) & 4))) << 4);
+    if (i < XD) {
+      off[i] = (uint32_t)min(m0 + r, a.M - 1) * a.ldx2 + k;
+    } else if constexpr (GLU) {   // of a wave's BN / 2 columns half are of the gate, then the same of the up half
+      const int q = r / (BN / 2), c = r % (BN / 2);
+      const int64_t n = min(n0 + q * (BN / 4) + c % (BN / 4), half - 1) + (c >= BN / 4 ? half : 0);
+      off[i] = (uint32_t)n * a.ldw2 + k;
+    } else {
+      off[i] = (uint32_t)min(n0 + r, a.N - 1) * a.ldw2 + k;
+    }
+  }
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
+  const uint32_t xdst = lds0 + wave * (XD * 1024), wdst = lds0 + XS * XB + wave * (WD * 1024);
+  auto dma = [&](int i, int64_t kb, uint32_t at) {   // kb: byte offset in the rows, at: of the stage
+    const uint32_t dst = (i < XD ? xdst + i * 1024 : wdst + (i - XD) * 1024) + at;
+    const char* base = (i < XD ? a.x : a.w) + kb;
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %2" : : "v"(off[i]), "s"(dst), "s"(base) : "memory", "m0");
+  };
+  const int all = (int)(a.K >> 6), per = own < 0 ? all : (all + a.slices - 1) / a.slices;
+  const int s0 = slice * per, steps = min(per, all - s0);   // (the plan leaves no slice empty)
+  auto kbytes = [&](int s) { return (int64_t)(s0 + min(s, steps - 1)) << 7; };   // (steps past the end load the last one again)
+
+  // Columns of a pair of tiles go to them by fours, so that a lane ends with eight neighbours.  Chunk c of a row of w lies in slot
+  // c ^ (row % 4 + 4 (row / 8 % 2)): eight lanes read eight slots of either matrix.
+  const int xrow = wm * (BM / 2) + r16, wrow = wn * (BN / 2) + 8 * (r16 >> 2) + (r16 & 3);
+  bf16x8_t fx[2][MT], fw[2][NT];                // operands of the two halves
+  auto read = [&](int j, int h, uint32_t xa, uint32_t wa) {   // j-th of R
+    const int slot = ((h * 4 + g) ^ (r16 & 7)) << 4;   // (of w: row % 4 = r16 % 4, row / 8 % 2 = r16 / 4 % 2: the same)
+    if (j < MT) fx[h][j] = *reinterpret_cast<const bf16x8_t*>(lds + xa + (xrow + 16 * j) * 128 + slot);
+    else fw[h][j - MT] = *reinterpret_cast<const bf16x8_t*>(lds + XS * XB + wa + (wrow + 32 * ((j - MT) >> 1) + 4 * ((j - MT) & 1)) * 128 + slot);
+  };
+  f32x4 acc[NT][MT];
+#pragma unroll
+  for (int n = 0; n < NT; ++n)
+#pragma unroll
+    for (int m = 0; m < MT; ++m) acc[n][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+#pragma unroll
+  for (int p = 0; p < WS; ++p)
+#pragma unroll
+    for (int i = 0; i < ND; ++i)
+      if (i >= XD || p < 2) dma(i, kbytes(p), p * (i < XD ? XB : WB));
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"(ND + (WS - 2) * WD) : "memory");   // the first stages are there
+#pragma unroll
+  for (int j = 0; j < R; ++j) {
+    read(j, 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  uint32_t xa = 0, wa = 0, xl = 2 * XB;   // this step's stages, and the one that x is loaded to
+  for (int s = 0; s < steps; ++s) {
+    const uint32_t xn = xa == (XS - 1) * XB ? 0 : xa + XB, wnext = wa == (WS - 1) * WB ? 0 : wa + WB;
+    const int64_t kx = kbytes(s + 2);
+#pragma unroll
+    for (int b = 0; b < R; ++b) {
+#pragma unroll
+      for (int i = b * XD / R; i < (b + 1) * XD / R; ++i) dma(i, kx, xl);
+      read(b, 1, xa, wa);
+#pragma unroll
+      for (int q = b * MM / R; q < (b + 1) * MM / R; ++q) gemm_product(acc[q / MT][q % MT], fw[0][q / MT], fx[0][q % MT]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(LATE) : "memory");
+    const int64_t kw = kbytes(s + WS);
+#pragma unroll
+    for (int b = 0; b < R; ++b) {
+      if (b < WD) dma(XD + b, kw, wa);
+      read(b, 0, xn, wnext);
+#pragma unroll
+      for (int q = b * MM / R; q < (b + 1) * MM / R; ++q) gemm_product(acc[q / MT][q % MT], fw[1][q / MT], fx[1][q % MT]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    xl = xa;
+    xa = xn;
+    wa = wnext;
+  }
+  // (no DMA may outlive the workgroup's LDS; the last products are not tracked by the compiler)
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_nop 15\n\ts_nop 7" ::: "memory");
+
+  if (own >= 0) {
+    const __amdgpu_buffer_rsrc_t mine = __builtin_amdgcn_make_buffer_rsrc(
+        a.slabs + (int64_t)own * a.slices * (FRAGS * 1024), 0, a.slices * FRAGS * 4096, 0x00020000);
+    auto at = [&](int s, int f) { return ((s * FRAGS + f) * 256 + tid) * 16; };
+#pragma unroll
+    for (int f = 0; f < FRAGS; ++f)
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[f / MT][f % MT]), mine, at(slice, f), 0, /*sc1*/ 16);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // every wave's sums are out ..
+    __syncthreads();
+    uint32_t* word = reinterpret_cast<uint32_t*>(lds);
+    if (tid == 0) word[0] = __hip_atomic_fetch_add(a.arrived + own, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // .. then one announces them
+    __syncthreads();
+    if (word[0] != (uint32_t)a.slices - 1) return;
+    constexpr int C = 8;   // fragments in flight
+#pragma unroll
+    for (int f0 = 0; f0 < FRAGS; f0 += C) {
+      f32x4 sum[C];
+#pragma unroll
+      for (int f = 0; f < C; ++f) sum[f] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int s = 0; s < a.slices; ++s) {   // (in slice order, whoever is last: the same bits every time)
+#pragma unroll
+        for (int f = 0; f < C; ++f)
+          sum[f] += __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(mine, at(s, f0 + f), 0, /*sc1*/ 16));
+      }
+#pragma unroll
+      for (int f = 0; f < C; ++f) acc[(f0 + f) / MT][(f0 + f) % MT] = sum[f];
+    }
+  }
+
+  // lane: columns 8 g .. + 7 of a pair of tiles, row r16
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    const int64_t row = m0 + wm * (BM / 2) + 16 * m + r16;
+    if (row >= a.M) continue;
+    bf16* y = a.y + row * a.ldy;
+#pragma unroll
+    for (int n = 0; n < (GLU ? NT / 2 : NT); n += 2) {
+      const int64_t col = n0 + wn * (GLU ? BN / 4 : BN / 2) + 16 * n + 8 * g;
+      if (col >= (GLU ? half : a.N)) continue;
+      float v[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        v[j] = acc[n + (j >> 2)][m][j & 3];
+        if constexpr (GLU) v[j] = clamped_glu_f32(v[j], acc[n + (j >> 2) + NT / 2][m][j & 3], a.limit, a.alpha, a.shift);
+      }
+      store_f32<8>(y + col, v);
+    }
+  }
+}
+
+__global__ void __launch_bounds__(256) gemm_clear_kernel(uint32_t* p, int n) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < n) p[i] = 0;
+}
+
+// Tiles, and what they take: us of a step of 64 k alone on the chip and with every CU busy (power), and of a tile beside its steps.
+// Fitted to 900 timings of 90 products of 65 - 5700 rows; by them the tile taken is 0.5 % behind the best one on average, 10 % at worst.
+struct GemmTile {
+  int bm, bn;
+  float step, busy, rest;
+};
+constexpr GemmTile GEMM_TILES[] = {{256, 256, 0.914f, 1.386f, 8.6f}, {256, 128, 0.521f, 0.778f, 5.0f}, {128, 128, 0.311f, 0.488f, 3.4f}, {128, 256, 0.542f, 0.800f, 5.3f},
+                                   {256, 192, 0.725f, 1.037f, 6.6f}, {192, 256, 0.743f, 1.071f, 6.6f}, {160, 256, 0.647f, 0.909f, 6.1f}};
+constexpr int GEMM_N_TILES = sizeof(GEMM_TILES) / sizeof(GEMM_TILES[0]), GEMM_256_192 = 4;   // (that one has no GLU)
+constexpr int GEMM_CUS = 256;
+constexpr float GEMM_CUT = 6.f, GEMM_SLABS = 3.5e6f;   // us of cutting tiles, bytes of their slabs that take one more
+
+struct GemmPlan {
+  int tile, mb, nb, whole, cut, slices;
+  float us;
+  size_t bytes;   // workspace: counters, then slabs
+};
+
+static GemmPlan gemm_plan_of(const slm_linear_args& a, int tile, int slices) {
+  const GemmTile& t = GEMM_TILES[tile];
+  const bool glu = a.epilogue == SLM_LIN_GLU;
+  const int64_t cols = glu ? a.N / 2 : a.N, wide = glu ? t.bn / 2 : t.bn;
+  GemmPlan p{};
+  p.tile = tile;
+  p.mb = (int)((a.M + t.bm - 1) / t.bm);
+  p.nb = (int)((cols + wide - 1) / wide);
+  const int tiles = p.mb * p.nb, left = tiles % GEMM_CUS, steps = (int)(a.K >> 6);
+  // the last round's tiles are cut by as many as leave it one round, at least four steps each
+  int s = slices;
+  if (s <= 0) {
+    const int most = t.bm * t.bn == 128 * 128 ? 8 : 4;
+    s = left ? GEMM_CUS / left : 1;
+    s = s < most ? s : most;
+    while (s > 1 && steps / s < 4) --s;
+  }
+  if (!left) s = 1;
+  s = s < steps ? s : steps;
+  while (s > 1 && (steps + s - 1) / s * (s - 1) >= steps) --s;   // no slice is empty
+  p.slices = s;
+  p.cut = s > 1 ? left : 0;
+  p.whole = tiles - p.cut;
+  const size_t slabs = (size_t)p.cut * s * t.bm * t.bn * 4;
+  p.bytes = p.cut ? 1024 + slabs : 0;
+  auto round = [&](int wgs, int n) { return t.rest + n * (t.step + (t.busy - t.step) * (float)wgs / GEMM_CUS); };
+  p.us = (float)(tiles / GEMM_CUS) * round(GEMM_CUS, steps);
+  if (p.cut) p.us += round(left * s, (steps + s - 1) / s) + GEMM_CUT + (float)slabs / GEMM_SLABS;
+  else if (left) p.us += round(left, steps);
+  return p;
+}
+// tile -1: the one that takes least; slices 0: as many as pay, 1: none
+static GemmPlan gemm_plan(const slm_linear_args& a, int tile, int slices) {
+  if (tile >= 0) return gemm_plan_of(a, tile, slices);
+  GemmPlan best{};
+  for (int t = 0; t < GEMM_N_TILES; ++t) {
+    if (t == GEMM_256_192 && a.epilogue == SLM_LIN_GLU) continue;
+    for (int s = slices > 0 ? slices : 0; s <= (slices > 0 ? slices : 1); ++s) {
+      const GemmPlan p = gemm_plan_of(a, t, s);
+      if (best.us == 0.f || p.us < best.us) best = p;
+    }
+  }
+  return best;
+}
+
+template <int BM, int BN, int WS, bool GLU>
+static int gemm_launch(const GemmK& k, hipStream_t st) {
+  constexpr int bytes = (3 * BM + WS * BN) * 128;
+  auto fn = gemm_kernel<BM, BN, WS, GLU>;
+  static bool opted[64] = {};   // > 64 KiB of dynamic LDS: once per kernel and device
+  int dev = 0;
+  (void)hipGetDevice(&dev);
+  if (dev < 0 || dev >= 64 || !opted[dev]) {
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    if (dev >= 0 && dev < 64) opted[dev] = true;
+  }
+  const unsigned wgs = (unsigned)((k.whole + 7) / 8 * 8 + (k.cut * k.slices + 7) / 8 * 8);
+  fn<<<dim3(wgs), dim3(256), bytes, st>>>(k);
+  return hip_check_launch();
+}
+template <bool GLU>
+static int gemm_tile(const GemmPlan& p, const GemmK& k, hipStream_t st) {
+  switch (p.tile) {
+    case 0: return gemm_launch<256, 256, 2, GLU>(k, st);
+    case 1: return gemm_launch<256, 128, 3, GLU>(k, st);
+    case 2: return gemm_launch<128, 128, 3, GLU>(k, st);
+    case 3: return gemm_launch<128, 256, 3, GLU>(k, st);
+    case 5: return gemm_launch<192, 256, 2, GLU>(k, st);
+    case 6: return gemm_launch<160, 256, 3, GLU>(k, st);
+    default:
+      if constexpr (!GLU) return gemm_launch<256, 192, 2, GLU>(k, st);
+      return SLM_ERR_UNSUPPORTED;
+  }
+}
+
+// What the kernel takes: 16-byte rows, byte offsets of 32 bits
+static int gemm_check(const slm_linear_args* a, int tile, int slices) {
+  if (!a || !a->x || !a->w || !a->y || a->M < 0 || a->N <= 0 || a->K <= 0 || a->K % 64 || a->N % 16 || a->batch != 1 || a->n_splits != 1 ||
+      a->ldx < a->K || a->ldw < a->K || (a->epilogue != SLM_LIN_STORE && a->epilogue != SLM_LIN_GLU) || tile < -1 || tile >= GEMM_N_TILES || slices < 0)
+    return SLM_ERR_INVALID_ARG;
+  const bool glu = a->epilogue == SLM_LIN_GLU;
+  if (a->ldy < (glu ? a->N / 2 : a->N)) return SLM_ERR_INVALID_ARG;
+  if (a->dtype != SLM_BF16 || (glu && (a->N % 32 || tile == GEMM_256_192))) return SLM_ERR_UNSUPPORTED;
+  if (a->ldx % 8 || a->ldw % 8 || a->ldy % 8 || !aligned16(a->x) || !aligned16(a->w) || !aligned16(a->y)) return SLM_ERR_ALIGNMENT;
+  const int64_t most = 1ll << 31;
+  if (a->M > most / 2 / a->ldx || a->N > most / 2 / a->ldw || a->M > (1 << 24) || a->N > (1 << 24)) return SLM_ERR_UNSUPPORTED;
+  return SLM_OK;
+}
+
+}  // namespace slm
+
+using namespace slm;
+
+extern "C" SLM_API size_t slm_gemm_workspace_bytes(const slm_linear_args* a, int32_t tile, int32_t slices) {
+  return gemm_check(a, tile, slices) == SLM_OK && a->M ? gemm_plan(*a, tile, slices).bytes : 0;
+}
+
+extern "C" SLM_API int slm_gemm(const slm_linear_args* a, void* workspace, size_t workspace_bytes, int32_t tile, int32_t slices, void* stream) {
+  const int rc = gemm_check(a, tile, slices);
+  if (rc != SLM_OK || a->M == 0) return rc;
+  GemmPlan p = gemm_plan(*a, tile, slices);
+  if (p.cut && (!workspace || workspace_bytes < p.bytes)) p = gemm_plan(*a, tile, 1);   // (no scratch: no cut)
+  if (p.cut && !aligned16(workspace)) return SLM_ERR_ALIGNMENT;
+  GemmK k{};
+  k.x = (const char*)a->x; k.w = (const char*)a->w; k.y = (bf16*)a->y;
+  k.M = a->M; k.N = a->N; k.K = a->K; k.ldy = a->ldy; k.ldx2 = (uint32_t)(a->ldx * 2); k.ldw2 = (uint32_t)(a->ldw * 2);
+  k.limit = a->limit; k.alpha = a->glu_alpha; k.shift = a->glu_shift;
+  k.mb = p.mb; k.nb = p.nb; k.whole = p.whole; k.cut = p.cut; k.slices = p.slices; k.group = 8;
+  k.arrived = (uint32_t*)workspace; k.slabs = (float*)((char*)workspace + 1024);
+  hipStream_t st = (hipStream_t)stream;
+  hip_clear_error();
+  if (p.cut) gemm_clear_kernel<<<dim3(1), dim3(256), 0, st>>>(k.arrived, p.cut);
+  return a->epilogue == SLM_LIN_GLU ? gemm_tile<true>(p, k, st) : gemm_tile<false>(p, k, st);
+}

@@ -14,8 +14,10 @@ from . import _lib
 from ._lib import SLM_BF16, SLM_F32, SlmError, latent_check
 from .kernels import reserve_workspace
 
-# rows up to which a bf16 product of row-major weights is streamed; above it the vendor GEMM does it
+# rows up to which a bf16 product of row-major weights is streamed
 STREAM_MAX_ROWS = 32
+# rows from which the tile kernel does a stored product of row-major weights
+TILE_MIN_ROWS = 129
 # the same of weights in the streamed layout (stream_layout()), where the product reduces or activates in its epilogue
 STREAM_LAYOUT_MAX_ROWS = 128
 # clamped GLU: y = g * sigmoid(alpha * g) * (u + shift)
@@ -237,6 +239,28 @@ def _store_rows(N: int, K: int) -> int:
     return 64 if N >= 8192 and K <= 2048 + 5 * (N - 8192) // 2 else STREAM_MAX_ROWS
 
 
+def _gemm(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, glu=None, tile: int = -1, slices: int = 0) -> bool:
+    """out = x w^T, or with glu = (limit, alpha, shift) the clamped GLU of its halves, by the tile kernel for many rows.  False:
+    shapes and strides that it does not take."""
+    M, N, K = x.size(0), w.size(0), w.size(1)
+    if (x.dtype != torch.bfloat16 or K % 64 or N % (32 if glu else 16) or x.stride(0) < K or (x.stride(0) | w.stride(0) | out.stride(0)) % 8 or
+            (x.data_ptr() | w.data_ptr() | out.data_ptr()) % 16 or max(M * x.stride(0), N * w.stride(0)) > 1 << 30 or max(M, N) > 1 << 24):
+        return False
+    a = _linear_args(x, w, M, N, K)
+    a.ldx, a.ldw, a.ldy, a.y, a.epilogue = x.stride(0), w.stride(0), out.stride(0), _p(out), _lib.LIN_STORE
+    if glu:
+        a.epilogue, a.limit, a.glu_alpha, a.glu_shift = _lib.LIN_GLU, *glu
+    L = _lib.latent_lib()
+    need, ws = L.slm_gemm_workspace_bytes(C.byref(a), tile, slices), None
+    if need:
+        try:   # (its own: products of other streams have theirs; without it no tile is cut)
+            ws = torch.empty(need, dtype=torch.uint8, device=x.device)
+        except torch.OutOfMemoryError:
+            need = 0
+    latent_check(L.slm_gemm(C.byref(a), ws.data_ptr() if ws is not None else None, need, tile, slices, _stream()), "slm_gemm")
+    return True
+
+
 def linear(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None, layout: Optional[torch.Tensor] = None) -> torch.Tensor:
     """x [M, K] W[N, K]^T -> [M, N] of the same dtype.  layout: stream_layout(w)."""
     M, N, K = _check_xw(x, w)
@@ -249,7 +273,9 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None,
         _run_stream(a)
         return out
     if not streams_rows(x):
-        return torch.mm(x, w.t(), out=out)
+        # (stored products of up to 128 rows are the vendor's, whose small tiles leave fewer CUs idle: 125 x 2048 x 4096 10.7 us against
+        # 18.5, 96 x 12288 x 2048 16.8 against 19.6, 85 x 12608 x 4096 32.7 against 35.0)
+        return out if M >= TILE_MIN_ROWS and _gemm(x, w, out) else torch.mm(x, w.t(), out=out)
     a = _linear_args(x, w, M, N, K)
     a.ldx, a.ldw, a.ldy, a.y, a.epilogue = x.stride(0), K, out.stride(0), _p(out), _lib.LIN_STORE
     _run_linear(a)
@@ -331,7 +357,7 @@ def linear_glu(x: torch.Tensor, w_gate_up: torch.Tensor, out: torch.Tensor, limi
         a.ldx, a.ldw, a.ldy, a.y, a.epilogue = x.stride(0), K, out.stride(0), _p(out), _lib.LIN_GLU
         a.limit, a.glu_alpha, a.glu_shift = float(limit), float(alpha), float(shift)
         (_run_linear if s is None else _run_stream)(a)
-    else:
+    elif not _gemm(x, w_gate_up, out, (float(limit), float(alpha), float(shift))):
         gu = torch.mm(x, w_gate_up.t())
         clamped_glu(gu, out, limit, alpha, shift)
     return out

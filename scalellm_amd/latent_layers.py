@@ -223,7 +223,7 @@ class LatentAttention:
             if plan is None:
                 plan = params.plans[a.window] = LatentPlan.build(portions, a.window, cache.block_size(), h.device)
             ctx = lk.latent_gather(cache.rows, plan.slots)
-            kv = torch.mm(ctx[:, :self.c_pad], self.w_ukv.t())
+            kv = lk.linear(ctx[:, :self.c_pad], self.w_ukv)
             lk.latent_prefill(proj, ctx, kv, out, plan.tiles, heads=a.heads, q_dim=self.q_dim, c_pad=self.c_pad,
                               v_pad=self.v_pad, gate_off=self.off_g, window=a.window, scale=a.scale)
         if T <= lk.slab_rows(self.l_o):

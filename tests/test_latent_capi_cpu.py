@@ -1,6 +1,7 @@
 """C ABI of libslm_latent.so: exports match include/slm_latent.h, arguments are validated before anything is launched."""
 import ctypes as C
 import os
+import random
 import re
 import subprocess
 
@@ -233,3 +234,34 @@ def test_products_of_changed_weights_are_slabs_as_without_a_layout():
     assert lk.slab_rows(layout) == 128
     layout.copy_of.add_(1)
     assert lk.slab_rows(layout) == lk.slab_rows(None) == 32
+
+
+def _gemm_args(M=300, N=544, K=704, epilogue=_lib.LIN_STORE):
+    a = _lib.LinearArgs()
+    a.x = a.w = a.y = 4096
+    a.M, a.N, a.K, a.ldx, a.ldw, a.ldy, a.batch, a.n_splits, a.dtype, a.epilogue = M, N, K, K, K, N, 1, 1, _lib.SLM_BF16, epilogue
+    return a
+
+
+def test_tiled_products_refuse_what_they_have_no_form_for():
+    L = _lib.latent_lib()
+    for field, bad, rc in (("K", 63, -1), ("N", 15, -1), ("ldx", 32, -1), ("ldy", 8, -1), ("dtype", _lib.SLM_F32, -2), ("ldx", 708, -5), ("n_splits", 2, -1),
+                           ("batch", 2, -1), ("epilogue", _lib.LIN_SLABS, -1), ("w", 4104, -5), ("y", 4100, -5), ("M", 1 << 22, -2)):
+        a = _gemm_args()
+        setattr(a, field, bad)
+        assert L.slm_gemm(C.byref(a), None, 0, -1, 0, None) == rc, field
+    assert L.slm_gemm(C.byref(_gemm_args()), None, 0, 7, 0, None) == -1
+    assert L.slm_gemm(C.byref(_gemm_args(epilogue=_lib.LIN_GLU)), None, 0, 4, 0, None) == -2
+    assert L.slm_gemm(C.byref(_gemm_args(M=0)), None, 0, -1, 0, None) == 0
+
+
+def test_tiled_products_scratch_is_bounded():
+    """Slabs of the cut tiles: at most one 256 x 256 tile a CU; none where nothing is cut."""
+    L, rng = _lib.latent_lib(), random.Random(5)
+    for _ in range(2000):
+        a = _gemm_args(rng.randint(1, 9000), 32 * rng.randint(1, 1000), 64 * rng.randint(1, 250), rng.choice((_lib.LIN_STORE, _lib.LIN_GLU)))
+        assert L.slm_gemm_workspace_bytes(C.byref(a), -1, 0) <= 1024 + 256 * 256 * 256 * 4
+        assert L.slm_gemm_workspace_bytes(C.byref(a), -1, 1) == 0
+    a = _gemm_args(2300, 4128, 320)
+    assert L.slm_gemm_workspace_bytes(C.byref(a), 2, 2) == 1024 + (18 * 33 % 256) * 2 * 128 * 128 * 4
+    assert L.slm_gemm_workspace_bytes(C.byref(a), 2, 4) == 1024 + (18 * 33 % 256) * 3 * 128 * 128 * 4   # five steps: no fourth slice

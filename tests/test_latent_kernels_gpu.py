@@ -141,6 +141,47 @@ def _streamed_products(M, N, K):
         _close(out, ref.clamped_glu(want[:, :N // 2], want[:, N // 2:], 0.6), torch.bfloat16, b16=2e-2)
 
 
+# Products of many rows, in every tile: rows and columns that fill no tile, one step of 64 k and fewer than there are stages, more tiles than
+# CUs with the rest cut in K (also by a count that leaves the last slice short), rows with a stride.  fp32 sums of exact products, one rounding;
+# the slices' sums come in a fixed order, so a second run gives the same bits.
+@pytest.mark.parametrize("tile", range(7))
+@pytest.mark.parametrize("M,N,K,slices", [(1, 16, 64, 1), (129, 272, 128, 2), (300, 544, 704, 3), (257, 96, 1088, 5), (160, 1312, 192, 1), (2300, 4128, 320, 2)])
+def test_tiled_products(M, N, K, slices, tile):
+    lk = _lk()
+    x = _rnd(1, M, K + 8, dtype=torch.bfloat16)[:, :K]
+    w = _rnd(2, N, K, dtype=torch.bfloat16, std=K ** -0.5)
+    want = _f64(x) @ _f64(w).T
+    wide = torch.full((M, N + 16), float("nan"), dtype=torch.bfloat16, device=DEV)
+    out = wide[:, 8:8 + N]
+    assert lk._gemm(x, w, out, tile=tile, slices=slices)
+    _close(out, want, torch.bfloat16)
+    assert wide[:, :8].isnan().all() and wide[:, 8 + N:].isnan().all()
+    again = torch.zeros(M, N, dtype=torch.bfloat16, device=DEV)
+    assert lk._gemm(x, w, again, tile=tile, slices=slices) and torch.equal(again, out)
+    if tile != 4 and N % 32 == 0:   # (that tile has no GLU)
+        glu = torch.full((M, N // 2 + 8), float("nan"), dtype=torch.bfloat16, device=DEV)
+        assert lk._gemm(x, w, glu[:, :N // 2], (0.6, lk.GLU_ALPHA, lk.GLU_SHIFT), tile, slices)
+        _close(glu[:, :N // 2], ref.clamped_glu(want[:, :N // 2], want[:, N // 2:], 0.6), torch.bfloat16, b16=2e-2)
+        assert glu[:, N // 2:].isnan().all()
+
+
+@pytest.mark.parametrize("M", [129, 700])
+def test_products_of_prompts_by_the_planned_tile(M):
+    lk, N, K = _lk(), 2080, 1024
+    x, w = _rnd(1, M, 2 * K, dtype=torch.bfloat16)[:, K:], _rnd(2, N, K, dtype=torch.bfloat16, std=K ** -0.5)
+    want, out = _f64(x) @ _f64(w).T, torch.zeros(M, N // 2, dtype=torch.bfloat16, device=DEV)
+    _close(lk.linear(x, w), want, torch.bfloat16)
+    lk.linear_glu(x, w, out, 0.6)
+    _close(out, ref.clamped_glu(want[:, :N // 2], want[:, N // 2:], 0.6), torch.bfloat16, b16=2e-2)
+    # without scratch nothing is cut; results are the same up to the order of sums
+    from scalellm_amd import _lib
+    a = lk._linear_args(x, w, M, N, K)
+    y = torch.zeros(M, N, dtype=torch.bfloat16, device=DEV)
+    a.ldx, a.ldw, a.ldy, a.y, a.epilogue = x.stride(0), K, N, lk._p(y), _lib.LIN_STORE
+    lk.latent_check(_lib.latent_lib().slm_gemm(lk.C.byref(a), None, 0, -1, 0, lk._stream()), "slm_gemm")
+    _close(y, want, torch.bfloat16)
+
+
 # every number of slabs, rows and columns that fill no workgroup, results at an odd address; one rounding to 16 bits
 @pytest.mark.parametrize("n", range(1, 9))
 @pytest.mark.parametrize("rows,half", [(1, 16), (33, 96), (128, 2752)])
