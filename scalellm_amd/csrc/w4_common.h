@@ -285,10 +285,21 @@ constexpr size_t W4_WS_LDS_BYTES = 7 * (256 * 64) + 4 * (8 * 1024) + 2 * 4 * (10
 
 // symmetric 256 x 256 kernel for large M x N (w4_xl.hip): 512 threads, 160 KiB LDS
 void launch_gemm_xl(const GemmKParams& kp, int dtype, int ng, int n_blocks, hipStream_t st);
-void launch_gemm_xl_sk(const GemmKParams& kp, int dtype, int ng, int n_wgs, hipStream_t st);
+void launch_gemm_xl_sk(const GemmKParams& kp, int ng, int n_wgs, hipStream_t st);   // (float16)
 constexpr int W4_XL_SK_WGS = 256;                                  // one workgroup per CU (160 KiB of LDS each)
 constexpr size_t W4_XL_SK_SLOT_BYTES = 256 * 256 * sizeof(float);  // a partial tile
 constexpr size_t W4_XL_SK_SYNC_BYTES = 2048;                       // ticket + one flag per workgroup
 constexpr size_t W4_XL_LDS_BYTES = 7 * (256 * 64) + 3 * (16 * 1024);
+
+// tiles of four waves for many rows, bf16 (w4_tile.hip)
+struct W4TilePlan {
+  int tile, mb, nb, tiles, slices;
+  float us;
+};
+// tile -1: the one that takes least; slices 0: as many as pay, 1: none
+W4TilePlan w4_tile_plan(int64_t M, int64_t N, int64_t K, int tile, int slices);
+void launch_w4_tile(const GemmKParams& kp, const W4TilePlan& p, void* workspace, int ng, hipStream_t st);
+constexpr size_t W4_TILE_SYNC_BYTES = 2048;                              // a counter per tile that is cut (at most 128) ..
+constexpr size_t W4_TILE_SLAB_BYTES = (size_t)256 * 256 * 256 * sizeof(float);   // .. and fp32 sums of at most one tile a CU
 
 }  // namespace slm

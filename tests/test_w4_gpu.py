@@ -747,3 +747,52 @@ def test_stream_k_form_seeded_fuzz(seed):
         assert torch.equal(sk, again), (M, K, N)
         err = _rel_err(sk.float().cpu().numpy(), tile.float().cpu().numpy())
         assert err < 2e-3, (M, K, N, err)
+
+
+# ---- tiles of four waves (w4_tile.hip) ------------------------------------------------------------------------
+# Every tile shape at rows and columns that fill no tile, one step of K's smallest unit and more, every group size (32: two scale groups a step), tiles that
+# are whole, cut in K, and cut so that the last slice is short; strided rows of either side, and results at an odd address.  fp32 sums of exact products of the
+# dequantised weights, one rounding: at most 2^-8 of a value, some 0.4 of that on average.
+@pytest.mark.parametrize("tile", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("M,K,N,gs", [(129, 128, 64, 128), (257, 1152, 96, 32), (300, 512, 544, 64), (200, 1024, 256, -1), (2304, 384, 4160, 128)])
+def test_four_wave_tiles(M, K, N, gs, tile):
+    from scalellm_amd import kernels
+    dtype, tdt = "bf16", torch.bfloat16
+    case = helpers.make_quant_case(M + K, K, N, gs if gs > 0 else K, "awq" if tile % 2 else "gptq", dtype)
+    plain = _pack(case, dtype)
+    w = kernels.w4_dequant(plain).double()
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    a = torch.randn(M, K + 8, device=DEV, dtype=tdt, generator=g)[:, :K]
+    b = torch.randn(N, device=DEV, dtype=tdt, generator=g)
+    want = a.double() @ w + b.double()
+    for cut in (0, 2, 3):
+        with kernels.tuning(SLM_W4_TILE=tile, SLM_W4_XL_SK=cut):
+            wide = torch.full((M, N + 9), float("nan"), device=DEV, dtype=tdt)
+            kernels.gptq_gemm(a, plain, wide[:, 1:N + 1], b)
+            c = torch.full((M, N), float("nan"), device=DEV, dtype=tdt)
+            kernels.gptq_gemm(a, plain, c, b)
+            assert torch.equal(wide[:, 1:N + 1], c) and wide[:, 0].isnan().all() and wide[:, N + 1:].isnan().all()
+            assert ((c.double() - want).norm() / want.norm()).item() < 2e-3
+            if N % 64 == 0:
+                paired = helpers.pack_case(case, dtype, paired=True)
+                half, ref = torch.empty(M, N // 2, device=DEV, dtype=tdt), torch.empty(M, N // 2, device=DEV, dtype=tdt)
+                n = torch.arange(N, device=DEV)
+                src = (n >> 6) * 32 + (n & 31) + torch.where(n & 32 != 0, N // 2, 0)
+                kernels.gptq_gemm(a, paired, half, b[src].contiguous(), silu_mul=True)
+                kernels.silu_and_mul(ref, c)
+                assert torch.equal(half, ref)
+
+
+def test_four_wave_tiles_without_scratch_are_not_cut():
+    """A call whose plan cuts tiles runs without the scratch of it too: the same sums in another order."""
+    from scalellm_amd import _lib, kernels
+    import ctypes as C
+    M, K, N = 400, 2048, 2048
+    case, packed, a, b = _sk_case(M, K, N, "bf16")
+    c, want = torch.empty(M, N, device=DEV, dtype=torch.bfloat16), torch.empty(M, N, device=DEV, dtype=torch.bfloat16)
+    kernels.gptq_gemm(a, packed, want)
+    g = kernels._gemm_args(a, packed, c, None, False)
+    assert _lib.lib().slm_w4a16_gemm_workspace_bytes(C.byref(g)) > 0
+    _lib.check(_lib.lib().slm_w4a16_gemm(C.byref(g), torch.cuda.current_stream().cuda_stream), "slm_w4a16_gemm")
+    torch.cuda.synchronize()
+    assert _rel_err(c.float().cpu().numpy(), want.float().cpu().numpy()) < 2e-3
