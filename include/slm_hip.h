@@ -306,6 +306,11 @@ typedef struct slm_w4_gemm_args {
  * at bs 128).  Results are correct either way; the SAME flag must be passed to the workspace / deferred-splits
  * queries (they describe the plan the call will take). */
 #define SLM_W4_SHARES_CHIP 4
+/* flags: sums may come in another order than without the flag, which lets bf16 products of many rows take faster tiles.  Each result is as near to the
+ * exact one as before, but a few round the other way; where weights have a mean -- GPTQ's zero points, one above the stored ones, give them a
+ * seventh of their spread -- outputs have a large part in common and layers behind them turn single roundings into a third of the outputs'
+ * spread, so the mirror in Python sets it for AWQ weights only. */
+#define SLM_W4_TILES 8
 
 SLM_API size_t slm_w4a16_gemm_workspace_bytes(const slm_w4_gemm_args* a);
 /* number of partial slabs the call will leave in the workspace (>= 2), or 0 when it writes c as usual */

@@ -534,6 +534,7 @@ W4Linear::W4Linear(const std::string& quant_method, const torch::Tensor& qweight
                    const std::optional<torch::Tensor>& g_idx, int64_t group_size, int64_t bits, bool paired) {
   const bool awq = quant_method == "awq";
   paired_ = paired;
+  order_ = awq && bits == 4 ? SLM_W4_TILES : 0;
   TORCH_CHECK(!paired || bits == 4, "paired (gate | up) packing is built for 4-bit weights");
   TORCH_CHECK(awq || quant_method == "gptq", "quant_method must be awq or gptq");
   TORCH_CHECK(bits == 4 || bits == 8, "bits must be 4 or 8, got ", bits);
@@ -668,6 +669,7 @@ torch::Tensor W4Linear::forward(const torch::Tensor& input, const std::optional<
   g.lda = a.stride(0); g.ldc = c.stride(0);
   g.group_size = group_size_;
   g.dtype = dtype_code(a);
+  g.flags = order_;
   if (g.M == 0) return c;
   const size_t need = slm_w4a16_gemm_workspace_bytes(&g);
   torch::Tensor ws;
@@ -696,6 +698,7 @@ slm_w4_gemm_args w4_args(const torch::Tensor& a, const void* wq, const void* sz,
 }  // namespace
 
 size_t W4Linear::workspace_bytes(int64_t M, int flags) const {
+  flags |= order_;
   slm_w4_gemm_args g{};
   g.wq = wq_.const_data_ptr(); g.sz = sz_.const_data_ptr();
   g.perm = perm_.defined() ? perm_.const_data_ptr<int32_t>() : nullptr;
@@ -708,6 +711,7 @@ size_t W4Linear::workspace_bytes(int64_t M, int flags) const {
 }
 
 int W4Linear::forward_into(const torch::Tensor& a, torch::Tensor& c, int flags, const torch::Tensor& workspace) const {
+  flags |= order_;
   c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(a.device());
   TORCH_CHECK(a.dim() == 2 && a.size(1) == k_src_ && a.stride(1) == 1 && a.scalar_type() == dtype_);
   TORCH_CHECK(!(flags & SLM_W4_SILU_MUL) || paired_, "SLM_W4_SILU_MUL needs weights packed paired");

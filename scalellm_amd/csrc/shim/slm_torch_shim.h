@@ -177,6 +177,7 @@ class W4Linear {
   int64_t K_ = 0, N_ = 0, group_size_ = 0;
   int64_t k_src_ = 0;  // width of the activations (== K_ unless the shard was padded)
   bool paired_ = false;
+  int order_ = 0;  // SLM_W4_TILES for AWQ weights (include/slm_hip.h)
   torch::ScalarType dtype_;
 };
 

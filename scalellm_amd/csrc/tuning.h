@@ -47,8 +47,8 @@ enum TuneKey : int {
   TUNE_ATTN_TILE_KV2,     // SLM_ATTN_TILE_KV2     two wave groups share a query tile's KV range in the prefill tile kernel: 1 always, 0 never (default: small plain-prefill grids)
   TUNE_W4_XL_MODEL,       // SLM_W4_XL_MODEL       0 = the 256 x 256 kernel only where its tiles fill whole rounds (no round-count comparison with 256 x 128 tiles)
   TUNE_W4_M128_ADMA,      // SLM_W4_M128_ADMA      activations of the 256-column form by LDS-DMA (1) or through registers (0)
-  TUNE_W4_XL_SK,          // SLM_W4_XL_SK          cutting of w4_tile.hip's last round of tiles in K: 0 never, n >= 2 in n slices (default: where it takes less)
-  TUNE_W4_TILE,           // SLM_W4_TILE           tile shape of w4_tile.hip: 1 .. 5, 0 = never that kernel (default: the one that takes least)
+  TUNE_W4_XL_SK,          // SLM_W4_XL_SK          stream-K form of the 256 x 256 kernel: 0 never, 2 wherever it applies (default 1: where the round model says it wins)
+  TUNE_W4_TILE,           // SLM_W4_TILE           w4_tile.hip: 1 .. 5 = that tile shape for every bf16 call, + 8 n = cut in n slices of K; 0 = never (default: where a call allows it and its tiles pay)
   TUNE_COUNT
 };
 

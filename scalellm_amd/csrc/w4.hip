@@ -32,8 +32,8 @@
 //    M <= 32                         w4_small.hip  lean weight stream (MFMA, post-scaled)
 //    32 < M <= 128, narrow layers    this file
 //    M > 128, >= 112 tiles of 256x128 w4_ws.hip     producer / consumer waves, LDS-DMA activations
-//    prefill-sized M x N             w4_xl.hip     symmetric 256 x 256 tiles (float16, or beside another stream)
-//    bf16, M > 320 or wide layers    w4_tile.hip   four waves a tile (not beside another stream)
+//    prefill-sized M x N             w4_xl.hip     symmetric 256 x 256 tiles
+//    the same in bf16                w4_tile.hip   four waves a tile (SLM_W4_TILES)
 // (DESIGN.md 3.3 has the measurements behind each boundary.)
 #include "w4_common.h"
 #include "tuning.h"
@@ -521,11 +521,11 @@ constexpr bool w4_post_fits(int mt, int ntw, int ng, int pc) {
 }
 constexpr bool w4_pre_fits(int /*mt*/, int ntw, int ng, int pc) { return !(ntw == 2 && ng == 4 && pc >= 2); }
 
-// Tiles of four waves (w4_tile.hip): in bf16 all of more than 320 rows; of wide layers, whose few rows of tiles fill the chip, all of more than 128.  us of
-// the other kernels / of these (group 128): 4096 x 28672 with SiLU 2183 rows 453 / 436, 640 rows 177 / 150, 320 rows 100 / 81, 160 rows 60 / 59; 2048 x
-// 16384 160 rows 32 / 23; 14336 x 4096 4096 rows 408 / 346, 320 rows 66 / 70; 4096 x 6144 2183 rows 116 / 100, 320 rows 33 / 39; 2048 x 4096 1000 rows
-// 40 / 24, 192 rows 16.9 / 17.3; 2048 x 2048 2183 rows 55 / 31, 320 rows 16.4 / 16.7.  (Narrow layers of up to 256 rows leave slabs to their norm.)
-// float16 keeps the order of sums that it has: a few of its results, after some layers, move by more than 6 % of their spread with another.
+// Tiles of four waves (w4_tile.hip), where the caller lets sums come in another order (SLM_W4_TILES): in bf16 all of more than 320 rows; of wide layers,
+// whose few rows of tiles fill the chip, all of more than 128.  us of the other kernels / of these (group 128): 4096 x 28672 with SiLU 2183 rows
+// 453 / 436, 640 rows 177 / 150, 320 rows 100 / 81, 160 rows 60 / 59; 2048 x 16384 160 rows 32 / 23; 14336 x 4096 4096 rows 408 / 346, 320 rows
+// 66 / 70; 4096 x 6144 2183 rows 116 / 100, 320 rows 33 / 39; 2048 x 4096 1000 rows 40 / 24, 192 rows 16.9 / 17.3; 2048 x 2048 2183 rows 55 / 31,
+// 320 rows 16.4 / 16.7.  (Narrow layers of up to 256 rows leave slabs to their norm.)
 static bool w4_tile_rows(int64_t M, int64_t K, int64_t N) { return M > 320 || (M > 128 && N >= 8192 && N * K >= (1 << 25)); }
 struct GemmPlan {
   int xl_sk, sk_per;      // stream-K form of the 256 x 256 kernel (w4_xl.hip): 128-deep chunks per workgroup
@@ -542,7 +542,7 @@ static int plan_gemm(const slm_w4_gemm_args* a, GemmPlan* pl) {
   if (a->M < 0 || a->K <= 0 || a->N <= 0) return SLM_ERR_INVALID_ARG;
   if (a->dtype != SLM_F16 && a->dtype != SLM_BF16) return SLM_ERR_UNSUPPORTED;
   if (a->K % W4_KC || a->N % 32) return SLM_ERR_UNSUPPORTED;  // reference: K%128, N%64
-  if (a->flags & ~(SLM_W4_DEFER_REDUCE | SLM_W4_SILU_MUL | SLM_W4_SHARES_CHIP)) return SLM_ERR_INVALID_ARG;
+  if (a->flags & ~(SLM_W4_DEFER_REDUCE | SLM_W4_SILU_MUL | SLM_W4_SHARES_CHIP | SLM_W4_TILES)) return SLM_ERR_INVALID_ARG;
   if (a->flags & SLM_W4_SILU_MUL) {
     if (a->flags & SLM_W4_DEFER_REDUCE) return SLM_ERR_INVALID_ARG;
     if (a->N % 64) return SLM_ERR_UNSUPPORTED;
@@ -846,23 +846,16 @@ static int plan_gemm(const slm_w4_gemm_args* a, GemmPlan* pl) {
   }
   pl->tiled = 0;
   const int tile = tune_get(TUNE_W4_TILE, -1);
-  if (a->dtype == SLM_BF16 && tile != 0 && (tile > 0 || w4_tile_rows(a->M, a->K, a->N)) && ((a->M - 1) * a->lda + a->K) * 2 < ((int64_t)1 << 31) &&
+  if (a->dtype == SLM_BF16 && tile != 0 && (tile > 0 || ((a->flags & SLM_W4_TILES) && w4_tile_rows(a->M, a->K, a->N))) && ((a->M - 1) * a->lda + a->K) * 2 < ((int64_t)1 << 31) &&
       !(a->flags & SLM_W4_SHARES_CHIP) && !tune_is_set(TUNE_W4_MT) && !tune_is_set(TUNE_W4_SPLITK)) {
     pl->tiled = 1;
     pl->xl_sk = 0;
     pl->split_k = 1;
-    const int cut = tune_get(TUNE_W4_XL_SK, -1);
-    pl->tile = w4_tile_plan(a->M, a->N, a->K, tile > 0 ? tile - 1 : -1, cut < 0 ? 0 : cut < 1 ? 1 : cut);
+    pl->tile = w4_tile_plan(a->M, a->N, a->K, tile > 0 ? tile % 8 - 1 : -1, tile > 0 ? tile / 8 : 0);
   }
   pl->part_bytes = pl->split_k > 1 ? (size_t)pl->split_k * a->M * a->N * sizeof(float) : 0;
   if (pl->xl_sk) pl->part_bytes = W4_XL_SK_WGS * W4_XL_SK_SLOT_BYTES + W4_XL_SK_SYNC_BYTES;
-  if (pl->tiled) {
-    // (where 256 x 256 tiles would leave a tenth of their rounds empty the scratch of a cut is asked for whether this plan cuts or not:
-    // what a caller sets aside for a shape does not hang on the fitted times)
-    const int64_t tiles = ((a->M + 255) / 256) * ((a->N + 255) / 256), rounds = (tiles + 255) / 256;
-    const bool part_filled = tiles * 10 < rounds * 256 * 9 && tune_get(TUNE_W4_XL_SK, -1) != 0;
-    pl->part_bytes = pl->tile.slices > 1 || part_filled ? W4_TILE_SYNC_BYTES + W4_TILE_SLAB_BYTES : 0;
-  }
+  if (pl->tiled) pl->part_bytes = pl->tile.slices > 1 ? W4_TILE_SYNC_BYTES + W4_TILE_SLAB_BYTES : 0;
   pl->aperm_bytes = a->perm ? (((size_t)a->M * a->K * 2 + 255) & ~(size_t)255) : 0;
   return SLM_OK;
 }
@@ -1093,7 +1086,7 @@ static int gemm_impl(const slm_w4_gemm_args* a, const slm_w4_norm_prologue* np, 
     kp.sk_sync = reinterpret_cast<unsigned*>(reinterpret_cast<char*>(a->workspace) + W4_XL_SK_WGS * W4_XL_SK_SLOT_BYTES);
     // the ticket and the flags start at zero on every call (a memset node under capture)
     if (hipMemsetAsync(kp.sk_sync, 0, W4_XL_SK_SYNC_BYTES, st) != hipSuccess) return hip_check_launch();
-    launch_gemm_xl_sk(kp, pl.ng, W4_XL_SK_WGS, st);
+    launch_gemm_xl_sk(kp, a->dtype, pl.ng, W4_XL_SK_WGS, st);
   } else
   if (pl.ks)
     launch_gemm_ks(kp, a->dtype, pl.ng, pl.ks_cw, pl.ks_nw, pl.n_nblocks * pl.split_k, st, pl.ks_mt);

@@ -418,10 +418,15 @@ static void launch_xl_sk(const GemmKParams& kp, int n_wgs, hipStream_t st) {
   hipLaunchKernelGGL(kfn, dim3((unsigned)n_wgs), dim3(512), W4_XL_LDS_BYTES, st, kp);
 }
 
-void launch_gemm_xl_sk(const GemmKParams& kp, int ng, int n_wgs, hipStream_t st) {
-  // (several row blocks always re-read the weights here: cacheable loads; bf16 has its own tiles, w4_tile.hip)
-  if (ng == 4) launch_xl_sk<f16_tag, 2, false>(kp, n_wgs, st);
-  else launch_xl_sk<f16_tag, 1, false>(kp, n_wgs, st);
+void launch_gemm_xl_sk(const GemmKParams& kp, int dtype, int ng, int n_wgs, hipStream_t st) {
+  // (several row blocks always re-read the weights here: cacheable loads)
+  if (dtype == SLM_BF16) {
+    if (ng == 4) launch_xl_sk<bf16_tag, 2, false>(kp, n_wgs, st);
+    else launch_xl_sk<bf16_tag, 1, false>(kp, n_wgs, st);
+  } else {
+    if (ng == 4) launch_xl_sk<f16_tag, 2, false>(kp, n_wgs, st);
+    else launch_xl_sk<f16_tag, 1, false>(kp, n_wgs, st);
+  }
 }
 
 template <typename T, int NGC, bool WNT>

@@ -414,7 +414,7 @@ class PackedW4:
     (qlinear_awq_marlin_impl.cpp:99-125,232-235; qlinear_gptq_marlin_impl.cpp:41-71,181-184).
     """
 
-    def __init__(self, wq, sz, perm, K, N, group_size, dtype, paired=False, k_src=None):
+    def __init__(self, wq, sz, perm, K, N, group_size, dtype, paired=False, k_src=None, any_order=False):
         self.wq, self.sz, self.perm = wq, sz, perm
         self.K, self.N, self.group_size, self.dtype = K, N, group_size, dtype
         # k_src: width of the activations the GEMM takes.  Equal to K except for a padded
@@ -423,6 +423,8 @@ class PackedW4:
         # paired: a merged [gate | up] weight whose packed column tiles alternate gate / up
         # (SLM_W4_PAIRED) -- the form gptq_gemm(..., silu_mul=True) needs
         self.paired = paired
+        # any_order: products' sums may come in another order (SLM_W4_TILES; include/slm_hip.h says why not everywhere)
+        self.any_order = any_order
 
 
 def _prepack(fmt: int, qweight, qzeros, scales, perm, K, N, group_size, paired=False) -> PackedW4:
@@ -451,7 +453,7 @@ def _prepack(fmt: int, qweight, qzeros, scales, perm, K, N, group_size, paired=F
                            perm.data_ptr() if perm is not None else None, K, N, gs,
                            _dtype_code(scales), wq.data_ptr(), sz.data_ptr(), _stream()),
           "slm_w4_prepack")
-    return PackedW4(wq, sz, perm, K, N, gs, scales.dtype, paired)
+    return PackedW4(wq, sz, perm, K, N, gs, scales.dtype, paired, any_order=fmt & ~_lib.SLM_W4_PAIRED == _lib.SLM_W4_AWQ)
 
 
 def awq_repack(qweight: torch.Tensor,  # [K, N/8] int32, AWQ interleave
@@ -714,7 +716,7 @@ def gptq_gemm(a: torch.Tensor, packed: PackedW4, c: torch.Tensor,
         npro.residual_out = norm.residual_out.data_ptr() if norm.residual_out is not None else None
         npro.weight = norm.weight.data_ptr()
         npro.normed_out = norm.normed_out.data_ptr() if norm.normed_out is not None else None
-    chip = _chip_flag()
+    chip = _chip_flag() | (_lib.SLM_W4_TILES if packed.any_order else 0)
     g.flags = chip
     if silu_mul:
         g.flags = _lib.SLM_W4_SILU_MUL | chip

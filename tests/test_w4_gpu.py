@@ -765,8 +765,8 @@ def test_four_wave_tiles(M, K, N, gs, tile):
     a = torch.randn(M, K + 8, device=DEV, dtype=tdt, generator=g)[:, :K]
     b = torch.randn(N, device=DEV, dtype=tdt, generator=g)
     want = a.double() @ w + b.double()
-    for cut in (0, 2, 3):
-        with kernels.tuning(SLM_W4_TILE=tile, SLM_W4_XL_SK=cut):
+    for cut in (1, 2, 3):
+        with kernels.tuning(SLM_W4_TILE=tile + 8 * cut):
             wide = torch.full((M, N + 9), float("nan"), device=DEV, dtype=tdt)
             kernels.gptq_gemm(a, plain, wide[:, 1:N + 1], b)
             c = torch.full((M, N), float("nan"), device=DEV, dtype=tdt)
@@ -792,7 +792,22 @@ def test_four_wave_tiles_without_scratch_are_not_cut():
     c, want = torch.empty(M, N, device=DEV, dtype=torch.bfloat16), torch.empty(M, N, device=DEV, dtype=torch.bfloat16)
     kernels.gptq_gemm(a, packed, want)
     g = kernels._gemm_args(a, packed, c, None, False)
+    g.flags = _lib.SLM_W4_TILES
     assert _lib.lib().slm_w4a16_gemm_workspace_bytes(C.byref(g)) > 0
     _lib.check(_lib.lib().slm_w4a16_gemm(C.byref(g), torch.cuda.current_stream().cuda_stream), "slm_w4a16_gemm")
     torch.cuda.synchronize()
     assert _rel_err(c.float().cpu().numpy(), want.float().cpu().numpy()) < 2e-3
+
+
+def test_four_wave_tiles_are_taken_where_a_call_allows_it():
+    """Another order of sums is the caller's to allow: AWQ weights do, GPTQ weights keep theirs whatever the rows; float16 has no such tiles."""
+    from scalellm_amd import kernels
+    for fmt, dtype, moved in (("awq", "bf16", True), ("gptq", "bf16", False), ("awq", "f16", False)):
+        case, packed, a, b = _sk_case(600, 4096, 4096, dtype, fmt=fmt)
+        c, old = torch.empty(600, 4096, device=DEV, dtype=a.dtype), torch.empty(600, 4096, device=DEV, dtype=a.dtype)
+        kernels.gptq_gemm(a, packed, c)
+        with kernels.tuning(SLM_W4_TILE=0):
+            kernels.gptq_gemm(a, packed, old)
+        torch.cuda.synchronize()
+        assert torch.equal(c, old) != moved
+        assert _rel_err(c.float().cpu().numpy(), old.float().cpu().numpy()) < 2e-3
