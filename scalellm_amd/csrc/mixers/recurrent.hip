@@ -6,10 +6,14 @@
 //            (state).  16 heads of 128 x 128: delta 128 rows 71 us with ordinary loads and stores and the inputs one after the
 //            other, 52 without (5.2 TB/s), 32 rows 18.4 and 14.1; lightning, the first alone, 128 rows 53 and 46 (5.8 TB/s), 32 rows
 //            14.4 and 12.7, 8 rows 6.0 and 5.5, 1 row 4.3 and 4.3.
-//   prepare  portions, cut into chunks of 16 tokens, every chunk at once: inputs activated and normed, decays summed, and
-//            what a chunk's tokens do to each other solved (a 16 x 16 triangular system).  Bound: VALU, HBM.
+//   prepare  portions, cut into chunks of 16 tokens, every chunk at once: inputs activated and normed, decays summed, what a chunk's tokens do to
+//            each other solved (a 16 x 16 triangular system), and everything that does not wait for the state multiplied out.  Bound: the
+//            latency of its inputs, which are loaded before the first is used, and the records it writes (2 TB/s).
 //   scan     portions: chunk after chunk.  The columns of S are independent, so a workgroup owns 16 of them and keeps them
-//            in registers from the portion's first token to its last; the products are 32-bit MFMAs.  Bound: fp32 MFMA.
+//            in registers from the portion's first token to its last; the products are 32-bit MFMAs.  Bound: a chain of two products and an
+//            exchange a chunk, 0.7 us, and the instructions around them.
+//   Both, us, 16 heads of 128 x 128 and 4096 tokens: delta 305 with the triangular system and B U in the scan, 64-bit addresses and a wave's
+//   read-outs by itself, 257 now; lightning 184 and 159; 8 x 500 tokens, 32 heads: 341 and 304, 209 and 186; 16 heads of 64, 2000 tokens: 120 and 85.
 //   gated_norm  the norm and gate behind a scan.
 #include "latent/latent_common.h"
 #include "slm_mixers.h"
@@ -18,7 +22,16 @@ namespace slm {
 
 constexpr bool DELTA_MODE(int m) { return m == SLM_REC_DELTA; }
 
+// n / d for finite n and d in 2^-100 .. 2^100: the reciprocal corrected once, its quotient once (half the instructions of the general division)
+__device__ __forceinline__ float quotient(float n, float d) {
+  float r = __builtin_amdgcn_rcpf(d);
+  r = __builtin_fmaf(__builtin_fmaf(-d, r, 1.0f), r, r);
+  const float q = n * r;
+  return __builtin_fmaf(__builtin_fmaf(-d, q, n), r, q);
+}
 __device__ __forceinline__ float silu_f32(float z) { return z / (1.0f + __expf(-z)); }
+// (below -69 a result is under 1e-28: exp(69) is what the quotient takes; above 100 it is z, an infinity too)
+__device__ __forceinline__ float silu_run(float z) { return z > 100.f ? z : quotient(z, 1.0f + __expf(fminf(-z, 69.f))); }
 // log(1 + x) = log(u) x / (u - 1) with u the rounded 1 + x: what the sum loses of x comes back (Kahan)
 __device__ __forceinline__ float softplus_f32(float z) {
   const float x = __expf(-fabsf(z)), u = 1.0f + x;
@@ -93,10 +106,11 @@ __device__ __forceinline__ void conv_run4(const slm_recurrent_args& a, const E* 
 #pragma unroll
   for (int j = 0; j < 4; ++j) w[j] = j < a.taps ? a.conv_w[(int64_t)(a.taps - 1 - j) * ch + c] : 0.f;
 #pragma unroll
-  for (int j = 1; j < 4; ++j) {
-    x[3 - j] = 0.f;
-    if (j < a.taps && p >= j)
-      x[3 - j] = row - j >= row0 ? to_f32(src[-j * a.ld_proj]) : to_f32(ring[(int64_t)((p - j) % a.taps) * ch + c]);
+  for (int j = 1; j < 4; ++j) {   // (no branch around a load; where there is no such input, an entry of the ring is read for nothing)
+    const bool there = j < a.taps && p >= j;
+    const E* before = row - j >= row0 ? src - j * a.ld_proj : ring + (int64_t)(there ? (p - j) % a.taps : 0) * ch + c;
+    x[3 - j] = to_f32(*before);
+    x[3 - j] = there ? x[3 - j] : 0.f;
   }
 #pragma unroll
   for (int t = 0; t < 16; ++t) x[3 + t] = to_f32(src[min(t, n - 1) * a.ld_proj]);
@@ -105,7 +119,7 @@ __device__ __forceinline__ void conv_run4(const slm_recurrent_args& a, const E* 
     float acc = w[3] * x[t];
 #pragma unroll
     for (int j = 2; j >= 0; --j) acc = __builtin_fmaf(w[j], x[3 + t - j], acc);
-    put(t, t < n ? silu_f32(acc) : 0.f);
+    put(t, t < n ? silu_run(acc) : 0.f);
   }
 }
 template <typename E>
@@ -294,28 +308,40 @@ __global__ void __launch_bounds__(1024) recurrent_step_kernel(const slm_recurren
 //   (I + diag(beta) A) U = diag(beta) (V - Kd S0)     A_ts = sum_d k_t k_s exp(L_t - L_s), s < t;  Kd_t = k_t exp(L_t)
 //   O  = Qd S0 + B U                                  B_ts = sum_d q_t k_s exp(L_t - L_s), s <= t; Qd_t = q_t exp(L_t)
 //   S1 = diag(exp(L_end)) S0 + Kr^T U                 Kr_t = k_t exp(L_end - L_t)
-// Every exponent is <= 0: nothing overflows however fast a channel forgets.  Without the delta rule U = V.
+// Every exponent is <= 0: nothing overflows however fast a channel forgets.  Without the delta rule U = V.  With T = (I + diag(beta) A)^-1 diag(beta),
+// what does not wait for S0 is worked out chunk by chunk in prepare, and the scan's chain is two products and an exchange long:
+//   U = V' - Kd' S0     O = O0 + Qd' S0     V' = T V, Kd' = T Kd, O0 = B T V, Qd' = Qd - B T Kd
 // A chunk's record for one head, in floats:
-//   Kd | Qd (16 x DK each) | Kr^T (DK x 16) | exp(L_end) (DK) | V^T (v_pad x 16) | T = (I + diag(beta) A)^-1 diag(beta) | B (16 x 16)
-// Matrices are tiles of 16 x 16 in the order the scan's lanes take them, four floats a lane: entry (m, k) at
-// tile_at(m, k), so that a wave reads a tile as 1 KiB in a row.  Kd, Qd: m token, k channel; Kr^T, V^T: m channel / column,
-// k token; T, B: m row, k column.
-__device__ __forceinline__ int tile_at(int m, int k) { return (((k >> 2) & 3) * 16 + (m & 15)) * 4 + (k & 3); }
+//   Kd' | Qd' (16 x DK each) | Kr^T (DK x 16) | exp(L_end) (DK) | V'^T | O0^T (v_pad x 16 each)
+// Matrices are tiles of 16 x 16 in the order the scan's lanes take them, four floats a lane: entry (m, k) at ((k / 4 % 4) 16 + m % 16) 4 + k % 4, so
+// that a wave reads a tile as 1 KiB in a row.  Kd', Qd': m token, k channel; Kr^T, V'^T, O0^T: m channel / column, k token.
 template <int DK>
 struct ChunkRecord {
   static constexpr int KD = 0, QD = 16 * DK, KR = 32 * DK, GE = 48 * DK, V = 49 * DK;
   int v_pad;
-  __device__ __forceinline__ int t() const { return V + 16 * v_pad; }
-  __device__ __forceinline__ int b() const { return t() + 256; }
-  __device__ __forceinline__ int64_t size() const { return b() + 256; }
+  __device__ __forceinline__ int o0() const { return V + 16 * v_pad; }
+  __device__ __forceinline__ int64_t size() const { return o0() + 16 * v_pad; }
 };
+// What 32-bit products have just left in x, before a branch that its first reader lies behind (the compiler counts the wait along one way there only)
+__device__ __forceinline__ void settle(f32x4& x) { asm volatile("s_nop 15" : "+v"(x)); }
+// c + x y^T over four contraction indexes a lane: lane (l16, g) has x [l16][4 g ..] and y [l16][4 g ..], and gets [4 g ..][l16]
+__device__ __forceinline__ f32x4 mma4(const f32x4& x, const f32x4& y, f32x4 c) {
+#pragma unroll
+  for (int r = 0; r < 4; ++r) c = __builtin_amdgcn_mfma_f32_16x16x4f32(x[r], y[r], c, 0, 0, 0);
+  return c;
+}
 
-// one workgroup per (chunk, head); every chunk of the step at once
+// one workgroup per (chunk, head); every chunk of the step at once.  A and B are 32-bit MFMAs of k exp(L), q exp(L) and k exp(-L) where no channel of
+// the chunk falls below 2^-96 (each entry's factors then are in range, their product is below 1); else entry by entry, an exponential for
+// each of the 16 x 16 x DK terms.
+constexpr float DIRECT_BELOW = -96.f;
 template <typename E, int MODE, int DK>
 __global__ void __launch_bounds__(256) recurrent_prepare_kernel(const slm_recurrent_args a) {
   constexpr bool DELTA = DELTA_MODE(MODE);
   constexpr int LD = DK + 4;                     // (the 16 rows a quarter-wave reads by 16 bytes are in different banks)
-  __shared__ __attribute__((aligned(16))) float sq[16 * LD], sk[16 * LD], sL[16 * LD];
+  constexpr int TPW = (DK / 16 + 3) / 4;         // channel tiles of a wave: wave, wave + 4 ..
+  __shared__ __attribute__((aligned(16))) float sq[16 * LD > 2048 ? 16 * LD : 2048], sk[16 * LD], sL[DELTA ? 16 * LD : 1], sb[16 * 20], sT[16 * 20];
+  extern __shared__ __attribute__((aligned(16))) float sv[];   // 16 x v_pad, as in the record
   __shared__ float sa[16][17], sbeta[16];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int head = blockIdx.x % a.heads;
@@ -333,6 +359,17 @@ __global__ void __launch_bounds__(256) recurrent_prepare_kernel(const slm_recurr
   const E* in = reinterpret_cast<const E*>(a.proj) + row * a.ld_proj;
   const float step_l = DELTA ? 0.f : fmaxf(log2f(a.decay[head]), -126.f);
 
+  // every input's load before its use: one after the other they were this kernel's length
+  constexpr int PER = DK / 16;   // (token, channel) pairs of a thread
+  float decay_in[PER], decay_bias[PER];
+  if constexpr (DELTA) {
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      const int t = min((tid + 256 * j) / DK, n - 1), c = min((tid + 256 * j) % DK, a.dim - 1);
+      decay_in[j] = to_f32(reinterpret_cast<const E*>(a.low)[(row + t) * a.ld_low + (int64_t)head * a.dim + c]);
+      decay_bias[j] = a.dt_bias[head * a.dim + c];
+    }
+  }
   if (DELTA && a.taps <= 4) {
     for (int i = tid; i < 2 * DK + a.v_pad; i += 256) {
       if (i < 2 * DK) {
@@ -347,7 +384,7 @@ __global__ void __launch_bounds__(256) recurrent_prepare_kernel(const slm_recurr
         }
       } else {
         const int c = i - 2 * DK;
-        float* dst = rec + ChunkRecord<DK>::V + (c >> 4) * 256 + (c & 15) * 4;
+        float* dst = sv + (c >> 4) * 256 + (c & 15) * 4;
         f32x4 four;
         auto put = [&](int t, float x) {
           four[t & 3] = x;
@@ -361,39 +398,54 @@ __global__ void __launch_bounds__(256) recurrent_prepare_kernel(const slm_recurr
         }
       }
     }
-  } else {
+  } else if constexpr (DELTA) {
     for (int i = tid; i < 16 * DK; i += 256) {
       const int t = i / DK, c = i % DK;
       float q = 0.f, k = 0.f;
       if (t < n && c < a.dim) {
-        if constexpr (DELTA) {
-          q = conv_input<E>(a, ring, row + t, row0, p + t, qh * a.dim + c);
-          k = conv_input<E>(a, ring, row + t, row0, p + t, qk + qh * a.dim + c);
-        } else {
-          q = silu_f32(to_f32(in[t * a.ld_proj + a.off_q + qh * a.dim + c]));
-          k = silu_f32(to_f32(in[t * a.ld_proj + a.off_k + qh * a.dim + c]));
-        }
+        q = conv_input<E>(a, ring, row + t, row0, p + t, qh * a.dim + c);
+        k = conv_input<E>(a, ring, row + t, row0, p + t, qk + qh * a.dim + c);
       }
       sq[t * LD + c] = q, sk[t * LD + c] = k;
     }
     for (int i = tid; i < 16 * a.v_pad; i += 256) {   // (in the record's order)
       const int t = ((i >> 6) & 3) * 4 + (i & 3), c = (i >> 8) * 16 + ((i >> 2) & 15);
-      float v = 0.f;
-      if (t < n && c < a.vdim) {
-        if constexpr (DELTA) v = conv_input<E>(a, ring, row + t, row0, p + t, 2 * qk + head * a.vdim + c);
-        else v = silu_f32(to_f32(in[t * a.ld_proj + a.off_v + head * a.vdim + c]));
+      sv[i] = t < n && c < a.vdim ? conv_input<E>(a, ring, row + t, row0, p + t, 2 * qk + head * a.vdim + c) : 0.f;
+    }
+  } else {
+    float q[PER], k[PER], v[4];
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      const int t = min((tid + 256 * j) / DK, n - 1), c = min((tid + 256 * j) % DK, a.dim - 1);
+      q[j] = to_f32(in[t * a.ld_proj + a.off_q + qh * a.dim + c]);
+      k[j] = to_f32(in[t * a.ld_proj + a.off_k + qh * a.dim + c]);
+    }
+    for (int i0 = tid; i0 < 16 * a.v_pad; i0 += 1024) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int t = min((i0 + 256 * j) / a.v_pad, n - 1), c = min((i0 + 256 * j) % a.v_pad, a.vdim - 1);
+        v[j] = to_f32(in[(int64_t)t * a.ld_proj + a.off_v + head * a.vdim + c]);
       }
-      rec[ChunkRecord<DK>::V + i] = v;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int t = (i0 + 256 * j) / a.v_pad, c = (i0 + 256 * j) % a.v_pad;
+        if (t < 16) sv[(c >> 4) * 256 + (t >> 2) * 64 + (c & 15) * 4 + (t & 3)] = t < n && c < a.vdim ? silu_run(v[j]) : 0.f;
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      const int t = (tid + 256 * j) / DK, c = (tid + 256 * j) % DK;
+      const bool there = t < n && c < a.dim;
+      sq[t * LD + c] = there ? silu_run(q[j]) : 0.f, sk[t * LD + c] = there ? silu_run(k[j]) : 0.f;
     }
   }
-  for (int i = tid; i < 16 * DK; i += 256) {
-    const int t = i / DK, c = i % DK;
-    float l = 0.f;
-    if (t < n && c < a.dim) {
-      if constexpr (DELTA) l = LOG2E_F * decay_exponent<E>(a, row + t, head, c);
-      else l = step_l;
+  if constexpr (DELTA) {
+    const float neg_a = a.neg_a[head];
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      const int t = (tid + 256 * j) / DK, c = (tid + 256 * j) % DK;
+      sL[t * LD + c] = t < n && c < a.dim ? LOG2E_F * (neg_a * softplus_f32(decay_in[j] + decay_bias[j])) : 0.f;
     }
-    sL[t * LD + c] = l;
   }
   if (DELTA && tid < 16) sbeta[tid] = tid < n ? sigmoid_full(to_f32(in[tid * a.ld_proj + a.off_b + head])) : 0.f;
   __syncthreads();
@@ -410,92 +462,147 @@ __global__ void __launch_bounds__(256) recurrent_prepare_kernel(const slm_recurr
       for (int c = lane; c < DK; c += 64) sq[t * LD + c] *= fq, sk[t * LD + c] *= fk;
     }
   }
+  float lowest = step_l * n;   // (without the delta rule a token's channels decay alike)
   if (tid < DK) {
-    float l = 0.f;
+    if constexpr (DELTA) {
+      float l = 0.f;
 #pragma unroll
-    for (int t = 0; t < 16; ++t) {
-      l += sL[t * LD + tid];
-      sL[t * LD + tid] = l;
+      for (int t = 0; t < 16; ++t) {
+        l += sL[t * LD + tid];
+        sL[t * LD + tid] = l;
+      }
+      lowest = l;
+    }
+    rec[ChunkRecord<DK>::GE + tid] = fast_exp2(lowest);
+  }
+  const bool direct = __syncthreads_or(lowest < DIRECT_BELOW || !(lowest <= 0.f));
+  const int l16 = lane & 15, g = lane >> 4;
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  auto lds4 = [](const float* p) { return *reinterpret_cast<const f32x4*>(p); };
+  auto summed = [&](int t, int c) { return DELTA ? sL[t * LD + c] : step_l * min(t + 1, n); };
+  auto exp4 = [](const f32x4& l) { return f32x4{fast_exp2(l.x), fast_exp2(l.y), fast_exp2(l.z), fast_exp2(l.w)}; };
+
+  f32x4 qd[TPW], pa = zero, pb = zero;   // lane: token l16, channels 4 g .. of a tile
+#pragma unroll
+  for (int j = 0; j < TPW; ++j) {
+    const int tile = wave + 4 * j;
+    if (tile >= DK / 16) continue;
+    const int at_t = l16 * LD + 16 * tile + 4 * g;
+    f32x4 l;
+    if constexpr (DELTA) l = lds4(sL + at_t);
+    else l = zero + summed(l16, 0);
+    const f32x4 e = exp4(l), k = lds4(sk + at_t);
+    qd[j] = lds4(sq + at_t) * e;
+    if (!direct) {
+      const f32x4 ks = k * exp4(-l);
+      if constexpr (DELTA) pa = mma4(k * e, ks, pa);
+      pb = mma4(qd[j], ks, pb);
     }
   }
-  __syncthreads();
-  {
+  settle(pa);
+  settle(pb);
+  if (!direct) {
+    f32x4 (*const part)[2][64] = reinterpret_cast<f32x4 (*)[2][64]>(sq);
+    __syncthreads();   // (nobody reads q any more)
+    if constexpr (DELTA) part[wave][0][lane] = pa;
+    part[wave][1][lane] = pb;
+    __syncthreads();
+    if (wave < 2 && (DELTA || wave == 1)) {   // lane: rows 4 g .., column l16
+      f32x4 sum = part[0][wave][lane];
+#pragma unroll
+      for (int w = 1; w < 4; ++w) sum += part[w][wave][lane];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int t = 4 * g + r;
+        if (wave == 0) sa[t][l16] = l16 < t ? sum[r] : 0.f;
+        else sb[t * 20 + l16] = l16 <= t ? sum[r] : 0.f;
+      }
+    }
+  } else {
     const int t = tid >> 4, s = tid & 15;
     float x = 0.f, y = 0.f;
     if (s <= t) {
-      if constexpr (DELTA) {
 #pragma unroll 2
-        for (int c = 0; c < DK; c += 4) {
-          const f32x4 ks = *reinterpret_cast<const f32x4*>(sk + s * LD + c), ls = *reinterpret_cast<const f32x4*>(sL + s * LD + c);
-          const f32x4 kt = *reinterpret_cast<const f32x4*>(sk + t * LD + c), lt = *reinterpret_cast<const f32x4*>(sL + t * LD + c);
-          const f32x4 qt = *reinterpret_cast<const f32x4*>(sq + t * LD + c);
+      for (int c = 0; c < DK; c += 4) {
+        const f32x4 ks = lds4(sk + s * LD + c), kt = lds4(sk + t * LD + c), qt = lds4(sq + t * LD + c);
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const float e = ks[j] * fast_exp2(lt[j] - ls[j]);
-            x = __builtin_fmaf(kt[j], e, x);
-            y = __builtin_fmaf(qt[j], e, y);
-          }
+        for (int j = 0; j < 4; ++j) {
+          const float e = ks[j] * fast_exp2(summed(t, c + j) - summed(s, c + j));
+          x = __builtin_fmaf(kt[j], e, x);
+          y = __builtin_fmaf(qt[j], e, y);
         }
-      } else {
-#pragma unroll 2
-        for (int c = 0; c < DK; c += 4) {
-          const f32x4 ks = *reinterpret_cast<const f32x4*>(sk + s * LD + c), qt = *reinterpret_cast<const f32x4*>(sq + t * LD + c);
-#pragma unroll
-          for (int j = 0; j < 4; ++j) y = __builtin_fmaf(qt[j], ks[j], y);
-        }
-        y *= fast_exp2(sL[t * LD] - sL[s * LD]);
       }
     }
-    rec[at.b() + tile_at(t, s)] = y;
+    sb[t * 20 + s] = y;
     sa[t][s] = x;
   }
-  for (int i = tid; i < 4 * DK; i += 256) {   // four floats each, in the record's order
-    const int tile = i >> 6, m = i & 15, k = ((i >> 4) & 3) * 4;
-    {
-      const int at_t = m * LD + 16 * tile + k;
-      const f32x4 l = *reinterpret_cast<const f32x4*>(sL + at_t), q = *reinterpret_cast<const f32x4*>(sq + at_t);
-      const f32x4 e = {fast_exp2(l.x), fast_exp2(l.y), fast_exp2(l.z), fast_exp2(l.w)};
-      if constexpr (DELTA) *reinterpret_cast<f32x4*>(rec + ChunkRecord<DK>::KD + 4 * i) = *reinterpret_cast<const f32x4*>(sk + at_t) * e;
-      *reinterpret_cast<f32x4*>(rec + ChunkRecord<DK>::QD + 4 * i) = q * e;
-    }
-    const int d = 16 * tile + m;
-    f32x4 kr;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) kr[j] = sk[(k + j) * LD + d] * fast_exp2(sL[15 * LD + d] - sL[(k + j) * LD + d]);
-    *reinterpret_cast<f32x4*>(rec + ChunkRecord<DK>::KR + 4 * i) = kr;
-  }
-  if (tid < DK) rec[ChunkRecord<DK>::GE + tid] = fast_exp2(sL[15 * LD + tid]);
+  __syncthreads();
+  f32x4 tv, bt = lds4(sb + l16 * 20 + 4 * g);   // rows l16, columns 4 g .. of T and of B T (without the delta rule: of B)
   if constexpr (DELTA) {
-    __syncthreads();
     if (tid < 16) {   // column tid of T by forward substitution
       float x[16];
 #pragma unroll
-      for (int t = 0; t < 16; ++t) {
-        float v = t == tid ? 1.0f : 0.f;
+      for (int t = 0; t < 16; ++t) x[t] = t == tid ? 1.0f : 0.f;
 #pragma unroll
-        for (int s = 0; s < t; ++s) v = __builtin_fmaf(-sa[t][s], x[s], v);
-        x[t] = sbeta[t] * v;
-        rec[at.t() + tile_at(t, tid)] = x[t];
+      for (int s = 0; s < 16; ++s) {
+        x[s] *= sbeta[s];
+        sT[s * 20 + tid] = x[s];
+#pragma unroll
+        for (int t = s + 1; t < 16; ++t) x[t] = __builtin_fmaf(-sa[t][s], x[s], x[t]);
       }
     }
+    __syncthreads();
+    tv = lds4(sT + l16 * 20 + 4 * g);
+    f32x4 tt;   // row l16, columns 4 g .. of T^T
+#pragma unroll
+    for (int r = 0; r < 4; ++r) tt[r] = sT[(4 * g + r) * 20 + l16];
+    bt = mma4(tt, bt, zero);
+    settle(bt);
+  }
+#pragma unroll
+  for (int j = 0; j < TPW; ++j) {
+    const int tile = wave + 4 * j;
+    if (tile >= DK / 16) continue;
+    const int d = 16 * tile + l16;
+    const float end = summed(15, d);
+    f32x4 kr, kd;   // channel d, tokens 4 g ..
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float k = sk[(4 * g + r) * LD + d], l = summed(4 * g + r, d);
+      kr[r] = k * fast_exp2(end - l);
+      kd[r] = k * fast_exp2(l);
+    }
+    float* at_tile = rec + 256 * tile + 4 * lane;
+    *reinterpret_cast<f32x4*>(at_tile + ChunkRecord<DK>::KR) = kr;
+    if constexpr (DELTA) {
+      *reinterpret_cast<f32x4*>(at_tile + ChunkRecord<DK>::KD) = mma4(kd, tv, zero);
+      qd[j] = mma4(-kd, bt, qd[j]);
+    }
+    *reinterpret_cast<f32x4*>(at_tile + ChunkRecord<DK>::QD) = qd[j];
+  }
+  for (int tile = wave; tile < a.v_pad / 16; tile += 4) {
+    const f32x4 v = lds4(sv + 256 * tile + 4 * lane);   // column l16, tokens 4 g ..
+    float* at_tile = rec + ChunkRecord<DK>::V + 256 * tile + 4 * lane;
+    *reinterpret_cast<f32x4*>(at_tile) = DELTA ? mma4(tv, v, zero) : v;
+    *reinterpret_cast<f32x4*>(at_tile + 16 * a.v_pad) = mma4(bt, v, zero);
   }
 }
 
 // One workgroup per (sequence, head, 16 NCT columns of S), chunk after chunk.  Its waves share the key channels: a wave
 // keeps TPW tiles [16 x 16] of every column tile of S in registers in the accumulator layout of the 32-bit MFMA (row 4 g + r,
 // column l16), which is the layout its right operand takes when the contraction index of product r is 4 g + r.  Partial
-// products with S0 meet in LDS, one barrier a chunk; U is computed by every wave; read-outs are completed a chunk later.  The operands of the next chunks travel
-// meanwhile.  Two column tiles read the records half as often: where enough workgroups are left.
+// products with S0 meet in LDS, one barrier a chunk, the read-outs' products run under it; read-outs are completed a chunk later.  The operands of the
+// next chunks travel meanwhile.  Two column tiles read the records half as often: where enough workgroups are left.
 template <int TPW, int NCT>
 struct ChunkOperands {
-  f32x4 kd[TPW], qd[TPW], kr[TPW], ge[TPW], t, b, v[NCT];
+  f32x4 kd[TPW], qd[TPW], kr[TPW], ge[TPW], v[NCT], o0[NCT];
 };
 
 template <typename E, int MODE, int DK, int W, int NCT>
 __global__ void __launch_bounds__(64 * W, 2) recurrent_scan_kernel(const slm_recurrent_args a) {
   constexpr bool DELTA = DELTA_MODE(MODE);
   constexpr int TPW = DK / 16 / W;
-  constexpr int NB = TPW <= (DELTA ? 1 : 2) ? 3 : 2;   // chunks in registers: one in use, the others on their way
+  constexpr int NB = TPW <= 1 || (TPW == 2 && (NCT == 1 || !DELTA)) ? 3 : 2;   // chunks in registers: one in use, the others on their way
   __shared__ f32x4 part_u[2][NCT][W][64], part_o[2][NCT][W][64];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, g = lane >> 4;
@@ -525,83 +632,109 @@ __global__ void __launch_bounds__(64 * W, 2) recurrent_scan_kernel(const slm_rec
 #pragma unroll
       for (int r = 0; r < 4; ++r) s[j][i][r] = p0 > 0 ? S[(int64_t)(16 * i + r) * a.v_pad + 16 * ct[j]] : 0.f;
 
-  // uniform bases and 32-bit lane offsets: an address is one register
-  auto vec = [](const float* base, uint32_t off) { return *reinterpret_cast<const f32x4*>(reinterpret_cast<const char*>(base) + off); };
-  const uint32_t off = (uint32_t)lane * 16, ge_off = (uint32_t)g * 16;
+  // a chunk's record is a buffer: a load is one instruction (of 64-bit addresses half of a chunk's 215 instructions were additions)
+  const int rec_bytes = (int)at.size() * 4;
+  const uint32_t off = (uint32_t)(lane * 16), koff = off + wave * (TPW * 1024), goff = (uint32_t)(g * 16 + wave * (TPW * 64) + ChunkRecord<DK>::GE * 4);
   auto load = [&](int c, ChunkOperands<TPW, NCT>& x) {
-    const float* rec = rec0 + c * rec_step;
+    const __amdgpu_buffer_rsrc_t rec = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(rec0 + c * rec_step), 0, rec_bytes, 0x00020000);
+    auto vec = [&](uint32_t at_lane, int from) { return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rec, at_lane, from, 0)); };
 #pragma unroll
     for (int i = 0; i < TPW; ++i) {
-      const int tile = TPW * wave + i;
-      if constexpr (DELTA) x.kd[i] = vec(rec + ChunkRecord<DK>::KD + 256 * tile, off);
-      x.qd[i] = vec(rec + ChunkRecord<DK>::QD + 256 * tile, off);
-      x.kr[i] = vec(rec + ChunkRecord<DK>::KR + 256 * tile, off);
-      x.ge[i] = vec(rec + ChunkRecord<DK>::GE + 16 * tile, ge_off);
+      if constexpr (DELTA) x.kd[i] = vec(koff + i * 1024, ChunkRecord<DK>::KD * 4);
+      x.qd[i] = vec(koff + i * 1024, ChunkRecord<DK>::QD * 4);
+      x.kr[i] = vec(koff + i * 1024, ChunkRecord<DK>::KR * 4);
+      x.ge[i] = vec(goff + i * 64, 0);
     }
-    if constexpr (DELTA) x.t = vec(rec + at.t(), off);
-    x.b = vec(rec + at.b(), off);
 #pragma unroll
-    for (int j = 0; j < NCT; ++j) x.v[j] = vec(rec + ChunkRecord<DK>::V + 256 * ct[j], off);
+    for (int j = 0; j < NCT; ++j) {
+      x.v[j] = vec(off, ChunkRecord<DK>::V * 4 + 1024 * ct[j]);
+      x.o0[j] = vec(off, at.o0() * 4 + 1024 * ct[j]);
+    }
   };
-  auto mma4 = [](const f32x4& x, const f32x4& y, f32x4 c) {
+  // the read-outs of a chunk, once every wave's part of them is there: of each lane's four rows a wave takes one (of 2 waves: two)
+  const int o_row = a.heads * a.v_pad * 4;   // bytes
+  float* const o_from = a.o + (row0 - a.n_single) * a.heads * a.v_pad;
+  const uint32_t o_off = (uint32_t)((4 * g + wave) * o_row + (head * a.v_pad + l16) * 4);
+  struct ReadOuts { float v[4 / W][NCT][W]; };
+  auto collect = [&](int c, ReadOuts& y) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) c = __builtin_amdgcn_mfma_f32_16x16x4f32(x[r], y[r], c, 0, 0, 0);
-    return c;
+    for (int r = 0; r < 4 / W; ++r)
+#pragma unroll
+      for (int j = 0; j < NCT; ++j)
+#pragma unroll
+        for (int w = 0; w < W; ++w) y.v[r][j][w] = reinterpret_cast<const float*>(&part_o[c & 1][j][w][lane])[r * W + wave];
   };
-  auto finish = [&](int c) {   // the read-outs of chunk c, once every wave's part of them is there
+  auto finish = [&](int c, const ReadOuts& y) {   // (rows past the portion's last, and chunk -1, are out of the buffer)
+    const __amdgpu_buffer_rsrc_t out = __builtin_amdgcn_make_buffer_rsrc(o_from + (int64_t)16 * c * a.heads * a.v_pad, 0, c < 0 ? 0 : min(n - 16 * c, 16) * o_row, 0x00020000);
 #pragma unroll
-    for (int j = 0; j < NCT; ++j)
-      if ((c * NCT + j + W / 2) % W == wave && cb * NCT + j < n_ct) {
-        f32x4 y = part_o[c & 1][j][0][lane];
+    for (int r = 0; r < 4 / W; ++r)
 #pragma unroll
-        for (int w = 1; w < W; ++w) y += part_o[c & 1][j][w][lane];
-        float* dst = a.o + ((row0 - a.n_single + 16 * c) * a.heads + head) * a.v_pad + 16 * ct[j];
-        const uint32_t o_off = (uint32_t)(4 * g * a.heads * a.v_pad + l16) * 4;
+      for (int j = 0; j < NCT; ++j) {
+        float sum = y.v[r][j][0];
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (16 * c + 4 * g + r < n)
-            *reinterpret_cast<float*>(reinterpret_cast<char*>(dst + (int64_t)r * a.heads * a.v_pad) + o_off) = y[r];
+        for (int w = 1; w < W; ++w) sum += y.v[r][j][w];
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, sum), out, o_off + r * W * o_row, 64 * ct[j], 0);
       }
+  };
+  // two sums of tiles side by side: the products of one wait for each other
+  auto products = [&](const f32x4 (&x)[TPW], int j, f32x4 c) {
+    f32x4 d = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int i = 0; i < TPW; ++i) {
+        f32x4& to = i & 1 ? d : c;
+        to = __builtin_amdgcn_mfma_f32_16x16x4f32(x[i][r], s[j][i][r], to, 0, 0, 0);
+      }
+    return TPW > 1 ? c + d : c;
   };
   auto chunk = [&](int c, const ChunkOperands<TPW, NCT>& x) {
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     const int b = c & 1;
-    f32x4 kr[NCT], o[NCT], u[NCT];
-#pragma unroll
-    for (int j = 0; j < NCT; ++j) kr[j] = o[j] = zero;
+    f32x4 o[NCT], u[NCT], pu[NCT][W];
+    ReadOuts y;
     if constexpr (DELTA) {
 #pragma unroll
-      for (int i = 0; i < TPW; ++i)
-#pragma unroll
-        for (int j = 0; j < NCT; ++j) kr[j] = mma4(x.kd[i], s[j][i], kr[j]);
-#pragma unroll
-      for (int j = 0; j < NCT; ++j) part_u[b][j][wave][lane] = kr[j];
+      for (int j = 0; j < NCT; ++j) part_u[b][j][wave][lane] = products(x.kd, j, zero);
+      __builtin_amdgcn_sched_barrier(0);
     }
-    // (what the next chunk does not wait for runs under the exchange)
+    // (the read-outs' products run under the writes of the exchange, of two column tiles the second's under its reads)
 #pragma unroll
-    for (int i = 0; i < TPW; ++i)
-#pragma unroll
-      for (int j = 0; j < NCT; ++j) o[j] = mma4(x.qd[i], s[j][i], o[j]);
+    for (int j = 0; j < (NCT + 1) / 2; ++j) o[j] = products(x.qd, j, wave == 0 ? x.o0[j] : zero);
+    __builtin_amdgcn_sched_barrier(0);
     lds_barrier();
+    if constexpr (DELTA) {
+#pragma unroll
+      for (int j = 0; j < NCT; ++j)
+#pragma unroll
+        for (int w = 0; w < W; ++w) pu[j][w] = part_u[b][j][w][lane];
+    }
+    collect(c - 1, y);   // (in front of the first chunk: of nothing, and not stored)
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = (NCT + 1) / 2; j < NCT; ++j) o[j] = products(x.qd, j, wave == 0 ? x.o0[j] : zero);
+    if constexpr (DELTA && NCT > 1) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int j = 0; j < NCT; ++j) {
       u[j] = x.v[j];
       if constexpr (DELTA) {
 #pragma unroll
-        for (int w = 0; w < W; ++w) u[j] -= part_u[b][j][w][lane];
-        u[j] = mma4(x.t, u[j], zero);
+        for (int w = 0; w < W; ++w) u[j] -= pu[j][w];
       }
     }
 #pragma unroll
-    for (int i = 0; i < TPW; ++i)
+    for (int j = 0; j < NCT; ++j)
 #pragma unroll
-      for (int j = 0; j < NCT; ++j) s[j][i] = mma4(x.kr[i], u[j], s[j][i] * x.ge[i]);
+      for (int i = 0; i < TPW; ++i) s[j][i] *= x.ge[i];
 #pragma unroll
-    for (int j = 0; j < NCT; ++j) {   // (the waves take B U, and the stores a barrier later, in turn)
-      if ((c * NCT + j) % W == wave) o[j] = mma4(x.b, u[j], o[j]);
-      part_o[b][j][wave][lane] = o[j];
-    }
-    if (c > 0) finish(c - 1);
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int i = 0; i < TPW; ++i)
+#pragma unroll
+        for (int j = 0; j < NCT; ++j) s[j][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.kr[i][r], u[j][r], s[j][i], 0, 0, 0);
+#pragma unroll
+    for (int j = 0; j < NCT; ++j) part_o[b][j][wave][lane] = o[j];
+    finish(c - 1, y);
   };
   ChunkOperands<TPW, NCT> x[NB];
 #pragma unroll
@@ -615,10 +748,17 @@ __global__ void __launch_bounds__(64 * W, 2) recurrent_scan_kernel(const slm_rec
     }
   }
 #pragma unroll
-  for (int i = 0; i + 1 < NB; ++i)
+  for (int i = 0; i + 1 < NB; ++i) {
+#pragma unroll
+    for (int j = 0; j < NCT; ++j)
+#pragma unroll
+      for (int t = 0; t < TPW; ++t) settle(s[j][t]);
     if (c0 + i < n_chunks) chunk(c0 + i, x[i]);
+  }
   lds_barrier();
-  finish(n_chunks - 1);
+  ReadOuts y;
+  collect(n_chunks - 1, y);
+  finish(n_chunks - 1, y);
 #pragma unroll
   for (int j = 0; j < NCT; ++j)
     if (cb * NCT + j < n_ct)
@@ -842,13 +982,14 @@ static int rec_scan(const slm_recurrent_args& a, hipStream_t st) {
 template <typename E, int MODE>
 static int rec_prepare(const slm_recurrent_args& a, hipStream_t st) {
   const dim3 grid((unsigned)((int64_t)a.n_chunks * a.heads)), block(256);
+  const size_t lds = (size_t)a.v_pad * 64;
   hip_clear_error();
   switch (a.dim_pad) {
-    case 32: recurrent_prepare_kernel<E, MODE, 32><<<grid, block, 0, st>>>(a); break;
-    case 64: recurrent_prepare_kernel<E, MODE, 64><<<grid, block, 0, st>>>(a); break;
-    case 128: recurrent_prepare_kernel<E, MODE, 128><<<grid, block, 0, st>>>(a); break;
-    case 192: recurrent_prepare_kernel<E, MODE, 192><<<grid, block, 0, st>>>(a); break;
-    default: recurrent_prepare_kernel<E, MODE, 256><<<grid, block, 0, st>>>(a);
+    case 32: recurrent_prepare_kernel<E, MODE, 32><<<grid, block, lds, st>>>(a); break;
+    case 64: recurrent_prepare_kernel<E, MODE, 64><<<grid, block, lds, st>>>(a); break;
+    case 128: recurrent_prepare_kernel<E, MODE, 128><<<grid, block, lds, st>>>(a); break;
+    case 192: recurrent_prepare_kernel<E, MODE, 192><<<grid, block, lds, st>>>(a); break;
+    default: recurrent_prepare_kernel<E, MODE, 256><<<grid, block, lds, st>>>(a);
   }
   return hip_check_launch();
 }
@@ -877,7 +1018,7 @@ extern "C" SLM_API int slm_recurrent_step(const slm_recurrent_args* a, void* str
 static bool rec_chunks_ok(const slm_recurrent_args& a) {
   return a.pre && a.chunks && a.seq_chunks && a.n_chunks >= 0 && (int64_t)a.n_chunks * a.heads <= 0x7fffffff;
 }
-extern "C" SLM_API int64_t slm_recurrent_record_floats(int32_t dim_pad, int32_t v_pad) { return 49 * (int64_t)dim_pad + 16 * (int64_t)v_pad + 512; }
+extern "C" SLM_API int64_t slm_recurrent_record_floats(int32_t dim_pad, int32_t v_pad) { return 49 * (int64_t)dim_pad + 32 * (int64_t)v_pad; }
 extern "C" SLM_API int slm_recurrent_prepare(const slm_recurrent_args* a, void* stream) {
   if (!a || !rec_sizes_ok(*a) || !rec_ptrs_ok(*a) || !rec_chunks_ok(*a)) return SLM_ERR_INVALID_ARG;
   if (!aligned16(a->pre)) return SLM_ERR_ALIGNMENT;

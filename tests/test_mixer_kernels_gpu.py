@@ -89,6 +89,20 @@ def test_channel_delta(heads, kv_heads, dim, vdim, taps, width, dtype):
     _serve(layer, width, dtype, lambda h: ref.channel_delta(h, _f64(w), m, 1e-5), 1e-5)
 
 
+# Channels that forget on both sides of 2^-96 a chunk, where what tokens do to each other is one product of factors, or an exponential a term; a chunk has
+# some of either, or of the first only.  Sums of 32 bits whatever the way: the bound is test_channel_delta's.
+@pytest.mark.parametrize("dtype", BOTH)
+@pytest.mark.parametrize("dim", [20, 128, 200])
+@pytest.mark.parametrize("faster", [(6.0, 0.0, 3.5), (3.0, 4.0, 4.4)])
+def test_channel_delta_that_forgets_fast(faster, dim, dtype):
+    from scalellm_amd.mixer_layers import ChannelDelta, ChannelDeltaArgs
+    m = {"heads": 3, "kv_heads": 3, "dim": dim, "vdim": 40, "conv": 4}
+    w = mixer_weights("channel_delta", m, 64, random_tensors(5))
+    w["A_log"] = w["A_log"] + torch.tensor(faster, dtype=w["A_log"].dtype)
+    layer = ChannelDelta(ChannelDeltaArgs(3, 3, dim, 40, 4), 64, 1e-5, w, dtype, DEV)
+    _serve(layer, 64, dtype, lambda h: ref.channel_delta(h, _f64(w), m, 1e-5), 1e-5)
+
+
 class _Alone:
     """One half of a parallel mixer as a layer of its own."""
 
