@@ -1099,6 +1099,7 @@ SLM_API int slm_paged_kv_varlen_mha(const slm_attn_args* a, void* stream) {
   kp.rows_lo = 0;
   kp.rows_hi = 0x7fffffff;
   kp.bal = pl.bal; kp.part_slots = pl.part_slots; kp.bal_qmin = pl.bal_qmin; kp.bal_align = ATTN_BAL_ALIGN;
+  kp.packed = 0;
   kp.prio = tune_get(TUNE_ATTN_PRIO, 1);  // measured on the two-lane bs 256 step: 25.08 -> 24.85 ms (2 x 2 runs)
   const bool scratch = a->workspace && a->workspace_bytes >= part_bytes(a, pl);
   const bool own_small = pl.small_splits > 1 && scratch;  // only the one-wave tiles are split (without scratch: none)

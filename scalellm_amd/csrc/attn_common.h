@@ -46,6 +46,7 @@ struct AttnKParams {
   int bal_align;
   int part_slots;  // partial slots per (token, head): n_splits (classic) or the piece bound (balanced)
   int part_rows;   // > 0: partials lie by (sequence, its token), part_rows of them a sequence: only short sequences have any
+  int packed;      // tile kernel: the grid counts the tiles of its own sequences (launch_attn_tile)
   int prio;        // > 0: the token kernel raises its wave priority (attn.hip)
 };
 
