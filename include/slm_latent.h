@@ -98,6 +98,8 @@ typedef struct slm_latent_append_args {
   float eps;
 } slm_latent_append_args;
 SLM_API int slm_latent_append(const slm_latent_append_args* a, void* stream);
+/* slm_latent_append, then slm_linear (STORE: the queries of q_abs's rows, absorbed); one launch where that is the same */
+SLM_API int slm_latent_append_absorb(const slm_latent_append_args* a, const slm_linear_args* absorb, void* stream);
 
 /* ---- 4. attention over the paged latent cache (absorbed queries), one work item per query row ----- */
 /* scores q_abs . row * scale over positions [max(0, p - window + 1), p]; out = soft-max weighted latent */

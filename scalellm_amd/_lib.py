@@ -292,6 +292,7 @@ def latent_lib() -> C.CDLL:
         ("slm_clamped_glu", C.c_int, [ptr, ptr, i64, i64, i64, i64, f32, f32, f32, i32, ptr]),
         ("slm_glu_slabs", C.c_int, [ptr, ptr, i64, i64, i32, i64, f32, f32, f32, ptr]),
         ("slm_latent_append", C.c_int, [P(LatentAppendArgs), ptr]),
+        ("slm_latent_append_absorb", C.c_int, [P(LatentAppendArgs), P(LinearArgs), ptr]),
         ("slm_latent_attn_workspace_bytes", C.c_size_t, [P(LatentAttnArgs)]),
         ("slm_latent_attn", C.c_int, [P(LatentAttnArgs), ptr]),
         ("slm_latent_attn_is_mfma", C.c_int, [i32, i32, i32]),

@@ -6,7 +6,7 @@
 // the 16 consecutive k of row r that start at 16 g -- the four lane groups of a row read one whole 128-byte
 // line in bf16 -- and feeds them to the MFMAs in an order of k that is the same for both operands, so no
 // shuffle is needed.  The waves' partial tiles meet in LDS; the epilogue runs there.
-#include "latent_common.h"
+#include "latent_append.h"
 
 namespace slm {
 
@@ -50,14 +50,13 @@ struct KStep<float> {
 
 // GLU: the NT blocks are NT / 2 pairs (gate block, up block half columns further)
 template <typename E, int MT, int NT, int U, int EPI>
-__global__ void __launch_bounds__(256) linear_kernel(const slm_linear_args a) {
+__device__ __forceinline__ void linear_block(const slm_linear_args& a, const int z) {
   constexpr bool GLU = EPI == SLM_LIN_GLU;
   constexpr int NOUT = GLU ? NT / 2 : NT;  // output column blocks
   static_assert(!GLU || NT % 2 == 0, "gate / up pairs");
   __shared__ f32x4 red[4][NT * MT][64];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r16 = lane & 15, g = lane >> 4;
-  const int z = blockIdx.z;
   const int item = z / a.n_splits, split = z % a.n_splits;
   const int64_t half = a.N / 2;
   const int64_t n_out = GLU ? half : a.N;
@@ -159,30 +158,50 @@ __global__ void __launch_bounds__(256) linear_kernel(const slm_linear_args a) {
 }
 
 template <typename E, int MT, int NT, int U, int EPI>
-static int lin_launch(const slm_linear_args& a, hipStream_t st) {
+__global__ void __launch_bounds__(256) linear_kernel(const slm_linear_args a) {
+  linear_block<E, MT, NT, U, EPI>(a, blockIdx.z);
+}
+// The first `slices` of the grid write a row of the latent cache per workgroup: neither part reads what the other writes.
+template <int MT, int NT, int U>
+__global__ void __launch_bounds__(256) linear_append_kernel(const slm_linear_args a, const slm_latent_append_args c, const int slices) {
+  if ((int)blockIdx.z >= slices) return linear_block<bf16, MT, NT, U, SLM_LIN_STORE>(a, blockIdx.z - slices);
+  const int64_t row = ((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
+  if (row < c.rows) latent_append_row<bf16, 4>(c, row);
+}
+
+template <typename E, int MT, int NT, int U, int EPI>
+static int lin_launch(const slm_linear_args& a, hipStream_t st, const slm_latent_append_args* c) {
   constexpr int NOUT = EPI == SLM_LIN_GLU ? NT / 2 : NT;
   const int64_t n_out = EPI == SLM_LIN_GLU ? a.N / 2 : a.N;
   const int64_t gx = (n_out + 16 * NOUT - 1) / (16 * NOUT), gy = (a.M + 16 * MT - 1) / (16 * MT);
   const int64_t gz = (int64_t)a.batch * a.n_splits;
   if (gx > 0x7fffffff || gy > 65535 || gz > 65535) return SLM_ERR_UNSUPPORTED;
   hip_clear_error();
+  if constexpr (sizeof(E) == 2 && EPI == SLM_LIN_STORE) {
+    if (c) {
+      const int64_t slices = (c->rows + gx * gy - 1) / (gx * gy);
+      if (gz + slices > 65535) return SLM_ERR_UNSUPPORTED;
+      linear_append_kernel<MT, NT, U><<<dim3((unsigned)gx, (unsigned)gy, (unsigned)(gz + slices)), dim3(256), 0, st>>>(a, *c, (int)slices);
+      return hip_check_launch();
+    }
+  }
   linear_kernel<E, MT, NT, U, EPI><<<dim3((unsigned)gx, (unsigned)gy, (unsigned)gz), dim3(256), 0, st>>>(a);
   return hip_check_launch();
 }
 // Tiles by row count: one row block streams W with many steps in flight; with more rows the reads of x weigh as much
 // as those of W, and wider column blocks (where enough of them are left to fill the chip) read x less often.
 template <typename E, int EPI>
-static int lin_shape(const slm_linear_args& a, hipStream_t st) {
+static int lin_shape(const slm_linear_args& a, hipStream_t st, const slm_latent_append_args* c = nullptr) {
   constexpr int P = EPI == SLM_LIN_GLU ? 2 : 1;
   if constexpr (sizeof(E) == 4) {
-    if (a.M <= 16) return lin_launch<E, 1, P, 1, EPI>(a, st);
-    return lin_launch<E, 2, 2, 1, EPI>(a, st);
+    if (a.M <= 16) return lin_launch<E, 1, P, 1, EPI>(a, st, c);
+    return lin_launch<E, 2, 2, 1, EPI>(a, st, c);
   } else {
-    if (a.M <= 4) return lin_launch<E, 1, P, 8 / P, EPI>(a, st);
-    if (a.M <= 16) return lin_launch<E, 1, P, 4 / P, EPI>(a, st);
+    if (a.M <= 4) return lin_launch<E, 1, P, 8 / P, EPI>(a, st, c);
+    if (a.M <= 16) return lin_launch<E, 1, P, 4 / P, EPI>(a, st, c);
     const bool wide = a.N / 64 * a.batch * a.n_splits >= 256;
-    if (a.M <= 32) return wide ? lin_launch<E, 2, 4, 1, EPI>(a, st) : lin_launch<E, 2, 2, 2, EPI>(a, st);
-    return wide ? lin_launch<E, 4, 4, 1, EPI>(a, st) : lin_launch<E, 4, 2, 2, EPI>(a, st);
+    if (a.M <= 32) return wide ? lin_launch<E, 2, 4, 1, EPI>(a, st, c) : lin_launch<E, 2, 2, 2, EPI>(a, st, c);
+    return wide ? lin_launch<E, 4, 4, 1, EPI>(a, st, c) : lin_launch<E, 4, 2, 2, EPI>(a, st, c);
   }
 }
 template <typename E>
@@ -200,7 +219,7 @@ static int lin_epi(const slm_linear_args& a, hipStream_t st) {
 
 using namespace slm;
 
-extern "C" SLM_API int slm_linear(const slm_linear_args* a, void* stream) {
+static int lin_check(const slm_linear_args* a) {
   if (!a || !a->x || !a->w || !a->y || a->M < 0 || a->N <= 0 || a->K <= 0 || a->K % 64 || a->N % 16 || a->batch < 1 ||
       a->n_splits < 1 || a->ldx < a->K || a->ldw < a->K || a->epilogue < 0 || a->epilogue > SLM_LIN_GATE)
     return SLM_ERR_INVALID_ARG;
@@ -212,6 +231,29 @@ extern "C" SLM_API int slm_linear(const slm_linear_args* a, void* stream) {
   if (a->epilogue == SLM_LIN_GLU && (a->N % 32 || a->batch != 1)) return SLM_ERR_INVALID_ARG;
   if (a->epilogue == SLM_LIN_SLABS && a->batch != 1) return SLM_ERR_INVALID_ARG;
   if (a->epilogue == SLM_LIN_GATE && !a->gate) return SLM_ERR_INVALID_ARG;
+  return SLM_OK;
+}
+
+extern "C" SLM_API int slm_linear(const slm_linear_args* a, void* stream) {
+  const int rc = lin_check(a);
+  if (rc != SLM_OK) return rc;
   if (a->M == 0) return SLM_OK;
   return a->dtype == SLM_BF16 ? lin_epi<bf16>(*a, (hipStream_t)stream) : lin_epi<float>(*a, (hipStream_t)stream);
+}
+
+// One launch where the rows leave the chip idle anyway: a launch that reads what the one in front of it wrote costs 4 us and more
+// whatever it does.  (A step of four layers, latent 512, two launches / one: 1 row of 32 heads 493 / 479 us, 32 rows of 16 heads 386 / 369,
+// 128 rows of 32 heads 1129 / 1124.)
+// And only where the product reads no column that the rotation writes (K is the queries' unrotated width, without padding).
+extern "C" SLM_API int slm_latent_append_absorb(const slm_latent_append_args* c, const slm_linear_args* a, void* stream) {
+  const int rc = lin_check(a);
+  if (rc != SLM_OK) return rc;
+  if (latent_append_invalid(c)) return SLM_ERR_INVALID_ARG;
+  if (a->epilogue != SLM_LIN_STORE || a->dtype != c->dtype) return SLM_ERR_INVALID_ARG;
+  const bool apart = a->x == c->proj && a->ldx == c->ld_proj && a->K <= c->q_dim && a->x_batch == c->q_dim + c->q_rot && a->batch <= c->heads &&
+                     c->q_abs && a->y == c->q_abs && a->N <= c->c_pad && a->y_batch == c->c_pad + c->r_pad && a->M <= c->abs_rows;
+  if (apart && a->M > 0 && c->rows <= 256 && a->dtype == SLM_BF16 && latent_append_by_four(*c))
+    return lin_shape<bf16, SLM_LIN_STORE>(*a, (hipStream_t)stream, c);
+  const int rd = slm_latent_append(c, stream);
+  return rd != SLM_OK ? rd : slm_linear(a, stream);
 }

@@ -372,10 +372,7 @@ def clamped_glu(gate_up: torch.Tensor, out: torch.Tensor, limit: float, alpha: f
                                                    float(alpha), float(shift), _code(out), _stream()), "slm_clamped_glu")
 
 
-def linear_heads(x: torch.Tensor, x_head: int, w: torch.Tensor, out: torch.Tensor, out_head: int,
-                 gate: Optional[torch.Tensor] = None) -> None:
-    """Per-head products: head h of `out` (columns from h * out_head) = columns from h * x_head of x times w[h]^T;
-    w [heads, N, K].  gate [rows, >= heads]: the result is multiplied by sigmoid(gate[:, h])."""
+def _heads_args(x: torch.Tensor, x_head: int, w: torch.Tensor, out: torch.Tensor, out_head: int) -> "_lib.LinearArgs":
     H, N, K = w.shape
     M = x.size(0)
     _need(x.dim() == 2 and out.dim() == 2 and out.size(0) == M and w.is_contiguous() and x.dtype == w.dtype == out.dtype and
@@ -385,7 +382,16 @@ def linear_heads(x: torch.Tensor, x_head: int, w: torch.Tensor, out: torch.Tenso
     a.ldx, a.ldw, a.ldy, a.y = x.stride(0), K, out.stride(0), _p(out)
     a.batch, a.x_batch, a.w_batch, a.y_batch = H, x_head, N * K, out_head
     a.epilogue = _lib.LIN_STORE
+    return a
+
+
+def linear_heads(x: torch.Tensor, x_head: int, w: torch.Tensor, out: torch.Tensor, out_head: int,
+                 gate: Optional[torch.Tensor] = None) -> None:
+    """Per-head products: head h of `out` (columns from h * out_head) = columns from h * x_head of x times w[h]^T;
+    w [heads, N, K].  gate [rows, >= heads]: the result is multiplied by sigmoid(gate[:, h])."""
+    a = _heads_args(x, x_head, w, out, out_head)
     if gate is not None:
+        M, H = x.size(0), w.size(0)
         _need(gate.size(0) == M and gate.size(1) >= H and gate.stride(1) == 1 and gate.dtype == x.dtype, "linear_heads: gate")
         a.epilogue, a.gate, a.ld_gate = _lib.LIN_GATE, _p(gate), gate.stride(0)
     _run_linear(a)
@@ -393,8 +399,9 @@ def linear_heads(x: torch.Tensor, x_head: int, w: torch.Tensor, out: torch.Tenso
 
 def latent_append(proj: torch.Tensor, cache: torch.Tensor, q_abs: Optional[torch.Tensor], norm_weight: torch.Tensor,
                   cos_sin: torch.Tensor, positions: torch.Tensor, slots: torch.Tensor, *, heads: int, q_dim: int, q_rot: int,
-                  rank: int, c_pad: int, off_c: int, off_r: int, eps: float) -> None:
-    """Latent RMS norm + rotation -> cache rows; the queries' rotated part in place (and behind c_pad of q_abs)."""
+                  rank: int, c_pad: int, off_c: int, off_r: int, eps: float, w_abs: Optional[torch.Tensor] = None) -> None:
+    """Latent RMS norm + rotation -> cache rows; the queries' rotated part in place (and behind c_pad of q_abs).  With w_abs
+    [heads, c_pad, K] the queries of q_abs's rows, absorbed, in front of it."""
     rows = proj.size(0)
     a = _lib.LatentAppendArgs()
     _need(proj.stride(1) == 1 and cache.dim() == 2 and cache.is_contiguous() and cache.dtype == proj.dtype, "latent_append: cache")
@@ -410,7 +417,12 @@ def latent_append(proj: torch.Tensor, cache: torch.Tensor, q_abs: Optional[torch
     if q_abs is not None and q_abs.size(0):
         _need(q_abs.is_contiguous() and q_abs.shape[1:] == (heads, cache.size(1)) and q_abs.size(0) <= rows, "latent_append: q_abs")
         a.q_abs, a.abs_rows = _p(q_abs), q_abs.size(0)
-    latent_check(_lib.latent_lib().slm_latent_append(C.byref(a), _stream()), "slm_latent_append")
+    if w_abs is None or not a.abs_rows:
+        latent_check(_lib.latent_lib().slm_latent_append(C.byref(a), _stream()), "slm_latent_append")
+        return
+    n = q_abs.size(0)
+    x = _heads_args(proj[:n], q_dim + q_rot, w_abs, q_abs.view(n, -1), cache.size(1))
+    latent_check(_lib.latent_lib().slm_latent_append_absorb(C.byref(a), C.byref(x), _stream()), "slm_latent_append_absorb")
 
 
 def latent_attention(q_abs: torch.Tensor, cache: torch.Tensor, out: torch.Tensor, positions: torch.Tensor, q_cu: torch.Tensor,

@@ -206,13 +206,12 @@ class LatentAttention:
         q_abs = proj.new_empty(n_tok, a.heads, self.c_pad + self.r_pad)
         lk.latent_append(proj, cache.rows, q_abs, self.norm, self.cos_sin, positions, params.new_cache_slots, heads=a.heads,
                          q_dim=self.q_dim, q_rot=self.r_pad, rank=a.kv_rank, c_pad=self.c_pad, off_c=self.off_c,
-                         off_r=self.off_r, eps=self.eps)
+                         off_r=self.off_r, eps=self.eps, w_abs=self.w_abs)
         out = proj.new_empty(T, self.o_k)
         if self.o_k != a.heads * self.v_pad:
             out[:, a.heads * self.v_pad:].zero_()
         if n_tok:
             pt = proj[:n_tok]
-            lk.linear_heads(pt, self.head_w, self.w_abs, q_abs.view(n_tok, -1), self.c_pad + self.r_pad)
             lat = proj.new_empty(n_tok, a.heads, self.c_pad)
             lk.latent_attention(q_abs, cache.rows, lat, positions, params.q_cu_seq_lens, params.block_tables,
                                 params.cu_block_lens, block_size=cache.block_size(), window=a.window, scale=a.scale,

@@ -332,6 +332,33 @@ def test_append_norms_rotates_and_writes_its_slots(heads, q_dim, rot, rank, dtyp
     assert not q_abs[:, :, c_pad + rot:].any() and (q_abs[:, :, :c_pad] == 5.0).all()
 
 
+# rows around the tiles of the product and the largest of the one launch; more rows appended than absorbed; a query width that is
+# padded for the product, and one whose rotated part a thread takes element by element: two launches
+@pytest.mark.parametrize("heads,q_dim,rot,rank", [(5, 128, 64, 512), (24, 64, 16, 96), (3, 96, 32, 70), (4, 64, 12, 64)])
+@pytest.mark.parametrize("rows,absorbed", [(1, 1), (5, 5), (16, 16), (33, 17), (65, 64), (256, 200), (257, 257)])
+def test_append_with_absorbed_queries(heads, q_dim, rot, rank, rows, absorbed):
+    """The same bits as the append and the product one after the other."""
+    from scalellm_amd.latent_layers import round_up, rotary_table
+    lk = _lk()
+    c_pad, r_pad, k = round_up(rank, 64), round_up(rot, 32), round_up(q_dim, 64)
+    cs = rotary_table(900.0, rot, 300, None, DEV)
+    hd = q_dim + r_pad
+    off_c = heads * hd
+    proj = _rnd(1, rows, off_c + c_pad + r_pad + 16, dtype=torch.bfloat16)
+    w, w_abs = _rnd(2, rank), _rnd(3, heads, c_pad, k, dtype=torch.bfloat16)
+    w_abs[:, :, q_dim:] = 0
+    pos = torch.arange(rows, dtype=torch.int32, device=DEV)
+    slots = torch.randperm(rows, generator=torch.Generator().manual_seed(5)).int().to(DEV)
+    sizes = dict(heads=heads, q_dim=q_dim, q_rot=r_pad, rank=rank, c_pad=c_pad, off_c=off_c, off_r=off_c + c_pad, eps=1e-5)
+    got, want = ([proj.clone(), torch.full((rows, c_pad + r_pad), 5.0, dtype=torch.bfloat16, device=DEV),
+                  torch.full((absorbed, heads, c_pad + r_pad), 5.0, dtype=torch.bfloat16, device=DEV)] for _ in range(2))
+    lk.latent_append(*got, w, cs, pos, slots, **sizes, w_abs=w_abs)
+    lk.latent_append(*want, w, cs, pos, slots, **sizes)
+    lk.linear_heads(want[0][:absorbed], hd, w_abs, want[2].view(absorbed, -1), c_pad + r_pad)
+    for g, x in zip(got, want):
+        assert torch.equal(g.view(torch.int16), x.view(torch.int16))
+
+
 # ---- attention over the cache ------------------------------------------------------------------
 class Paged:
     """Sequences of the given lengths on shuffled blocks, cache rows random (or given)."""
