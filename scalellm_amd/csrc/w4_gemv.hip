@@ -13,7 +13,7 @@
 //   * the activations (at most 4 x K values) are staged ONCE per workgroup in LDS together with
 //     their per-group sums X_g; the main loop reads them as broadcast ds_read_b128 (all lanes of a
 //     half-wave share the address) -- so the only VMEM in the loop is the weight stream, every
-//     wave keeps an 8-chunk register ring (8 KiB) in flight with exact counted waits;
+//     wave keeps a register ring of 4 (one row) or 8 chunks in flight with exact counted waits;
 //   * K is split across the waves of a workgroup (8 waves = TW column tiles x KS K-slices) and
 //     reduced through LDS at the end: no global split-K, no second launch.
 // Numerics: fp32 accumulation of exact products, affine correction in fp32 (the post-scaled form of
@@ -43,18 +43,26 @@ struct GemvParams {
   int silu;      // SLM_W4_SILU_MUL: tw is even, tiles (2j, 2j+1) = (gate, up), c is [M, N/2]
 };
 
-// weight ring depth (64-deep chunks per wave).  Measured alternatives for the norm-prologue kernel
-// (Llama-3-8B bs=1 step, ring 8 issued first by every wave = 2.28 ms): ring 16 -> 2.36 ms (loads
-// return in order, so the prologue's own loads wait behind a twice as long burst); the four norm
-// waves issuing their ring only after row 0's loads landed -> 2.31 ms (their stream starts late).
-constexpr int GV_RING = 8;
+// Weight ring depth (64-deep chunks per wave).  A wave's loads return in order, and a compute unit's L1 serves its waves
+// nearly so: what is asked for behind a ring waits until the ring has come from HBM.  One row: the activations (or what
+// the norm prologue reads) are in flight in FRONT of the ring, and the ring is short, so that the next wave's activations
+// do not wait for it either.  Four layers of Llama-3-8B in a captured step, AWQ, us a launch, ring of 8 in front of the
+// activations / ring of 8 behind them / of 4 / of 16: gate_up with prologue 17.1 / 14.5 / 14.2 / 16.8, qkv with prologue
+// 9.5 / 7.5 / 7.2 / 9.2, o and down 8.3 / 7.8 / 7.3 / -.  By themselves, weights from HBM: 4096 x 4096 6.3 -> 5.4, 14336 x 4096
+// 12.5 -> 10.9, 4096 x 28672 15.2 -> 14.0, 28672 x 8192 27.4 -> 26.4.  (A branch around the loads past the slice's end costs more than
+// the loads, which the caches serve: 4096 x 28672 24.0.)
+constexpr int GV_RING_ROW = 4, GV_RING_ROWS = 8;
 
 // NGC: scale groups per 64-deep chunk (2 for group 32, 1 otherwise); MT: token rows (1, 2, 4)
 // REFILL: the K slice of a wave is longer than the ring (otherwise every chunk is preloaded)
 // NORM: RMSNorm prologue (slm_w4a16_gemv_norm); its own instantiation so that the plain kernel keeps
-// its register count
-template <typename T, int NGC, int MT, bool REFILL, bool NORM>
+// its register count.  2: one row of up to 4096 columns that comes as one or two slabs, a residual with it:
+// a vector of 8 columns per thread, and the sums X_g are taken from the registers.  The same bits.
+template <typename T, int NGC, int MT, bool REFILL, int NORM>
 __global__ void __launch_bounds__(512) w4a16_gemv_kernel(const GemvParams p) {
+  constexpr int GV_RING = MT == 1 ? GV_RING_ROW : GV_RING_ROWS;
+  constexpr bool ROW = NORM == 0 && MT == 1;
+  static_assert(NORM != 2 || MT == 1, "one row");
   extern __shared__ __attribute__((aligned(16))) char smem[];
   // LDS: A [MT][K] T | X32 [MT][K/32] f32 (activation sums per 32 of K) | reduction [8][MT][32] f32
   // (| NORM: h [K] f32 | 4 f32)
@@ -68,8 +76,8 @@ __global__ void __launch_bounds__(512) w4a16_gemv_kernel(const GemvParams p) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int64_t n_tiles = p.N / 32;
 
-  // ---- this wave's column tile and K slice; its weight ring is issued FIRST so that the HBM
-  // latency of the first chunks overlaps the activation staging below ----
+  // ---- this wave's column tile and K slice; its weight ring is issued before anything waits, so that the
+  // HBM latency of the first chunks overlaps the activation staging below ----
   const int tw_i = wave % p.tw, ks_i = wave / p.tw;
   const int split_id = (int)blockIdx.x / p.n_wgs, wg = (int)blockIdx.x % p.n_wgs;
   int64_t nt = (int64_t)wg * p.tw + tw_i;
@@ -89,6 +97,30 @@ __global__ void __launch_bounds__(512) w4a16_gemv_kernel(const GemvParams p) {
   const uint32_t wstride = (uint32_t)(n_tiles * 1024);  // bytes per 64-deep chunk
   const uint32_t szstride = (uint32_t)(p.N * 4);        // bytes per scale group
   const int cpg_shift = p.gs_shift >= 30 ? 30 : (p.gs_shift > 6 ? p.gs_shift - 6 : 0);  // log2(chunks per group)
+  // one row without a prologue: a thread's first four vectors of 8 columns
+  u32x4 a_v[ROW ? 4 : 1];
+  auto a_load = [&](int v) {
+    return *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint16_t*>(p.a) + (int64_t)min(v, (int)(p.K / 8) - 1) * 8);
+  };
+  if constexpr (ROW) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) a_v[i] = a_load(tid + 512 * i);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  const int nv_t = min(tid, (int)(p.K / 8) - 1);   // (NORM 2: this thread's vector)
+  u32x4 n_w, n_r;
+  f32x4 n_s[2][2];
+  if constexpr (NORM == 2) {
+    const int64_t second = p.norm_splits > 1 ? p.K : 0;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      n_s[0][i] = *reinterpret_cast<const f32x4*>(p.norm_part + nv_t * 8 + 4 * i);
+      n_s[1][i] = *reinterpret_cast<const f32x4*>(p.norm_part + second + nv_t * 8 + 4 * i);
+    }
+    n_r = *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint16_t*>(p.norm_res_in) + nv_t * 8);
+    n_w = *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint16_t*>(p.norm_weight) + nv_t * 8);
+    __builtin_amdgcn_sched_barrier(0);
+  }
   u32x4 wreg[GV_RING];
   uint32_t szreg[GV_RING][NGC];
   auto w_load = [&](int c, u32x4& w, uint32_t (&sz)[NGC]) {
@@ -106,8 +138,68 @@ __global__ void __launch_bounds__(512) w4a16_gemv_kernel(const GemvParams p) {
     __builtin_amdgcn_sched_barrier(0);
   }
 
+  // the sum of a row's 32 columns: four neighbours' sums of 8, in the order of the loop over the table below
+  auto x_sum = [&](const u32x4& o, int v) {
+    const float x0 = (lo_f32<T>(o.x) + hi_f32<T>(o.x)) + (lo_f32<T>(o.y) + hi_f32<T>(o.y)) +
+                     (lo_f32<T>(o.z) + hi_f32<T>(o.z)) + (lo_f32<T>(o.w) + hi_f32<T>(o.w));
+    const float x1 = __shfl_down(x0, 1), x2 = __shfl_down(x0, 2), x3 = __shfl_down(x0, 3);
+    if (v < p.K / 8 && (v & 3) == 0) x_lds[v >> 2] = 0.f + x0 + x1 + x2 + x3;
+  };
+
   // ---- phase 0: activations -> LDS (rows >= M replicate the last row; never stored) ----
-  if constexpr (NORM) {
+  if constexpr (NORM == 2) {
+    float* h_lds = red + 8 * 32;
+    float* nred = h_lds + p.K;
+    const bool has = tid < p.K / 8, writer = blockIdx.x == 0;
+    float f[8];
+    {
+      u32x4 a;   // (splitk_sum4 of one or two slabs)
+      f32x4 s[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+        s[i] = zero + (p.norm_splits > 1 ? n_s[0][i] + n_s[1][i] : n_s[0][i]);
+      }
+      a.x = pack2<T>(s[0].x, s[0].y); a.y = pack2<T>(s[0].z, s[0].w);
+      a.z = pack2<T>(s[1].x, s[1].y); a.w = pack2<T>(s[1].z, s[1].w);
+      f[0] = lo_f32<T>(a.x) + lo_f32<T>(n_r.x); f[1] = hi_f32<T>(a.x) + hi_f32<T>(n_r.x);
+      f[2] = lo_f32<T>(a.y) + lo_f32<T>(n_r.y); f[3] = hi_f32<T>(a.y) + hi_f32<T>(n_r.y);
+      f[4] = lo_f32<T>(a.z) + lo_f32<T>(n_r.z); f[5] = hi_f32<T>(a.z) + hi_f32<T>(n_r.z);
+      f[6] = lo_f32<T>(a.w) + lo_f32<T>(n_r.w); f[7] = hi_f32<T>(a.w) + hi_f32<T>(n_r.w);
+    }
+    if (has) {
+      *reinterpret_cast<f32x4*>(h_lds + tid * 8) = f32x4{f[0], f[1], f[2], f[3]};
+      *reinterpret_cast<f32x4*>(h_lds + tid * 8 + 4) = f32x4{f[4], f[5], f[6], f[7]};
+      if (writer) {
+        u32x4 w;
+        w.x = pack2<T>(f[0], f[1]); w.y = pack2<T>(f[2], f[3]);
+        w.z = pack2<T>(f[4], f[5]); w.w = pack2<T>(f[6], f[7]);
+        *reinterpret_cast<u32x4*>(reinterpret_cast<uint16_t*>(p.norm_res_out) + tid * 8) = w;
+      }
+    }
+    __syncthreads();
+    if (tid < 256) {   // (vectors tid and tid + 256 of a thread, and the tree, as rms_norm_kernel)
+      float ss = 0.f;
+      if (has) ss = rms_sumsq8(f, ss);
+      if (tid + 256 < p.K / 8) {
+        const f32x4 h0 = *reinterpret_cast<const f32x4*>(h_lds + (tid + 256) * 8);
+        const f32x4 h1 = *reinterpret_cast<const f32x4*>(h_lds + (tid + 256) * 8 + 4);
+        const float g[8] = {h0.x, h0.y, h0.z, h0.w, h1.x, h1.y, h1.z, h1.w};
+        ss = rms_sumsq8(g, ss);
+      }
+      ss = group_sum<64>(ss);
+      if ((tid & 63) == 0) nred[tid >> 6] = ss;
+    }
+    __syncthreads();
+    const float tot = nred[0] + nred[1] + nred[2] + nred[3];
+    const float rs = rsqrtf(tot / (float)p.K + p.norm_eps);
+    const u32x4 o = rms_apply8<T>(f, rs, n_w);
+    if (has) {
+      *reinterpret_cast<u32x4*>(a_lds + tid * 8) = o;
+      if (writer && p.norm_out) *reinterpret_cast<u32x4*>(reinterpret_cast<uint16_t*>(p.norm_out) + tid * 8) = o;
+    }
+    x_sum(o, tid);
+  } else if constexpr (NORM == 1) {
     // Norm prologue: a[m, :] = rms_norm(x[m, :] + residual[m, :]) * weight, with x possibly given
     // as the fp32 split-K slabs of the producing GEMM -- the arithmetic, the thread -> column
     // mapping and the reduction tree of rms_norm_kernel (glue.hip), executed by the first 256
@@ -188,6 +280,14 @@ __global__ void __launch_bounds__(512) w4a16_gemv_kernel(const GemvParams p) {
       }
       __syncthreads();  // nred and h_lds are reused by the next row
     }
+  } else if constexpr (ROW) {
+    auto put = [&](const u32x4& o, int v) {
+      if (v < p.K / 8) *reinterpret_cast<u32x4*>(a_lds + (size_t)v * 8) = o;
+      x_sum(o, v);
+    };
+#pragma unroll
+    for (int i = 0; i < 4; ++i) put(a_v[i], tid + 512 * i);
+    for (int v0 = 2048; v0 < p.K / 8; v0 += 512) put(a_load(v0 + tid), v0 + tid);
   } else {
     const int vec_per_row = (int)(p.K / 8);
     for (int v = tid; v < MT * vec_per_row; v += 512) {
@@ -199,6 +299,7 @@ __global__ void __launch_bounds__(512) w4a16_gemv_kernel(const GemvParams p) {
     }
   }
   __syncthreads();
+  if constexpr (NORM != 2 && !ROW) {
   // activation sums per 32 of K (fp32): the affine correction needs sum_k x_k over whatever part
   // of a scale group a wave's K slice covers, so the table is kept at the finest granularity
   for (int t = tid; t < MT * n32; t += 512) {
@@ -213,6 +314,7 @@ __global__ void __launch_bounds__(512) w4a16_gemv_kernel(const GemvParams p) {
     x_lds[t] = s;
   }
   __syncthreads();
+  }
 
   // ---- phase 1: the weight stream ----
   uint32_t magic_v = W4Magic<T>::bits;
@@ -357,10 +459,12 @@ static void launch_gemv_m(const GemvParams& gp, int n_wgs, size_t lds, hipStream
   // without them) -- they keep the issue pattern the compiler's counted waits were built for.  The
   // no-refill instantiations were only reachable through a tuning knob and were the ones at the
   // 256-VGPR cap with spills; they are no longer built.
+  const bool one_row = gp.M <= 1 && gp.norm_part && gp.norm_splits <= 2 && gp.norm_res_in && gp.K <= 4096;
 #define SLM_GEMV(MTT)                                                                          \
   do {                                                                                         \
-    auto kfn = gp.norm_weight ? w4a16_gemv_kernel<T, NGC, MTT, true, true>                     \
-                              : w4a16_gemv_kernel<T, NGC, MTT, true, false>;                   \
+    auto kfn = !gp.norm_weight ? w4a16_gemv_kernel<T, NGC, MTT, true, 0>                       \
+               : one_row       ? w4a16_gemv_kernel<T, NGC, MTT, true, MTT == 1 ? 2 : 1>        \
+                               : w4a16_gemv_kernel<T, NGC, MTT, true, 1>;                      \
     if (lds > 65536) {                                                                         \
       (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kfn),                            \
                                 hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);       \

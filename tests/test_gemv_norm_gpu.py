@@ -87,6 +87,45 @@ def test_norm_prologue_is_bit_identical_to_norm_then_gemv(M, K, N, gs, source, w
         assert torch.equal(c, c_ref), f"max |diff| {(c.float() - c_ref.float()).abs().max().item()}"
 
 
+# one and two slabs of one row, up to 4096 columns: the prologue whose loads go in front of the weight ring; one more of each: not
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("n_slabs", [1, 2, 3])
+@pytest.mark.parametrize("K", [128, 1920, 4096, 4224])
+def test_one_row_of_slabs_is_bit_identical_to_norm_then_gemv(K, n_slabs, dtype):
+    from scalellm_amd import kernels
+    tdt = torch.bfloat16 if dtype == "bf16" else torch.float16
+    packed = helpers.pack_case(helpers.make_quant_case(K + n_slabs, K, 96, 64, "awq", dtype), dtype)
+    g = torch.Generator(device=DEV).manual_seed(K + n_slabs)
+    w = (1 + 0.1 * torch.randn(K, device=DEV, generator=g)).to(tdt)
+    res = torch.randn(1, K, device=DEV, dtype=tdt, generator=g)
+    slabs = torch.randn(n_slabs, 1, K, device=DEV, generator=g)
+    x = torch.full((1, K), float("nan"), device=DEV, dtype=tdt)  # never read
+    got, want = ([torch.full((1, n), float("nan"), device=DEV, dtype=tdt) for n in (96, K, K)] for _ in range(2))
+    pro = kernels.NormPrologue(w, 1e-5, residual=res.clone(), residual_out=got[1], partials=kernels.DeferredPartials.from_slabs(slabs),
+                               normed_out=got[2])
+    kernels.gptq_gemm(x, packed, got[0], norm=pro)
+    want[1].copy_(res)
+    kernels.rms_norm(want[2], x, w, 1e-5, want[1], partials=kernels.DeferredPartials.from_slabs(slabs))
+    kernels.gptq_gemm(want[2], packed, want[0])
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+
+
+# a thread's first four vectors in front of the ring (up to 16384 columns), the others behind it
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("K", [128, 4096, 4224, 16384, 16512])
+def test_one_row_is_the_first_of_two(K, dtype, tune):
+    from scalellm_amd import kernels
+    tune(SLM_W4_GEMV=2)  # two rows on the GEMV too
+    tdt = torch.bfloat16 if dtype == "bf16" else torch.float16
+    packed = helpers.pack_case(helpers.make_quant_case(K, K, 96, 64, "awq", dtype), dtype)
+    x = torch.randn(2, K, device=DEV, generator=torch.Generator(device=DEV).manual_seed(K)).to(tdt)
+    one, two = (torch.full((m, 96), float("nan"), device=DEV, dtype=tdt) for m in (1, 2))
+    kernels.gptq_gemm(x[:1], packed, one)
+    kernels.gptq_gemm(x, packed, two)
+    assert not two.isnan().any() and torch.equal(one, two[:1])
+
+
 def test_norm_prologue_consumes_a_real_deferred_gemv_and_keeps_its_own_slabs_apart():
     """o_proj (deferred: slabs in buffer 0) -> [norm + qkv-like GEMV, itself deferred: its slabs must
     go to buffer 1, it is still reading buffer 0] -> RMSNorm of the result."""
