@@ -170,25 +170,36 @@ __global__ void __launch_bounds__(NW * 64, 2) w4a16_gemm_ks_kernel(const GemmKPa
     return (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(b_rs, (int)b_voff, (int)((uint32_t)(nt0 + tc) * 64u), 0);
   };
 
-  // prologue, in the order the steady state issues (scales and bias of a tile, then its weights):
-  // the loop-carried vmcnt waits are merged with this path, so a different order here would make
-  // every wait in the loop conservative.  The ring goes first (HBM latency), the activations (L2)
-  // queue behind it.
+  // The ring's first turn, in the order the steady state issues (scales and bias of a tile, its weights, the stores
+  // of the tile before it -- here out of range): the loop-carried vmcnt waits are merged with this path, so a different
+  // order here would make every wait in the loop conservative (measured in the ISA without the stores: vmcnt(12) instead
+  // of 16).
+  constexpr int TURN = RD * (CW * NG + 1 + 2 * CW + 2 * MT * RPW);   // VMEM operations of it
+  auto ring_issue = [&]() {
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int d = 0; d < RD; ++d) {
+    for (int d = 0; d < RD; ++d) {
 #pragma unroll
-    for (int c = 0; c < CW; ++c) {
+      for (int c = 0; c < CW; ++c) {
 #pragma unroll
-      for (int g = 0; g < NG; ++g) szr[d][c][g] = sz_load(d, c, g);
+        for (int g = 0; g < NG; ++g) szr[d][c][g] = sz_load(d, c, g);
+      }
+      bsr[d] = b_load(d);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int c = 0; c < CW; ++c) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) ring[d][c][h] = w_load(d, c, h);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < MT * RPW; ++i) {
+        __builtin_amdgcn_raw_buffer_store_b16((uint16_t)0, c_rs, (int)KS_OOB, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b32(0u, part_rs, (int)KS_OOB, 0, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
     }
-    bsr[d] = b_load(d);
-#pragma unroll
-    for (int c = 0; c < CW; ++c) {
-#pragma unroll
-      for (int h = 0; h < 2; ++h) ring[d][c][h] = w_load(d, c, h);
-    }
-  }
-  __builtin_amdgcn_sched_barrier(0);
+  };
   stamp(1);
   {  // probe (SLM_W4_KS_DBG bits 8..14): delay the second wave of every SIMD by 256-cycle steps
     const int nsl = (p.ks_dbg >> 8) & 127;
@@ -292,22 +303,15 @@ __global__ void __launch_bounds__(NW * 64, 2) w4a16_gemm_ks_kernel(const GemmKPa
       stamp(c0 == 0 ? 2 : 31);
       if (c0 == 0)  // counters zeroed (top of the kernel) before anybody can publish a tile
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-      // the DMA is invisible to the compiler: explicit wait (also lands the ring, issued before it)
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      if (c0 == 0) {
-        // ... and the compiler does not know the ring has landed: without these uses it merges
-        // "prologue loads pending" into the loop's vmcnt bookkeeping and every wait of the steady
-        // state comes out 4 loads too conservative (measured in the ISA: vmcnt(12) instead of 16)
-#pragma unroll
-        for (int d = 0; d < RD; ++d) {
-#pragma unroll
-          for (int c = 0; c < CW; ++c) {
-            asm volatile("" : "+v"(ring[d][c][0]), "+v"(ring[d][c][1]));
-#pragma unroll
-            for (int g = 0; g < NG; ++g) asm volatile("" : "+v"(szr[d][c][g]));
-          }
-          asm volatile("" : "+v"(bsr[d]));
-        }
+      // The DMA is invisible to the compiler: explicit waits.  The ring goes behind the last of it: loads return in
+      // order, and in front of the activations (L2) it kept them until it had come from HBM.  32 rows, us, in front / behind:
+      // 4096 x 4096 8.9 / 8.0, 4096 x 6144 9.4 / 8.5, 8192 x 2048 10.8 / 10.1, 14336 x 4096 15.6 / 15.3, 4096 x 28672 19.8 / 19.6;
+      // 16 rows 8.0 / 7.1, 8.5 / 7.7, 10.0 / 9.3, 14.3 / 14.0, 18.6 / 18.6.
+      if (c0 + 2 >= VC) {
+        ring_issue();
+        asm volatile("s_waitcnt vmcnt(%0)" : : "n"(TURN < 63 ? TURN : 63) : "memory");
+      } else {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       }
 #pragma unroll
       for (int v = c0; v < c0 + 2 && v < VC; ++v) {
