@@ -56,13 +56,13 @@ constexpr int GV_RING_ROW = 4, GV_RING_ROWS = 8;
 // NGC: scale groups per 64-deep chunk (2 for group 32, 1 otherwise); MT: token rows (1, 2, 4)
 // REFILL: the K slice of a wave is longer than the ring (otherwise every chunk is preloaded)
 // NORM: RMSNorm prologue (slm_w4a16_gemv_norm); its own instantiation so that the plain kernel keeps
-// its register count.  2: one row of up to 4096 columns that comes as one or two slabs, a residual with it:
+// its register count.  2: one row of up to 4096 columns that comes as one or two slabs, a residual with it, 3: as it is, without one:
 // a vector of 8 columns per thread, and the sums X_g are taken from the registers.  The same bits.
 template <typename T, int NGC, int MT, bool REFILL, int NORM>
 __global__ void __launch_bounds__(512) w4a16_gemv_kernel(const GemvParams p) {
   constexpr int GV_RING = MT == 1 ? GV_RING_ROW : GV_RING_ROWS;
   constexpr bool ROW = NORM == 0 && MT == 1;
-  static_assert(NORM != 2 || MT == 1, "one row");
+  static_assert(NORM < 2 || MT == 1, "one row");
   extern __shared__ __attribute__((aligned(16))) char smem[];
   // LDS: A [MT][K] T | X32 [MT][K/32] f32 (activation sums per 32 of K) | reduction [8][MT][32] f32
   // (| NORM: h [K] f32 | 4 f32)
@@ -107,7 +107,7 @@ __global__ void __launch_bounds__(512) w4a16_gemv_kernel(const GemvParams p) {
     for (int i = 0; i < 4; ++i) a_v[i] = a_load(tid + 512 * i);
     __builtin_amdgcn_sched_barrier(0);
   }
-  const int nv_t = min(tid, (int)(p.K / 8) - 1);   // (NORM 2: this thread's vector)
+  const int nv_t = min(tid, (int)(p.K / 8) - 1);   // (NORM 2, 3: this thread's vector)
   u32x4 n_w, n_r;
   f32x4 n_s[2][2];
   if constexpr (NORM == 2) {
@@ -118,6 +118,9 @@ __global__ void __launch_bounds__(512) w4a16_gemv_kernel(const GemvParams p) {
       n_s[1][i] = *reinterpret_cast<const f32x4*>(p.norm_part + second + nv_t * 8 + 4 * i);
     }
     n_r = *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint16_t*>(p.norm_res_in) + nv_t * 8);
+  }
+  if constexpr (NORM == 3) n_r = *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint16_t*>(p.norm_x) + nv_t * 8);
+  if constexpr (NORM >= 2) {
     n_w = *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint16_t*>(p.norm_weight) + nv_t * 8);
     __builtin_amdgcn_sched_barrier(0);
   }
@@ -147,12 +150,13 @@ __global__ void __launch_bounds__(512) w4a16_gemv_kernel(const GemvParams p) {
   };
 
   // ---- phase 0: activations -> LDS (rows >= M replicate the last row; never stored) ----
-  if constexpr (NORM == 2) {
+  if constexpr (NORM >= 2) {
     float* h_lds = red + 8 * 32;
     float* nred = h_lds + p.K;
     const bool has = tid < p.K / 8, writer = blockIdx.x == 0;
-    float f[8];
-    {
+    float f[8] = {lo_f32<T>(n_r.x), hi_f32<T>(n_r.x), lo_f32<T>(n_r.y), hi_f32<T>(n_r.y),
+                  lo_f32<T>(n_r.z), hi_f32<T>(n_r.z), lo_f32<T>(n_r.w), hi_f32<T>(n_r.w)};
+    if constexpr (NORM == 2) {
       u32x4 a;   // (splitk_sum4 of one or two slabs)
       f32x4 s[2];
 #pragma unroll
@@ -162,15 +166,15 @@ __global__ void __launch_bounds__(512) w4a16_gemv_kernel(const GemvParams p) {
       }
       a.x = pack2<T>(s[0].x, s[0].y); a.y = pack2<T>(s[0].z, s[0].w);
       a.z = pack2<T>(s[1].x, s[1].y); a.w = pack2<T>(s[1].z, s[1].w);
-      f[0] = lo_f32<T>(a.x) + lo_f32<T>(n_r.x); f[1] = hi_f32<T>(a.x) + hi_f32<T>(n_r.x);
-      f[2] = lo_f32<T>(a.y) + lo_f32<T>(n_r.y); f[3] = hi_f32<T>(a.y) + hi_f32<T>(n_r.y);
-      f[4] = lo_f32<T>(a.z) + lo_f32<T>(n_r.z); f[5] = hi_f32<T>(a.z) + hi_f32<T>(n_r.z);
-      f[6] = lo_f32<T>(a.w) + lo_f32<T>(n_r.w); f[7] = hi_f32<T>(a.w) + hi_f32<T>(n_r.w);
+      f[0] = lo_f32<T>(a.x) + f[0]; f[1] = hi_f32<T>(a.x) + f[1];
+      f[2] = lo_f32<T>(a.y) + f[2]; f[3] = hi_f32<T>(a.y) + f[3];
+      f[4] = lo_f32<T>(a.z) + f[4]; f[5] = hi_f32<T>(a.z) + f[5];
+      f[6] = lo_f32<T>(a.w) + f[6]; f[7] = hi_f32<T>(a.w) + f[7];
     }
     if (has) {
       *reinterpret_cast<f32x4*>(h_lds + tid * 8) = f32x4{f[0], f[1], f[2], f[3]};
       *reinterpret_cast<f32x4*>(h_lds + tid * 8 + 4) = f32x4{f[4], f[5], f[6], f[7]};
-      if (writer) {
+      if (NORM == 2 && writer) {
         u32x4 w;
         w.x = pack2<T>(f[0], f[1]); w.y = pack2<T>(f[2], f[3]);
         w.z = pack2<T>(f[4], f[5]); w.w = pack2<T>(f[6], f[7]);
@@ -299,7 +303,7 @@ __global__ void __launch_bounds__(512) w4a16_gemv_kernel(const GemvParams p) {
     }
   }
   __syncthreads();
-  if constexpr (NORM != 2 && !ROW) {
+  if constexpr (NORM < 2 && !ROW) {
   // activation sums per 32 of K (fp32): the affine correction needs sum_k x_k over whatever part
   // of a scale group a wave's K slice covers, so the table is kept at the finest granularity
   for (int t = tid; t < MT * n32; t += 512) {
@@ -459,11 +463,15 @@ static void launch_gemv_m(const GemvParams& gp, int n_wgs, size_t lds, hipStream
   // without them) -- they keep the issue pattern the compiler's counted waits were built for.  The
   // no-refill instantiations were only reachable through a tuning knob and were the ones at the
   // 256-VGPR cap with spills; they are no longer built.
-  const bool one_row = gp.M <= 1 && gp.norm_part && gp.norm_splits <= 2 && gp.norm_res_in && gp.K <= 4096;
+  const int one_row = gp.M > 1 || gp.K > 4096                                      ? 0
+                      : gp.norm_part && gp.norm_splits <= 2 && gp.norm_res_in ? 2
+                      : !gp.norm_part && !gp.norm_res_in                      ? 3
+                                                                              : 0;
 #define SLM_GEMV(MTT)                                                                          \
   do {                                                                                         \
     auto kfn = !gp.norm_weight ? w4a16_gemv_kernel<T, NGC, MTT, true, 0>                       \
-               : one_row       ? w4a16_gemv_kernel<T, NGC, MTT, true, MTT == 1 ? 2 : 1>        \
+               : one_row == 2  ? w4a16_gemv_kernel<T, NGC, MTT, true, MTT == 1 ? 2 : 1>        \
+               : one_row == 3  ? w4a16_gemv_kernel<T, NGC, MTT, true, MTT == 1 ? 3 : 1>        \
                                : w4a16_gemv_kernel<T, NGC, MTT, true, 1>;                      \
     if (lds > 65536) {                                                                         \
       (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kfn),                            \
