@@ -30,8 +30,12 @@ __device__ __forceinline__ float quotient(float n, float d) {
   return __builtin_fmaf(__builtin_fmaf(-d, q, n), r, q);
 }
 __device__ __forceinline__ float silu_f32(float z) { return z / (1.0f + __expf(-z)); }
-// (below -69 a result is under 1e-28: exp(69) is what the quotient takes; above 100 it is z, an infinity too)
-__device__ __forceinline__ float silu_run(float z) { return z > 100.f ? z : quotient(z, 1.0f + __expf(fminf(-z, 69.f))); }
+// (below -69, where 1 + exp(-z) is exp(-z) and past what the quotient takes, it is z exp(z); above 100 it is z, an infinity too)
+__device__ __forceinline__ float silu_run(float z) {
+  const bool low = z < -69.f;
+  const float e = __expf(low ? z : -z);
+  return z > 100.f ? z : low ? z * e : quotient(z, 1.0f + e);
+}
 // log(1 + x) = log(u) x / (u - 1) with u the rounded 1 + x: what the sum loses of x comes back (Kahan)
 __device__ __forceinline__ float softplus_f32(float z) {
   const float x = __expf(-fabsf(z)), u = 1.0f + x;

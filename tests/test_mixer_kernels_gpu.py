@@ -132,6 +132,57 @@ def test_lightning_attention(dim, vdim, decay, dtype):
     _serve(_Alone(half, width, False), width, dtype, lambda h: 0.75 * ref.lightning_attention(h, _f64(w), m["right"], 1e-5), 1e-5)
 
 
+@np.errstate(over="ignore")
+def _lightning_by_hand(proj, H, D, V, decay, weight, eps):
+    """The layer behind its projections [q | k | v | g], token by token in 64 bits."""
+    x = proj.double().cpu().numpy()
+    act = lambda z: z * ref.sigmoid(z)  # noqa: E731
+    S, out, qk = np.zeros((H, D, V)), [], H * D
+    for r in x:
+        q, k, v = act(r[:qk]).reshape(H, D), act(r[qk:2 * qk]).reshape(H, D), act(r[2 * qk:2 * qk + H * V]).reshape(H, V)
+        S = np.asarray(decay)[:, None, None] * S + k[:, :, None] * v[:, None, :]
+        o = np.einsum("hdv,hd->hv", S, q).reshape(-1)
+        out.append(ref.rms_norm(o, weight, eps) * ref.sigmoid(r[2 * qk + H * V:2 * qk + 2 * H * V]))
+    return np.array(out)
+
+
+def _lightning_of(proj, H, D, V, decay, dtype):
+    """The same rows as one portion and one by one."""
+    from scalellm_amd.engine import Sequence
+    from scalellm_amd.mixer_layers import LightningArgs, LightningAttention
+    w = {n: torch.zeros(H * d, 64) for n, d in (("q", D), ("k", D), ("v", V), ("g", V))}
+    half = LightningAttention(LightningArgs(H, D, V, decay), 64, 1e-5, {**w, "norm": torch.ones(H * V), "o": torch.zeros(64, H * V)}, dtype, DEV)
+    got = []
+    for n in (proj.size(0), 1):
+        b = _Batch()
+        state, seq, rows = half.new_state(b.limits(dtype)), Sequence(0, [0] * proj.size(0)), []
+
+        def layer(x, *how):
+            out = x.new_empty(x.size(0), half.out_width)
+            half.forward(x, *how, out)
+            return out
+        while seq.n_cached < proj.size(0):
+            rows += b.run(layer, state, {0: proj}, [(seq, n)])
+        got.append(torch.cat(rows))
+    return got
+
+
+# 16-bit inputs go down to -3e38, and what an activation makes of them is 0 whether a token comes alone or in a portion
+@pytest.mark.parametrize("dtype", BOTH)
+def test_activations_of_values_far_below_zero(dtype):
+    H, D, V, decay = 2, 32, 48, (0.9, 0.6)
+    g = torch.Generator().manual_seed(12)
+    proj = torch.randn(37, 2 * H * (D + V), generator=g)
+    for i, z in enumerate((-3e38, -1e30, -1e28, -1000.0, -90.0, -75.0, -69.5, -60.0)):
+        for at in (0, H * D, 2 * H * D):   # of q, k and v
+            proj[:, at + 3 * i] = z
+            proj[i, at + 30] = z
+    proj = proj.to(device=DEV, dtype=dtype)
+    want = _lightning_by_hand(proj, H, D, V, decay, 1.0, 1e-5)
+    for got in _lightning_of(proj, H, D, V, decay, dtype):
+        _close(got, want, dtype, 3e-5, 4e-2)
+
+
 @pytest.mark.parametrize("dtype", BOTH)
 @pytest.mark.parametrize("m", [window(1, 1, 2, 1, 2, 1, 0), window(6, 3, 22, 18, 10, 21, 5, 5.0), window(4, 4, 64, 96, 64, 16, 16),
                                window(34, 2, 128, 64, 0, 40, 70, 8.0), window(3, 1, 96, 192, 50, 0, 0, 0.0), window(2, 2, 256, 256, 128, 33, 3),
