@@ -335,9 +335,10 @@ __device__ __forceinline__ f32x4 mma4(const f32x4& x, const f32x4& y, f32x4 c) {
   return c;
 }
 
-// one workgroup per (chunk, head); every chunk of the step at once.  A and B are 32-bit MFMAs of k exp(L), q exp(L) and k exp(-L) where no channel of
-// the chunk falls below 2^-96 (each entry's factors then are in range, their product is below 1); else entry by entry, an exponential for
-// each of the 16 x 16 x DK terms.
+// one workgroup per (chunk, head); every chunk of the step at once.  With the delta rule A and B are 32-bit MFMAs of k exp(L), q exp(L) and k exp(-L) where
+// no channel of the chunk falls below 2^-96 (k is a unit vector: each entry's factors then are in range, their product is below 1); else entry by
+// entry, an exponential for each of the 16 x 16 x DK terms.  Without it a token's channels decay alike: B is q k^T, whose entries are scaled, of
+// whatever size keys are.
 constexpr float DIRECT_BELOW = -96.f;
 template <typename E, int MODE, int DK>
 __global__ void __launch_bounds__(256) recurrent_prepare_kernel(const slm_recurrent_args a) {
@@ -479,7 +480,7 @@ __global__ void __launch_bounds__(256) recurrent_prepare_kernel(const slm_recurr
     }
     rec[ChunkRecord<DK>::GE + tid] = fast_exp2(lowest);
   }
-  const bool direct = __syncthreads_or(lowest < DIRECT_BELOW || !(lowest <= 0.f));
+  const bool direct = __syncthreads_or(DELTA && (lowest < DIRECT_BELOW || !(lowest <= 0.f)));
   const int l16 = lane & 15, g = lane >> 4;
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
   auto lds4 = [](const float* p) { return *reinterpret_cast<const f32x4*>(p); };
@@ -495,17 +496,19 @@ __global__ void __launch_bounds__(256) recurrent_prepare_kernel(const slm_recurr
     f32x4 l;
     if constexpr (DELTA) l = lds4(sL + at_t);
     else l = zero + summed(l16, 0);
-    const f32x4 e = exp4(l), k = lds4(sk + at_t);
-    qd[j] = lds4(sq + at_t) * e;
-    if (!direct) {
+    const f32x4 e = exp4(l), k = lds4(sk + at_t), q = lds4(sq + at_t);
+    qd[j] = q * e;
+    if constexpr (!DELTA) {
+      pb = mma4(q, k, pb);
+    } else if (!direct) {
       const f32x4 ks = k * exp4(-l);
-      if constexpr (DELTA) pa = mma4(k * e, ks, pa);
+      pa = mma4(k * e, ks, pa);
       pb = mma4(qd[j], ks, pb);
     }
   }
   settle(pa);
   settle(pb);
-  if (!direct) {
+  if (!DELTA || !direct) {
     f32x4 (*const part)[2][64] = reinterpret_cast<f32x4 (*)[2][64]>(sq);
     __syncthreads();   // (nobody reads q any more)
     if constexpr (DELTA) part[wave][0][lane] = pa;
@@ -519,7 +522,7 @@ __global__ void __launch_bounds__(256) recurrent_prepare_kernel(const slm_recurr
       for (int r = 0; r < 4; ++r) {
         const int t = 4 * g + r;
         if (wave == 0) sa[t][l16] = l16 < t ? sum[r] : 0.f;
-        else sb[t * 20 + l16] = l16 <= t ? sum[r] : 0.f;
+        else sb[t * 20 + l16] = l16 > t ? 0.f : DELTA ? sum[r] : sum[r] * fast_exp2(step_l * (min(t + 1, n) - min(l16 + 1, n)));
       }
     }
   } else {

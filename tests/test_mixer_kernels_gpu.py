@@ -183,6 +183,21 @@ def test_activations_of_values_far_below_zero(dtype):
         _close(got, want, dtype, 3e-5, 4e-2)
 
 
+# Keys are not normed: large ones in a head that forgets almost 2^-96 a chunk, and much more (where a product of exponentials would leave the range).
+# (The norm behind squares read-outs, so those stay under 1e19 here: keys of 1e16 make some of 1e17.)
+@pytest.mark.parametrize("dtype", BOTH)
+@pytest.mark.parametrize("size", [1e12, 1e16])
+def test_lightning_attention_of_large_keys(size, dtype):
+    H, D, V, decay = 3, 32, 48, (0.0167, 0.9, 1e-6)
+    g = torch.Generator().manual_seed(13)
+    proj = torch.randn(37, 2 * H * (D + V), generator=g)
+    proj[:, H * D:2 * H * D] *= size
+    proj = proj.to(device=DEV, dtype=dtype)
+    want = _lightning_by_hand(proj, H, D, V, decay, 1.0, 1e-5)
+    for got in _lightning_of(proj, H, D, V, decay, dtype):
+        _close(got, want, dtype, 3e-5, 4e-2)
+
+
 @pytest.mark.parametrize("dtype", BOTH)
 @pytest.mark.parametrize("m", [window(1, 1, 2, 1, 2, 1, 0), window(6, 3, 22, 18, 10, 21, 5, 5.0), window(4, 4, 64, 96, 64, 16, 16),
                                window(34, 2, 128, 64, 0, 40, 70, 8.0), window(3, 1, 96, 192, 50, 0, 0, 0.0), window(2, 2, 256, 256, 128, 33, 3),
