@@ -846,7 +846,8 @@ static int plan_gemm(const slm_w4_gemm_args* a, GemmPlan* pl) {
   }
   pl->tiled = 0;
   const int tile = tune_get(TUNE_W4_TILE, -1);
-  if (a->dtype == SLM_BF16 && tile != 0 && (tile > 0 || ((a->flags & SLM_W4_TILES) && w4_tile_rows(a->M, a->K, a->N))) && ((a->M - 1) * a->lda + a->K) * 2 < ((int64_t)1 << 31) &&
+  // (never a GEMV: its activations may be what a norm prologue makes, and not in memory)
+  if (a->dtype == SLM_BF16 && !pl->gemv && tile != 0 && (tile > 0 || ((a->flags & SLM_W4_TILES) && w4_tile_rows(a->M, a->K, a->N))) && ((a->M - 1) * a->lda + a->K) * 2 < ((int64_t)1 << 31) &&
       !(a->flags & SLM_W4_SHARES_CHIP) && !tune_is_set(TUNE_W4_MT) && !tune_is_set(TUNE_W4_SPLITK)) {
     pl->tiled = 1;
     pl->xl_sk = 0;

@@ -452,6 +452,33 @@ def test_gemv_norm_prologue_host_side():
     assert L.slm_w4a16_gemv_norm(C.byref(g), C.byref(n), None) == 0   # empty batch
 
 
+def test_forced_tiles_leave_gemvs_alone():
+    """SLM_W4_TILE asks for tiles that read their activations from memory; a one-row GEMV may get them from a norm prologue, so its plan
+    is the same with the knob as without it."""
+    L = _lib.lib()
+    assert L.slm_tuning_clear(None) == 0
+    g = W4GemmArgs()
+    g.K, g.N, g.lda, g.ldc, g.group_size, g.dtype, g.flags = 4096, 4096, 4096, 4096, 128, 1, _lib.SLM_W4_DEFER_REDUCE
+
+    def plans():
+        out = []
+        for g.M in (1, 2, 4, 5, 200):
+            out.append((L.slm_w4a16_gemv_norm_supported(C.byref(g)), L.slm_w4a16_gemm_deferred_splits(C.byref(g)), L.slm_w4a16_gemm_workspace_bytes(C.byref(g))))
+        return out
+    for mode in (1, 2):   # (2: GEMVs of up to 4 rows)
+        assert L.slm_tuning_set(b"SLM_W4_GEMV", mode) == 0
+        try:
+            before = plans()
+            assert [p[0] for p in before] == [1, mode - 1, mode - 1, 0, 0] and before[0][1] > 0
+            for tile in range(1, 6):
+                assert L.slm_tuning_set(b"SLM_W4_TILE", tile) == 0
+                now = plans()
+                assert [n for b, n in zip(before, now) if b[0]] == [b for b in before if b[0]]
+                assert now[4][1] == 0   # (200 rows are tiles, which leave no slabs)
+        finally:
+            assert L.slm_tuning_clear(None) == 0
+
+
 def test_ctypes_structs_match_the_c_header(tmp_path):
     """ABI drift guard: size and every field offset of the ctypes mirrors (_lib.py) equal what a C
     compiler makes of include/slm_hip.h."""
