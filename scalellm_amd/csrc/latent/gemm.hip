@@ -21,6 +21,7 @@
 // 153 / 120, 1000 x 4096 x 14336 129 / 107, 600 x 28672 x 4096 GLU 148 / 134, 300 x 4096 x 14336 73 / 63, 200 x 16384 x 2048 GLU 31 / 23,
 // 8192^3 701 / 729; short and narrow 207 x 4096 x 4096 18.5 / 19.8, 178 x 3664 x 2048 10.6 / 14.6 (of up to 128 rows: the vendor's).
 #include "latent_common.h"
+#include "tile_common.h"
 
 namespace slm {
 
@@ -40,12 +41,6 @@ __device__ __forceinline__ void gemm_product(f32x4& c, const bf16x8_t& w, const 
   asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(w), "v"(x));
 }
 
-// A run of `n` items for each of the 8 XCDs, which workgroups go round: item of a workgroup, -1 for none
-__device__ __forceinline__ int xcd_run(int wg, int n) {
-  const int per = (n + 7) >> 3, i = wg >> 3, t = (wg & 7) * per + i;
-  return i < per && t < n ? t : -1;
-}
-
 template <int BM, int BN, int WS, bool GLU>
 __global__ void __launch_bounds__(256, 1) gemm_kernel(const GemmK a) {
   constexpr int XS = 3;                              // stages of x; WS: of w
@@ -54,7 +49,6 @@ __global__ void __launch_bounds__(256, 1) gemm_kernel(const GemmK a) {
   constexpr int XD = BM / 32, WD = BN / 32, ND = XD + WD;   // DMA instructions of a wave and step (8 rows each)
   constexpr int R = MT + NT, MM = MT * NT;           // LDS reads and products of a half step
   constexpr int LATE = XD + (WS == 3 ? WD : 0);      // DMA under way that the next step does not need
-  constexpr int FRAGS = MM;
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r16 = lane & 15, g = lane >> 4, wm = wave & 1, wn = wave >> 1;
@@ -159,47 +153,19 @@ __global__ void __launch_bounds__(256, 1) gemm_kernel(const GemmK a) {
     xa = xn;
     wa = wnext;
   }
-  // (no DMA may outlive the workgroup's LDS; the last products are not tracked by the compiler)
-  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_nop 15\n\ts_nop 7" ::: "memory");
+  tile_settle(acc);
+  if (own >= 0 && !tile_add_slices(acc, a.slabs + (int64_t)own * a.slices * (MM * 1024), a.arrived + own, slice, a.slices, lds)) return;
 
-  if (own >= 0) {
-    const __amdgpu_buffer_rsrc_t mine = __builtin_amdgcn_make_buffer_rsrc(
-        a.slabs + (int64_t)own * a.slices * (FRAGS * 1024), 0, a.slices * FRAGS * 4096, 0x00020000);
-    auto at = [&](int s, int f) { return ((s * FRAGS + f) * 256 + tid) * 16; };
-#pragma unroll
-    for (int f = 0; f < FRAGS; ++f)
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[f / MT][f % MT]), mine, at(slice, f), 0, /*sc1*/ 16);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // every wave's sums are out ..
-    __syncthreads();
-    uint32_t* word = reinterpret_cast<uint32_t*>(lds);
-    if (tid == 0) word[0] = __hip_atomic_fetch_add(a.arrived + own, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // .. then one announces them
-    __syncthreads();
-    if (word[0] != (uint32_t)a.slices - 1) return;
-    constexpr int C = 8;   // fragments in flight
-#pragma unroll
-    for (int f0 = 0; f0 < FRAGS; f0 += C) {
-      f32x4 sum[C];
-#pragma unroll
-      for (int f = 0; f < C; ++f) sum[f] = f32x4{0.f, 0.f, 0.f, 0.f};
-      for (int s = 0; s < a.slices; ++s) {   // (in slice order, whoever is last: the same bits every time)
-#pragma unroll
-        for (int f = 0; f < C; ++f)
-          sum[f] += __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(mine, at(s, f0 + f), 0, /*sc1*/ 16));
-      }
-#pragma unroll
-      for (int f = 0; f < C; ++f) acc[(f0 + f) / MT][(f0 + f) % MT] = sum[f];
-    }
-  }
-
-  // lane: columns 8 g .. + 7 of a pair of tiles, row r16
+  // lane: columns 8 g .. + 7 of a pair of tiles, row r16 (worked out again: kept through the products they spill)
+  const int el = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), e16 = el & 15, eg = el >> 4;
 #pragma unroll
   for (int m = 0; m < MT; ++m) {
-    const int64_t row = m0 + wm * (BM / 2) + 16 * m + r16;
+    const int64_t row = m0 + wm * (BM / 2) + 16 * m + e16;
     if (row >= a.M) continue;
     bf16* y = a.y + row * a.ldy;
 #pragma unroll
     for (int n = 0; n < (GLU ? NT / 2 : NT); n += 2) {
-      const int64_t col = n0 + wn * (GLU ? BN / 4 : BN / 2) + 16 * n + 8 * g;
+      const int64_t col = n0 + wn * (GLU ? BN / 4 : BN / 2) + 16 * n + 8 * eg;
       if (col >= (GLU ? half : a.N)) continue;
       float v[8];
 #pragma unroll
@@ -210,11 +176,6 @@ __global__ void __launch_bounds__(256, 1) gemm_kernel(const GemmK a) {
       store_f32<8>(y + col, v);
     }
   }
-}
-
-__global__ void __launch_bounds__(256) gemm_clear_kernel(uint32_t* p, int n) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i < n) p[i] = 0;
 }
 
 // Tiles, and what they take: us of a step of 64 k alone on the chip and with every CU busy (power), and of a tile beside its steps.
@@ -284,13 +245,8 @@ template <int BM, int BN, int WS, bool GLU>
 static int gemm_launch(const GemmK& k, hipStream_t st) {
   constexpr int bytes = (3 * BM + WS * BN) * 128;
   auto fn = gemm_kernel<BM, BN, WS, GLU>;
-  static bool opted[64] = {};   // > 64 KiB of dynamic LDS: once per kernel and device
-  int dev = 0;
-  (void)hipGetDevice(&dev);
-  if (dev < 0 || dev >= 64 || !opted[dev]) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-    if (dev >= 0 && dev < 64) opted[dev] = true;
-  }
+  static bool asked[64] = {};
+  tile_allow_lds(fn, bytes, asked);
   const unsigned wgs = (unsigned)((k.whole + 7) / 8 * 8 + (k.cut * k.slices + 7) / 8 * 8);
   fn<<<dim3(wgs), dim3(256), bytes, st>>>(k);
   return hip_check_launch();
@@ -346,6 +302,6 @@ extern "C" SLM_API int slm_gemm(const slm_linear_args* a, void* workspace, size_
   k.arrived = (uint32_t*)workspace; k.slabs = (float*)((char*)workspace + 1024);
   hipStream_t st = (hipStream_t)stream;
   hip_clear_error();
-  if (p.cut) gemm_clear_kernel<<<dim3(1), dim3(256), 0, st>>>(k.arrived, p.cut);
+  if (p.cut) tile_clear_kernel<<<dim3(1), dim3(256), 0, st>>>(k.arrived, p.cut);
   return a->epilogue == SLM_LIN_GLU ? gemm_tile<true>(p, k, st) : gemm_tile<false>(p, k, st);
 }

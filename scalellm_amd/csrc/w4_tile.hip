@@ -20,6 +20,7 @@
 // a paired weight owes to that of the plain one (the last of several rounds alone would gain 2 % on some sizes).
 #include <type_traits>
 
+#include "tile_common.h"
 #include "w4_common.h"
 
 namespace slm {
@@ -72,12 +73,6 @@ __device__ __forceinline__ void in_turn(const F& f) {
   }
 }
 
-// A run of `n` items for each of the 8 XCDs, which workgroups go round: item of a workgroup, -1 for none
-__device__ __forceinline__ int tile_xcd_run(int wg, int n) {
-  const int per = (n + 7) >> 3, i = wg >> 3, t = (wg & 7) * per + i;
-  return i < per && t < n ? t : -1;
-}
-
 constexpr int W4_TILE_LDS(int bm, int bn, int ngc) { return 3 * bm * 128 + 4 * 4 * (bn / 128 * 1024 + ngc * 256); }
 
 // NGC: scale groups of a step (2 of 32 rows; else 1)
@@ -93,14 +88,13 @@ __global__ void __launch_bounds__(256, 1) w4_tile_kernel(const W4TileK a) {
   constexpr int MM = MT * NT;                        // products of a half step, in MT blocks with an LDS read each
   constexpr int U = 2 * NT;                          // half words that become operands in a half step
   constexpr int LATE = 2 * NR + XD;                  // DMA under way that the next step does not need
-  constexpr int FRAGS = MM;
   static_assert(NT < MT && NR <= MT && XD <= MT && U <= MT, "blocks");
   static_assert(R0 + RS * RB == W4_TILE_LDS(BM, BN, NGC) && R0 + RS * RB <= 160 * 1024, "LDS");
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r16 = lane & 15, g = lane >> 4;
 
-  const int item = tile_xcd_run(blockIdx.x, a.tiles * a.slices);
+  const int item = xcd_run(blockIdx.x, a.tiles * a.slices);
   if (item < 0) return;
   const int t = item / a.slices, slice = item - t * a.slices;
   // `group` row blocks by columns: neighbours in a run share rows of x and of w in their L2
@@ -232,37 +226,8 @@ __global__ void __launch_bounds__(256, 1) w4_tile_kernel(const W4TileK a) {
     xa = xn;
     ra = rn;
   }
-  // (no DMA may outlive the workgroup's LDS; the last products are not tracked by the compiler)
-  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_nop 15\n\ts_nop 7" ::: "memory");
-
-  if (a.slices > 1) {
-    const __amdgpu_buffer_rsrc_t mine = __builtin_amdgcn_make_buffer_rsrc(
-        a.slabs + (int64_t)t * a.slices * (FRAGS * 1024), 0, a.slices * FRAGS * 4096, 0x00020000);
-    auto at = [&](int s, int f) { return ((s * FRAGS + f) * 256 + tid) * 16; };
-#pragma unroll
-    for (int f = 0; f < FRAGS; ++f)
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[f / MT][f % MT]), mine, at(slice, f), 0, /*sc1*/ 16);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // every wave's sums are out ..
-    __syncthreads();
-    uint32_t* word = reinterpret_cast<uint32_t*>(lds);
-    if (tid == 0) word[0] = __hip_atomic_fetch_add(a.arrived + t, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // .. then one announces them
-    __syncthreads();
-    if (word[0] != (uint32_t)a.slices - 1) return;
-    constexpr int C = 8;   // fragments in flight
-#pragma unroll
-    for (int f0 = 0; f0 < FRAGS; f0 += C) {
-      f32x4 sum[C];
-#pragma unroll
-      for (int f = 0; f < C; ++f) sum[f] = f32x4{0.f, 0.f, 0.f, 0.f};
-      for (int s = 0; s < a.slices; ++s) {   // (in slice order, whoever is last: the same bits every time)
-#pragma unroll
-        for (int f = 0; f < C; ++f)
-          sum[f] += __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(mine, at(s, f0 + f), 0, /*sc1*/ 16));
-      }
-#pragma unroll
-      for (int f = 0; f < C; ++f) acc[(f0 + f) / MT][(f0 + f) % MT] = sum[f];
-    }
-  }
+  tile_settle(acc);
+  if (a.slices > 1 && !tile_add_slices(acc, a.slabs + (int64_t)t * a.slices * (MM * 1024), a.arrived + t, slice, a.slices, lds)) return;
 
   // Out through LDS, 64 rows at a time: a loop over rows then stores whole lines and applies the rest, in code short enough for the instruction
   // cache (written out per accumulator this was 10000 instructions, and 13 us more of the 101 of a tile of 4096 of k).
@@ -319,11 +284,6 @@ __global__ void __launch_bounds__(256, 1) w4_tile_kernel(const W4TileK a) {
   }
 }
 
-__global__ void __launch_bounds__(256) w4_tile_clear_kernel(uint32_t* p, int n) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i < n) p[i] = 0;
-}
-
 // Tiles, and what they take: us of a step of 64 k alone on the chip and with every CU busy (power), and of a tile beside its steps.
 // Fitted to 1900 timings of 163 products of 129 - 5120 rows; by them the tile taken is 1.3 % behind the best one on average.
 struct W4Tile {
@@ -378,13 +338,8 @@ template <int BM, int BN, int NGC>
 static void w4_tile_launch(const W4TileK& k, hipStream_t st) {
   constexpr int bytes = W4_TILE_LDS(BM, BN, NGC);
   auto fn = w4_tile_kernel<BM, BN, NGC>;
-  static bool opted[64] = {};   // > 64 KiB of dynamic LDS: once per kernel and device
-  int dev = 0;
-  (void)hipGetDevice(&dev);
-  if (dev < 0 || dev >= 64 || !opted[dev]) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-    if (dev >= 0 && dev < 64) opted[dev] = true;
-  }
+  static bool asked[64] = {};
+  tile_allow_lds(fn, bytes, asked);
   const unsigned wgs = (unsigned)((k.tiles * k.slices + 7) / 8 * 8);
   fn<<<dim3(wgs), dim3(256), bytes, st>>>(k);
 }
@@ -408,7 +363,7 @@ void launch_w4_tile(const GemmKParams& kp, const W4TilePlan& p, void* workspace,
   k.silu = kp.silu;
   k.wide = kp.ldc % 8 == 0 && aligned16(kp.c);
   k.arrived = (uint32_t*)workspace; k.slabs = (float*)((char*)workspace + W4_TILE_SYNC_BYTES);
-  if (p.slices > 1) w4_tile_clear_kernel<<<dim3(1), dim3(256), 0, st>>>(k.arrived, p.tiles);
+  if (p.slices > 1) tile_clear_kernel<<<dim3(1), dim3(256), 0, st>>>(k.arrived, p.tiles);
   ng == 4 ? w4_tile_shape<2>(p.tile, k, st) : w4_tile_shape<1>(p.tile, k, st);
 }
 
