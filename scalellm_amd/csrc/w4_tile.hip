@@ -73,6 +73,24 @@ __device__ __forceinline__ void in_turn(const F& f) {
   }
 }
 
+// Half a step's work on words lies so in its blocks: unit u of 2 nt (column tile u / 2) in the last block b with b * 2 nt / mt == u, and the DMA that
+// overwrites a stage in the last tw + ngc blocks, in front of their units: the first scales, words, second scales.  In the first half step the
+// stage that it overwrites is the one whose words (and second scales) for k 32 .. 63 are still on their way to registers; the DMA waits for
+// those it overwrites, and the order sees to it that their first unit, which waits for them anyway, is not in a later block.
+constexpr int w4_tile_unit_block(int u, int mt, int nt) {
+  int b = 0;
+  while ((b + 1) * 2 * nt / mt <= u) ++b;
+  return b;
+}
+constexpr bool w4_tile_words_in_order(int mt, int nt, int tw, int ngc) {
+  const int first = mt - tw - ngc;   // block of the first scales
+  for (int n = 0; n < nt; ++n) {
+    const int taken = w4_tile_unit_block(2 * n, mt, nt);
+    if (first + 1 + n / 2 < taken || (ngc == 2 && first + 1 + tw < taken)) return false;
+  }
+  return true;
+}
+
 constexpr int W4_TILE_LDS(int bm, int bn, int ngc) { return 3 * bm * 128 + 4 * 4 * (bn / 128 * 1024 + ngc * 256); }
 
 // NGC: scale groups of a step (2 of 32 rows; else 1)
@@ -89,6 +107,7 @@ __global__ void __launch_bounds__(256, 1) w4_tile_kernel(const W4TileK a) {
   constexpr int U = 2 * NT;                          // half words that become operands in a half step
   constexpr int LATE = 2 * NR + XD;                  // DMA under way that the next step does not need
   static_assert(NT < MT && NR <= MT && XD <= MT && U <= MT, "blocks");
+  static_assert(w4_tile_words_in_order(MT, NT, TW, NGC), "a stage's words are taken before they are overwritten");
   static_assert(R0 + RS * RB == W4_TILE_LDS(BM, BN, NGC) && R0 + RS * RB <= 160 * 1024, "LDS");
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -124,15 +143,16 @@ __global__ void __launch_bounds__(256, 1) w4_tile_kernel(const W4TileK a) {
     const char* base = a.x + ((int64_t)at_step(s) << 7);
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %2" : : "v"(xoff[i]), "s"(xdst + at + i * 1024), "s"(base) : "memory", "m0");
   };
-  auto dma_w = [&](int i, int s, uint32_t at) {   // i-th of NR
-    const int c = at_step(s);
-    if (i < TW) {
+  auto dma_w = [&](int i, int s, uint32_t at) {   // i-th of NR: scales, words, second scales
+    const int c = at_step(s), w = i - 1;
+    if (w >= 0 && w < TW) {
       const char* base = reinterpret_cast<const char*>(a.wq) + (int64_t)c * n_tiles * 1024;
-      asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %2" : : "v"(woff[i < TW ? i : 0]), "s"(rdst + at + i * 1024), "s"(base) : "memory", "m0");
+      asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %2" : : "v"(woff[w >= 0 && w < TW ? w : 0]), "s"(rdst + at + w * 1024), "s"(base) : "memory", "m0");
     } else {
-      const int64_t grp = NGC == 2 ? 2 * c + (i - TW) : c >> a.cpg_shift;
+      const int h = i > TW;
+      const int64_t grp = NGC == 2 ? 2 * c + h : c >> a.cpg_shift;
       const char* base = reinterpret_cast<const char*>(a.sz) + grp * a.N * 4;
-      asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, %2" : : "v"(zoff), "s"(rdst + at + TW * 1024 + (i - TW) * 256), "s"(base) : "memory", "m0");
+      asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, %2" : : "v"(zoff), "s"(rdst + at + TW * 1024 + h * 256), "s"(base) : "memory", "m0");
     }
   };
 
@@ -150,6 +170,7 @@ __global__ void __launch_bounds__(256, 1) w4_tile_kernel(const W4TileK a) {
     words[h][n] = *reinterpret_cast<const uint32_t*>(lds + wfrom + at + (n >> 1) * 1024 + (n & 1) * 64 + h * 8);
     if (h == 0 || NGC == 2) scales[NGC == 2 ? h : 0][n] = *reinterpret_cast<const uint32_t*>(lds + zfrom + at + (NGC == 2 ? h * 256 : 0) + (n >> 1) * 128 + (n & 1) * 16);
   };
+  auto taken = [&](uint32_t& v) { asm volatile("" : : "v"(v)); };
   W4Pieces dq[NT];
   auto piece = [&](int u, int q, int h) {   // q-th of four of unit u: words of half h
     const int n = u >> 1;
@@ -209,7 +230,13 @@ __global__ void __launch_bounds__(256, 1) w4_tile_kernel(const W4TileK a) {
   for (int s = 0; s < steps; ++s) {
     const uint32_t xn = xa == (XS - 1) * XB ? 0 : xa + XB, rn = ra == (RS - 1) * RB ? 0 : ra + RB;
     in_turn<MT>([&](auto b) {
-      if constexpr (b >= MT - NR) dma_w(b - (MT - NR), s + RS, ra);
+      if constexpr (b >= MT - NR) {
+        constexpr int i = b - (MT - NR);
+        // (what is fetched from there is waited for here at the latest)
+        if constexpr (i >= 1 && i <= TW) taken(words[1][2 * i - 2]), taken(words[1][2 * i - 1]);
+        if constexpr (i > TW) in_turn<NT>([&](auto n) { taken(scales[NGC - 1][n]); });
+        dma_w(i, s + RS, ra);
+      }
       read(b, 1, xa);
       if constexpr (b >= 1 && b <= NT) fetch(b - 1, 0, rn);
       block(b, FIRST);
