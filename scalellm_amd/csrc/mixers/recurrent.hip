@@ -660,8 +660,10 @@ __global__ void __launch_bounds__(64 * W, 2) recurrent_scan_kernel(const slm_rec
   };
   // the read-outs of a chunk, once every wave's part of them is there: of each lane's four rows a wave takes one (of 2 waves: two)
   const int o_row = a.heads * a.v_pad * 4;   // bytes
-  float* const o_from = a.o + (row0 - a.n_single) * a.heads * a.v_pad;
-  const uint32_t o_off = (uint32_t)((4 * g + wave) * o_row + (head * a.v_pad + l16) * 4);
+  float* const o_from = a.o + (row0 - a.n_single) * a.heads * a.v_pad + 16 * ct[0];
+  uint32_t o_off[NCT];   // (no scalar offset: that of a lane alone tells what is out of the buffer)
+#pragma unroll
+  for (int j = 0; j < NCT; ++j) o_off[j] = (uint32_t)((4 * g + wave) * o_row + (head * a.v_pad + 16 * (ct[j] - ct[0]) + l16) * 4);
   struct ReadOuts { float v[4 / W][NCT][W]; };
   auto collect = [&](int c, ReadOuts& y) {
 #pragma unroll
@@ -672,7 +674,7 @@ __global__ void __launch_bounds__(64 * W, 2) recurrent_scan_kernel(const slm_rec
         for (int w = 0; w < W; ++w) y.v[r][j][w] = reinterpret_cast<const float*>(&part_o[c & 1][j][w][lane])[r * W + wave];
   };
   auto finish = [&](int c, const ReadOuts& y) {   // (rows past the portion's last, and chunk -1, are out of the buffer)
-    const __amdgpu_buffer_rsrc_t out = __builtin_amdgcn_make_buffer_rsrc(o_from + (int64_t)16 * c * a.heads * a.v_pad, 0, c < 0 ? 0 : min(n - 16 * c, 16) * o_row, 0x00020000);
+    const __amdgpu_buffer_rsrc_t out = __builtin_amdgcn_make_buffer_rsrc(o_from + (int64_t)16 * c * a.heads * a.v_pad, 0, c < 0 ? 0 : min(n - 16 * c, 16) * o_row - 64 * ct[0], 0x00020000);
 #pragma unroll
     for (int r = 0; r < 4 / W; ++r)
 #pragma unroll
@@ -680,7 +682,7 @@ __global__ void __launch_bounds__(64 * W, 2) recurrent_scan_kernel(const slm_rec
         float sum = y.v[r][j][0];
 #pragma unroll
         for (int w = 1; w < W; ++w) sum += y.v[r][j][w];
-        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, sum), out, o_off + r * W * o_row, 64 * ct[j], 0);
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, sum), out, o_off[j] + r * W * o_row, 0, 0);
       }
   };
   // two sums of tiles side by side: the products of one wait for each other
