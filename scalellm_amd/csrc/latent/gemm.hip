@@ -2,7 +2,7 @@
 //
 // Four waves, one to a SIMD, hold a quarter of the tile each: 128 x 128 products of 16 x 16 x 32 in 256 accumulators read 0.5 KB
 // of LDS per 1024 matrix-pipe cycles and SIMD, where eight waves of 128 x 64 read 0.75 -- and what bounds a large product here is power
-// (8192^3: 582 us on zeros, 767 on normal numbers), which operand traffic is part of (32 x 32 x 16 products: 815).  The
+// (8192^3: 572 us on zeros, 724 on normal numbers), which operand traffic is part of (with 32 x 32 x 16 products 6 % more).  The
 // accumulators are pinned to the second half of the register file by inline asm: left to itself the compiler spreads them over
 // both and copies 1000 registers a step.
 //
@@ -10,16 +10,18 @@
 // the DMA does on its global side.  Each step's products come in two halves of 32 k: the first runs over the LDS reads of the
 // second, the second over those of the next step's first.  One barrier a step, between the halves: there this stage has been read
 // by all waves and the next one has landed.  x has three stages and its DMA runs half a step apart from that of w: all 16
-// instructions of a step at once back up in the address unit, and a wave alone on its SIMD stalls with them (582 us against
-// 665).  256 x 256: 160 KB of LDS.
+// instructions of a step at once back up in the address unit, and a wave alone on its SIMD stalls with them (on zeros 14 %
+// more).  256 x 256: 160 KB of LDS.
 //
 // Tiles that do not fill the last round of the chip are cut in K (slices > 1): every slice leaves fp32 sums past the caches, the last one
 // to arrive (a counter per tile) adds them up in slice order and stores.  Nobody waits for anybody.
 //
-// us, vendor product (and the GLU's launch) / this, normal numbers: 5692 x 28672 x 4096 GLU 1093 / 997 (1.34 PFLOP/s), 5692 x 4096 x 14336 739 / 485,
-// 5692 x 4096 x 4096 149 / 147, 3226 x 28672 x 4096 GLU 712 / 571, 3226 x 16896 x 4096 443 / 349, 4096 x 16384 x 2048 GLU 227 / 216, 4096 x 8512 x 2048
-// 153 / 120, 1000 x 4096 x 14336 129 / 107, 600 x 28672 x 4096 GLU 148 / 134, 300 x 4096 x 14336 73 / 63, 200 x 16384 x 2048 GLU 31 / 23,
-// 8192^3 701 / 729; short and narrow 207 x 4096 x 4096 18.5 / 19.8, 178 x 3664 x 2048 10.6 / 14.6 (of up to 128 rows: the vendor's).
+// us by the device, vendor product (and the GLU's launch) / this, normal numbers: 5692 x 28672 x 4096 GLU 1073 / 1005 (1.33 PFLOP/s),
+// 5692 x 4096 x 14336 740 / 500, 5692 x 4096 x 4096 148 / 148, 3226 x 28672 x 4096 GLU 708 / 570, 3226 x 16896 x 4096 449 / 352, 4096 x 16384 x 2048 GLU
+// 230 / 219, 4096 x 8512 x 2048 155 / 121, 1000 x 4096 x 14336 134 / 108, 600 x 28672 x 4096 GLU 148 / 134, 300 x 4096 x 14336 70 / 63,
+// 207 x 16384 x 2048 GLU 31 / 24.  Behind the vendor product where its tiles fill whole rounds (8192^3 685 / 724, 4096^3 89 / 96), with one row of tiles
+// over large weights (129 x 28672 x 4096 56 / 70), and on short and narrow products (207 x 4096 x 4096 17.6 / 20.8, 207 x 3664 x 2048 11.1 / 14.6,
+// 207 x 512 x 2048 8.4 / 15.3), which its callers take here for the sake of the host.
 #include "latent_common.h"
 #include "tile_common.h"
 

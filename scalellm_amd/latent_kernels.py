@@ -16,7 +16,7 @@ from .kernels import reserve_workspace
 
 # rows up to which a bf16 product of row-major weights is streamed
 STREAM_MAX_ROWS = 32
-# rows from which the tile kernel does a stored product of row-major weights
+# rows from which the tile kernel may do a stored product of row-major weights
 TILE_MIN_ROWS = 129
 # the same of weights in the streamed layout (stream_layout()), where the product reduces or activates in its epilogue
 STREAM_LAYOUT_MAX_ROWS = 128
@@ -239,6 +239,19 @@ def _store_rows(N: int, K: int) -> int:
     return 64 if N >= 8192 and K <= 2048 + 5 * (N - 8192) // 2 else STREAM_MAX_ROWS
 
 
+def _tile_pays(M: int, N: int, K: int, glu: bool) -> bool:
+    """Is a product that the tile kernel takes its own, or the vendor's?  us by the device, vendor / tiles, where they are the vendor's:
+    129 - 160 rows of large weights, whose one row of tiles reads them slower (28672 x 4096 GLU 62 / 77, from 161 rows 67 / 65; of the largest up to 192
+    rows: 16384 x 8192, 170 rows, 75 / 93), and
+    256 x 256 tiles that fill whole rounds of the chip (4096 x 4096, K 2048 49 / 53, 4096 89 / 96; 4096 x 16384 x 4096 364 / 395).
+    Short and narrow products are up to 8 us longer by the device (200 x 512 x 2048 8 / 15, 200 x 4096 x 4096 18 / 21) and stay here all the same: steps
+    with prompts run eagerly, and the vendor product takes 8 us more of the host for each (18 / 10).  Steps of four layers with one prompt of
+    150 - 300 tokens, all their products by the vendor / here: 2b 847 / 580 and 836 / 618, 8b 975 / 903 and 1189 / 1065."""
+    if 128 < M <= (192 if N * K >= 1 << 27 else 160) and N * K >= 1 << 26:
+        return False
+    return glu or M <= 1024 or K < 1024 or -(-M // 256) * -(-N // 256) % 256 != 0
+
+
 def _gemm(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, glu=None, tile: int = -1, slices: int = 0) -> bool:
     """out = x w^T, or with glu = (limit, alpha, shift) the clamped GLU of its halves, by the tile kernel for many rows.  False:
     shapes and strides that it does not take."""
@@ -275,7 +288,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None,
     if not streams_rows(x):
         # (stored products of up to 128 rows are the vendor's, whose small tiles leave fewer CUs idle: 125 x 2048 x 4096 10.7 us against
         # 18.5, 96 x 12288 x 2048 16.8 against 19.6, 85 x 12608 x 4096 32.7 against 35.0)
-        return out if M >= TILE_MIN_ROWS and _gemm(x, w, out) else torch.mm(x, w.t(), out=out)
+        return out if M >= TILE_MIN_ROWS and _tile_pays(M, N, K, False) and _gemm(x, w, out) else torch.mm(x, w.t(), out=out)
     a = _linear_args(x, w, M, N, K)
     a.ldx, a.ldw, a.ldy, a.y, a.epilogue = x.stride(0), K, out.stride(0), _p(out), _lib.LIN_STORE
     _run_linear(a)
@@ -338,8 +351,8 @@ def linear_slabs(x: torch.Tensor, w: torch.Tensor, layout: Optional[torch.Tensor
 
 def linear_glu(x: torch.Tensor, w_gate_up: torch.Tensor, out: torch.Tensor, limit: float, alpha: float = GLU_ALPHA,
                shift: float = GLU_SHIFT, layout: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """out = clamped GLU of the two halves of x [gate | up]^T: the activation is the product's epilogue where a
-    streaming kernel runs, one more launch behind the vendor GEMM otherwise.  layout: stream_layout(w_gate_up, glu=True)."""
+    """out = clamped GLU of the two halves of x [gate | up]^T: the activation is the product's epilogue where a streaming kernel or
+    the tile kernel runs, one more launch behind the vendor GEMM otherwise.  layout: stream_layout(w_gate_up, glu=True)."""
     M, N, K = _check_xw(x, w_gate_up)
     half = N // 2
     _need(out.shape == (M, half) and out.stride(1) == 1 and out.dtype == x.dtype, "linear_glu: out [M, N / 2]")
@@ -357,7 +370,7 @@ def linear_glu(x: torch.Tensor, w_gate_up: torch.Tensor, out: torch.Tensor, limi
         a.ldx, a.ldw, a.ldy, a.y, a.epilogue = x.stride(0), K, out.stride(0), _p(out), _lib.LIN_GLU
         a.limit, a.glu_alpha, a.glu_shift = float(limit), float(alpha), float(shift)
         (_run_linear if s is None else _run_stream)(a)
-    elif not _gemm(x, w_gate_up, out, (float(limit), float(alpha), float(shift))):
+    elif not (_tile_pays(M, N, K, True) and _gemm(x, w_gate_up, out, (float(limit), float(alpha), float(shift)))):
         gu = torch.mm(x, w_gate_up.t())
         clamped_glu(gu, out, limit, alpha, shift)
     return out

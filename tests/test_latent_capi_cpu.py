@@ -225,6 +225,19 @@ def test_stored_products_are_streamed_where_that_is_faster(N, K, rows, monkeypat
         assert _route(monkeypatch, lambda lk, x, w, layout: lk.linear(x, w, layout=layout), M, N, K) == ("stream" if M <= rows else "vendor"), M
 
 
+def test_products_of_many_rows_are_the_vendors_where_that_is_faster():
+    from scalellm_amd.latent_kernels import _tile_pays as pays
+    # one row of tiles over large weights, and past it
+    assert not pays(129, 28672, 4096, True) and not pays(160, 28672, 4096, False) and pays(161, 28672, 4096, True)
+    assert not pays(192, 16384, 8192, True) and pays(193, 16384, 8192, True) and pays(160, 16384, 4095, True) and pays(128, 28672, 4096, True)
+    # whole rounds of 256 x 256 tiles, a tile's last rows missing too; one tile more or less; short contractions and few rows; with the GLU
+    assert not pays(4096, 4096, 4096, False) and not pays(3841, 4096, 2048, False) and not pays(2048, 16384, 1024, False)
+    assert pays(3840, 4096, 4096, False) and pays(4097, 4096, 4096, False) and pays(4096, 4352, 4096, False)
+    assert pays(4096, 4096, 960, False) and pays(1024, 16384, 4096, False) and pays(4096, 4096, 4096, True)
+    # short and narrow ones are the tiles'
+    assert pays(200, 512, 2048, False) and pays(129, 3664, 2048, False)
+
+
 def test_products_of_changed_weights_are_slabs_as_without_a_layout():
     import torch
     from scalellm_amd import latent_kernels as lk
