@@ -657,7 +657,7 @@ class LlamaDecodeStep:
         single rank; tables and ids that its kernel does not take go through torch."""
         s, table = self.shape, self.embed
         weight = self.layers[0]["in_norm"] if self.layers and not self._folds(tokens.numel()) else None
-        if (tokens.dtype != torch.int32 or not tokens.is_contiguous() or not table.is_contiguous() or table.dtype != resid.dtype or
+        if (not tokens.is_cuda or tokens.dtype != torch.int32 or not tokens.is_contiguous() or not table.is_contiguous() or table.dtype != resid.dtype or
                 table.shape != (s.vocab, s.hidden) or s.hidden % 8 or s.hidden > 16384 or table.data_ptr() % 16 or
                 (weight is not None and (weight.dtype != table.dtype or not weight.is_contiguous() or weight.data_ptr() % 16))):
             resid.copy_(table[tokens.long()])

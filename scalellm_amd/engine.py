@@ -111,10 +111,10 @@ class Step:
 
 class StepBuilder:
     """portion_min (of the model): entries that bring at least so many tokens go behind the others and are described
-    as portions; None: the model serves every row alike."""
+    as portions; None: the model serves every row alike.  vocab: token ids are below it (None: they are not looked at)."""
 
-    def __init__(self, allocator: BlockAllocator, device, portion_min: Optional[int] = None):
-        self.allocator, self.device, self.portion_min = allocator, device, portion_min
+    def __init__(self, allocator: BlockAllocator, device, portion_min: Optional[int] = None, vocab: Optional[int] = None):
+        self.allocator, self.device, self.portion_min, self.vocab = allocator, device, portion_min, vocab
 
     def build(self, entries: Seq[Tuple[Sequence, int]], logit_rows: Optional[Dict[int, Seq[int]]] = None) -> Step:
         """entries: (sequence, number of its next tokens).  logit_rows: entry -> places among its new tokens whose
@@ -144,7 +144,10 @@ class StepBuilder:
             bcu.append(bcu[-1] + blocks.size)
             q_cu.append(q_cu[-1] + n)
             kv_cu.append(kv_cu[-1] + c + n)
-        arrays = [np.concatenate(tokens), np.concatenate(pos), np.concatenate(slots), np.concatenate(table),
+        ids = np.concatenate(tokens)
+        if self.vocab is not None and (ids.min() < 0 or ids.max() >= self.vocab):   # (here they are on the host: kernels do not refuse any)
+            raise ValueError(f"token ids are 0 .. {self.vocab - 1}")
+        arrays = [ids, np.concatenate(pos), np.concatenate(slots), np.concatenate(table),
                   np.asarray(bcu), np.asarray(q_cu), np.asarray(kv_cu)]
         if self.allocator.n_states:
             arrays.append(np.asarray([entries[i][0].state for i in order]))
@@ -244,14 +247,14 @@ class LLMEngine:
         self.model, self.device = model, torch.device(device)
         self.options = o = options or EngineOptions()
         self.allocator = BlockAllocator(n_blocks, block_size, getattr(model, "n_states", 0))
-        self.builder = StepBuilder(self.allocator, self.device, getattr(model, "portion_min", None))
+        shape = getattr(model, "shape", None)
+        self.max_positions = getattr(model, "max_positions", None) or shape.max_position
+        self.vocab = getattr(model, "vocab", None) or shape.vocab
+        self.builder = StepBuilder(self.allocator, self.device, getattr(model, "portion_min", None), self.vocab)
         self.scheduler = Scheduler(self.allocator, o.max_seqs, o.max_step_tokens)
         self.runner = ModelRunner(model, self.device, ModelRunnerOptions(
             block_size=block_size, cuda_graph_max_seq_len=o.graph_max_seq_len, cuda_graph_batch_sizes=list(o.graph_batch_sizes)),
             return_logits=True)
-        shape = getattr(model, "shape", None)
-        self.max_positions = getattr(model, "max_positions", None) or shape.max_position
-        self.vocab = getattr(model, "vocab", None) or shape.vocab
         self._next_id = 0
 
     def capture_graphs(self) -> None:

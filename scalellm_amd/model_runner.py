@@ -204,7 +204,16 @@ class ModelRunner:
         g.capture(self._run)
         self.graphs[batch_size] = g
 
+    def _check_ids(self, tokens: torch.Tensor) -> None:
+        """Refuses ids that no row of the embedding has, as torch's indexing would, where the ids are on the host.  Kernels
+        refuse none: an id on the device outside the table makes its row NaN (LlamaDecodeStep)."""
+        vocab = getattr(self.model, "vocab", None) or getattr(getattr(self.model, "shape", None), "vocab", None)
+        if vocab and tokens.numel() and not -vocab <= int(tokens.min()) <= int(tokens.max()) < vocab:
+            raise IndexError(f"token ids are below {vocab}")
+
     def forward(self, tokens, positions, params: InputParameters, num_sequences: Optional[int] = None):
+        if tokens.device.type == "cpu":
+            self._check_ids(tokens)
         bs = int(params.q_cu_seq_lens.numel() - 1) if num_sequences is None else num_sequences
         g = self.graphs.get(bs)
         # (a graph gives the last row of every sequence: other rows are an eager step's)

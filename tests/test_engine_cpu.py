@@ -13,6 +13,7 @@ from scalellm_amd.dagupel import DagupelConfig
 from scalellm_amd.engine import BlockAllocator, EngineOptions, LLMEngine, OutOfBlocks, Scheduler, Sequence, StepBuilder
 from scalellm_amd.latent_layers import LatentPlan, YarnScaling, rotary_table
 from scalellm_amd.layers import Portion
+from scalellm_amd.model_runner import ModelRunner, ModelRunnerOptions
 from scalellm_amd.registry import ModelLimits, architecture_of, load_model, model_class
 from scalellm_amd.sampling import Sampler, SamplingParams
 
@@ -170,6 +171,32 @@ def test_step_builder_orders_portions_behind_tokens():
     assert StepBuilder(alloc, "cpu").build([(a, 6), (c, 1)]).params.portions == []
     with pytest.raises(ValueError):
         b.build([(c, 2)])
+
+
+def test_token_ids_outside_the_vocabulary_are_refused_on_the_host():
+    """Where a step is built, and by the runner where they come as a host tensor: kernels refuse none."""
+    alloc = BlockAllocator(20, 4)
+    b = StepBuilder(alloc, "cpu", vocab=12)
+    assert b.build([(Sequence("a", [0, 11]), 2)]).tokens.tolist() == [0, 11]
+    for ids in ([3, 12], [-1, 3]):
+        with pytest.raises(ValueError):
+            b.build([(Sequence("b", [1]), 1), (Sequence("c", ids), 2)])
+    assert b.build([(Sequence("d", [3, 12]), 1)]).tokens.tolist() == [3]   # (the one that is not fed yet)
+
+    class Model:
+        vocab = 12
+
+        def forward(self, tokens, positions, params):
+            return tokens
+    runner = ModelRunner(Model(), "cpu", ModelRunnerOptions())
+    params = b.build([(Sequence("e", [1, 2]), 2)]).params
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32)  # noqa: E731
+    assert runner.forward(i32([11, -12]), i32([0, 1]), params).tolist() == [11, -12]   # (from the end, as torch counts)
+    for ids in ([12, 0], [0, -13]):
+        with pytest.raises(IndexError):
+            runner.forward(i32(ids), i32([0, 1]), params)
+    with pytest.raises(ValueError):   # (through the engine, entries that no request check has seen)
+        LLMEngine(Counter(8, 4), 8, 4, "cpu").run_entries([(Sequence("f", [Counter.vocab]), 1)])
 
 
 @pytest.mark.parametrize("window", [0, 1, 7, 16, 200])

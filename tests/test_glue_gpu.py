@@ -270,3 +270,13 @@ def test_last_rows(lens, dim):
     x = torch.randn(sum(lens), dim, device=DEV).to(torch.bfloat16)
     q_cu = torch.tensor([0, *np.cumsum(lens)], dtype=torch.int32, device=DEV)
     assert torch.equal(kernels.last_rows(x, q_cu), x[(q_cu[1:] - 1).long()])
+
+
+def test_step_takes_token_ids_from_the_host():
+    """Ids in a host tensor, as torch's indexing takes them: the same step as with ids on the device."""
+    from scalellm_amd.decode import LlamaDecodeStep, LlamaShape, make_decode_inputs
+    shape = LlamaShape.tiny()
+    tokens, positions, params, n_blocks = make_decode_inputs(6, 40, 16, torch.device(DEV), seed=3, vocab=shape.vocab)
+    model = LlamaDecodeStep(shape, 6, n_blocks, 16, dtype=torch.bfloat16, device=torch.device(DEV), seed=0, kv_fill="randn", group_size=128)
+    want = model.forward(tokens, positions, params, return_logits=True).clone()
+    assert torch.equal(model.forward(tokens.cpu(), positions, params, return_logits=True), want)
