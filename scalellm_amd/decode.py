@@ -724,16 +724,18 @@ class LlamaDecodeStep:
             o_buf, down_buf = b["o"][:T], b["down"][:T]
 
         self._run_layers(T, positions, params, o_buf, down_buf, ar, normed_in)
-        # final-norm output of each sequence's last token: all rows where every sequence brings one (what _lane_split relies on too)
+        # last: final-norm output of each sequence's last token -- all rows where every sequence brings one (what _lane_split relies on too).
+        # last_hidden keeps it; of a captured step it is memory of the step's, which the next one overwrites.
         q_cu = params.q_cu_seq_lens
         if params.q_max_seq_len == 1 and T == q_cu.numel() - 1:
-            self.last_hidden = normed
+            last = normed
+            self.last_hidden = normed if torch.cuda.is_current_stream_capturing() else normed.clone()
         elif q_cu.dtype == torch.int32 and q_cu.is_contiguous() and s.hidden % 8 == 0:
-            self.last_hidden = kernels.last_rows(normed, q_cu)
+            self.last_hidden = last = kernels.last_rows(normed, q_cu)
         else:
-            self.last_hidden = normed[(q_cu[1:] - 1).long()]
-        logits = self.last_hidden @ self.lm_head  # plain library GEMM (hipBLASLt): not on the graded path
-        if ar is not None and not return_logits and self.last_hidden.size(0) <= ar.max_tokens \
+            self.last_hidden = last = normed[(q_cu[1:] - 1).long()]
+        logits = last @ self.lm_head  # plain library GEMM (hipBLASLt): not on the graded path
+        if ar is not None and not return_logits and last.size(0) <= ar.max_tokens \
                 and 4 * pa.world_size <= s.hidden:
             return self._greedy_over_vocab_shards(logits, ar)
         if pa.world_size > 1:

@@ -272,11 +272,25 @@ def test_last_rows(lens, dim):
     assert torch.equal(kernels.last_rows(x, q_cu), x[(q_cu[1:] - 1).long()])
 
 
-def test_step_takes_token_ids_from_the_host():
-    """Ids in a host tensor, as torch's indexing takes them: the same step as with ids on the device."""
+def _tiny_llama():
     from scalellm_amd.decode import LlamaDecodeStep, LlamaShape, make_decode_inputs
     shape = LlamaShape.tiny()
     tokens, positions, params, n_blocks = make_decode_inputs(6, 40, 16, torch.device(DEV), seed=3, vocab=shape.vocab)
     model = LlamaDecodeStep(shape, 6, n_blocks, 16, dtype=torch.bfloat16, device=torch.device(DEV), seed=0, kv_fill="randn", group_size=128)
+    return model, tokens, positions, params
+
+
+def test_step_takes_token_ids_from_the_host():
+    """Ids in a host tensor, as torch's indexing takes them: the same step as with ids on the device."""
+    model, tokens, positions, params = _tiny_llama()
     want = model.forward(tokens, positions, params, return_logits=True).clone()
     assert torch.equal(model.forward(tokens.cpu(), positions, params, return_logits=True), want)
+
+
+def test_last_hidden_of_a_step_outlives_the_next_one():
+    model, tokens, positions, params = _tiny_llama()
+    logits = model.forward(tokens, positions, params, return_logits=True)
+    hidden, rows = model.last_hidden, model.last_hidden.clone()
+    assert torch.equal(rows @ model.lm_head, logits)
+    model.forward((tokens + 1) % model.shape.vocab, positions, params)
+    assert torch.equal(hidden, rows) and not torch.equal(model.last_hidden, rows)
