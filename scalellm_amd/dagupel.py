@@ -165,7 +165,8 @@ class DagupelStep:
         first = self.layers[0].norm1 if self.layers else None
         lk.residual_norm(resid, h, first, c.eps, embed=(tokens, self.table, positions, self.pos_table))
         n = len(self.layers)
-        rows = lk.wanted_rows(params, T if n else 0)   # (None: the last sum's launch norms them too)
+        # (None: the last sum's launch norms them too -- not where somebody sees, and may change, the stream behind it)
+        rows = lk.wanted_rows(params, T if n and self.on_layer is None else 0)
         for i, L in enumerate(self.layers):
             nxt = self.layers[i + 1].norm1 if i + 1 < n else self.final_norm if rows is None else None
             delta = L.attn.forward(h, positions, self.caches[i], params)

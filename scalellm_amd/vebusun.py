@@ -190,7 +190,8 @@ class VebusunStep:
         resid = torch.empty(T, c.width, dtype=torch.float32, device=self.device)
         h = torch.empty(T, self.k_width, dtype=self.dtype, device=self.device)
         n = len(self.layers)
-        rows = lk.wanted_rows(params, T if n else 0)   # (None: the last sum's launch norms them too)
+        # (None: the last sum's launch norms them too -- not where somebody sees, and may change, the stream behind it)
+        rows = lk.wanted_rows(params, T if n and self.on_layer is None else 0)
         lk.residual_norm(resid, h, self.layers[0].norm1 if n else None, c.eps, embed=(tokens, self.embed, None, None), mult=c.embedding_scale)
         for i, L in enumerate(self.layers):
             nxt = self.layers[i + 1].norm1 if i + 1 < n else self.final_norm if rows is None else None

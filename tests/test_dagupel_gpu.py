@@ -100,6 +100,17 @@ def test_residual_stream_after_every_layer(name):
         np.testing.assert_allclose(g, w, atol=2e-5 * np.abs(w).max(), err_msg=f"layer {i}")
 
 
+def test_logits_follow_a_stream_that_is_changed_behind_the_last_layer():
+    """Steps of single tokens, whose last norm needs no launch of its own, as steps with prompts."""
+    cfg, t, tokens, _ = _model("odd")
+    engine = _engine(cfg, t, torch.float32)
+    engine.model.on_layer = lambda i, x: x.zero_() if i == len(cfg["layers"]) - 1 else None
+    s = _seq("s", tokens[:9])
+    for n in (7, 1, 1):
+        _, logits = engine.run_entries([(s, n)])
+        assert not logits.any()   # (the norm of zeros)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("name", ["odd", "wide", "deep"])
 def test_mixed_batches_and_reused_blocks(name, dtype):
