@@ -848,7 +848,8 @@ static int plan_gemm(const slm_w4_gemm_args* a, GemmPlan* pl) {
   const int tile = tune_get(TUNE_W4_TILE, -1);
   // (never a GEMV: its activations may be what a norm prologue makes, and not in memory)
   if (a->dtype == SLM_BF16 && !pl->gemv && tile != 0 && (tile > 0 || ((a->flags & SLM_W4_TILES) && w4_tile_rows(a->M, a->K, a->N))) && ((a->M - 1) * a->lda + a->K) * 2 < ((int64_t)1 << 31) &&
-      !(a->flags & SLM_W4_SHARES_CHIP) && !tune_is_set(TUNE_W4_MT) && !tune_is_set(TUNE_W4_SPLITK)) {
+      !(a->flags & SLM_W4_SHARES_CHIP) && !tune_is_set(TUNE_W4_MT) && !tune_is_set(TUNE_W4_SPLITK) &&
+      (tile > 0 || !(tune_is_set(TUNE_W4_XL_SK) || tune_is_set(TUNE_W4_XL_MODEL)))) {   // (a knob of the other kernels asks for them)
     pl->tiled = 1;
     pl->xl_sk = 0;
     pl->split_k = 1;

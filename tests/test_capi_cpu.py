@@ -452,6 +452,25 @@ def test_gemv_norm_prologue_host_side():
     assert L.slm_w4a16_gemv_norm(C.byref(g), C.byref(n), None) == 0   # empty batch
 
 
+def test_knobs_of_the_256_row_kernels_reach_calls_that_may_take_tiles():
+    """Calls that let sums come in another order take four-wave tiles; a set knob of the 256 x 256 kernel asks for that one."""
+    L = _lib.lib()
+    assert L.slm_tuning_clear(None) == 0
+    g = W4GemmArgs()
+    g.M, g.K, g.N, g.lda, g.ldc, g.group_size, g.dtype = 2648, 4096, 4096, 4096, 4096, 128, 1
+    size = lambda flags: (setattr(g, "flags", flags), L.slm_w4a16_gemm_workspace_bytes(C.byref(g)))[1]  # noqa: E731
+    assert size(0) > 0 and size(_lib.SLM_W4_TILES) == 0   # (stream-K scratch; 176 tiles are not cut)
+    for knob, value in ((b"SLM_W4_XL_SK", 2), (b"SLM_W4_XL_SK", 0), (b"SLM_W4_XL_MODEL", 0)):
+        assert L.slm_tuning_set(knob, value) == 0
+        try:
+            assert size(_lib.SLM_W4_TILES) == size(0)
+            assert (size(0) > 0) == (knob != b"SLM_W4_XL_SK" or value == 2)
+            assert L.slm_tuning_set(b"SLM_W4_TILE", 1) == 0
+            assert size(_lib.SLM_W4_TILES) == 0   # (both set: the tiles)
+        finally:
+            assert L.slm_tuning_clear(None) == 0
+
+
 def test_forced_tiles_leave_gemvs_alone():
     """SLM_W4_TILE asks for tiles that read their activations from memory; a one-row GEMV may get them from a norm prologue, so its plan
     is the same with the knob as without it."""
