@@ -55,7 +55,7 @@ __device__ __forceinline__ bool tile_add_slices(f32x4 (&acc)[NT][MT], float* sla
   return true;
 }
 
-// (a kernel, not a memset: the call may be captured)
+// (a kernel: the call may be captured, and memset nodes of a graph have given wrong results on later replays)
 static __global__ void __launch_bounds__(256) tile_clear_kernel(uint32_t* p, int n) {
   const int i = blockIdx.x * 256 + threadIdx.x;
   if (i < n) p[i] = 0;

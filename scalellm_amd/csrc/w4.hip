@@ -35,6 +35,7 @@
 //    prefill-sized M x N             w4_xl.hip     symmetric 256 x 256 tiles
 //    the same in bf16                w4_tile.hip   four waves a tile (SLM_W4_TILES)
 // (DESIGN.md 3.3 has the measurements behind each boundary.)
+#include "tile_common.h"
 #include "w4_common.h"
 #include "tuning.h"
 
@@ -1086,8 +1087,8 @@ static int gemm_impl(const slm_w4_gemm_args* a, const slm_w4_norm_prologue* np, 
   } else if (pl.xl_sk) {
     kp.sk_part = reinterpret_cast<float*>(a->workspace);
     kp.sk_sync = reinterpret_cast<unsigned*>(reinterpret_cast<char*>(a->workspace) + W4_XL_SK_WGS * W4_XL_SK_SLOT_BYTES);
-    // the ticket and the flags start at zero on every call (a memset node under capture)
-    if (hipMemsetAsync(kp.sk_sync, 0, W4_XL_SK_SYNC_BYTES, st) != hipSuccess) return hip_check_launch();
+    // the ticket and the flags start at zero on every call
+    tile_clear_kernel<<<dim3(W4_XL_SK_SYNC_BYTES / 1024), dim3(256), 0, st>>>(kp.sk_sync, (int)(W4_XL_SK_SYNC_BYTES / 4));
     launch_gemm_xl_sk(kp, a->dtype, pl.ng, W4_XL_SK_WGS, st);
   } else
   if (pl.ks)

@@ -657,7 +657,7 @@ def test_stream_k_form_matches_the_oracle_and_the_tile_form(M, K, N, dtype):
 
 def test_stream_k_form_repeats_bit_identically_and_replays_under_a_graph():
     """The owner adds the partial tiles of the workgroups in front of it in workgroup order, whoever finishes
-    first: 20 launches next to a bandwidth hog give the same bits; captured (the memset node that clears the ticket
+    first: 20 launches next to a bandwidth hog give the same bits; captured (the launch that clears the ticket
     and the flags + the kernel) and replayed, too."""
     from scalellm_amd import kernels
     M, K, N = 2648, 4096, 4096
@@ -680,12 +680,39 @@ def test_stream_k_form_repeats_bit_identically_and_replays_under_a_graph():
         g = torch.cuda.CUDAGraph()
         with torch.cuda.graph(g):
             kernels.gptq_gemm(a, packed, c)
-            kernels.gptq_gemm(a, packed, c)   # (twice: the second call's memset node follows the first's kernel)
+            kernels.gptq_gemm(a, packed, c)   # (twice: the second call's clearing follows the first's kernel)
         for _ in range(3):
             c.fill_(float("nan"))
             g.replay()
             torch.cuda.synchronize()
             assert torch.equal(c, first)
+
+
+@pytest.mark.parametrize("knobs", [dict(SLM_W4_XL_SK=2), dict(SLM_W4_TILE=1 + 8 * 3), dict()])
+def test_products_record_no_memset_into_a_graph(knobs):
+    """What calls of many rows clear, they clear by kernels: stream-K, four-wave tiles that are cut, the plan's own choice."""
+    import ctypes as C
+    from scalellm_amd import kernels
+    M, K, N = 2648, 4096, 4096
+    _, packed, a, _ = _sk_case(M, K, N, "bf16", fmt="gptq")
+    c = torch.empty(M, N, device=DEV, dtype=torch.bfloat16)
+    with kernels.tuning(**knobs):
+        kernels.gptq_gemm(a, packed, c)
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph(keep_graph=True)
+        with torch.cuda.graph(g):
+            kernels.gptq_gemm(a, packed, c)
+    hip = C.CDLL("libamdhip64.so")
+    graph, n = C.c_void_p(g.raw_cuda_graph()), C.c_size_t(0)
+    assert hip.hipGraphGetNodes(graph, None, C.byref(n)) == 0 and n.value > 0
+    nodes = (C.c_void_p * n.value)()
+    assert hip.hipGraphGetNodes(graph, nodes, C.byref(n)) == 0
+    kinds = []
+    for node in nodes:
+        kind = C.c_int(-1)
+        assert hip.hipGraphNodeGetType(C.c_void_p(node), C.byref(kind)) == 0
+        kinds.append(kind.value)
+    assert set(kinds) == {0}   # (hipGraphNodeTypeKernel)
 
 
 def test_stream_k_form_is_planned_where_the_round_model_says_so():
