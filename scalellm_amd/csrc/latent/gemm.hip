@@ -100,6 +100,7 @@ __global__ void __launch_bounds__(256, 1) gemm_kernel(const GemmK a) {
   };
   const int all = (int)(a.K >> 6), per = own < 0 ? all : (all + a.slices - 1) / a.slices;
   const int s0 = slice * per, steps = min(per, all - s0);   // (the plan leaves no slice empty)
+  __builtin_assume(steps > 0);   // (else the accumulators are set up once more, for a loop of none)
   auto kbytes = [&](int s) { return (int64_t)(s0 + min(s, steps - 1)) << 7; };   // (steps past the end load the last one again)
 
   // Columns of a pair of tiles go to them by fours, so that a lane ends with eight neighbours.  Chunk c of a row of w lies in slot

@@ -138,6 +138,7 @@ __global__ void __launch_bounds__(256, 1) w4_tile_kernel(const W4TileK a) {
   const uint32_t xdst = lds0 + wave * (XD * 1024), rdst = lds0 + R0 + wave * OWN;
   const int all = (int)(a.K >> 6), per = (all + a.slices - 1) / a.slices;
   const int s0 = slice * per, steps = min(per, all - s0);   // (the plan leaves no slice empty)
+  __builtin_assume(steps > 0);   // (else the accumulators are set up once more, for a loop of none)
   auto at_step = [&](int s) { return s0 + min(s, steps - 1); };   // (steps past the end load the last one again)
   auto dma_x = [&](int i, int s, uint32_t at) {
     const char* base = a.x + ((int64_t)at_step(s) << 7);
