@@ -100,7 +100,6 @@ __global__ void __launch_bounds__(256, 1) gemm_kernel(const GemmK a) {
   };
   const int all = (int)(a.K >> 6), per = own < 0 ? all : (all + a.slices - 1) / a.slices;
   const int s0 = slice * per, steps = min(per, all - s0);   // (the plan leaves no slice empty)
-  __builtin_assume(steps > 0);   // (else the accumulators are set up once more, for a loop of none)
   auto kbytes = [&](int s) { return (int64_t)(s0 + min(s, steps - 1)) << 7; };   // (steps past the end load the last one again)
 
   // Columns of a pair of tiles go to them by fours, so that a lane ends with eight neighbours.  Chunk c of a row of w lies in slot
@@ -130,7 +129,8 @@ __global__ void __launch_bounds__(256, 1) gemm_kernel(const GemmK a) {
     __builtin_amdgcn_sched_barrier(0);
   }
   uint32_t xa = 0, wa = 0, xl = 2 * XB;   // this step's stages, and the one that x is loaded to
-  for (int s = 0; s < steps; ++s) {
+  int s = 0;   // (a loop of no steps would have the accumulators set up once more)
+  do {
     const uint32_t xn = xa == (XS - 1) * XB ? 0 : xa + XB, wnext = wa == (WS - 1) * WB ? 0 : wa + WB;
     const int64_t kx = kbytes(s + 2);
 #pragma unroll
@@ -155,7 +155,7 @@ __global__ void __launch_bounds__(256, 1) gemm_kernel(const GemmK a) {
     xl = xa;
     xa = xn;
     wa = wnext;
-  }
+  } while (++s < steps);
   tile_settle(acc);
   if (own >= 0 && !tile_add_slices(acc, a.slabs + (int64_t)own * a.slices * (MM * 1024), a.arrived + own, slice, a.slices, lds)) return;
 

@@ -138,7 +138,6 @@ __global__ void __launch_bounds__(256, 1) w4_tile_kernel(const W4TileK a) {
   const uint32_t xdst = lds0 + wave * (XD * 1024), rdst = lds0 + R0 + wave * OWN;
   const int all = (int)(a.K >> 6), per = (all + a.slices - 1) / a.slices;
   const int s0 = slice * per, steps = min(per, all - s0);   // (the plan leaves no slice empty)
-  __builtin_assume(steps > 0);   // (else the accumulators are set up once more, for a loop of none)
   auto at_step = [&](int s) { return s0 + min(s, steps - 1); };   // (steps past the end load the last one again)
   auto dma_x = [&](int i, int s, uint32_t at) {
     const char* base = a.x + ((int64_t)at_step(s) << 7);
@@ -228,7 +227,8 @@ __global__ void __launch_bounds__(256, 1) w4_tile_kernel(const W4TileK a) {
     __builtin_amdgcn_sched_barrier(0);
   }
   uint32_t xa = 0, ra = 0;   // this step's stages
-  for (int s = 0; s < steps; ++s) {
+  int s = 0;   // (a loop of no steps would have the accumulators set up once more)
+  do {
     const uint32_t xn = xa == (XS - 1) * XB ? 0 : xa + XB, rn = ra == (RS - 1) * RB ? 0 : ra + RB;
     in_turn<MT>([&](auto b) {
       if constexpr (b >= MT - NR) {
@@ -253,7 +253,7 @@ __global__ void __launch_bounds__(256, 1) w4_tile_kernel(const W4TileK a) {
     });
     xa = xn;
     ra = rn;
-  }
+  } while (++s < steps);
   tile_settle(acc);
   if (a.slices > 1 && !tile_add_slices(acc, a.slabs + (int64_t)t * a.slices * (MM * 1024), a.arrived + t, slice, a.slices, lds)) return;
 
