@@ -313,6 +313,8 @@ typedef struct slm_w4_gemm_args {
 #define SLM_W4_TILES 8
 
 SLM_API size_t slm_w4a16_gemm_workspace_bytes(const slm_w4_gemm_args* a);
+/* what of it the call cannot do without: with less than workspace_bytes four-wave tiles are not cut in K (slower where they are few) */
+SLM_API size_t slm_w4a16_gemm_workspace_required(const slm_w4_gemm_args* a);
 /* number of partial slabs the call will leave in the workspace (>= 2), or 0 when it writes c as usual */
 SLM_API int32_t slm_w4a16_gemm_deferred_splits(const slm_w4_gemm_args* a);
 SLM_API int slm_w4a16_gemm(const slm_w4_gemm_args* a, void* stream);

@@ -145,30 +145,31 @@ void LlamaForCausalLMHip::verify_loaded_weights() const {
 }
 
 // ---- per-lane scratch --------------------------------------------------------------------------
-const torch::Tensor& LlamaForCausalLMHip::scratch(int lane, size_t bytes) {
-  auto& t = scratch_[lane];
-  if (!t.defined() || static_cast<size_t>(t.nbytes()) < bytes) {
-    TORCH_CHECK(!capturing(), "LlamaForCausalLMHip: call reserve() before graph capture (scratch of ", bytes, " bytes)");
-    // a buffer that was ever handed to a kernel is never released: graphs captured earlier replay
-    // against its raw address (the rule of kernels.py / slm_torch_shim.cpp)
-    if (t.defined()) retired_.push_back(t);
-    t = torch::empty({static_cast<int64_t>(std::max<size_t>({bytes, size_t(1) << 20, t.defined() ? 2 * static_cast<size_t>(t.nbytes()) : 0}))},
-                     torch::dtype(torch::kUInt8).device(options_.device()));
+const torch::Tensor& LlamaForCausalLMHip::grown(torch::Tensor& t, size_t bytes, size_t required, const char* what) {
+  if (t.defined() && static_cast<size_t>(t.nbytes()) >= bytes) return t;
+  if (capturing() && required == 0) return t;
+  TORCH_CHECK(!capturing(), "LlamaForCausalLMHip: call reserve() before graph capture (", what, " of ", bytes, " bytes)");
+  torch::Tensor more;
+  try {
+    more = torch::empty({static_cast<int64_t>(std::max<size_t>({bytes, size_t(1) << 20, t.defined() ? 2 * static_cast<size_t>(t.nbytes()) : 0}))},
+                        torch::dtype(torch::kUInt8).device(options_.device()));
+  } catch (const c10::OutOfMemoryError&) {
+    if (required > 0) throw;
+    return t;
   }
+  // a buffer that was ever handed to a kernel is never released: graphs captured earlier replay
+  // against its raw address (the rule of kernels.py / slm_torch_shim.cpp)
+  if (t.defined()) retired_.push_back(t);
+  t = more;
   return t;
 }
 
-const torch::Tensor& LlamaForCausalLMHip::deferred(int lane, int slot, size_t bytes) {
-  auto& t = deferred_[lane][slot];
-  if (!t.defined() || static_cast<size_t>(t.nbytes()) < bytes) {
-    TORCH_CHECK(!capturing(), "LlamaForCausalLMHip: call reserve() before graph capture (slab buffer of ", bytes, " bytes)");
-    // a buffer that was ever handed to a kernel is never released: graphs captured earlier replay
-    // against its raw address (the rule of kernels.py / slm_torch_shim.cpp)
-    if (t.defined()) retired_.push_back(t);
-    t = torch::empty({static_cast<int64_t>(std::max<size_t>({bytes, size_t(1) << 20, t.defined() ? 2 * static_cast<size_t>(t.nbytes()) : 0}))},
-                     torch::dtype(torch::kUInt8).device(options_.device()));
-  }
-  return t;
+const torch::Tensor& LlamaForCausalLMHip::scratch(int lane, size_t bytes, size_t required) {
+  return grown(scratch_[lane], bytes, required, "scratch");
+}
+
+const torch::Tensor& LlamaForCausalLMHip::deferred(int lane, int slot, size_t bytes, size_t required) {
+  return grown(deferred_[lane][slot], bytes, required, "slab buffer");
 }
 
 void LlamaForCausalLMHip::reserve(int64_t n_tokens) {
@@ -318,8 +319,8 @@ void LlamaForCausalLMHip::pre_attn(Lane& ln, size_t li, std::vector<KVCache>& kv
   // the qkv projection is column-parallel: its split-K slabs can go to the RoPE + append kernel on
   // any world size
   const int flags = SLM_W4_DEFER_REDUCE | chip_flag_;
-  const size_t need = w.workspace_bytes(n, flags);
-  ln.qkv_splits = w.forward_into(ln.normed, ln.qkv, flags, deferred(ln.idx, 0, need));
+  const size_t need = w.workspace_bytes(n, flags), required = w.workspace_required(n, flags);
+  ln.qkv_splits = w.forward_into(ln.normed, ln.qkv, flags, deferred(ln.idx, 0, need, required));
   const int64_t nq = n_heads_ * D, nkv = n_kv_heads_ * D;
   auto q = ln.qkv.narrow(1, 0, nq).view({n, n_heads_, D});
   auto k = ln.qkv.narrow(1, nq, nkv).view({n, n_kv_heads_, D});
@@ -390,26 +391,25 @@ void LlamaForCausalLMHip::post_attn(Lane& ln, size_t li) {
   {
     auto& w = L.o->packed();
     const int flags = (single ? SLM_W4_DEFER_REDUCE : 0) | chip_flag_;
-    const size_t need = w.workspace_bytes(n, flags);
-    const int splits = w.forward_into(a2, ln.o_buf, flags, single ? deferred(ln.idx, 0, need) : scratch(ln.idx, need));
+    const size_t need = w.workspace_bytes(n, flags), required = w.workspace_required(n, flags);
+    const int splits = w.forward_into(a2, ln.o_buf, flags, single ? deferred(ln.idx, 0, need, required) : scratch(ln.idx, need, required));
     reduce_add_norm(ln, 0, ln.o_buf, L.post_norm, splits, 0);
   }
   {
     auto& w = L.gate_up->packed();
     if (w.paired()) {
-      const size_t need = w.workspace_bytes(n, SLM_W4_SILU_MUL | chip_flag_);
-      w.forward_into(ln.normed, ln.act, SLM_W4_SILU_MUL | chip_flag_, scratch(ln.idx, need));
+      const int flags = SLM_W4_SILU_MUL | chip_flag_;
+      w.forward_into(ln.normed, ln.act, flags, scratch(ln.idx, w.workspace_bytes(n, flags), w.workspace_required(n, flags)));
     } else {
-      const size_t need = w.workspace_bytes(n, chip_flag_);
-      w.forward_into(ln.normed, ln.gate_up, chip_flag_, scratch(ln.idx, need));
+      w.forward_into(ln.normed, ln.gate_up, chip_flag_, scratch(ln.idx, w.workspace_bytes(n, chip_flag_), w.workspace_required(n, chip_flag_)));
       llm::kernel::silu_and_mul(ln.act, ln.gate_up);
     }
   }
   {
     auto& w = L.down->packed();
     const int flags = (single ? SLM_W4_DEFER_REDUCE : 0) | chip_flag_;
-    const size_t need = w.workspace_bytes(n, flags);
-    const int splits = w.forward_into(ln.act, ln.down_buf, flags, single ? deferred(ln.idx, 0, need) : scratch(ln.idx, need));
+    const size_t need = w.workspace_bytes(n, flags), required = w.workspace_required(n, flags);
+    const int splits = w.forward_into(ln.act, ln.down_buf, flags, single ? deferred(ln.idx, 0, need, required) : scratch(ln.idx, need, required));
     const auto& nxt = li + 1 < layers_.size() ? layers_[li + 1].input_norm : final_norm_;
     reduce_add_norm(ln, 1, ln.down_buf, nxt, splits, 0);
   }

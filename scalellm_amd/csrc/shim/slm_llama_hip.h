@@ -126,8 +126,10 @@ class LlamaForCausalLMHip {
   void plain_layer(Lane& ln, size_t li, std::vector<KVCache>& kv);
   void reduce_add_norm(Lane& ln, int which, torch::Tensor& partial, const torch::Tensor& weight, int splits, int slot);
   void run_two_lanes(Lane& l0, Lane& l1, std::vector<KVCache>& kv);
-  const torch::Tensor& scratch(int lane, size_t bytes);
-  const torch::Tensor& deferred(int lane, int slot, size_t bytes);
+  // (grown to `bytes`; where it may not or cannot grow and a call does without, required = 0: what there is)
+  const torch::Tensor& scratch(int lane, size_t bytes, size_t required = 1);
+  const torch::Tensor& deferred(int lane, int slot, size_t bytes, size_t required = 1);
+  const torch::Tensor& grown(torch::Tensor& t, size_t bytes, size_t required, const char* what);
 
   LlamaArgs args_;
   QuantArgs quant_args_;

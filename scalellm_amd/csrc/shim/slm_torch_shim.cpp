@@ -59,16 +59,21 @@ torch::Tensor workspace_for(const torch::Tensor& like, size_t bytes, size_t requ
   auto& ws = g_ws[dev];
   if (!ws.defined() || static_cast<size_t>(ws.nbytes()) < bytes) {
     const auto capturing = c10::hip::currentStreamCaptureStatusMayInitCtx();
-    if (capturing != c10::hip::CaptureStatus::None && required == 0) return {};
+    if (capturing != c10::hip::CaptureStatus::None && required == 0) return {};   // (the call does without)
     TORCH_CHECK(capturing == c10::hip::CaptureStatus::None,
                 "slm: the kernel workspace must be sized before graph capture (need ", bytes,
                 " bytes): warm the step up first or call paged_kv_varlen_mha_set_workspace()");
     size_t size = std::max<size_t>(bytes, 1 << 20);
-    if (ws.defined()) {
-      size = std::max<size_t>(size, 2 * static_cast<size_t>(ws.nbytes()));
-      g_retired.push_back(ws);
+    if (ws.defined()) size = std::max<size_t>(size, 2 * static_cast<size_t>(ws.nbytes()));
+    torch::Tensor grown;
+    try {
+      grown = torch::empty({static_cast<int64_t>(size)}, torch::dtype(torch::kUInt8).device(like.device()));
+    } catch (const c10::OutOfMemoryError&) {
+      if (required > 0) throw;
+      return {};
     }
-    ws = torch::empty({static_cast<int64_t>(size)}, torch::dtype(torch::kUInt8).device(like.device()));
+    if (ws.defined()) g_retired.push_back(ws);
+    ws = grown;
   }
   return ws;
 }
@@ -673,8 +678,8 @@ torch::Tensor W4Linear::forward(const torch::Tensor& input, const std::optional<
   if (g.M == 0) return c;
   const size_t need = slm_w4a16_gemm_workspace_bytes(&g);
   torch::Tensor ws;
-  if (need > 0) {
-    ws = workspace_for(a, need, need);
+  if (need > 0) ws = workspace_for(a, need, slm_w4a16_gemm_workspace_required(&g));
+  if (ws.defined()) {
     g.workspace = ws.mutable_data_ptr();
     g.workspace_bytes = ws.nbytes();
   }
@@ -697,7 +702,7 @@ slm_w4_gemm_args w4_args(const torch::Tensor& a, const void* wq, const void* sz,
 }
 }  // namespace
 
-size_t W4Linear::workspace_bytes(int64_t M, int flags) const {
+size_t W4Linear::scratch_bytes(int64_t M, int flags, bool required) const {
   flags |= order_;
   slm_w4_gemm_args g{};
   g.wq = wq_.const_data_ptr(); g.sz = sz_.const_data_ptr();
@@ -707,7 +712,7 @@ size_t W4Linear::workspace_bytes(int64_t M, int flags) const {
   g.dtype = dtype_ == torch::kBFloat16 ? SLM_BF16 : SLM_F16;
   g.flags = flags;
   if ((flags & SLM_W4_DEFER_REDUCE) && !slm_w4a16_gemm_deferred_splits(&g)) g.flags &= ~SLM_W4_DEFER_REDUCE;
-  return slm_w4a16_gemm_workspace_bytes(&g);
+  return required ? slm_w4a16_gemm_workspace_required(&g) : slm_w4a16_gemm_workspace_bytes(&g);
 }
 
 int W4Linear::forward_into(const torch::Tensor& a, torch::Tensor& c, int flags, const torch::Tensor& workspace) const {
@@ -726,10 +731,10 @@ int W4Linear::forward_into(const torch::Tensor& a, torch::Tensor& c, int flags, 
     deferred = slm_w4a16_gemm_deferred_splits(&g);
     if (!deferred) g.flags &= ~SLM_W4_DEFER_REDUCE;
   }
-  const size_t need = slm_w4a16_gemm_workspace_bytes(&g);
-  if (need > 0) {
-    TORCH_CHECK(workspace.defined() && static_cast<size_t>(workspace.nbytes()) >= need,
-                "W4Linear::forward_into: scratch of ", need, " bytes needed (reserve it before the step)");
+  const size_t required = slm_w4a16_gemm_workspace_required(&g);
+  TORCH_CHECK(required == 0 || (workspace.defined() && static_cast<size_t>(workspace.nbytes()) >= required),
+              "W4Linear::forward_into: scratch of ", required, " bytes needed (reserve it before the step)");
+  if (workspace.defined()) {
     g.workspace = workspace.mutable_data_ptr();
     g.workspace_bytes = workspace.nbytes();
   }

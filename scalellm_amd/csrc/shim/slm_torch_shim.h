@@ -161,14 +161,16 @@ class W4Linear {
   // or SLM_W4_SILU_MUL (paired weights: c is [M, N/2] = silu(gate) * up).  Returns the number of
   // fp32 slabs left in `workspace` (>= 2: c was NOT written) or 0 (c written as usual).
   int forward_into(const torch::Tensor& a, torch::Tensor& c, int flags, const torch::Tensor& workspace) const;
-  // scratch bytes forward_into needs for M rows with these flags (0 = none)
-  size_t workspace_bytes(int64_t M, int flags) const;
+  // scratch bytes forward_into makes use of for M rows with these flags (0 = none), and what of it it cannot do without
+  size_t workspace_bytes(int64_t M, int flags) const { return scratch_bytes(M, flags, false); }
+  size_t workspace_required(int64_t M, int flags) const { return scratch_bytes(M, flags, true); }
   bool paired() const { return paired_; }
 
   int64_t in_features() const { return k_src_; }
   int64_t out_features() const { return N_; }
 
  private:
+  size_t scratch_bytes(int64_t M, int flags, bool required) const;
   // a row-parallel shard of an act-order checkpoint: g_idx [K] sharded, scales / qzeros the FULL
   // tables (qlinear_gptq_marlin_impl.cpp:236-243) -> padded groups, packed K_ > k_src_
   void pack_uneven_groups(const torch::Tensor& qweight, const torch::Tensor& qzeros, const torch::Tensor& scales,

@@ -996,6 +996,12 @@ SLM_API size_t slm_w4a16_gemm_workspace_bytes(const slm_w4_gemm_args* a) {
   return pl.part_bytes + pl.aperm_bytes;
 }
 
+SLM_API size_t slm_w4a16_gemm_workspace_required(const slm_w4_gemm_args* a) {
+  GemmPlan pl;
+  if (plan_gemm(a, &pl) != SLM_OK) return 0;
+  return (pl.tiled ? 0 : pl.part_bytes) + pl.aperm_bytes;
+}
+
 SLM_API int32_t slm_w4a16_gemm_deferred_splits(const slm_w4_gemm_args* a) {
   GemmPlan pl;
   if (plan_gemm(a, &pl) != SLM_OK) return 0;

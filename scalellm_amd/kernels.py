@@ -143,10 +143,10 @@ def _grow(table, nbytes: int, dev: torch.device, what: str) -> torch.Tensor:
             raise SlmError(f"{what} must be reserved before graph capture "
                            f"(need {nbytes} bytes): call reserve_workspace() first")
         size = max(int(nbytes), 1 << 20, 2 * ws.numel() if ws is not None else 0)
+        new = torch.empty(size, dtype=torch.uint8, device=dev)
         if ws is not None:
             _retired.append(ws)  # never freed: earlier captures still point into it
-        ws = torch.empty(size, dtype=torch.uint8, device=dev)
-        table[key] = ws
+        ws = table[key] = new
     return ws
 
 
@@ -167,6 +167,16 @@ def _fits_or_grows(nbytes: int, dev: torch.device) -> bool:
     """Does the scratch hold nbytes, or may it be grown now?"""
     ws = _workspaces.get(_dev_key(dev))
     return (ws is not None and ws.numel() >= nbytes) or not torch.cuda.is_current_stream_capturing()
+
+
+def _wanted_workspace(nbytes: int, dev: torch.device) -> Optional[torch.Tensor]:
+    """The scratch, grown if need be; None where it may not (being captured) or cannot (out of memory) grow."""
+    if not _fits_or_grows(nbytes, dev):
+        return None
+    try:
+        return reserve_workspace(nbytes, dev)
+    except torch.OutOfMemoryError:
+        return None
 
 
 def retired_workspace_bytes() -> int:
@@ -728,6 +738,10 @@ def gptq_gemm(a: torch.Tensor, packed: PackedW4, c: torch.Tensor,
             g.flags = chip
     need = L.slm_w4a16_gemm_workspace_bytes(C.byref(g))
     ws = None
+    if need and not deferred and L.slm_w4a16_gemm_workspace_required(C.byref(g)) < need:
+        ws = _wanted_workspace(need, a.device)   # (or the call does without)
+        if ws is None:
+            need = L.slm_w4a16_gemm_workspace_required(C.byref(g))
     if need:
         # deferred slabs live in their own buffer: attention split-KV scratch, other split-K GEMMs
         # and act-order copies (which all use the shared workspace) can never overwrite them

@@ -471,6 +471,22 @@ def test_knobs_of_the_256_row_kernels_reach_calls_that_may_take_tiles():
             assert L.slm_tuning_clear(None) == 0
 
 
+def test_scratch_that_products_cannot_do_without():
+    """Four-wave tiles run without the scratch they are cut by; every other plan needs all that it asks for."""
+    L = _lib.lib()
+    assert L.slm_tuning_clear(None) == 0
+    g = W4GemmArgs()
+    g.K, g.N, g.lda, g.ldc, g.group_size, g.dtype = 4096, 4096, 4096, 4096, 128, 1
+    for g.M in (1, 8, 40, 100, 200, 400, 2648):
+        for g.flags in (0, _lib.SLM_W4_DEFER_REDUCE, _lib.SLM_W4_TILES):
+            want, required = L.slm_w4a16_gemm_workspace_bytes(C.byref(g)), L.slm_w4a16_gemm_workspace_required(C.byref(g))
+            assert required == (0 if g.flags == _lib.SLM_W4_TILES and g.M > 320 else want), (g.M, g.flags)
+    g.M, g.flags = 400, _lib.SLM_W4_TILES
+    assert L.slm_w4a16_gemm_workspace_bytes(C.byref(g)) > 0
+    g.perm = 4096   # (the permuted activations are no option)
+    assert L.slm_w4a16_gemm_workspace_required(C.byref(g)) == 400 * 4096 * 2
+
+
 def test_forced_tiles_leave_gemvs_alone():
     """SLM_W4_TILE asks for tiles that read their activations from memory; a one-row GEMV may get them from a norm prologue, so its plan
     is the same with the knob as without it."""

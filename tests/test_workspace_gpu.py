@@ -111,6 +111,50 @@ def test_growth_during_capture_is_refused():
     assert raised, "growing the workspace inside a capture must raise, not allocate"
 
 
+def _short_of_scratch(run):
+    """Runs with an empty table of scratch buffers (the old one is kept alive: earlier graphs point into it)."""
+    from scalellm_amd import kernels
+    kept = dict(kernels._workspaces)
+    kernels._workspaces.clear()
+    try:
+        return run()
+    finally:
+        kernels._workspaces.clear()
+        kernels._workspaces.update(kept)
+
+
+@pytest.mark.parametrize("why", ["captured", "full"])
+def test_products_of_many_rows_do_without_scratch(why, monkeypatch):
+    """Tiles that would be cut in K by scratch that is not there are not cut: while a graph is captured, and on a card that is full."""
+    from scalellm_amd import kernels
+    M, K, N = 400, 2048, 1024
+    case = helpers.make_quant_case(78, K, N, 128, "awq", "bf16")
+    packed = helpers.pack_case(case, "bf16", DEV)
+    x = torch.randn(M, K, device=DEV, dtype=torch.bfloat16)
+    want, c = (torch.empty(M, N, device=DEV, dtype=torch.bfloat16) for _ in range(2))
+    kernels.gptq_gemm(x, packed, want)
+    torch.cuda.synchronize()
+
+    def captured():
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            kernels.gptq_gemm(x, packed, c)
+        for _ in range(3):
+            c.zero_()
+            g.replay()
+            torch.cuda.synchronize()
+
+    def full():
+        def none(*_):
+            raise torch.OutOfMemoryError("full")
+        monkeypatch.setattr(kernels, "reserve_workspace", none)
+        kernels.gptq_gemm(x, packed, c)
+        torch.cuda.synchronize()
+    _short_of_scratch(captured if why == "captured" else full)
+    # (the same fp32 sums in another order: single roundings to bf16, 2^-8 of a value, of a share of the values)
+    assert (c.double() - want.double()).norm() < 2e-3 * want.double().norm()
+
+
 def test_deferred_partials_are_isolated_and_versioned():
     """the slabs a deferred split-K GEMM leaves behind must survive any other
     workspace user running between producer and consumer; a handle overwritten by a later deferred
