@@ -307,9 +307,10 @@ typedef struct slm_w4_gemm_args {
  * queries (they describe the plan the call will take). */
 #define SLM_W4_SHARES_CHIP 4
 /* flags: sums may come in another order than without the flag, which lets bf16 products of many rows take faster tiles.  Each result is as near to the
- * exact one as before, but a few round the other way; where weights have a mean -- GPTQ's zero points, one above the stored ones, give them a
- * seventh of their spread -- outputs have a large part in common and layers behind them turn single roundings into a third of the outputs'
- * spread, so the mirror in Python sets it for AWQ weights only. */
+ * exact one as before, but a few round the other way.  Where weights have a mean in common, so have outputs, and layers behind them turn those
+ * roundings into more: four layers of weights with a mean of a seventh of their spread gave logits that differ by a third of their root mean square
+ * at one place (nibbles and stored zero points drawn alike; a checkpoint's zero points follow its weights, and its weights' mean is small).  The mirrors set
+ * it for AWQ weights, as measured; GPTQ weights keep the order they had. */
 #define SLM_W4_TILES 8
 
 SLM_API size_t slm_w4a16_gemm_workspace_bytes(const slm_w4_gemm_args* a);

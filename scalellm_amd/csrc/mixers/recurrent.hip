@@ -13,7 +13,7 @@
 //            in registers from the portion's first token to its last; the products are 32-bit MFMAs.  Bound: a chain of two products and an
 //            exchange a chunk, 0.7 us, and the instructions around them.
 //   Both, us, 16 heads of 128 x 128 and 4096 tokens: delta 305 with the triangular system and B U in the scan, 64-bit addresses and a wave's
-//   read-outs by itself, 257 now; lightning 184 and 159; 8 x 500 tokens, 32 heads: 341 and 304, 209 and 186; 16 heads of 64, 2000 tokens: 120 and 85.
+//   read-outs by itself, 262 now; lightning 184 and 163; 8 x 500 tokens, 32 heads: 341 and 309, 209 and 188; 16 heads of 64, 2000 tokens: 120 and 86.
 //   gated_norm  the norm and gate behind a scan.
 #include "latent/latent_common.h"
 #include "slm_mixers.h"

@@ -433,7 +433,7 @@ class PackedW4:
         # paired: a merged [gate | up] weight whose packed column tiles alternate gate / up
         # (SLM_W4_PAIRED) -- the form gptq_gemm(..., silu_mul=True) needs
         self.paired = paired
-        # any_order: products' sums may come in another order (SLM_W4_TILES; include/slm_hip.h says why not everywhere)
+        # any_order: products' sums may come in another order (SLM_W4_TILES; include/slm_hip.h says what that can do)
         self.any_order = any_order
 
 
