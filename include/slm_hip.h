@@ -5,7 +5,7 @@
  * Drop-in boundary: every entry point below replaces one C++ kernel-level
  * symbol of the reference (vectorch-ai/ScaleLLM, paths relative to the
  * reference root).  The reference passes torch::Tensor; a thin libtorch shim
- * (scalellm_amd/csrc/shim/, see INTEGRATION.md) adapts tensor -> (pointer,
+ * (scalellm_amd/csrc/shim/) adapts tensor -> (pointer,
  * strides, sizes) and calls these functions, so the reference src/layers tree compiles
  * unchanged.
  *
@@ -123,7 +123,7 @@ typedef struct slm_attn_args {
                              * correct whatever the value (a wrong "uniform" claim costs balance, not bits) */
   int32_t phase;            /* 0 = the whole call (default).  A call that splits the KV range runs as stream
                              * kernel(s) + a combine pass; a host that overlaps calls on two streams (the two
-                             * decode lanes, DESIGN.md 3.6) may issue the halves separately: 1 = everything BUT
+                             * decode lanes) may issue the halves separately: 1 = everything BUT
                              * the combine pass, 2 = the combine pass only (a no-op when the plan needs none).
                              * Same arguments for both; phase 1 then phase 2 on one stream == phase 0. */
   int32_t reserved;
@@ -176,7 +176,7 @@ SLM_API int slm_set_kv_cache(const int32_t* slot_ids,  /* [n_tokens]           *
 /*      AWQ : qweight [K, N/8] int32, qzeros [G, N/8] int32, both with the    */
 /*            [0,2,4,6,1,3,5,7] nibble interleave, zero = stored;             */
 /*            scales  [G, N] T.                                               */
-/*    Output layout (owned by this library):                   */
+/*    Output layout (owned by this library):                                  */
 /*      wq  [K/64][N/32][64 lanes][4] uint32  -- lane l, word j holds the 8   */
 /*           nibbles n = 32*nt + (l&31), k = 64*kt + 16*j + 8*(l>>5) + p'     */
 /*           in a pair-interleaved nibble order (MFMA 32x32x16 B-fragment);   */
@@ -299,7 +299,7 @@ typedef struct slm_w4_gemm_args {
  * packed column order.  Needs N % 64 == 0; cannot be combined with SLM_W4_DEFER_REDUCE. */
 #define SLM_W4_SILU_MUL 2
 /* flags: the call SHARES THE CHIP with kernels of another stream that must keep running next to it (the two
- * half-batch decode lanes of DESIGN.md 3.6: one lane's GEMMs run under the other lane's attention stream).  A
+ * half-batch decode lanes: one lane's GEMMs run under the other lane's attention stream).  A
  * scheduling hint: the plan then avoids launch shapes whose workgroups cannot sit on a CU beside other waves --
  * the two-row-tile K-sliced stream for 33 <= M <= 64 (512 threads x 236 VGPRs: alone it is the faster kernel,
  * 89 vs 96 us per Llama-3-8B layer; beside an attention stream its workgroups wait for whole CUs, 14.2 -> 21.5 ms
@@ -353,7 +353,7 @@ SLM_API int slm_w4_dequant(const void* wq, const void* sz, int64_t K, int64_t N,
                            int64_t group_size, int32_t dtype, void* w_out, void* stream);
 
 /* ========================================================================== */
-/* 5. Glue ops of one decoder layer (SURVEY 8f "next" rows f1/f2).            */
+/* 5. Glue ops of one decoder layer.                                          */
 /*    replaces  kernel::apply_rotary_pos_emb  src/kernels/pos_embedding_      */
 /*              kernels.cu:35-121; kernel::rms_norm / rms_norm_residual       */
 /*              src/kernels/layernorm_kernels.cu:15,125;                      */
@@ -426,7 +426,7 @@ SLM_API int slm_rope_kv_append_splitk(const float* partials /* [n_splits, T, N] 
 SLM_API int slm_silu_mul(void* out /* [T, d] */, const void* x /* [T, 2d]: gate | up */,
                          int64_t n_tokens, int64_t d, int32_t dtype, void* stream);
 
-/* ---- device-side input advance for the next decode step (SURVEY 8f row f4) ----------------------
+/* ---- device-side input advance for the next decode step ----------------------
  * Replaces, for a steady decode batch (q_len = 1 per sequence), the per-step host rebuild + H2D
  * copies of Batch::prepare_model_input (engine/batch.cpp:97-255, model_runner.cpp:194-203):
  * updates the graph's static input buffers IN PLACE on the device so a captured step can be
@@ -473,7 +473,7 @@ SLM_API int slm_build_step_inputs(const int32_t* q_lens /* [n_seqs] */, int32_t*
                                   int32_t* overflow_flag /* [1], may be NULL */, void* stream);
 
 /* ========================================================================== */
-/* 6. xGMI all-reduce fused with residual-add + RMSNorm    */
+/* 6. xGMI all-reduce fused with residual-add + RMSNorm                       */
 /*    replaces  ProcessGroupNCCL::allreduce  (ncclAllReduce SUM, in place)    */
 /*              src/model_parallel/process_group.cpp:135-153                  */
 /*    callers   reduce_from_model_parallel_region, model_parallel.cpp:33-44,  */
@@ -552,7 +552,7 @@ SLM_API int slm_allreduce_simulate(const slm_ar_args* ranks, int32_t world, void
 /* 7. Host policy: one lane or two for a pure-decode step (round 5)           */
 /*    no reference counterpart -- the two half-batch lanes are this build's   */
 /*    own schedule of the decoder stack (models/meta/llama.h:123-345 is one   */
-/*    serial chain per step); DESIGN.md 3.6.  Pure host code, no device work: */
+/*    serial chain per step).  Pure host code, no device work:                */
 /*    ONE source of the rule for the Python mirror (decode.two_lane_split)    */
 /*    and the C++ host step (slm::LlamaForCausalLMHip::lane_split).           */
 /*    The rule: (a) hard conditions -- lanes_min != 0, a pure-decode batch in */

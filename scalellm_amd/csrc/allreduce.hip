@@ -1,5 +1,5 @@
 // allreduce.hip -- two-shot all-reduce over peer-mapped (xGMI) buffers, fused with the residual add
-// and RMSNorm that follow every row-parallel linear of a decoder layer (SURVEY 8f row f3).
+// and RMSNorm that follow every row-parallel linear of a decoder layer.
 //
 // Replaces ProcessGroupNCCL::allreduce (reference src/model_parallel/process_group.cpp:135-153, as
 // called by reduce_from_model_parallel_region, model_parallel.cpp:33-44) + kernel::rms_norm_residual

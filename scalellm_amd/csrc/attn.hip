@@ -2,7 +2,7 @@
 //
 // Replaces llm::paged_kv_varlen_mha (reference src/kernels/attention/attn_api.cpp:14-73,
 // kernel src/kernels/attention/kernel/sm80_kernel_mha.cuh:174-335).  Designed from the
-// byte stream, not from the reference's 64x64 MMA tile (SURVEY 0.3):
+// byte stream, not from the reference's 64x64 MMA tile:
 //
 //  * token-major work items: one workgroup = (query token, group of KV heads, q-head chunk,
 //    KV split).  Decode (q_len = 1), speculative verify (q_len = k+1) and prefill chunks are
@@ -15,8 +15,8 @@
 //  * every lane group owns its (kv head, row phase): it keeps running (m, l, O[GC][8]) in
 //    registers for the GC query heads that share the kv head -- no cross-lane traffic in the
 //    loop except the LPR-lane DPP reduction of the q.k partial sums, no LDS on the data path
-//    (K/V are streamed once; nothing is reused across waves -- see DESIGN.md for why LDS
-//    staging is not used on the decode stream).
+//    (K/V are streamed once; nothing is reused across waves, so LDS staging would add a trip
+//    and save none).
 //  * block table slice staged in LDS once per workgroup (one coalesced read), slot =
 //    tbl[row >> log2(bs)] + (row & (bs-1)) -- bit-exact with sm80_kernel_mha.cuh:146-152.
 //  * U-deep register ring of 16-B K/V loads per lane keeps >= 2*U KiB per wave in flight.

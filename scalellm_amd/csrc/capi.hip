@@ -148,7 +148,7 @@ SLM_API int32_t slm_decode_lane_split(const slm_lane_query* q) {
     std::lock_guard<std::mutex> lk(g_lane_mu);
     if (const LaneEntry* e = lane_lookup(q)) return e->two_us < 0.985f * e->one_us ? half : 0;
   }
-  // ... else the constants (DESIGN.md 3.6; profiles/r04_lanes_sweep_w2.jsonl): 96 <= T <= 256, long
+  // ... else the constants (profiles/r04_lanes_sweep_w2.jsonl): 96 <= T <= 256, long
   // sequences (>= 12 MiB of K + V each), the KV stream >= 8 x the layer's weights
   const int64_t eb = q->kv_elem_bytes > 0 ? q->kv_elem_bytes : 2;
   const int64_t kv_seq = 2 * eb * q->n_kv_heads * q->head_dim * (int64_t)q->kv_max_seq_len;

@@ -1,5 +1,4 @@
-// glue.hip -- the small memory-bound ops either side of the hot path inside one decoder layer
-// (SURVEY 8f rows f1/f2), hand-written for gfx950: 16-byte vector accesses, wave64 reductions.
+// glue.hip -- the small memory-bound ops either side of the hot path inside one decoder layer, hand-written for gfx950: 16-byte vector accesses, wave64 reductions.
 //
 //  slm_rms_norm        <- kernel::rms_norm / rms_norm_residual  (reference
 //                         src/kernels/layernorm_kernels.cu:15,125; math src/layers/normalization.h

@@ -40,7 +40,7 @@ __global__ void __launch_bounds__(256) set_kv_cache_kernel(
   }
 }
 
-// decode-step input advance (SURVEY 8f f4): every thread touches only its own elements, so the
+// decode-step input advance: every thread touches only its own elements, so the
 // update is race-free in place
 __global__ void __launch_bounds__(256) decode_advance_kernel(
     int32_t* __restrict__ positions, int32_t* __restrict__ kv_cu_lens,
@@ -64,7 +64,7 @@ __global__ void __launch_bounds__(256) decode_advance_kernel(
   kv_cu_lens[b] += b;  // b = 0 .. n_seqs: every sequence before this offset grew by one token
 }
 
-// Step-input build for ANY batch shape (SURVEY 8f f4, beyond steady decode): prefix sums of the
+// Step-input build for ANY batch shape (beyond steady decode): prefix sums of the
 // per-sequence lengths, then positions and cache slots of every new token.  ONE workgroup: a step
 // has at most a few thousand sequences and tokens, the work is two scans and a fill (microseconds),
 // and a single workgroup needs no cross-workgroup ordering between the scan and the fill.

@@ -1,5 +1,5 @@
 // slm_attn_handler_hip.h -- the attention-handler layer of the reference over the HIP kernels,
-// compiled C++ (SURVEY 8 row a7).
+// compiled C++.
 //
 // Mirrors, member for member, what src/layers/attention/{handler.h, scale_attn_handler.{h,cpp},
 // attention.{h,cpp}} expose to the model code: AttentionHandler (the virtual interface,

@@ -18,7 +18,7 @@
 // boost, which this image does not have, so the few members these classes touch are mirrored
 // below under the SAME names and signatures (state_dict.h:28-40, parallel_args.h, quant_args.h);
 // inside a ScaleLLM tree the four `slm::` types are replaced by `using llm::...` and
-// ParallelLinearImpl by the reference's (INTEGRATION.md section 3) -- the class bodies compile
+// ParallelLinearImpl by the reference's -- the class bodies compile
 // unchanged.
 #pragma once
 #include <torch/torch.h>

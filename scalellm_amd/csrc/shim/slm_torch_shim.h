@@ -1,7 +1,7 @@
 // slm_torch_shim.h -- libtorch adapter: the reference's C++ operator signatures on top of the
 // C-ABI HIP kernel library (include/slm_hip.h).  A ScaleLLM build links this instead of
 // src/kernels/attention, src/kernels/kv_cache_kernels.cu, src/kernels/pos_embedding_kernels.cu and
-// src/kernels/quantization/marlin; src/layers/** then compiles unchanged (INTEGRATION.md).
+// src/kernels/quantization/marlin; src/layers/** then compiles unchanged.
 //
 // Signatures below are the reference's, verbatim in types / order / meaning:
 //   llm::paged_kv_varlen_mha           src/kernels/attention/attn_api.h:12-27
@@ -9,7 +9,7 @@
 //   llm::kernel::apply_rotary_pos_emb  src/kernels/pos_embedding_kernels.h
 // The int4 path is offered at the layer boundary the survey recommends (ParallelLinearImpl,
 // src/layers/linear/parallel_linear.h:17-37): slm::W4Linear owns the MFMA-native packed layout
-// and is what a QLinearHipImpl subclass wraps (INTEGRATION.md shows the 40-line subclass).
+// and is what a QLinearHipImpl subclass wraps (40 lines: slm_qlinear_hip.h).
 // slm::ProcessGroupRCCL implements llm::ProcessGroup's contract (process_group.h:10-60) on RCCL.
 #pragma once
 #include <torch/torch.h>
@@ -258,7 +258,7 @@ class LocalShardProcessGroup : public ProcessGroup {
 
 // The two row-parallel reductions of a decoder layer as ONE launch per rank each: two-shot
 // all-reduce over peer-mapped buffers fused with the residual add + RMSNorm that follows
-// (slm_allreduce, include/slm_hip.h section 6; SURVEY 8f f3).  Replaces, at the call sites of
+// (slm_allreduce, include/slm_hip.h section 6).  Replaces, at the call sites of
 // reduce_from_model_parallel_region (model_parallel.cpp:33-44) in the row-parallel linears, the
 // pair ProcessGroup::allreduce (process_group.cpp:135-153) + kernel::rms_norm_residual
 // (layernorm_kernels.cu:125).  Thread-per-GPU shape, like create_process_groups: create() is

@@ -34,7 +34,6 @@
 //    M > 128, >= 112 tiles of 256x128 w4_ws.hip     producer / consumer waves, LDS-DMA activations
 //    prefill-sized M x N             w4_xl.hip     symmetric 256 x 256 tiles
 //    the same in bf16                w4_tile.hip   four waves a tile (SLM_W4_TILES)
-// (DESIGN.md 3.3 has the measurements behind each boundary.)
 #include "tile_common.h"
 #include "w4_common.h"
 #include "tuning.h"

@@ -3,7 +3,7 @@
 // Same operator as w4.hip (replaces marlin::gptq_gemm, reference gptq_gemm.cu:585-710), same packed
 // layout (w4.hip header), same bit-faithful dequant (W4Dq<T>, marlin/numeric_conversion.h:19-62).
 //
-// Why 256 x 256: the measured global -> LDS rate of a CU (~23 B/clk, DESIGN.md 3.3) is what bounds
+// Why 256 x 256: the measured global -> LDS rate of a CU (~23 B/clk) is what bounds
 // the 256 x 128 wave-specialised kernel (36 B/clk of A + W needed to run the matrix pipe flat out);
 // a 256 x 256 tile needs 20 B/clk.  256 accumulator tiles do not fit a producer/consumer split, so
 // all eight waves are symmetric: wave (mh, nq) owns the 128 x 64 block (4 m-tiles x 2 n-tiles =

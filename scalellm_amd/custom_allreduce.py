@@ -1,4 +1,4 @@
-"""Host side of the xGMI all-reduce fused with residual-add + RMSNorm (SURVEY 8f row f3).
+"""Host side of the xGMI all-reduce fused with residual-add + RMSNorm.
 
 Replaces, for the decode-size messages of the row-parallel linears, the pair
     ProcessGroupNCCL::allreduce            src/model_parallel/process_group.cpp:135-153

@@ -4,7 +4,7 @@ drive the hot path the way the reference's LlamaModelImpl::forward does (src/mod
 :123-265): per layer RMSNorm -> qkv -> RoPE+append -> paged attention -> o_proj (row-parallel,
 all-reduce) -> RMSNorm -> gate_up -> SiLU*mul -> down (row-parallel, all-reduce); then final norm,
 lm_head (column-parallel, gathered) and greedy argmax.  All four linears are int4 (AWQ or GPTQ)
--- the reference snapshot leaves fused qkv / gate_up un-quantised (SURVEY 0.5); here the whole
+-- the reference snapshot leaves fused qkv / gate_up un-quantised; here the whole
 layer is int4.  Weights are synthetic (seeded); there is no checkpoint IO on this path.
 
 One process per GPU; TP shards heads (attention needs no collective) and the GEMMs' N / K.
@@ -175,7 +175,7 @@ class LlamaDecodeStep:
         # parity test can rebuild the same model from them on the CPU oracle
         self.ckpt = [] if keep_checkpoint else None
         # optional custom_allreduce.XgmiAllReduce: the two row-parallel reductions of a layer then
-        # run as ONE launch each, fused with the residual add + RMSNorm that follows (SURVEY 8f f3)
+        # run as ONE launch each, fused with the residual add + RMSNorm that follows
         # Round 5: a PAIR (lane 0, lane 1) lets a tensor-parallel rank run two lanes: every lane owns a whole
         # instance of the protocol (signal block + two alternating message buffers), so the lanes'
         # reductions -- on two streams, in the same order on every rank -- never share a flag or a buffer
@@ -811,8 +811,8 @@ def make_batch_inputs(q_lens, kv_lens, block_size: int, device, seed: int = 0, v
     brings q_lens[i] new tokens (1 = decode, k + 1 = speculative verify, a chunk = chunked prefill)
     on top of kv_lens[i] - q_lens[i] tokens of history (kv_lens INCLUDE the new tokens, as
     kv_cu_seq_lens does); blocks are a seeded random permutation (unique first-slot ids, block 0
-    unused).  What BASELINE configs[4] batches look like, and the ragged decode batch of SURVEY
-    8(d) config 2 (q_lens all 1, kv_lens ~ U[2048, 4096])."""
+    unused).  Steps that mix chunked prompts, verification and decoding look so, and ragged decode
+    batches (q_lens all 1, kv_lens ~ U[2048, 4096])."""
     import numpy as np
     q_lens = [int(x) for x in q_lens]
     kv_lens = [int(x) for x in kv_lens]

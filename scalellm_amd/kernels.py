@@ -9,7 +9,7 @@ library libslm_hip.so (include/slm_hip.h) on torch's CURRENT stream:
   awq_repack / gptq_repack / gptq_gemm
                        <- marlin::awq_repack / gptq_repack / gptq_gemm
                                                         src/kernels/quantization/marlin.h:17-37
-  rms_norm / apply_rotary_pos_emb(+append) / silu_and_mul   
+  rms_norm / apply_rotary_pos_emb(+append) / silu_and_mul
 
 PyTorch is plumbing here (device memory, streams); every op is a HIP kernel of ours.
 There is NO fallback: a missing library or a non-GPU tensor raises.
@@ -361,7 +361,7 @@ def set_kv_cache(slot_ids: torch.Tensor, keys: torch.Tensor, values: torch.Tenso
 def decode_advance(positions: torch.Tensor, kv_cu_lens: torch.Tensor, new_cache_slots: torch.Tensor,
                    block_table: torch.Tensor, block_cu_lens: torch.Tensor, block_size: int,
                    overflow_flag: torch.Tensor | None = None) -> None:
-    """Device-side input build for the next decode step (SURVEY 8f f4): in-place update of the
+    """Device-side input build for the next decode step: in-place update of the
     graph's static int32 inputs, replacing the per-step host rebuild + H2D copies of
     Batch::prepare_model_input (engine/batch.cpp:97-255, model_runner.cpp:194-203) for a steady
     decode batch.  Slot arithmetic = Sequence::kv_cache_slots (request/sequence.cpp:303-317)."""
@@ -386,7 +386,7 @@ def build_step_inputs(q_lens: torch.Tensor, kv_cached: torch.Tensor, block_table
                       block_cu_lens: torch.Tensor, block_size: int, positions: torch.Tensor,
                       q_cu_lens: torch.Tensor, kv_cu_lens: torch.Tensor, new_cache_slots: torch.Tensor,
                       commit: bool = True, overflow_flag: torch.Tensor | None = None) -> None:
-    """Device-side input build for ANY batch (SURVEY 8f f4 beyond steady decode): q_cu_seq_lens,
+    """Device-side input build for ANY batch (beyond steady decode): q_cu_seq_lens,
     kv_cu_seq_lens, positions and new_cache_slots of a step from the per-sequence (new tokens,
     tokens cached) arrays and the persistent block table -- the integer work of
     Batch::prepare_model_input (engine/batch.cpp:97-255) without its per-token host loops and

@@ -5,7 +5,7 @@ Mirror of the reference's src/model_parallel:
   ParallelArgs          <- llm::ParallelArgs          parallel_args.h
   gather/reduce/scatter_*_model_parallel_region       model_parallel.cpp:13-65
 
-MI355X-first difference (DESIGN.md "multi-GPU"): the reference drives N GPUs from N THREADS of
+MI355X-first difference: the reference drives N GPUs from N THREADS of
 one process through raw NCCL (ncclCommInitAll, process_group.cpp:98-123) because torch's
 ProcessGroupNCCL is multi-process only.  Here the unit is one PROCESS per GPU (torchrun), the
 communicator is torch.distributed with backend "nccl" (= RCCL on ROCm) over xGMI, and the

@@ -22,8 +22,8 @@ One extension over the reference (round 5): a model may
 (`graph_variants` / `graph_variant_for` / `graph_variant`, see LlamaDecodeStep).  A captured graph
 freezes the step's host-side decisions at the capture-time hints, but two of them belong to the batch
 that is replayed: one half-batch lane or two (the policy wants the batch's REAL context length, not
-`cuda_graph_max_seq_len`) and the uniform-batch hint `kv_total_len` (who fills it: INTEGRATION.md
-"kv_total_len").  With variants the runner captures one graph per (lanes, uniform) combination of a
+`cuda_graph_max_seq_len`) and the uniform-batch hint `kv_total_len` (which
+whoever builds the batch fills).  With variants the runner captures one graph per (lanes, uniform) combination of a
 batch size -- same static buffers, one shared graph memory pool -- and picks at replay from the
 batch's own hints; a model without the three methods gets exactly the reference's one graph.
 """
