@@ -256,7 +256,7 @@ def _gemm(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, glu=None, tile: i
     """out = x w^T, or with glu = (limit, alpha, shift) the clamped GLU of its halves, by the tile kernel for many rows.  False:
     shapes and strides that it does not take."""
     M, N, K = x.size(0), w.size(0), w.size(1)
-    if (x.dtype != torch.bfloat16 or K % 64 or N % (32 if glu else 16) or x.stride(0) < K or (x.stride(0) | w.stride(0) | out.stride(0)) % 8 or
+    if (x.dtype != torch.bfloat16 or not N or not K or K % 64 or N % (32 if glu else 16) or x.stride(0) < K or (x.stride(0) | w.stride(0) | out.stride(0)) % 8 or
             (x.data_ptr() | w.data_ptr() | out.data_ptr()) % 16 or max(M * x.stride(0), N * w.stride(0)) > 1 << 30 or max(M, N) > 1 << 24):
         return False
     a = _linear_args(x, w, M, N, K)

@@ -108,6 +108,14 @@ def test_linear_epilogues(M, N, K, dtype):
         _close(out, ref.clamped_glu(want[:, :N // 2], want[:, N // 2:], 0.6), dtype, f32=1e-5, b16=2e-2)
 
 
+@pytest.mark.parametrize("N,K", [(0, 128), (48, 0)])
+def test_products_of_many_rows_of_nothing(N, K):
+    lk = _lk()
+    for M in (100, 200):
+        y = lk.linear(torch.ones(M, K, dtype=torch.bfloat16, device=DEV), torch.ones(N, K, dtype=torch.bfloat16, device=DEV))
+        assert y.shape == (M, N) and not y.any()
+
+
 # row counts at the edges of every tile, columns that fill no panel of 64 and those that decide between tile widths, step
 # counts below and at a ring and a split.  fp32 sums of exact products of bf16: 1e-5 of the largest as above.
 @pytest.mark.parametrize("M", [1, 2, 16, 17, 32, 33, 64, 65, 127, 128, 140])
