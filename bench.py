@@ -1,5 +1,5 @@
 #!/usr/bin/env python3
-"""bench.py -- decode hot-path benchmark (driver contract: see the task statement / DESIGN.md).
+"""bench.py -- decode hot-path benchmark (one JSON line on standard output).
 
   python bench.py --gpus 1 --steps K --warmup W
   python -m torch.distributed.run --nnodes=1 --nproc-per-node N --master-addr 127.0.0.1 \
@@ -56,7 +56,7 @@ def _rccl_version():
 
 
 def attn_algo_bytes(bs, kv_len, n_heads, n_kv_heads, head_dim, block, q_len=1, esize=2):
-    """SURVEY 8d: K+V once, Q+O once, int32 indices once.  `kv_len`: one length for a uniform batch or
+    """K+V once, Q+O once, int32 indices once.  `kv_len`: one length for a uniform batch or
     the list of per-sequence lengths (ragged batch)."""
     lens = [int(kv_len)] * bs if isinstance(kv_len, int) else [int(x) for x in kv_len]
     assert len(lens) == bs
@@ -67,7 +67,7 @@ def attn_algo_bytes(bs, kv_len, n_heads, n_kv_heads, head_dim, block, q_len=1, e
 
 
 def step_algo_bytes(model, bs, kv_lens, block):
-    """Algorithmic HBM bytes of ONE decode step of this rank's shard (SURVEY 8d, summed): per layer the
+    """Algorithmic HBM bytes of ONE decode step of this rank's shard (summed): per layer the
     paged-attention bytes of the whole batch + the four int4 linears (packed weights + scale/zero words +
     activations in and out), plus the lm_head weight (read once per step) and the embedding rows."""
     s = model.shape
@@ -292,7 +292,7 @@ def cpu_baseline(model, tokens, params, sample_seqs, kv_len, block):
     # int4 linears: fresh random AWQ-format tensors of the layer's four shapes (host side), at the
     # batch's REAL row count: the reference dequantises every weight once per forward
     # (qlinear_impl.cpp:171-183) whatever the batch, so that cost -- and MKL's efficiency -- must be
-    # measured at M = batch, not on a 16-row sample scaled up (round-3 review, weak 8)
+    # measured at M = batch, not on a 16-row sample scaled up
     M = int(tokens.numel())
     rng = np.random.default_rng(0)
     shapes = [(s.hidden, (s.n_heads + 2 * s.n_kv_heads) * s.head_dim), (s.n_heads * s.head_dim, s.hidden),
@@ -414,7 +414,7 @@ def _probe_xgmi_main():
         # The launch must also survive capture + replay, and in the SEQUENCE the timed step runs:
         # the row-parallel int4 GEMM writes this rank's partial sums into the message buffer with PLAIN
         # stores, and the very next graph node is the fused reduce whose peers read that buffer over
-        # the fabric (DESIGN 3.5: the kernel boundary writes the producer's L2 back; the peers' loads
+        # the fabric (the kernel boundary writes the producer's L2 back; the peers' loads
         # are sc0 sc1 and miss every cache).  A fill_() here would test a different producer.
         from scalellm_amd import kernels as K
         from scalellm_amd.decode import _rand_int4_linear
@@ -500,11 +500,11 @@ def main():
     ap.add_argument("--steps", type=int, default=10)
     ap.add_argument("--warmup", type=int, default=3)
     ap.add_argument("--bits", type=int, default=4, choices=[4, 8], help="weight bits of the quantised linears "
-                    "(8 = the reference's num_bits = 8 path: two int4 planes on the int4 kernels; not the BASELINE metric)")
+                    "(8 = the reference's num_bits = 8 path: two int4 planes on the int4 kernels; not the headline metric)")
     ap.add_argument("--model", default="8b", choices=["8b", "70b", "dagupel", "vebusun"], help="8b = Llama-3-8B-shaped, "
-                    "AWQ int4 g128, bs=256 (BASELINE.json metric configuration, configs[1]/[2]); 70b = "
+                    "AWQ int4 g128, bs=256 (the headline workload); 70b = "
                     "Llama-3-70B-shaped (in-tree defaults models/meta/llama.h:348-362), GPTQ symmetric "
-                    "int4 g128, bs=128, TP = --gpus (configs[3]; TP=1 fits one MI355X: 35 GB of weights "
+                    "int4 g128, bs=128, TP = --gpus (TP=1 fits one MI355X: 35 GB of weights "
                     "+ 172 GB of KV); dagupel = prefill / decode lines of the latent-attention design beside the Llama step "
                     "(options of its own: tools/bench_dagupel.py); vebusun = the same for the delta-rule / parallel-mixer "
                     "design (tools/bench_vebusun.py)")
@@ -512,7 +512,7 @@ def main():
     ap.add_argument("--seqlen", type=int, default=4096)
     ap.add_argument("--block", type=int, default=16)
     ap.add_argument("--layers", type=int, default=0, help="override layer count (debug only: "
-                    "a reduced model is NOT the BASELINE config and is flagged in the output)")
+                    "a reduced model is NOT the headline workload and is flagged in the output)")
     ap.add_argument("--quant", default="", choices=["", "awq", "gptq"], help="default awq (8b) / "
                     "gptq with symmetric zero points (70b)")
     ap.add_argument("--no-graph", action="store_true")
@@ -523,18 +523,18 @@ def main():
                     help="consistent: every rank draws the full-head history and keeps its shard, so "
                     "TP=N and TP=1 decode the same model state (tests compare their tokens)")
     ap.add_argument("--advance", action="store_true", help="include the device-side input build "
-                    "(slm_decode_advance, SURVEY 8f f4) in the step: every replay appends one token "
+                    "(slm_decode_advance) in the step: every replay appends one token "
                     "per sequence, so kv_len grows by one per step from --seqlen")
     ap.add_argument("--lanes", type=int, default=-1, help="two half-batch lanes on two streams for pure-decode "
                     "batches of >= N tokens (0 = never; default: SLM_DECODE_LANES or the library's auto policy)")
     ap.add_argument("--host", default="auto", choices=["auto", "py", "cpp"], help="who composes the step: the "
-                    "compiled C++ host step (csrc/shim/slm_llama_hip.cpp through _slm_shim.so; north_star: 'host code "
+                    "compiled C++ host step (csrc/shim/slm_llama_hip.cpp through _slm_shim.so: 'host code "
                     "stays C++') or the Python mirror (decode.LlamaDecodeStep over ctypes); same kernels, same launch "
                     "sequence.  auto (default): C++ on a single GPU with 4-bit weights -- the Python mirror's time is "
                     "printed beside it as config.python_mirror_ms --, the mirror otherwise (TP ranks, --simulate-tp, "
                     "8-bit weights: what the C++ step's bench plumbing does not cover)")
-    ap.add_argument("--ragged", action="store_true", help="serving-shaped batch (SURVEY 8(d) config 2): "
-                    "kv_len ~ U[seqlen/2, seqlen] per sequence (numpy default_rng(1)); not the BASELINE metric line")
+    ap.add_argument("--ragged", action="store_true", help="serving-shaped batch: "
+                    "kv_len ~ U[seqlen/2, seqlen] per sequence (numpy default_rng(1)); not the headline metric line")
     ap.add_argument("--simulate-tp", type=int, default=0, help="tuning aid: run rank 0's shard of a "
                     "TP=N step on one GPU with the collectives stubbed (flagged in the output)")
     args = ap.parse_args()
@@ -561,7 +561,7 @@ def main():
 
     shape = LlamaShape.llama3_70b() if args.model == "70b" else LlamaShape.llama3_8b()
     quant = args.quant or ("gptq" if args.model == "70b" else "awq")
-    gptq_sym = args.model == "70b"  # BASELINE configs[3]: GPTQ symmetric (zero = 8), group 128
+    gptq_sym = args.model == "70b"  # GPTQ symmetric (zero = 8), group 128
     reduced = False
     if args.layers > 0 and args.layers != shape.n_layers:
         shape.n_layers, reduced = args.layers, True
@@ -581,7 +581,7 @@ def main():
                                                                  spare_blocks=spare)
     t_init = time.perf_counter()
     # N > 1: the two row-parallel reductions per layer run as the xGMI all-reduce fused with the
-    # residual add + RMSNorm (SURVEY 8f f3) when every rank can map its peers AND the start-up
+    # residual add + RMSNorm when every rank can map its peers AND the start-up
     # self-test reproduces the sequential sum bit for bit (asked first in throw-away child
     # processes, then repeated here); otherwise RCCL all-reduce + slm_rms_norm.
     # SLM_CUSTOM_AR=0 forces the RCCL path.
@@ -592,7 +592,7 @@ def main():
         custom_ar = try_create_xgmi_allreduce(
             pg.rank, pg.world_size, bs, shape.hidden, torch.bfloat16, device,
             log=lambda m: print(f"[bench] {m}", file=sys.stderr))
-        # two lanes on a tensor-parallel rank (round 5): a second, independent instance of the protocol
+        # two lanes on a tensor-parallel rank: a second, independent instance of the protocol
         # for lane 1 (its own signal block and message buffers).  Only when lanes are asked for: the
         # automatic policy keeps TP shards on one lane (their per-rank KV stream is short).
         if custom_ar is not None and args.lanes > 0:
@@ -619,7 +619,7 @@ def main():
     if args.lanes >= 0:
         model.lanes_min = args.lanes
     model.reserve_workspaces(bs, L)
-    # start-up probe of the lane policy (round 5): with lanes on "auto" the step's shape is timed as one lane
+    # start-up probe of the lane policy: with lanes on "auto" the step's shape is timed as one lane
     # and as two on a few layers, and the measurement -- not the Llama-3-8B constants -- decides
     lane_probe = None
     if model.lanes_min < 0 and not args.advance and os.environ.get("SLM_LANE_PROBE", "1") != "0":
@@ -773,7 +773,7 @@ def main():
     nbytes = attn_algo_bytes(attn_rows, attn_lens, model.n_heads, model.n_kv_heads, shape.head_dim, B)
     alone_gbps = nbytes / avg_us / 1e3  # GB/s, the launch replayed ALONE after the timed loop
     # the gate_up GEMM at the row count the step launches it with (a lane's rows under two lanes), and at
-    # the full batch for continuity with rounds 1-3 (before the profiler children below: same clocks
+    # the full batch for continuity with earlier figures (before the profiler children below: same clocks
     # as the timed steps)
     gemm = measure_gemm(model, attn_rows)
     if attn_rows != bs:
@@ -789,7 +789,7 @@ def main():
     # not re-derived here -- the MFMA tile kernel for wide GQA groups, the token-major stream otherwise
     on_tile = kernels.paged_kv_varlen_mha_decode_kernel(
         attn_rows, attn_rows, model.n_heads, model.n_kv_heads, shape.head_dim, B, 1, L, model.dtype) == "attn_tile_kernel"
-    # Round 5: `achieved` / `frac` describe the launch AS THE TIMED LOOP RUNS IT.
+    # `achieved` / `frac` describe the launch AS THE TIMED LOOP RUNS IT.
     # With two lanes that is the launch next to the other lane's int4 GEMMs -- timed inside eager two-lane
     # steps, HIP events on the launching stream right around every attention call (behind the event that
     # chains the lanes' KV streams, so no waiting is included); the same launch replayed alone is reported

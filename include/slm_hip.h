@@ -382,7 +382,7 @@ SLM_API int slm_last_rows(void* out, const void* x, const int32_t* ends, int64_t
 /* LayerNorm with weight and optional bias (bias == NULL: none), fp32 statistics, one rounding:
  * out = T((x - mean) * rsqrt(var + eps) * weight + bias).  replaces kernel::layer_norm
  * (src/kernels/layernorm_kernels.cu:185-256; LayerNormImpl::forward src/layers/normalization.h:86-95)
- * for the LayerNorm model families (GPT-2: BASELINE configs[0], GPT-NeoX, Bloom, MPT).  dim % 8 == 0,
+ * for the LayerNorm model families (GPT-2, GPT-NeoX, Bloom, MPT).  dim % 8 == 0,
  * dim <= 16384, contiguous rows. */
 SLM_API int slm_layer_norm(void* out, const void* x, const void* weight, const void* bias /* or NULL */,
                            int64_t n_tokens, int64_t dim, float eps, int32_t dtype, void* stream);
@@ -549,8 +549,8 @@ SLM_API int slm_allreduce(const slm_ar_args* args, void* stream);
 SLM_API int slm_allreduce_simulate(const slm_ar_args* ranks, int32_t world, void* stream);
 
 /* ========================================================================== */
-/* 7. Host policy: one lane or two for a pure-decode step (round 5)           */
-/*    no reference counterpart -- the two half-batch lanes are this build's   */
+/* 7. Host policy: one lane or two for a pure-decode step                     */
+/*    no reference counterpart -- the two half-batch lanes are this library's */
 /*    own schedule of the decoder stack (models/meta/llama.h:123-345 is one   */
 /*    serial chain per step).  Pure host code, no device work:                */
 /*    ONE source of the rule for the Python mirror (decode.two_lane_split)    */

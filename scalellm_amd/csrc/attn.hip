@@ -48,12 +48,12 @@ __device__ __forceinline__ u32x4 ld16(const void* p) {
 // FX: the rare score transforms (logits soft-cap and/or alibi) are compiled in; the FX = false fast
 // path folds the softmax scale into one fma per score, like the reference's exp2(x*s - max*s)
 // (common/online_softmax.cuh:39-162).
-// W (round 4): 16-byte chunks of a K / V row per lane.  W = 1: LPR lanes x 8 dims cover the row.  W = 2: a
+// W: 16-byte chunks of a K / V row per lane.  W = 1: LPR lanes x 8 dims cover the row.  W = 2: a
 // lane owns TWO chunks (dims [8 sub, 8 sub + 8) and [8 LPR + 8 sub, ...)), so half as many lanes share a row:
 // the 16-lane reduction of every score becomes an 8-lane one, and the softmax arithmetic every lane of a
 // group repeats for its rows is done for half as many rows per lane -- the same bytes in flight (U rows x W
 // chunks), ~37 % fewer VALU instructions per KV byte.  The stream kernel was at the HBM rate already; what
-// this buys is ISSUE SLOTS for the int4 GEMMs that share the SIMDs in the two-lane decode step (DESIGN 7-0a).
+// this buys is ISSUE SLOTS for the int4 GEMMs that share the SIMDs in the two-lane decode step.
 template <typename T, int LPR, int GC, int U, bool NT, bool FX, int W = 1>
 __global__ void __launch_bounds__(512) attn_token_kernel(const AttnKParams p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -82,7 +82,7 @@ __global__ void __launch_bounds__(512) attn_token_kernel(const AttnKParams p) {
   // token -> sequence: q_cu[b] <= tok < q_cu[b+1].  Pure decode batches (one query token per
   // sequence: q_cu[i] == i) are recognised with two independent loads instead of log2(batch)
   // dependent ones -- the binary search is ~0.4 us per step of start-up latency in front of every
-  // workgroup's stream, which is what small batches are made of (DESIGN 3.1).
+  // workgroup's stream, which is what small batches are made of.
   int b;
   const int tq0 = p.q_cu[min(tok, p.batch)], tq1 = p.q_cu[min(tok + 1, p.batch)];
   if (tok < p.batch && tq0 == tok && tq1 == tok + 1) {
@@ -1090,7 +1090,7 @@ SLM_API int slm_paged_kv_varlen_mha(const slm_attn_args* a, void* stream) {
   // max_q_len is the same scheduling contract as the reference's grid (tile_scheduler.cuh:23-27).
   // A forced split count keeps the call on the token-major kernel.
   // Sequence classes by query rows per KV head (rows = q_len * group), decided on the DEVICE from
-  // q_cu_lens, so one call handles mixed prefill / verify / decode batches (BASELINE config 5):
+  // q_cu_lens, so one call handles mixed prefill / verify / decode batches:
   //   rows <= group (q_len = 1)   token-major stream kernel (attn_token_kernel)
   //   group < rows <= 32          MFMA tile kernel, one-wave tiles   (speculative verify)
   //   rows > 32                   MFMA tile kernel, 2/4-wave tiles   (prefill, chunked prefill)

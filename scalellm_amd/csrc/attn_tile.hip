@@ -72,11 +72,11 @@ typedef __attribute__((address_space(3))) tr_v4s tr_lds_v4s;
 // the causal diagonal of every row of the wave then skip the whole mask / bias arithmetic
 // (scale + max only) -- left generic, the compiler if-converts the feature tests into straight-line
 // code (16 tanh + 16 int->float + 5 compare/select per score, ~2/3 of the loop's VALU work).
-// KVT / DB (round 4, the prefill classes): KV tiles of 64 rows -- two S^T blocks per wave and tile, so
+// KVT / DB (the prefill classes): KV tiles of 64 rows -- two S^T blocks per wave and tile, so
 // half the barriers, table lookups and loop overhead per KV row -- in a DOUBLE-BUFFERED LDS image: the
 // next tile's registers are stored into the other buffer right after this tile's MFMAs, ONE barrier per
 // tile (the single-buffer form needs "everybody done reading" + "everybody done writing").
-// DMA (round 5, the double-buffered classes): the next tile travels HBM -> LDS by LDS-DMA
+// DMA (the double-buffered classes): the next tile travels HBM -> LDS by LDS-DMA
 // (buffer_load_dwordx4 ... lds) instead of through 32 staging VGPRs + ds_write.  Measured on the
 // register-staged form (tools/probes/experiments/attn_tile_pipe_halfsteps_and_lds_ahead.md): with the
 // staging taken out of the loop the kernel runs 19...29 % faster -- global-load issue, per-lane 64-bit
@@ -93,7 +93,7 @@ typedef __attribute__((address_space(3))) tr_v4s tr_lds_v4s;
 //   * the cache slots of a tile's 64 rows are looked up ONCE per workgroup (64 threads, one row each, two
 //     tiles ahead) and handed round through LDS, instead of by every thread for its own rows.
 // Needs slot strides < 16 KiB (the descriptor's 14-bit stride field); the launcher falls back otherwise.
-// PIPE (round 5, on the DMA form): the wave is software-pipelined ACROSS tiles -- two score blocks live:
+// PIPE (on the DMA form): the wave is software-pipelined ACROSS tiles -- two score blocks live:
 //     A(t): S' = K[t+1] . Q^T  (16 MFMAs at head_dim 128)   ||   P = exp2(S * c - m), l += sum P   (tile t)
 //     B(t): O += V[t]^T . P    (16 MFMAs)                    ||   row max of S', lazy-rescale decision for t + 1
 // Unpipelined, a wave's tile is QK^T -> softmax -> P.V strictly in turn (each needs the previous result) and the
@@ -103,7 +103,7 @@ typedef __attribute__((address_space(3))) tr_v4s tr_lds_v4s;
 // still suffice: iteration t reads K[t+1] (buffer (t+1)&1) and V[t] (t&1) and fills K[t+2] -> t&1 (last read
 // by QK^T(t) in iteration t-1) and V[t+1] -> (t+1)&1 (last read by P.V(t-1)).  One barrier per 64 rows as before;
 // 32 more VGPRs (the second score block), which the DMA form freed.  Cross-half exchanges by v_permlane32_swap.
-// KV2 (round 5, on the PIPE form; plain causal prefill): TWO GROUPS of NW waves share a workgroup's 32 NW query
+// KV2 (on the PIPE form; plain causal prefill): TWO GROUPS of NW waves share a workgroup's 32 NW query
 // rows and split its KV range -- group g takes the 64-row tiles g, g + 2, g + 4, ... with its own K / V buffers,
 // slot ring and online-softmax state; the two (m, l, O) meet once, through LDS, at the end.  A causal prefill of
 // one long sequence is the serial chain of its longest query tile (32 KV tiles at 2 k: ~55 of the kernel's 59 us
@@ -753,7 +753,7 @@ __global__ void __launch_bounds__(64 * NW * (KV2 ? 2 : 1)) __attribute__((amdgpu
         for (int r = 0; r < 16; ++r) oacc[d][r] *= alpha;
     }
     // P as packed MFMA B fragments (the softmax registers ARE the operand order of P.V).  One-wave (verify)
-    // class, round 5: exponentiate and pack per 8-score group -- 8 floats live instead of 16, which takes the
+    // class: exponentiate and pack per 8-score group -- 8 floats live instead of 16, which takes the
     // soft-cap / alibi / window instantiation from 3 spilled VGPRs to none at its 256-register cap; the
     // multi-wave classes keep all 16 * NH scores in flight and pack inside the MFMA loop (same arithmetic, same
     // summation order either way).

@@ -37,7 +37,7 @@ LlamaForCausalLMHip::LlamaForCausalLMHip(const LlamaArgs& args, const QuantArgs&
   const int64_t tp = parallel_args.world_size();
   // a FusedAllReduce makes the row-parallel layers return this rank's PARTIAL sums (their process group
   // is withheld below); only the fused composition reduces them (reduce_add_norm) -- the plain call
-  // sequence would feed partial sums straight into rms_norm_residual (round-4 advisor finding)
+  // sequence would feed partial sums straight into rms_norm_residual
   TORCH_CHECK(!far_ || opt.fused, "LlamaForCausalLMHip: a FusedAllReduce needs Options::fused = true "
               "(the plain composition reduces through ProcessGroup::allreduce)");
   TORCH_CHECK(args.n_heads % tp == 0 && args.intermediate_size % tp == 0 && args.hidden_size % tp == 0 &&
@@ -197,7 +197,7 @@ void LlamaForCausalLMHip::reserve(int64_t n_tokens) {
 // ---- lanes -------------------------------------------------------------------------------------
 bool LlamaForCausalLMHip::tp_lanes_ok() const {
   // may this rank's row-parallel reductions run on two streams at once?  One rank: nothing to reduce; a
-  // fused all-reduce instance PER LANE (round 5); the one-GPU stand-in group.  A plain RCCL communicator: no.
+  // fused all-reduce instance PER LANE; the one-GPU stand-in group.  A plain RCCL communicator: no.
   if (parallel_args_.world_size() == 1) return true;
   if (far_) return far_lane1_ != nullptr;
   return dynamic_cast<const LocalShardProcessGroup*>(parallel_args_.process_group()) != nullptr;
@@ -511,7 +511,7 @@ torch::Tensor LlamaForCausalLMHip::forward(const torch::Tensor& tokens, const to
     // The layers repack their checkpoint tensors lazily, at the first forward (as the reference does inside its
     // warm-up: weight_repacked_), on whatever stream is current.  With two lanes on two streams that would be a
     // race on the FIRST two-lane step: lane 0 reaches a layer first and repacks it on its stream, lane 1 then
-    // finds it "packed" and reads it on the side stream with nothing ordering the two (round 6: NaN rows of
+    // finds it "packed" and reads it on the side stream with nothing ordering the two (seen: NaN rows of
     // lane 1 on the first step only).  So every layer is packed here, on the caller's stream, before the fork.
     if (!all_packed_) {
       for (auto& L : layers_) { L.qkv->packed(); L.o->packed(); L.gate_up->packed(); L.down->packed(); }

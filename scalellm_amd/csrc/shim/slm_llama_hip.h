@@ -1,5 +1,5 @@
 // slm_llama_hip.h -- the Llama decoder stack of the reference composed in C++ from the HIP layer
-// classes of this directory: the HOST side of the decode hot path, compiled (north_star: "host code
+// classes of this directory: the HOST side of the decode hot path, compiled ("host code
 // stays C++ calling HIP through a thin C-ABI kernel library").
 //
 // Mirrors src/models/meta/llama.h:123-345:
@@ -67,7 +67,7 @@ class LlamaForCausalLMHip {
   LlamaForCausalLMHip(const LlamaArgs& args, const QuantArgs& quant_args, const ParallelArgs& parallel_args,
                       const torch::TensorOptions& options, const Options& opt,
                       std::shared_ptr<FusedAllReduce> fused_allreduce = nullptr,
-                      // round 5: a second, independent instance for lane 1 lets a tensor-parallel rank run two
+                      // a second, independent instance for lane 1 lets a tensor-parallel rank run two
                       // lanes (each lane's reductions meet the peers' same lane: own signal block, own buffers)
                       std::shared_ptr<FusedAllReduce> fused_allreduce_lane1 = nullptr);
 

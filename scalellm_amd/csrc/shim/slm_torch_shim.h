@@ -7,7 +7,7 @@
 //   llm::paged_kv_varlen_mha           src/kernels/attention/attn_api.h:12-27
 //   llm::kernel::set_kv_cache          src/kernels/kv_cache_kernels.h:6-11
 //   llm::kernel::apply_rotary_pos_emb  src/kernels/pos_embedding_kernels.h
-// The int4 path is offered at the layer boundary the survey recommends (ParallelLinearImpl,
+// The int4 path is offered at the layer boundary (ParallelLinearImpl,
 // src/layers/linear/parallel_linear.h:17-37): slm::W4Linear owns the MFMA-native packed layout
 // and is what a QLinearHipImpl subclass wraps (40 lines: slm_qlinear_hip.h).
 // slm::ProcessGroupRCCL implements llm::ProcessGroup's contract (process_group.h:10-60) on RCCL.

@@ -246,7 +246,7 @@ __global__ void __launch_bounds__(256, (POST && PC * MT == 4 && MT < 4) ? 1 : 2)
   uint32_t szcur[NTW][PC][NG], sznext[NTW][PC][NG];
   auto w_issue = [&](int t, int h, int cfirst) {  // half-chunk h of the pass starting at cfirst
     const uint32_t* wp = p.wq + ((((int64_t)cfirst * 2 + h) * n_tiles + ntile[t]) * 64 + lane) * 4;
-    // plain (cacheable) loads, not non-temporal ones (round 4): a layer's weights are re-read within
+    // plain (cacheable) loads, not non-temporal ones: a layer's weights are re-read within
     // ~0.4 ms -- by the second BM = 64 row block at M = 65...128 and by the second lane of the two-lane
     // decode step -- and a cacheable line is still in the Infinity Cache then.  Two-lane bs 256 step
     // 24.85 -> 23.98 ms, one lane 26.1 -> 25.9; stand-alone with rotating weights 3-6 % slower (124 ->
@@ -565,7 +565,7 @@ static int plan_gemm(const slm_w4_gemm_args* a, GemmPlan* pl) {
     // BM = 128 when its tiles alone fill the chip, or when K is deep AND there are enough column
     // tiles to spread (a deep, very narrow shard -- 70B TP=8 qkv: 8192 x 1280 -- runs 20 % faster
     // on twice as many BM = 64 tiles: 22.0 -> 17.7 us)
-    // (round 4: the deep-K rule starts at 64 tiles, not 32.  Llama-3-8B's down_proj -- 14336 x 4096, 32 tiles --
+    // (the deep-K rule starts at 64 tiles, not 32.  Llama-3-8B's down_proj -- 14336 x 4096, 32 tiles --
     // is 3 % faster alone on BM = 128 (33.0 vs 34.1 us at M = 128), but in the two-lane decode step its 64 KiB,
     // ~200-VGPR workgroups share a CU badly with the attention stream's: 79 -> 135 us per call once the stream
     // kernel keeps two row chunks per lane, 58 us on BM = 64 tiles like the other three layers)
@@ -585,7 +585,7 @@ static int plan_gemm(const slm_w4_gemm_args* a, GemmPlan* pl) {
     const int64_t tiles16 = ((a->M + 255) / 256) * ((a->N + 255) / 256);
     const int64_t rounds = (tiles16 + 255) / 256;
     if (a_fits && tiles16 >= 224 && tiles16 * 100 >= rounds * 256 * 87) mt = 16;
-    // ... and when the 256 x 128 tiles need MORE rounds than they save (round 5, M = 2648 -- the mixed step's row
+    // ... and when the 256 x 128 tiles need MORE rounds than they save (M = 2648 -- the mixed step's row
     // count: o 4096 x 4096 = 176 / 352 tiles: one 69 %-full round of 256 x 256 tiles 102.6 us against two rounds of
     // 256 x 128 tiles 117.4; down 340.8 against 382.8): a 256 x 128 tile takes 0.58 of a 256 x 256 tile's time
     // (profiles/r05_gemm_large_m.jsonl; layer chain 1282 -> 1192 us at M = 2648, 1400 -> 1322 at 3072,
@@ -595,7 +595,7 @@ static int plan_gemm(const slm_w4_gemm_args* a, GemmPlan* pl) {
     if (a_fits && mt == 8 && rounds8 >= 2 && rounds * 100 < rounds8 * 58 && tiles16 * 100 >= rounds * 256 * 65 &&
         tune_get(TUNE_W4_XL_MODEL, 1) != 0)
       mt = 16;
-    // Round 6: the STREAM-K form of the 256 x 256 kernel (w4_xl.hip): the tile x K work cut into 256 equal ranges
+    // the STREAM-K form of the 256 x 256 kernel (w4_xl.hip): the tile x K work cut into 256 equal ranges
     // -- no round of tiles is left part-filled.  Cost model in units of one 256 x 256 tile's time: the chosen
     // kernel's rounds (a 256 x 128 tile: 0.58) against 1.4 x tiles16 / 256 (measured 1.28...1.41 over M = 1536...3072:
     // a second pipeline fill per workgroup, the partial tiles' round trip, a fuller chip's lower clock;
@@ -725,7 +725,7 @@ static int plan_gemm(const slm_w4_gemm_args* a, GemmPlan* pl) {
     }
   }
   pl->ks_mt = 1;
-  // 33 <= M <= 64 (round 4; the default outside the two-lane steps since round 6): the K-sliced stream with TWO row tiles -- every
+  // 33 <= M <= 64 (the default outside the two-lane steps): the K-sliced stream with TWO row tiles -- every
   // weight word unpacked once for two MFMAs.  One chunk of K per wave (the activations of both row
   // tiles fill the registers), 8 waves: a workgroup covers 1024 of K, the rest is split across
   // workgroups (fp32 slabs, summed by the consumer under SLM_W4_DEFER_REDUCE or by the reduce kernel).
@@ -736,7 +736,7 @@ static int plan_gemm(const slm_w4_gemm_args* a, GemmPlan* pl) {
   // (two lanes of 64 rows) 14.2 -> 21.5 ms -- and the stand-alone gain is small because A (512 KB at
   // M = 64, K = 4096) cannot stay on one CU: either K is split over CUs (slab traffic, this kernel) or
   // A is re-streamed per column tile (the general kernel); the step from M = 32 stays.
-  // Round 6: ON by default where the caller does not say the call shares the chip (SLM_W4_SHARES_CHIP, set by
+  // ON by default where the caller does not say the call shares the chip (SLM_W4_SHARES_CHIP, set by
   // the two-lane decode steps): M = 33 / 48 / 64 layer chain 96 / 97 / 101 -> 89 / 90 / 93 us, bs = 64 step
   // 9.17 -> 8.95 ms (profiles/r06_ks_mt2_default.jsonl).  SLM_W4_KS_MT2 = 0 never, 1 / 2 always (2: any split).
   const int mt2_knob = tune_get(TUNE_W4_KS_MT2, -1);
@@ -771,7 +771,7 @@ static int plan_gemm(const slm_w4_gemm_args* a, GemmPlan* pl) {
       pl->n_nblocks = (n_tiles + tpw - 1) / tpw;
     }
   }
-  // 65 <= M <= 128 (round 5): all rows in ONE workgroup (w4_m128.hip) -- every weight word fetched and
+  // 65 <= M <= 128: all rows in ONE workgroup (w4_m128.hip) -- every weight word fetched and
   // dequantised once for 4 MFMAs instead of once per 64-row block for 2 -- in 132-VGPR / 32-KiB workgroups
   // that sit twice on a CU next to the decode attention stream of the other lane.  Split-K aims at two
   // workgroups per CU with >= 512 of K each (the consumers take up to 16 slabs).

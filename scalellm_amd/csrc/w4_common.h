@@ -19,7 +19,7 @@ struct W4Dq<bf16_tag> {
   // shift + 8 cvt + 4 v_pk_fma_f32 + 4 cvt_pk = 19 VALU (the magic-number route through fp32 took 27
   // and produced the same bits).
   //
-  // Round 5: 15 VALU per word, same bits.  A nibble in a byte, 0x0q, IS the OCP E4M3 encoding of
+  // 15 VALU per word, same bits.  A nibble in a byte, 0x0q, IS the OCP E4M3 encoding of
   // q * 2^-9 (codes 0..7 are the subnormals m * 2^-9, codes 8..15 the first binade (8 + m) * 2^-9: one
   // linear ramp), so ONE v_cvt_pk_f32_fp8 turns two nibbles into two floats where v_cvt_f32_ubyteN
   // took one instruction each: 3 mask / shift + 4 cvt_pk_f32_fp8 + 4 v_pk_fma_f32 + 4 cvt_pk.  The
@@ -173,7 +173,7 @@ struct GemmKParams {
   int ks_tpw;     // w4_ks.hip: consecutive column tiles per workgroup (n_nblocks = tile runs)
   int ks_groups;  // w4_ks.hip: K / group_size (rows of the scale table)
   int ks_dbg;     // w4_ks.hip: probe bits (SLM_W4_KS_DBG), 0 in production
-  // w4_xl.hip, stream-K form (round 6): workgroup g (a ticket drawn at start) owns the 128-deep chunks
+  // w4_xl.hip, stream-K form: workgroup g (a ticket drawn at start) owns the 128-deep chunks
   // [g * sk_per, (g + 1) * sk_per) of the tile-major work list (tiles x n_chunks); sk_sync = {ticket, flag[g] ...},
   // zero at launch; sk_part = one 256 x 256 fp32 tile image per workgroup (fragment-major)
   int sk_per;
@@ -274,7 +274,7 @@ bool gemm_ks_config_ok(int ng, int cw, int nw, int mt = 1);
 constexpr size_t w4_ks_lds_bytes(int nw) { return (size_t)4 * nw * 4096 + 64; }  // 4 partial slots + counters
 
 // 65 <= M <= 128: all rows in one workgroup, 64-deep chunks, two workgroups per CU next to the decode
-// attention stream (w4_m128.hip, round 5); wd = weight ring depth, (64-deep chunks per split) % wd == 0
+// attention stream (w4_m128.hip); wd = weight ring depth, (64-deep chunks per split) % wd == 0
 void launch_gemm_m128(const GemmKParams& kp, int dtype, int group_size, int wd, int kw, int ct, int adma, int n_blocks, hipStream_t st);
 constexpr size_t W4_M128_LDS_BYTES = 2 * 128 * 128;
 

@@ -1,10 +1,10 @@
 // w4_ks.hip -- int4-weight x fp16/bf16-activation GEMM for M <= 32: the K-SLICED weight stream.
 //
 // Same operator as w4.hip (replaces marlin::gptq_gemm, reference gptq_gemm.cu:585-710, on the
-// small-batch decode shapes: Llama-3-8B AWQ, bs = 32), same packed layout
+// small-batch decode shapes -- Llama-3-8B AWQ, bs = 32), same packed layout
 // and scale/zero table (w4.hip header), same post-scaled numerics as w4_small.hip.
 //
-// What rounds 2-3 measured (profiles/r03_ks_*): at M <= 32 the weight stream itself is
+// Measured (profiles/r03_ks_*): at M <= 32 the weight stream itself is
 // VALU-issue-bound on the int4 unpack (a SIMD issues one VALU/MFMA instruction per 4 cycles: 7 VALU +
 // 1 MFMA per 8-weight word = 32 cycles = the MFMA's own pipe time), and w4_small.hip loses another 2x
 // around it: activation fragments re-read from LDS per MFMA (LDS-bandwidth-bound), a second MFMA per
@@ -72,7 +72,7 @@ constexpr int KS_SLOTS = 4;  // partial-tile slots in LDS (see the slot arithmet
 
 // CW: 128-deep chunks of K per wave (1, 2, 4);  NG: scale groups per chunk (1: group >= 128,
 // 2: 64, 4: 32);  NW: waves per workgroup (4, 8);  TL: timeline probe (tools/probe_ks_timeline.py)
-// MT: 32-row tiles of tokens (1: M <= 32; 2: 33 <= M <= 64, round 4).  With MT = 2 every weight word is
+// MT: 32-row tiles of tokens (1: M <= 32; 2: 33 <= M <= 64).  With MT = 2 every weight word is
 // unpacked ONCE and feeds two MFMAs (one per row tile): the stream that was VALU-issue-bound on the
 // unpack at M <= 32 (7 VALU + 1 MFMA per word) becomes 7 VALU + 2 MFMAs -- matrix-pipe-bound -- instead
 // of a second 55 us pass or the general kernel's 94-100 us (LDS fragment reads per MFMA, a barrier per
@@ -80,7 +80,7 @@ constexpr int KS_SLOTS = 4;  // partial-tile slots in LDS (see the slot arithmet
 // for ONE chunk per wave: K is split over the 8 waves x ceil(K / 1024) workgroups (fp32 slabs, summed
 // by the consumer or the reduce kernel).  A 64 x 32 partial tile goes through the LDS meeting as two
 // consecutive entries of the slot sequence (2t, 2t + 1).
-// (A fragment-major activation layout was measured in round 5 -- 3.6 % -- and is kept only as
+// (A fragment-major activation layout was measured -- 3.6 % -- and is kept only as
 // tools/probes/experiments/w4_ks_fragment_major_activations.diff.)
 template <typename T, int CW, int NG, int NW, bool TL = false, bool PK = false, int MT = 1>
 __global__ void __launch_bounds__(NW * 64, 2) w4a16_gemm_ks_kernel(const GemmKParams p) {

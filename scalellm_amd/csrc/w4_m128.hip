@@ -1,13 +1,13 @@
-// w4_m128.hip -- int4-weight x fp16/bf16-activation GEMM for 65 <= M <= 128 (round 5).
+// w4_m128.hip -- int4-weight x fp16/bf16-activation GEMM for 65 <= M <= 128.
 //
 // Same operator as w4.hip (replaces marlin::gptq_gemm, reference gptq_gemm.cu:585-710; Marlin's
 // thread-block tile for this regime is gemm_kernel.cuh:49 with thread_m_blocks = 4), same packed
 // layout and scale/zero table (w4.hip header), same bit-faithful dequant (W4Dq<T>,
-// marlin/numeric_conversion.h:19-62).  This is the row count the two-lane decode step (decode.py,
-// DESIGN 3.6) runs ALL of its GEMMs at -- 128 rows per lane -- next to the other lane's attention
+// marlin/numeric_conversion.h:19-62).  This is the row count the two-lane decode step (decode.py)
+// runs ALL of its GEMMs at -- 128 rows per lane -- next to the other lane's attention
 // stream, and the row count of every 70B layer at bs = 128.
 //
-// What the general kernel does there, and why it is slow (round-4 review, weak 2): BM = 64 tiles --
+// What the general kernel does there, and why it is slow: BM = 64 tiles --
 // every weight word is fetched and dequantised by TWO workgroups (one per 64-row block), 19 VALU per
 // word for 2 MFMAs; next to the attention stream (one wave per SIMD, ~65 % of the issue slots, high
 // priority) the GEMM is bound by its instruction count: 193 VALU per 16 MFMAs.  Its BM = 128 form
@@ -15,7 +15,7 @@
 // workgroup (200 VGPRs, 80 KiB) instead of two -- and measured slower in the step.
 //
 // This kernel: all 128 rows in one workgroup (MT = 4: a weight word is dequantised ONCE, 15 VALU with
-// the round-5 fp8-pair route, for 4 MFMAs = 3.75 VALU per MFMA), built to sit TWICE on a CU beside
+// the fp8-pair route, for 4 MFMAs = 3.75 VALU per MFMA), built to sit TWICE on a CU beside
 // the attention workgroup:
 //   * K chunks of 64 (one 16-B weight load per lane = exactly one kt block of the packed layout),
 //     double-buffered in 2 x 16 KiB of LDS (128 rows x 128 B, XOR-swizzled: slot ^ ((row >> 1) & 7)
@@ -48,7 +48,7 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t m128_rsrc(const void* base, ui
 //     registers for a whole chunk before it is stored (two staging sets, 32 VGPRs): the wait at the bottom of
 //     chunk c is for loads issued a full chunk earlier, and -- VMEM returns in order -- the weight loads issued
 //     behind them get two chunks of slack instead of one.
-// KW: waves per column tile (1 / 2).  2 (round 5): a 512-thread workgroup whose wave pairs (w, w + 4) share a column
+// KW: waves per column tile (1 / 2).  2: a 512-thread workgroup whose wave pairs (w, w + 4) share a column
 //     tile and split every 64-deep chunk between them -- wave w takes k-steps 0, 1 (the first 8 bytes of the lane's
 //     weight vector), wave w + 4 k-steps 2, 3 -- each with its own accumulators, summed once through LDS at the end.
 //     Same tile, same bytes, same instructions in total; but a launch whose grid gives a CU ONE workgroup (gate_up at
@@ -60,7 +60,7 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t m128_rsrc(const void* base, ui
 //     (~21 B/clk per CU) -- not HBM, not the matrix pipe -- is what a 70B-sized layer waits for (gate_up:
 //     448 workgroups x 2.5 MB = 1.17 GB = 91 us at 12.9 TB/s of aggregate ingest, 144 us measured).  Eight
 //     column tiles share one panel: 0.70 GB.
-// ADMA (round 5): the activation chunk goes L2 -> LDS by LDS-DMA (buffer_load_dwordx4 ... lds: a wave instruction
+// ADMA: the activation chunk goes L2 -> LDS by LDS-DMA (buffer_load_dwordx4 ... lds: a wave instruction
 //     writes 1 KiB = 8 rows of the 128-B-row image linearly, so the XOR swizzle is applied on the SOURCE side:
 //     lane l of instruction i fetches row 8i + l/8, 16-B slot (l % 8) ^ ((row >> 1) & 7)) instead of through
 //     staging VGPRs and ds_write_b128.  A probe build without any activation staging ran the 70B shapes 10...14 %
@@ -160,7 +160,7 @@ w4a16_gemm_m128_kernel(const GemmKParams p) {
     for (int i = 0; i < (ADMA ? 0 : AI); ++i) *reinterpret_cast<u32x4*>(smem + buf * M128_BUF + a_lds[i]) = areg[set][i];
   };
   // weights: plain (cacheable) loads -- the other lane of the decode step re-reads the layer within
-  // ~0.4 ms and finds it in the Infinity Cache (w4.hip, round 4)
+  // ~0.4 ms and finds it in the Infinity Cache (w4.hip)
   struct WVec { uint32_t w[JW]; };
   auto w_load = [&](int c) -> WVec {
     WVec v;

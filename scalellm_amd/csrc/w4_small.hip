@@ -189,7 +189,7 @@ __global__ void __launch_bounds__(256, 2) w4a16_gemm_small_kernel(const GemmKPar
             // so the mask rides in an SGPR and the magic in a VGPR, both opaque to the optimiser (with
             // literals hipcc emits v_and + v_or).  A plain expression, NOT inline asm: hipcc inserts
             // no hazard wait states behind an asm statement, and an MFMA issued right behind an asm
-            // v_and_or_b32 reads stale B operands (seen in round 2 with independent MFMA chains).
+            // v_and_or_b32 reads stale B operands (seen with independent MFMA chains).
             const uint32_t x = q == 0 ? word : word >> (4 * q);
             o[q] = (x & mask_s) | magic_v;
           }

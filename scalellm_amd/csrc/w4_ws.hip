@@ -62,7 +62,7 @@ static_assert(WS_AL <= WS_A_UNITS - 1, "the slot of unit g + WS_AL must have bee
 // NGC: scale groups per 64-deep chunk (2 for group 32, else 1)
 // WNT: non-temporal weight loads -- right when every weight is read ONCE per launch (one block of 256
 // rows: the decode batch), wrong when several row blocks re-read the weights (prefill: cacheable lines
-// are served from L2 / Infinity Cache the second time; round 4: M = 1024 layer 533 -> 508 us)
+// are served from L2 / Infinity Cache the second time; M = 1024 layer 533 -> 508 us)
 template <typename T, int NGC, bool WNT>
 __global__ void __launch_bounds__(512, 2) w4a16_gemm_ws_kernel(const GemmKParams p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];

@@ -34,7 +34,7 @@ static_assert(XL_AL <= XL_A_UNITS - 2, "slot of unit g + XL_AL was released befo
 // NGC: scale groups per 64-deep chunk (2 for group 32, else 1)
 // WNT: non-temporal weight loads -- right when every weight is read ONCE per launch (one block of 256
 // rows: the decode batch), wrong when several row blocks re-read the weights (prefill: cacheable lines
-// are served from L2 / Infinity Cache the second time; round 4: M = 1024 layer 533 -> 508 us)
+// are served from L2 / Infinity Cache the second time; M = 1024 layer 533 -> 508 us)
 // One output tile (column block nb, row block mb) over the 64-deep chunks [c0, c1) of K: prologue + main loop, the
 // sums left in `acc` (C^T accumulators).  MULTI: the caller runs several passes in one launch (the stream-K form
 // below): the pass ends drained (no DMA / load in flight, every wave past its last LDS read).
@@ -293,7 +293,7 @@ __global__ void __launch_bounds__(512, 2) w4a16_gemm_xl_kernel(const GemmKParams
   xl_store<T>(p, acc, nb, mb, ks, p.split_k == 1);
 }
 
-// ---- stream-K form (round 6) ---------------------------------------------------------------------------------
+// ---- stream-K form ---------------------------------------------------------------------------------
 // Tiles that do not fill whole rounds of the 256 CUs (M = 2648, N = 4096: 176 tiles = one 69 %-full round) leave
 // the rest of the chip idle for a whole tile time.  Here the WORK -- tiles x 128-deep chunks of K, tile-major --
 // is cut into 256 equal ranges, one per workgroup (the reference's own answer: Marlin's striped partition,

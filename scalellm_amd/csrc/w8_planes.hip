@@ -3,7 +3,7 @@
 // The reference's quantised linears accept 4 and 8 bits (qlinear_awq_marlin_impl.cpp:25-26,
 // qlinear_gptq_marlin_impl.cpp; CPU path construct_weights, qlinear_impl.cpp:21-100, generic in
 // `bits`); marlin::gptq_gemm / gptq_repack / awq_repack take num_bits (marlin.h:17-37).  Every
-// BASELINE config is int4, so the 8-bit case gets no kernel of its own -- it is REWRITTEN, exactly,
+// headline workload is int4, so the 8-bit case gets no kernel of its own -- it is REWRITTEN, exactly,
 // into the operator the int4 kernels already implement:
 //
 //   q = 16 hi + lo,  z = 16 zh + zl   (hi, lo, zl in 0..15;  zh = z >> 4 in 0..16)

@@ -137,7 +137,7 @@ def two_lane_split(shape: "LlamaShape", n_heads: int, n_kv_heads: int, world_siz
     (csrc/shim/slm_llama_hip.cpp) cannot drift apart.
 
     Two lanes need: one rank -- or a tensor-parallel rank whose row-parallel reductions can run on two
-    streams at once (tp_lanes_ok: one fused xGMI all-reduce instance PER LANE, round 5; a plain RCCL
+    streams at once (tp_lanes_ok: one fused xGMI all-reduce instance PER LANE; a plain RCCL
     communicator cannot) --, a pure decode batch in the reference's graph-replay sense (every sequence
     brings exactly one token: q_max_seq_len == 1 and n_tokens == n_seqs, the condition ModelRunner replays
     on, model_runner.cpp:112-140, under which q_cu_seq_lens is the identity), >= 64 tokens, and --
@@ -176,7 +176,7 @@ class LlamaDecodeStep:
         self.ckpt = [] if keep_checkpoint else None
         # optional custom_allreduce.XgmiAllReduce: the two row-parallel reductions of a layer then
         # run as ONE launch each, fused with the residual add + RMSNorm that follows
-        # Round 5: a PAIR (lane 0, lane 1) lets a tensor-parallel rank run two lanes: every lane owns a whole
+        # a PAIR (lane 0, lane 1) lets a tensor-parallel rank run two lanes: every lane owns a whole
         # instance of the protocol (signal block + two alternating message buffers), so the lanes'
         # reductions -- on two streams, in the same order on every rank -- never share a flag or a buffer
         if isinstance(custom_allreduce, (list, tuple)):
@@ -332,7 +332,7 @@ class LlamaDecodeStep:
     # ------------------------------------------------------------------------------------------
     # One decoder stack over a range of token rows ("lane").  A step normally has ONE lane (all rows,
     # the caller's stream).  A large pure-decode batch on a single GPU may run as TWO half-batch lanes
-    # on two streams (round 4, experiment 9 of the round-3 review): the decode attention is HBM-bound
+    # on two streams: the decode attention is HBM-bound
     # and the int4 GEMMs are matrix-pipe / L2-bound, so one half's GEMMs run under the other half's
     # attention.  The attention launches of the two lanes are chained by events (A0(l) -> A1(l) ->
     # A0(l+1) ...): exactly one attention kernel streams the KV cache at any time and each lane's
@@ -364,7 +364,7 @@ class LlamaDecodeStep:
                               params.q_cu_seq_lens.numel() - 1, params.q_max_seq_len, params.kv_max_seq_len,
                               tp_lanes_ok=True)
 
-    # ---- graph variants (ModelRunner, round 5) -------------------------------
+    # ---- graph variants (ModelRunner) -------------------------------
     # A captured graph freezes every host-side decision of the step at the CAPTURE-time hints
     # (kv_max_seq_len = cuda_graph_max_seq_len, model_runner.cpp:88-90).  Two of those decisions depend on
     # the batch that is replayed, not on the bound: one lane or two (the policy wants the batch's real
@@ -393,7 +393,7 @@ class LlamaDecodeStep:
         return lanes, bool(uniform)
 
     def probe_lanes(self, n_tokens: int, kv_len: int, n_layers: int = 8, reps: int = 3):
-        """START-UP probe of the lane policy (round 5): time the first `n_layers` decoder layers (the stack alone:
+        """START-UP probe of the lane policy: time the first `n_layers` decoder layers (the stack alone:
         no embedding, no lm_head -- they cost a 2-layer probe more than the layers and drown the signal) of a uniform
         pure-decode batch (n_tokens sequences x kv_len tokens, synthetic block table over this model's own KV
         cache) as ONE lane and as TWO, each captured into a hipGraph and replayed `reps` times, and record
@@ -631,7 +631,7 @@ class LlamaDecodeStep:
                     if prev is not None and self.lanes_chain:
                         ln.stream.wait_event(prev)
                     # the KV STREAM is what the chain serialises: the token is handed on right behind the
-                    # stream kernel, the split-KV combine pass of a ragged batch (round 5: ~5 us that only
+                    # stream kernel, the split-KV combine pass of a ragged batch (~5 us that only
                     # reads this lane's partials) runs outside the chained section
                     self._attn(ln, li, phase=1)
                     prev = torch.cuda.Event()

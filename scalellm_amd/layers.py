@@ -14,7 +14,7 @@ the reference so parity tests read like the reference's own layer tests.
                           first forward, all-reduce then bias for row-parallel)
   LayerNorm            <- llm::LayerNormImpl          src/layers/normalization.h:68-110
   Activation           <- llm::Activation             src/layers/activation.h:36-46, activation.cpp:80-140
-                          (the LayerNorm model families -- GPT-2, BASELINE configs[0] -- next to the
+                          (the LayerNorm model families -- GPT-2 -- next to the
                           RMSNorm / SiLU pair the Llama path uses)
 """
 from __future__ import annotations

@@ -72,7 +72,7 @@ class ProcessGroup:
             use_gpu = device is not None and device.type == "cuda"
             os.environ.setdefault("MASTER_ADDR", "127.0.0.1")
             os.environ.setdefault("MASTER_PORT", "29511")
-            # dmabuf IPC only on this pool's driver (see README / environment notes)
+            # dmabuf IPC only on the driver used here
             os.environ.setdefault("HSA_ENABLE_IPC_MODE_LEGACY", "0")
             kw = {}
             if use_gpu:

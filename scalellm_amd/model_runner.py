@@ -18,7 +18,7 @@ Same contract as the reference:
 The model is anything with `forward(tokens, positions, params, **kw) -> Tensor` whose output lives
 in a static buffer (scalellm_amd.decode.LlamaDecodeStep returns views of its own buffers).
 
-One extension over the reference (round 5): a model may offer GRAPH VARIANTS
+One extension over the reference: a model may offer GRAPH VARIANTS
 (`graph_variants` / `graph_variant_for` / `graph_variant`, see LlamaDecodeStep).  A captured graph
 freezes the step's host-side decisions at the capture-time hints, but two of them belong to the batch
 that is replayed: one half-batch lane or two (the policy wants the batch's REAL context length, not
@@ -44,7 +44,7 @@ class ModelRunnerOptions:
     cuda_graph_max_seq_len: int = 2048
     cuda_graph_batch_sizes: List[int] = field(default_factory=list)
     num_decoding_tokens: int = 1
-    # extension (round 5): context lengths at which capture_cuda_graphs() runs the model's start-up lane
+    # extension: context lengths at which capture_cuda_graphs() runs the model's start-up lane
     # probe for the captured batch size (LlamaDecodeStep.probe_lanes: the same layers timed as one lane and
     # as two; recorded in the library's policy table), so that the one-lane / two-lane variant a replayed
     # batch gets is a MEASURED decision near its real context length.  Empty = the policy's constants.
