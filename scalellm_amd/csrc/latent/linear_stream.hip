@@ -1,5 +1,5 @@
 // linear_stream.hip -- y = x W^T in bf16 for up to 128 rows (decode batches, sampled rows), from weights that were
-// laid out for it at load.  Bound: the HBM stream of W.
+// laid out for it at load.  Bound: the HBM stream of W; above 64 rows what a CU has under way of x and W together.
 //
 // Layout of W (slm_linear_stream): panels of 64 columns, in a panel steps of 64 k, in a step four blocks of 16 columns,
 // each two MFMA operands of 1 KB: lane (r = lane % 16, g = lane / 16) of operand h holds column r, k = 32 h + 8 g .. + 7.
@@ -15,9 +15,15 @@
 //            take every WK-th step (twice the waves on a CU where a launch has one workgroup for it)
 // Loads of W and x run D steps ahead in a register ring: the loop has no branch in it, so every wait is for the oldest.
 //
+// What bounds the wave-N form: a CU has some 32 KB of loads under way, which come back in order, so x waits behind W and both
+// together come at 50 - 57 GB/s a CU, whatever is asked for how early (rings of 4 or 8 steps, three or six stages of LDS-DMA: level).  A
+// step's bytes are 16 KB of x at 128 rows and 8 KB of W for 64 columns; with 64 rows or 128 columns the memory's own rate is near.  So
+// row counts have their own tiles (up to 96 rows 96 instead of 128: 28672 x 4096 45.6 / 42.5 us, 14336 -> 4096 27.3 / 26.2).
+//
 // us at 28672 x 4096 (GLU) / 14336 -> 4096 (slabs) / 16384 x 2048, against the kernel of linear.hip, and above 32 rows the
-// vendor product: 1 row 37.7, 20.4, 12.8 (46, 27.6, 16.4); 16 rows 38.6, 20.7, 13.1 (67, 38, 22); 32 rows 38.9, 21.1, 14.1
-// (63, 41, 21); 64 rows 44, 24, 14.8 (57 + 5 for the GLU's launch, 42, 18); 128 rows 52, 34, 22 (59 + 5, 78, 22).
+// vendor product: 1 row 37.7, 20.4, 12.8 (46, 27.6, 16.4); 16 rows 38.6, 20.7, 13.1 (67, 38, 22); 32 rows 36.2, 19.4, 12.6
+// (63, 41, 21); 64 rows 38.4, 22.7, 14.6 (57 + 5 for the GLU's launch, 42, 18); 96 rows 42.5, 26.2, 16.5 (55 with the launch, -, 22); 128 rows
+// 47.3, 29.8, 19.0 (59 with the launch, 78, 23).
 #include "latent_common.h"
 
 namespace slm {
@@ -157,9 +163,10 @@ __global__ void __launch_bounds__(256) linear_wave_k_kernel(const slm_linear_arg
 template <int MT, int NT, int WK, int D, int EPI>
 __global__ void __launch_bounds__(256 * WK) linear_wave_n_kernel(const slm_linear_args a) {
   constexpr bool GLU = EPI == SLM_LIN_GLU;
-  constexpr int ROW = 128 * WK + 16;      // bytes of a row of x in LDS: 16 rows start in 16 different bank quads
+  constexpr int GROUP = MT * 16 * 128;    // bytes of a group's step of x in LDS: 16-byte chunk c of row r lies in slot c ^ (r & 7)
+  constexpr int AHEAD = MT < 3 ? 1 : NT == 1 ? 3 : 2;
   constexpr int XU = MT * 16 * 8 / 256;   // 16-byte units a thread stages
-  constexpr int XB = MT * 16 * ROW, PART = 4 * NT * MT * 1024;
+  constexpr int XB = WK * GROUP, PART = 4 * NT * MT * 1024;
   constexpr int PARTS = (WK - 1) * PART > (GLU && NT == 1 ? PART : 0) ? (WK - 1) * PART : (GLU && NT == 1 ? PART : 0);
   static_assert(MT >= 2 && D % 2 == 0 && (!GLU || NT < 3), "tiles");
   __shared__ __attribute__((aligned(16))) char lds[2 * XB > PARTS ? 2 * XB : PARTS];
@@ -181,7 +188,7 @@ __global__ void __launch_bounds__(256 * WK) linear_wave_n_kernel(const slm_linea
     const int u = tid + 256 * WK * i, r = u / (8 * WK), c = u % (8 * WK);
     xp[i] = reinterpret_cast<const bf16*>(a.x) + min(m0 + r, a.M - 1) * a.ldx;
     xk[i] = 8 * c;
-    xd[i] = r * ROW + c * 16;
+    xd[i] = c / 8 * GROUP + r * 128 + ((c ^ r) & 7) * 16;
   }
   f32x4 acc[NT][MT];
 #pragma unroll
@@ -190,54 +197,82 @@ __global__ void __launch_bounds__(256 * WK) linear_wave_n_kernel(const slm_linea
     for (int v = 0; v < MT; ++v) acc[t][v] = f32x4{0.f, 0.f, 0.f, 0.f};
   StreamK w[D][NT];
   u32x4 x[D][XU];
-  auto load = [&](int u, int i) {   // (a group past the last step reads that step again: not multiplied)
-    const int k0 = (s0 + i * WK) << 6;
-#pragma unroll
-    for (int t = 0; t < XU; ++t) x[u][t] = *reinterpret_cast<const u32x4*>(xp[t] + min(k0 + xk[t], (int)a.K - 8));
-    const int64_t s = min(s0 + i * WK + kg, steps - 1);
-#pragma unroll
-    for (int t = 0; t < NT; ++t) stream_load_w(w[u][t], wp[t] + s * STREAM_STEP);
+  auto load_x = [&](int u, int t, int i) {   // (a group past the last step reads that step again: not multiplied)
+    x[u][t] = *reinterpret_cast<const u32x4*>(xp[t] + min(((s0 + i * WK) << 6) + xk[t], (int)a.K - 8));
   };
-  auto put = [&](int u, int buf) {
-#pragma unroll
-    for (int t = 0; t < XU; ++t) *reinterpret_cast<u32x4*>(lds + buf * XB + xd[t]) = x[u][t];
+  auto load_w = [&](int u, int t, int i) {
+    stream_load_w(w[u][t], wp[t] + (int64_t)min(s0 + i * WK + kg, steps - 1) * STREAM_STEP);
   };
-  auto multiply = [&](int u, int buf) {
-    const char* base = lds + buf * XB + r16 * ROW + kg * 128 + g * 16;
+  auto put = [&](int u, int t, int buf) { *reinterpret_cast<u32x4*>(lds + buf * XB + xd[t]) = x[u][t]; };
+  // Fragments are read ahead of their products, loads and the next step's x go between them, one or two at a time: a wave that reads, waits
+  // and multiplies in turn, and asks for all its loads at the end, waits for LDS and the address unit most of a step (128 rows, 28672 x 4096 / 14336
+  // -> 4096 / 6752 x 4096: 51.2 / 33.9 / 35.3 us; fragments ahead 49.2 / 32.8 / 33.1; rows of LDS without a conflict, where 144-byte ones took 12
+  // cycles a read instead of 4, 47.9 / 31.3 / 29.3; loads between the products 47.3 / 29.8 / 28.0).
+  StreamK f[AHEAD + 1];
+  const int fragment[2] = {kg * GROUP + r16 * 128 + ((g ^ r16) & 7) * 16, kg * GROUP + r16 * 128 + (((4 + g) ^ r16) & 7) * 16};
+  auto fetch = [&](int v, int buf) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) f[v % (AHEAD + 1)].v[h] = *reinterpret_cast<const bf16x8_t*>(lds + buf * XB + v * 2048 + fragment[h]);
+  };
+  // step i + u: its products; between them the next step's x is written, x of D steps on and w of D - 1 steps on are asked for
+  auto step = [&](int u, int i, bool mine, bool more) {
+    constexpr int U = D - 1;
+    if (mine) {
+#pragma unroll
+      for (int v = 0; v < AHEAD; ++v) fetch(v, u & 1);
+      __builtin_amdgcn_sched_barrier(0);
+    }
 #pragma unroll
     for (int v = 0; v < MT; ++v) {
-      StreamK f;
-      f.v[0] = *reinterpret_cast<const bf16x8_t*>(base + v * 16 * ROW);
-      f.v[1] = *reinterpret_cast<const bf16x8_t*>(base + v * 16 * ROW + 64);
+      if (mine && v + AHEAD < MT) fetch(v + AHEAD, u & 1);
 #pragma unroll
-      for (int t = 0; t < NT; ++t) acc[t][v] = stream_mma(w[u][t], f, acc[t][v]);
+      for (int t = v * XU / MT; t < (v + 1) * XU / MT; ++t) {
+        if (more) load_x(u, t, min(i + u + D, its - 1));
+        put((u + 1) % D, t, (u + 1) & 1);
+      }
+#pragma unroll
+      for (int t = v * NT / MT; t < (v + 1) * NT / MT; ++t)
+        if (more) load_w((u + U) % D, t, min(i + u + U, its - 1));
+      __builtin_amdgcn_sched_barrier(0);
+      if (mine) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int t = 0; t < NT; ++t) acc[t][v] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[u][t].v[h], f[v % (AHEAD + 1)].v[h], acc[t][v], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
   };
   if (its > 0) {
     // One barrier a step: the next step's x is written while this one's is read; the buffer it goes to was last read
     // in front of the previous barrier.
 #pragma unroll
-    for (int u = 0; u < D; ++u) load(u, min(u, its - 1));
+    for (int u = 0; u < D; ++u) {
+#pragma unroll
+      for (int t = 0; t < XU; ++t) load_x(u, t, min(u, its - 1));
+      if (u < D - 1) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t) load_w(u, t, min(u, its - 1));
+      }
+    }
     __builtin_amdgcn_sched_barrier(0);
-    put(0, 0);
+#pragma unroll
+    for (int t = 0; t < XU; ++t) put(0, t, 0);
     lds_barrier();
     int i = 0;
     for (; i + D < its; i += D) {
 #pragma unroll
       for (int u = 0; u < D; ++u) {
-        put((u + 1) % D, (u + 1) & 1);
-        multiply(u, u & 1);
-        __builtin_amdgcn_sched_barrier(0);
-        load(u, min(i + u + D, its - 1));
-        __builtin_amdgcn_sched_barrier(0);
+        step(u, i, true, true);
         lds_barrier();
       }
     }
 #pragma unroll
+    for (int t = 0; t < NT; ++t) load_w(D - 1, t, min(i + D - 1, its - 1));
+#pragma unroll
     for (int u = 0; u < D; ++u) {
       if (i + u < its) {
-        put((u + 1) % D, (u + 1) & 1);
-        if ((i + u) * WK + kg < cnt) multiply(u, u & 1);
+        step(u, i, (i + u) * WK + kg < cnt, false);
         lds_barrier();
       }
     }
@@ -329,6 +364,7 @@ static int stream_shape(const slm_linear_args& a, hipStream_t st) {
     return wide ? wave_n_launch<2, 2, 1, 4, EPI>(a, st) : wave_n_launch<2, 1, 2, 4, EPI>(a, st);
   }
   if (a.M <= 64) return wide ? wave_n_launch<4, 2, 1, 4, EPI>(a, st) : wave_n_launch<4, 1, 1, 4, EPI>(a, st);
+  if (a.M <= 96) return wide ? wave_n_launch<6, 2, 1, 4, EPI>(a, st) : wave_n_launch<6, 1, 1, 4, EPI>(a, st);
   return wide ? wave_n_launch<8, 2, 2, 2, EPI>(a, st) : wave_n_launch<8, 1, 1, 4, EPI>(a, st);
 }
 

@@ -133,6 +133,13 @@ def test_streamed_products_of_many_steps(M, N, K):
     _streamed_products(M, N, K)
 
 
+# The edges of the 96-row tiles, with columns that make them narrow and wide, and step counts below, at and past their ring.
+@pytest.mark.parametrize("M", [80, 96, 97])
+@pytest.mark.parametrize("N,K", [(80, 192), (2048, 320), (16896, 256), (28672, 704), (1024, 8256)])
+def test_streamed_products_of_96_row_tiles(M, N, K):
+    _streamed_products(M, N, K)
+
+
 def _streamed_products(M, N, K):
     lk = _lk()
     x = _rnd(1, M, K + 8, dtype=torch.bfloat16)[:, :K]
