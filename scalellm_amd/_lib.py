@@ -296,6 +296,7 @@ def latent_lib() -> C.CDLL:
         ("slm_latent_append_absorb", C.c_int, [P(LatentAppendArgs), P(LinearArgs), ptr]),
         ("slm_latent_attn_workspace_bytes", C.c_size_t, [P(LatentAttnArgs)]),
         ("slm_latent_attn", C.c_int, [P(LatentAttnArgs), ptr]),
+        ("slm_latent_attn_values", C.c_int, [P(LatentAttnArgs), P(LinearArgs), ptr]),
         ("slm_latent_attn_is_mfma", C.c_int, [i32, i32, i32]),
         ("slm_latent_gather", C.c_int, [ptr, ptr, ptr, i64, i64, ptr]),
         ("slm_latent_prefill", C.c_int, [P(LatentPrefillArgs), ptr]),

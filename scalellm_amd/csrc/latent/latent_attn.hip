@@ -23,11 +23,15 @@
 // 64 rows of 500 - 1000 keys 32.5 -> 30.6.  Ranges that are split leave fp32 partials for latent_attn_combine_kernel.
 //
 // latent_attn_any_kernel: any size, any dtype, VALU: the 32-bit path and sizes without an MFMA form.
+#include <algorithm>
+
 #include "latent_common.h"
+#include "tile_common.h"
 
 namespace slm {
 
 constexpr int LA_MAX_SPLITS = 128;
+constexpr int LA_VALUES_WEIGHTS = 512;   // rows and splits of a workgroup of latent_values_kernel
 
 struct LatentAttnK {
   slm_latent_attn_args a;
@@ -417,6 +421,110 @@ __global__ void __launch_bounds__(256) latent_attn_combine_kernel(const LatentAt
       u32x2{pack2<bf16_tag>(o.x, o.y), pack2<bf16_tag>(o.z, o.w)};
 }
 
+// The splits' merge and what is multiplied out behind it (W_uv and the output gate, v) in one launch.  A workgroup has rows_per rows of a
+// head, all their columns and up to 128 of the product's: the merged rows lie in LDS in 16-bit, W comes there by LDS-DMA while the splits are read, a
+// wave owns 16 columns.  16-byte chunk c of row r lies in slot c ^ (r & SW).
+// Bound: latency, and 130 - 190 KB a CU of splits and W.  With the attention in front of it, us, two launches / this, latent 512 -> 128, 4000 keys:
+// 16 heads 8 rows 21.7 / 20.2, 32 rows 40.0 / 36.7, 128 rows 111.6 / 104.0; 32 heads 4 rows 20.1 / 19.4, 32 rows 45.8 / 42.1, 128 rows 114.5 / 109.1.
+template <int KP>
+__global__ void __launch_bounds__(512) latent_values_kernel(const LatentAttnK p, const slm_linear_args v, const int rows_per) {
+  constexpr int C4 = KP / 4, PH = 512 / C4, SW = KP >= 128 ? 15 : 7, U = 8;
+  __shared__ __attribute__((aligned(16))) char merged[16 * KP * 2];
+  __shared__ float weight[LA_VALUES_WEIGHTS], total[16];
+  __shared__ f32x4 part[PH][C4];
+  extern __shared__ __attribute__((aligned(16))) char w_lds[];   // [8 waves][16 columns][KP]
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, g = lane >> 4;
+  const int head = blockIdx.x, n = p.n_splits;   // (heads go round the XCDs: a head's workgroups share W in an L2)
+  const int64_t row0 = (int64_t)blockIdx.y * rows_per;
+  const int rows = (int)min((int64_t)rows_per, p.a.rows - row0);
+  auto pair = [&](int r) { return (row0 + r) * p.a.heads + head; };
+
+  // threads: column quad, and a row or (fewer rows than phases) a share of a row's splits
+  const int c4 = tid % C4, phase = tid / C4;
+  int row_phases = PH;
+  while (row_phases > 1 && row_phases / 2 >= rows) row_phases /= 2;
+  const int shares = PH / row_phases, sg = phase / row_phases, r_first = phase % row_phases;
+  const int per_row = (n + shares - 1) / shares, items = (rows + row_phases - 1) / row_phases * per_row;
+  auto split = [&](int i) { return sg + i % per_row * shares; };
+  auto load = [&](int i) {
+    const int r = min(r_first + i / per_row * row_phases, rows - 1), s = min(split(i), n - 1);
+    return *reinterpret_cast<const f32x4*>(p.o_part + (pair(r) * n + s) * KP + 4 * c4);
+  };
+  f32x4 x[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) x[u] = load(min(u, items - 1));
+
+  // rows wave, wave + 8: two splits a lane
+  for (int r = wave; r < rows; r += 8) {
+    const float* ml = p.ml_part + 2 * pair(r) * n;
+    const float m0 = lane < n ? ml[2 * lane] : M_INIT_F, m1 = lane + 64 < n ? ml[2 * lane + 128] : M_INIT_F;
+    const float l0 = lane < n ? ml[2 * lane + 1] : 0.f, l1 = lane + 64 < n ? ml[2 * lane + 129] : 0.f;
+    const float m = wave_max(fmaxf(m0, m1)), e0 = fast_exp2(m0 - m), e1 = fast_exp2(m1 - m), l = wave_sum(l0 * e0 + l1 * e1);
+    if (lane < n) weight[r * n + lane] = e0;
+    if (lane + 64 < n) weight[r * n + lane + 64] = e1;
+    if (lane == 0) total[r] = 1.0f / l;
+  }
+  const int64_t n0 = ((int64_t)blockIdx.z * 8 + wave) * 16;
+  const bool columns = n0 < v.N;
+  char* const mine = w_lds + wave * (16 * KP * 2);
+  if (columns) {
+    const char* const w = reinterpret_cast<const char*>(v.w) + (head * v.w_batch + n0 * KP) * 2;
+    const uint32_t dst0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)mine;
+#pragma unroll
+    for (int i = 0; i < KP / 32; ++i) {
+      const int r = (i * 1024 + lane * 16) / (KP * 2), c = (lane * 16) % (KP * 2) / 16;
+      const uint32_t off = (uint32_t)(r * (KP * 2) + ((c ^ (r & SW)) << 4)), dst = dst0 + i * 1024;
+      asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %2" : : "v"(off), "s"(dst), "s"(w) : "memory", "m0");
+    }
+  }
+  __syncthreads();
+  auto keep = [&](int r, f32x4 o) {
+    o *= total[r];
+    *reinterpret_cast<u32x2*>(merged + r * (KP * 2) + (((c4 >> 1) ^ (r & SW)) << 4) + (c4 & 1) * 8) = u32x2{pack2<bf16_tag>(o.x, o.y), pack2<bf16_tag>(o.z, o.w)};
+  };
+  f32x4 o = {0.f, 0.f, 0.f, 0.f};
+  for (int i0 = 0; i0 < items; i0 += U) {
+    if (i0 > 0) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) x[u] = load(min(i0 + u, items - 1));
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int i = i0 + u, r = r_first + i / per_row * row_phases, s = split(i);
+      if (i < items && r < rows) {
+        if (s < n) o += x[u] * weight[r * n + s];
+        if (shares == 1 && i % per_row == per_row - 1) {
+          keep(r, o);
+          o = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+      }
+    }
+  }
+  if (shares > 1) {
+    part[phase][c4] = o;
+    __syncthreads();
+    if (sg == 0 && r_first < rows) {
+      for (int s = 1; s < shares; ++s) o += part[s * row_phases + r_first][c4];
+      keep(r_first, o);
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (a wave's own columns)
+  __syncthreads();
+  if (!columns) return;
+  f32x4 y[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+  for (int s = 0; s < KP / 32; ++s) {
+    const int at = r16 * (KP * 2) + (((4 * s + g) ^ (r16 & SW)) << 4);
+    y[s & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8_t*>(mine + at), *reinterpret_cast<const bf16x8_t*>(merged + at), y[s & 1], 0, 0, 0);
+  }
+  if (r16 >= rows) return;
+  const int64_t row = row0 + r16;
+  f32x4 out = y[0] + y[1];
+  if (v.epilogue == SLM_LIN_GATE) out *= sigmoid_f32(to_f32(reinterpret_cast<const bf16*>(v.gate)[row * v.ld_gate + head]));
+  *reinterpret_cast<u32x2*>(reinterpret_cast<bf16*>(v.y) + head * v.y_batch + row * v.ldy + n0 + 4 * g) =
+      u32x2{pack2<bf16_tag>(out.x, out.y), pack2<bf16_tag>(out.z, out.w)};
+}
+
 static void la_combine(const LatentAttnK& p, hipStream_t st) {
   const int64_t quads = p.a.rows * p.a.heads * (p.a.c_pad / 4);
   if (p.n_splits <= 8) latent_attn_combine_kernel<1><<<dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, st>>>(p);
@@ -517,6 +625,27 @@ static int la_splits(const slm_latent_attn_args& a) {
   return n < 1 ? 1 : (int)n;
 }
 
+template <int KP>
+static void la_values_launch(const LatentAttnK& p, const slm_linear_args& v, int rows_per, hipStream_t st) {
+  constexpr int bytes = 8 * 16 * KP * 2;
+  auto fn = latent_values_kernel<KP>;
+  static bool asked[64] = {};
+  tile_allow_lds(fn, bytes, asked);
+  fn<<<dim3((unsigned)p.a.heads, (unsigned)((p.a.rows + rows_per - 1) / rows_per), (unsigned)((v.N + 127) / 128)), dim3(512), bytes, st>>>(p, v, rows_per);
+}
+// Rows of a head per workgroup, as many as leave one round of workgroups; 0: two launches.  Those where there are fewer than 128 pairs of row and head: one
+// row's 128 splits are then a quarter of a megabyte for each of few workgroups, where the merge by itself spreads them over the chip (1 row, 32 heads:
+// 9.4 us the two).
+static int la_values_rows(const LatentAttnK& p, const slm_linear_args& v) {
+  const slm_latent_attn_args& a = p.a;
+  if (v.x != a.out || v.M != a.rows || v.K != a.c_pad || v.ldw != v.K || v.x_batch != a.c_pad || v.ldx != (int64_t)a.heads * a.c_pad || v.batch != a.heads ||
+      v.dtype != SLM_BF16 || v.y_batch % 4 || v.ldy % 4 || (uintptr_t)v.y % 8 || v.w_batch % 8)
+    return 0;
+  const int64_t pairs = a.rows * a.heads;
+  const int64_t r = std::min<int64_t>(16, (pairs + 255) / 256);
+  return pairs >= 128 * r && r * p.n_splits <= LA_VALUES_WEIGHTS && (a.rows + r - 1) / r <= 65535 ? (int)r : 0;
+}
+
 template <int KP, int RP, int MH>
 static void la_launch(const LatentAttnK& p, hipStream_t st) {
   const int hblocks = (p.a.heads + 16 * MH - 1) / (16 * MH);
@@ -558,7 +687,7 @@ extern "C" SLM_API size_t slm_latent_attn_workspace_bytes(const slm_latent_attn_
   const int n = la_splits(*a);
   return n <= 1 ? 0 : (size_t)a->rows * a->heads * n * (a->c_pad + 2) * 4;
 }
-extern "C" SLM_API int slm_latent_attn(const slm_latent_attn_args* a, void* stream) {
+static int la_run(const slm_latent_attn_args* a, const slm_linear_args* v, void* stream) {
   const int rc = la_check(a);
   if (rc != SLM_OK) return rc;
   if (!a->q_abs || !a->cache || !a->out || !a->positions || !a->q_cu || !a->block_table || !a->block_cu) return SLM_ERR_INVALID_ARG;
@@ -589,12 +718,33 @@ extern "C" SLM_API int slm_latent_attn(const slm_latent_attn_args* a, void* stre
       case 256: la_rot<256>(p, st); break;
       default: la_rot<512>(p, st);
     }
-    if (p.n_splits > 1) la_combine(p, st);
+    if (p.n_splits > 1) {
+      const int rows = v ? la_values_rows(p, *v) : 0;
+      if (rows) {
+        switch (a->c_pad) {
+          case 64: la_values_launch<64>(p, *v, rows, st); break;
+          case 128: la_values_launch<128>(p, *v, rows, st); break;
+          case 256: la_values_launch<256>(p, *v, rows, st); break;
+          default: la_values_launch<512>(p, *v, rows, st);
+        }
+        return hip_check_launch();
+      }
+      la_combine(p, st);
+    }
   } else {
     const dim3 grid((unsigned)(a->rows * a->heads));
     const size_t lds = (size_t)(a->c_pad + a->r_pad) * 4;
     if (a->dtype == SLM_BF16) latent_attn_any_kernel<bf16><<<grid, dim3(256), lds, st>>>(p);
     else latent_attn_any_kernel<float><<<grid, dim3(256), lds, st>>>(p);
   }
-  return hip_check_launch();
+  const int rl = hip_check_launch();
+  return rl != SLM_OK || !v ? rl : slm_linear(v, stream);
+}
+extern "C" SLM_API int slm_latent_attn(const slm_latent_attn_args* a, void* stream) { return la_run(a, nullptr, stream); }
+extern "C" SLM_API int slm_latent_attn_values(const slm_latent_attn_args* a, const slm_linear_args* v, void* stream) {
+  if (!v || !v->w || !v->y || v->M < 0 || v->N <= 0 || v->N % 16 || v->n_splits != 1 || (v->epilogue != SLM_LIN_STORE && v->epilogue != SLM_LIN_GATE) ||
+      (v->epilogue == SLM_LIN_GATE && !v->gate))
+    return SLM_ERR_INVALID_ARG;
+  if (!aligned16(v->w)) return SLM_ERR_ALIGNMENT;
+  return la_run(a, v, stream);
 }

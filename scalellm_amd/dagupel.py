@@ -3,8 +3,8 @@ residual stream, with learned positions and layers that may share another layer'
 
 The step function is the framework's: forward(tokens, positions, InputParameters) over a paged cache, driven by
 ModelRunner (graphs for decode batches) and engine.LLMEngine.  Launches of a decode layer: projection, append
-(latent norm + rotation + cache write), absorbed query product, attention (+ merge of its splits), value product with
-the output gate, output projection (split-K slabs), add + norm, gate_up with the activation, down (slabs), add + norm.
+(latent norm + rotation + cache write) with the absorbed query product, attention, merge of its splits with the value product and the
+output gate, output projection (split-K slabs), add + norm, gate_up with the activation, down (slabs), add + norm.
 """
 from __future__ import annotations
 

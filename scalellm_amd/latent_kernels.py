@@ -398,16 +398,20 @@ def _heads_args(x: torch.Tensor, x_head: int, w: torch.Tensor, out: torch.Tensor
     return a
 
 
-def linear_heads(x: torch.Tensor, x_head: int, w: torch.Tensor, out: torch.Tensor, out_head: int,
-                 gate: Optional[torch.Tensor] = None) -> None:
-    """Per-head products: head h of `out` (columns from h * out_head) = columns from h * x_head of x times w[h]^T;
-    w [heads, N, K].  gate [rows, >= heads]: the result is multiplied by sigmoid(gate[:, h])."""
+def _gated_heads(x, x_head, w, out, out_head, gate) -> "_lib.LinearArgs":
     a = _heads_args(x, x_head, w, out, out_head)
     if gate is not None:
         M, H = x.size(0), w.size(0)
         _need(gate.size(0) == M and gate.size(1) >= H and gate.stride(1) == 1 and gate.dtype == x.dtype, "linear_heads: gate")
         a.epilogue, a.gate, a.ld_gate = _lib.LIN_GATE, _p(gate), gate.stride(0)
-    _run_linear(a)
+    return a
+
+
+def linear_heads(x: torch.Tensor, x_head: int, w: torch.Tensor, out: torch.Tensor, out_head: int,
+                 gate: Optional[torch.Tensor] = None) -> None:
+    """Per-head products: head h of `out` (columns from h * out_head) = columns from h * x_head of x times w[h]^T;
+    w [heads, N, K].  gate [rows, >= heads]: the result is multiplied by sigmoid(gate[:, h])."""
+    _run_linear(_gated_heads(x, x_head, w, out, out_head, gate))
 
 
 def latent_append(proj: torch.Tensor, cache: torch.Tensor, q_abs: Optional[torch.Tensor], norm_weight: torch.Tensor,
@@ -440,8 +444,9 @@ def latent_append(proj: torch.Tensor, cache: torch.Tensor, q_abs: Optional[torch
 
 def latent_attention(q_abs: torch.Tensor, cache: torch.Tensor, out: torch.Tensor, positions: torch.Tensor, q_cu: torch.Tensor,
                      block_table: torch.Tensor, block_cu: torch.Tensor, *, block_size: int, window: int, scale: float,
-                     max_kv_len: int, n_splits: int = 0, generic: bool = False) -> None:
-    """out[row, head] = soft-max(q_abs . cache rows * scale) weighted latent over the row's visible positions."""
+                     max_kv_len: int, n_splits: int = 0, generic: bool = False, values: Optional[tuple] = None) -> None:
+    """out[row, head] = soft-max(q_abs . cache rows * scale) weighted latent over the row's visible positions.  values = (w, y, y_head, gate):
+    then linear_heads() of it, w [heads, N, c_pad]; `out` is scratch."""
     rows, heads, R = q_abs.shape
     c_pad = out.size(2)
     _need(q_abs.is_contiguous() and out.is_contiguous() and out.shape[:2] == q_abs.shape[:2] and cache.size(1) == R and
@@ -462,7 +467,12 @@ def latent_attention(q_abs: torch.Tensor, cache: torch.Tensor, out: torch.Tensor
     if need:
         ws = reserve_workspace(need, q_abs.device)
         a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
-    latent_check(L.slm_latent_attn(C.byref(a), _stream()), "slm_latent_attn")
+    if values is None:
+        latent_check(L.slm_latent_attn(C.byref(a), _stream()), "slm_latent_attn")
+        return
+    w, y, y_head, gate = values
+    v = _gated_heads(out.view(rows, -1), c_pad, w, y, y_head, gate)
+    latent_check(L.slm_latent_attn_values(C.byref(a), C.byref(v), _stream()), "slm_latent_attn_values")
 
 
 def latent_gather(cache: torch.Tensor, slots: torch.Tensor) -> torch.Tensor:

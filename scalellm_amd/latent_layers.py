@@ -215,8 +215,7 @@ class LatentAttention:
             lat = proj.new_empty(n_tok, a.heads, self.c_pad)
             lk.latent_attention(q_abs, cache.rows, lat, positions, params.q_cu_seq_lens, params.block_tables,
                                 params.cu_block_lens, block_size=cache.block_size(), window=a.window, scale=a.scale,
-                                max_kv_len=params.kv_max_seq_len)
-            lk.linear_heads(lat.view(n_tok, -1), self.c_pad, self.w_uv, out[:n_tok], self.v_pad, gate=pt[:, self.off_g:])
+                                max_kv_len=params.kv_max_seq_len, values=(self.w_uv, out[:n_tok], self.v_pad, pt[:, self.off_g:]))
         if portions:
             plan = params.plans.get(a.window)
             if plan is None:

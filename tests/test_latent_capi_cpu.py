@@ -72,6 +72,12 @@ def test_invalid_arguments_come_back_as_status():
     assert L.slm_latent_attn(C.byref(b), None) == -1
     b.block_size, b.dtype = 16, 0
     assert L.slm_latent_attn(C.byref(b), None) == -2
+    v = _lib.LinearArgs()
+    assert L.slm_latent_attn_values(C.byref(b), None, None) == L.slm_latent_attn_values(C.byref(b), C.byref(v), None) == -1
+    v.w, v.y, v.N, v.n_splits, v.epilogue = 4104, 4096, 64, 1, _lib.LIN_STORE
+    assert L.slm_latent_attn_values(C.byref(b), C.byref(v), None) == -5
+    v.w, v.epilogue = 4096, _lib.LIN_GATE
+    assert L.slm_latent_attn_values(C.byref(b), C.byref(v), None) == -1   # no gate
     assert L.slm_latent_gather(None, None, None, 1, 64, None) == -1
     for args in ((None, 4096, 64, 64, 0), (4096, 4096, 72, 64, 0), (4096, 4096, 64, 72, 0), (4096, 4096, 96, 64, 1)):
         assert L.slm_stream_layout(*args, None) == -1

@@ -430,6 +430,32 @@ def test_latent_attention_sizes(c_pad, r_pad, heads, dtype):
             _close(out, want, dtype, f32=1e-5, b16=1.5e-2)
 
 
+# The merge and the product behind it in one launch against the two: rows that leave the last workgroup of a head short, one row a workgroup and
+# sixteen, splits by the rule and forced (few rows: two launches), columns below, at and past a workgroup's 128, with the gate and without.  The merged
+# rows are rounded to 16 bits either way; another order of the splits' sums moves a rounding now and then, so 2^-8 of a few of a product's terms.
+@pytest.mark.parametrize("c_pad,heads,vdim,rows,n_splits", [
+    (512, 16, 128, 9, 0), (512, 32, 128, 33, 0), (512, 32, 128, 4, 0), (512, 16, 128, 1, 0), (512, 24, 144, 100, 2), (256, 40, 96, 30, 3),
+    (256, 16, 32, 33, 0), (128, 48, 64, 31, 5), (64, 17, 48, 90, 8), (64, 64, 16, 127, 2), (512, 128, 128, 1, 128), (64, 160, 32, 2, 100)])
+def test_latent_attention_with_its_values(c_pad, heads, vdim, rows, n_splits):
+    lk, r_pad, dt = _lk(), 64, torch.bfloat16
+    lens = [40 + 53 * i % 700 for i in range(rows)]
+    pg = Paged(lens, 16, c_pad, r_pad, dt)
+    q = _rnd(1, rows, heads, c_pad + r_pad, dtype=dt)
+    w, gate = _rnd(2, heads, vdim, c_pad, dtype=dt, std=c_pad ** -0.5), _rnd(3, rows, heads + 3, dtype=dt)
+    where = (pg.dev([n - 1 for n in lens]), pg.dev(range(rows + 1)), pg.dev(pg.table), pg.dev(pg.cu))
+    kw = dict(block_size=16, window=0, scale=0.1, max_kv_len=max(lens), n_splits=n_splits)
+    for g in (None, gate):
+        lat = torch.empty(rows, heads, c_pad, dtype=dt, device=DEV)
+        got, want = (torch.full((rows, heads * (vdim + 4) + 8), 7.0, dtype=dt, device=DEV) for _ in range(2))
+        lk.latent_attention(q, pg.cache, lat, *where, values=(w, got, vdim + 4, g), **kw)
+        lk.latent_attention(q, pg.cache, lat, *where, **kw)
+        lk.linear_heads(lat.view(rows, -1), c_pad, w, want, vdim + 4, gate=g)
+        _close(got, _f64(want), dt, b16=1e-2)
+        assert float((got.float() - want.float()).norm() / want.float().norm()) < 2e-3
+        assert (got.view(-1)[:1] != 7).all() and (got[:, heads * (vdim + 4):] == 7).all()
+        assert (got[:, :heads * (vdim + 4)].view(rows, heads, vdim + 4)[:, :, vdim:] == 7).all()
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_latent_attention_sees_exactly_its_window(dtype):
     """One key that outweighs all others: present at distance window - 1, gone at distance window."""
