@@ -11,9 +11,9 @@
 //            latency of its inputs, which are loaded before the first is used, and the records it writes (2 TB/s).
 //   scan     portions: chunk after chunk.  The columns of S are independent, so a workgroup owns 16 of them and keeps them
 //            in registers from the portion's first token to its last; the products are 32-bit MFMAs.  Bound: a chain of two products and an
-//            exchange a chunk, 0.7 us, and the instructions around them.
+//            exchange a chunk, 0.6 us, and the instructions around them.
 //   Both, us, 16 heads of 128 x 128 and 4096 tokens: delta 305 with the triangular system and B U in the scan, 64-bit addresses and a wave's
-//   read-outs by itself, 262 now; lightning 184 and 163; 8 x 500 tokens, 32 heads: 341 and 309, 209 and 188; 16 heads of 64, 2000 tokens: 120 and 86.
+//   read-outs by itself, 239 now; lightning 184 and 134; 8 x 500 tokens, 32 heads: 341 and 309, 209 and 183; 16 heads of 64, 2000 tokens: 120 and 82.
 //   gated_norm  the norm and gate behind a scan.
 #include "latent/latent_common.h"
 #include "slm_mixers.h"
@@ -642,21 +642,20 @@ __global__ void __launch_bounds__(64 * W, 2) recurrent_scan_kernel(const slm_rec
   // a chunk's record is a buffer: a load is one instruction (of 64-bit addresses half of a chunk's 215 instructions were additions)
   const int rec_bytes = (int)at.size() * 4;
   const uint32_t off = (uint32_t)(lane * 16), koff = off + wave * (TPW * 1024), goff = (uint32_t)(g * 16 + wave * (TPW * 64) + ChunkRecord<DK>::GE * 4);
-  auto load = [&](int c, ChunkOperands<TPW, NCT>& x) {
-    const __amdgpu_buffer_rsrc_t rec = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(rec0 + c * rec_step), 0, rec_bytes, 0x00020000);
+  constexpr int PIECES = TPW * (DELTA ? 4 : 3) + 2 * NCT, SLOTS = 4 * ((DELTA ? 2 : 1) * NCT + 1);
+  auto record = [&](int c) { return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(rec0 + c * rec_step), 0, rec_bytes, 0x00020000); };
+  auto load = [&](const __amdgpu_buffer_rsrc_t& rec, ChunkOperands<TPW, NCT>& x, int k) {   // k-th of PIECES
     auto vec = [&](uint32_t at_lane, int from) { return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rec, at_lane, from, 0)); };
-#pragma unroll
-    for (int i = 0; i < TPW; ++i) {
-      if constexpr (DELTA) x.kd[i] = vec(koff + i * 1024, ChunkRecord<DK>::KD * 4);
-      x.qd[i] = vec(koff + i * 1024, ChunkRecord<DK>::QD * 4);
-      x.kr[i] = vec(koff + i * 1024, ChunkRecord<DK>::KR * 4);
-      x.ge[i] = vec(goff + i * 64, 0);
+    if (k < 2 * NCT) {
+      if (k % 2 == 0) x.v[k / 2] = vec(off, ChunkRecord<DK>::V * 4 + 1024 * ct[k / 2]);
+      else x.o0[k / 2] = vec(off, at.o0() * 4 + 1024 * ct[k / 2]);
+      return;
     }
-#pragma unroll
-    for (int j = 0; j < NCT; ++j) {
-      x.v[j] = vec(off, ChunkRecord<DK>::V * 4 + 1024 * ct[j]);
-      x.o0[j] = vec(off, at.o0() * 4 + 1024 * ct[j]);
-    }
+    const int i = (k - 2 * NCT) % TPW, what = (k - 2 * NCT) / TPW;
+    if (what == 0) x.ge[i] = vec(goff + i * 64, 0);
+    else if (what == 1) x.qd[i] = vec(koff + i * 1024, ChunkRecord<DK>::QD * 4);
+    else if (what == 2) x.kr[i] = vec(koff + i * 1024, ChunkRecord<DK>::KR * 4);
+    else x.kd[i] = vec(koff + i * 1024, ChunkRecord<DK>::KD * 4);
   };
   // the read-outs of a chunk, once every wave's part of them is there: of each lane's four rows a wave takes one (of 2 waves: two)
   const int o_row = a.heads * a.v_pad * 4;   // bytes
@@ -686,30 +685,45 @@ __global__ void __launch_bounds__(64 * W, 2) recurrent_scan_kernel(const slm_rec
       }
   };
   // two sums of tiles side by side: the products of one wait for each other
-  auto products = [&](const f32x4 (&x)[TPW], int j, f32x4 c) {
+  auto products = [&](const f32x4 (&x)[TPW], int j, f32x4 c, auto between) {
     f32x4 d = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
+    for (int r = 0; r < 4; ++r) {
 #pragma unroll
       for (int i = 0; i < TPW; ++i) {
         f32x4& to = i & 1 ? d : c;
         to = __builtin_amdgcn_mfma_f32_16x16x4f32(x[i][r], s[j][i][r], to, 0, 0, 0);
       }
+      between();
+    }
     return TPW > 1 ? c + d : c;
   };
-  auto chunk = [&](int c, const ChunkOperands<TPW, NCT>& x) {
+  // Chunk c; between its products the loads of chunk `later`, one at a time: the 40 of a workgroup all at once back up in the address unit, and
+  // the waves with them (4096 tokens, 16 heads: delta 187 -> 160 us, of 136 without loads; lightning 124 -> 103; 1000 tokens, 32 heads 51 -> 45, 34 -> 27).
+  auto chunk = [&](int c, const ChunkOperands<TPW, NCT>& x, int later, ChunkOperands<TPW, NCT>& xl, bool more) {
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     const int b = c & 1;
     f32x4 o[NCT], u[NCT], pu[NCT][W];
     ReadOuts y;
+    const __amdgpu_buffer_rsrc_t rec = record(later);
+    int slot = 0;
+    auto between = [&]() {
+      if (more) {
+#pragma unroll
+        for (int k = 0; k < PIECES; ++k)
+          if (k >= slot * PIECES / SLOTS && k < (slot + 1) * PIECES / SLOTS) load(rec, xl, k);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      ++slot;
+    };
     if constexpr (DELTA) {
 #pragma unroll
-      for (int j = 0; j < NCT; ++j) part_u[b][j][wave][lane] = products(x.kd, j, zero);
+      for (int j = 0; j < NCT; ++j) part_u[b][j][wave][lane] = products(x.kd, j, zero, between);
       __builtin_amdgcn_sched_barrier(0);
     }
     // (the read-outs' products run under the writes of the exchange, of two column tiles the second's under its reads)
 #pragma unroll
-    for (int j = 0; j < (NCT + 1) / 2; ++j) o[j] = products(x.qd, j, wave == 0 ? x.o0[j] : zero);
+    for (int j = 0; j < (NCT + 1) / 2; ++j) o[j] = products(x.qd, j, wave == 0 ? x.o0[j] : zero, between);
     __builtin_amdgcn_sched_barrier(0);
     lds_barrier();
     if constexpr (DELTA) {
@@ -721,7 +735,7 @@ __global__ void __launch_bounds__(64 * W, 2) recurrent_scan_kernel(const slm_rec
     collect(c - 1, y);   // (in front of the first chunk: of nothing, and not stored)
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int j = (NCT + 1) / 2; j < NCT; ++j) o[j] = products(x.qd, j, wave == 0 ? x.o0[j] : zero);
+    for (int j = (NCT + 1) / 2; j < NCT; ++j) o[j] = products(x.qd, j, wave == 0 ? x.o0[j] : zero, between);
     if constexpr (DELTA && NCT > 1) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int j = 0; j < NCT; ++j) {
@@ -736,25 +750,28 @@ __global__ void __launch_bounds__(64 * W, 2) recurrent_scan_kernel(const slm_rec
 #pragma unroll
       for (int i = 0; i < TPW; ++i) s[j][i] *= x.ge[i];
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
+    for (int r = 0; r < 4; ++r) {
 #pragma unroll
       for (int i = 0; i < TPW; ++i)
 #pragma unroll
         for (int j = 0; j < NCT; ++j) s[j][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.kr[i][r], u[j][r], s[j][i], 0, 0, 0);
+      between();
+    }
 #pragma unroll
     for (int j = 0; j < NCT; ++j) part_o[b][j][wave][lane] = o[j];
     finish(c - 1, y);
   };
   ChunkOperands<TPW, NCT> x[NB];
 #pragma unroll
-  for (int i = 0; i + 1 < NB; ++i) load(min(i, n_chunks - 1), x[i]);
+  for (int i = 0; i + 1 < NB; ++i) {
+    const __amdgpu_buffer_rsrc_t rec = record(min(i, n_chunks - 1));
+#pragma unroll
+    for (int k = 0; k < PIECES; ++k) load(rec, x[i], k);
+  }
   int c0 = 0;   // (whole rounds without a branch around the loads: a join would make every wait one for the youngest)
   for (; c0 + NB <= n_chunks; c0 += NB) {
 #pragma unroll
-    for (int i = 0; i < NB; ++i) {
-      load(min(c0 + i + NB - 1, n_chunks - 1), x[(i + NB - 1) % NB]);
-      chunk(c0 + i, x[i]);
-    }
+    for (int i = 0; i < NB; ++i) chunk(c0 + i, x[i], min(c0 + i + NB - 1, n_chunks - 1), x[(i + NB - 1) % NB], true);
   }
 #pragma unroll
   for (int i = 0; i + 1 < NB; ++i) {
@@ -762,7 +779,7 @@ __global__ void __launch_bounds__(64 * W, 2) recurrent_scan_kernel(const slm_rec
     for (int j = 0; j < NCT; ++j)
 #pragma unroll
       for (int t = 0; t < TPW; ++t) settle(s[j][t]);
-    if (c0 + i < n_chunks) chunk(c0 + i, x[i]);
+    if (c0 + i < n_chunks) chunk(c0 + i, x[i], 0, x[i], false);
   }
   lds_barrier();
   ReadOuts y;
