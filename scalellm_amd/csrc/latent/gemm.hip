@@ -13,14 +13,19 @@
 // instructions of a step at once back up in the address unit, and a wave alone on its SIMD stalls with them (on zeros 14 %
 // more).  256 x 256: 160 KB of LDS.
 //
+// A workgroup goes from tile to tile: the DMA of a tile's last steps brings the first stages of the next one, which so are there when the
+// epilogue ends.  That is 5 us of a tile's 97 (256 x 256, K 4096), but power takes most of it back: 5692 x 28672 x 4096 992 -> 978 us,
+// 4096 x 8512 x 2048 122 -> 118, 3226 x 16896 x 4096 358 -> 352, 5692 x 4096 x 14336 502 -> 498.  (Where it goes in the loop matters: sources chosen by
+// the step cost 3 % of every product; the steps come in parts instead.)
+//
 // Tiles that do not fill the last round of the chip are cut in K (slices > 1): every slice leaves fp32 sums past the caches, the last one
 // to arrive (a counter per tile) adds them up in slice order and stores.  Nobody waits for anybody.
 //
-// us by the device, vendor product (and the GLU's launch) / this, normal numbers: 5692 x 28672 x 4096 GLU 1073 / 1005 (1.33 PFLOP/s),
-// 5692 x 4096 x 14336 740 / 500, 5692 x 4096 x 4096 148 / 148, 3226 x 28672 x 4096 GLU 708 / 570, 3226 x 16896 x 4096 449 / 352, 4096 x 16384 x 2048 GLU
-// 230 / 219, 4096 x 8512 x 2048 155 / 121, 1000 x 4096 x 14336 134 / 108, 600 x 28672 x 4096 GLU 148 / 134, 300 x 4096 x 14336 70 / 63,
-// 207 x 16384 x 2048 GLU 31 / 24.  Behind the vendor product where its tiles fill whole rounds (8192^3 685 / 724, 4096^3 89 / 96), with one row of tiles
-// over large weights (129 x 28672 x 4096 56 / 70), and on short and narrow products (207 x 4096 x 4096 17.6 / 20.8, 207 x 3664 x 2048 11.1 / 14.6,
+// us by the device, vendor product (and the GLU's launch) / this, normal numbers: 5692 x 28672 x 4096 GLU 1073 / 978 (1.37 PFLOP/s),
+// 5692 x 4096 x 14336 740 / 497, 5692 x 4096 x 4096 149 / 146, 3226 x 28672 x 4096 GLU 708 / 560, 3226 x 16896 x 4096 449 / 351, 4096 x 16384 x 2048 GLU
+// 230 / 209, 4096 x 8512 x 2048 155 / 118, 1000 x 4096 x 14336 134 / 109, 600 x 28672 x 4096 GLU 148 / 134, 300 x 4096 x 14336 70 / 63,
+// 207 x 16384 x 2048 GLU 31 / 24.  Behind the vendor product where its tiles fill whole rounds (8192^3 691 / 728, 4096^3 89 / 96), with one row of tiles
+// over large weights (129 x 28672 x 4096 56 / 70), and on short and narrow products (207 x 4096 x 4096 17.6 / 20.1, 207 x 3664 x 2048 11.1 / 14.6,
 // 207 x 512 x 2048 8.4 / 15.3), which its callers take here for the sake of the host.
 #include "latent_common.h"
 #include "tile_common.h"
@@ -55,52 +60,70 @@ __global__ void __launch_bounds__(256, 1) gemm_kernel(const GemmK a) {
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r16 = lane & 15, g = lane >> 4, wm = wave & 1, wn = wave >> 1;
 
-  // (whole tiles: a multiple of 8 workgroups)
-  const int whole_wgs = (a.whole + 7) & ~7;
-  int t, slice = 0, own = -1;
-  if ((int)blockIdx.x < whole_wgs) {
-    t = xcd_run(blockIdx.x, a.whole);
-    if (t < 0) return;
-  } else {
-    const int u = xcd_run((int)blockIdx.x - whole_wgs, a.cut * a.slices);
-    if (u < 0) return;
-    own = u / a.slices;
-    slice = u - own * a.slices;
-    t = a.whole + own;
-  }
-  // `group` row blocks by columns: neighbours in a run share rows of x and of w in their L2
-  const int gsz = a.group * a.nb, gi = t / gsz, in = t - gi * gsz;
-  const int rows_in = min(a.group, a.mb - gi * a.group);
-  const int mb = gi * a.group + in % rows_in, nb = in / rows_in;
-  const int64_t half = a.N / 2;
-  const int64_t m0 = (int64_t)mb * BM, n0 = (int64_t)nb * (GLU ? BN / 2 : BN);
+  // What a workgroup does one after the other: items blockIdx.x, + gridDim.x, ..  (whole tiles: a multiple of 8 of them)
+  struct Item {
+    int m0, n0, slice, own, s0, steps;
+  };
+  const int whole_items = (a.whole + 7) & ~7, all = (int)(a.K >> 6);
+  auto item = [&](int v, Item& it) -> bool {
+    int t;
+    it.slice = 0;
+    it.own = -1;
+    it.s0 = 0;
+    it.steps = all;
+    if (v < whole_items) {
+      t = xcd_run(v, a.whole);
+      if (t < 0) return false;
+    } else {
+      const int u = xcd_run(v - whole_items, a.cut * a.slices);
+      if (u < 0) return false;
+      it.own = u / a.slices;
+      it.slice = u - it.own * a.slices;
+      t = a.whole + it.own;
+      const int per = (all + a.slices - 1) / a.slices;
+      it.s0 = it.slice * per;
+      it.steps = min(per, all - it.s0);   // (the plan leaves no slice empty)
+    }
+    // `group` row blocks by columns: neighbours in a run share rows of x and of w in their L2
+    const int gsz = a.group * a.nb, gi = t / gsz, in = t - gi * gsz;
+    const int rows_in = min(a.group, a.mb - gi * a.group);
+    it.m0 = (gi * a.group + in % rows_in) * BM;
+    it.n0 = in / rows_in * (GLU ? BN / 2 : BN);
+    return true;
+  };
+  Item cur, nxt;
+  if (!item(blockIdx.x, cur)) return;
+  const int half = (int)(a.N / 2);
 
   // instruction i of this wave brings 8 rows of 128 bytes (rows past the end: the last one, not stored)
   uint32_t off[ND];
-#pragma unroll
-  for (int i = 0; i < ND; ++i) {
-    const int r = (i < XD ? (wave * XD + i) : (wave * WD + i - XD)) * 8 + (lane >> 3);
-    const uint32_t k = (uint32_t)(((lane & 7) ^ (i < XD ? r & 7 : (r & 3) | ((r >> 1) & 4))) << 4);
+  auto offset = [&](int i, const Item& it, int l) {
+    const int r = (i < XD ? (wave * XD + i) : (wave * WD + i - XD)) * 8 + (l >> 3);
+    const uint32_t k = (uint32_t)(((l & 7) ^ (i < XD ? r & 7 : (r & 3) | ((r >> 1) & 4))) << 4);
     if (i < XD) {
-      off[i] = (uint32_t)min(m0 + r, a.M - 1) * a.ldx2 + k;
+      off[i] = (uint32_t)min(it.m0 + r, (int)a.M - 1) * a.ldx2 + k;
     } else if constexpr (GLU) {   // of a wave's BN / 2 columns half are of the gate, then the same of the up half
       const int q = r / (BN / 2), c = r % (BN / 2);
-      const int64_t n = min(n0 + q * (BN / 4) + c % (BN / 4), half - 1) + (c >= BN / 4 ? half : 0);
+      const int n = min(it.n0 + q * (BN / 4) + c % (BN / 4), half - 1) + (c >= BN / 4 ? half : 0);
       off[i] = (uint32_t)n * a.ldw2 + k;
     } else {
-      off[i] = (uint32_t)min(n0 + r, a.N - 1) * a.ldw2 + k;
+      off[i] = (uint32_t)min(it.n0 + r, (int)a.N - 1) * a.ldw2 + k;
     }
-  }
+  };
+#pragma unroll
+  for (int i = 0; i < ND; ++i) offset(i, cur, lane);
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
   const uint32_t xdst = lds0 + wave * (XD * 1024), wdst = lds0 + XS * XB + wave * (WD * 1024);
-  auto dma = [&](int i, int64_t kb, uint32_t at) {   // kb: byte offset in the rows, at: of the stage
+  auto dma = [&](int i, uint32_t kb, uint32_t at) {   // kb: byte offset in the rows, at: of the stage
     const uint32_t dst = (i < XD ? xdst + i * 1024 : wdst + (i - XD) * 1024) + at;
     const char* base = (i < XD ? a.x : a.w) + kb;
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %2" : : "v"(off[i]), "s"(dst), "s"(base) : "memory", "m0");
   };
-  const int all = (int)(a.K >> 6), per = own < 0 ? all : (all + a.slices - 1) / a.slices;
-  const int s0 = slice * per, steps = min(per, all - s0);   // (the plan leaves no slice empty)
-  auto kbytes = [&](int s) { return (int64_t)(s0 + min(s, steps - 1)) << 7; };   // (steps past the end load the last one again)
+  // (what is made of it is made where it stands: kept through the products it spills)
+  auto here = [](int l) {
+    asm volatile("" : "+v"(l));
+    return l;
+  };
 
   // Columns of a pair of tiles go to them by fours, so that a lane ends with eight neighbours.  Chunk c of a row of w lies in slot
   // c ^ (row % 4 + 4 (row / 8 % 2)): eight lanes read eight slots of either matrix.
@@ -111,17 +134,26 @@ __global__ void __launch_bounds__(256, 1) gemm_kernel(const GemmK a) {
     if (j < MT) fx[h][j] = *reinterpret_cast<const bf16x8_t*>(lds + xa + (xrow + 16 * j) * 128 + slot);
     else fw[h][j - MT] = *reinterpret_cast<const bf16x8_t*>(lds + XS * XB + wa + (wrow + 32 * ((j - MT) >> 1) + 4 * ((j - MT) & 1)) * 128 + slot);
   };
+  // (rows there and back: a product takes one operand of the one before it, which is 0.5 % of a large product's time)
+  auto turn = [](int q) { return q / MT % 2 ? MT - 1 - q % MT : q % MT; };
   f32x4 acc[NT][MT];
 #pragma unroll
   for (int n = 0; n < NT; ++n)
 #pragma unroll
     for (int m = 0; m < MT; ++m) acc[n][m] = f32x4{0.f, 0.f, 0.f, 0.f};
 
+  int v = blockIdx.x;
+  bool more = item(v + (int)gridDim.x, nxt);   // (then every item has more than WS steps)
+  // byte offsets in the rows of the step that x and w are loaded for; steps past the end of the last item load its last one again
+  uint32_t kx = (uint32_t)cur.s0 << 7, kw = kx, last = kx + ((uint32_t)(cur.steps - 1) << 7);
 #pragma unroll
-  for (int p = 0; p < WS; ++p)
+  for (int p = 0; p < WS; ++p) {
 #pragma unroll
     for (int i = 0; i < ND; ++i)
-      if (i >= XD || p < 2) dma(i, kbytes(p), p * (i < XD ? XB : WB));
+      if (i >= XD || p < 2) dma(i, i < XD ? kx : kw, p * (i < XD ? XB : WB));
+    if (p < 2) kx = min(kx + 128, last);
+    kw = min(kw + 128, last);
+  }
   asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"(ND + (WS - 2) * WD) : "memory");   // the first stages are there
 #pragma unroll
   for (int j = 0; j < R; ++j) {
@@ -129,55 +161,85 @@ __global__ void __launch_bounds__(256, 1) gemm_kernel(const GemmK a) {
     __builtin_amdgcn_sched_barrier(0);
   }
   uint32_t xa = 0, wa = 0, xl = 2 * XB;   // this step's stages, and the one that x is loaded to
-  int s = 0;   // (a loop of no steps would have the accumulators set up once more)
-  do {
-    const uint32_t xn = xa == (XS - 1) * XB ? 0 : xa + XB, wnext = wa == (WS - 1) * WB ? 0 : wa + WB;
-    const int64_t kx = kbytes(s + 2);
+  for (;;) {
+    // The last steps' DMA is the next item's first: it runs under the epilogue.  So the steps come in parts, w's sources change WS of them before
+    // the end, x's two.
+    int left = more ? cur.steps - WS : cur.steps, part = more ? WS : 1;
+    for (;;) {
+      do {
+        const uint32_t xn = xa == (XS - 1) * XB ? 0 : xa + XB, wnext = wa == (WS - 1) * WB ? 0 : wa + WB;
 #pragma unroll
-    for (int b = 0; b < R; ++b) {
+        for (int b = 0; b < R; ++b) {
 #pragma unroll
-      for (int i = b * XD / R; i < (b + 1) * XD / R; ++i) dma(i, kx, xl);
-      read(b, 1, xa, wa);
+          for (int i = b * XD / R; i < (b + 1) * XD / R; ++i) dma(i, kx, xl);
+          read(b, 1, xa, wa);
 #pragma unroll
-      for (int q = b * MM / R; q < (b + 1) * MM / R; ++q) gemm_product(acc[q / MT][q % MT], fw[0][q / MT], fx[0][q % MT]);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(LATE) : "memory");
-    const int64_t kw = kbytes(s + WS);
+          for (int q = b * MM / R; q < (b + 1) * MM / R; ++q) gemm_product(acc[q / MT][turn(q)], fw[0][q / MT], fx[0][turn(q)]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(LATE) : "memory");
+        kx = min(kx + 128, last);
 #pragma unroll
-    for (int b = 0; b < R; ++b) {
-      if (b < WD) dma(XD + b, kw, wa);
-      read(b, 0, xn, wnext);
+        for (int b = 0; b < R; ++b) {
+          if (b < WD) dma(XD + b, kw, wa);
+          read(b, 0, xn, wnext);
 #pragma unroll
-      for (int q = b * MM / R; q < (b + 1) * MM / R; ++q) gemm_product(acc[q / MT][q % MT], fw[1][q / MT], fx[1][q % MT]);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    xl = xa;
-    xa = xn;
-    wa = wnext;
-  } while (++s < steps);
-  tile_settle(acc);
-  if (own >= 0 && !tile_add_slices(acc, a.slabs + (int64_t)own * a.slices * (MM * 1024), a.arrived + own, slice, a.slices, lds)) return;
-
-  // lane: columns 8 g .. + 7 of a pair of tiles, row r16 (worked out again: kept through the products they spill)
-  const int el = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), e16 = el & 15, eg = el >> 4;
+          for (int q = b * MM / R; q < (b + 1) * MM / R; ++q) gemm_product(acc[q / MT][turn(q)], fw[1][q / MT], fx[1][turn(q)]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        kw = min(kw + 128, last);
+        xl = xa;
+        xa = xn;
+        wa = wnext;
+      } while (--left > 0);
+      if (part == 1) break;
+      const int l = here(lane);
+      if (part == WS) {
+        last = (uint32_t)(nxt.s0 + nxt.steps - 1) << 7;
+        kw = (uint32_t)nxt.s0 << 7;
 #pragma unroll
-  for (int m = 0; m < MT; ++m) {
-    const int64_t row = m0 + wm * (BM / 2) + 16 * m + e16;
-    if (row >= a.M) continue;
-    bf16* y = a.y + row * a.ldy;
-#pragma unroll
-    for (int n = 0; n < (GLU ? NT / 2 : NT); n += 2) {
-      const int64_t col = n0 + wn * (GLU ? BN / 4 : BN / 2) + 16 * n + 8 * eg;
-      if (col >= (GLU ? half : a.N)) continue;
-      float v[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        v[j] = acc[n + (j >> 2)][m][j & 3];
-        if constexpr (GLU) v[j] = clamped_glu_f32(v[j], acc[n + (j >> 2) + NT / 2][m][j & 3], a.limit, a.alpha, a.shift);
+        for (int i = XD; i < ND; ++i) offset(i, nxt, l);
       }
-      store_f32<8>(y + col, v);
+      if (part == 2) {
+        kx = (uint32_t)nxt.s0 << 7;
+#pragma unroll
+        for (int i = 0; i < XD; ++i) offset(i, nxt, l);
+      }
+      left = part == 2 ? 2 : 1;
+      --part;
     }
+    if (!more) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    tile_products_settle(acc);
+    if (cur.own >= 0 && !tile_add_slices(acc, a.slabs + (int64_t)cur.own * a.slices * (MM * 1024), a.arrived + cur.own, cur.slice, a.slices, lds)) return;
+
+    // lane: columns 8 g .. + 7 of a pair of tiles, row r16
+    const int el = here(lane), e16 = el & 15, eg = el >> 4;
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+      const int row = cur.m0 + wm * (BM / 2) + 16 * m + e16;
+      bf16* y = a.y + row * a.ldy;
+#pragma unroll
+      for (int n = 0; n < (GLU ? NT / 2 : NT); n += 2) {
+        const int col = cur.n0 + wn * (GLU ? BN / 4 : BN / 2) + 16 * n + 8 * eg;
+        float o[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          o[j] = acc[n + (j >> 2)][m][j & 3];
+          if constexpr (GLU) o[j] = clamped_glu_f32(o[j], acc[n + (j >> 2) + NT / 2][m][j & 3], a.limit, a.alpha, a.shift);
+        }
+        if (row < a.M && col < (GLU ? half : (int)a.N)) store_f32<8>(y + col, o);
+      }
+#pragma unroll
+      for (int n = 0; n < NT; ++n) {
+        acc[n][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+        asm volatile("" : "+a"(acc[n][m]));
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (!more) return;
+    cur = nxt;
+    v += gridDim.x;
+    more = item(v + (int)gridDim.x, nxt);
   }
 }
 
@@ -250,7 +312,11 @@ static int gemm_launch(const GemmK& k, hipStream_t st) {
   auto fn = gemm_kernel<BM, BN, WS, GLU>;
   static bool asked[64] = {};
   tile_allow_lds(fn, bytes, asked);
-  const unsigned wgs = (unsigned)((k.whole + 7) / 8 * 8 + (k.cut * k.slices + 7) / 8 * 8);
+  // A workgroup goes from one to the next only where the shortest, the last slice, is long enough to load the next one's first stages, and a slice
+  // is the last of a workgroup's items (the plan's slices fill one round at most, behind whole ones).
+  const int parts = (k.cut * k.slices + 7) / 8 * 8, items = (k.whole + 7) / 8 * 8 + parts, all = (int)(k.K >> 6);
+  const int shortest = k.cut ? all - (all + k.slices - 1) / k.slices * (k.slices - 1) : all;
+  const unsigned wgs = (unsigned)(shortest > WS && items > GEMM_CUS && parts <= GEMM_CUS ? GEMM_CUS : items);
   fn<<<dim3(wgs), dim3(256), bytes, st>>>(k);
   return hip_check_launch();
 }

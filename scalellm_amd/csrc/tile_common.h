@@ -11,15 +11,21 @@ __device__ __forceinline__ int xcd_run(int wg, int n) {
   return i < per && t < n ? t : -1;
 }
 
-// Behind the last product: no DMA may outlive the workgroup's LDS, and the compiler knows nothing of products that inline asm made.  Whoever reads
-// an accumulator takes it from behind the wait.
+// Behind the last product: the compiler knows nothing of products that inline asm made.  Whoever reads an accumulator takes it from behind the wait.
 template <int NT, int MT>
-__device__ __forceinline__ void tile_settle(f32x4 (&acc)[NT][MT]) {
-  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_nop 15\n\ts_nop 7" ::: "memory");
+__device__ __forceinline__ void tile_products_settle(f32x4 (&acc)[NT][MT]) {
+  asm volatile("s_nop 15\n\ts_nop 7" ::: "memory");
 #pragma unroll
   for (int n = 0; n < NT; ++n)
 #pragma unroll
     for (int m = 0; m < MT; ++m) asm volatile("" : "+a"(acc[n][m]));
+}
+
+// The same where no DMA may outlive the workgroup's LDS
+template <int NT, int MT>
+__device__ __forceinline__ void tile_settle(f32x4 (&acc)[NT][MT]) {
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+  tile_products_settle(acc);
 }
 
 // The tile's fp32 sums go past the caches to its slabs, [slices][NT MT][256] f32x4; the last slice to arrive (*arrived, zero before) adds them up in
@@ -50,7 +56,10 @@ __device__ __forceinline__ bool tile_add_slices(f32x4 (&acc)[NT][MT], float* sla
         sum[f] += __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(mine, at(s, f0 + f), 0, /*sc1*/ 16));
     }
 #pragma unroll
-    for (int f = 0; f < C; ++f) acc[(f0 + f) / MT][(f0 + f) % MT] = sum[f];
+    for (int f = 0; f < C; ++f) {
+      acc[(f0 + f) / MT][(f0 + f) % MT] = sum[f];
+      asm volatile("" : "+a"(acc[(f0 + f) / MT][(f0 + f) % MT]));   // (one place for them: else what follows has a copy of all, in front of the branch too)
+    }
   }
   return true;
 }

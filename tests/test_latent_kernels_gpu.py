@@ -180,6 +180,14 @@ def test_tiled_products(M, N, K, slices, tile):
         assert glu[:, N // 2:].isnan().all()
 
 
+# More tiles than CUs, so that a workgroup goes from one to the next: steps at, one and two past the stages that are loaded ahead, two rounds and
+# three, a last round that is cut, also so that its last slice is at the stages (then a workgroup has one item, as with K 192 and three of them).
+@pytest.mark.parametrize("tile", range(7))
+@pytest.mark.parametrize("M,N,K,slices", [(2300, 7456, 192, 1), (2300, 7456, 256, 1), (2300, 7456, 320, 1), (1100, 16416, 704, 2), (2300, 8224, 576, 3)])
+def test_tiled_products_of_several_rounds(M, N, K, slices, tile):
+    test_tiled_products(M, N, K, slices, tile)
+
+
 @pytest.mark.parametrize("M", [129, 700])
 def test_products_of_prompts_by_the_planned_tile(M):
     lk, N, K = _lk(), 2080, 1024
