@@ -143,7 +143,8 @@ __device__ __forceinline__ float silu_mul1(const float g, const float u) {
 // stored) -> silu_mul1
 template <typename T>
 __device__ __forceinline__ float silu_mul_acc(const float gate_acc, const float up_acc) {
-  return silu_mul1(lo_f32<T>((uint32_t)pack1<T>(gate_acc)), lo_f32<T>((uint32_t)pack1<T>(up_acc)));
+  const uint32_t both = pack2<T>(gate_acc, up_acc);
+  return silu_mul1(lo_f32<T>(both), hi_f32<T>(both));
 }
 
 // 8 x silu_mul1, rounded RN to T

@@ -259,59 +259,88 @@ __global__ void __launch_bounds__(256, 1) w4_tile_kernel(const W4TileK a) {
   tile_settle(acc);
   if (a.slices > 1 && !tile_add_slices(acc, a.slabs + (int64_t)t * a.slices * (MM * 1024), a.arrived + t, slice, a.slices, lds)) return;
 
-  // Out through LDS, 64 rows at a time: a loop over rows then stores whole lines and applies the rest, in code short enough for the instruction
-  // cache (written out per accumulator this was 10000 instructions, and 13 us more of the 101 of a tile of 4096 of k).
+  // Out through LDS, 64 rows at a time, and from there in whole lines.  A wave has its own columns' rows to itself, so that their order alone is enough;
+  // of one packed tile a wave a pair's gate is in one wave, its up in the next, and they take half of the rows each.  Rows are read four at a
+  // time: one after the other, and with a bias added where there is none, 2183 x 4096 x 28672 with the SiLU took 430 us, 422 now, 2183 x 4096 x 4096 77
+  // and 75.4.  (Most of what is left, 6 us a tile, is the stores of all CUs at the same time.)
+  // (The code for 64 rows is there once, apart from the accumulators: written out per accumulator it was 10000 instructions, and 13 us more.)
   constexpr int CW = BN / 4, LR = CW * 4 + 16;       // columns of a wave, bytes of a row of them
   static_assert(4 * 64 * LR <= R0 + RS * RB, "LDS of 64 rows");
-  const bool pairs_of_waves = TW == 1 && a.silu;     // a pair's gate is in one wave, its up in the next: they take half of the rows each
-  const int from = pairs_of_waves ? wave & 2 : wave;
-  const int per_row = a.silu ? 4 : CW / 8;           // lanes of a row, eight columns each
-  const int row0 = lane / per_row + (pairs_of_waves ? (wave & 1) * 32 : 0), rows = (pairs_of_waves ? (wave & 1) * 32 + 32 : 64), by = 64 / per_row;
-  const int lcol = lane % per_row * 8;
-  const int64_t col = n0 + from * CW + lcol;
   char* const mine = lds + wave * (64 * LR) + r16 * LR + g * 32;
-  const char* const gate = lds + from * (64 * LR) + lcol * 4;
-  const char* const up = gate + (TW == 2 ? 128 : 64 * LR);
-  const bool inside = col < a.N;
-  float bias[2][8];
+  auto out = [&](auto with_silu, auto with_bias) __attribute__((always_inline)) {
+    constexpr bool SILU = decltype(with_silu)::value, BIAS = decltype(with_bias)::value, PAIRS = TW == 1 && SILU;
+    constexpr int PER_ROW = SILU ? 4 : CW / 8, BY = 64 / PER_ROW;   // lanes of a row, eight columns each; rows at a time
+    constexpr int TURNS = (PAIRS ? 32 : 64) / BY, AT_ONCE = TURNS < 4 ? TURNS : 4;
+    const int from = PAIRS ? wave & 2 : wave, lcol = lane % PER_ROW * 8, row0 = lane / PER_ROW + (PAIRS ? (wave & 1) * 32 : 0);
+    const int64_t col = n0 + from * CW + lcol;
+    const char* const gate = lds + from * (64 * LR) + lcol * 4 + row0 * LR;
+    const char* const up = gate + (TW == 2 ? 128 : 64 * LR);
+    const bool inside = col < a.N;
+    float bias[2][8];
+    if constexpr (BIAS) {
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    bias[0][j] = a.bias && inside ? lo_f32<bf16_tag>((uint32_t)a.bias[col + j]) : -0.f;   // (x + -0 is x)
-    bias[1][j] = a.bias && inside && a.silu ? lo_f32<bf16_tag>((uint32_t)a.bias[col + 32 + j]) : -0.f;
-  }
-  uint16_t* const c = a.c + (a.silu ? (col >> 6) * 32 + lcol : col);
-  auto sums = [&](const char* src, int half, float (&v)[8]) {
-    const f32x4 lo = *reinterpret_cast<const f32x4*>(src), hi = *reinterpret_cast<const f32x4*>(src + 16);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = (j < 4 ? lo[j & 3] : hi[j & 3]) + bias[half][j];
-  };
-#pragma unroll
-  for (int q = 0; q < BM / 64; ++q) {
-    __syncthreads();
-#pragma unroll
-    for (int m = 0; m < 4; ++m)
-#pragma unroll
-      for (int n = 0; n < NT; ++n) *reinterpret_cast<f32x4*>(mine + 16 * m * LR + (n >> 1) * 128 + (n & 1) * 16) = acc[n][4 * q + m];
+      for (int j = 0; j < 8; ++j) {
+        bias[0][j] = inside ? lo_f32<bf16_tag>((uint32_t)a.bias[col + j]) : 0.f;
+        bias[1][j] = inside && SILU ? lo_f32<bf16_tag>((uint32_t)a.bias[col + 32 + j]) : 0.f;
+      }
+    }
+    uint16_t* const c = a.c + (SILU ? (col >> 6) * 32 + lcol : col);
     __syncthreads();
 #pragma unroll 1
-    for (int r = row0; r < rows; r += by) {
-      const int64_t row = m0 + 64 * q + r;
-      if (row >= a.M || !inside) continue;
-      float v[8], u[8];
-      sums(gate + r * LR, 0, v);
-      if (a.silu) {
-        sums(up + r * LR, 1, u);
+    for (int q = 0; q < BM / 64; ++q) {
+      if (PAIRS && q > 0) __syncthreads();
+      in_turn<BM / 64>([&](auto which) __attribute__((always_inline)) {
+        constexpr int Q = which;
+        if (q == Q) {   // (different code to the compiler: one code for all of them would index the accumulators, in memory)
+          asm volatile("; rows from 64 * %0" : : "n"(Q));
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = silu_mul_acc<bf16_tag>(v[j], u[j]);
+          for (int m = 0; m < 4; ++m)
+#pragma unroll
+            for (int n = 0; n < NT; ++n) *reinterpret_cast<f32x4*>(mine + 16 * m * LR + (n >> 1) * 128 + (n & 1) * 16) = acc[n][4 * Q + m];
+          asm volatile("; rows from 64 * %0" : : "n"(Q));
+        }
+      });
+      if constexpr (PAIRS) __syncthreads();
+      else __builtin_amdgcn_wave_barrier();
+#pragma unroll 1
+      for (int i0 = 0; i0 < TURNS; i0 += AT_ONCE) {
+        f32x4 v[AT_ONCE][2], u[AT_ONCE][2];
+#pragma unroll
+        for (int i = 0; i < AT_ONCE; ++i)
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            v[i][h] = *reinterpret_cast<const f32x4*>(gate + (i0 + i) * (BY * LR) + 16 * h);
+            if constexpr (SILU) u[i][h] = *reinterpret_cast<const f32x4*>(up + (i0 + i) * (BY * LR) + 16 * h);
+          }
+#pragma unroll
+        for (int i = 0; i < AT_ONCE; ++i) {
+          const int64_t row = m0 + 64 * q + row0 + (i0 + i) * BY;
+          float y[8];
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            y[j] = v[i][j >> 2][j & 3];
+            if constexpr (BIAS) y[j] += bias[0][j];
+            if constexpr (SILU) {
+              float z = u[i][j >> 2][j & 3];
+              if constexpr (BIAS) z += bias[1][j];
+              y[j] = silu_mul_acc<bf16_tag>(y[j], z);
+            }
+          }
+          const u32x4 o = {pack2<bf16_tag>(y[0], y[1]), pack2<bf16_tag>(y[2], y[3]), pack2<bf16_tag>(y[4], y[5]), pack2<bf16_tag>(y[6], y[7])};
+          if (row < a.M && inside) {
+            uint16_t* const dst = c + row * a.ldc;
+            if (a.wide) *reinterpret_cast<u32x4*>(dst) = o;
+            else
+#pragma unroll
+              for (int j = 0; j < 8; ++j) dst[j] = (uint16_t)(o[j >> 1] >> (16 * (j & 1)));
+          }
+        }
       }
-      const u32x4 o = {pack2<bf16_tag>(v[0], v[1]), pack2<bf16_tag>(v[2], v[3]), pack2<bf16_tag>(v[4], v[5]), pack2<bf16_tag>(v[6], v[7])};
-      uint16_t* dst = c + row * a.ldc;
-      if (a.wide) *reinterpret_cast<u32x4*>(dst) = o;
-      else
-#pragma unroll
-        for (int j = 0; j < 8; ++j) dst[j] = (uint16_t)(o[j >> 1] >> (16 * (j & 1)));
+      if constexpr (!PAIRS) __builtin_amdgcn_wave_barrier();
     }
-  }
+  };
+  if (a.silu) a.bias ? out(std::true_type{}, std::true_type{}) : out(std::true_type{}, std::false_type{});
+  else a.bias ? out(std::false_type{}, std::true_type{}) : out(std::false_type{}, std::false_type{});
 }
 
 // Tiles, and what they take: us of a step of 64 k alone on the chip and with every CU busy (power), and of a tile beside its steps.
