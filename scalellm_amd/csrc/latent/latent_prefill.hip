@@ -2,56 +2,93 @@
 // a portion can see are gathered and multiplied by W_uk / W_uv once (a plain product), and the portion runs as
 // ordinary multi-head attention with unequal query / value widths, causal and windowed, output gate fused.
 //
-// Work item: one workgroup = (tile of 128 query rows of one sequence, head); four waves of 32 query rows.
-//   S^T[64 keys x 32 q] = K Q^T    v_mfma_f32_32x32x16_bf16, A = K rows from LDS (row stride an odd number of 16-byte
-//                                  units), B = Q rows in registers.  K row = unrotated part (per head) | rotated
-//                                  part (shared by the heads, out of the gathered latent rows)
-//   soft-max                       a lane holds 32 scores of ONE query row: register reductions + one lane-half exchange
-//   O^T[v x 32 q] += V^T P^T       P^T stays in registers: the C-fragment key order {4h + e, 8 + 4h + e} is used as the
-//                                  contraction order; V^T comes out of the row-major tile by the transpose read
-// The next tile travels global -> registers while this one is consumed.  Bound: MFMA.
-#include "latent_common.h"
+// Work item: one workgroup = (tile of 128 query rows of one sequence, head), prompt_attn.h.  K row = unrotated part (per head) |
+// rotated part (shared by the heads, out of the gathered latent rows).
+#include "prompt_attn.h"
 
 namespace slm {
-
-typedef short trp_v4 __attribute__((ext_vector_type(4)));
-typedef short trp_v8 __attribute__((ext_vector_type(8)));
-typedef __attribute__((address_space(3))) trp_v4 trp_lds_v4;
 
 struct LatentPrefillK {
   slm_latent_prefill_args a;
   float scale2;
 };
 
-template <int DQ, int VP>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+template <int DQ, int VP, int GROUPS, int KEYS>
+struct LatentWork {
+  const LatentPrefillK& p;
+  const int lane, group;
+  int ctx0, lo, hi, groups, n_turns, q_chunks;
+  int qpos, klo, wq0, wq1;          // in context indexes: the lane's row, the first key of its window; the wave's rows
+  const bf16 *kv, *ctx;
+  int kv_w, ctx_w;                  // bytes of a row
+
+  __device__ __forceinline__ int start_of(int turn) const { return lo + (groups * turn + group) * KEYS; }
+  __device__ __forceinline__ int row(int turn, int r) const { return ctx0 + min(start_of(turn) + r, hi - 1); }
+  __device__ __forceinline__ const void* key(int at, int c) const {
+    const bool own = c < q_chunks;                     // per head, or shared by the heads
+    return reinterpret_cast<const char*>((own ? kv : ctx - 8 * q_chunks) + 8 * c) + (int64_t)at * (own ? kv_w : ctx_w);
+  }
+  __device__ __forceinline__ const void* value(int at, int c) const {
+    return reinterpret_cast<const char*>(kv + 8 * (q_chunks + c)) + (int64_t)at * kv_w;
+  }
+  __device__ __forceinline__ void start() {}
+  __device__ __forceinline__ void begin(int) {}
+  __device__ __forceinline__ void end(int) {}
+  // tiles no row of the wave sees: past its diagonal, before its window
+  __device__ __forceinline__ bool seen(int turn) const {
+    const int k0 = start_of(turn);
+    return k0 <= wq1 && (p.a.window <= 0 || k0 + KEYS > wq0 - p.a.window + 1);
+  }
+  __device__ __forceinline__ void mask(int turn, f32x16 (&s)[KEYS / 32]) const {
+    const int k0 = start_of(turn);
+    if (k0 + KEYS - 1 <= wq0 && (p.a.window <= 0 || k0 >= wq1 - p.a.window + 1)) return;
+    const int at = k0 + 4 * (lane >> 5), last = qpos - at, from = klo - at;
+#pragma unroll
+    for (int n = 0; n < KEYS / 32; ++n)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int k = 32 * n + 8 * (r >> 2) + (r & 3);
+        s[n][r] = (k > last) | (k < from) ? -INFINITY : s[n][r];
+      }
+  }
+  __device__ __forceinline__ float score(float x) const { return x; }
+  __device__ __forceinline__ float top(float x) const { return x * p.scale2; }
+  __device__ __forceinline__ float below(float x, float m) const { return __builtin_fmaf(x, p.scale2, -m); }
+};
+
+template <int DQ, int VP, int GROUPS>
+__global__ void __launch_bounds__(256 * GROUPS) __attribute__((amdgpu_waves_per_eu(2)))
 latent_prefill_kernel(const LatentPrefillK p) {
-  constexpr int KT = 64;
-  constexpr int KLS = DQ * 2 + 16;
-  constexpr int VLS = VP * 2 + ((VP * 2) % 128 == 0 ? 64 : 0);
   constexpr int QS = DQ / 16, DT = VP / 32;
-  constexpr int KCH = DQ / 8, VCH = VP / 8;          // 16-byte chunks of a row
-  constexpr int NK = KT * KCH / 256, NV = KT * VCH / 256;
-  static_assert(KT * KCH % 256 == 0 && KT * VCH % 256 == 0, "whole chunks per thread");
-  __shared__ __attribute__((aligned(16))) char k_lds[KT * KLS];
-  __shared__ __attribute__((aligned(16))) char v_lds[KT * VLS];
+  // two workgroups on a CU, or two groups of waves: at most 80 KB each (256 + 128 columns: 112 us with 64 keys, 84 with 32)
+  constexpr int KEYS = DQ + VP > 320 ? 32 : 64;
+  __shared__ __attribute__((aligned(1024))) char lds[prompt_lds_bytes<DQ, VP, GROUPS, KEYS>()];
 
   const slm_latent_prefill_args& a = p.a;
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tid = threadIdx.x & 255, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int group = GROUPS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
   const int l31 = lane & 31, hh = lane >> 5;
   // heads fastest: the query tiles of one head stay on one XCD (heads % 8 == 0) and share its keys in L2;
   // tiles come longest first from the host
   const int head = blockIdx.x % a.heads;
   const int32_t* td = a.tiles + 6 * (blockIdx.x / a.heads);
   const int row0 = td[0], n_rows = td[1], ctx0 = td[2], ctx_len = td[3], ctx_pos = td[4], pos0 = td[5];
+  const int qi = min(wave * 32 + l31, n_rows - 1);     // this lane's query row
 
+  LatentWork<DQ, VP, GROUPS, KEYS> w{p, lane, group};
   // visible keys of the tile, as indexes into its context
-  int lo = 0, hi = min(ctx_len, pos0 + n_rows - ctx_pos);
-  if (a.window > 0) lo = max(0, pos0 - a.window + 1 - ctx_pos);
-  const int n_tiles = (hi - lo + KT - 1) / KT;
+  w.ctx0 = ctx0, w.lo = 0, w.hi = min(ctx_len, pos0 + n_rows - ctx_pos);
+  if (a.window > 0) w.lo = max(0, pos0 - a.window + 1 - ctx_pos);
+  const int n_tiles = (w.hi - w.lo + KEYS - 1) / KEYS;
+  w.groups = prompt_groups<GROUPS>(n_tiles), w.n_turns = (n_tiles + w.groups - 1) / w.groups;
+  w.q_chunks = a.q_dim / 8;
+  w.qpos = pos0 + qi - ctx_pos;
+  w.klo = a.window > 0 ? max(0, w.qpos - a.window + 1) : 0;
+  w.wq0 = pos0 - ctx_pos + min(wave * 32, n_rows - 1), w.wq1 = pos0 - ctx_pos + min(wave * 32 + 31, n_rows - 1);
+  w.kv = reinterpret_cast<const bf16*>(a.kv) + (int64_t)head * (a.q_dim + a.v_pad);
+  w.ctx = reinterpret_cast<const bf16*>(a.ctx) + a.c_pad;
+  w.kv_w = a.heads * (a.q_dim + a.v_pad) * 2, w.ctx_w = (a.c_pad + a.r_pad) * 2;
 
-  // this lane's query row
-  const int qi = min(wave * 32 + l31, n_rows - 1);
   const bf16* qrow = reinterpret_cast<const bf16*>(a.q) + (int64_t)(row0 + qi) * a.ld_q;
   bf16x8_t qf[QS];
   {
@@ -59,141 +96,18 @@ latent_prefill_kernel(const LatentPrefillK p) {
 #pragma unroll
     for (int s = 0; s < QS; ++s) qf[s] = *reinterpret_cast<const bf16x8_t*>(q + 16 * s);
   }
-  const int qpos = pos0 + qi - ctx_pos;  // in context indexes
-  const int klo = a.window > 0 ? max(0, qpos - a.window + 1) : 0;
-  // of the whole wave, for the tiles that need no mask
-  const int wq0 = pos0 - ctx_pos + min(wave * 32, n_rows - 1), wq1 = pos0 - ctx_pos + min(wave * 32 + 31, n_rows - 1);
-
-  const int q_chunks = a.q_dim / 8;
-  const int64_t ctx_w = a.c_pad + a.r_pad, kv_w = (int64_t)a.heads * (a.q_dim + a.v_pad);
-  const bf16* kv = reinterpret_cast<const bf16*>(a.kv) + (int64_t)head * (a.q_dim + a.v_pad);
-  const bf16* ctx = reinterpret_cast<const bf16*>(a.ctx) + a.c_pad;
-
-  u32x4 ks[NK], vs[NV];
-  auto load_tile = [&](int k0) {
-#pragma unroll
-    for (int i = 0; i < NK; ++i) {
-      const int idx = tid + 256 * i, r = idx / KCH, c = idx % KCH;
-      const int64_t key = ctx0 + min(k0 + r, hi - 1);
-      const bf16* src = c < q_chunks ? kv + key * kv_w + 8 * c : ctx + key * ctx_w + 8 * (c - q_chunks);
-      ks[i] = *reinterpret_cast<const u32x4*>(src);
-    }
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int idx = tid + 256 * i, r = idx / VCH, c = idx % VCH;
-      const int64_t key = ctx0 + min(k0 + r, hi - 1);
-      vs[i] = *reinterpret_cast<const u32x4*>(kv + key * kv_w + a.q_dim + 8 * c);
-    }
-  };
-  auto store_tile = [&]() {
-#pragma unroll
-    for (int i = 0; i < NK; ++i) {
-      const int idx = tid + 256 * i;
-      *reinterpret_cast<u32x4*>(k_lds + idx / KCH * KLS + idx % KCH * 16) = ks[i];
-    }
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int idx = tid + 256 * i;
-      *reinterpret_cast<u32x4*>(v_lds + idx / VCH * VLS + idx % VCH * 16) = vs[i];
-    }
-  };
-
   f32x16 o[DT];
-#pragma unroll
-  for (int d = 0; d < DT; ++d)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) o[d][r] = 0.f;
-  float m_run = M_INIT_F, l_run = 0.f;
-
-  // transpose read: key 4 hh + (lane % 16) / 4, columns 16 (lane / 16 % 2) + 4 (lane % 4)
-  const uint32_t tr_base = (uint32_t)(uintptr_t)v_lds +
-                           (uint32_t)((4 * hh + ((lane & 15) >> 2)) * VLS + ((lane >> 4) & 1) * 32 + (lane & 3) * 8);
-  const char* k_base = k_lds + l31 * KLS + hh * 16;
-
-  load_tile(lo);
-  for (int t = 0; t < n_tiles; ++t) {
-    const int k0 = lo + t * KT;
-    store_tile();
-    lds_barrier();
-    if (t + 1 < n_tiles) load_tile(k0 + KT);
-    // tiles no row of this wave sees (past its diagonal, before its window) are skipped
-    const bool seen = k0 <= wq1 && (a.window <= 0 || k0 + KT > wq0 - a.window + 1);
-    if (seen) {
-      f32x16 s[2];
-#pragma unroll
-      for (int n = 0; n < 2; ++n) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) s[n][r] = 0.f;
-#pragma unroll
-        for (int i = 0; i < QS; ++i)
-          s[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-              *reinterpret_cast<const bf16x8_t*>(k_base + 32 * n * KLS + 32 * i), qf[i], s[n], 0, 0, 0);
-      }
-      const bool inside = k0 + KT - 1 <= wq0 && (a.window <= 0 || k0 >= wq1 - a.window + 1);
-      if (!inside) {
-#pragma unroll
-        for (int n = 0; n < 2; ++n)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int key = k0 + 32 * n + 8 * (r >> 2) + 4 * hh + (r & 3);
-            if (key > qpos || key < klo) s[n][r] = -INFINITY;
-          }
-      }
-      float mx = s[0][0];
-#pragma unroll
-      for (int n = 0; n < 2; ++n)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[n][r]);
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-      const float m_new = fmaxf(m_run, mx * p.scale2);
-      const float alpha = fast_exp2(m_run - m_new);
-      m_run = m_new;
-      float sum = 0.f;
-      bf16x8_t pf[4];
-#pragma unroll
-      for (int f = 0; f < 4; ++f) {
-        u32x4 w;
-#pragma unroll
-        for (int j = 0; j < 8; j += 2) {
-          const int r = (f & 1) * 8 + j;
-          const float e0 = fast_exp2(__builtin_fmaf(s[f >> 1][r], p.scale2, -m_new));
-          const float e1 = fast_exp2(__builtin_fmaf(s[f >> 1][r + 1], p.scale2, -m_new));
-          sum += e0 + e1;
-          w[j >> 1] = pack2<bf16_tag>(e0, e1);
-        }
-        pf[f] = __builtin_bit_cast(bf16x8_t, w);
-      }
-      l_run = l_run * alpha + sum;
-      if (__any(alpha != 1.0f)) {
-#pragma unroll
-        for (int d = 0; d < DT; ++d)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) o[d][r] *= alpha;
-      }
-#pragma unroll
-      for (int f = 0; f < 4; ++f)
-#pragma unroll
-        for (int d = 0; d < DT; ++d) {
-          const uint32_t ad = tr_base + (uint32_t)(16 * f * VLS + 64 * d);
-          const trp_v4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((trp_lds_v4*)ad);
-          const trp_v4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((trp_lds_v4*)(ad + 8 * VLS));
-          const trp_v8 v = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
-          o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, v), pf[f], o[d], 0, 0, 0);
-        }
-    }
-    lds_barrier();
-  }
-
-  l_run += __shfl_xor(l_run, 32, 64);
-  if (wave * 32 + l31 >= n_rows) return;
-  const float w = sigmoid_f32((float)reinterpret_cast<const bf16*>(a.gate)[(int64_t)(row0 + qi) * a.ld_q + a.gate_off + head]) / l_run;
+  float m_run, l_run;
+  prompt_attention<DQ, VP, GROUPS, KEYS>(w, lds, qf, o, m_run, l_run);
+  if (group || wave * 32 + l31 >= n_rows) return;
+  const float f = sigmoid_f32((float)reinterpret_cast<const bf16*>(a.gate)[(int64_t)(row0 + qi) * a.ld_q + a.gate_off + head]) / l_run;
   bf16* out = reinterpret_cast<bf16*>(a.out) + (int64_t)(row0 + qi) * a.ld_out + head * VP + 4 * hh;
 #pragma unroll
   for (int d = 0; d < DT; ++d)
 #pragma unroll
     for (int r = 0; r < 16; r += 4)
-      *reinterpret_cast<u32x2*>(out + 32 * d + 2 * r) = u32x2{pack2<bf16_tag>(o[d][r] * w, o[d][r + 1] * w),
-                                                              pack2<bf16_tag>(o[d][r + 2] * w, o[d][r + 3] * w)};
+      *reinterpret_cast<u32x2*>(out + 32 * d + 2 * r) = u32x2{pack2<bf16_tag>(o[d][r] * f, o[d][r + 1] * f),
+                                                              pack2<bf16_tag>(o[d][r + 2] * f, o[d][r + 3] * f)};
 }
 
 static bool lp_ok(int dq, int vp) {
@@ -202,7 +116,9 @@ static bool lp_ok(int dq, int vp) {
 }
 template <int DQ, int VP>
 static void lp_launch(const LatentPrefillK& p, hipStream_t st) {
-  latent_prefill_kernel<DQ, VP><<<dim3((unsigned)((int64_t)p.a.n_tiles * p.a.heads)), dim3(256), 0, st>>>(p);
+  const int64_t workgroups = (int64_t)p.a.n_tiles * p.a.heads;
+  if (prompt_two_groups(workgroups, p.a.n_ctx, p.a.n_tiles)) latent_prefill_kernel<DQ, VP, 2><<<dim3((unsigned)workgroups), dim3(512), 0, st>>>(p);
+  else latent_prefill_kernel<DQ, VP, 1><<<dim3((unsigned)workgroups), dim3(256), 0, st>>>(p);
 }
 template <int DQ>
 static void lp_v(const LatentPrefillK& p, hipStream_t st) {

@@ -548,6 +548,49 @@ def test_latent_attention_of_a_stream_past_the_caches(heads, lens):
 
 
 # ---- prompt portions ---------------------------------------------------------------------------
+@pytest.mark.parametrize("q_dim,r_pad,v_pad", [(32, 32, 32), (64, 32, 64), (64, 64, 128), (96, 64, 32), (128, 64, 128), (192, 64, 128)])
+@pytest.mark.parametrize("window", [0, 100])
+def test_portions_with_and_without_shared_tiles(q_dim, r_pad, v_pad, window):
+    """Few workgroups (two groups of waves share a portion's tiles) and many (one group), at the edges of the tiles of 64
+    keys (32 from 256 + 128 columns) and 128 rows, the fewest shared tiles, odd and even numbers of them."""
+    from scalellm_amd.latent_layers import LatentPlan
+    from scalellm_amd.layers import Portion
+    lk, H, c_pad, block, dt = _lk(), 16, 64, 16, torch.bfloat16
+    spans = [(1, 1), (64, 64), (65, 65), (129, 129), (5, 260), (200, 320), (31, 321), (130, 449), (400, 600), (2, 500), (3, 1000)]   # rows, context
+    nb = [(k + block - 1) // block for _, k in spans]
+    first = np.concatenate([[0], np.cumsum(nb)])
+    cache = _rnd(3, sum(nb) * block, c_pad + r_pad, dtype=dt)
+    T, dq = sum(n for n, _ in spans), q_dim + r_pad
+    proj, w = _rnd(1, T, H * dq + 16, dtype=dt), _rnd(2, H * (q_dim + v_pad), c_pad, dtype=dt, std=c_pad ** -0.5)
+    portions, row = [], 0
+    for i, (n, k) in enumerate(spans):
+        portions.append(Portion(row, n, k, (np.arange(first[i], first[i + 1]) * block).astype(np.int32)))
+        row += n
+    got = {}
+    for many in (False, True):
+        out = torch.full((T, H * v_pad), float("nan"), dtype=dt, device=DEV)
+        for ps in ([portions] if many else [[p] for p in portions]):   # 17 tiles of 16 heads, and up to 4
+            plan = LatentPlan.build(ps, window, block, DEV)
+            assert (len(plan.tiles) * H > 256) == many
+            ctx = lk.latent_gather(cache, plan.slots)
+            kv = torch.mm(ctx[:, :c_pad], w.t())
+            lk.latent_prefill(proj, ctx, kv, out, plan.tiles, heads=H, q_dim=q_dim, c_pad=c_pad, v_pad=v_pad, gate_off=H * dq,
+                              window=window, scale=2 * dq ** -0.5)
+        got[many] = out.double()
+    for i, ((n, k), p) in enumerate(zip(spans, portions)):
+        rows = cache[int(first[i]) * block:int(first[i]) * block + k]
+        x, kr, pr = torch.mm(rows[:, :c_pad], w.t()).double().view(k, H, -1), rows[:, c_pad:].double(), proj[p.row0:p.row0 + n].double()
+        pos, j = torch.arange(k - n, k, device=DEV)[:, None], torch.arange(k, device=DEV)[None]
+        seen = (j <= pos) & (pos - j < window if window else True)
+        for h in range(H):
+            q = pr[:, h * dq:(h + 1) * dq]
+            s = ((q[:, :q_dim] @ x[:, h, :q_dim].t() + q[:, q_dim:] @ kr.t()) * 2 * dq ** -0.5).masked_fill(~seen, -float("inf"))
+            want = torch.softmax(s, 1) @ x[:, h, q_dim:] * torch.sigmoid(pr[:, H * dq + h])[:, None]
+            for out in got.values():   # 16-bit weights and results: 2^-9 of each, relative to the row
+                err = (out[p.row0:p.row0 + n, h * v_pad:(h + 1) * v_pad] - want).norm(dim=1)
+                assert (err <= 2.0 ** -7 * want.norm(dim=1) + 2.0 ** -8).all()
+
+
 @pytest.mark.parametrize("q_dim,r_pad,v_pad", [(32, 32, 32), (32, 64, 64), (64, 64, 128), (128, 32, 64), (128, 64, 128), (192, 64, 64)])
 @pytest.mark.parametrize("window", [0, 1, 40, 64, 129, 300])
 def test_portion_attention(q_dim, r_pad, v_pad, window):

@@ -267,6 +267,53 @@ def test_attention_kernels_agree(heads, kv_heads, D, V, size, keep, softcap, sin
     _close(out.view(len(lens), heads, V), want, torch.bfloat16, b16=4e-2)
 
 
+@pytest.mark.parametrize("D,V", [(128, 128), (64, 64), (96, 128), (192, 64), (64, 192), (192, 128), (256, 256)])
+@pytest.mark.parametrize("size,keep,softcap,sink", [(0, 0, 0.0, False), (150, 70, 6.0, True), (40, 0, 6.0, False), (0, 0, 50.0, True)])
+def test_portions_with_and_without_shared_tiles(D, V, size, keep, softcap, sink):
+    """Few workgroups (two groups of waves share a portion's tiles) and many (one group), at the edges of the tiles of 64 keys
+    and 128 rows, the fewest shared tiles, odd and even numbers of them."""
+    from scalellm_amd import mixer_kernels as mk
+    from scalellm_amd.layers import InputParameters, Portion
+    from scalellm_amd.mixer_layers import WindowPlan
+    g = torch.Generator().manual_seed(6)
+    B, heads, kv_heads = 16, 16, 8
+    spans = [(1, 1), (64, 64), (65, 65), (129, 129), (5, 260), (200, 320), (31, 321), (130, 449), (400, 600), (2, 500), (3, 1000)]   # rows, context
+    nb = [(k + B - 1) // B for _, k in spans]
+    perm = torch.randperm(sum(nb), generator=g).to(torch.int32) * B
+    cu = np.concatenate([[0], np.cumsum(nb)])
+    r = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16).to(DEV)  # noqa: E731
+    kc, vc, q = r(sum(nb) * B, kv_heads, D), r(sum(nb) * B, kv_heads, V), r(sum(n for n, _ in spans), heads * D)
+    sk = (torch.randn(heads, generator=g) + 2).to(DEV) if sink else None
+    how = dict(heads=heads, window=size, keep_first=keep, scale=2 * D ** -0.5, softcap=softcap, out_scale=0.5)
+    portions, want, row = [], [], 0
+    for i, (n, k) in enumerate(spans):
+        portions.append(Portion(row, n, k, perm[cu[i]:cu[i + 1]].numpy()))
+        j = torch.arange(k)
+        at = (perm[cu[i] + j // B].long() + j % B).to(DEV)
+        pos, j = torch.arange(k - n, k, device=DEV)[:, None], j.to(DEV)[None]
+        seen = (j <= pos) & ((pos - j < size) | (j < keep) if size else True)
+        for h in range(heads):
+            x = q[row:row + n, h * D:(h + 1) * D].double() @ kc[at, h // 2].double().t() * how["scale"]
+            x = (softcap * torch.tanh(x / softcap) if softcap else x).masked_fill(~seen, -float("inf"))
+            if sink:
+                x = torch.cat([x, sk[h].double().expand(n, 1)], 1)
+            want.append(0.5 * (torch.softmax(x, 1)[:, :k] @ vc[at, h // 2].double()))
+        row += n
+    got = {}
+    for many in (False, True):
+        out = torch.full((row, heads * V), float("nan"), dtype=torch.bfloat16, device=DEV)
+        for ps in ([portions] if many else [[p] for p in portions]):   # 17 tiles of 16 heads, and up to 4
+            plan = WindowPlan.of(InputParameters(*[None] * 5, portions=ps), size, keep, B, DEV)
+            assert (len(plan.tiles) * heads > 256) == many
+            mk.window_prefill(q, kc, vc, out, sk, plan.slots, plan.tiles, **how)
+        got[many] = out.double()
+    for i, (n, _) in enumerate(spans):
+        for h in range(heads):
+            w, p0 = want[i * heads + h], portions[i].row0
+            for out in got.values():   # 16-bit weights and results: 2^-9 of each, relative to the row
+                assert ((out[p0:p0 + n, h * V:(h + 1) * V] - w).norm(dim=1) <= 2.0 ** -7 * w.norm(dim=1) + 2.0 ** -8).all()
+
+
 @pytest.mark.parametrize("dtype", BOTH)
 @pytest.mark.parametrize("per_head", [True, False])
 @pytest.mark.parametrize("heads,vdim", [(1, 1), (3, 13), (16, 128), (5, 200)])
