@@ -48,7 +48,7 @@ enum TuneKey : int {
   TUNE_W4_XL_MODEL,       // SLM_W4_XL_MODEL       0 = the 256 x 256 kernel only where its tiles fill whole rounds (no round-count comparison with 256 x 128 tiles)
   TUNE_W4_M128_ADMA,      // SLM_W4_M128_ADMA      activations of the 256-column form by LDS-DMA (1) or through registers (0)
   TUNE_W4_XL_SK,          // SLM_W4_XL_SK          stream-K form of the 256 x 256 kernel: 0 never, 2 wherever it applies (default 1: where the round model says it wins)
-  TUNE_W4_TILE,           // SLM_W4_TILE           w4_tile.hip: 1 .. 5 = that tile shape for every bf16 call but GEMVs, + 8 n = cut in n slices of K; 0 = never (default: where a call allows it and its tiles pay)
+  TUNE_W4_TILE,           // SLM_W4_TILE           w4_tile.hip: 1 .. 6 = that tile shape for every bf16 call but GEMVs, + 8 n = cut in n slices of K; 0 = never (default: where a call allows it and its tiles pay)
   TUNE_COUNT
 };
 

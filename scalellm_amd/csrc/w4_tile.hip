@@ -259,22 +259,23 @@ __global__ void __launch_bounds__(256, 1) w4_tile_kernel(const W4TileK a) {
   tile_settle(acc);
   if (a.slices > 1 && !tile_add_slices(acc, a.slabs + (int64_t)t * a.slices * (MM * 1024), a.arrived + t, slice, a.slices, lds)) return;
 
-  // Out through LDS, 64 rows at a time, and from there in whole lines.  A wave has its own columns' rows to itself, so that their order alone is enough;
+  // Out through LDS, 64 (32) rows at a time, and from there in whole lines.  A wave has its own columns' rows to itself, so that their order alone is enough;
   // of one packed tile a wave a pair's gate is in one wave, its up in the next, and they take half of the rows each.  Rows are read four at a
   // time: one after the other, and with a bias added where there is none, 2183 x 4096 x 28672 with the SiLU took 430 us, 422 now, 2183 x 4096 x 4096 77
   // and 75.4.  (Most of what is left, 6 us a tile, is the stores of all CUs at the same time.)
-  // (The code for 64 rows is there once, apart from the accumulators: written out per accumulator it was 10000 instructions, and 13 us more.)
+  // (The code for these rows is there once, apart from the accumulators: written out per accumulator it was 10000 instructions, and 13 us more.)
   constexpr int CW = BN / 4, LR = CW * 4 + 16;       // columns of a wave, bytes of a row of them
-  static_assert(4 * 64 * LR <= R0 + RS * RB, "LDS of 64 rows");
-  char* const mine = lds + wave * (64 * LR) + r16 * LR + g * 32;
+  constexpr int OR = BM % 64 ? 32 : 64;              // rows at a time
+  static_assert(4 * OR * LR <= R0 + RS * RB, "LDS of the rows");
+  char* const mine = lds + wave * (OR * LR) + r16 * LR + g * 32;
   auto out = [&](auto with_silu, auto with_bias) __attribute__((always_inline)) {
     constexpr bool SILU = decltype(with_silu)::value, BIAS = decltype(with_bias)::value, PAIRS = TW == 1 && SILU;
     constexpr int PER_ROW = SILU ? 4 : CW / 8, BY = 64 / PER_ROW;   // lanes of a row, eight columns each; rows at a time
-    constexpr int TURNS = (PAIRS ? 32 : 64) / BY, AT_ONCE = TURNS < 4 ? TURNS : 4;
-    const int from = PAIRS ? wave & 2 : wave, lcol = lane % PER_ROW * 8, row0 = lane / PER_ROW + (PAIRS ? (wave & 1) * 32 : 0);
+    constexpr int TURNS = (PAIRS ? OR / 2 : OR) / BY, AT_ONCE = TURNS < 4 ? TURNS : 4;
+    const int from = PAIRS ? wave & 2 : wave, lcol = lane % PER_ROW * 8, row0 = lane / PER_ROW + (PAIRS ? (wave & 1) * (OR / 2) : 0);
     const int64_t col = n0 + from * CW + lcol;
-    const char* const gate = lds + from * (64 * LR) + lcol * 4 + row0 * LR;
-    const char* const up = gate + (TW == 2 ? 128 : 64 * LR);
+    const char* const gate = lds + from * (OR * LR) + lcol * 4 + row0 * LR;
+    const char* const up = gate + (TW == 2 ? 128 : OR * LR);
     const bool inside = col < a.N;
     float bias[2][8];
     if constexpr (BIAS) {
@@ -287,17 +288,17 @@ __global__ void __launch_bounds__(256, 1) w4_tile_kernel(const W4TileK a) {
     uint16_t* const c = a.c + (SILU ? (col >> 6) * 32 + lcol : col);
     __syncthreads();
 #pragma unroll 1
-    for (int q = 0; q < BM / 64; ++q) {
+    for (int q = 0; q < BM / OR; ++q) {
       if (PAIRS && q > 0) __syncthreads();
-      in_turn<BM / 64>([&](auto which) __attribute__((always_inline)) {
+      in_turn<BM / OR>([&](auto which) __attribute__((always_inline)) {
         constexpr int Q = which;
         if (q == Q) {   // (different code to the compiler: one code for all of them would index the accumulators, in memory)
-          asm volatile("; rows from 64 * %0" : : "n"(Q));
+          asm volatile("; rows from %0" : : "n"(OR * Q));
 #pragma unroll
-          for (int m = 0; m < 4; ++m)
+          for (int m = 0; m < OR / 16; ++m)
 #pragma unroll
-            for (int n = 0; n < NT; ++n) *reinterpret_cast<f32x4*>(mine + 16 * m * LR + (n >> 1) * 128 + (n & 1) * 16) = acc[n][4 * Q + m];
-          asm volatile("; rows from 64 * %0" : : "n"(Q));
+            for (int n = 0; n < NT; ++n) *reinterpret_cast<f32x4*>(mine + 16 * m * LR + (n >> 1) * 128 + (n & 1) * 16) = acc[n][OR / 16 * Q + m];
+          asm volatile("; rows from %0" : : "n"(OR * Q));
         }
       });
       if constexpr (PAIRS) __syncthreads();
@@ -314,7 +315,7 @@ __global__ void __launch_bounds__(256, 1) w4_tile_kernel(const W4TileK a) {
           }
 #pragma unroll
         for (int i = 0; i < AT_ONCE; ++i) {
-          const int64_t row = m0 + 64 * q + row0 + (i0 + i) * BY;
+          const int64_t row = m0 + OR * q + row0 + (i0 + i) * BY;
           float y[8];
 #pragma unroll
           for (int j = 0; j < 8; ++j) {
@@ -344,13 +345,16 @@ __global__ void __launch_bounds__(256, 1) w4_tile_kernel(const W4TileK a) {
 }
 
 // Tiles, and what they take: us of a step of 64 k alone on the chip and with every CU busy (power), and of a tile beside its steps.
-// Fitted to 1900 timings of 163 products of 129 - 5120 rows; by them the tile taken is 1.3 % behind the best one on average.
+// A CU holds two of 128 x 128; from the second on a step of both takes 0.8 of `busy` and more.  Fitted to 2000 timings of 170 products of
+// 129 - 5120 rows; by them the tile taken is 0.5 % behind the best one on average, 5 % at worst (without 160 x 256, and with 128 x 128 as one
+// that fills a CU: 3.7 % and 19 %).  160 x 256: 2183 x 14336 x 4096 are 224 tiles, 228 us, where 192 x 256 leaves 64 CUs idle and takes 241;
+// 2183 x 4096 x 4096 69.4 and 75.6; 160 x 4096 x 28672 with the SiLU 51 and 61.
 struct W4Tile {
-  int bm, bn;
+  int bm, bn, on_cu;
   float step, busy, rest;
 };
-constexpr W4Tile W4_TILES[] = {{256, 256, 1.031f, 1.312f, 19.4f}, {256, 128, 0.647f, 0.904f, 2.3f}, {128, 128, 0.510f, 0.489f, -0.3f},
-                               {128, 256, 0.778f, 0.974f, 2.1f}, {192, 256, 0.889f, 1.157f, 6.9f}};
+constexpr W4Tile W4_TILES[] = {{256, 256, 1, 1.174f, 1.389f, 9.9f}, {256, 128, 1, 0.711f, 0.854f, 6.7f}, {128, 128, 2, 0.575f, 0.980f, 3.7f},
+                               {128, 256, 1, 0.871f, 0.887f, 6.3f}, {192, 256, 1, 0.966f, 1.106f, 8.5f}, {160, 256, 1, 0.862f, 0.975f, 7.9f}};
 constexpr int W4_N_TILES = sizeof(W4_TILES) / sizeof(W4_TILES[0]);
 constexpr int W4_TILE_CUS = 256;
 constexpr float W4_TILE_CUT = 4.6f, W4_TILE_SLABS = 4.1e6f;   // us of cutting tiles, bytes of their slabs that take one more
@@ -375,9 +379,13 @@ static W4TilePlan w4_tile_plan_of(int64_t M, int64_t N, int64_t K, int tile, int
   while (s > 1 && (steps + s - 1) / s * (s - 1) >= steps) --s;   // no slice is empty
   p.slices = s > 1 ? s : 1;
   const size_t slabs = (size_t)p.tiles * s * t.bm * t.bn * 4;
-  auto round = [&](int wgs, int n) { return t.rest + n * (t.step + (t.busy - t.step) * (float)wgs / W4_TILE_CUS); };
-  const int left = p.tiles % W4_TILE_CUS;
-  p.us = (float)(p.tiles / W4_TILE_CUS) * round(W4_TILE_CUS, steps);
+  auto round = [&](int wgs, int n) {
+    const float load = (float)wgs / W4_TILE_CUS;
+    if (t.on_cu == 2) return t.rest + n * (load <= 1.f ? t.step : t.busy * (0.6f + 0.2f * load));
+    return t.rest + n * (t.step + (t.busy - t.step) * load);
+  };
+  const int full = W4_TILE_CUS * t.on_cu, left = p.tiles % full;
+  p.us = (float)(p.tiles / full) * round(full, steps);
   if (p.slices > 1) p.us = round(p.tiles * s, (steps + s - 1) / s) + W4_TILE_CUT + (float)slabs / W4_TILE_SLABS;
   else if (left) p.us += round(left, steps);
   return p;
@@ -409,7 +417,8 @@ static void w4_tile_shape(int tile, const W4TileK& k, hipStream_t st) {
     case 1: return w4_tile_launch<256, 128, NGC>(k, st);
     case 2: return w4_tile_launch<128, 128, NGC>(k, st);
     case 3: return w4_tile_launch<128, 256, NGC>(k, st);
-    default: return w4_tile_launch<192, 256, NGC>(k, st);
+    case 4: return w4_tile_launch<192, 256, NGC>(k, st);
+    default: return w4_tile_launch<160, 256, NGC>(k, st);
   }
 }
 

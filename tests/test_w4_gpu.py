@@ -810,6 +810,29 @@ def test_four_wave_tiles(M, K, N, gs, tile):
                 assert torch.equal(half, ref)
 
 
+@pytest.mark.parametrize("M,K,N,gs", [(129, 128, 64, 128), (160, 128, 256, 64), (161, 1152, 96, 32), (320, 512, 544, 64), (2304, 384, 4160, 128)])
+def test_four_wave_tiles_of_160_rows(M, K, N, gs):
+    """Rows that fill the tile, one more and fewer; it leaves through LDS 32 rows at a time, the others 64."""
+    test_four_wave_tiles(M, K, N, gs, 6)
+
+
+@pytest.mark.parametrize("tile", [1, 2, 3, 4, 5, 6])
+def test_four_wave_tiles_without_a_bias(tile):
+    """The same as with a bias of zeros, whole and cut."""
+    from scalellm_amd import kernels
+    M, K, N, dtype, tdt = 333, 640, 576, "bf16", torch.bfloat16
+    case = helpers.make_quant_case(M, K, N, 128, "awq", dtype)
+    plain, paired = _pack(case, dtype), helpers.pack_case(case, dtype, paired=True)
+    a, zeros = torch.randn(M, K, device=DEV, dtype=tdt), torch.zeros(N, device=DEV, dtype=tdt)
+    for cut in (1, 2):
+        with kernels.tuning(SLM_W4_TILE=tile + 8 * cut):
+            for w, width, silu in ((plain, N, False), (paired, N // 2, True)):
+                got, want = (torch.full((M, width), float("nan"), device=DEV, dtype=tdt) for _ in range(2))
+                kernels.gptq_gemm(a, w, got, silu_mul=silu)
+                kernels.gptq_gemm(a, w, want, zeros, silu_mul=silu)
+                assert torch.equal(got, want)
+
+
 def test_four_wave_tiles_without_scratch_are_not_cut():
     """A call whose plan cuts tiles runs without the scratch of it too: the same sums in another order."""
     from scalellm_amd import _lib, kernels
