@@ -8,12 +8,13 @@
 //            14.4 and 12.7, 8 rows 6.0 and 5.5, 1 row 4.3 and 4.3.
 //   prepare  portions, cut into chunks of 16 tokens, every chunk at once: inputs activated and normed, decays summed, what a chunk's tokens do to
 //            each other solved (a 16 x 16 triangular system), and everything that does not wait for the state multiplied out.  Bound: the
-//            latency of its inputs, which are loaded before the first is used, and the records it writes (2 TB/s).
+//            latency of its inputs, which are loaded before the first is used, its vector instructions (1650 a wave) and the records it writes (2 TB/s).
+//            A wave's eight lengths have their root and quotient in a lane each: by all lanes one after the other 92 us (16 heads, 4096 tokens), 83.
 //   scan     portions: chunk after chunk.  The columns of S are independent, so a workgroup owns 16 of them and keeps them
 //            in registers from the portion's first token to its last; the products are 32-bit MFMAs.  Bound: a chain of two products and an
 //            exchange a chunk, 0.6 us, and the instructions around them.
 //   Both, us, 16 heads of 128 x 128 and 4096 tokens: delta 305 with the triangular system and B U in the scan, 64-bit addresses and a wave's
-//   read-outs by itself, 239 now; lightning 184 and 134; 8 x 500 tokens, 32 heads: 341 and 309, 209 and 183; 16 heads of 64, 2000 tokens: 120 and 82.
+//   read-outs by itself, 232 now; lightning 184 and 134; 8 x 500 tokens, 32 heads: 341 and 307, 209 and 183; 16 heads of 64, 2000 tokens: 120 and 82.
 //   gated_norm  the norm and gate behind a scan.
 #include "latent/latent_common.h"
 #include "slm_mixers.h"
@@ -36,10 +37,10 @@ __device__ __forceinline__ float silu_run(float z) {
   const float e = __expf(low ? z : -z);
   return z > 100.f ? z : low ? z * e : quotient(z, 1.0f + e);
 }
-// log(1 + x) = log(u) x / (u - 1) with u the rounded 1 + x: what the sum loses of x comes back (Kahan)
+// log(1 + x) = log(u) x / (u - 1) with u the rounded 1 + x: what the sum loses of x comes back (Kahan); where u is not 1 both are above 2^-25
 __device__ __forceinline__ float softplus_f32(float z) {
   const float x = __expf(-fabsf(z)), u = 1.0f + x;
-  const float l = u == 1.0f ? x : __logf(u) * (x / (u - 1.0f));
+  const float l = u == 1.0f ? x : __logf(u) * quotient(x, u - 1.0f);
   return fmaxf(z, 0.f) + l;
 }
 __device__ __forceinline__ float sigmoid_full(float z) { return 1.0f / (1.0f + expf(-z)); }
@@ -454,17 +455,35 @@ __global__ void __launch_bounds__(256) recurrent_prepare_kernel(const slm_recurr
   }
   if (DELTA && tid < 16) sbeta[tid] = tid < n ? sigmoid_full(to_f32(in[tid * a.ld_proj + a.off_b + head])) : 0.f;
   __syncthreads();
-  if constexpr (DELTA) {   // unit vectors: four tokens per wave
+  if constexpr (DELTA) {   // unit vectors: four tokens per wave; a lane takes the root and quotient of one of their eight sums
+    constexpr int CW = (DK + 63) / 64;
+    float q[4][CW], k[4][CW], sum = 0.f;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int t = 4 * wave + j;
       float nq = 0.f, nk = 0.f;
-      for (int c = lane; c < DK; c += 64) {
-        nq = __builtin_fmaf(sq[t * LD + c], sq[t * LD + c], nq);
-        nk = __builtin_fmaf(sk[t * LD + c], sk[t * LD + c], nk);
+#pragma unroll
+      for (int i = 0; i < CW; ++i) {
+        const int c = lane + 64 * i;
+        const bool there = DK % 64 == 0 || c < DK;
+        q[j][i] = there ? sq[t * LD + c] : 0.f, k[j][i] = there ? sk[t * LD + c] : 0.f;
+        nq = __builtin_fmaf(q[j][i], q[j][i], nq);
+        nk = __builtin_fmaf(k[j][i], k[j][i], nk);
       }
-      const float fq = a.q_scale / sqrtf(wave_sum(nq) + a.unit_eps), fk = 1.0f / sqrtf(wave_sum(nk) + a.unit_eps);
-      for (int c = lane; c < DK; c += 64) sq[t * LD + c] *= fq, sk[t * LD + c] *= fk;
+      nq = wave_sum(nq), nk = wave_sum(nk);
+      sum = lane == j ? nq : lane == 4 + j ? nk : sum;
+    }
+    const float f = (lane < 4 ? a.q_scale : 1.0f) / sqrtf(sum + a.unit_eps);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int t = 4 * wave + j;
+      const float fq = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, f), j));
+      const float fk = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, f), 4 + j));
+#pragma unroll
+      for (int i = 0; i < CW; ++i) {
+        const int c = lane + 64 * i;
+        if (DK % 64 == 0 || c < DK) sq[t * LD + c] = q[j][i] * fq, sk[t * LD + c] = k[j][i] * fk;
+      }
     }
   }
   float lowest = step_l * n;   // (without the delta rule a token's channels decay alike)
