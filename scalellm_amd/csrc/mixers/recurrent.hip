@@ -8,13 +8,13 @@
 //            14.4 and 12.7, 8 rows 6.0 and 5.5, 1 row 4.3 and 4.3.
 //   prepare  portions, cut into chunks of 16 tokens, every chunk at once: inputs activated and normed, decays summed, what a chunk's tokens do to
 //            each other solved (a 16 x 16 triangular system), and everything that does not wait for the state multiplied out.  Bound: the
-//            latency of its inputs, which are loaded before the first is used, its vector instructions (1650 a wave) and the records it writes (2 TB/s).
+//            latency of its inputs, which are loaded before the first is used, its vector instructions (1600 a wave) and the records it writes (2 TB/s).
 //            A wave's eight lengths have their root and quotient in a lane each: by all lanes one after the other 92 us (16 heads, 4096 tokens), 83.
 //   scan     portions: chunk after chunk.  The columns of S are independent, so a workgroup owns 16 of them and keeps them
 //            in registers from the portion's first token to its last; the products are 32-bit MFMAs.  Bound: a chain of two products and an
 //            exchange a chunk, 0.6 us, and the instructions around them.
 //   Both, us, 16 heads of 128 x 128 and 4096 tokens: delta 305 with the triangular system and B U in the scan, 64-bit addresses and a wave's
-//   read-outs by itself, 232 now; lightning 184 and 134; 8 x 500 tokens, 32 heads: 341 and 307, 209 and 183; 16 heads of 64, 2000 tokens: 120 and 82.
+//   read-outs by itself, 222 now; lightning 184 and 131; 8 x 500 tokens, 32 heads: 341 and 293, 209 and 181; 16 heads of 64, 2000 tokens: 120 and 82.
 //   gated_norm  the norm and gate behind a scan.
 #include "latent/latent_common.h"
 #include "slm_mixers.h"
@@ -31,16 +31,21 @@ __device__ __forceinline__ float quotient(float n, float d) {
   return __builtin_fmaf(__builtin_fmaf(-d, q, n), r, q);
 }
 __device__ __forceinline__ float silu_f32(float z) { return z / (1.0f + __expf(-z)); }
-// (below -69, where 1 + exp(-z) is exp(-z) and past what the quotient takes, it is z exp(z); above 100 it is z, an infinity too)
+// z / (1 + exp(-z)) by the same steps; below -69, where 1 + exp(-z) is exp(-z) and past what they take, z exp(z) / 1 (1 + exp(z) is 1); of an
+// infinity, whose remainder is not a number, the quotient remains.  No branch: tokens run side by side (16 heads, 4096 tokens: 84 us with two
+// branches a token, 76 without).
 __device__ __forceinline__ float silu_run(float z) {
   const bool low = z < -69.f;
-  const float e = __expf(low ? z : -z);
-  return z > 100.f ? z : low ? z * e : quotient(z, 1.0f + e);
+  const float e = __expf(low ? z : -z), d = 1.0f + e, n = low ? z * e : z;
+  float r = __builtin_amdgcn_rcpf(d);
+  r = __builtin_fmaf(__builtin_fmaf(-d, r, 1.0f), r, r);
+  const float q = n * r;
+  return __builtin_fmaf(fmaxf(__builtin_fmaf(-d, q, n), -3.4028235e38f), r, q);
 }
 // log(1 + x) = log(u) x / (u - 1) with u the rounded 1 + x: what the sum loses of x comes back (Kahan); where u is not 1 both are above 2^-25
 __device__ __forceinline__ float softplus_f32(float z) {
   const float x = __expf(-fabsf(z)), u = 1.0f + x;
-  const float l = u == 1.0f ? x : __logf(u) * quotient(x, u - 1.0f);
+  const float q = __logf(u) * quotient(x, u - 1.0f), l = u == 1.0f ? x : q;
   return fmaxf(z, 0.f) + l;
 }
 __device__ __forceinline__ float sigmoid_full(float z) { return 1.0f / (1.0f + expf(-z)); }
@@ -124,7 +129,8 @@ __device__ __forceinline__ void conv_run4(const slm_recurrent_args& a, const E* 
     float acc = w[3] * x[t];
 #pragma unroll
     for (int j = 2; j >= 0; --j) acc = __builtin_fmaf(w[j], x[3 + t - j], acc);
-    put(t, t < n ? silu_run(acc) : 0.f);
+    const float y = silu_run(acc);
+    put(t, t < n ? y : 0.f);
   }
 }
 template <typename E>
@@ -435,14 +441,16 @@ __global__ void __launch_bounds__(256) recurrent_prepare_kernel(const slm_recurr
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int t = (i0 + 256 * j) / a.v_pad, c = (i0 + 256 * j) % a.v_pad;
-        if (t < 16) sv[(c >> 4) * 256 + (t >> 2) * 64 + (c & 15) * 4 + (t & 3)] = t < n && c < a.vdim ? silu_run(v[j]) : 0.f;
+        const float y = silu_run(v[j]);
+        if (t < 16) sv[(c >> 4) * 256 + (t >> 2) * 64 + (c & 15) * 4 + (t & 3)] = t < n && c < a.vdim ? y : 0.f;
       }
     }
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
       const int t = (tid + 256 * j) / DK, c = (tid + 256 * j) % DK;
       const bool there = t < n && c < a.dim;
-      sq[t * LD + c] = there ? silu_run(q[j]) : 0.f, sk[t * LD + c] = there ? silu_run(k[j]) : 0.f;
+      const float y = silu_run(q[j]), z = silu_run(k[j]);
+      sq[t * LD + c] = there ? y : 0.f, sk[t * LD + c] = there ? z : 0.f;
     }
   }
   if constexpr (DELTA) {
@@ -450,7 +458,8 @@ __global__ void __launch_bounds__(256) recurrent_prepare_kernel(const slm_recurr
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
       const int t = (tid + 256 * j) / DK, c = (tid + 256 * j) % DK;
-      sL[t * LD + c] = t < n && c < a.dim ? LOG2E_F * (neg_a * softplus_f32(decay_in[j] + decay_bias[j])) : 0.f;
+      const float l = LOG2E_F * (neg_a * softplus_f32(decay_in[j] + decay_bias[j]));
+      sL[t * LD + c] = t < n && c < a.dim ? l : 0.f;
     }
   }
   if (DELTA && tid < 16) sbeta[tid] = tid < n ? sigmoid_full(to_f32(in[tid * a.ld_proj + a.off_b + head])) : 0.f;
