@@ -12,9 +12,9 @@
 //            A wave's eight lengths have their root and quotient in a lane each: by all lanes one after the other 92 us (16 heads, 4096 tokens), 83.
 //   scan     portions: chunk after chunk.  The columns of S are independent, so a workgroup owns 16 of them and keeps them
 //            in registers from the portion's first token to its last; the products are 32-bit MFMAs.  Bound: a chain of two products and an
-//            exchange a chunk, 0.6 us, and the instructions around them.
+//            exchange a chunk, 0.6 us (24 products of 32 cycles a wave are 0.35), and the instructions around them.
 //   Both, us, 16 heads of 128 x 128 and 4096 tokens: delta 305 with the triangular system and B U in the scan, 64-bit addresses and a wave's
-//   read-outs by itself, 222 now; lightning 184 and 131; 8 x 500 tokens, 32 heads: 341 and 293, 209 and 181; 16 heads of 64, 2000 tokens: 120 and 82.
+//   read-outs by itself, 212 now; lightning 184 and 131; 8 x 500 tokens, 32 heads: 341 and 293, 209 and 181; 16 heads of 64, 2000 tokens: 120 and 82.
 //   gated_norm  the norm and gate behind a scan.
 #include "latent/latent_common.h"
 #include "slm_mixers.h"
@@ -713,21 +713,25 @@ __global__ void __launch_bounds__(64 * W, 2) recurrent_scan_kernel(const slm_rec
       }
   };
   // two sums of tiles side by side: the products of one wait for each other
-  auto products = [&](const f32x4 (&x)[TPW], int j, f32x4 c, auto between) {
-    f32x4 d = {0.f, 0.f, 0.f, 0.f};
+  auto some_products = [&](const f32x4 (&x)[TPW], int j, f32x4& c, f32x4& d, int from, int to, auto between) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
+      if (r < from || r >= to) continue;
 #pragma unroll
       for (int i = 0; i < TPW; ++i) {
-        f32x4& to = i & 1 ? d : c;
-        to = __builtin_amdgcn_mfma_f32_16x16x4f32(x[i][r], s[j][i][r], to, 0, 0, 0);
+        f32x4& sum = i & 1 ? d : c;
+        sum = __builtin_amdgcn_mfma_f32_16x16x4f32(x[i][r], s[j][i][r], sum, 0, 0, 0);
       }
       between();
     }
+  };
+  auto products = [&](const f32x4 (&x)[TPW], int j, f32x4 c, auto between) {
+    f32x4 d = {0.f, 0.f, 0.f, 0.f};
+    some_products(x, j, c, d, 0, 4, between);
     return TPW > 1 ? c + d : c;
   };
   // Chunk c; between its products the loads of chunk `later`, one at a time: the 40 of a workgroup all at once back up in the address unit, and
-  // the waves with them (4096 tokens, 16 heads: delta 187 -> 160 us, of 136 without loads; lightning 124 -> 103; 1000 tokens, 32 heads 51 -> 45, 34 -> 27).
+  // the waves with them (4096 tokens, 16 heads: delta 187 -> 160 us, of 136 without loads, before the read-outs were halved; lightning 124 -> 103; 1000 tokens, 32 heads 51 -> 45, 34 -> 27).
   auto chunk = [&](int c, const ChunkOperands<TPW, NCT>& x, int later, ChunkOperands<TPW, NCT>& xl, bool more) {
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     const int b = c & 1;
@@ -749,9 +753,16 @@ __global__ void __launch_bounds__(64 * W, 2) recurrent_scan_kernel(const slm_rec
       for (int j = 0; j < NCT; ++j) part_u[b][j][wave][lane] = products(x.kd, j, zero, between);
       __builtin_amdgcn_sched_barrier(0);
     }
-    // (the read-outs' products run under the writes of the exchange, of two column tiles the second's under its reads)
+    // (half of the read-outs' products run under the writes of the exchange, half under its reads: 16 heads, 4096 tokens 161 us with all of one
+    // column tile's under the writes, 164 under the reads, 153)
+    constexpr int UNDER_WRITES = DELTA ? 2 : 4;
+    f32x4 od = zero;
+    if constexpr (NCT == 1) {
+      o[0] = wave == 0 ? x.o0[0] : zero;
+      some_products(x.qd, 0, o[0], od, 0, UNDER_WRITES, between);
+    }
 #pragma unroll
-    for (int j = 0; j < (NCT + 1) / 2; ++j) o[j] = products(x.qd, j, wave == 0 ? x.o0[j] : zero, between);
+    for (int j = 0; j < NCT / 2; ++j) o[j] = products(x.qd, j, wave == 0 ? x.o0[j] : zero, between);
     __builtin_amdgcn_sched_barrier(0);
     lds_barrier();
     if constexpr (DELTA) {
@@ -762,9 +773,13 @@ __global__ void __launch_bounds__(64 * W, 2) recurrent_scan_kernel(const slm_rec
     }
     collect(c - 1, y);   // (in front of the first chunk: of nothing, and not stored)
     __builtin_amdgcn_sched_barrier(0);
+    if constexpr (NCT == 1) {
+      some_products(x.qd, 0, o[0], od, UNDER_WRITES, 4, between);
+      if constexpr (TPW > 1) o[0] += od;
+    }
 #pragma unroll
     for (int j = (NCT + 1) / 2; j < NCT; ++j) o[j] = products(x.qd, j, wave == 0 ? x.o0[j] : zero, between);
-    if constexpr (DELTA && NCT > 1) __builtin_amdgcn_sched_barrier(0);
+    if constexpr (DELTA) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int j = 0; j < NCT; ++j) {
       u[j] = x.v[j];
