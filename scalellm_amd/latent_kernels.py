@@ -232,10 +232,10 @@ def _run_stream(a) -> None:
 
 def _store_rows(N: int, K: int) -> int:
     """Rows up to which a product that is only stored is streamed.  Without slabs its workgroups are its columns': from 33
-    rows the vendor GEMM, which splits K for itself, is level or ahead under 8192 columns (6752 x 4096, 64 rows: 19.2 us
-    against 22.6) and a little above where K is long (vendor / streamed, 64 rows: 8192 x 2048 13.8 / 12.9, x 4096 19.1 / 22.3, x 8192
-    32.5 / 40.8; 9216 x 4096 26.4 / 22.9, x 8192 40.2 / 42.4; 12288 x 8192 44.0 / 43.3), and above 64 rows always (16896 x 4096, 128
-    rows: 46.6 against 47.0; 64 rows: 44.0 against 38.5)."""
+    rows the vendor GEMM, which splits K for itself, is level or ahead under 8192 columns (6752 x 4096, 64 rows: 17.8 us
+    against 21.8) and a little above where K is long (vendor / streamed, 64 rows: 8192 x 2048 13.7 / 12.4, x 4096 18.6 / 21.9, x 8192
+    32.7 / 41.0; 9216 x 4096 26.4 / 22.5, x 8192 40.2 / 42.1; 12288 x 8192 44.8 / 43.1).  Above 64 rows it is level for wide products
+    (16896 x 4096: 128 rows 42.1 / 43.0, 64 rows 39.6 / 33.9; 12608 x 4096, 85 rows 29.0 / 25.7) and far ahead for narrow ones."""
     return 64 if N >= 8192 and K <= 2048 + 5 * (N - 8192) // 2 else STREAM_MAX_ROWS
 
 
@@ -243,7 +243,7 @@ def _tile_pays(M: int, N: int, K: int, glu: bool) -> bool:
     """Is a product that the tile kernel takes its own, or the vendor's?  us by the device, vendor / tiles, where they are the vendor's:
     129 - 160 rows of large weights, whose one row of tiles reads them slower (28672 x 4096 GLU 62 / 77, from 161 rows 67 / 65; of the largest up to 192
     rows: 16384 x 8192, 170 rows, 75 / 93), and
-    256 x 256 tiles that fill whole rounds of the chip (4096 x 4096, K 2048 49 / 53, 4096 89 / 96; 4096 x 16384 x 4096 364 / 395).
+    256 x 256 tiles that fill whole rounds of the chip (4096 x 4096, K 2048 49 / 54, 4096 90 / 97; 4096 x 16384 x 4096 364 / 398).
     Short and narrow products are up to 8 us longer by the device (200 x 512 x 2048 8 / 15, 200 x 4096 x 4096 18 / 21) and stay here all the same: steps
     with prompts run eagerly, and the vendor product takes 8 us more of the host for each (18 / 10).  Steps of four layers with one prompt of
     150 - 300 tokens, all their products by the vendor / here: 2b 847 / 580 and 836 / 618, 8b 975 / 903 and 1189 / 1065."""
@@ -286,8 +286,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None,
         _run_stream(a)
         return out
     if not streams_rows(x):
-        # (stored products of up to 128 rows are the vendor's, whose small tiles leave fewer CUs idle: 125 x 2048 x 4096 10.7 us against
-        # 18.5, 96 x 12288 x 2048 16.8 against 19.6, 85 x 12608 x 4096 32.7 against 35.0)
+        # (stored products of 65 to 128 rows are the vendor's, whose small tiles leave fewer CUs idle: 125 x 2048 x 4096 10.9 us against
+        # 26.9 streamed; of the widest up to 96 rows streaming would be 2 to 3 us shorter, 96 x 12288 x 2048 17.2 against 15.3)
         return out if M >= TILE_MIN_ROWS and _tile_pays(M, N, K, False) and _gemm(x, w, out) else torch.mm(x, w.t(), out=out)
     a = _linear_args(x, w, M, N, K)
     a.ldx, a.ldw, a.ldy, a.y, a.epilogue = x.stride(0), K, out.stride(0), _p(out), _lib.LIN_STORE
@@ -308,11 +308,12 @@ def linear_f32(x: torch.Tensor, w: torch.Tensor, alpha: float = 1.0, layout: Opt
 
 def stream_split_count(n_out: int, k: int, rows: int) -> int:
     """Slabs of a streamed product: as many as give every CU a workgroup of 64 columns, at least 8 steps of 64 each (a slab
-    is written and read: 4096 columns, 128 rows, 4 against 8 slabs 34 us against 29, and 4 us less behind it).  Above 32 rows a step is
+    is written and read: 4096 x 14336, 128 rows, 4 against 8 slabs 30.4 us against 28.3, and 1 us less behind it).  Above 32 rows a step is
     0.3 to 0.5 us long, so short products of few columns take 4 steps each (with the norm behind them, 100 rows, before / after / vendor
     product: 512 x 512 10.0 / 8.1 / 7.6, 2048 x 896 13.4 / 10.0 / 10.3, 1024 x 1536
     10.7 / 9.5 / 10.1, 4096 x 768 13.2 / 11.4 / 10.9; more columns leave no CUs for it: 5504 x 640 13.3 / 13.3 / 10.9), and large ones
-    above 64 rows two workgroups a CU, which hide each other's waits (8192 x 8192 43.5 / 37.0 / 41.8, 8192 x 14336 69.3 / 51.6 / 71.2)."""
+    above 64 rows two workgroups a CU, which hide each other's waits (with the norm, 128 rows, 2 / 4 / 8 slabs: 8192 x 8192 38.1 / 36.3 / 46.6,
+    8192 x 14336 63.1 / 55.3 / 67.6)."""
     panels = (n_out + 63) // 64
     wgs = 512 if rows > 64 and n_out > 4096 and k >= (8192 if n_out <= 8192 else 4096) else 256
     step = 256 if rows > STREAM_MAX_ROWS and ((k < 2048 and n_out <= 2048) or (k < 1024 and n_out <= 4096)) else 512
@@ -321,10 +322,10 @@ def stream_split_count(n_out: int, k: int, rows: int) -> int:
 
 def glu_split_count(n_out: int, k: int, rows: int) -> int:
     """Slabs of a streamed product in front of the GLU; 1: the GLU is its epilogue.  A workgroup of that form walks all of K, 0.29 us a
-    step of 64 up to 64 rows and 0.53 above, however few columns there are; slabs share it out for one launch more (epilogue / slabs /
+    step of 64 up to 64 rows and 0.43 above, however few columns there are; slabs share it out for one launch more (epilogue / slabs /
     vendor product and GLU, us, 64 rows: 1024 x 1024 7.9 / 6.3 / 10.8, 1024 x 8192 39.0 / 10.9 / 15.9, 4096 x 4096 22.3 / 13.0 / 17.9, 8192 x 1024 8.6 / 9.9 /
-    14.8; 128 rows: 512 x 512 8.6 / 7.3 / 8.7, 4096 x 4096 36.3 / 19.1 / 27.0, 8192 x 8192 67.7 / 36.5 / 50.5, 14336 x 2048 21.8 / 26.7 / 21.4, 14336 x 8192
-    68.2 / 54.6 / 65.7).  Up to 32 rows the epilogue is ahead of row-major weights at every size."""
+    14.8; 128 rows: 512 x 512 7.2 / 7.4 / 8.8, 4096 x 4096 28.8 / 23.1 / 28.7, 8192 x 8192 62.3 / 55.6 / 66.6; by the epilogue, vendor: 14336 x 2048 26.3 / 34.5,
+    14336 x 8192 89 / 118).  Up to 32 rows the epilogue is ahead of row-major weights at every size."""
     if rows <= STREAM_MAX_ROWS or (k < 1536 and n_out > 4096):
         return 1
     return stream_split_count(n_out, k, rows)
