@@ -77,9 +77,9 @@ __device__ __forceinline__ void prompt_attention(Work& work, char* lds, const bf
                                                  float& m_run, float& l_run) {
   constexpr int QS = DQ / 16, DT = VP / 32, KC = DQ / 8, VC = VP / 8;
   constexpr int N = KEYS / 32, NA = N * QS, NB = 2 * N * DT;   // products of the two halves of a turn
-  constexpr int KL = KC * KEYS / 256, VL = VC * KEYS / 256;    // loads of a wave per tile
+  constexpr int KL = (KC * KEYS + 255) / 256, VL = (VC * KEYS + 255) / 256;   // loads of a wave per tile
   constexpr int K_TILE = KEYS * DQ * 2, V_TILE = KEYS * VP * 2;
-  static_assert((KC * KEYS) % 256 == 0 && (VC * KEYS) % 256 == 0, "whole loads");
+  static_assert((KC * KEYS) % 64 == 0 && (VC * KEYS) % 64 == 0, "whole loads");
   constexpr int LS = NA / 2;                           // slots with loads, from the first
   constexpr int AHEAD = 4, TOP = 3;                    // slots that a fragment is read ahead; first slot with exponentials
   static_assert(NA >= AHEAD && NB >= AHEAD && NA > TOP, "slots");
@@ -92,8 +92,16 @@ __device__ __forceinline__ void prompt_attention(Work& work, char* lds, const bf
   const int n_turns = __builtin_amdgcn_readfirstlane(work.n_turns);
 
   // load i of this wave: chunks 64 (wave + 4 i) + lane of the tile
-  auto k_row = [&](int i) __attribute__((always_inline)) { return (int)((64u * (wave + 4 * i) + lane) / KC); };
-  auto v_row = [&](int i) __attribute__((always_inline)) { return (int)((64u * (wave + 4 * i) + lane) / VC); };
+  // (96 columns of 32 keys: the last load is of two waves only)
+  constexpr bool K_PART = KC * KEYS % 256 != 0, V_PART = VC * KEYS % 256 != 0;
+  auto k_row = [&](int i) __attribute__((always_inline)) {
+    const int r = (int)((64u * (wave + 4 * i) + lane) / KC);
+    return K_PART ? min(r, KEYS - 1) : r;
+  };
+  auto v_row = [&](int i) __attribute__((always_inline)) {
+    const int r = (int)((64u * (wave + 4 * i) + lane) / VC);
+    return V_PART ? min(r, KEYS - 1) : r;
+  };
   // (skipped inside the asm statement: a branch around it would let the compiler move the vector work between the blocks)
   auto to_lds = [&](const void* src, uint32_t dst, int on) __attribute__((always_inline)) {
     asm volatile("s_cmp_eq_u32 %2, 0\n\ts_cbranch_scc1 1f\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off\n1:"
@@ -101,10 +109,12 @@ __device__ __forceinline__ void prompt_attention(Work& work, char* lds, const bf
   };
   auto load_k = [&](int i, int handle, int buf, int on) __attribute__((always_inline)) {
     const int r = k_row(i), c = (int)((64u * (wave + 4 * i) + lane) % KC);
+    if (K_PART) on = on && 64 * (wave + 4 * i) < KC * KEYS;
     to_lds(work.key(handle, c ^ KR::k_turn(r)), base + buf * K_TILE + 1024 * (wave + 4 * i), on);
   };
   auto load_v = [&](int i, int handle, int buf, int on) __attribute__((always_inline)) {
     const int r = v_row(i), c = (int)((64u * (wave + 4 * i) + lane) % VC);
+    if (V_PART) on = on && 64 * (wave + 4 * i) < VC * KEYS;
     to_lds(work.value(handle, c ^ VR::v_turn(r)), base + 2 * K_TILE + buf * V_TILE + 1024 * (wave + 4 * i), on);
   };
   auto landed = [&]() __attribute__((always_inline)) { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
@@ -132,7 +142,7 @@ __device__ __forceinline__ void prompt_attention(Work& work, char* lds, const bf
   auto whole = [](f32x16(&x)[DT]) __attribute__((always_inline)) {
 #pragma unroll
     for (int d = 0; d < DT; ++d) {
-      if constexpr (DQ + VP > 256 && VP > 128) asm volatile("" : "+a"(x[d]));
+      if constexpr (DQ + VP >= 512) asm volatile("" : "+a"(x[d]));
       else asm volatile("" : "+v"(x[d]));
     }
   };
@@ -231,8 +241,8 @@ __device__ __forceinline__ void prompt_attention(Work& work, char* lds, const bf
     if (work.seen(turn)) {
       unrolled<NB>([&](auto i) __attribute__((always_inline)) {
         constexpr int slot = i, d = slot % DT;
-        o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[slot % AHEAD], __builtin_bit_cast(bf16x8_t, pw[slot / DT]), o[d], 0, 0, 0);
-        if constexpr (slot + AHEAD < NB) fr[slot % AHEAD] = read_v(b, slot + AHEAD);
+        o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[(slot + NA) % AHEAD], __builtin_bit_cast(bf16x8_t, pw[slot / DT]), o[d], 0, 0, 0);
+        if constexpr (slot + AHEAD < NB) fr[(slot + NA) % AHEAD] = read_v(b, slot + AHEAD);
         score_slot(i, std::integral_constant<int, NB>{});
         __builtin_amdgcn_sched_barrier(0);
       });

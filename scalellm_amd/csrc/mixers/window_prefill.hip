@@ -1,21 +1,26 @@
 // window_prefill.hip -- windowed grouped-query attention of prompt portions on MFMA: kept first tokens, capped scores,
 // a sink.  The portion's context is a list of cache slots (kept positions, then the window of its first row onwards).
 //
-// Work item: one workgroup = (tile of 128 query rows of one sequence, head), prompt_attn.h; tiles of 64 keys, those of the kept
+// Work item: one workgroup = (tile of 128 query rows of one sequence, head), prompt_attn.h; tiles of 64 or 32 keys, those of the kept
 // tokens, then those of the tile's own window.  The slots of a tile reach LDS three turns ahead of its keys.
 #include "latent/prompt_attn.h"
 #include "window_common.h"
 
 namespace slm {
 
-constexpr int KEYS = 64;   // of a tile
+// Keys of a tile, and waves of a SIMD.  Beside the sums and queries of wide heads the scores of 32 keys leave room for a second wave, and the tiles for a
+// second workgroup on the CU; at 256 + 256 there is none either way.  us, 64 keys and one wave / 32 and two, 16 heads, 4096 rows and 32 heads, 8 x 512 rows
+// of 2200 to 3584: 192 + 128 173 / 144, 410 / 246; 96 + 192 179 / 140, 428 / 245; 64 + 256 195 / 149, 464 / 265; 192 + 256 228 / 247, 539 / 402.  (256 + 256, one wave:
+// 64 keys 234, 556, 32 keys 323, 776.)
+constexpr int window_keys(int columns) { return columns > 256 && columns < 512 ? 32 : 64; }
+constexpr int window_waves(int columns) { return columns < 512 ? 2 : 1; }
 
-template <int DQ, int VP, int GROUPS, bool CAP>
+template <int GROUPS, int KEYS, bool CAP>
 struct WindowWork {
   const slm_window_prefill_args& a;
   int(*const slots)[KEYS];   // of four turns, the present one and the three to come
   const int wave, lane, group;
-  int ctx0, kept, shift, n_keep, lo, hi, n_head, n_tiles, groups, n_turns, next;
+  int ctx0, n_keep, lo, hi, n_head, n_tiles, groups, n_turns, next;
   int qidx, klo, wq0, wq1;          // in context indexes: the lane's row, the first key of its window; the wave's rows
   const bf16 *kc, *vc;
   int k_w, v_w;                     // bytes of a cache row
@@ -26,37 +31,40 @@ struct WindowWork {
   __device__ __forceinline__ int tile_end(int t) const { return t < n_head ? n_keep : hi; }
   __device__ __forceinline__ int slot_of(int turn) const {
     const int t = min(tile_of(turn), n_tiles - 1);
-    return a.slots[ctx0 + min(tile_start(t) + lane, tile_end(t) - 1)];
+    return a.slots[ctx0 + min(tile_start(t) + (lane & (KEYS - 1)), tile_end(t) - 1)];
   }
   __device__ __forceinline__ int row(int turn, int r) const { return slots[turn & 3][r]; }
   __device__ __forceinline__ const void* key(int slot, int c) const { return reinterpret_cast<const char*>(kc + 8 * c) + (int64_t)slot * k_w; }
   __device__ __forceinline__ const void* value(int slot, int c) const { return reinterpret_cast<const char*>(vc + 8 * c) + (int64_t)slot * v_w; }
+  __device__ __forceinline__ void keep(int turn, int slot) {
+    if (KEYS == 64 || lane < KEYS) slots[turn & 3][lane] = slot;
+  }
   __device__ __forceinline__ void start() {
     if (wave == 0)
-      for (int i = 0; i < 3; ++i) slots[i][lane] = slot_of(i);
+      for (int i = 0; i < 3; ++i) keep(i, slot_of(i));
     __syncthreads();
   }
   __device__ __forceinline__ void begin(int turn) {
     if (wave == 0) next = slot_of(turn + 3);
   }
   __device__ __forceinline__ void end(int turn) {
-    if (wave == 0) slots[(turn + 3) & 3][lane] = next;
+    if (wave == 0) keep(turn + 3, next);
   }
   // tiles no row of the wave sees: past its diagonal, before its window
   __device__ __forceinline__ bool seen(int turn) const {
     const int t = tile_of(turn), k0 = tile_start(t);
     return t < n_tiles && k0 <= wq1 && (a.window <= 0 || k0 < n_keep || k0 + KEYS > wq0 - a.window + 1);
   }
-  __device__ __forceinline__ void mask(int turn, f32x16 (&s)[2]) const {
+  __device__ __forceinline__ void mask(int turn, f32x16 (&s)[KEYS / 32]) const {
     const int t = tile_of(turn), k0 = tile_start(t), k_end = tile_end(t);
     if (k0 + KEYS - 1 <= wq0 && k0 + KEYS <= k_end && (a.window <= 0 || k0 >= wq1 - a.window + 1)) return;
-    const int at = k0 + 4 * (lane >> 5), last = min(qidx, k_end - 1) - at, from = klo - at, keep = n_keep - at;
+    const int at = k0 + 4 * (lane >> 5), last = min(qidx, k_end - 1) - at, from = klo - at, kept = n_keep - at;
 #pragma unroll
-    for (int n = 0; n < 2; ++n)
+    for (int n = 0; n < KEYS / 32; ++n)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int k = 32 * n + 8 * (r >> 2) + (r & 3);
-        s[n][r] = (k > last) | ((k < from) & (k >= keep)) ? -INFINITY : s[n][r];
+        s[n][r] = (k > last) | ((k < from) & (k >= kept)) ? -INFINITY : s[n][r];
       }
   }
   // without a cap scale s; with one, cap tanh(s scale / cap) - cap = -2 cap / (1 + exp(2 s scale / cap)): the constant drops
@@ -70,9 +78,9 @@ struct WindowWork {
 };
 
 template <int DQ, int VP, int GROUPS, bool CAP>
-__global__ void __launch_bounds__(256 * GROUPS) __attribute__((amdgpu_waves_per_eu(DQ + VP > 256 ? 1 : 2)))
+__global__ void __launch_bounds__(256 * GROUPS) __attribute__((amdgpu_waves_per_eu(window_waves(DQ + VP))))
 window_prefill_kernel(const slm_window_prefill_args a) {
-  constexpr int QS = DQ / 16, DT = VP / 32;
+  constexpr int QS = DQ / 16, DT = VP / 32, KEYS = window_keys(DQ + VP);
   __shared__ __attribute__((aligned(1024))) char lds[prompt_lds_bytes<DQ, VP, GROUPS, KEYS>()];
   __shared__ int slots[GROUPS][4][KEYS];
 
@@ -87,7 +95,7 @@ window_prefill_kernel(const slm_window_prefill_args a) {
   const int shift = first - kept;                      // position = index + shift behind the kept tokens
   const int qi = min(wave * 32 + l31, n_rows - 1);     // this lane's query row
 
-  WindowWork<DQ, VP, GROUPS, CAP> w{a, slots[group], wave, lane, group};
+  WindowWork<GROUPS, KEYS, CAP> w{a, slots[group], wave, lane, group};
   // context indexes the tile needs: [0, n_keep) and [lo, hi)
   w.ctx0 = ctx0, w.hi = min(ctx_len, pos0 + n_rows - shift);
   w.n_keep = a.window > 0 ? min(max(a.keep_first, 0), w.hi) : 0;
@@ -103,7 +111,7 @@ window_prefill_kernel(const slm_window_prefill_args a) {
   w.kc = reinterpret_cast<const bf16*>(a.key_cache) + (int64_t)g * DQ;
   w.vc = reinterpret_cast<const bf16*>(a.value_cache) + (int64_t)g * VP;
   w.k_w = a.kv_heads * DQ * 2, w.v_w = a.kv_heads * VP * 2;
-    const float cap2 = CAP ? a.softcap * LOG2E_F : 0.f;
+  const float cap2 = CAP ? a.softcap * LOG2E_F : 0.f;
   w.factor = CAP ? 2.0f * LOG2E_F * a.scale / a.softcap : a.scale * LOG2E_F, w.cap_k = CAP ? -0.5f / cap2 : 0.f;
 
   bf16x8_t qf[QS];
