@@ -117,7 +117,7 @@ static bool lp_ok(int dq, int vp) {
 template <int DQ, int VP>
 static void lp_launch(const LatentPrefillK& p, hipStream_t st) {
   const int64_t workgroups = (int64_t)p.a.n_tiles * p.a.heads;
-  if (prompt_two_groups(workgroups, p.a.n_ctx, p.a.n_tiles)) latent_prefill_kernel<DQ, VP, 2><<<dim3((unsigned)workgroups), dim3(512), 0, st>>>(p);
+  if (prompt_two_groups(workgroups, p.a.n_ctx, p.a.n_tiles, p.a.window)) latent_prefill_kernel<DQ, VP, 2><<<dim3((unsigned)workgroups), dim3(512), 0, st>>>(p);
   else latent_prefill_kernel<DQ, VP, 1><<<dim3((unsigned)workgroups), dim3(256), 0, st>>>(p);
 }
 template <int DQ>

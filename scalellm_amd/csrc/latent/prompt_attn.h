@@ -56,11 +56,14 @@ __device__ __forceinline__ int prompt_groups(int tiles) { return GROUPS == 2 && 
 // Two groups up to 256 workgroups, one on each of the CUs: a workgroup's own chain of tiles then sets the time, and half of it
 // is gained; and up to 512 if the prompts are there from their beginnings (no more context rows than rows of the query tiles),
 // whose tiles are unequal: a CU with one workgroup of eight waves takes the next when it is through, where two of four waves
-// leave the long one alone at the end.  From there on one group, whose workgroups overlap each other's beginnings and ends.
+// leave the long one alone at the end.  A window makes their tiles alike; below 2048 keys one group is the better one then, too.
+// From there on one group, whose workgroups overlap each other's beginnings and ends.
 // us, one group / two: window 128 wide, 16 heads, 1 x 1000 rows 33 / 28, 4096 rows (512 workgroups) 131 / 120, 32 heads, 3072
-// rows (768) 114 / 126; latent 192 + 128, 32 heads, 4 x 128 rows of 3200 80 / 67, 8 x 256 rows of 2304 (512) 120 / 145.
-inline bool prompt_two_groups(int64_t workgroups, int64_t n_ctx, int64_t n_tiles) {
-  return workgroups <= 256 || (workgroups <= 512 && n_ctx <= 128 * n_tiles);
+// rows (768) 114 / 126; 4096 rows by the window, 128 keys 26 / 34, 512 40 / 47, 1024 60 / 66, 2048 95 / 103, 3072 106 / 106 (2 x 2048
+// rows: 1536 60 / 63, 2048 67 / 63); latent 192 + 128, 32 heads, 4 x 128 rows of 3200 80 / 67, 8 x 256 rows of 2304 (512) 120 / 145, 16
+// heads, 4096 rows, window 128 29 / 36, 1024 61 / 68.
+inline bool prompt_two_groups(int64_t workgroups, int64_t n_ctx, int64_t n_tiles, int64_t window) {
+  return workgroups <= 256 || (workgroups <= 512 && n_ctx <= 128 * n_tiles && (window <= 0 || window >= 2048));
 }
 
 template <int DQ, int VP, int GROUPS, int KEYS>

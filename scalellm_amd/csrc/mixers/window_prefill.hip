@@ -152,7 +152,7 @@ static void wp_launch(const slm_window_prefill_args& a, hipStream_t st) {
   const std::false_type plain;
   if constexpr (DQ + VP <= 256) {                      // (as wide as two groups' tiles fit)
     const std::integral_constant<int, 2> two;
-    if (prompt_two_groups(workgroups, a.n_ctx, a.n_tiles)) return a.softcap > 0.f ? launch(two, capped) : launch(two, plain);
+    if (prompt_two_groups(workgroups, a.n_ctx, a.n_tiles, a.window)) return a.softcap > 0.f ? launch(two, capped) : launch(two, plain);
   }
   const std::integral_constant<int, 1> one;
   a.softcap > 0.f ? launch(one, capped) : launch(one, plain);
