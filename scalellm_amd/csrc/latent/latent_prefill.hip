@@ -56,8 +56,12 @@ struct LatentWork {
   __device__ __forceinline__ float below(float x, float m) const { return __builtin_fmaf(x, p.scale2, -m); }
 };
 
+// Waves of a SIMD: a third for 64 + 64 columns, whose registers are six too many for it otherwise (32 heads, us, two / three: 4 prompts of 1100 to 2047 68.5 /
+// 62.3, 16 x 512 rows by a window of 512 84 / 76)
+constexpr int latent_waves(int dq, int vp, int groups) { return groups == 1 && dq + vp <= 128 ? 3 : 2; }
+
 template <int DQ, int VP, int GROUPS>
-__global__ void __launch_bounds__(256 * GROUPS) __attribute__((amdgpu_waves_per_eu(2)))
+__global__ void __launch_bounds__(256 * GROUPS) __attribute__((amdgpu_waves_per_eu(latent_waves(DQ, VP, GROUPS))))
 latent_prefill_kernel(const LatentPrefillK p) {
   constexpr int QS = DQ / 16, DT = VP / 32;
   // two workgroups on a CU, or two groups of waves: at most 80 KB each (256 + 128 columns: 112 us with 64 keys, 84 with 32)
