@@ -627,7 +627,7 @@ __global__ void __launch_bounds__(256) attn_combine_kernel(const AttnKParams p, 
   }
 #pragma unroll
   for (int d = 1; d < 64; d <<= 1) L += __shfl_xor(L, d, 64);
-  __builtin_amdgcn_wave_barrier();  // wsm row is wave-private; LDS ops of one wave are ordered
+  wave_lds_order();  // (wsm row is wave-private)
 
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll

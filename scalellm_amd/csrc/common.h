@@ -147,6 +147,14 @@ __device__ __forceinline__ float silu_mul_acc(const float gate_acc, const float 
   return silu_mul1(lo_f32<T>(both), hi_f32<T>(both));
 }
 
+// LDS that a wave has to itself: behind this its lanes read what the others wrote in front.  The hardware takes a wave's LDS operations in order; the
+// fences keep the compiler from another order (no instruction).
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // 8 x silu_mul1, rounded RN to T
 template <typename T>
 __device__ __forceinline__ u32x4 silu_mul8(const u32x4 g, const u32x4 u) {

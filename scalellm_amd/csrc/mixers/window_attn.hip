@@ -169,7 +169,7 @@ __global__ void __launch_bounds__(256) window_attn_any_kernel(const slm_window_a
     l = l * f + wave_sum(e);
     sp[wave][lane] = e;
     ss[wave][lane] = slot;
-    __builtin_amdgcn_wave_barrier();
+    wave_lds_order();
 #pragma unroll
     for (int j = 0; j < WA_MAX / 64; ++j) o[j] *= f;
     for (int t = 0; t < n; ++t) {
@@ -179,7 +179,7 @@ __global__ void __launch_bounds__(256) window_attn_any_kernel(const slm_window_a
       for (int j = 0; j < WA_MAX / 64; ++j)
         if (lane + 64 * j < a.v_pad) o[j] = __builtin_fmaf(e_t, to_f32(v[lane + 64 * j]), o[j]);
     }
-    __builtin_amdgcn_wave_barrier();
+    wave_lds_order();
   }
   if (lane == 0) sm[wave] = m, sl[wave] = l;
 #pragma unroll

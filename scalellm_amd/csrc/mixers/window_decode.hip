@@ -166,9 +166,7 @@ __global__ void __launch_bounds__(256) window_decode_kernel(const WindowDecodeK 
 #pragma unroll
       for (int i = 0; i < NT; ++i) o[i] *= alpha;
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");   // (the tile is the wave's own: order, no barrier)
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    wave_lds_order();   // (the tile is the wave's own)
 #pragma unroll
     for (int i = 0; i < NT; ++i) {
       const uint32_t ad = tr_base + 32u * i;
@@ -177,9 +175,7 @@ __global__ void __launch_bounds__(256) window_decode_kernel(const WindowDecodeK 
       const wdr_v8 v = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
       o[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, v), pf, o[i], 0, 0, 0);
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    wave_lds_order();
   }
   l_run = over_groups(l_run, false);
   if (g == 0) sm[wave][l16] = m_run, sl[wave][l16] = l_run;

@@ -302,7 +302,7 @@ __global__ void __launch_bounds__(256, 1) w4_tile_kernel(const W4TileK a) {
         }
       });
       if constexpr (PAIRS) __syncthreads();
-      else __builtin_amdgcn_wave_barrier();
+      else wave_lds_order();
 #pragma unroll 1
       for (int i0 = 0; i0 < TURNS; i0 += AT_ONCE) {
         f32x4 v[AT_ONCE][2], u[AT_ONCE][2];
@@ -337,7 +337,7 @@ __global__ void __launch_bounds__(256, 1) w4_tile_kernel(const W4TileK a) {
           }
         }
       }
-      if constexpr (!PAIRS) __builtin_amdgcn_wave_barrier();
+      if constexpr (!PAIRS) wave_lds_order();
     }
   };
   if (a.silu) a.bias ? out(std::true_type{}, std::true_type{}) : out(std::true_type{}, std::false_type{});
