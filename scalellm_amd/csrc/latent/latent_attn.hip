@@ -746,5 +746,7 @@ extern "C" SLM_API int slm_latent_attn_values(const slm_latent_attn_args* a, con
       (v->epilogue == SLM_LIN_GATE && !v->gate))
     return SLM_ERR_INVALID_ARG;
   if (!aligned16(v->w)) return SLM_ERR_ALIGNMENT;
+  const int rc = linear_check(v);   // (whichever way it goes, and in front of the attention)
+  if (rc != SLM_OK) return rc;
   return la_run(a, v, stream);
 }

@@ -111,6 +111,9 @@ __device__ __forceinline__ int seq_of_row(const int32_t* q_cu, int batch, int ro
 
 constexpr float M_INIT_F = -1.0e30f;
 
+// what slm_linear refuses (linear.hip)
+int linear_check(const slm_linear_args* a);
+
 // barrier for LDS traffic only: outstanding global loads (register prefetch) stay in flight
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 

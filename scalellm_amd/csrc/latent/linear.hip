@@ -215,11 +215,7 @@ static int lin_epi(const slm_linear_args& a, hipStream_t st) {
   }
 }
 
-}  // namespace slm
-
-using namespace slm;
-
-static int lin_check(const slm_linear_args* a) {
+int linear_check(const slm_linear_args* a) {
   if (!a || !a->x || !a->w || !a->y || a->M < 0 || a->N <= 0 || a->K <= 0 || a->K % 64 || a->N % 16 || a->batch < 1 ||
       a->n_splits < 1 || a->ldx < a->K || a->ldw < a->K || a->epilogue < 0 || a->epilogue > SLM_LIN_GATE)
     return SLM_ERR_INVALID_ARG;
@@ -234,8 +230,12 @@ static int lin_check(const slm_linear_args* a) {
   return SLM_OK;
 }
 
+}  // namespace slm
+
+using namespace slm;
+
 extern "C" SLM_API int slm_linear(const slm_linear_args* a, void* stream) {
-  const int rc = lin_check(a);
+  const int rc = linear_check(a);
   if (rc != SLM_OK) return rc;
   if (a->M == 0) return SLM_OK;
   return a->dtype == SLM_BF16 ? lin_epi<bf16>(*a, (hipStream_t)stream) : lin_epi<float>(*a, (hipStream_t)stream);
@@ -246,7 +246,7 @@ extern "C" SLM_API int slm_linear(const slm_linear_args* a, void* stream) {
 // 128 rows of 32 heads 1129 / 1124.)
 // And only where the product reads no column that the rotation writes (K is the queries' unrotated width, without padding).
 extern "C" SLM_API int slm_latent_append_absorb(const slm_latent_append_args* c, const slm_linear_args* a, void* stream) {
-  const int rc = lin_check(a);
+  const int rc = linear_check(a);
   if (rc != SLM_OK) return rc;
   if (latent_append_invalid(c)) return SLM_ERR_INVALID_ARG;
   if (a->epilogue != SLM_LIN_STORE || a->dtype != c->dtype) return SLM_ERR_INVALID_ARG;

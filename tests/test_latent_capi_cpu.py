@@ -78,6 +78,16 @@ def test_invalid_arguments_come_back_as_status():
     assert L.slm_latent_attn_values(C.byref(b), C.byref(v), None) == -5
     v.w, v.epilogue = 4096, _lib.LIN_GATE
     assert L.slm_latent_attn_values(C.byref(b), C.byref(v), None) == -1   # no gate
+    # what slm_linear refuses is refused in front of the attention's launch (there is no device here: a launch is another error)
+    b.dtype, b.max_kv_len = _lib.SLM_BF16, 64
+    b.q_abs = b.cache = b.out = b.positions = b.q_cu = b.block_table = b.block_cu = 4096
+    v.x, v.epilogue, v.M, v.K, v.ldx, v.ldw, v.batch, v.dtype = 4096, _lib.LIN_STORE, 3, 64, 256, 64, 4, _lib.SLM_BF16
+    for field, bad, rc in (("x", None, -1), ("K", 63, -1), ("ldx", 32, -1), ("ldw", 32, -1), ("batch", 0, -1), ("dtype", 0, -2), ("ldx", 260, -5),
+                           ("x_batch", 4, -5), ("w_batch", 4, -5), ("x", 4104, -5)):
+        keep = getattr(v, field)
+        setattr(v, field, bad)
+        assert L.slm_latent_attn_values(C.byref(b), C.byref(v), None) == rc, field
+        setattr(v, field, keep)
     assert L.slm_latent_gather(None, None, None, 1, 64, None) == -1
     for args in ((None, 4096, 64, 64, 0), (4096, 4096, 72, 64, 0), (4096, 4096, 64, 72, 0), (4096, 4096, 96, 64, 1)):
         assert L.slm_stream_layout(*args, None) == -1
