@@ -670,6 +670,7 @@ __global__ void __launch_bounds__(64 * W, 2) recurrent_scan_kernel(const slm_rec
   // a chunk's record is a buffer: a load is one instruction (of 64-bit addresses half of a chunk's 215 instructions were additions)
   const int rec_bytes = (int)at.size() * 4;
   const uint32_t off = (uint32_t)(lane * 16), koff = off + wave * (TPW * 1024), goff = (uint32_t)(g * 16 + wave * (TPW * 64) + ChunkRecord<DK>::GE * 4);
+  static_assert(NCT == 1 || NCT % 2 == 0, "half of the column tiles' read-outs under the writes, half under the reads");
   constexpr int PIECES = TPW * (DELTA ? 4 : 3) + 2 * NCT, SLOTS = 4 * ((DELTA ? 2 : 1) * NCT + 1);
   auto record = [&](int c) { return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(rec0 + c * rec_step), 0, rec_bytes, 0x00020000); };
   auto load = [&](const __amdgpu_buffer_rsrc_t& rec, ChunkOperands<TPW, NCT>& x, int k) {   // k-th of PIECES
