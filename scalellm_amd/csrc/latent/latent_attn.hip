@@ -635,7 +635,8 @@ static void la_values_launch(const LatentAttnK& p, const slm_linear_args& v, int
 }
 // Rows of a head per workgroup, as many as leave one round of workgroups; 0: two launches.  Those where there are fewer than 128 pairs of row and head: one
 // row's 128 splits are then a quarter of a megabyte for each of few workgroups, where the merge by itself spreads them over the chip (1 row, 32 heads:
-// 9.4 us the two).
+// 9.4 us the two).  Of values wider than a workgroup's 128 columns several workgroups merge the same splits, which pays only where all of them are one
+// round (256 wide, us, two launches / one: 16 heads 8 rows of 1500 keys 17.9 / 16.5, 16 rows of 300 16.2 / 19.5; 32 heads 8 rows of 1500 20.7 / 23.8).
 static int la_values_rows(const LatentAttnK& p, const slm_linear_args& v) {
   const slm_latent_attn_args& a = p.a;
   if (v.x != a.out || v.M != a.rows || v.K != a.c_pad || v.ldw != v.K || v.x_batch != a.c_pad || v.ldx != (int64_t)a.heads * a.c_pad || v.batch != a.heads ||
@@ -643,7 +644,9 @@ static int la_values_rows(const LatentAttnK& p, const slm_linear_args& v) {
     return 0;
   const int64_t pairs = a.rows * a.heads;
   const int64_t r = std::min<int64_t>(16, (pairs + 255) / 256);
-  return pairs >= 128 * r && r * p.n_splits <= LA_VALUES_WEIGHTS && (a.rows + r - 1) / r <= 65535 ? (int)r : 0;
+  const int64_t row_blocks = (a.rows + r - 1) / r;
+  if (v.N > 128 && a.heads * row_blocks * ((v.N + 127) / 128) > 256) return 0;
+  return pairs >= 128 * r && r * p.n_splits <= LA_VALUES_WEIGHTS && row_blocks <= 65535 ? (int)r : 0;
 }
 
 template <int KP, int RP, int MH>

@@ -446,12 +446,13 @@ def test_latent_attention_sizes(c_pad, r_pad, heads, dtype):
 
 
 # The merge and the product behind it in one launch against the two: rows that leave the last workgroup of a head short, one row a workgroup and
-# sixteen, splits by the rule and forced (two launches for few rows, one split, or more weights than fit), columns below, at and past a workgroup's 128, with the gate and without.  The merged
-# rows are rounded to 16 bits either way; another order of the splits' sums moves a rounding now and then, so 2^-8 of a few of a product's terms.
+# sixteen, splits by the rule and forced (two launches for few rows, one split, or more weights than fit), columns below, at and past a workgroup's
+# 128 (then two launches, unless all workgroups are one round), with the gate and without.  The merged rows are rounded to 16 bits either way; another order of the splits' sums moves a rounding now and then, so 2^-8 of a few of a product's terms.
 @pytest.mark.parametrize("c_pad,heads,vdim,rows,n_splits,one_launch", [
-    (512, 16, 128, 9, 0, True), (512, 32, 128, 33, 0, True), (512, 32, 128, 4, 0, True), (512, 16, 128, 1, 0, False), (512, 24, 144, 100, 2, True),
+    (512, 16, 128, 9, 0, True), (512, 32, 128, 33, 0, True), (512, 32, 128, 4, 0, True), (512, 16, 128, 1, 0, False), (512, 24, 144, 100, 2, False),
     (256, 40, 96, 30, 3, True), (256, 16, 32, 33, 0, True), (128, 48, 64, 31, 5, True), (64, 17, 48, 90, 8, True), (64, 64, 16, 127, 2, True),
-    (512, 128, 128, 1, 128, True), (64, 160, 32, 2, 100, True), (512, 16, 128, 40, 1, False), (64, 64, 16, 127, 40, False), (256, 127, 32, 1, 4, False)])
+    (512, 128, 128, 1, 128, True), (64, 160, 32, 2, 100, True), (512, 16, 128, 40, 1, False), (64, 64, 16, 127, 40, False), (256, 127, 32, 1, 4, False),
+    (512, 24, 128, 100, 2, True), (512, 32, 144, 4, 0, True), (256, 16, 256, 8, 3, True), (256, 16, 256, 9, 3, False)])
 def test_latent_attention_with_its_values(c_pad, heads, vdim, rows, n_splits, one_launch):
     lk, r_pad, dt = _lk(), 64, torch.bfloat16
     lens = [40 + 53 * i % 700 for i in range(rows)]
