@@ -120,7 +120,7 @@ typedef struct slm_latent_attn_args {
 SLM_API size_t slm_latent_attn_workspace_bytes(const slm_latent_attn_args* a);
 SLM_API int slm_latent_attn(const slm_latent_attn_args* a, void* stream);
 /* slm_latent_attn, then slm_linear (STORE or GATE) of a->out's heads; one launch less, and nothing written to a->out, where the    */
-/* ranges are split and enough rows and heads fill the chip                                             */
+/* ranges are split and enough rows and heads fill the chip in one round.  What either refuses is refused before anything runs */
 SLM_API int slm_latent_attn_values(const slm_latent_attn_args* a, const slm_linear_args* values, void* stream);
 /* 1 if the MFMA kernel serves these sizes, 0: the any-size kernel */
 SLM_API int slm_latent_attn_is_mfma(int32_t c_pad, int32_t r_pad, int32_t dtype);

@@ -2,7 +2,7 @@
 //
 // Four waves, one to a SIMD, hold a quarter of the tile each: 128 x 128 products of 16 x 16 x 32 in 256 accumulators read 0.5 KB
 // of LDS per 1024 matrix-pipe cycles and SIMD, where eight waves of 128 x 64 read 0.75 -- and what bounds a large product here is power
-// (8192^3: 572 us on zeros, 724 on normal numbers), which operand traffic is part of (with 32 x 32 x 16 products 6 % more).  The
+// (8192^3: 576 us on zeros, 718 on normal numbers), which operand traffic is part of (with 32 x 32 x 16 products 6 % more).  The
 // accumulators are pinned to the second half of the register file by inline asm: left to itself the compiler spreads them over
 // both and copies 1000 registers a step.
 //
@@ -14,19 +14,19 @@
 // more).  256 x 256: 160 KB of LDS.
 //
 // A workgroup goes from tile to tile: the DMA of a tile's last steps brings the first stages of the next one, which so are there when the
-// epilogue ends.  That is 5 us of a tile's 97 (256 x 256, K 4096), but power takes most of it back: 5692 x 28672 x 4096 992 -> 978 us,
-// 4096 x 8512 x 2048 122 -> 118, 3226 x 16896 x 4096 358 -> 352, 5692 x 4096 x 14336 502 -> 498.  (Where it goes in the loop matters: sources chosen by
+// epilogue ends.  That is 5 us of a tile's 97 (256 x 256, K 4096), but power takes most of it back (us, both timed in turn): 3226 x 16896 x 4096
+// 358 -> 350, 4096 x 8512 x 2048 119 -> 115, 4096 x 16384 x 4096 395 -> 388, 5692 x 4096 x 14336 492 -> 490, 8192^3 level.  (Where it goes in the loop matters: sources chosen by
 // the step cost 3 % of every product; the steps come in parts instead.)
 //
 // Tiles that do not fill the last round of the chip are cut in K (slices > 1): every slice leaves fp32 sums past the caches, the last one
 // to arrive (a counter per tile) adds them up in slice order and stores.  Nobody waits for anybody.
 //
-// us by the device, vendor product (and the GLU's launch) / this, normal numbers: 5692 x 28672 x 4096 GLU 1073 / 978 (1.37 PFLOP/s),
-// 5692 x 4096 x 14336 740 / 497, 5692 x 4096 x 4096 149 / 146, 3226 x 28672 x 4096 GLU 708 / 560, 3226 x 16896 x 4096 449 / 351, 4096 x 16384 x 2048 GLU
-// 230 / 209, 4096 x 8512 x 2048 155 / 118, 1000 x 4096 x 14336 134 / 109, 600 x 28672 x 4096 GLU 148 / 134, 300 x 4096 x 14336 70 / 63,
-// 207 x 16384 x 2048 GLU 31 / 24.  Behind the vendor product where its tiles fill whole rounds (8192^3 691 / 728, 4096^3 89 / 96), with one row of tiles
-// over large weights (129 x 28672 x 4096 56 / 70), and on short and narrow products (207 x 4096 x 4096 17.6 / 20.1, 207 x 3664 x 2048 11.1 / 14.6,
-// 207 x 512 x 2048 8.4 / 15.3), which its callers take here for the sake of the host.
+// us by the device, vendor product (and the GLU's launch) / this, normal numbers: 5692 x 28672 x 4096 GLU 1069 / 975 (1.37 PFLOP/s),
+// 5692 x 4096 x 14336 737 / 490, 5692 x 4096 x 4096 148 / 145, 3226 x 28672 x 4096 GLU 703 / 559, 3226 x 16896 x 4096 441 / 350, 4096 x 16384 x 2048 GLU
+// 226 / 206, 4096 x 8512 x 2048 152 / 115, 1000 x 4096 x 14336 131 / 108, 600 x 28672 x 4096 GLU 147 / 132, 300 x 4096 x 14336 72 / 64,
+// 207 x 16384 x 2048 GLU 30 / 22.  Behind the vendor product where its tiles fill whole rounds (8192^3 678 / 718, 4096^3 89 / 94), with one row of tiles
+// over large weights (129 x 28672 x 4096 GLU 59 / 74), and on short and narrow products (207 x 4096 x 4096 17.5 / 20.6, 207 x 3664 x 2048 11.1 / 14.9,
+// 207 x 512 x 2048 8.5 / 15.8), which its callers take here for the sake of the host.
 #include "latent_common.h"
 #include "tile_common.h"
 
@@ -244,7 +244,8 @@ __global__ void __launch_bounds__(256, 1) gemm_kernel(const GemmK a) {
 }
 
 // Tiles, and what they take: us of a step of 64 k alone on the chip and with every CU busy (power), and of a tile beside its steps.
-// Fitted to 900 timings of 90 products of 65 - 5700 rows; by them the tile taken is 0.5 % behind the best one on average, 10 % at worst.
+// Fitted to 900 timings of 90 products of 65 - 5700 rows, with a workgroup for each tile.  Since workgroups go from tile to tile the tile taken is 0.8 %
+// behind the best one on average (154 products of 161 - 8400 rows); constants fitted to these were 0.9 % behind.
 struct GemmTile {
   int bm, bn;
   float step, busy, rest;

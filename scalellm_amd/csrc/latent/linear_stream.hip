@@ -340,7 +340,7 @@ static int wave_n_launch(const slm_linear_args& a, hipStream_t st) {
 // Up to 16 rows the widest tile whose workgroups leave no round of the 256 CUs more than a quarter empty: fewer, longer
 // runs (28672 columns, 1 row: NT 4 37.7 us, NT 1 45; 16896 columns, a second round of 8 workgroups: 32 against 29.3).
 // With more rows the columns of a wave weigh against the rounds they need, ties to the wider (x is read half as often):
-// 64 rows x 28672 44 us against 51, 64 rows x 16384 19.3 against 14.8.  Up to 32 rows and under 112 panels the chip is
+// 64 rows x 28672 x 4096 41 us against 48, 64 rows x 16384 x 2048 20.6 against 15.7.  Up to 32 rows and under 112 panels the chip is
 // filled by 32-column tiles (6784 columns: 15.6 us against 18.4).
 template <int EPI>
 static int stream_shape(const slm_linear_args& a, hipStream_t st) {

@@ -14,7 +14,7 @@
 //            in registers from the portion's first token to its last; the products are 32-bit MFMAs.  Bound: a chain of two products and an
 //            exchange a chunk, 0.6 us (24 products of 32 cycles a wave are 0.35), and the instructions around them.
 //   Both, us, 16 heads of 128 x 128 and 4096 tokens: delta 305 with the triangular system and B U in the scan, 64-bit addresses and a wave's
-//   read-outs by itself, 212 now; lightning 184 and 131; 8 x 500 tokens, 32 heads: 341 and 293, 209 and 181; 16 heads of 64, 2000 tokens: 120 and 82.
+//   read-outs by itself, 212 now; lightning 184 and 133; 8 x 500 tokens, 32 heads: 341 and 285, 209 and 178; 16 heads of 64, 2000 tokens: 120 and 75.
 //   gated_norm  the norm and gate behind a scan.
 #include "latent/latent_common.h"
 #include "slm_mixers.h"

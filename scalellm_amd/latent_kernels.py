@@ -241,10 +241,10 @@ def _store_rows(N: int, K: int) -> int:
 
 def _tile_pays(M: int, N: int, K: int, glu: bool) -> bool:
     """Is a product that the tile kernel takes its own, or the vendor's?  us by the device, vendor / tiles, where they are the vendor's:
-    129 - 160 rows of large weights, whose one row of tiles reads them slower (28672 x 4096 GLU 62 / 77, from 161 rows 67 / 65; of the largest up to 192
+    129 - 160 rows of large weights, whose one row of tiles reads them slower (28672 x 4096 GLU 59 / 74, from 161 rows 67 / 65; of the largest up to 192
     rows: 16384 x 8192, 170 rows, 75 / 93), and
-    256 x 256 tiles that fill whole rounds of the chip (4096 x 4096, K 2048 49 / 54, 4096 90 / 97; 4096 x 16384 x 4096 364 / 398).
-    Short and narrow products are up to 8 us longer by the device (200 x 512 x 2048 8 / 15, 200 x 4096 x 4096 18 / 21) and stay here all the same: steps
+    256 x 256 tiles that fill whole rounds of the chip (4096 x 4096, K 2048 49 / 53, 4096 89 / 94; 4096 x 16384 x 4096 363 / 388).
+    Short and narrow products are up to 8 us longer by the device (207 x 512 x 2048 8.5 / 15.8, 207 x 4096 x 4096 17.5 / 20.6) and stay here all the same: steps
     with prompts run eagerly, and the vendor product takes 8 us more of the host for each (18 / 10).  Steps of four layers with one prompt of
     150 - 300 tokens, all their products by the vendor / here: 2b 847 / 580 and 836 / 618, 8b 975 / 903 and 1189 / 1065."""
     if 128 < M <= (192 if N * K >= 1 << 27 else 160) and N * K >= 1 << 26:

@@ -447,7 +447,8 @@ def test_latent_attention_sizes(c_pad, r_pad, heads, dtype):
 
 # The merge and the product behind it in one launch against the two: rows that leave the last workgroup of a head short, one row a workgroup and
 # sixteen, splits by the rule and forced (two launches for few rows, one split, or more weights than fit), columns below, at and past a workgroup's
-# 128 (then two launches, unless all workgroups are one round), with the gate and without.  The merged rows are rounded to 16 bits either way; another order of the splits' sums moves a rounding now and then, so 2^-8 of a few of a product's terms.
+# 128 (then two launches, unless all workgroups are one round), with the gate and without.  The merged rows are rounded to 16 bits either way; another
+# order of the splits' sums moves a rounding now and then, so 2^-8 of a few of a product's terms.
 @pytest.mark.parametrize("c_pad,heads,vdim,rows,n_splits,one_launch", [
     (512, 16, 128, 9, 0, True), (512, 32, 128, 33, 0, True), (512, 32, 128, 4, 0, True), (512, 16, 128, 1, 0, False), (512, 24, 144, 100, 2, False),
     (256, 40, 96, 30, 3, True), (256, 16, 32, 33, 0, True), (128, 48, 64, 31, 5, True), (64, 17, 48, 90, 8, True), (64, 64, 16, 127, 2, True),
