@@ -234,8 +234,9 @@ def _store_rows(N: int, K: int) -> int:
     """Rows up to which a product that is only stored is streamed.  Without slabs its workgroups are its columns': from 33
     rows the vendor GEMM, which splits K for itself, is level or ahead under 8192 columns (6752 x 4096, 64 rows: 17.8 us
     against 21.8) and a little above where K is long (vendor / streamed, 64 rows: 8192 x 2048 13.7 / 12.4, x 4096 18.6 / 21.9, x 8192
-    32.7 / 41.0; 9216 x 4096 26.4 / 22.5, x 8192 40.2 / 42.1; 12288 x 8192 44.8 / 43.1).  Above 64 rows it is level for wide products
-    (16896 x 4096: 128 rows 42.1 / 43.0, 64 rows 39.6 / 33.9; 12608 x 4096, 85 rows 29.0 / 25.7) and far ahead for narrow ones."""
+    32.7 / 41.0; 9216 x 4096 26.4 / 22.5, x 8192 40.2 / 42.1; 12288 x 8192 44.8 / 43.1).  Above 64 rows it is far ahead for
+    narrow products; of the widest up to 96 rows it is 2 to 3 us behind (12608 x 4096, 85 rows 29.0 / 25.7; 12288 x 2048, 96 rows 17.2 / 15.3), which this
+    line doesn't follow, and level from there on (16896 x 4096, 128 rows 42.1 / 43.0; 64 rows 39.6 / 33.9)."""
     return 64 if N >= 8192 and K <= 2048 + 5 * (N - 8192) // 2 else STREAM_MAX_ROWS
 
 
