@@ -16,9 +16,9 @@
 // Tiles reach LDS without registers (global_load_lds), two K and two V tiles; K is loaded two tiles ahead and V one, one
 // barrier a tile.  Such a load writes 1 KB in lane order, so rows have no padding and their 16-byte chunks are permuted
 // instead: 16 rows of K, or 4 rows x 64 bytes of V, meet all 64 banks.
-// Against products and vector work one after the other, one K and one V tile through registers and two barriers a tile, us:
-// window 128 wide with a cap, 16 heads, 4096 rows 151 -> 120; 32 heads, 8 x 512 rows of 2200 to 3584 280 -> 244; latent
-// 192 + 128, 32 heads, 4 prompts of 1100 to 2047 144 -> 137.  There 26 of 137 are the loads (36 % miss L2; 32 KB of a CU are
+// Against products and vector work one after the other, one K and one V tile through registers and two barriers a tile, us, in turn:
+// window 128 wide with a cap, 16 heads, 4096 rows 142 -> 103; 32 heads, 8 x 512 rows of 2200 to 3584 264 -> 222; latent
+// 192 + 128, 32 heads, 4 prompts of 1100 to 2047 141 -> 123.  There 26 of 137 are the loads (36 % miss L2; 32 KB of a CU are
 // in flight).  Rescaling only after the maximum has grown by 2^8 takes 3 % off, but the largest weight is then no longer a
 // 16-bit number and the error grows by 5 %.
 #pragma once
@@ -186,17 +186,23 @@ __device__ __forceinline__ void prompt_attention(Work& work, char* lds, const bf
   score_slot(std::integral_constant<int, 0>{}, std::integral_constant<int, 1>{});
   landed();   // (the first tile of K is read before the third is loaded over it)
 
-  for (int turn = 0; turn < n_turns; ++turn) {
-    const int b = turn & 1, more_k = turn + 2 < n_turns, more_v = turn + 1 < n_turns;
-    work.begin(turn);
+  // The last turn is code of its own: there is no tile behind it whose scores to multiply and cap, a quarter of a chain of three tiles' (us: latent 64 + 32 / 64
+  // columns, 32 heads, 16 x 512 rows by a window of 64 47 / 44; window 128 wide with a cap, 16 heads, 4096 rows 108 / 103, 32 heads, 8 x 512 rows of 2200 to 3584
+  // 229 / 222).
+  auto one_turn = [&](int turn, auto is_last) __attribute__((always_inline)) {
+    constexpr bool LAST = decltype(is_last)::value;
+    const int b = turn & 1, more_k = turn + 2 < n_turns;
+    if (!LAST) work.begin(turn);
     asm volatile("" : "+v"(k_at), "+v"(v_x), "+v"(k_lane), "+v"(v_lane));   // (their combinations are not kept over the turns)
     int rows[KL + VL];
     auto row = [&](auto l) __attribute__((always_inline)) {
       if constexpr (l < KL) rows[l] = work.row(turn + 2, k_row(l));
       else if constexpr (l < KL + VL) rows[l] = work.row(turn + 1, v_row(l - KL));
     };
-    unrolled<2>(row);
-    unrolled<AHEAD>([&](auto i) __attribute__((always_inline)) { fr[i] = read_k(1 - b, i); });
+    if constexpr (!LAST) {
+      unrolled<2>(row);
+      unrolled<AHEAD>([&](auto i) __attribute__((always_inline)) { fr[i] = read_k(1 - b, i); });
+    }
     work.mask(turn, s);
     whole(o);
     __builtin_amdgcn_sched_barrier(0);
@@ -204,13 +210,13 @@ __device__ __forceinline__ void prompt_attention(Work& work, char* lds, const bf
     u32x4 pw[2 * N];
     unrolled<NA>([&](auto i) __attribute__((always_inline)) {
       constexpr int slot = i;
-      product_a(i, 1 - b);
+      if constexpr (!LAST) product_a(i, 1 - b);
       if constexpr (slot + AHEAD >= NA) fr[slot % AHEAD] = read_v(b, slot + AHEAD - NA);
       constexpr int l0 = std::min(slot * (KL + VL) / LS, KL + VL), l1 = std::min((slot + 1) * (KL + VL) / LS, KL + VL);
-      unrolled<l1 - l0>([&](auto e) __attribute__((always_inline)) {
+      unrolled<LAST ? 0 : l1 - l0>([&](auto e) __attribute__((always_inline)) {
         constexpr int l = l0 + e;
         if constexpr (l < KL) load_k(l, rows[l], b, more_k);
-        else load_v(l - KL, rows[l], 1 - b, more_v);
+        else load_v(l - KL, rows[l], 1 - b, 1);
         row(std::integral_constant<int, l + 2>{});
       });
       if constexpr (slot < 2) {
@@ -249,20 +255,25 @@ __device__ __forceinline__ void prompt_attention(Work& work, char* lds, const bf
         constexpr int slot = i, d = slot % DT;
         o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[(slot + NA) % AHEAD], __builtin_bit_cast(bf16x8_t, pw[slot / DT]), o[d], 0, 0, 0);
         if constexpr (slot + AHEAD < NB) fr[(slot + NA) % AHEAD] = read_v(b, slot + AHEAD);
-        score_slot(i, std::integral_constant<int, NB>{});
+        if constexpr (!LAST) score_slot(i, std::integral_constant<int, NB>{});
         __builtin_amdgcn_sched_barrier(0);
       });
-    } else {                                           // (no row of the wave sees a key of this tile: p is 0, V is not touched)
+    } else if constexpr (!LAST) {                      // (no row of the wave sees a key of this tile: p is 0, V is not touched)
       unrolled<1>([&](auto i) __attribute__((always_inline)) { score_slot(i, std::integral_constant<int, 1>{}); });
     }
-    work.end(turn);
-    landed();
-  }
+    if constexpr (!LAST) {
+      work.end(turn);
+      landed();
+    }
+  };
+  for (int turn = 0; turn + 1 < n_turns; ++turn) one_turn(turn, std::false_type{});
+  one_turn(n_turns - 1, std::true_type{});
 
   whole(o);
   l_run += __shfl_xor(l_run, 32, 64);
   if constexpr (GROUPS == 2) {
     if (work.groups == 1) return;
+    lds_barrier();                                     // (the last tiles are read)
     static_assert(DT * 4 * 256 * 16 + 2048 <= prompt_lds_bytes<DQ, VP, 2, KEYS>(), "the sums of the second group");
     float* const ml = reinterpret_cast<float*>(lds) + tid;
     f32x4* const part = reinterpret_cast<f32x4*>(lds + 2048) + tid;
