@@ -18,8 +18,8 @@
 // instead: 16 rows of K, or 4 rows x 64 bytes of V, meet all 64 banks.
 // Against products and vector work one after the other, one K and one V tile through registers and two barriers a tile, us, in turn:
 // window 128 wide with a cap, 16 heads, 4096 rows 142 -> 103; 32 heads, 8 x 512 rows of 2200 to 3584 264 -> 222; latent
-// 192 + 128, 32 heads, 4 prompts of 1100 to 2047 141 -> 123.  There 26 of 137 are the loads (36 % miss L2; 32 KB of a CU are
-// in flight).  Rescaling only after the maximum has grown by 2^8 takes 3 % off, but the largest weight is then no longer a
+// 192 + 128, 32 heads, 4 prompts of 1100 to 2047 141 -> 123.  There 26 were the loads, of 137 (36 % miss L2;
+// 32 KB of a CU are in flight).  Rescaling only after the maximum has grown by 2^8 takes 3 % off, but the largest weight is then no longer a
 // 16-bit number and the error grows by 5 %.
 #pragma once
 #include <algorithm>
