@@ -287,6 +287,7 @@ def latent_lib() -> C.CDLL:
         ("slm_residual_norm", C.c_int, [P(ResidualNormArgs), ptr]),
         ("slm_linear", C.c_int, [P(LinearArgs), ptr]),
         ("slm_linear_stream", C.c_int, [P(LinearArgs), ptr]),
+        ("slm_linear_stream_half", C.c_int, [P(LinearArgs), ptr]),
         ("slm_gemm_workspace_bytes", C.c_size_t, [P(LinearArgs), i32, i32]),
         ("slm_gemm", C.c_int, [P(LinearArgs), ptr, C.c_size_t, i32, i32, ptr]),
         ("slm_stream_layout", C.c_int, [ptr, ptr, i64, i64, i32, ptr]),

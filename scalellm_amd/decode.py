@@ -21,7 +21,7 @@ from typing import List, Optional
 
 import torch
 
-from . import kernels
+from . import build as slm_build, kernels, latent_kernels as lk
 from .layers import (Attention, ColumnParallelQLinear, HipAttnHandler, InputParameters, KVCache, uniform_kv_hint,
                      QuantArgs, RowParallelQLinear)
 from .model_parallel import ParallelArgs
@@ -267,6 +267,7 @@ class LlamaDecodeStep:
         lm_head = (torch.randn(H, shape.vocab, device=self.device, generator=gen) * 0.02).to(dtype)
         self.lm_head = lm_head[:, r * shape.vocab // tp:(r + 1) * shape.vocab // tp].contiguous()
         del embed, lm_head
+        self._head_layout: Optional[torch.Tensor] = None   # of lm_head, for steps of few rows (_lay_out_head)
         self.kv_head0 = kv_head0
         T = max_batch_tokens
         e = lambda *s: torch.empty(*s, dtype=dtype, device=self.device)  # noqa: E731
@@ -328,6 +329,31 @@ class LlamaDecodeStep:
                 kernels.reserve_workspace(need_for(rows), self.device, deferred_nbytes=16 * rows * widest * 4)
         if 0 < h0 < n_tokens and self._side_stream is None:
             self._side_stream = torch.cuda.Stream(device=self.device)
+        if not torch.cuda.is_current_stream_capturing():
+            self._lay_out_head()
+
+    # elements of a vocabulary product from which its weight is laid out once more for few rows: below, both ways are a launch of 2 to 6 us
+    HEAD_LAYOUT_MIN = 1 << 22
+
+    def _lay_out_head(self) -> None:
+        """lm_head in the order the streamed product reads it, where half of the memory that is left holds it: up to 128 rows of logits are then one linear
+        read (us, 16 bits, vendor product / streamed: 32768 x 4096 1 row 52 / 42, 32 rows 51 / 43, 128 rows 57 / 52; 128256 x 4096 190 / 157, 204 / 168,
+        244 / 231; 8192 x 1024 9.1 / 4.7, 12.0 / 6.3, 13.9 / 9.9)."""
+        w = self.lm_head
+        if self._head_layout is not None and lk.layout_is_current(self._head_layout, w):
+            return
+        self._head_layout = None
+        if not w.is_cuda or w.numel() < self.HEAD_LAYOUT_MIN or (w.size(1) + 63) // 64 * 64 * w.size(0) * w.element_size() > lk.spare_memory(w.device):
+            return
+        slm_build.ensure("latent")
+        try:
+            self._head_layout = lk.stream_layout_columns(w)
+        except torch.OutOfMemoryError:
+            pass
+
+    def weights_version(self):
+        """Changes when lm_head is changed in place or replaced while products read a copy of it (None: they read the weight itself)."""
+        return None if self._head_layout is None else (self.lm_head.data_ptr(), self._head_layout.copy_of._version)
 
     # ------------------------------------------------------------------------------------------
     # One decoder stack over a range of token rows ("lane").  A step normally has ONE lane (all rows,
@@ -734,7 +760,7 @@ class LlamaDecodeStep:
             self.last_hidden = last = kernels.last_rows(normed, q_cu)
         else:
             self.last_hidden = last = normed[(q_cu[1:] - 1).long()]
-        logits = last @ self.lm_head  # plain library GEMM (hipBLASLt): not on the graded path
+        logits = lk.linear_columns(last, self.lm_head, self._head_layout)
         if ar is not None and not return_logits and last.size(0) <= ar.max_tokens \
                 and 4 * pa.world_size <= s.hidden:
             return self._greedy_over_vocab_shards(logits, ar)

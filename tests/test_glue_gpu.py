@@ -294,3 +294,35 @@ def test_last_hidden_of_a_step_outlives_the_next_one():
     assert torch.equal(rows @ model.lm_head, logits)
     model.forward((tokens + 1) % model.shape.vocab, positions, params)
     assert torch.equal(hidden, rows) and not torch.equal(model.last_hidden, rows)
+
+
+def test_logits_of_a_head_that_is_laid_out_once_more():
+    """Up to 128 rows from the copy, as long as lm_head is what it was: changed in place or replaced, products are its own; both hosts give the same bits.  One
+    rounding to 8 significant bits."""
+    from scalellm_amd import cpp_host
+    from scalellm_amd.decode import LlamaDecodeStep, LlamaShape, make_decode_inputs
+    shape = LlamaShape(hidden=512, n_heads=8, n_kv_heads=2, head_dim=64, intermediate=512, n_layers=1, vocab=8208, max_position=128)
+    tokens, positions, params, n_blocks = make_decode_inputs(130, 20, 16, torch.device(DEV), seed=3, vocab=shape.vocab)
+    model = LlamaDecodeStep(shape, 130, n_blocks, 16, dtype=torch.bfloat16, device=torch.device(DEV), kv_fill="randn", keep_checkpoint=True)
+    assert model.weights_version() is None
+    model.reserve_workspaces(130, 20)
+    assert model._head_layout is not None
+    for n in (130, 3):
+        t, p, prm, _ = make_decode_inputs(n, 20, 16, torch.device(DEV), seed=3, vocab=shape.vocab)
+        got = model.forward(t, p, prm, return_logits=True)
+        want = model.last_hidden.double() @ model.lm_head.double()
+        assert (got.double() - want).abs().max() <= 2.0 ** -8 * 1.02 * want.abs().max()
+        cpp = cpp_host.from_decode_step(model, 16, 130)
+        assert torch.equal(cpp.decode_step(t, p, cpp_host.cpp_params(prm), True), got)
+    version = model.weights_version()
+    model.lm_head[:, 5] = 0.0
+    assert model.weights_version() != version
+    assert not model.forward(t, p, prm, return_logits=True)[:, 5].any()
+    version, model.lm_head = model.weights_version(), model.lm_head + 1.0
+    assert model.weights_version() != version
+    got = model.forward(t, p, prm, return_logits=True)
+    assert torch.equal(got, model.last_hidden @ model.lm_head)
+    model.reserve_workspaces(130, 20)
+    again = model.forward(t, p, prm, return_logits=True)
+    want = model.last_hidden.double() @ model.lm_head.double()
+    assert model._head_layout.copy_of is model.lm_head and (again.double() - want).abs().max() <= 2.0 ** -8 * 1.02 * want.abs().max()
