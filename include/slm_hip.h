@@ -351,6 +351,11 @@ SLM_API int slm_w4a16_gemv_norm(const slm_w4_gemm_args* a, const slm_w4_norm_pro
 /* Slow dequantise-to-dense helper (debug / parity): w_out [K, N] T.          */
 SLM_API int slm_w4_dequant(const void* wq, const void* sz, int64_t K, int64_t N,
                            int64_t group_size, int32_t dtype, void* w_out, void* stream);
+/* The same as rows: w_out [N, K] T, 16-byte aligned; of a paired weight the  */
+/* gate's rows, then the up half's.  Made once per weight, for slm_gemm.      */
+SLM_API int slm_w4_dequant_rows(const void* wq, const void* sz, int64_t K, int64_t N,
+                                int64_t group_size, int32_t dtype, int32_t paired, void* w_out,
+                                void* stream);
 
 /* ========================================================================== */
 /* 5. Glue ops of one decoder layer.                                          */

@@ -161,6 +161,9 @@ def lib() -> C.CDLL:
         ("slm_w4_dequant", C.c_int,
          [C.c_void_p, C.c_void_p, C.c_int64, C.c_int64, C.c_int64, C.c_int32, C.c_void_p,
           C.c_void_p]),
+        ("slm_w4_dequant_rows", C.c_int,
+         [C.c_void_p, C.c_void_p, C.c_int64, C.c_int64, C.c_int64, C.c_int32, C.c_int32, C.c_void_p,
+          C.c_void_p]),
         ("slm_rms_norm", C.c_int,
          [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int64, C.c_int64, C.c_float,
           C.c_int32, C.c_void_p]),
@@ -290,6 +293,7 @@ def latent_lib() -> C.CDLL:
         ("slm_linear_stream_half", C.c_int, [P(LinearArgs), ptr]),
         ("slm_gemm_workspace_bytes", C.c_size_t, [P(LinearArgs), i32, i32]),
         ("slm_gemm", C.c_int, [P(LinearArgs), ptr, C.c_size_t, i32, i32, ptr]),
+        ("slm_gemm_half", C.c_int, [P(LinearArgs), ptr, C.c_size_t, i32, i32, ptr]),
         ("slm_stream_layout", C.c_int, [ptr, ptr, i64, i64, i32, ptr]),
         ("slm_clamped_glu", C.c_int, [ptr, ptr, i64, i64, i64, i64, f32, f32, f32, i32, ptr]),
         ("slm_glu_slabs", C.c_int, [ptr, ptr, i64, i64, i32, i64, f32, f32, f32, ptr]),

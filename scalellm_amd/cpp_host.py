@@ -1,7 +1,7 @@
 """Python handle on the C++ HOST STEP (csrc/shim/slm_llama_hip.{h,cpp}: slm::LlamaForCausalLMHip, the
 decoder stack of src/models/meta/llama.h:123-345 composed in C++ from the layer classes of
-csrc/shim/) -- what `bench.py --host cpp` times and tests/test_cpp_host_step_gpu.py holds
-bit-identical to the Python mirror (decode.LlamaDecodeStep).  Nothing here computes: it loads
+csrc/shim/) -- what `bench.py --host cpp` times and tests/test_cpp_host_step_gpu.py holds bit-identical to
+the Python mirror (decode.LlamaDecodeStep; its steps of many rows apart, once they run on 16-bit copies of the weights).  Nothing here computes: it loads
 _slm_shim.so, hands it the checkpoint-format tensors under their HuggingFace names, the KV cache
 tensors and the step's integer inputs."""
 from __future__ import annotations

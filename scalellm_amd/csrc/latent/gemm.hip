@@ -1,4 +1,4 @@
-// gemm.hip -- y = x W^T in bf16 for many rows (prompts, mixed steps), from row-major x and W, with the GLU as an epilogue.
+// gemm.hip -- y = x W^T in bf16 or half precision for many rows (prompts, mixed steps), from row-major x and W, with the GLU as an epilogue.
 //
 // Four waves, one to a SIMD, hold a quarter of the tile each: 128 x 128 products of 16 x 16 x 32 in 256 accumulators read 0.5 KB
 // of LDS per 1024 matrix-pipe cycles and SIMD, where eight waves of 128 x 64 read 0.75 -- and what bounds a large product here is power
@@ -27,6 +27,8 @@
 // 207 x 16384 x 2048 GLU 30 / 22.  Behind the vendor product where its tiles fill whole rounds (8192^3 678 / 718, 4096^3 89 / 94), with one row of tiles
 // over large weights (129 x 28672 x 4096 GLU 59 / 74), and on short and narrow products (207 x 4096 x 4096 17.5 / 20.6, 207 x 3664 x 2048 11.1 / 14.9,
 // 207 x 512 x 2048 8.5 / 15.8), which its callers take here for the sake of the host.
+#include <type_traits>
+
 #include "latent_common.h"
 #include "tile_common.h"
 
@@ -35,7 +37,7 @@ namespace slm {
 struct GemmK {
   const char* x;
   const char* w;
-  bf16* y;
+  uint16_t* y;
   float* slabs;            // [tiles cut][slices][fragments][256] f32x4
   uint32_t* arrived;       // [tiles cut], zero
   int64_t M, N, K, ldy;
@@ -44,11 +46,14 @@ struct GemmK {
   float limit, alpha, shift;
 };
 
-__device__ __forceinline__ void gemm_product(f32x4& c, const bf16x8_t& w, const bf16x8_t& x) {
-  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(w), "v"(x));
+// T: bf16_tag or f16_tag
+template <typename T>
+__device__ __forceinline__ void gemm_product(f32x4& c, const u32x4& w, const u32x4& x) {
+  if constexpr (std::is_same<T, bf16_tag>::value) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(w), "v"(x));
+  else asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(c) : "v"(w), "v"(x));
 }
 
-template <int BM, int BN, int WS, bool GLU>
+template <typename T, int BM, int BN, int WS, bool GLU>
 __global__ void __launch_bounds__(256, 1) gemm_kernel(const GemmK a) {
   constexpr int XS = 3;                              // stages of x; WS: of w
   constexpr int XB = BM * 128, WB = BN * 128;        // bytes of a stage
@@ -128,11 +133,11 @@ __global__ void __launch_bounds__(256, 1) gemm_kernel(const GemmK a) {
   // Columns of a pair of tiles go to them by fours, so that a lane ends with eight neighbours.  Chunk c of a row of w lies in slot
   // c ^ (row % 4 + 4 (row / 8 % 2)): eight lanes read eight slots of either matrix.
   const int xrow = wm * (BM / 2) + r16, wrow = wn * (BN / 2) + 8 * (r16 >> 2) + (r16 & 3);
-  bf16x8_t fx[2][MT], fw[2][NT];                // operands of the two halves
+  u32x4 fx[2][MT], fw[2][NT];                   // operands of the two halves
   auto read = [&](int j, int h, uint32_t xa, uint32_t wa) {   // j-th of R
     const int slot = ((h * 4 + g) ^ (r16 & 7)) << 4;   // (of w: row % 4 = r16 % 4, row / 8 % 2 = r16 / 4 % 2: the same)
-    if (j < MT) fx[h][j] = *reinterpret_cast<const bf16x8_t*>(lds + xa + (xrow + 16 * j) * 128 + slot);
-    else fw[h][j - MT] = *reinterpret_cast<const bf16x8_t*>(lds + XS * XB + wa + (wrow + 32 * ((j - MT) >> 1) + 4 * ((j - MT) & 1)) * 128 + slot);
+    if (j < MT) fx[h][j] = *reinterpret_cast<const u32x4*>(lds + xa + (xrow + 16 * j) * 128 + slot);
+    else fw[h][j - MT] = *reinterpret_cast<const u32x4*>(lds + XS * XB + wa + (wrow + 32 * ((j - MT) >> 1) + 4 * ((j - MT) & 1)) * 128 + slot);
   };
   // (rows there and back: a product takes one operand of the one before it, which is 0.5 % of a large product's time)
   auto turn = [](int q) { return q / MT % 2 ? MT - 1 - q % MT : q % MT; };
@@ -174,7 +179,7 @@ __global__ void __launch_bounds__(256, 1) gemm_kernel(const GemmK a) {
           for (int i = b * XD / R; i < (b + 1) * XD / R; ++i) dma(i, kx, xl);
           read(b, 1, xa, wa);
 #pragma unroll
-          for (int q = b * MM / R; q < (b + 1) * MM / R; ++q) gemm_product(acc[q / MT][turn(q)], fw[0][q / MT], fx[0][turn(q)]);
+          for (int q = b * MM / R; q < (b + 1) * MM / R; ++q) gemm_product<T>(acc[q / MT][turn(q)], fw[0][q / MT], fx[0][turn(q)]);
           __builtin_amdgcn_sched_barrier(0);
         }
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(LATE) : "memory");
@@ -184,7 +189,7 @@ __global__ void __launch_bounds__(256, 1) gemm_kernel(const GemmK a) {
           if (b < WD) dma(XD + b, kw, wa);
           read(b, 0, xn, wnext);
 #pragma unroll
-          for (int q = b * MM / R; q < (b + 1) * MM / R; ++q) gemm_product(acc[q / MT][turn(q)], fw[1][q / MT], fx[1][turn(q)]);
+          for (int q = b * MM / R; q < (b + 1) * MM / R; ++q) gemm_product<T>(acc[q / MT][turn(q)], fw[1][q / MT], fx[1][turn(q)]);
           __builtin_amdgcn_sched_barrier(0);
         }
         kw = min(kw + 128, last);
@@ -217,7 +222,7 @@ __global__ void __launch_bounds__(256, 1) gemm_kernel(const GemmK a) {
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
       const int row = cur.m0 + wm * (BM / 2) + 16 * m + e16;
-      bf16* y = a.y + row * a.ldy;
+      uint16_t* y = a.y + row * a.ldy;
 #pragma unroll
       for (int n = 0; n < (GLU ? NT / 2 : NT); n += 2) {
         const int col = cur.n0 + wn * (GLU ? BN / 4 : BN / 2) + 16 * n + 8 * eg;
@@ -227,7 +232,8 @@ __global__ void __launch_bounds__(256, 1) gemm_kernel(const GemmK a) {
           o[j] = acc[n + (j >> 2)][m][j & 3];
           if constexpr (GLU) o[j] = clamped_glu_f32(o[j], acc[n + (j >> 2) + NT / 2][m][j & 3], a.limit, a.alpha, a.shift);
         }
-        if (row < a.M && col < (GLU ? half : (int)a.N)) store_f32<8>(y + col, o);
+        if (row < a.M && col < (GLU ? half : (int)a.N))
+          *reinterpret_cast<u32x4*>(y + col) = u32x4{pack2<T>(o[0], o[1]), pack2<T>(o[2], o[3]), pack2<T>(o[4], o[5]), pack2<T>(o[6], o[7])};
       }
 #pragma unroll
       for (int n = 0; n < NT; ++n) {
@@ -307,10 +313,10 @@ static GemmPlan gemm_plan(const slm_linear_args& a, int tile, int slices) {
   return best;
 }
 
-template <int BM, int BN, int WS, bool GLU>
+template <typename T, int BM, int BN, int WS, bool GLU>
 static int gemm_launch(const GemmK& k, hipStream_t st) {
   constexpr int bytes = (3 * BM + WS * BN) * 128;
-  auto fn = gemm_kernel<BM, BN, WS, GLU>;
+  auto fn = gemm_kernel<T, BM, BN, WS, GLU>;
   static bool asked[64] = {};
   tile_allow_lds(fn, bytes, asked);
   // A workgroup goes from one to the next only where the shortest, the last slice, is long enough to load the next one's first stages, and a slice
@@ -321,29 +327,29 @@ static int gemm_launch(const GemmK& k, hipStream_t st) {
   fn<<<dim3(wgs), dim3(256), bytes, st>>>(k);
   return hip_check_launch();
 }
-template <bool GLU>
+template <typename T, bool GLU>
 static int gemm_tile(const GemmPlan& p, const GemmK& k, hipStream_t st) {
   switch (p.tile) {
-    case 0: return gemm_launch<256, 256, 2, GLU>(k, st);
-    case 1: return gemm_launch<256, 128, 3, GLU>(k, st);
-    case 2: return gemm_launch<128, 128, 3, GLU>(k, st);
-    case 3: return gemm_launch<128, 256, 3, GLU>(k, st);
-    case 5: return gemm_launch<192, 256, 2, GLU>(k, st);
-    case 6: return gemm_launch<160, 256, 3, GLU>(k, st);
+    case 0: return gemm_launch<T, 256, 256, 2, GLU>(k, st);
+    case 1: return gemm_launch<T, 256, 128, 3, GLU>(k, st);
+    case 2: return gemm_launch<T, 128, 128, 3, GLU>(k, st);
+    case 3: return gemm_launch<T, 128, 256, 3, GLU>(k, st);
+    case 5: return gemm_launch<T, 192, 256, 2, GLU>(k, st);
+    case 6: return gemm_launch<T, 160, 256, 3, GLU>(k, st);
     default:
-      if constexpr (!GLU) return gemm_launch<256, 192, 2, GLU>(k, st);
+      if constexpr (!GLU) return gemm_launch<T, 256, 192, 2, GLU>(k, st);
       return SLM_ERR_UNSUPPORTED;
   }
 }
 
 // What the kernel takes: 16-byte rows, byte offsets of 32 bits
-static int gemm_check(const slm_linear_args* a, int tile, int slices) {
+static int gemm_check(const slm_linear_args* a, int tile, int slices, int dtype) {
   if (!a || !a->x || !a->w || !a->y || a->M < 0 || a->N <= 0 || a->K <= 0 || a->K % 64 || a->N % 16 || a->batch != 1 || a->n_splits != 1 ||
       a->ldx < a->K || a->ldw < a->K || (a->epilogue != SLM_LIN_STORE && a->epilogue != SLM_LIN_GLU) || tile < -1 || tile >= GEMM_N_TILES || slices < 0)
     return SLM_ERR_INVALID_ARG;
   const bool glu = a->epilogue == SLM_LIN_GLU;
   if (a->ldy < (glu ? a->N / 2 : a->N)) return SLM_ERR_INVALID_ARG;
-  if (a->dtype != SLM_BF16 || (glu && (a->N % 32 || tile == GEMM_256_192))) return SLM_ERR_UNSUPPORTED;
+  if (a->dtype != dtype || (glu && (a->N % 32 || tile == GEMM_256_192))) return SLM_ERR_UNSUPPORTED;
   if (a->ldx % 8 || a->ldw % 8 || a->ldy % 8 || !aligned16(a->x) || !aligned16(a->w) || !aligned16(a->y)) return SLM_ERR_ALIGNMENT;
   const int64_t most = 1ll << 31;
   if (a->M > most / 2 / a->ldx || a->N > most / 2 / a->ldw || a->M > (1 << 24) || a->N > (1 << 24)) return SLM_ERR_UNSUPPORTED;
@@ -355,17 +361,18 @@ static int gemm_check(const slm_linear_args* a, int tile, int slices) {
 using namespace slm;
 
 extern "C" SLM_API size_t slm_gemm_workspace_bytes(const slm_linear_args* a, int32_t tile, int32_t slices) {
-  return gemm_check(a, tile, slices) == SLM_OK && a->M ? gemm_plan(*a, tile, slices).bytes : 0;
+  return gemm_check(a, tile, slices, SLM_BF16) == SLM_OK && a->M ? gemm_plan(*a, tile, slices).bytes : 0;
 }
 
-extern "C" SLM_API int slm_gemm(const slm_linear_args* a, void* workspace, size_t workspace_bytes, int32_t tile, int32_t slices, void* stream) {
-  const int rc = gemm_check(a, tile, slices);
+template <typename T>
+static int gemm_run(const slm_linear_args* a, void* workspace, size_t workspace_bytes, int32_t tile, int32_t slices, void* stream) {
+  const int rc = gemm_check(a, tile, slices, std::is_same<T, bf16_tag>::value ? SLM_BF16 : SLM_F16);
   if (rc != SLM_OK || a->M == 0) return rc;
   GemmPlan p = gemm_plan(*a, tile, slices);
   if (p.cut && (!workspace || workspace_bytes < p.bytes)) p = gemm_plan(*a, tile, 1);   // (no scratch: no cut)
   if (p.cut && !aligned16(workspace)) return SLM_ERR_ALIGNMENT;
   GemmK k{};
-  k.x = (const char*)a->x; k.w = (const char*)a->w; k.y = (bf16*)a->y;
+  k.x = (const char*)a->x; k.w = (const char*)a->w; k.y = (uint16_t*)a->y;
   k.M = a->M; k.N = a->N; k.K = a->K; k.ldy = a->ldy; k.ldx2 = (uint32_t)(a->ldx * 2); k.ldw2 = (uint32_t)(a->ldw * 2);
   k.limit = a->limit; k.alpha = a->glu_alpha; k.shift = a->glu_shift;
   k.mb = p.mb; k.nb = p.nb; k.whole = p.whole; k.cut = p.cut; k.slices = p.slices; k.group = 8;
@@ -373,5 +380,11 @@ extern "C" SLM_API int slm_gemm(const slm_linear_args* a, void* workspace, size_
   hipStream_t st = (hipStream_t)stream;
   hip_clear_error();
   if (p.cut) tile_clear_kernel<<<dim3(1), dim3(256), 0, st>>>(k.arrived, p.cut);
-  return a->epilogue == SLM_LIN_GLU ? gemm_tile<true>(p, k, st) : gemm_tile<false>(p, k, st);
+  return a->epilogue == SLM_LIN_GLU ? gemm_tile<T, true>(p, k, st) : gemm_tile<T, false>(p, k, st);
+}
+extern "C" SLM_API int slm_gemm(const slm_linear_args* a, void* workspace, size_t workspace_bytes, int32_t tile, int32_t slices, void* stream) {
+  return gemm_run<bf16_tag>(a, workspace, workspace_bytes, tile, slices, stream);
+}
+extern "C" SLM_API int slm_gemm_half(const slm_linear_args* a, void* workspace, size_t workspace_bytes, int32_t tile, int32_t slices, void* stream) {
+  return gemm_run<f16_tag>(a, workspace, workspace_bytes, tile, slices, stream);
 }

@@ -127,6 +127,27 @@ __global__ void __launch_bounds__(256) w4_dequant_kernel(const uint32_t* __restr
   }
 }
 
+// The same as rows W[N, K], of a paired weight all of the gate's, then the up's: what products of many rows multiply by where there is memory for it.
+// A wave has a packed tile, 32 rows of 128 bytes, each of them written whole (four layers of the 8b size, 1.7 GB of rows, beside the other preparations of a
+// model: by the kernel above and a transposition 5.4 ms, 1.5 with their allocation).
+template <typename T>
+__global__ void __launch_bounds__(256) w4_dequant_rows_kernel(const u32x4* __restrict__ wq, const uint32_t* __restrict__ sz, int64_t K, int64_t N, int64_t gs,
+                                                              int paired, uint16_t* __restrict__ w_out) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x, tile = i >> 6, n_tiles = N >> 5, nt = tile % n_tiles, kt = tile / n_tiles;
+  if (kt * 64 >= K) return;
+  const int lane = (int)(i & 63), c = lane & 31, h = lane >> 5;
+  const u32x4 w = wq[i];
+  uint16_t* const row = w_out + (paired ? (nt & 1) * (N / 2) + (nt >> 1) * 32 + c : nt * 32 + c) * K;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int64_t k = kt * 64 + 16 * j + 8 * h;
+    const W4Dq<T> dq(sz[k / gs * N + nt * 32 + c]);
+    uint32_t o[4];
+    dq.word(w[j], o);
+    *reinterpret_cast<u32x4*>(row + k) = u32x4{o[0], o[1], o[2], o[3]};
+  }
+}
+
 // A'[m, k] = A[m, perm[k]]  (act-order; reference permute_cols_kernel gptq_gemm.cu:69-118)
 __global__ void __launch_bounds__(256) w4_permute_cols_kernel(const uint16_t* __restrict__ a,
                                                               const int* __restrict__ perm,
@@ -986,6 +1007,21 @@ SLM_API int slm_w4_dequant(const void* wq, const void* sz, int64_t K, int64_t N,
                        (const uint32_t*)sz, K, N, group_size, (uint16_t*)w_out);
   else
     return SLM_ERR_UNSUPPORTED;
+  return hip_check_launch();
+}
+
+SLM_API int slm_w4_dequant_rows(const void* wq, const void* sz, int64_t K, int64_t N, int64_t group_size, int32_t dtype, int32_t paired, void* w_out,
+                                void* stream) {
+  if (!wq || !sz || !w_out) return SLM_ERR_INVALID_ARG;
+  if (K <= 0 || N <= 0 || K % 64 || N % (paired ? 64 : 32) || group_size < 16 || K % group_size || group_size % 8) return SLM_ERR_UNSUPPORTED;
+  if (dtype != SLM_F16 && dtype != SLM_BF16) return SLM_ERR_UNSUPPORTED;
+  if (!aligned16(wq) || !aligned16(w_out)) return SLM_ERR_ALIGNMENT;
+  const int64_t blocks = (K * N / 32 + 255) / 256;
+  if (blocks > 0x7fffffff) return SLM_ERR_UNSUPPORTED;
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  hip_clear_error();
+  auto fn = dtype == SLM_BF16 ? w4_dequant_rows_kernel<bf16_tag> : w4_dequant_rows_kernel<f16_tag>;
+  fn<<<dim3((unsigned)blocks), dim3(256), 0, st>>>((const u32x4*)wq, (const uint32_t*)sz, K, N, group_size, paired, (uint16_t*)w_out);
   return hip_check_launch();
 }
 

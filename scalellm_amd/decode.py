@@ -305,7 +305,7 @@ class LlamaDecodeStep:
                         seg.copy_(blk[:seg.numel()])
 
     def reserve_workspaces(self, n_tokens: int, max_kv_len: int) -> None:
-        """Grow the kernel workspace once, before graph capture."""
+        """Grow the kernel workspace once, before graph capture, and lay weights out once more for the steps of up to n_tokens rows."""
         s = self.shape
 
         def need_for(rows: int) -> int:
@@ -331,6 +331,17 @@ class LlamaDecodeStep:
             self._side_stream = torch.cuda.Stream(device=self.device)
         if not torch.cuda.is_current_stream_capturing():
             self._lay_out_head()
+            self._lay_out_dense(n_tokens)
+
+    def _lay_out_dense(self, n_tokens: int) -> None:
+        """16-bit copies of the linears' weights for steps of many rows, where such come and half of the memory that is left holds them."""
+        linears = [L[name] for L in self.layers for name in ("qkv", "o", "gate_up", "down")]
+        if not linears or n_tokens < linears[0].dense_rows() or not self.lm_head.is_cuda:
+            return
+        slm_build.ensure("latent")
+        spare = lk.spare_memory(self.lm_head.device)
+        for linear in linears:
+            spare -= linear.lay_out_dense(spare)
 
     # elements of a vocabulary product from which its weight is laid out once more for few rows: below, both ways are a launch of 2 to 6 us
     HEAD_LAYOUT_MIN = 1 << 22

@@ -770,6 +770,15 @@ def w4_dequant(packed: PackedW4) -> torch.Tensor:
     return w
 
 
+def w4_dequant_rows(packed: PackedW4) -> torch.Tensor:
+    """The same as rows [N, K]; of a paired weight all of the gate's, then the up half's."""
+    L = _lib.lib()
+    w = torch.empty(packed.N, packed.K, dtype=packed.dtype, device=packed.wq.device)
+    check(L.slm_w4_dequant_rows(packed.wq.data_ptr(), packed.sz.data_ptr(), packed.K, packed.N, packed.group_size,
+                                SLM_BF16 if packed.dtype == torch.bfloat16 else SLM_F16, int(packed.paired), w.data_ptr(), _stream()), "slm_w4_dequant_rows")
+    return w
+
+
 # ---------------------------------------------------------------------------------------
 # glue ops (next rows f1/f2)
 # ---------------------------------------------------------------------------------------

@@ -257,10 +257,12 @@ def _gemm(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, glu=None, tile: i
     """out = x w^T, or with glu = (limit, alpha, shift) the clamped GLU of its halves, by the tile kernel for many rows.  False:
     shapes and strides that it does not take."""
     M, N, K = x.size(0), w.size(0), w.size(1)
-    if (x.dtype != torch.bfloat16 or not N or not K or K % 64 or N % (32 if glu else 16) or x.stride(0) < K or (x.stride(0) | w.stride(0) | out.stride(0)) % 8 or
+    half = x.dtype == torch.float16
+    if (not (half or x.dtype == torch.bfloat16) or w.dtype != x.dtype or out.dtype != x.dtype or not N or not K or K % 64 or N % (32 if glu else 16) or x.stride(0) < K or (x.stride(0) | w.stride(0) | out.stride(0)) % 8 or
             (x.data_ptr() | w.data_ptr() | out.data_ptr()) % 16 or max(M * x.stride(0), N * w.stride(0)) > 1 << 30 or max(M, N) > 1 << 24):
         return False
-    a = _linear_args(x, w, M, N, K)
+    a = _lib.LinearArgs()
+    a.x, a.w, a.M, a.N, a.K, a.alpha, a.batch, a.n_splits, a.dtype = _p(x), _p(w), M, N, K, 1.0, 1, 1, SLM_BF16
     a.ldx, a.ldw, a.ldy, a.y, a.epilogue = x.stride(0), w.stride(0), out.stride(0), _p(out), _lib.LIN_STORE
     if glu:
         a.epilogue, a.limit, a.glu_alpha, a.glu_shift = _lib.LIN_GLU, *glu
@@ -271,8 +273,13 @@ def _gemm(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, glu=None, tile: i
             ws = torch.empty(need, dtype=torch.uint8, device=x.device)
         except torch.OutOfMemoryError:
             need = 0
-    latent_check(L.slm_gemm(C.byref(a), ws.data_ptr() if ws is not None else None, need, tile, slices, _stream()), "slm_gemm")
+    if half:
+        a.dtype = _lib.SLM_F16
+    latent_check((L.slm_gemm_half if half else L.slm_gemm)(C.byref(a), ws.data_ptr() if ws is not None else None, need, tile, slices, _stream()), "slm_gemm")
     return True
+
+
+gemm = _gemm   # (for other modules)
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None, layout: Optional[torch.Tensor] = None) -> torch.Tensor:

@@ -19,12 +19,13 @@ the reference so parity tests read like the reference's own layer tests.
 """
 from __future__ import annotations
 
+import math
 from dataclasses import dataclass, field
 from typing import Dict, Optional, Sequence, Tuple
 
 import torch
 
-from . import kernels
+from . import kernels, latent_kernels as lk
 from .model_parallel import (ParallelArgs, gather_from_model_parallel_region,
                              reduce_from_model_parallel_region)
 
@@ -247,6 +248,7 @@ class _QLinearBase:
         self.bias: Optional[torch.Tensor] = None
         self._ckpt: Dict[str, torch.Tensor] = {}
         self._packed: Optional[kernels.PackedW4] = None
+        self._dense: Optional[torch.Tensor] = None   # lay_out_dense()
         self.paired = False  # merged [gate | up] weight packed for the fused SiLU*mul epilogue
 
     # checkpoint-format tensors for THIS rank's shard
@@ -254,7 +256,7 @@ class _QLinearBase:
         for name in ("qweight", "qzeros", "scales", "g_idx", "bias"):
             if name in sd:
                 self._ckpt[name] = sd[name].to(self.device)
-        self._packed = None
+        self._packed = self._dense = None
 
     def verify_loaded_weights(self) -> None:
         for name in ("qweight", "qzeros", "scales"):
@@ -280,12 +282,45 @@ class _QLinearBase:
                                         dim=1).reshape(-1).contiguous()
         self._ckpt = {}
 
+    def dense_rows(self) -> int:
+        """Rows from which products run on the 16-bit copy where there is one.  A tile of int4 weights becomes 16-bit operands once for each of its row
+        blocks, 1.2 vector instructions beside each product, which shows wherever a full chip's power isn't the limit (a layer's four products by themselves,
+        us, int4 / copy: 8b bf16 400 rows 245 / 242, 640 309 / 293, 2183 850 / 775, 5120 1830 / 1649; half precision, whose int4 kernels are the older ones, 320 rows
+        243 / 210, 2183 979 / 814; 2b bf16 512 rows 113 / 109, 2183 308 / 273, half 320 rows 112 / 101, 2183 433 / 283).  Below, int4 is a quarter of the bytes
+        (8b, 129 rows, gate_up 56 / 77).  Eager steps of four layers with one prompt, us: 8b bf16 210 rows 820 / 851, 290 929 / 965, 340 1027 / 1015, 400 1132 /
+        1069; half 210 rows 828 / 853, 290 1068 / 971."""
+        return 288 if self.dtype == torch.float16 else 384
+
+    def lay_out_dense(self, spare: int) -> int:
+        """The weight in 16 bits, [N, K] row-major ([gate | up] of a merged one), the values products of many rows make of int4 for every tile: once, where
+        `spare` bytes hold it.  Returns the bytes it took.  Weights whose sums keep their order (PackedW4.any_order), act-order and 8-bit ones have none."""
+        if self._dense is not None:
+            return 0
+        if self._packed is None:
+            self._repack()
+        p = self._packed
+        groups = p.group_size in (32, 64, p.K) or (p.group_size >= 128 and p.group_size & (p.group_size - 1) == 0)   # (what the int4 products take)
+        if not groups or not p.any_order or p.perm is not None or p.k_src != p.K or p.K % 128 or p.N % 32 or 2 * p.N * p.K > spare:
+            return 0
+        try:
+            self._dense = kernels.w4_dequant_rows(p)
+        except torch.OutOfMemoryError:
+            return 0
+        return 2 * p.N * p.K
+
     def _gemm(self, x: torch.Tensor, bias: Optional[torch.Tensor],
               out: Optional[torch.Tensor], defer_splitk: bool = False,
               norm: Optional[kernels.NormPrologue] = None) -> torch.Tensor:
         if self._packed is None:
             self._repack()
         x2 = x.reshape(-1, x.size(-1))
+        if self._dense is not None and bias is None and norm is None and x2.size(0) >= self.dense_rows() and x2.size(1) == self._packed.K:
+            if out is None:
+                out = torch.empty(x2.size(0), self._packed.N // (2 if self.paired else 1), dtype=x.dtype, device=x.device)
+            kernels._gemm_args(x2, self._packed, out, None, self.paired)   # (what the int4 product refuses)
+            if lk.gemm(x2, self._dense, out, (math.inf, 1.0, 0.0) if self.paired else None):
+                self.deferred, self.deferred_splits = kernels.DeferredPartials(), 0
+                return out
         if self.paired:
             if out is None:
                 out = torch.empty(x2.size(0), self._packed.N // 2, dtype=x.dtype, device=x.device)

@@ -206,6 +206,25 @@ def test_tiled_products(M, N, K, slices, tile):
         assert glu[:, N // 2:].isnan().all()
 
 
+# The same in half precision: every tile, rows and columns that fill none, tiles that are cut, and more of them than CUs.
+@pytest.mark.parametrize("tile", range(7))
+@pytest.mark.parametrize("M,N,K,slices", [(1, 32, 64, 1), (300, 544, 704, 3), (2300, 7456, 192, 1)])
+def test_tiled_products_in_half_precision(M, N, K, slices, tile):
+    lk = _lk()
+    x = _rnd(1, M, K + 8, dtype=torch.float16)[:, :K]
+    w = _rnd(2, N, K, dtype=torch.float16, std=K ** -0.5)
+    want = x.double() @ w.double().t()
+    wide = torch.full((M, N + 16), float("nan"), dtype=torch.float16, device=DEV)
+    assert lk.gemm(x, w, wide[:, 8:8 + N], None, tile, slices)
+    assert (wide[:, 8:8 + N].double() - want).abs().max() <= 2.0 ** -11 * 1.02 * want.abs().max()
+    assert wide[:, :8].isnan().all() and wide[:, 8 + N:].isnan().all()
+    if tile != 4:   # (that one has no GLU)
+        glu = torch.full((M, N // 2 + 8), float("nan"), dtype=torch.float16, device=DEV)
+        assert lk.gemm(x, w, glu[:, :N // 2], (0.6, lk.GLU_ALPHA, lk.GLU_SHIFT), tile, slices)
+        out = torch.from_numpy(ref.clamped_glu(want[:, :N // 2].cpu().numpy(), want[:, N // 2:].cpu().numpy(), 0.6)).to(DEV)
+        assert (glu[:, :N // 2].double() - out).abs().max() <= 2.0 ** -11 * 1.05 * out.abs().max() and glu[:, N // 2:].isnan().all()
+
+
 # More tiles than CUs, so that a workgroup goes from one to the next: steps at, one and two past the stages that are loaded ahead, two rounds and
 # three, a last round that is cut, also so that its last slice is at the stages (then a workgroup has one item, as with K 192 and three of them).
 @pytest.mark.parametrize("tile", range(7))

@@ -861,3 +861,56 @@ def test_four_wave_tiles_are_taken_where_a_call_allows_it():
         torch.cuda.synchronize()
         assert torch.equal(c, old) != moved
         assert _rel_err(c.float().cpu().numpy(), old.float().cpu().numpy()) < 2e-3
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("K,N,gs,fmt", [(64, 64, 32, "awq"), (192, 320, 64, "awq"), (1152, 96, 128, "gptq"), (576, 128, -1, "awq")])
+def test_rows_of_dequantised_weights(K, N, gs, fmt, dtype):
+    """The same bits as the [K, N] form; of a paired weight the gate's rows, then the up half's."""
+    from scalellm_amd import kernels
+    case = helpers.make_quant_case(3, K, N, gs, fmt, dtype)
+    for paired in (False, True) if N % 64 == 0 else (False,):
+        p = helpers.pack_case(case, dtype, paired=paired)
+        w = kernels.w4_dequant(p).t()
+        if paired:
+            w = w.reshape(N // 64, 2, 32, K).transpose(0, 1).reshape(N, K)
+        assert torch.equal(kernels.w4_dequant_rows(p), w)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("paired", [False, True])
+def test_layers_of_many_rows_take_the_copy(paired, dtype):
+    """From dense_rows() on, within roundings of the exact product; below, without a copy, with a bias and where sums keep their order the int4 kernels."""
+    from scalellm_amd import kernels, layers
+    from scalellm_amd.decode import _rand_int4_linear
+    from scalellm_amd.model_parallel import ParallelArgs
+    K, N = 640, 448
+
+    def made(fmt, bias=False):
+        gen = torch.Generator(device=DEV).manual_seed(5)
+        lin = layers.ColumnParallelQLinear(K, N, bias, layers.QuantArgs(fmt, 4, 64), False, ParallelArgs(), dtype, DEV, act_mul="silu" if paired else None)
+        ck = _rand_int4_linear(gen, K, N, 64, fmt, dtype, DEV)
+        lin.load_state_dict({**ck, "bias": torch.ones(N, device=DEV, dtype=dtype)} if bias else ck)
+        return lin
+    lin, int4 = made("awq"), made("awq")
+    assert lin.lay_out_dense(2 * K * N - 1) == 0 and lin.lay_out_dense(2 * K * N) == 2 * K * N and lin.lay_out_dense(1 << 40) == 0
+    unit = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    for M in (lin.dense_rows() - 1, lin.dense_rows(), 1000):
+        x = torch.randn(M, K + 8, device=DEV, generator=torch.Generator(device=DEV).manual_seed(M)).to(dtype)[:, :K].div_(8)
+        got = lin.forward(x)
+        assert not lin.deferred
+        if M < lin.dense_rows():
+            assert torch.equal(got, int4.forward(x))
+            continue
+        want = x.double() @ lin._dense.double().t()
+        if paired:
+            want = torch.nn.functional.silu(want[:, :N // 2]) * want[:, N // 2:]
+        # (one rounding of fp32 sums of K exact products, and of the GLU's few operations)
+        assert (got.double() - want).abs().max() <= 1.02 * unit * want.abs().max()
+    with pytest.raises(kernels.SlmError):
+        lin.forward(x, out=torch.empty(M, N + 8, device=DEV, dtype=dtype))
+    lin.load_state_dict({})
+    assert lin._dense is None
+    for other in (made("gptq"), made("awq", bias=True)):
+        want = other.forward(x)
+        assert (other.lay_out_dense(1 << 40) > 0) == other.has_bias and torch.equal(other.forward(x), want)
