@@ -37,6 +37,9 @@ namespace slm {
 #endif
 constexpr bool PV_DOT2 = SLM_ATTN_PV_DOT2 != 0;
 
+using CInt = const int __attribute__((address_space(4)));
+__device__ __forceinline__ CInt* as_const(const int* p) { return (CInt*)(uintptr_t)p; }
+
 template <bool NT>
 __device__ __forceinline__ u32x4 ld16(const void* p) {
   if constexpr (NT)
@@ -79,24 +82,35 @@ __global__ void __launch_bounds__(512) attn_token_kernel(const AttnKParams p) {
   const int hgb = bid % p.nhgb;
   const int tok = bid / p.nhgb;
 
-  // token -> sequence: q_cu[b] <= tok < q_cu[b+1].  Pure decode batches (one query token per
-  // sequence: q_cu[i] == i) are recognised with two independent loads instead of log2(batch)
-  // dependent ones -- the binary search is ~0.4 us per step of start-up latency in front of every
-  // workgroup's stream, which is what small batches are made of.
+  // token -> sequence: q_cu[b] <= tok < q_cu[b+1].  What a batch of one query token per sequence (q_cu[i] == i) needs is read
+  // at once, before any of it is looked at, and kept if the guess holds: one round trip in front of the block table's where
+  // the lengths, the row class and the table's place were four one after another (1 sequence of 4 k keys, 32 / 8 heads: 13.4
+  // -> 13.0 us, 32 of 2 .. 4 k with a binary search less: 70.1 -> 68.6).  The arrays are read through scalar loads, which
+  // this kernel's own stores would forbid the compiler.
+  const int tc = min(tok, p.batch), tn = min(tok + 1, p.batch);
+  CInt *q_cu = as_const(p.q_cu), *kv_cu = as_const(p.kv_cu), *bcu = as_const(p.bcu);
+  int q0 = q_cu[tc], q1 = q_cu[tn], kv0 = kv_cu[tc], kv1 = kv_cu[tn], bcu0 = bcu[tc];
+  int q_end = q_cu[p.batch], Wtot = kv_cu[p.batch];
+  int ends[4];  // the histories' ends, for the balanced partition's search
+  if (p.bal) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) ends[c] = p.kv_cu[min(lane + 64 * c + 1, p.batch)];
+  }
+  asm("" : "+s"(q_end), "+s"(Wtot));  // (not to be moved down to their use)
   int b;
-  const int tq0 = p.q_cu[min(tok, p.batch)], tq1 = p.q_cu[min(tok + 1, p.batch)];
-  if (tok < p.batch && tq0 == tok && tq1 == tok + 1) {
+  if (tok < p.batch && q0 == tok && q1 == tok + 1) {
     b = tok;
   } else {
     int lo_b = 0, hi_b = p.batch;
     while (lo_b < hi_b) {
       const int mid = (lo_b + hi_b) >> 1;
-      if (p.q_cu[mid + 1] <= tok)
+      if (q_cu[mid + 1] <= tok)
         lo_b = mid + 1;
       else
         hi_b = mid;
     }
     b = lo_b;
+    if (b < p.batch) q0 = q_cu[b], q1 = q_cu[b + 1], kv0 = kv_cu[b], kv1 = kv_cu[b + 1], bcu0 = bcu[b];
   }
   // Balanced pure-decode partition (p.bal; plan_attn): this workgroup is number w of its head
   // group and owns the tokens [g, g1) of the concatenated histories; it walks the sequences that
@@ -107,25 +121,33 @@ __global__ void __launch_bounds__(512) attn_token_kernel(const AttnKParams p) {
   // means q_cu[i] == i.  A batch that keeps q = 0 sequences next to graph-padding rows
   // (slm_build_step_inputs allows it) fails the check and runs the classic partition, which follows
   // q_cu (same grid; part_slots > n_splits, so the partial slots are there).
-  const bool bal = p.bal && p.q_cu[p.batch] == p.batch;
+  const bool bal = p.bal && q_end == p.batch;
   int bal_g = 0, bal_g1 = 0, bal_Q = 1;  // (all < 2^31: kv_cu is int32)
   if (bal) {
-    const int Wtot = p.kv_cu[p.batch];
     bal_Q = attn_bal_q(p, Wtot);
     const int64_t g64 = (int64_t)(tok * p.n_splits + split) * bal_Q;
     if (g64 >= (int64_t)Wtot) return;
     bal_g = (int)g64;
     bal_g1 = Wtot - bal_g > bal_Q ? bal_g + bal_Q : Wtot;
-    int lo_b = 0, hi_b = p.batch;  // sequence holding token g: kv_cu[b] <= g < kv_cu[b + 1]
-    while (lo_b < hi_b) {
+    // sequence holding token g: kv_cu[b] <= g < kv_cu[b + 1] (256 ends at once, most batches without a further read)
+    int lo_b = 0, hi_b = p.batch;
+    while (hi_b - lo_b > 256) {
       const int mid = (lo_b + hi_b) >> 1;
-      if (p.kv_cu[mid + 1] <= bal_g) lo_b = mid + 1; else hi_b = mid;
+      if (kv_cu[mid + 1] <= bal_g) lo_b = mid + 1; else hi_b = mid;
     }
-    b = lo_b;
+    if (p.batch > 256) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) ends[c] = p.kv_cu[min(lo_b + lane + 64 * c + 1, p.batch)];
+    }
+    int below = 0;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) below += __popcll(__ballot(lo_b + lane + 64 * c < hi_b && ends[c] <= bal_g));
+    b = lo_b + below;
+    if (b < p.batch) kv0 = kv_cu[b], kv1 = kv_cu[b + 1], bcu0 = bcu[b];
   }
   if (b >= p.batch) return;  // padding token past q_cu[batch]
   if (!bal) {
-    const int rows = (p.q_cu[b + 1] - p.q_cu[b]) * p.group;
+    const int rows = (q1 - q0) * p.group;
     if (rows < p.rows_lo || rows >= p.rows_hi) return;  // another launch owns this sequence
   }
 
@@ -161,7 +183,6 @@ __global__ void __launch_bounds__(512) attn_token_kernel(const AttnKParams p) {
   bool single = p.n_splits == 1;  // the pass covers its sequence alone: it writes the final output
   bool skip = false;
   if (bal) {
-    const int kv0 = p.kv_cu[b], kv1 = p.kv_cu[b + 1];
     tok_p = b;  // pure decode: token index == sequence index
     s_lo = bal_g - kv0;
     s_hi = min(kv1, bal_g1) - kv0;
@@ -183,10 +204,9 @@ __global__ void __launch_bounds__(512) attn_token_kernel(const AttnKParams p) {
       }
     }
   } else {
-    const int q_start = p.q_cu[b];
-    const int q_len = p.q_cu[b + 1] - q_start;
-    const int kv_len = p.kv_cu[b + 1] - p.kv_cu[b];
-    const int diag = kv_len - q_len + (tok - q_start);  // last visible kv index (causal)
+    const int q_len = q1 - q0;
+    const int kv_len = kv1 - kv0;
+    const int diag = kv_len - q_len + (tok - q0);  // last visible kv index (causal)
     const int hi = min(diag + 1, kv_len);
     const int lo = (p.window >= 0) ? max(0, diag - p.window) : 0;
     // split range, aligned to RPI rows
@@ -222,8 +242,6 @@ __global__ void __launch_bounds__(512) attn_token_kernel(const AttnKParams p) {
 #pragma unroll
     for (int j = 0; j < OD; ++j) o[h][j] = 0.f;
   }
-
-  const int bcu0 = p.bcu[b];
 
   u32x4 kr[U][W], vr[U][W];
 
@@ -519,10 +537,11 @@ __global__ void __launch_bounds__(512) attn_token_kernel(const AttnKParams p) {
   if (!bal) break;
   // next piece: the following non-empty sequence, if this workgroup's range reaches into it
   do {
-    ++b;
-  } while (b < p.batch && p.kv_cu[b + 1] == p.kv_cu[b]);
+    if (++b >= p.batch) break;
+    kv0 = kv_cu[b], kv1 = kv_cu[b + 1], bcu0 = bcu[b];
+  } while (kv1 == kv0);
   if (b >= p.batch) break;
-  bal_g = p.kv_cu[b];
+  bal_g = kv0;
   if (bal_g >= bal_g1) break;
   }  // piece loop
 }
