@@ -42,6 +42,8 @@ typedef struct slm_residual_norm_args {
   float eps, norm_alpha;
   float delta_mult;         /* factor of what is added: the delta, or the embedding row                 */
   int32_t n_slabs, mode, dtype, norm, row_shift;
+  int32_t n_clear;          /* words of clear, at most 65536                                            */
+  uint32_t* clear;          /* EMBED: NULL, or words that are set to zero (rows > 0)                    */
 } slm_residual_norm_args;
 enum { SLM_NORM_RMS = 0, SLM_NORM_TANH = 1 };
 enum { SLM_RN_EMBED = 0, SLM_RN_ADD = 1, SLM_RN_SLABS = 2, SLM_RN_PLAIN = 3 };
@@ -69,6 +71,12 @@ SLM_API int slm_linear(const slm_linear_args* a, void* stream);
 SLM_API int slm_linear_stream(const slm_linear_args* a, void* stream);
 /* The same in half precision (dtype SLM_F16), STORE                                                     */
 SLM_API int slm_linear_stream_half(const slm_linear_args* a, void* stream);
+/* A stored product cut in K by n_splits, joined in the launch: STORE, bf16, 17 to 128 rows, N <= 32 *     */
+/* SLM_STREAM_TICKETS, n_splits <= 16.  workspace: content does not matter; tickets [SLM_STREAM_TICKETS]    */
+/* are zero before and after (products of one stream may share them: slm_residual_norm_args::clear)         */
+#define SLM_STREAM_TICKETS 512
+SLM_API size_t slm_linear_stream_join_bytes(const slm_linear_args* a);
+SLM_API int slm_linear_stream_join(const slm_linear_args* a, void* workspace, size_t workspace_bytes, uint32_t* tickets, void* stream);
 /* lays contiguous w [N, K] of 16 bits out so: out holds ceil(N / 64) * 64 * K elements                   */
 SLM_API int slm_stream_layout(void* out, const void* w, int64_t N, int64_t K, int32_t glu, void* stream);
 /* The same for many rows in bf16, batch 1, STORE or GLU, rows of x, w and y on 16 bytes, x and w below 2 GB: tiles of  */

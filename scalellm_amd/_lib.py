@@ -229,11 +229,12 @@ class ResidualNormArgs(C.Structure):
     """slm_residual_norm_args."""
     _fields_ = _fields((C.c_void_p, "resid delta slabs tokens positions embed pos_table row_index weight bias out"),
                        (C.c_int64, "rows width ld_delta ld_embed ld_out slab_stride"),
-                       (C.c_float, "eps norm_alpha delta_mult"), (C.c_int32, "n_slabs mode dtype norm row_shift"))
+                       (C.c_float, "eps norm_alpha delta_mult"), (C.c_int32, "n_slabs mode dtype norm row_shift n_clear"), (C.c_void_p, "clear"))
 
 
 NORM_RMS, NORM_TANH = range(2)
 RN_EMBED, RN_ADD, RN_SLABS, RN_PLAIN = range(4)
+STREAM_TICKETS = 512
 
 
 class LinearArgs(C.Structure):
@@ -291,6 +292,8 @@ def latent_lib() -> C.CDLL:
         ("slm_linear", C.c_int, [P(LinearArgs), ptr]),
         ("slm_linear_stream", C.c_int, [P(LinearArgs), ptr]),
         ("slm_linear_stream_half", C.c_int, [P(LinearArgs), ptr]),
+        ("slm_linear_stream_join_bytes", C.c_size_t, [P(LinearArgs)]),
+        ("slm_linear_stream_join", C.c_int, [P(LinearArgs), ptr, C.c_size_t, ptr, ptr]),
         ("slm_gemm_workspace_bytes", C.c_size_t, [P(LinearArgs), i32, i32]),
         ("slm_gemm", C.c_int, [P(LinearArgs), ptr, C.c_size_t, i32, i32, ptr]),
         ("slm_gemm_half", C.c_int, [P(LinearArgs), ptr, C.c_size_t, i32, i32, ptr]),

@@ -78,9 +78,51 @@ __device__ __forceinline__ void stream_store(const slm_linear_args& a, int split
 template <int EPI>
 __device__ __forceinline__ int64_t stream_column(int64_t nb) { return EPI == SLM_LIN_GLU ? (nb >> 1) * 16 : nb * 16; }
 
-template <typename E, int MT, int NT, int D, int EPI>
-__global__ void __launch_bounds__(256) linear_wave_k_kernel(const slm_linear_args a) {
+// Products that are cut in K and stored in one launch.  A workgroup's fp32 sums go past the caches to its tile's slabs, the last of the tile's splits to
+// arrive adds all of them up in their order -- the same bits whoever is last -- and stores.  It leaves the counter at zero, as it was found.
+// For stored products whose columns leave CUs idle: bound by what a CU has under way, a product of 106 workgroups takes as long on 106 CUs as one of
+// twice the columns on 212.  Joining costs 2 to 4 us, two thirds of it the sums' way out and back (us, whole / cut in 2: 6752 x 4096 64 rows 22.2 / 17.7,
+// 128 rows 28.2 / 22.8; 6464 x 2048 12.3 / 10.7, 16.0 / 13.9).  A step of four layers, 128 rows: 1074 / 1052 us (8b, latent), 887 / 876 (2b, recurrent).
+struct StreamJoin {
+  float* slabs;          // [tiles][splits][fragments][256] f32x4
+  uint32_t* arrived;     // [tiles], zero
+};
+// F fragments of thread t (of 256; others only take part in the barriers).  word: 4 bytes of LDS that nobody reads past the first barrier
+template <int F>
+__device__ __forceinline__ bool stream_join(f32x4 (&acc)[F], const StreamJoin& j, int split, int splits, int t, uint32_t* word) {
+  const __amdgpu_buffer_rsrc_t slabs =
+      __builtin_amdgcn_make_buffer_rsrc(j.slabs + (int64_t)blockIdx.x * splits * (F * 1024), 0, splits * F * 4096, 0x00020000);
+  auto at = [&](int s, int f) { return ((s * F + f) * 256 + t) * 16; };
+  if (t < 256) {
+#pragma unroll
+    for (int f = 0; f < F; ++f) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[f]), slabs, at(split, f), 0, /*sc1*/ 16);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // every wave's sums are out ..
+  __syncthreads();
+  if (threadIdx.x == 0) *word = __hip_atomic_fetch_add(j.arrived + blockIdx.x, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // .. then one announces them
+  __syncthreads();
+  if (*word != (uint32_t)splits - 1) return false;
+  if (threadIdx.x == 0) __hip_atomic_store(j.arrived + blockIdx.x, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (t >= 256) return true;
+  if (splits == 2) {   // (its own are at hand; the other order has the same sum)
+#pragma unroll
+    for (int f = 0; f < F; ++f) acc[f] += __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(slabs, at(1 - split, f), 0, /*sc1*/ 16));
+    return true;
+  }
+#pragma unroll
+  for (int f = 0; f < F; ++f) acc[f] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int s = 0; s < splits; ++s) {
+#pragma unroll
+    for (int f = 0; f < F; ++f) acc[f] += __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(slabs, at(s, f), 0, /*sc1*/ 16));
+  }
+  return true;
+}
+
+// JOIN: by stream_join, one row of tiles
+template <typename E, int MT, int NT, int D, int EPI, bool JOIN>
+__global__ void __launch_bounds__(256) linear_wave_k_kernel(const slm_linear_args a, const StreamJoin j) {
   constexpr bool GLU = EPI == SLM_LIN_GLU;
+  static_assert(!JOIN || (EPI == SLM_LIN_STORE && NT * MT == 4), "a tile a wave");
   static_assert(!GLU || NT % 2 == 0, "gate / up pairs");
   __shared__ f32x4 red[4][NT * MT][64];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -158,19 +200,27 @@ __global__ void __launch_bounds__(256) linear_wave_k_kernel(const slm_linear_arg
   __syncthreads();
   // a tile per wave: lane = (columns 4 g .. + 3, row r16), the layout of the products
   constexpr int TILES = (GLU ? NT / 2 : NT) * MT;
+  auto total = [&](int tile) { return red[0][tile][lane] + red[1][tile][lane] + red[2][tile][lane] + red[3][tile][lane]; };
+  if constexpr (JOIN) {
+    f32x4 y[1] = {total(wave)};
+    if (!stream_join(y, j, split, a.n_splits, tid, reinterpret_cast<uint32_t*>(red))) return;
+    const int64_t nb = nb0 + wave / MT, m = m0 + 16 * (wave % MT) + r16;
+    if (nb < blocks && m < a.M) stream_store<E, EPI>(a, 0, m, nb * 16 + 4 * g, y[0], y[0]);
+    return;
+  }
   for (int i = wave; i < TILES; i += 4) {
     const int t = i / MT * (GLU ? 2 : 1), v = i % MT;
     const int64_t nb = nb0 + t, m = m0 + 16 * v + r16;
     if (nb >= blocks || m >= a.M) continue;
-    auto total = [&](int tile) { return red[0][tile][lane] + red[1][tile][lane] + red[2][tile][lane] + red[3][tile][lane]; };
     const f32x4 y = total(t * MT + v);
     stream_store<E, EPI>(a, split, m, stream_column<EPI>(nb) + 4 * g, y, GLU ? total((t + 1) * MT + v) : y);
   }
 }
 
-template <typename E, int MT, int NT, int WK, int D, int EPI>
-__global__ void __launch_bounds__(256 * WK) linear_wave_n_kernel(const slm_linear_args a) {
+template <typename E, int MT, int NT, int WK, int D, int EPI, bool JOIN>
+__global__ void __launch_bounds__(256 * WK) linear_wave_n_kernel(const slm_linear_args a, const StreamJoin j) {
   constexpr bool GLU = EPI == SLM_LIN_GLU;
+  static_assert(!JOIN || EPI == SLM_LIN_STORE, "joined products are stored");
   constexpr int GROUP = MT * 16 * 128;    // bytes of a group's step of x in LDS: 16-byte chunk c of row r lies in slot c ^ (r & 7)
   constexpr int AHEAD = MT < 3 ? 1 : NT == 1 ? 3 : 2;
   constexpr int XU = MT * 16 * 8 / 256;   // 16-byte units a thread stages
@@ -313,6 +363,10 @@ __global__ void __launch_bounds__(256 * WK) linear_wave_n_kernel(const slm_linea
     __syncthreads();
     if (wn & 1) return;
   }
+  if constexpr (JOIN) {
+    f32x4 (&flat)[NT * MT] = reinterpret_cast<f32x4 (&)[NT * MT]>(acc);
+    if (!stream_join(flat, j, split, a.n_splits, tid, reinterpret_cast<uint32_t*>(lds))) return;
+  }
   if (kg > 0) return;
 #pragma unroll
   for (int t = 0; t < NT; t += (GLU && NT > 1 ? 2 : 1)) {
@@ -332,16 +386,29 @@ __global__ void __launch_bounds__(256 * WK) linear_wave_n_kernel(const slm_linea
 // column tiles of 16 per NT; the grid's x extent
 static int64_t stream_tiles(const slm_linear_args& a, int per) { return (a.N / 16 + per - 1) / per; }
 
+// (one row of tiles: M <= 128, joined products)
 template <typename E, int MT, int NT, int D, int EPI>
-static int wave_k_launch(const slm_linear_args& a, hipStream_t st) {
-  const int64_t gy = (a.M + 16 * MT - 1) / (16 * MT);
-  linear_wave_k_kernel<E, MT, NT, D, EPI><<<dim3((unsigned)stream_tiles(a, NT), (unsigned)gy, (unsigned)a.n_splits), dim3(256), 0, st>>>(a);
+static int wave_k_launch(const slm_linear_args& a, hipStream_t st, const StreamJoin* j) {
+  const dim3 grid((unsigned)stream_tiles(a, NT), (unsigned)((a.M + 16 * MT - 1) / (16 * MT)), (unsigned)a.n_splits);
+  if constexpr (std::is_same<E, bf16>::value && EPI == SLM_LIN_STORE && MT == 2) {
+    if (j) {
+      linear_wave_k_kernel<E, MT, NT, D, EPI, true><<<grid, dim3(256), 0, st>>>(a, *j);
+      return hip_check_launch();
+    }
+  }
+  linear_wave_k_kernel<E, MT, NT, D, EPI, false><<<grid, dim3(256), 0, st>>>(a, StreamJoin{});
   return hip_check_launch();
 }
 template <typename E, int MT, int NT, int WK, int D, int EPI>
-static int wave_n_launch(const slm_linear_args& a, hipStream_t st) {
-  const int64_t gy = (a.M + 16 * MT - 1) / (16 * MT);
-  linear_wave_n_kernel<E, MT, NT, WK, D, EPI><<<dim3((unsigned)stream_tiles(a, 4 * NT), (unsigned)gy, (unsigned)a.n_splits), dim3(256 * WK), 0, st>>>(a);
+static int wave_n_launch(const slm_linear_args& a, hipStream_t st, const StreamJoin* j) {
+  const dim3 grid((unsigned)stream_tiles(a, 4 * NT), (unsigned)((a.M + 16 * MT - 1) / (16 * MT)), (unsigned)a.n_splits);
+  if constexpr (std::is_same<E, bf16>::value && EPI == SLM_LIN_STORE) {
+    if (j) {
+      linear_wave_n_kernel<E, MT, NT, WK, D, EPI, true><<<grid, dim3(256 * WK), 0, st>>>(a, *j);
+      return hip_check_launch();
+    }
+  }
+  linear_wave_n_kernel<E, MT, NT, WK, D, EPI, false><<<grid, dim3(256 * WK), 0, st>>>(a, StreamJoin{});
   return hip_check_launch();
 }
 
@@ -351,7 +418,7 @@ static int wave_n_launch(const slm_linear_args& a, hipStream_t st) {
 // 64 rows x 28672 x 4096 41 us against 48, 64 rows x 16384 x 2048 20.6 against 15.7.  Up to 32 rows and under 112 panels the chip is
 // filled by 32-column tiles (6784 columns: 15.6 us against 18.4).
 template <typename E, int EPI>
-static int stream_shape(const slm_linear_args& a, hipStream_t st) {
+static int stream_shape(const slm_linear_args& a, hipStream_t st, const StreamJoin* j = nullptr) {
   constexpr bool GLU = EPI == SLM_LIN_GLU;
   const int64_t s = a.n_splits;
   auto full = [&](int nt) {
@@ -359,21 +426,21 @@ static int stream_shape(const slm_linear_args& a, hipStream_t st) {
     return 4 * w >= 3 * 256 * ((w + 255) / 256);
   };
   if (a.M <= 16) {
-    if (full(4)) return wave_k_launch<E, 1, 4, 3, EPI>(a, st);
+    if (full(4)) return wave_k_launch<E, 1, 4, 3, EPI>(a, st, j);
     if constexpr (!GLU) {
-      if (!full(2)) return wave_k_launch<E, 1, 1, 8, EPI>(a, st);
+      if (!full(2)) return wave_k_launch<E, 1, 1, 8, EPI>(a, st, j);
     }
-    return wave_k_launch<E, 1, 2, 4, EPI>(a, st);
+    return wave_k_launch<E, 1, 2, 4, EPI>(a, st, j);
   }
   const int64_t rounds1 = (stream_tiles(a, 4) * s + 255) / 256, rounds2 = (stream_tiles(a, 8) * s + 255) / 256;
   const bool wide = 2 * rounds2 <= rounds1;
   if (a.M <= 32) {
-    if (stream_tiles(a, 4) * s < 112) return wave_k_launch<E, 2, 2, 4, EPI>(a, st);
-    return wide ? wave_n_launch<E, 2, 2, 1, 4, EPI>(a, st) : wave_n_launch<E, 2, 1, 2, 4, EPI>(a, st);
+    if (stream_tiles(a, 4) * s < 112) return wave_k_launch<E, 2, 2, 4, EPI>(a, st, j);
+    return wide ? wave_n_launch<E, 2, 2, 1, 4, EPI>(a, st, j) : wave_n_launch<E, 2, 1, 2, 4, EPI>(a, st, j);
   }
-  if (a.M <= 64) return wide ? wave_n_launch<E, 4, 2, 1, 4, EPI>(a, st) : wave_n_launch<E, 4, 1, 1, 4, EPI>(a, st);
-  if (a.M <= 96) return wide ? wave_n_launch<E, 6, 2, 1, 4, EPI>(a, st) : wave_n_launch<E, 6, 1, 1, 4, EPI>(a, st);
-  return wide ? wave_n_launch<E, 8, 2, 2, 2, EPI>(a, st) : wave_n_launch<E, 8, 1, 1, 4, EPI>(a, st);
+  if (a.M <= 64) return wide ? wave_n_launch<E, 4, 2, 1, 4, EPI>(a, st, j) : wave_n_launch<E, 4, 1, 1, 4, EPI>(a, st, j);
+  if (a.M <= 96) return wide ? wave_n_launch<E, 6, 2, 1, 4, EPI>(a, st, j) : wave_n_launch<E, 6, 1, 1, 4, EPI>(a, st, j);
+  return wide ? wave_n_launch<E, 8, 2, 2, 2, EPI>(a, st, j) : wave_n_launch<E, 8, 1, 1, 4, EPI>(a, st, j);
 }
 
 // A thread moves 16 bytes; a wave writes 1 KB and reads 16 half lines whose other halves the next wave reads (once per
@@ -401,12 +468,12 @@ extern "C" SLM_API int slm_stream_layout(void* out, const void* w, int64_t N, in
   return hip_check_launch();
 }
 
-static int stream_check(const slm_linear_args* a, int dtype) {
+static int stream_check(const slm_linear_args* a, int dtype, bool join = false) {
   if (!a || !a->x || !a->w || !a->y || a->M < 0 || a->N <= 0 || a->K <= 0 || a->K % 64 || a->N % 16 || a->batch != 1 ||
       a->n_splits < 1 || a->ldx < a->K || a->epilogue < 0 || a->epilogue > SLM_LIN_GLU)
     return SLM_ERR_INVALID_ARG;
   const bool glu = a->epilogue == SLM_LIN_GLU;
-  if ((glu && a->N % 64) || (a->n_splits > 1 && a->epilogue != SLM_LIN_SLABS)) return SLM_ERR_INVALID_ARG;
+  if ((glu && a->N % 64) || (a->n_splits > 1 && a->epilogue != SLM_LIN_SLABS && !join)) return SLM_ERR_INVALID_ARG;
   if (a->ldy < (glu ? a->N / 2 : a->N)) return SLM_ERR_INVALID_ARG;
   if (a->dtype != dtype || a->K > (1 << 28) || a->N > (1 << 30) || a->M > (1 << 20) || a->n_splits > 65535) return SLM_ERR_UNSUPPORTED;
   return a->ldx % 8 || !aligned16(a->x) || !aligned16(a->w) ? SLM_ERR_ALIGNMENT : SLM_OK;
@@ -430,4 +497,24 @@ extern "C" SLM_API int slm_linear_stream_half(const slm_linear_args* a, void* st
   if (a->M == 0) return SLM_OK;
   hip_clear_error();
   return stream_shape<_Float16, SLM_LIN_STORE>(*a, (hipStream_t)stream);
+}
+
+// Joined products: STORE, 17 to 128 rows, at most SLM_STREAM_TICKETS tiles of 32 columns
+static bool stream_join_ok(const slm_linear_args* a) {
+  return a->epilogue == SLM_LIN_STORE && a->M > 16 && a->M <= 128 && a->n_splits <= 16 && stream_tiles(*a, 2) <= SLM_STREAM_TICKETS;
+}
+extern "C" SLM_API size_t slm_linear_stream_join_bytes(const slm_linear_args* a) {
+  if (stream_check(a, SLM_BF16, true) != SLM_OK || !stream_join_ok(a)) return 0;
+  const int64_t rows = a->M <= 32 ? 32 : a->M <= 64 ? 64 : a->M <= 96 ? 96 : 128;
+  return (size_t)(a->n_splits * rows * stream_tiles(*a, 8) * 128 * 4);   // (whole tiles of up to 128 columns)
+}
+extern "C" SLM_API int slm_linear_stream_join(const slm_linear_args* a, void* workspace, size_t workspace_bytes, uint32_t* tickets, void* stream) {
+  const int rc = stream_check(a, SLM_BF16, true);
+  if (rc != SLM_OK) return rc;
+  if (!stream_join_ok(a)) return SLM_ERR_UNSUPPORTED;
+  if (!tickets || !workspace || workspace_bytes < slm_linear_stream_join_bytes(a)) return SLM_ERR_WORKSPACE;
+  if (!aligned16(workspace)) return SLM_ERR_ALIGNMENT;
+  const StreamJoin j{(float*)workspace, tickets};
+  hip_clear_error();
+  return stream_shape<bf16, SLM_LIN_STORE>(*a, (hipStream_t)stream, &j);
 }

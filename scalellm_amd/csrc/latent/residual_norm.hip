@@ -33,6 +33,9 @@ __global__ void __launch_bounds__(T) residual_norm_kernel(const slm_residual_nor
   const int tid = threadIdx.x;
   const int64_t row = blockIdx.x;
   const int width = (int)a.width;
+  if (MODE == SLM_RN_EMBED && row == 0) {   // (somebody's counters: a launch less)
+    for (int i = tid; i < a.n_clear; i += T) a.clear[i] = 0;
+  }
   const int64_t src_row = (MODE == SLM_RN_PLAIN && a.row_index) ? a.row_index[row] + a.row_shift : row;
   float* r = a.resid + src_row * a.width;
   const E* e0 = nullptr;
@@ -220,6 +223,7 @@ extern "C" SLM_API int slm_residual_norm(const slm_residual_norm_args* a, void* 
   if (a->mode == SLM_RN_SLABS && (!a->slabs || a->n_slabs < 1 || a->ld_delta < a->width)) return SLM_ERR_INVALID_ARG;
   if (a->weight ? (!a->out || a->ld_out < a->width) : a->mode == SLM_RN_PLAIN) return SLM_ERR_INVALID_ARG;
   if (a->norm < 0 || a->norm > SLM_NORM_TANH || (a->weight && a->norm == SLM_NORM_TANH && !a->bias)) return SLM_ERR_INVALID_ARG;
+  if (a->n_clear < 0 || a->n_clear > 65536 || (a->n_clear && (!a->clear || a->mode != SLM_RN_EMBED))) return SLM_ERR_INVALID_ARG;
   if (a->dtype == SLM_BF16) return rn_mode<bf16>(*a, (hipStream_t)stream);
   if (a->dtype == SLM_F32) return rn_mode<float>(*a, (hipStream_t)stream);
   return SLM_ERR_UNSUPPORTED;

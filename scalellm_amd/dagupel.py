@@ -162,14 +162,15 @@ class DagupelStep:
         c, T = self.config, tokens.numel()
         resid = torch.empty(T, c.width, dtype=torch.float32, device=self.device)
         h = torch.empty(T, self.k_width, dtype=self.dtype, device=self.device)
+        tickets = lk.step_tickets(T, self.device)
         first = self.layers[0].norm1 if self.layers else None
-        lk.residual_norm(resid, h, first, c.eps, embed=(tokens, self.table, positions, self.pos_table))
+        lk.residual_norm(resid, h, first, c.eps, embed=(tokens, self.table, positions, self.pos_table), clear=tickets)
         n = len(self.layers)
         # (None: the last sum's launch norms them too -- not where somebody sees, and may change, the stream behind it)
         rows = lk.wanted_rows(params, T if n and self.on_layer is None else 0)
         for i, L in enumerate(self.layers):
             nxt = self.layers[i + 1].norm1 if i + 1 < n else self.final_norm if rows is None else None
-            delta = L.attn.forward(h, positions, self.caches[i], params)
+            delta = L.attn.forward(h, positions, self.caches[i], params, tickets)
             if L.mlp is not None:
                 lk.residual_norm(resid, h, L.norm2, c.eps, delta=delta)
                 delta = L.mlp.forward(h)

@@ -71,11 +71,11 @@ class Slabs:
 
 def residual_norm(resid: torch.Tensor, out: Optional[torch.Tensor], weight, eps: float,
                   delta=None, embed=None, row_index: Optional[torch.Tensor] = None, mult: float = 1.0,
-                  row_shift: int = 0) -> None:
+                  row_shift: int = 0, clear: Optional[torch.Tensor] = None) -> None:
     """resid (fp32 [rows, width]) += mult * delta (a [rows, >= width] tensor or Slabs), or
     resid = mult * (table[tokens] (+ pos[positions])) for embed = (tokens, table, positions, pos); then
     out = rms_norm(resid) * weight, or a TanhNorm given as weight, zero padded to out's width.  weight = None: the sum only.
-    row_index: out row r is the norm of stream row row_index[r] + row_shift; nothing is added."""
+    row_index: out row r is the norm of stream row row_index[r] + row_shift; nothing is added.  clear (int32, with embed): set to zero."""
     a = _lib.ResidualNormArgs()
     rows, width = resid.shape
     _need(resid.dtype == torch.float32 and resid.is_contiguous(), "residual_norm: resid is contiguous fp32")
@@ -108,6 +108,9 @@ def residual_norm(resid: torch.Tensor, out: Optional[torch.Tensor], weight, eps:
             _i32(row_index, rows, "row_index")
             a.row_index, a.row_shift = _p(row_index), row_shift
     a.rows = rows
+    if clear is not None:
+        _need(embed is not None and clear.dtype == torch.int32 and clear.is_contiguous() and clear.device == resid.device, "residual_norm: clear")
+        a.clear, a.n_clear = _p(clear), clear.numel()
     if isinstance(weight, TanhNorm):
         t, weight = weight, weight.weight
         _need(t.bias.dtype == torch.float32 and t.bias.numel() == width and t.bias.is_contiguous(), "norm bias: fp32 [width]")
@@ -240,6 +243,42 @@ def _store_rows(N: int, K: int) -> int:
     return 64 if N >= 8192 and K <= 2048 + 5 * (N - 8192) // 2 else STREAM_MAX_ROWS
 
 
+def step_tickets(rows: int, device) -> Optional[torch.Tensor]:
+    """What linear()'s products cut in K count their arrivals by in a step of so many rows (None: not cut): cleared by the residual_norm() of the
+    embedding that they follow, left at zero by each of them, of one step alone."""
+    return torch.empty(_lib.STREAM_TICKETS, dtype=torch.int32, device=device) if 16 < rows <= STREAM_LAYOUT_MAX_ROWS else None
+
+
+def join_count(N: int, K: int, rows: int) -> int:
+    """Slices of K of a product that is only stored and cut in one launch; 1: not cut.  As many as give every CU a workgroup of 64 columns, ten steps
+    of 64 each at least: joining them costs 2 to 4 us.  us, vendor / whole / cut, 64 and 128 rows: 6752 x 4096 in 2 18.9 / 22.6 / 17.7, 26.4 / 28.2 / 22.8;
+    6464 x 2048 in 2 13.2 / 12.3 / 10.7, 15.4 / 16.0 / 13.9; 3664 x 2048 in 3 12.1 / 11.7 / 9.1, 14.7 / 15.4 / 11.8; 4096 x 4096 in 4 15.1 / 21.4 / 12.0, 24.4 /
+    27.5 / 15.0; 2048 x 8192 in 8 22.3 / 37.7 / 13.2, 21.2 / 49.0 / 16.4; 8192 x 8192 in 2 35.0 / 44.4 / 30.0, 49.6 / 53.1 / 38.8; 512 x 4096 in 6 14.1 / 19.5 /
+    8.6, 14.4 / 25.9 / 11.3; short ones are whole (6464 x 1024 11.9 / 7.6 / 7.9, 12.6 / 9.9 / 10.4).  Between half and five eighths of the CUs long ones are
+    cut in three for workgroups of 128 columns (9216 x 4096 25.7 / 22.9 / 19.9, 30.3 / 28.9 / 26.5), wider ones are whole (12608 x 4096 25.7 / 24.5 / 26.1).  Up to
+    32 rows only long products gain (6752 x 4096 15.9 / 15.3 / 13.7, 3664 x 2048 11.7 / 8.2 / 8.1)."""
+    if not 16 < rows <= STREAM_LAYOUT_MAX_ROWS or N > 32 * _lib.STREAM_TICKETS or (rows <= STREAM_MAX_ROWS and K < 4096):
+        return 1
+    panels = (N + 63) // 64
+    if 128 < panels <= 160 and K >= 4096:
+        return 3
+    return max(1, min(8, 256 // panels, K // 640))
+
+
+def _joined(a, n: int, tickets: torch.Tensor, device) -> bool:
+    """The stored product in n slices of K; False: no memory for them."""
+    L = _lib.latent_lib()
+    _need(tickets.dtype == torch.int32 and tickets.is_contiguous() and tickets.numel() >= _lib.STREAM_TICKETS and tickets.device == device, "linear: tickets")
+    a.n_splits = n
+    try:   # (the launch's own: products of other streams have theirs)
+        ws = torch.empty(L.slm_linear_stream_join_bytes(C.byref(a)), dtype=torch.uint8, device=device)
+    except torch.OutOfMemoryError:
+        a.n_splits = 1
+        return False
+    latent_check(L.slm_linear_stream_join(C.byref(a), ws.data_ptr(), ws.numel(), tickets.data_ptr(), _stream()), "slm_linear_stream_join")
+    return True
+
+
 def _tile_pays(M: int, N: int, K: int, glu: bool) -> bool:
     """Is a product that the tile kernel takes its own, or the vendor's?  us by the device, vendor / tiles, where they are the vendor's:
     129 - 160 rows of large weights, whose one row of tiles reads them slower (28672 x 4096 GLU 59 / 74, from 161 rows 67 / 65; of the largest up to 192
@@ -282,20 +321,24 @@ def _gemm(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, glu=None, tile: i
 gemm = _gemm   # (for other modules)
 
 
-def linear(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None, layout: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """x [M, K] W[N, K]^T -> [M, N] of the same dtype.  layout: stream_layout(w)."""
+def linear(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None, layout: Optional[torch.Tensor] = None,
+           tickets: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """x [M, K] W[N, K]^T -> [M, N] of the same dtype.  layout: stream_layout(w); tickets: step_tickets(), cleared."""
     M, N, K = _check_xw(x, w)
     if out is None:
         out = torch.empty(M, N, dtype=x.dtype, device=x.device)
     _need(out.shape == (M, N) and out.stride(1) == 1 and out.dtype == x.dtype, "linear: out [M, N]")
-    a = _stream_args(x, w, layout, M, N, K, _store_rows(N, K))
+    n = join_count(N, K, M) if tickets is not None else 1
+    # (with tickets what is not cut is short or wide, and streamed: us, vendor / whole, 96 and 128 rows: 12608 x 4096 30.5 / 27.7, 32.3 / 30.9; 16384 x 4096
+    # 38.2 / 31.1, 38.8 / 34.9; 10240 x 2048 16.8 / 14.9, 18.2 / 16.8)
+    a = _stream_args(x, w, layout, M, N, K, _store_rows(N, K) if tickets is None else STREAM_LAYOUT_MAX_ROWS)
     if a is not None:
         a.ldy, a.y, a.epilogue = out.stride(0), _p(out), _lib.LIN_STORE
-        _run_stream(a)
+        if n == 1 or not _joined(a, n, tickets, x.device):
+            _run_stream(a)
         return out
     if not streams_rows(x):
-        # (stored products of 65 to 128 rows are the vendor's, whose small tiles leave fewer CUs idle: 125 x 2048 x 4096 10.9 us against
-        # 26.9 streamed; of the widest up to 96 rows streaming would be 2 to 3 us shorter, 96 x 12288 x 2048 17.2 against 15.3)
+        # (of row-major weights stored products of up to 128 rows are the vendor's, whose small tiles leave fewer CUs idle)
         return out if M >= TILE_MIN_ROWS and _tile_pays(M, N, K, False) and _gemm(x, w, out) else torch.mm(x, w.t(), out=out)
     a = _linear_args(x, w, M, N, K)
     a.ldx, a.ldw, a.ldy, a.y, a.epilogue = x.stride(0), K, out.stride(0), _p(out), _lib.LIN_STORE

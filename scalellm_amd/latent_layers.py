@@ -197,10 +197,10 @@ class LatentAttention:
     def new_cache(self, n_blocks: int, block_size: int) -> LatentKVCache:
         return LatentKVCache(n_blocks, block_size, self.c_pad, self.r_pad, self.w_in.dtype, self.w_in.device)
 
-    def forward(self, h: torch.Tensor, positions: torch.Tensor, cache: LatentKVCache, params: InputParameters):
-        """h [rows, padded width] -> what the residual stream receives (a tensor or split-K slabs)."""
+    def forward(self, h: torch.Tensor, positions: torch.Tensor, cache: LatentKVCache, params: InputParameters, tickets: Optional[torch.Tensor] = None):
+        """h [rows, padded width] -> what the residual stream receives (a tensor or split-K slabs).  tickets: of the step (latent_kernels)."""
         a, T = self.args, h.size(0)
-        proj = lk.linear(h, self.w_in, layout=self.l_in)
+        proj = lk.linear(h, self.w_in, layout=self.l_in, tickets=tickets)
         portions = params.portions if self.portions_ok else ()
         n_tok = portions[0].row0 if portions else T
         q_abs = proj.new_empty(n_tok, a.heads, self.c_pad + self.r_pad)

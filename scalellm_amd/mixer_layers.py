@@ -218,8 +218,8 @@ class ParallelMixer:
     def new_cache(self, limits):
         return self.left.new_cache(limits), self.right.new_state(limits)
 
-    def forward(self, h: torch.Tensor, positions: torch.Tensor, cache, params: InputParameters):
-        proj = lk.linear(h, self.w_in, layout=self.l_in)
+    def forward(self, h: torch.Tensor, positions: torch.Tensor, cache, params: InputParameters, tickets: Optional[torch.Tensor] = None):
+        proj = lk.linear(h, self.w_in, layout=self.l_in, tickets=tickets)
         out = proj.new_empty(h.size(0), self.o_k)
         self.left.forward(proj[:, :self.split], positions, cache[0], params, out[:, :self.left.out_width])
         self.right.forward(proj[:, self.split:], positions, cache[1], params, out[:, self.left.out_width:])
@@ -278,10 +278,10 @@ class ChannelDelta:
         s = self.spec
         return RecurrentState(limits.n_states, s.heads, s.dim_pad, s.v_pad, self.device, s.taps, s.channels, self.dtype)
 
-    def forward(self, h: torch.Tensor, positions: torch.Tensor, state: RecurrentState, params: InputParameters):
+    def forward(self, h: torch.Tensor, positions: torch.Tensor, state: RecurrentState, params: InputParameters, tickets: Optional[torch.Tensor] = None):
         s, T = self.spec, h.size(0)
         n = single_rows(params, T)
-        proj = lk.linear(h, self.w_in, layout=self.l_in)
+        proj = lk.linear(h, self.w_in, layout=self.l_in, tickets=tickets)
         low_in = proj[:, self.off_a1:]
         low = proj.new_empty(T, 2 * self.low_n)
         # (one launch; 128 rows x 2048 columns 4.9 us against two vendor products of 5.6)

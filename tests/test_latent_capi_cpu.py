@@ -294,3 +294,28 @@ def test_tiled_products_scratch_is_bounded():
     a = _gemm_args(2300, 4128, 320)
     assert L.slm_gemm_workspace_bytes(C.byref(a), 2, 2) == 1024 + (18 * 33 % 256) * 2 * 128 * 128 * 4
     assert L.slm_gemm_workspace_bytes(C.byref(a), 2, 4) == 1024 + (18 * 33 % 256) * 3 * 128 * 128 * 4   # five steps: no fourth slice
+
+
+def test_slices_of_joined_products():
+    """The rule over all sizes that it accepts: within the counters, no slice of fewer than ten steps, nothing for other rows; what the C entry takes."""
+    import ctypes as C
+    import random
+    from scalellm_amd import _lib, latent_kernels as lk
+    L, rng = _lib.latent_lib(), random.Random(5)
+    for _ in range(3000):
+        M, N, K = rng.randint(1, 140), 16 * rng.randint(1, 1200), 64 * rng.randint(1, 260)
+        n = lk.join_count(N, K, M)
+        assert 1 <= n <= 8
+        a = _lib.LinearArgs()
+        a.x = a.w = a.y = 1 << 20
+        a.M, a.N, a.K, a.ldx, a.ldy, a.batch, a.n_splits, a.dtype = M, N, K, K, N, 1, n, _lib.SLM_BF16
+        size = L.slm_linear_stream_join_bytes(C.byref(a))
+        if not 16 < M <= 128 or N > 16384:
+            assert n == 1 and size == 0
+            assert L.slm_linear_stream_join(C.byref(a), 1 << 20, 1 << 40, 1 << 20, None) == -2
+        else:
+            assert size >= n * M * N * 4
+            assert L.slm_linear_stream_join(C.byref(a), 1 << 20, size - 1, 1 << 20, None) < 0
+            assert L.slm_linear_stream_join(C.byref(a), 1 << 20, size, None, None) < 0
+        if n > 1:
+            assert K // 64 // n >= 10

@@ -165,6 +165,54 @@ def _streamed_products(M, N, K):
 
 # Weights whose columns are the results: the streamed form's edges in both 16-bit types (rows at the edges of its tiles, columns that fill no panel, parts that
 # are turned at a time, steps below and past the rings), rows with a stride.  fp32 sums of exact products, one rounding.
+@pytest.mark.parametrize("M", [17, 32, 33, 64, 65, 96, 97, 128])
+@pytest.mark.parametrize("N,K,n", [(16, 64, 3), (80, 704, 2), (3664, 1984, 3), (6752, 2112, 2), (9216, 1088, 3), (1040, 4160, 16), (16384, 192, 1)])
+def test_products_cut_in_k_and_joined(M, N, K, n):
+    """Splits without a step, last panels that are not whole, tiles of 32, 64 and 128 columns; the counters are zero again after every launch."""
+    lk = _lk()
+    from scalellm_amd import _lib
+    x, w = _rnd(1, M, K + 8, dtype=torch.bfloat16)[:, :K], _rnd(2, N, K, dtype=torch.bfloat16)
+    resid, h, table = torch.empty(1, 64, device="cuda"), torch.empty(1, 64, device="cuda"), torch.ones(1, 64, device="cuda")
+    tickets = torch.full((_lib.STREAM_TICKETS,), 7, dtype=torch.int32, device="cuda")
+    lk.residual_norm(resid, h, torch.ones(64, device="cuda"), 1e-5, embed=(torch.zeros(1, dtype=torch.int32, device="cuda"), table, None, None), clear=tickets)
+    want, outs = _f64(x) @ _f64(w).T, []
+    layout = lk.stream_layout(w)
+    for _ in range(3):
+        out = torch.full((M, N + 4), 9.0, dtype=torch.bfloat16, device="cuda")
+        a = lk._stream_args(x, w, layout, M, N, K, 128)
+        a.ldy, a.y, a.epilogue = out.stride(0), out.data_ptr(), _lib.LIN_STORE
+        assert lk._joined(a, n, tickets, x.device)
+        assert int(tickets.abs().max()) == 0
+        assert bool((out[:, N:] == 9.0).all())
+        outs.append(out[:, :N])
+    # one rounding to bf16 (2^-9) of sums whose 32-bit error is far below it
+    assert (np.abs(_f64(outs[0]) - want) - np.abs(want) * 2.0 ** -8).max() < 2e-5 * K ** 0.5
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+    got = lk.linear(x, w, layout=layout, tickets=tickets)   # (as many as pay, or none)
+    assert (np.abs(_f64(got) - want) - np.abs(want) * 2.0 ** -8).max() < 2e-5 * K ** 0.5 and int(tickets.abs().max()) == 0
+
+
+def test_joined_products_in_a_graph():
+    lk = _lk()
+    M, N, K = 100, 3664, 2048
+    x, w = _rnd(1, M, K, dtype=torch.bfloat16), _rnd(2, N, K, dtype=torch.bfloat16)
+    layout, tickets = lk.stream_layout(w), torch.zeros(512, dtype=torch.int32, device="cuda")
+    assert lk.join_count(N, K, M) > 1
+    lk.linear(x, w, layout=layout, tickets=tickets)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        first = lk.linear(x, w, layout=layout, tickets=tickets)
+        again = lk.linear(first[:, :K], w, layout=layout, tickets=tickets)
+    for i in range(4):
+        x.copy_(_rnd(3 + i, M, K, dtype=torch.bfloat16))
+        graph.replay()
+        torch.cuda.synchronize()
+        a = lk.linear(x, w, layout=layout, tickets=tickets)
+        b = lk.linear(a[:, :K], w, layout=layout, tickets=tickets)
+        assert torch.equal(first, a) and torch.equal(again, b)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("M", [1, 16, 17, 33, 65, 97, 128, 129])
 @pytest.mark.parametrize("K,N", [(64, 16), (192, 4112), (2112, 8240)])
