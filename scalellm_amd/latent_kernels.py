@@ -8,11 +8,12 @@ from __future__ import annotations
 import ctypes as C
 from typing import List, Optional, Tuple
 
+import numpy as np
 import torch
 
 from . import _lib
 from ._lib import SLM_BF16, SLM_F32, SlmError, latent_check
-from .kernels import reserve_workspace
+from .kernels import current_stream_handle as _stream, reserve_workspace
 
 # rows up to which a bf16 product of row-major weights is streamed
 STREAM_MAX_ROWS = 32
@@ -32,10 +33,6 @@ def _code(t: torch.Tensor) -> int:
     raise SlmError(f"unsupported dtype {t.dtype}: bfloat16 / float32 only")
 
 
-def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
-
-
 def _p(t: Optional[torch.Tensor]):
     if t is None:
         return None
@@ -51,6 +48,25 @@ def _need(ok: bool, what: str) -> None:
 
 def _i32(t: torch.Tensor, n: int, what: str) -> None:
     _need(t.dtype == torch.int32 and t.is_contiguous() and t.numel() >= n, f"{what}: contiguous int32 [>= {n}]")
+
+
+def arrays_to_device(arrays, device) -> List[torch.Tensor]:
+    """Contiguous int32 numpy arrays as tensors on the device, in one copy that nobody waits for: a copy out of pageable memory waits for all that
+    the stream has to do, and the device then for the host."""
+    if torch.device(device).type != "cuda":
+        return [torch.from_numpy(a).to(device) for a in arrays]
+    _need(not torch.cuda.is_current_stream_capturing(), "a step's plan is made of host data: it can't be captured")
+    _need(all(a.dtype == np.int32 for a in arrays), "plans are int32")
+    at, total = [], 0
+    for a in arrays:
+        at.append(total)
+        total += (a.size + 3) // 4 * 4   # (each on 16 bytes)
+    host = torch.empty(total, dtype=torch.int32, pin_memory=True)   # (torch's host pool keeps it until the copy is done)
+    flat = host.numpy()
+    for i, a in zip(at, arrays):
+        flat[i:i + a.size] = a.reshape(-1)
+    dev = host.to(device, non_blocking=True)
+    return [dev[i:i + a.size].view(a.shape) for i, a in zip(at, arrays)]
 
 
 class TanhNorm:
@@ -295,16 +311,14 @@ def _tile_pays(M: int, N: int, K: int, glu: bool) -> bool:
 def _gemm(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, glu=None, tile: int = -1, slices: int = 0) -> bool:
     """out = x w^T, or with glu = (limit, alpha, shift) the clamped GLU of its halves, by the tile kernel for many rows.  False:
     shapes and strides that it does not take."""
-    M, N, K = x.size(0), w.size(0), w.size(1)
-    half = x.dtype == torch.float16
-    if (not (half or x.dtype == torch.bfloat16) or w.dtype != x.dtype or out.dtype != x.dtype or not N or not K or K % 64 or N % (32 if glu else 16) or x.stride(0) < K or (x.stride(0) | w.stride(0) | out.stride(0)) % 8 or
-            (x.data_ptr() | w.data_ptr() | out.data_ptr()) % 16 or max(M * x.stride(0), N * w.stride(0)) > 1 << 30 or max(M, N) > 1 << 24):
+    M, (N, K), dtype = x.size(0), w.shape, x.dtype
+    half, ldx, ldw, ldy = dtype == torch.float16, x.stride(0), w.stride(0), out.stride(0)
+    if (not (half or dtype == torch.bfloat16) or w.dtype != dtype or out.dtype != dtype or not N or not K or K % 64 or N % (32 if glu else 16) or
+            ldx < K or (ldx | ldw | ldy) % 8 or (x.data_ptr() | w.data_ptr() | out.data_ptr()) % 16 or max(M * ldx, N * ldw) > 1 << 30 or max(M, N) > 1 << 24):
         return False
-    a = _lib.LinearArgs()
-    a.x, a.w, a.M, a.N, a.K, a.alpha, a.batch, a.n_splits, a.dtype = _p(x), _p(w), M, N, K, 1.0, 1, 1, SLM_BF16
-    a.ldx, a.ldw, a.ldy, a.y, a.epilogue = x.stride(0), w.stride(0), out.stride(0), _p(out), _lib.LIN_STORE
-    if glu:
-        a.epilogue, a.limit, a.glu_alpha, a.glu_shift = _lib.LIN_GLU, *glu
+    limit, alpha, shift = glu or (0.0, 0.0, 0.0)
+    # (in the order of the fields: a third of what setting them one by one takes)
+    a = _lib.LinearArgs(_p(x), _p(w), _p(out), None, M, N, K, ldx, ldw, ldy, 0, 0, 0, 0, 1.0, limit, alpha, shift, 1, 1, _lib.LIN_GLU if glu else _lib.LIN_STORE, SLM_BF16)
     L = _lib.latent_lib()
     need, ws = L.slm_gemm_workspace_bytes(C.byref(a), tile, slices), None
     if need:

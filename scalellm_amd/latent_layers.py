@@ -101,7 +101,7 @@ class LatentPlan:
     @staticmethod
     def build(portions: Sequence[Portion], window: int, block_size: int, device) -> "LatentPlan":
         slots, tiles = LatentPlan.host(portions, window, block_size)
-        return LatentPlan(torch.from_numpy(slots).to(device), torch.from_numpy(tiles).to(device))
+        return LatentPlan(*lk.arrays_to_device((slots, tiles), device))
 
 
 # ---------------------------------------------------------------------------------------

@@ -15,7 +15,7 @@ import torch
 from . import _lib
 from ._lib import mixers_check
 from .kernels import reserve_workspace
-from .latent_kernels import _code, _i32, _need, _p, _stream
+from .latent_kernels import _code, _i32, _need, _p, _stream, arrays_to_device
 from .layers import InputParameters, RecurrentState
 
 
@@ -141,7 +141,7 @@ class ChunkPlan:
         plan = params.plans.get("chunks")
         if plan is None:
             chunks, first = ChunkPlan.host(params.portions, n_single)
-            plan = params.plans["chunks"] = ChunkPlan(torch.from_numpy(chunks).to(device), torch.from_numpy(first).to(device))
+            plan = params.plans["chunks"] = ChunkPlan(*arrays_to_device((chunks, first), device))
         return plan
 
 

@@ -92,7 +92,7 @@ class WindowPlan:
         plan = params.plans.get(key)
         if plan is None:
             slots, tiles = WindowPlan.host(params.portions, window, keep_first, block_size)
-            plan = params.plans[key] = WindowPlan(torch.from_numpy(slots).to(device), torch.from_numpy(tiles).to(device))
+            plan = params.plans[key] = WindowPlan(*lk.arrays_to_device((slots, tiles), device))
         return plan
 
 
