@@ -296,6 +296,7 @@ def latent_lib() -> C.CDLL:
         ("slm_linear_stream_join", C.c_int, [P(LinearArgs), ptr, C.c_size_t, ptr, ptr]),
         ("slm_gemm_workspace_bytes", C.c_size_t, [P(LinearArgs), i32, i32]),
         ("slm_gemm", C.c_int, [P(LinearArgs), ptr, C.c_size_t, i32, i32, ptr]),
+        ("slm_gemm_counted", C.c_int, [P(LinearArgs), ptr, C.c_size_t, ptr, i32, i32, ptr]),
         ("slm_gemm_half", C.c_int, [P(LinearArgs), ptr, C.c_size_t, i32, i32, ptr]),
         ("slm_stream_layout", C.c_int, [ptr, ptr, i64, i64, i32, ptr]),
         ("slm_clamped_glu", C.c_int, [ptr, ptr, i64, i64, i64, i64, f32, f32, f32, i32, ptr]),

@@ -365,7 +365,7 @@ extern "C" SLM_API size_t slm_gemm_workspace_bytes(const slm_linear_args* a, int
 }
 
 template <typename T>
-static int gemm_run(const slm_linear_args* a, void* workspace, size_t workspace_bytes, int32_t tile, int32_t slices, void* stream) {
+static int gemm_run(const slm_linear_args* a, void* workspace, size_t workspace_bytes, uint32_t* tickets, int32_t tile, int32_t slices, void* stream) {
   const int rc = gemm_check(a, tile, slices, std::is_same<T, bf16_tag>::value ? SLM_BF16 : SLM_F16);
   if (rc != SLM_OK || a->M == 0) return rc;
   GemmPlan p = gemm_plan(*a, tile, slices);
@@ -376,15 +376,18 @@ static int gemm_run(const slm_linear_args* a, void* workspace, size_t workspace_
   k.M = a->M; k.N = a->N; k.K = a->K; k.ldy = a->ldy; k.ldx2 = (uint32_t)(a->ldx * 2); k.ldw2 = (uint32_t)(a->ldw * 2);
   k.limit = a->limit; k.alpha = a->glu_alpha; k.shift = a->glu_shift;
   k.mb = p.mb; k.nb = p.nb; k.whole = p.whole; k.cut = p.cut; k.slices = p.slices; k.group = 8;
-  k.arrived = (uint32_t*)workspace; k.slabs = (float*)((char*)workspace + 1024);
+  k.arrived = tickets ? tickets : (uint32_t*)workspace; k.slabs = (float*)((char*)workspace + 1024);
   hipStream_t st = (hipStream_t)stream;
   hip_clear_error();
-  if (p.cut) tile_clear_kernel<<<dim3(1), dim3(256), 0, st>>>(k.arrived, p.cut);
+  if (p.cut && !tickets) tile_clear_kernel<<<dim3(1), dim3(256), 0, st>>>(k.arrived, p.cut);
   return a->epilogue == SLM_LIN_GLU ? gemm_tile<T, true>(p, k, st) : gemm_tile<T, false>(p, k, st);
 }
 extern "C" SLM_API int slm_gemm(const slm_linear_args* a, void* workspace, size_t workspace_bytes, int32_t tile, int32_t slices, void* stream) {
-  return gemm_run<bf16_tag>(a, workspace, workspace_bytes, tile, slices, stream);
+  return gemm_run<bf16_tag>(a, workspace, workspace_bytes, nullptr, tile, slices, stream);
 }
 extern "C" SLM_API int slm_gemm_half(const slm_linear_args* a, void* workspace, size_t workspace_bytes, int32_t tile, int32_t slices, void* stream) {
-  return gemm_run<f16_tag>(a, workspace, workspace_bytes, tile, slices, stream);
+  return gemm_run<f16_tag>(a, workspace, workspace_bytes, nullptr, tile, slices, stream);
+}
+extern "C" SLM_API int slm_gemm_counted(const slm_linear_args* a, void* workspace, size_t workspace_bytes, uint32_t* tickets, int32_t tile, int32_t slices, void* stream) {
+  return tickets ? gemm_run<bf16_tag>(a, workspace, workspace_bytes, tickets, tile, slices, stream) : SLM_ERR_INVALID_ARG;
 }

@@ -173,7 +173,7 @@ class DagupelStep:
             delta = L.attn.forward(h, positions, self.caches[i], params, tickets)
             if L.mlp is not None:
                 lk.residual_norm(resid, h, L.norm2, c.eps, delta=delta)
-                delta = L.mlp.forward(h)
+                delta = L.mlp.forward(h, tickets)
             lk.residual_norm(resid, h, nxt, c.eps, delta=delta)
             if self.on_layer is not None:
                 self.on_layer(i, resid)

@@ -260,9 +260,13 @@ def _store_rows(N: int, K: int) -> int:
 
 
 def step_tickets(rows: int, device) -> Optional[torch.Tensor]:
-    """What linear()'s products cut in K count their arrivals by in a step of so many rows (None: not cut): cleared by the residual_norm() of the
+    """What linear()'s products cut in K count their arrivals by in a step of so many rows (None: nothing is cut): cleared by the residual_norm() of the
     embedding that they follow, left at zero by each of them, of one step alone."""
-    return torch.empty(_lib.STREAM_TICKETS, dtype=torch.int32, device=device) if 16 < rows <= STREAM_LAYOUT_MAX_ROWS else None
+    return torch.empty(_lib.STREAM_TICKETS, dtype=torch.int32, device=device) if rows > 16 else None
+
+
+def _check_tickets(tickets: torch.Tensor, device) -> None:
+    _need(tickets.dtype == torch.int32 and tickets.is_contiguous() and tickets.numel() >= _lib.STREAM_TICKETS and tickets.device == device, "linear: tickets")
 
 
 def join_count(N: int, K: int, rows: int) -> int:
@@ -284,7 +288,7 @@ def join_count(N: int, K: int, rows: int) -> int:
 def _joined(a, n: int, tickets: torch.Tensor, device) -> bool:
     """The stored product in n slices of K; False: no memory for them."""
     L = _lib.latent_lib()
-    _need(tickets.dtype == torch.int32 and tickets.is_contiguous() and tickets.numel() >= _lib.STREAM_TICKETS and tickets.device == device, "linear: tickets")
+    _check_tickets(tickets, device)
     a.n_splits = n
     try:   # (the launch's own: products of other streams have theirs)
         ws = torch.empty(L.slm_linear_stream_join_bytes(C.byref(a)), dtype=torch.uint8, device=device)
@@ -308,9 +312,9 @@ def _tile_pays(M: int, N: int, K: int, glu: bool) -> bool:
     return glu or M <= 1024 or K < 1024 or -(-M // 256) * -(-N // 256) % 256 != 0
 
 
-def _gemm(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, glu=None, tile: int = -1, slices: int = 0) -> bool:
-    """out = x w^T, or with glu = (limit, alpha, shift) the clamped GLU of its halves, by the tile kernel for many rows.  False:
-    shapes and strides that it does not take."""
+def _gemm(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, glu=None, tile: int = -1, slices: int = 0, tickets: Optional[torch.Tensor] = None) -> bool:
+    """out = x w^T, or with glu = (limit, alpha, shift) the clamped GLU of its halves, by the tile kernel for many rows.  tickets (bf16): step_tickets(),
+    cleared.  False: shapes and strides that it does not take."""
     M, (N, K), dtype = x.size(0), w.shape, x.dtype
     half, ldx, ldw, ldy = dtype == torch.float16, x.stride(0), w.stride(0), out.stride(0)
     if (not (half or dtype == torch.bfloat16) or w.dtype != dtype or out.dtype != dtype or not N or not K or K % 64 or N % (32 if glu else 16) or
@@ -326,6 +330,10 @@ def _gemm(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, glu=None, tile: i
             ws = torch.empty(need, dtype=torch.uint8, device=x.device)
         except torch.OutOfMemoryError:
             need = 0
+    if need and tickets is not None and not half:
+        _check_tickets(tickets, x.device)
+        latent_check(L.slm_gemm_counted(C.byref(a), ws.data_ptr(), need, tickets.data_ptr(), tile, slices, _stream()), "slm_gemm_counted")
+        return True
     if half:
         a.dtype = _lib.SLM_F16
     latent_check((L.slm_gemm_half if half else L.slm_gemm)(C.byref(a), ws.data_ptr() if ws is not None else None, need, tile, slices, _stream()), "slm_gemm")
@@ -353,7 +361,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None,
         return out
     if not streams_rows(x):
         # (of row-major weights stored products of up to 128 rows are the vendor's, whose small tiles leave fewer CUs idle)
-        return out if M >= TILE_MIN_ROWS and _tile_pays(M, N, K, False) and _gemm(x, w, out) else torch.mm(x, w.t(), out=out)
+        return out if M >= TILE_MIN_ROWS and _tile_pays(M, N, K, False) and _gemm(x, w, out, tickets=tickets) else torch.mm(x, w.t(), out=out)
     a = _linear_args(x, w, M, N, K)
     a.ldx, a.ldw, a.ldy, a.y, a.epilogue = x.stride(0), K, out.stride(0), _p(out), _lib.LIN_STORE
     _run_linear(a)
@@ -450,7 +458,7 @@ def linear_slabs(x: torch.Tensor, w: torch.Tensor, layout: Optional[torch.Tensor
 
 
 def linear_glu(x: torch.Tensor, w_gate_up: torch.Tensor, out: torch.Tensor, limit: float, alpha: float = GLU_ALPHA,
-               shift: float = GLU_SHIFT, layout: Optional[torch.Tensor] = None) -> torch.Tensor:
+               shift: float = GLU_SHIFT, layout: Optional[torch.Tensor] = None, tickets: Optional[torch.Tensor] = None) -> torch.Tensor:
     """out = clamped GLU of the two halves of x [gate | up]^T: the activation is the product's epilogue where a streaming kernel or
     the tile kernel runs, one more launch behind the vendor GEMM otherwise.  layout: stream_layout(w_gate_up, glu=True)."""
     M, N, K = _check_xw(x, w_gate_up)
@@ -470,7 +478,7 @@ def linear_glu(x: torch.Tensor, w_gate_up: torch.Tensor, out: torch.Tensor, limi
         a.ldx, a.ldw, a.ldy, a.y, a.epilogue = x.stride(0), K, out.stride(0), _p(out), _lib.LIN_GLU
         a.limit, a.glu_alpha, a.glu_shift = float(limit), float(alpha), float(shift)
         (_run_linear if s is None else _run_stream)(a)
-    elif not (_tile_pays(M, N, K, True) and _gemm(x, w_gate_up, out, (float(limit), float(alpha), float(shift)))):
+    elif not (_tile_pays(M, N, K, True) and _gemm(x, w_gate_up, out, (float(limit), float(alpha), float(shift)), tickets=tickets)):
         gu = torch.mm(x, w_gate_up.t())
         clamped_glu(gu, out, limit, alpha, shift)
     return out

@@ -221,12 +221,12 @@ class LatentAttention:
             if plan is None:
                 plan = params.plans[a.window] = LatentPlan.build(portions, a.window, cache.block_size(), h.device)
             ctx = lk.latent_gather(cache.rows, plan.slots)
-            kv = lk.linear(ctx[:, :self.c_pad], self.w_ukv)
+            kv = lk.linear(ctx[:, :self.c_pad], self.w_ukv, tickets=tickets)
             lk.latent_prefill(proj, ctx, kv, out, plan.tiles, heads=a.heads, q_dim=self.q_dim, c_pad=self.c_pad,
                               v_pad=self.v_pad, gate_off=self.off_g, window=a.window, scale=a.scale)
         if T <= lk.slab_rows(self.l_o):
             return lk.linear_slabs(out, self.w_o, self.l_o)
-        return lk.linear(out, self.w_o)
+        return lk.linear(out, self.w_o, tickets=tickets)
 
 
 # ---------------------------------------------------------------------------------------
@@ -249,9 +249,9 @@ class ClampedGLU:
         self.w_down[:width, :ff] = w["down"].to(device=device, dtype=dtype)
         lk.lay_out([self], None if layouts else 0)
 
-    def forward(self, h: torch.Tensor):
+    def forward(self, h: torch.Tensor, tickets: Optional[torch.Tensor] = None):
         act = h.new_empty(h.size(0), self.w_down.size(1))
-        lk.linear_glu(h, self.w_gate_up, act, self.limit, self.alpha, self.shift, self.l_gate_up)
+        lk.linear_glu(h, self.w_gate_up, act, self.limit, self.alpha, self.shift, self.l_gate_up, tickets)
         if h.size(0) <= lk.slab_rows(self.l_down):
             return lk.linear_slabs(act, self.w_down, self.l_down)
-        return lk.linear(act, self.w_down)
+        return lk.linear(act, self.w_down, tickets=tickets)

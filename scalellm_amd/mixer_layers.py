@@ -29,9 +29,9 @@ def single_rows(params: InputParameters, rows: int) -> int:
     return rows
 
 
-def out_product(x: torch.Tensor, w: torch.Tensor, layout: Optional[torch.Tensor] = None):
-    """What the residual stream receives: split-K slabs for few rows, a tensor otherwise.  layout: lk.stream_layout(w)."""
-    return lk.linear_slabs(x, w, layout) if x.size(0) <= lk.slab_rows(layout) else lk.linear(x, w)
+def out_product(x: torch.Tensor, w: torch.Tensor, layout: Optional[torch.Tensor] = None, tickets: Optional[torch.Tensor] = None):
+    """What the residual stream receives: split-K slabs for few rows, a tensor otherwise.  layout: lk.stream_layout(w), tickets: lk.step_tickets()."""
+    return lk.linear_slabs(x, w, layout) if x.size(0) <= lk.slab_rows(layout) else lk.linear(x, w, tickets=tickets)
 
 
 def _rows_of(n: int, k: int, width: int, parts, dtype, device) -> torch.Tensor:
@@ -223,7 +223,7 @@ class ParallelMixer:
         out = proj.new_empty(h.size(0), self.o_k)
         self.left.forward(proj[:, :self.split], positions, cache[0], params, out[:, :self.left.out_width])
         self.right.forward(proj[:, self.split:], positions, cache[1], params, out[:, self.left.out_width:])
-        return out_product(out, self.w_o, self.l_o)
+        return out_product(out, self.w_o, self.l_o, tickets)
 
 
 # ---------------------------------------------------------------------------------------
@@ -289,11 +289,11 @@ class ChannelDelta:
             lk.linear_heads(low_in, self.low_k, self.w_low, low, self.low_n)
         else:
             for i in range(2):
-                lk.linear(low_in[:, i * self.low_k:(i + 1) * self.low_k], self.w_low[i], low[:, i * self.low_n:(i + 1) * self.low_n])
+                lk.linear(low_in[:, i * self.low_k:(i + 1) * self.low_k], self.w_low[i], low[:, i * self.low_n:(i + 1) * self.low_n], tickets=tickets)
         out = proj.new_empty(T, self.o_k)
         step = (s, proj, low, state, positions, params.q_cu_seq_lens, params.state_slots, n)
         if n:
             mk.recurrent_step(*step, out=out[:n])
         if n < T:
             mk.gated_norm(mk.recurrent_portions(*step, mk.ChunkPlan.of(params, n, proj.device)), s.vdim, low[n:, self.low_n:], s.norm_weight, out[n:], eps=self.eps, per_head=True)
-        return out_product(out, self.w_o, self.l_o)
+        return out_product(out, self.w_o, self.l_o, tickets)

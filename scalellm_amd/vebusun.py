@@ -199,7 +199,7 @@ class VebusunStep:
             delta = L.mixer.forward(h, positions, self.caches[i], params, tickets)
             if L.mlp is not None:
                 lk.residual_norm(resid, h, L.norm2, c.eps, delta=delta, mult=c.residual_mult)
-                delta = L.mlp.forward(h)
+                delta = L.mlp.forward(h, tickets)
             lk.residual_norm(resid, h, nxt, c.eps, delta=delta, mult=c.residual_mult)
             if self.on_layer is not None:
                 self.on_layer(i, resid)

@@ -281,6 +281,27 @@ def test_tiled_products_of_several_rounds(M, N, K, slices, tile):
     test_tiled_products(M, N, K, slices, tile)
 
 
+@pytest.mark.parametrize("M,N,K,slices,glu", [(257, 96, 1088, 5, False), (300, 544, 704, 3, True), (1100, 16416, 704, 2, False), (207, 4096, 2048, 0, False)])
+def test_tiled_products_with_counters_of_the_callers(M, N, K, slices, glu):
+    """The same bits as with counters of the launch's own, which are zero again behind it; eagerly and in a graph."""
+    lk = _lk()
+    x, w = _rnd(1, M, K, dtype=torch.bfloat16), _rnd(2, N, K, dtype=torch.bfloat16, std=K ** -0.5)
+    how = dict(glu=(7.0, 1.0, 0.0) if glu else None, slices=slices)
+    want, got = (torch.zeros(M, N // 2 if glu else N, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    tickets = torch.zeros(512, dtype=torch.int32, device="cuda")
+    assert lk._gemm(x, w, want, **how) and lk._gemm(x, w, got, tickets=tickets, **how)
+    assert torch.equal(want, got) and int(tickets.abs().max()) == 0
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        for _ in range(2):
+            lk._gemm(x, w, got, tickets=tickets, **how)
+    for i in range(3):
+        x.copy_(_rnd(3 + i, M, K, dtype=torch.bfloat16))
+        graph.replay()
+        lk._gemm(x, w, want, **how)
+        assert torch.equal(want, got) and int(tickets.abs().max()) == 0
+
+
 @pytest.mark.parametrize("M", [129, 700])
 def test_products_of_prompts_by_the_planned_tile(M):
     lk, N, K = _lk(), 2080, 1024
