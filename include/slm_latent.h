@@ -84,8 +84,10 @@ SLM_API int slm_stream_layout(void* out, const void* w, int64_t N, int64_t K, in
 /* last round are cut in K by n.  Without the workspace (optional, content does not matter) nothing is cut.     */
 SLM_API size_t slm_gemm_workspace_bytes(const slm_linear_args* a, int32_t tile, int32_t slices);
 SLM_API int slm_gemm(const slm_linear_args* a, void* workspace, size_t workspace_bytes, int32_t tile, int32_t slices, void* stream);
-/* The same with counters of the caller's, tickets [SLM_STREAM_TICKETS], zero before and after: a launch less where it is cut */
-SLM_API int slm_gemm_counted(const slm_linear_args* a, void* workspace, size_t workspace_bytes, uint32_t* tickets, int32_t tile, int32_t slices, void* stream);
+/* The same, or in half precision (by dtype), with counters of the caller's, counters [SLM_GEMM_COUNTERS], zero before, of this */
+/* product alone: a launch less where it is cut                                                                  */
+#define SLM_GEMM_COUNTERS 256
+SLM_API int slm_gemm_counted(const slm_linear_args* a, void* workspace, size_t workspace_bytes, uint32_t* counters, int32_t tile, int32_t slices, void* stream);
 /* The same in half precision (dtype SLM_F16); its workspace is that of the call in bf16                        */
 SLM_API int slm_gemm_half(const slm_linear_args* a, void* workspace, size_t workspace_bytes, int32_t tile, int32_t slices, void* stream);
 /* y = g sigmoid(alpha g) (u + shift), g = min(gate, limit), u = clamp(up, +-limit) (limit may be        */

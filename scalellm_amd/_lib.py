@@ -234,7 +234,7 @@ class ResidualNormArgs(C.Structure):
 
 NORM_RMS, NORM_TANH = range(2)
 RN_EMBED, RN_ADD, RN_SLABS, RN_PLAIN = range(4)
-STREAM_TICKETS = 512
+STREAM_TICKETS, GEMM_COUNTERS = 512, 256
 
 
 class LinearArgs(C.Structure):

@@ -260,6 +260,7 @@ constexpr GemmTile GEMM_TILES[] = {{256, 256, 0.914f, 1.386f, 8.6f}, {256, 128, 
                                    {256, 192, 0.725f, 1.037f, 6.6f}, {192, 256, 0.743f, 1.071f, 6.6f}, {160, 256, 0.647f, 0.909f, 6.1f}};
 constexpr int GEMM_N_TILES = sizeof(GEMM_TILES) / sizeof(GEMM_TILES[0]), GEMM_256_192 = 4;   // (that one has no GLU)
 constexpr int GEMM_CUS = 256;
+static_assert(SLM_GEMM_COUNTERS >= GEMM_CUS, "a counter for each tile of a round");
 constexpr float GEMM_CUT = 6.f, GEMM_SLABS = 3.5e6f;   // us of cutting tiles, bytes of their slabs that take one more
 
 struct GemmPlan {
@@ -365,7 +366,7 @@ extern "C" SLM_API size_t slm_gemm_workspace_bytes(const slm_linear_args* a, int
 }
 
 template <typename T>
-static int gemm_run(const slm_linear_args* a, void* workspace, size_t workspace_bytes, uint32_t* tickets, int32_t tile, int32_t slices, void* stream) {
+static int gemm_run(const slm_linear_args* a, void* workspace, size_t workspace_bytes, uint32_t* counters, int32_t tile, int32_t slices, void* stream) {
   const int rc = gemm_check(a, tile, slices, std::is_same<T, bf16_tag>::value ? SLM_BF16 : SLM_F16);
   if (rc != SLM_OK || a->M == 0) return rc;
   GemmPlan p = gemm_plan(*a, tile, slices);
@@ -376,10 +377,10 @@ static int gemm_run(const slm_linear_args* a, void* workspace, size_t workspace_
   k.M = a->M; k.N = a->N; k.K = a->K; k.ldy = a->ldy; k.ldx2 = (uint32_t)(a->ldx * 2); k.ldw2 = (uint32_t)(a->ldw * 2);
   k.limit = a->limit; k.alpha = a->glu_alpha; k.shift = a->glu_shift;
   k.mb = p.mb; k.nb = p.nb; k.whole = p.whole; k.cut = p.cut; k.slices = p.slices; k.group = 8;
-  k.arrived = tickets ? tickets : (uint32_t*)workspace; k.slabs = (float*)((char*)workspace + 1024);
+  k.arrived = counters ? counters : (uint32_t*)workspace; k.slabs = (float*)((char*)workspace + 1024);
   hipStream_t st = (hipStream_t)stream;
   hip_clear_error();
-  if (p.cut && !tickets) tile_clear_kernel<<<dim3(1), dim3(256), 0, st>>>(k.arrived, p.cut);
+  if (p.cut && !counters) tile_clear_kernel<<<dim3(1), dim3(256), 0, st>>>(k.arrived, p.cut);
   return a->epilogue == SLM_LIN_GLU ? gemm_tile<T, true>(p, k, st) : gemm_tile<T, false>(p, k, st);
 }
 extern "C" SLM_API int slm_gemm(const slm_linear_args* a, void* workspace, size_t workspace_bytes, int32_t tile, int32_t slices, void* stream) {
@@ -388,6 +389,8 @@ extern "C" SLM_API int slm_gemm(const slm_linear_args* a, void* workspace, size_
 extern "C" SLM_API int slm_gemm_half(const slm_linear_args* a, void* workspace, size_t workspace_bytes, int32_t tile, int32_t slices, void* stream) {
   return gemm_run<f16_tag>(a, workspace, workspace_bytes, nullptr, tile, slices, stream);
 }
-extern "C" SLM_API int slm_gemm_counted(const slm_linear_args* a, void* workspace, size_t workspace_bytes, uint32_t* tickets, int32_t tile, int32_t slices, void* stream) {
-  return tickets ? gemm_run<bf16_tag>(a, workspace, workspace_bytes, tickets, tile, slices, stream) : SLM_ERR_INVALID_ARG;
+extern "C" SLM_API int slm_gemm_counted(const slm_linear_args* a, void* workspace, size_t workspace_bytes, uint32_t* counters, int32_t tile, int32_t slices, void* stream) {
+  if (!a || !counters) return SLM_ERR_INVALID_ARG;
+  return a->dtype == SLM_F16 ? gemm_run<f16_tag>(a, workspace, workspace_bytes, counters, tile, slices, stream)
+                             : gemm_run<bf16_tag>(a, workspace, workspace_bytes, counters, tile, slices, stream);
 }

@@ -99,10 +99,9 @@ __device__ __forceinline__ bool stream_join(f32x4 (&acc)[F], const StreamJoin& j
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // every wave's sums are out ..
   __syncthreads();
-  if (threadIdx.x == 0) *word = __hip_atomic_fetch_add(j.arrived + blockIdx.x, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // .. then one announces them
+  if (threadIdx.x == 0) *word = atomicInc(j.arrived + blockIdx.x, (uint32_t)splits - 1);   // .. then one announces them (the last one's turns to zero)
   __syncthreads();
   if (*word != (uint32_t)splits - 1) return false;
-  if (threadIdx.x == 0) __hip_atomic_store(j.arrived + blockIdx.x, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   if (t >= 256) return true;
   if (splits == 2) {   // (its own are at hand; the other order has the same sum)
 #pragma unroll

@@ -33,8 +33,8 @@ __global__ void __launch_bounds__(T) residual_norm_kernel(const slm_residual_nor
   const int tid = threadIdx.x;
   const int64_t row = blockIdx.x;
   const int width = (int)a.width;
-  if (MODE == SLM_RN_EMBED && row == 0) {   // (somebody's counters: a launch less)
-    for (int i = tid; i < a.n_clear; i += T) a.clear[i] = 0;
+  if constexpr (MODE == SLM_RN_EMBED) {   // (somebody's counters: a launch less)
+    for (int64_t i = row * T + tid; i < a.n_clear; i += a.rows * T) a.clear[i] = 0;
   }
   const int64_t src_row = (MODE == SLM_RN_PLAIN && a.row_index) ? a.row_index[row] + a.row_shift : row;
   float* r = a.resid + src_row * a.width;

@@ -28,7 +28,7 @@ __device__ __forceinline__ void tile_settle(f32x4 (&acc)[NT][MT]) {
   tile_products_settle(acc);
 }
 
-// The tile's fp32 sums go past the caches to its slabs, [slices][NT MT][256] f32x4; the last slice to arrive (*arrived, zero before and after) adds them up in
+// The tile's fp32 sums go past the caches to its slabs, [slices][NT MT][256] f32x4; the last slice to arrive (*arrived, zero before) adds them up in
 // slice order -- the same bits whoever is last -- and is the one that gets true.  Nobody waits for anybody.  256 threads; lds: 4 bytes of it.
 template <int NT, int MT>
 __device__ __forceinline__ bool tile_add_slices(f32x4 (&acc)[NT][MT], float* slabs, uint32_t* arrived, int slice, int slices, char* lds) {
@@ -45,7 +45,6 @@ __device__ __forceinline__ bool tile_add_slices(f32x4 (&acc)[NT][MT], float* sla
   if (tid == 0) word[0] = __hip_atomic_fetch_add(arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // .. then one announces them
   __syncthreads();
   if (word[0] != (uint32_t)slices - 1) return false;
-  if (tid == 0) __hip_atomic_store(arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
   for (int f0 = 0; f0 < FRAGS; f0 += C) {
     f32x4 sum[C];

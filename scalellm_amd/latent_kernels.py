@@ -259,14 +259,30 @@ def _store_rows(N: int, K: int) -> int:
     return 64 if N >= 8192 and K <= 2048 + 5 * (N - 8192) // 2 else STREAM_MAX_ROWS
 
 
-def step_tickets(rows: int, device) -> Optional[torch.Tensor]:
-    """What linear()'s products cut in K count their arrivals by in a step of so many rows (None: nothing is cut): cleared by the residual_norm() of the
-    embedding that they follow, left at zero by each of them, of one step alone."""
-    return torch.empty(_lib.STREAM_TICKETS, dtype=torch.int32, device=device) if rows > 16 else None
+class StepTickets:
+    """What the products of one step that are cut in K count their arrivals by: `words`, cleared by the residual_norm() of the embedding that they
+    follow.  Streamed products share the first ones, which each of them leaves at zero; a tile product takes some of its own."""
+    __slots__ = ("words", "at")
+
+    def __init__(self, words: torch.Tensor):
+        self.words, self.at = words, _lib.STREAM_TICKETS
+
+    def take(self) -> Optional[torch.Tensor]:
+        """Counters of the next tile product; None: none left (it clears some itself)."""
+        at, self.at = self.at, self.at + _lib.GEMM_COUNTERS
+        return self.words[at:self.at] if self.at <= self.words.numel() else None
 
 
-def _check_tickets(tickets: torch.Tensor, device) -> None:
-    _need(tickets.dtype == torch.int32 and tickets.is_contiguous() and tickets.numel() >= _lib.STREAM_TICKETS and tickets.device == device, "linear: tickets")
+def step_tickets(rows: int, products: int, device) -> Optional[StepTickets]:
+    """For a step of so many rows and at most so many tile products (None: nothing is cut)."""
+    if rows <= 16:
+        return None
+    n = 0 if rows < TILE_MIN_ROWS else min(products, 240)
+    return StepTickets(torch.empty(_lib.STREAM_TICKETS + n * _lib.GEMM_COUNTERS, dtype=torch.int32, device=device))
+
+
+def _check_counters(t: torch.Tensor, n: int, device) -> None:
+    _need(t.dtype == torch.int32 and t.is_contiguous() and t.numel() >= n and t.device == device, "linear: counters")
 
 
 def join_count(N: int, K: int, rows: int) -> int:
@@ -285,17 +301,17 @@ def join_count(N: int, K: int, rows: int) -> int:
     return max(1, min(8, 256 // panels, K // 640))
 
 
-def _joined(a, n: int, tickets: torch.Tensor, device) -> bool:
+def _joined(a, n: int, words: torch.Tensor, device) -> bool:
     """The stored product in n slices of K; False: no memory for them."""
     L = _lib.latent_lib()
-    _check_tickets(tickets, device)
+    _check_counters(words, _lib.STREAM_TICKETS, device)
     a.n_splits = n
     try:   # (the launch's own: products of other streams have theirs)
         ws = torch.empty(L.slm_linear_stream_join_bytes(C.byref(a)), dtype=torch.uint8, device=device)
     except torch.OutOfMemoryError:
         a.n_splits = 1
         return False
-    latent_check(L.slm_linear_stream_join(C.byref(a), ws.data_ptr(), ws.numel(), tickets.data_ptr(), _stream()), "slm_linear_stream_join")
+    latent_check(L.slm_linear_stream_join(C.byref(a), ws.data_ptr(), ws.numel(), words.data_ptr(), _stream()), "slm_linear_stream_join")
     return True
 
 
@@ -312,8 +328,8 @@ def _tile_pays(M: int, N: int, K: int, glu: bool) -> bool:
     return glu or M <= 1024 or K < 1024 or -(-M // 256) * -(-N // 256) % 256 != 0
 
 
-def _gemm(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, glu=None, tile: int = -1, slices: int = 0, tickets: Optional[torch.Tensor] = None) -> bool:
-    """out = x w^T, or with glu = (limit, alpha, shift) the clamped GLU of its halves, by the tile kernel for many rows.  tickets (bf16): step_tickets(),
+def _gemm(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, glu=None, tile: int = -1, slices: int = 0, tickets: Optional[StepTickets] = None) -> bool:
+    """out = x w^T, or with glu = (limit, alpha, shift) the clamped GLU of its halves, by the tile kernel for many rows.  tickets: step_tickets(),
     cleared.  False: shapes and strides that it does not take."""
     M, (N, K), dtype = x.size(0), w.shape, x.dtype
     half, ldx, ldw, ldy = dtype == torch.float16, x.stride(0), w.stride(0), out.stride(0)
@@ -330,12 +346,13 @@ def _gemm(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, glu=None, tile: i
             ws = torch.empty(need, dtype=torch.uint8, device=x.device)
         except torch.OutOfMemoryError:
             need = 0
-    if need and tickets is not None and not half:
-        _check_tickets(tickets, x.device)
-        latent_check(L.slm_gemm_counted(C.byref(a), ws.data_ptr(), need, tickets.data_ptr(), tile, slices, _stream()), "slm_gemm_counted")
-        return True
     if half:
         a.dtype = _lib.SLM_F16
+    counters = tickets.take() if need and tickets is not None else None
+    if counters is not None:
+        _check_counters(counters, _lib.GEMM_COUNTERS, x.device)
+        latent_check(L.slm_gemm_counted(C.byref(a), ws.data_ptr(), need, counters.data_ptr(), tile, slices, _stream()), "slm_gemm_counted")
+        return True
     latent_check((L.slm_gemm_half if half else L.slm_gemm)(C.byref(a), ws.data_ptr() if ws is not None else None, need, tile, slices, _stream()), "slm_gemm")
     return True
 
@@ -344,7 +361,7 @@ gemm = _gemm   # (for other modules)
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None, layout: Optional[torch.Tensor] = None,
-           tickets: Optional[torch.Tensor] = None) -> torch.Tensor:
+           tickets: Optional[StepTickets] = None) -> torch.Tensor:
     """x [M, K] W[N, K]^T -> [M, N] of the same dtype.  layout: stream_layout(w); tickets: step_tickets(), cleared."""
     M, N, K = _check_xw(x, w)
     if out is None:
@@ -356,7 +373,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None,
     a = _stream_args(x, w, layout, M, N, K, _store_rows(N, K) if tickets is None else STREAM_LAYOUT_MAX_ROWS)
     if a is not None:
         a.ldy, a.y, a.epilogue = out.stride(0), _p(out), _lib.LIN_STORE
-        if n == 1 or not _joined(a, n, tickets, x.device):
+        if n == 1 or not _joined(a, n, tickets.words, x.device):
             _run_stream(a)
         return out
     if not streams_rows(x):
@@ -458,7 +475,7 @@ def linear_slabs(x: torch.Tensor, w: torch.Tensor, layout: Optional[torch.Tensor
 
 
 def linear_glu(x: torch.Tensor, w_gate_up: torch.Tensor, out: torch.Tensor, limit: float, alpha: float = GLU_ALPHA,
-               shift: float = GLU_SHIFT, layout: Optional[torch.Tensor] = None, tickets: Optional[torch.Tensor] = None) -> torch.Tensor:
+               shift: float = GLU_SHIFT, layout: Optional[torch.Tensor] = None, tickets: Optional[StepTickets] = None) -> torch.Tensor:
     """out = clamped GLU of the two halves of x [gate | up]^T: the activation is the product's epilogue where a streaming kernel or
     the tile kernel runs, one more launch behind the vendor GEMM otherwise.  layout: stream_layout(w_gate_up, glu=True)."""
     M, N, K = _check_xw(x, w_gate_up)

@@ -197,7 +197,7 @@ class LatentAttention:
     def new_cache(self, n_blocks: int, block_size: int) -> LatentKVCache:
         return LatentKVCache(n_blocks, block_size, self.c_pad, self.r_pad, self.w_in.dtype, self.w_in.device)
 
-    def forward(self, h: torch.Tensor, positions: torch.Tensor, cache: LatentKVCache, params: InputParameters, tickets: Optional[torch.Tensor] = None):
+    def forward(self, h: torch.Tensor, positions: torch.Tensor, cache: LatentKVCache, params: InputParameters, tickets: Optional[lk.StepTickets] = None):
         """h [rows, padded width] -> what the residual stream receives (a tensor or split-K slabs).  tickets: of the step (latent_kernels)."""
         a, T = self.args, h.size(0)
         proj = lk.linear(h, self.w_in, layout=self.l_in, tickets=tickets)
@@ -249,7 +249,7 @@ class ClampedGLU:
         self.w_down[:width, :ff] = w["down"].to(device=device, dtype=dtype)
         lk.lay_out([self], None if layouts else 0)
 
-    def forward(self, h: torch.Tensor, tickets: Optional[torch.Tensor] = None):
+    def forward(self, h: torch.Tensor, tickets: Optional[lk.StepTickets] = None):
         act = h.new_empty(h.size(0), self.w_down.size(1))
         lk.linear_glu(h, self.w_gate_up, act, self.limit, self.alpha, self.shift, self.l_gate_up, tickets)
         if h.size(0) <= lk.slab_rows(self.l_down):

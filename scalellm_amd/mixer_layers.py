@@ -29,7 +29,7 @@ def single_rows(params: InputParameters, rows: int) -> int:
     return rows
 
 
-def out_product(x: torch.Tensor, w: torch.Tensor, layout: Optional[torch.Tensor] = None, tickets: Optional[torch.Tensor] = None):
+def out_product(x: torch.Tensor, w: torch.Tensor, layout: Optional[torch.Tensor] = None, tickets: Optional[lk.StepTickets] = None):
     """What the residual stream receives: split-K slabs for few rows, a tensor otherwise.  layout: lk.stream_layout(w), tickets: lk.step_tickets()."""
     return lk.linear_slabs(x, w, layout) if x.size(0) <= lk.slab_rows(layout) else lk.linear(x, w, tickets=tickets)
 
@@ -218,7 +218,7 @@ class ParallelMixer:
     def new_cache(self, limits):
         return self.left.new_cache(limits), self.right.new_state(limits)
 
-    def forward(self, h: torch.Tensor, positions: torch.Tensor, cache, params: InputParameters, tickets: Optional[torch.Tensor] = None):
+    def forward(self, h: torch.Tensor, positions: torch.Tensor, cache, params: InputParameters, tickets: Optional[lk.StepTickets] = None):
         proj = lk.linear(h, self.w_in, layout=self.l_in, tickets=tickets)
         out = proj.new_empty(h.size(0), self.o_k)
         self.left.forward(proj[:, :self.split], positions, cache[0], params, out[:, :self.left.out_width])
@@ -278,7 +278,7 @@ class ChannelDelta:
         s = self.spec
         return RecurrentState(limits.n_states, s.heads, s.dim_pad, s.v_pad, self.device, s.taps, s.channels, self.dtype)
 
-    def forward(self, h: torch.Tensor, positions: torch.Tensor, state: RecurrentState, params: InputParameters, tickets: Optional[torch.Tensor] = None):
+    def forward(self, h: torch.Tensor, positions: torch.Tensor, state: RecurrentState, params: InputParameters, tickets: Optional[lk.StepTickets] = None):
         s, T = self.spec, h.size(0)
         n = single_rows(params, T)
         proj = lk.linear(h, self.w_in, layout=self.l_in, tickets=tickets)

@@ -189,11 +189,11 @@ class VebusunStep:
         c, T = self.config, tokens.numel()
         resid = torch.empty(T, c.width, dtype=torch.float32, device=self.device)
         h = torch.empty(T, self.k_width, dtype=self.dtype, device=self.device)
-        tickets = lk.step_tickets(T, self.device)
+        tickets = lk.step_tickets(T, 8 * len(self.layers), self.device)   # (at most 7 products a layer)
         n = len(self.layers)
         # (None: the last sum's launch norms them too -- not where somebody sees, and may change, the stream behind it)
         rows = lk.wanted_rows(params, T if n and self.on_layer is None else 0)
-        lk.residual_norm(resid, h, self.layers[0].norm1 if n else None, c.eps, embed=(tokens, self.embed, None, None), mult=c.embedding_scale, clear=tickets)
+        lk.residual_norm(resid, h, self.layers[0].norm1 if n else None, c.eps, embed=(tokens, self.embed, None, None), mult=c.embedding_scale, clear=None if tickets is None else tickets.words)
         for i, L in enumerate(self.layers):
             nxt = self.layers[i + 1].norm1 if i + 1 < n else self.final_norm if rows is None else None
             delta = L.mixer.forward(h, positions, self.caches[i], params, tickets)

@@ -188,7 +188,7 @@ def test_products_cut_in_k_and_joined(M, N, K, n):
     # one rounding to bf16 (2^-9) of sums whose 32-bit error is far below it
     assert (np.abs(_f64(outs[0]) - want) - np.abs(want) * 2.0 ** -8).max() < 2e-5 * K ** 0.5
     assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
-    got = lk.linear(x, w, layout=layout, tickets=tickets)   # (as many as pay, or none)
+    got = lk.linear(x, w, layout=layout, tickets=lk.StepTickets(tickets))   # (as many as pay, or none)
     assert (np.abs(_f64(got) - want) - np.abs(want) * 2.0 ** -8).max() < 2e-5 * K ** 0.5 and int(tickets.abs().max()) == 0
 
 
@@ -196,7 +196,7 @@ def test_joined_products_in_a_graph():
     lk = _lk()
     M, N, K = 100, 3664, 2048
     x, w = _rnd(1, M, K, dtype=torch.bfloat16), _rnd(2, N, K, dtype=torch.bfloat16)
-    layout, tickets = lk.stream_layout(w), torch.zeros(512, dtype=torch.int32, device="cuda")
+    layout, tickets = lk.stream_layout(w), lk.StepTickets(torch.zeros(512, dtype=torch.int32, device="cuda"))
     assert lk.join_count(N, K, M) > 1
     lk.linear(x, w, layout=layout, tickets=tickets)
     torch.cuda.synchronize()
@@ -281,25 +281,32 @@ def test_tiled_products_of_several_rounds(M, N, K, slices, tile):
     test_tiled_products(M, N, K, slices, tile)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("M,N,K,slices,glu", [(257, 96, 1088, 5, False), (300, 544, 704, 3, True), (1100, 16416, 704, 2, False), (207, 4096, 2048, 0, False)])
-def test_tiled_products_with_counters_of_the_callers(M, N, K, slices, glu):
-    """The same bits as with counters of the launch's own, which are zero again behind it; eagerly and in a graph."""
+def test_tiled_products_with_counters_of_the_callers(M, N, K, slices, glu, dtype):
+    """The same bits as with counters of the launch's own; eagerly and in a graph."""
     lk = _lk()
-    x, w = _rnd(1, M, K, dtype=torch.bfloat16), _rnd(2, N, K, dtype=torch.bfloat16, std=K ** -0.5)
+    x, w = _rnd(1, M, K, dtype=dtype), _rnd(2, N, K, dtype=dtype, std=K ** -0.5)
     how = dict(glu=(7.0, 1.0, 0.0) if glu else None, slices=slices)
-    want, got = (torch.zeros(M, N // 2 if glu else N, dtype=torch.bfloat16, device="cuda") for _ in range(2))
-    tickets = torch.zeros(512, dtype=torch.int32, device="cuda")
-    assert lk._gemm(x, w, want, **how) and lk._gemm(x, w, got, tickets=tickets, **how)
-    assert torch.equal(want, got) and int(tickets.abs().max()) == 0
+    want, got = (torch.zeros(M, N // 2 if glu else N, dtype=dtype, device="cuda") for _ in range(2))
+    words = torch.zeros(512 + 3 * 256, dtype=torch.int32, device="cuda")
+    tickets = lk.StepTickets(words)
+    assert lk._gemm(x, w, want, **how)
+    for _ in range(4):   # (the last one finds none left)
+        got.zero_()
+        assert lk._gemm(x, w, got, tickets=tickets, **how) and torch.equal(want, got)
+    assert int(words[:512].abs().max()) == 0 and bool((words.view(-1, 256)[2:] == words[512:768]).all())
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
+        words.zero_()
+        tickets = lk.StepTickets(words)
         for _ in range(2):
             lk._gemm(x, w, got, tickets=tickets, **how)
     for i in range(3):
-        x.copy_(_rnd(3 + i, M, K, dtype=torch.bfloat16))
+        x.copy_(_rnd(3 + i, M, K, dtype=dtype))
         graph.replay()
         lk._gemm(x, w, want, **how)
-        assert torch.equal(want, got) and int(tickets.abs().max()) == 0
+        assert torch.equal(want, got)
 
 
 @pytest.mark.parametrize("M", [129, 700])
