@@ -25,8 +25,8 @@
 // 5692 x 4096 x 14336 737 / 490, 5692 x 4096 x 4096 148 / 145, 3226 x 28672 x 4096 GLU 703 / 559, 3226 x 16896 x 4096 441 / 350, 4096 x 16384 x 2048 GLU
 // 226 / 206, 4096 x 8512 x 2048 152 / 115, 1000 x 4096 x 14336 131 / 108, 600 x 28672 x 4096 GLU 147 / 132, 300 x 4096 x 14336 72 / 64,
 // 207 x 16384 x 2048 GLU 30 / 22.  Behind the vendor product where its tiles fill whole rounds (8192^3 678 / 718, 4096^3 89 / 94), with one row of tiles
-// over large weights (129 x 28672 x 4096 GLU 59 / 74), and on short and narrow products (207 x 4096 x 4096 17.5 / 20.6, 207 x 3664 x 2048 11.1 / 14.9,
-// 207 x 512 x 2048 8.5 / 15.8), which its callers take here for the sake of the host.
+// over large weights (129 x 28672 x 4096 GLU 59 / 74), and on short and narrow products (weights out of memory: 197 x 2048 x 2048 11.8 / 13.7, 284 x 3664 x
+// 2048 15.3 / 16.0; but 197 x 4096 x 4096 22.2 / 20.3, 197 x 4096 x 14336 56 / 45), which its callers take here for the sake of the host.
 #include <type_traits>
 
 #include "latent_common.h"
@@ -258,7 +258,7 @@ struct GemmTile {
 };
 constexpr GemmTile GEMM_TILES[] = {{256, 256, 0.914f, 1.386f, 8.6f}, {256, 128, 0.521f, 0.778f, 5.0f}, {128, 128, 0.311f, 0.488f, 3.4f}, {128, 256, 0.542f, 0.800f, 5.3f},
                                    {256, 192, 0.725f, 1.037f, 6.6f}, {192, 256, 0.743f, 1.071f, 6.6f}, {160, 256, 0.647f, 0.909f, 6.1f}};
-constexpr int GEMM_N_TILES = sizeof(GEMM_TILES) / sizeof(GEMM_TILES[0]), GEMM_256_192 = 4;   // (that one has no GLU)
+constexpr int GEMM_N_TILES = sizeof(GEMM_TILES) / sizeof(GEMM_TILES[0]), GEMM_128_128 = 2, GEMM_256_192 = 4;   // (the last has no GLU)
 constexpr int GEMM_CUS = 256;
 static_assert(SLM_GEMM_COUNTERS >= GEMM_CUS, "a counter for each tile of a round");
 constexpr float GEMM_CUT = 6.f, GEMM_SLABS = 3.5e6f;   // us of cutting tiles, bytes of their slabs that take one more
@@ -300,6 +300,20 @@ static GemmPlan gemm_plan_of(const slm_linear_args& a, int tile, int slices) {
   else if (left) p.us += round(left, steps);
   return p;
 }
+// Slices of a product whose tiles of 128 x 128 leave the chip's one round partly empty.  Its weights come from memory, for which a step is 0.42 to 0.52 us
+// whatever the tile does (the constants above are of products that wait for their operands less); joining s slices is 2.4 + 1.15 s: the last one
+// reads s tiles of 64 KB one after the other.  us, 197 rows, slices 1 / 2 / 3 / 4 / 6 / 8: 2048 x 2048 18.7 / 15.2 / 13.9 / 13.7 / 14.9 / 16.5, 2048 x 8192 60.0 /
+// 39.0 / 30.2 / 26.5 / 23.7 / 25.2, 4096 x 14336 (1 to 4) 114 / 68 / 53 / 45, 3664 x 2048 18.9 / 15.7 / 14.9 / 15.2, 6752 x 4096 35.3 / 27.2; 512 rows, 4096 x
+// 4096 37.4 / 27.6; 4096 x 512 6.9 / 9.9.
+static int gemm_few_tiles(int tiles, int steps) {
+  int best = 1;
+  float least = 0.f;
+  for (int s = 1; s <= 8 && (s == 1 || (tiles * s <= GEMM_CUS && steps / s >= 4)); ++s) {
+    const float us = (float)((steps + s - 1) / s) * (0.42f + 0.1f * (float)(tiles * s) / GEMM_CUS) + (s > 1 ? 2.4f + 1.15f * (float)s : 0.f);
+    if (s == 1 || us < least) best = s, least = us;
+  }
+  return best;
+}
 // tile -1: the one that takes least; slices 0: as many as pay, 1: none
 static GemmPlan gemm_plan(const slm_linear_args& a, int tile, int slices) {
   if (tile >= 0) return gemm_plan_of(a, tile, slices);
@@ -311,6 +325,8 @@ static GemmPlan gemm_plan(const slm_linear_args& a, int tile, int slices) {
       if (best.us == 0.f || p.us < best.us) best = p;
     }
   }
+  if (slices <= 0 && best.tile == GEMM_128_128 && best.mb * best.nb < GEMM_CUS)
+    best = gemm_plan_of(a, GEMM_128_128, gemm_few_tiles(best.mb * best.nb, (int)(a.K >> 6)));
   return best;
 }
 
