@@ -169,6 +169,58 @@ __global__ void __launch_bounds__(256) linear_append_kernel(const slm_linear_arg
   if (row < c.rows) latent_append_row<bf16, 4>(c, row);
 }
 
+// The same where K is one head's queries and more than 32 rows come: a wave takes 64 rows x 32 columns and all of K, so that nothing meets in LDS, and a
+// lane ends with eight neighbouring columns, one store of 16 bytes where linear_block has eight of two.  Row i of operand t is column 8 (i / 4) + i % 4 + 4 t;
+// the order of k and of the sums is linear_block's: the same bits.
+// Bound: the stores (128 rows of 32 heads: 4.7 MB).  us, linear_block / this: 32 heads of 128 -> 512 columns 48 rows 5.0 / 4.0, 128 rows 7.8 / 5.4; 16 heads
+// 64 rows 4.0 / 4.1, 128 rows 5.1 / 4.3; 32 heads -> 256 128 rows 5.1 / 4.3; but 16 heads -> 128 128 rows 3.8 / 4.0.
+template <int KS>   // K / 64
+__global__ void __launch_bounds__(256) linear_append_heads_kernel(const slm_linear_args a, const slm_latent_append_args c, const int slices) {
+  if ((int)blockIdx.z < slices) {
+    const int64_t row = ((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
+    if (row < c.rows) latent_append_row<bf16, 4>(c, row);
+    return;
+  }
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, g = lane >> 4;
+  const int64_t item = blockIdx.z - slices, n0 = (int64_t)blockIdx.x * 128 + wave * 32, m0 = (int64_t)blockIdx.y * 64;
+  const bf16* w = reinterpret_cast<const bf16*>(a.w) + item * a.w_batch + (n0 + 8 * (r16 >> 2) + (r16 & 3)) * a.ldw + 16 * g;
+  const bf16* x = reinterpret_cast<const bf16*>(a.x) + item * a.x_batch + 16 * g;
+  KStep<bf16> wf[2][KS], xf[4][KS];
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int s = 0; s < KS; ++s) wf[t][s].load(w + 4 * t * a.ldw + 64 * s);
+#pragma unroll
+  for (int m = 0; m < 4; ++m)
+#pragma unroll
+    for (int s = 0; s < KS; ++s) xf[m][s].load(x + min(m0 + 16 * m + r16, a.M - 1) * a.ldx + 64 * s);
+#pragma unroll
+  for (int m = 0; m < 4; ++m) {
+    f32x4 y[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      y[t] = KStep<bf16>::mma(wf[t][0], xf[m][0], f32x4{0.f, 0.f, 0.f, 0.f});
+      if constexpr (KS == 2) y[t] += KStep<bf16>::mma(wf[t][1], xf[m][1], f32x4{0.f, 0.f, 0.f, 0.f});
+    }
+    const int64_t row = m0 + 16 * m + r16;
+    if (row < a.M)
+      *reinterpret_cast<u32x4*>(reinterpret_cast<bf16*>(a.y) + item * a.y_batch + row * a.ldy + n0 + 8 * g) =
+          u32x4{pack2<bf16_tag>(y[0][0], y[0][1]), pack2<bf16_tag>(y[0][2], y[0][3]), pack2<bf16_tag>(y[1][0], y[1][1]), pack2<bf16_tag>(y[1][2], y[1][3])};
+  }
+}
+static bool append_heads_ok(const slm_linear_args& a) {
+  return a.M > 32 && (a.K == 64 || a.K == 128) && a.N % 128 == 0 && a.ldy % 8 == 0 && a.y_batch % 8 == 0 && aligned16(a.y) && a.M <= 256 && a.N * a.batch >= 8192;
+}
+static int append_heads_launch(const slm_linear_args& a, const slm_latent_append_args& c, hipStream_t st) {
+  const int64_t gx = a.N / 128, gy = (a.M + 63) / 64, slices = (c.rows + gx * gy - 1) / (gx * gy);
+  if (a.batch + slices > 65535) return SLM_ERR_UNSUPPORTED;
+  const dim3 grid((unsigned)gx, (unsigned)gy, (unsigned)(a.batch + slices));
+  hip_clear_error();
+  if (a.K == 64) linear_append_heads_kernel<1><<<grid, dim3(256), 0, st>>>(a, c, (int)slices);
+  else linear_append_heads_kernel<2><<<grid, dim3(256), 0, st>>>(a, c, (int)slices);
+  return hip_check_launch();
+}
+
 template <typename E, int MT, int NT, int U, int EPI>
 static int lin_launch(const slm_linear_args& a, hipStream_t st, const slm_latent_append_args* c) {
   constexpr int NOUT = EPI == SLM_LIN_GLU ? NT / 2 : NT;
@@ -253,7 +305,7 @@ extern "C" SLM_API int slm_latent_append_absorb(const slm_latent_append_args* c,
   const bool apart = a->x == c->proj && a->ldx == c->ld_proj && a->K <= c->q_dim && a->x_batch == c->q_dim + c->q_rot && a->batch <= c->heads &&
                      c->q_abs && a->y == c->q_abs && a->N <= c->c_pad && a->y_batch == c->c_pad + c->r_pad && a->M <= c->abs_rows;
   if (apart && a->M > 0 && c->rows <= 256 && a->dtype == SLM_BF16 && latent_append_by_four(*c))
-    return lin_shape<bf16, SLM_LIN_STORE>(*a, (hipStream_t)stream, c);
+    return append_heads_ok(*a) ? append_heads_launch(*a, *c, (hipStream_t)stream) : lin_shape<bf16, SLM_LIN_STORE>(*a, (hipStream_t)stream, c);
   const int rd = slm_latent_append(c, stream);
   return rd != SLM_OK ? rd : slm_linear(a, stream);
 }

@@ -503,6 +503,12 @@ def test_append_with_absorbed_queries(heads, q_dim, rot, rank, rows, absorbed):
         assert torch.equal(g.view(torch.int16), x.view(torch.int16))
 
 
+@pytest.mark.parametrize("heads,q_dim,rot,rank", [(16, 128, 64, 512), (40, 64, 16, 250), (64, 128, 32, 128)])
+@pytest.mark.parametrize("rows,absorbed", [(33, 33), (64, 64), (70, 65), (128, 127), (256, 256)])
+def test_append_with_absorbed_queries_of_many_heads(heads, q_dim, rot, rank, rows, absorbed):
+    test_append_with_absorbed_queries(heads, q_dim, rot, rank, rows, absorbed)
+
+
 # ---- attention over the cache ------------------------------------------------------------------
 class Paged:
     """Sequences of the given lengths on shuffled blocks, cache rows random (or given)."""
