@@ -117,9 +117,13 @@ __device__ __forceinline__ bool stream_join(f32x4 (&acc)[F], const StreamJoin& j
   return true;
 }
 
+struct NoJoin {};
+template <bool JOIN>
+using JoinArgs = std::conditional_t<JOIN, StreamJoin, NoJoin>;
+
 // JOIN: by stream_join, one row of tiles
 template <typename E, int MT, int NT, int D, int EPI, bool JOIN>
-__global__ void __launch_bounds__(256) linear_wave_k_kernel(const slm_linear_args a, const StreamJoin j) {
+__global__ void __launch_bounds__(256) linear_wave_k_kernel(const slm_linear_args a, const JoinArgs<JOIN> j) {
   constexpr bool GLU = EPI == SLM_LIN_GLU;
   static_assert(!JOIN || (EPI == SLM_LIN_STORE && NT * MT == 4), "a tile a wave");
   static_assert(!GLU || NT % 2 == 0, "gate / up pairs");
@@ -217,7 +221,7 @@ __global__ void __launch_bounds__(256) linear_wave_k_kernel(const slm_linear_arg
 }
 
 template <typename E, int MT, int NT, int WK, int D, int EPI, bool JOIN>
-__global__ void __launch_bounds__(256 * WK) linear_wave_n_kernel(const slm_linear_args a, const StreamJoin j) {
+__global__ void __launch_bounds__(256 * WK) linear_wave_n_kernel(const slm_linear_args a, const JoinArgs<JOIN> j) {
   constexpr bool GLU = EPI == SLM_LIN_GLU;
   static_assert(!JOIN || EPI == SLM_LIN_STORE, "joined products are stored");
   constexpr int GROUP = MT * 16 * 128;    // bytes of a group's step of x in LDS: 16-byte chunk c of row r lies in slot c ^ (r & 7)
@@ -395,7 +399,7 @@ static int wave_k_launch(const slm_linear_args& a, hipStream_t st, const StreamJ
       return hip_check_launch();
     }
   }
-  linear_wave_k_kernel<E, MT, NT, D, EPI, false><<<grid, dim3(256), 0, st>>>(a, StreamJoin{});
+  linear_wave_k_kernel<E, MT, NT, D, EPI, false><<<grid, dim3(256), 0, st>>>(a, NoJoin{});
   return hip_check_launch();
 }
 template <typename E, int MT, int NT, int WK, int D, int EPI>
@@ -407,7 +411,7 @@ static int wave_n_launch(const slm_linear_args& a, hipStream_t st, const StreamJ
       return hip_check_launch();
     }
   }
-  linear_wave_n_kernel<E, MT, NT, WK, D, EPI, false><<<grid, dim3(256 * WK), 0, st>>>(a, StreamJoin{});
+  linear_wave_n_kernel<E, MT, NT, WK, D, EPI, false><<<grid, dim3(256 * WK), 0, st>>>(a, NoJoin{});
   return hip_check_launch();
 }
 

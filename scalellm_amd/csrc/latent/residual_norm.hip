@@ -33,9 +33,11 @@ __global__ void __launch_bounds__(T) residual_norm_kernel(const slm_residual_nor
   const int tid = threadIdx.x;
   const int64_t row = blockIdx.x;
   const int width = (int)a.width;
-  if constexpr (MODE == SLM_RN_EMBED) {   // (somebody's counters: a launch less)
-    for (int64_t i = row * T + tid; i < a.n_clear; i += a.rows * T) a.clear[i] = 0;
-  }
+  auto clear = [&]() {   // (somebody's counters: a launch less.  Last: a store in front of the loads is waited for with them)
+    if constexpr (MODE == SLM_RN_EMBED) {
+      for (int64_t i = row * T + tid; i < a.n_clear; i += a.rows * T) a.clear[i] = 0;
+    }
+  };
   const int64_t src_row = (MODE == SLM_RN_PLAIN && a.row_index) ? a.row_index[row] + a.row_shift : row;
   float* r = a.resid + src_row * a.width;
   const E* e0 = nullptr;
@@ -96,7 +98,7 @@ __global__ void __launch_bounds__(T) residual_norm_kernel(const slm_residual_nor
       for (int j = 0; j < V; ++j) ss = __builtin_fmaf(x[s][j], x[s][j], ss);
     }
   }
-  if (!a.weight) return;  // (uniform: only the sum was asked for)
+  if (!a.weight) return clear();  // (uniform: only the sum was asked for)
   const bool rms = a.norm == SLM_NORM_RMS;
   const float rs = rms ? 1.0f / sqrtf(row_sum<T>(ss, red) / (float)width + a.eps) : 0.f;
   E* o = reinterpret_cast<E*>(a.out) + row * a.ld_out;
@@ -118,6 +120,7 @@ __global__ void __launch_bounds__(T) residual_norm_kernel(const slm_residual_nor
     }
   }
   for (int i = width + tid; i < (int)a.ld_out; i += RN_THREADS) o[i] = (E)0.f;
+  clear();
 }
 
 // V columns a thread: 8 where every row lies on 16 bytes, else 4.  5692 rows of 14336: 107 us -> 97 (490 MB; a 64-bit division a thread before).

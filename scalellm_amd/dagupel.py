@@ -162,7 +162,7 @@ class DagupelStep:
         c, T = self.config, tokens.numel()
         resid = torch.empty(T, c.width, dtype=torch.float32, device=self.device)
         h = torch.empty(T, self.k_width, dtype=self.dtype, device=self.device)
-        tickets = lk.step_tickets(T, 8 * len(self.layers), self.device)   # (at most 7 products a layer)
+        tickets = lk.step_tickets(T, self.k_width, 8 * len(self.layers), self.device)   # (at most 7 products a layer)
         first = self.layers[0].norm1 if self.layers else None
         lk.residual_norm(resid, h, first, c.eps, embed=(tokens, self.table, positions, self.pos_table), clear=None if tickets is None else tickets.words)
         n = len(self.layers)

@@ -273,9 +273,9 @@ class StepTickets:
         return self.words[at:self.at] if self.at <= self.words.numel() else None
 
 
-def step_tickets(rows: int, products: int, device) -> Optional[StepTickets]:
-    """For a step of so many rows and at most so many tile products (None: nothing is cut)."""
-    if rows <= 16:
+def step_tickets(rows: int, width: int, products: int, device) -> Optional[StepTickets]:
+    """For a step of so many rows of a stream of that width and at most so many tile products (None: nothing is cut)."""
+    if rows <= 16 or (rows <= STREAM_MAX_ROWS and width < 4096):   # (join_count)
         return None
     n = 0 if rows < TILE_MIN_ROWS else min(products, 240)
     return StepTickets(torch.empty(_lib.STREAM_TICKETS + n * _lib.GEMM_COUNTERS, dtype=torch.int32, device=device))

@@ -189,7 +189,7 @@ class VebusunStep:
         c, T = self.config, tokens.numel()
         resid = torch.empty(T, c.width, dtype=torch.float32, device=self.device)
         h = torch.empty(T, self.k_width, dtype=self.dtype, device=self.device)
-        tickets = lk.step_tickets(T, 8 * len(self.layers), self.device)   # (at most 7 products a layer)
+        tickets = lk.step_tickets(T, self.k_width, 8 * len(self.layers), self.device)   # (at most 7 products a layer)
         n = len(self.layers)
         # (None: the last sum's launch norms them too -- not where somebody sees, and may change, the stream behind it)
         rows = lk.wanted_rows(params, T if n and self.on_layer is None else 0)
