@@ -688,12 +688,15 @@ struct AttnPlan {
   // balanced pure-decode partition (AttnKParams::bal): partial slots per (token, head) and the
   // piece-size floor that keeps a sequence's pieces within them
   int bal, part_slots, bal_qmin;
+  int slots_least;  // partial slots that scratch has to hold (part_slots: where it holds them)
   // the one-wave tile class of a mixed call whose other rows are not split: its KV splits (1: none either) and its longest
   // sequence, whose tokens have a row of partials each (AttnKParams::part_rows)
   int small_splits, small_rows;
   bool singles_on_tile;  // q_len = 1 sequences go to the one-wave tiles
 };
 constexpr int ATTN_BAL_ALIGN = 64;
+// shortest piece that keeps a sequence's pieces within the slots
+static int bal_piece(int64_t max_kv_len, int slots) { return (int)std::max<int64_t>((max_kv_len + slots - 2) / (slots - 1), 1); }
 
 // q_len = 1 sequences on the MFMA tile kernel?  With a wide GQA group the token kernel's VALU work
 // per KV byte (one dot-product / P.V chain per query head) is what bounds it -- G = 8: 4.4-5.3 TB/s
@@ -900,7 +903,7 @@ static int plan_attn(const slm_attn_args* a, AttnPlan* pl) {
   // combine launch exits.  Not with a caller-forced split count (tests pin the classic form),
   // not with a sliding window (the visible range is no longer a prefix sum).
   pl->bal = 0;
-  pl->part_slots = n_splits;
+  pl->part_slots = pl->slots_least = n_splits;
   pl->bal_qmin = 1;
   // Measured (profiles/r03_attn_serving.jsonl, classic -> balanced): bs = 256 ragged 5.80 -> 6.43 TB/s,
   // uniform 6.91 -> 6.85 (the combine launch that only exits); bs = 32 ragged 5.07 -> 5.37, uniform
@@ -930,9 +933,13 @@ static int plan_attn(const slm_attn_args* a, AttnPlan* pl) {
     int slots = n_splits + 1 > 9 ? n_splits + 1 : 9;
     if (slots > COMBINE_MAX_SPLITS) slots = COMBINE_MAX_SPLITS;
     pl->bal = 1;
-    pl->part_slots = slots;
-    const int64_t qmin = (a->max_kv_len + slots - 2) / (slots - 1);
-    pl->bal_qmin = (int)(qmin > 1 ? qmin : 1);
+    // The hint is a bound (of a captured graph: the longest context it serves), and pieces of an eighth of it leave most of the chip idle where histories
+    // are short: 32 pieces, as long as their scratch is small (32 sequences under a bound of 4096, 32 / 8 heads, us, 8 / 32 pieces: 300 keys 42.4 /
+    // 21.4, 1000 44.4 / 35.3, 2500 61.6 / 61.7, 4096 90.1 / 89.5).
+    const int64_t row_bytes = (int64_t)a->n_tokens * a->n_heads * (a->head_dim + 2) * 4;
+    pl->slots_least = slots;
+    pl->part_slots = slots < 33 && 33 * row_bytes <= (256ll << 20) ? 33 : slots;
+    pl->bal_qmin = bal_piece(a->max_kv_len, pl->part_slots);
     if (pl->n_splits >= slots) pl->n_splits = slots - 1;  // P = n_tokens * n_splits workgroups per head group
   }
   // A mixed call whose prompts need no split: the one-wave tiles have their own count, a wave for every SIMD as above.  Their
@@ -1058,6 +1065,7 @@ SLM_API size_t slm_paged_kv_varlen_mha_workspace_bytes(const slm_attn_args* a) {
 SLM_API size_t slm_paged_kv_varlen_mha_workspace_required(const slm_attn_args* a) {
   AttnPlan pl;
   if (plan_attn(a, &pl) != SLM_OK) return 0;
+  pl.part_slots = pl.slots_least;
   return pl.n_splits > 1 || pl.bal ? part_bytes(a, pl) : 0;
 }
 
@@ -1079,6 +1087,10 @@ SLM_API int slm_paged_kv_varlen_mha(const slm_attn_args* a, void* stream) {
       return SLM_ERR_ALIGNMENT;
 
   if (a->phase < 0 || a->phase > 2) return SLM_ERR_INVALID_ARG;
+  if (pl.bal && pl.part_slots > pl.slots_least && (!a->workspace || a->workspace_bytes < part_bytes(a, pl))) {   // (fewer, longer pieces)
+    pl.part_slots = pl.slots_least;
+    pl.bal_qmin = bal_piece(a->max_kv_len, pl.part_slots);
+  }
   const bool do_stream = a->phase != 2, do_combine = a->phase != 1;
   AttnKParams kp;
   kp.out = a->out; kp.q = a->query; kp.kc = a->key_cache; kp.vc = a->value_cache;
