@@ -621,6 +621,12 @@ static int la_splits(const slm_latent_attn_args& a) {
   const int per_cu = a.c_pad > 64 ? 1 : 2;
   int64_t n = 256 * per_cu / (wgs > 0 ? wgs : 1);
   if (n > tiles) n = tiles;
+  // Four tiles a split at least, above 32 (64 for one workgroup a split and for narrow latents): the key count is a bound, of a captured graph that of its
+  // longest context, and what merges the splits reads those without a key too.  Bound 4096, as many as go / this, us, 300, 1000, 2500, 4096 keys: latent 512, 16
+  // heads 1 row 14.5 / 13.2, 15.3 / 13.6, 15.9 / 15.2, 16.1 / 15.4; 2 rows 17.8 / 13.6, 17.8 / 13.7, 18.3 / 16.0, 18.9 / 17.2; 32 heads 1 row 17.9 / 14.0, 17.9 / 14.0, 18.0 /
+  // 16.1, 18.3 / 17.1; 256, 16 heads 2 rows 12.8 / 11.8, 12.8 / 11.8, -, 14.4 / 13.7.
+  const int64_t enough = std::max<int64_t>(a.c_pad >= 512 && wgs > 1 ? 32 : 64, tiles / 4);
+  if (n > enough) n = enough;
   if (n > LA_MAX_SPLITS) n = LA_MAX_SPLITS;
   return n < 1 ? 1 : (int)n;
 }
@@ -634,8 +640,9 @@ static void la_values_launch(const LatentAttnK& p, const slm_linear_args& v, int
   fn<<<dim3((unsigned)p.a.heads, (unsigned)((p.a.rows + rows_per - 1) / rows_per), (unsigned)((v.N + 127) / 128)), dim3(512), bytes, st>>>(p, v, rows_per);
 }
 // Rows of a head per workgroup, as many as leave one round of workgroups; 0: two launches.  Those where there are fewer than 128 pairs of row and head: one
-// row's 128 splits are then a quarter of a megabyte for each of few workgroups, where the merge by itself spreads them over the chip (1 row, 32 heads:
-// 9.4 us the two).  Of values wider than a workgroup's 128 columns several workgroups merge the same splits, which pays only where all of them are one
+// row's 64 or 128 splits are then up to a quarter of a megabyte for each of few workgroups, where the merge by itself spreads them over the chip -- but for the
+// widest latent's 32 splits and 32 pairs and more (with the attention, us, two launches / one: 32 heads 1 row of 300 keys 14.5 / 14.0, of 4096 17.6 / 17.1; 16 heads 4
+// rows 15.4 / 14.7, 19.3 / 18.5).  Of values wider than a workgroup's 128 columns several workgroups merge the same splits, which pays only where all of them are one
 // round (256 wide, us, two launches / one: 16 heads 8 rows of 1500 keys 17.9 / 16.5, 16 rows of 300 16.2 / 19.5; 32 heads 8 rows of 1500 20.7 / 23.8).
 static int la_values_rows(const LatentAttnK& p, const slm_linear_args& v) {
   const slm_latent_attn_args& a = p.a;
@@ -646,7 +653,8 @@ static int la_values_rows(const LatentAttnK& p, const slm_linear_args& v) {
   const int64_t r = std::min<int64_t>(16, (pairs + 255) / 256);
   const int64_t row_blocks = (a.rows + r - 1) / r;
   if (v.N > 128 && a.heads * row_blocks * ((v.N + 127) / 128) > 256) return 0;
-  return pairs >= 128 * r && r * p.n_splits <= LA_VALUES_WEIGHTS && row_blocks <= 65535 ? (int)r : 0;
+  const bool fill = pairs >= 128 * r || (a.c_pad >= 512 && pairs >= 32 && p.n_splits <= 32);
+  return fill && r * p.n_splits <= LA_VALUES_WEIGHTS && row_blocks <= 65535 ? (int)r : 0;
 }
 
 template <int KP, int RP, int MH>

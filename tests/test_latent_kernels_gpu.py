@@ -595,6 +595,13 @@ def test_latent_attention_with_its_values(c_pad, heads, vdim, rows, n_splits, on
         assert (got[:, :heads * (vdim + 4)].view(rows, heads, vdim + 4)[:, :, vdim:] == 7).all()
 
 
+# (few pairs of a row and a head, of the widest latent)
+@pytest.mark.parametrize("heads,vdim,rows,n_splits,one_launch", [(16, 128, 2, 0, True), (16, 128, 7, 32, True), (32, 128, 1, 20, True), (32, 128, 1, 33, False),
+                                                                 (31, 128, 1, 8, False), (32, 144, 1, 8, True)])
+def test_latent_attention_of_few_rows_with_its_values(heads, vdim, rows, n_splits, one_launch):
+    test_latent_attention_with_its_values(512, heads, vdim, rows, n_splits, one_launch)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_latent_attention_sees_exactly_its_window(dtype):
     """One key that outweighs all others: present at distance window - 1, gone at distance window."""
