@@ -9,7 +9,8 @@ A "step" is ONE decode step of a Llama-3-8B-shaped model over one synthetic batc
 sequences with 4096 tokens of paged KV history each (block_size 16, bf16 KV), all four linears
 int4 (AWQ, group 128) -- BASELINE.json's metric configuration.  Every op of the step is one of
 this repo's HIP kernels (RMSNorm, int4 GEMM, RoPE+KV-append, paged attention, SiLU*mul) except
-the lm_head product of more than 128 rows (below, it is streamed from a second layout) and the argmax (plain library ops).  The step is captured into a hipGraph and replayed, as the reference's ModelRunner does
+the lm_head GEMM and the argmax (plain library ops).  The step is captured into a hipGraph and
+replayed, as the reference's ModelRunner does
 (src/engine/model_runner.cpp:141-211).
 
 N > 1 runs the SAME global batch tensor-parallel over RCCL/xGMI (heads and GEMM N/K sharded,

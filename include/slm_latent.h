@@ -69,15 +69,13 @@ SLM_API int slm_linear(const slm_linear_args* a, void* stream);
 /* s of panel p holds row 64 p + 16 c + l % 16, k = 64 s + 32 h + 8 (l / 16) .. + 7.  GLU: N % 64 == 0    */
 /* and the rows are taken 16 of the gate, the same 16 of the up half, in turn.  ldw is not read.          */
 SLM_API int slm_linear_stream(const slm_linear_args* a, void* stream);
-/* The same in half precision (dtype SLM_F16), STORE                                                     */
-SLM_API int slm_linear_stream_half(const slm_linear_args* a, void* stream);
 /* A stored product cut in K by n_splits, joined in the launch: STORE, bf16, 17 to 128 rows, N <= 32 *     */
 /* SLM_STREAM_TICKETS, n_splits <= 16.  workspace: content does not matter; tickets [SLM_STREAM_TICKETS]    */
 /* are zero before and after (products of one stream may share them: slm_residual_norm_args::clear)         */
 #define SLM_STREAM_TICKETS 512
 SLM_API size_t slm_linear_stream_join_bytes(const slm_linear_args* a);
 SLM_API int slm_linear_stream_join(const slm_linear_args* a, void* workspace, size_t workspace_bytes, uint32_t* tickets, void* stream);
-/* lays contiguous w [N, K] of 16 bits out so: out holds ceil(N / 64) * 64 * K elements                   */
+/* lays contiguous w [N, K] bf16 out so: out holds ceil(N / 64) * 64 * K elements                         */
 SLM_API int slm_stream_layout(void* out, const void* w, int64_t N, int64_t K, int32_t glu, void* stream);
 /* The same for many rows in bf16, batch 1, STORE or GLU, rows of x, w and y on 16 bytes, x and w below 2 GB: tiles of  */
 /* up to 256 x 256.  tile: -1 or an index of the tiles (tests); slices: 0 as many as pay, n: the tiles of the   */

@@ -291,7 +291,6 @@ def latent_lib() -> C.CDLL:
         ("slm_residual_norm", C.c_int, [P(ResidualNormArgs), ptr]),
         ("slm_linear", C.c_int, [P(LinearArgs), ptr]),
         ("slm_linear_stream", C.c_int, [P(LinearArgs), ptr]),
-        ("slm_linear_stream_half", C.c_int, [P(LinearArgs), ptr]),
         ("slm_linear_stream_join_bytes", C.c_size_t, [P(LinearArgs)]),
         ("slm_linear_stream_join", C.c_int, [P(LinearArgs), ptr, C.c_size_t, ptr, ptr]),
         ("slm_gemm_workspace_bytes", C.c_size_t, [P(LinearArgs), i32, i32]),

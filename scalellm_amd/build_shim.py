@@ -3,7 +3,7 @@ surface) in-tree with g++ against the installed torch-ROCm headers.
 
     python -m scalellm_amd.build_shim [--force]
 
-Host code only -- the device code lives in libslm_hip.so and libslm_latent.so, which this links against.
+Host code only -- the device code lives in libslm_hip.so, which this links against.
 """
 from __future__ import annotations
 
@@ -28,7 +28,7 @@ def build(force: bool = False) -> str:
     slm_build.build()
     srcs = [os.path.join(SHIM, f) for f in ("slm_torch_shim.cpp", "slm_qlinear_hip.cpp", "slm_attn_handler_hip.cpp", "slm_llama_hip.cpp", "slm_shim_pybind.cpp")]
     deps = srcs + [os.path.join(SHIM, "slm_torch_shim.h"), os.path.join(SHIM, "slm_qlinear_hip.h"), os.path.join(SHIM, "slm_attn_handler_hip.h"), os.path.join(SHIM, "slm_llama_hip.h"),
-                   os.path.join(ROOT, "include", "slm_hip.h"), os.path.join(ROOT, "include", "slm_latent.h")]
+                   os.path.join(ROOT, "include", "slm_hip.h")]
     if not force and os.path.exists(OUT) and all(os.path.getmtime(OUT) > os.path.getmtime(d) for d in deps):
         return OUT
     tlib = ce.library_paths()[0]
@@ -40,7 +40,7 @@ def build(force: bool = False) -> str:
            "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
            "-DTORCH_EXTENSION_NAME=_slm_shim", *inc, *srcs, "-o", OUT, f"-L{tlib}", f"-L{CSRC}",
            "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-ltorch_hip", "-ltorch_python",
-           "-lrccl", "-lslm_hip", "-lslm_latent", f"-Wl,-rpath,{tlib}", "-Wl,-rpath,$ORIGIN"]
+           "-lrccl", "-lslm_hip", f"-Wl,-rpath,{tlib}", "-Wl,-rpath,$ORIGIN"]
     subprocess.check_call(cmd)
     print(f"[scalellm_amd.build_shim] built {OUT}")
     return OUT

@@ -1,4 +1,4 @@
-// linear_stream.hip -- y = x W^T in bf16 (only stored: in half precision too) for up to 128 rows (decode batches, sampled rows), from weights that were
+// linear_stream.hip -- y = x W^T in bf16 for up to 128 rows (decode batches, sampled rows), from weights that were
 // laid out for it at load.  Bound: the HBM stream of W; above 64 rows what a CU has under way of x and W together.
 //
 // Layout of W (slm_linear_stream): panels of 64 columns, in a panel steps of 64 k, in a step four blocks of 16 columns,
@@ -23,37 +23,33 @@
 // us at 28672 x 4096 (GLU) / 14336 -> 4096 (slabs) / 16384 x 2048, against the kernel of linear.hip, and above 32 rows the
 // vendor product: 1 row 37.7, 20.4, 12.8 (46, 27.6, 16.4); 16 rows 38.6, 20.7, 13.1 (67, 38, 22); 32 rows 36.2, 19.4, 12.6
 // (63, 41, 21); 64 rows 38.4, 22.7, 14.6 (57 + 5 for the GLU's launch, 42, 18); 96 rows 42.5, 26.2, 16.5 (55 with the launch, -, 22); 128 rows
-// 47.3, 29.8, 19.0 (59 with the launch, 78, 23).  Stored products of columns (a vocabulary's, bf16 and half alike), this / the vendor product of [K, N]:
-// 32768 x 4096 1 row 42 / 52, 32 rows 43 / 51, 128 rows 52 / 57; 128256 x 4096 157 / 190, 168 / 204, 231 / 244.
+// 47.3, 29.8, 19.0 (59 with the launch, 78, 23).
 #include <type_traits>
 
 #include "latent_common.h"
 
 namespace slm {
 
-struct StreamK {   // 64 k of a 16-row block: two operands of 16-bit values
-  u32x4 v[2];
+struct StreamK {   // 64 k of a 16-row block: two operands
+  bf16x8_t v[2];
 };
-template <typename E>
-__device__ __forceinline__ f32x4 stream_product(const u32x4& a, const u32x4& b, f32x4 c) {
-  if constexpr (std::is_same<E, bf16>::value)
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
+__device__ __forceinline__ f32x4 stream_mma(const StreamK& a, const StreamK& b, f32x4 c) {
+  c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.v[0], b.v[0], c, 0, 0, 0);
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.v[1], b.v[1], c, 0, 0, 0);
 }
 // (read once: past the caches' replacement, 10 % at 235 MB)
-__device__ __forceinline__ void stream_load_w(StreamK& d, const uint16_t* p) {
-  d.v[0] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
-  d.v[1] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p + 512));
+__device__ __forceinline__ void stream_load_w(StreamK& d, const bf16* p) {
+  d.v[0] = __builtin_bit_cast(bf16x8_t, __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p)));
+  d.v[1] = __builtin_bit_cast(bf16x8_t, __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p + 512)));
 }
 // this lane's first element of 16-column block nb
-__device__ __forceinline__ const uint16_t* stream_block(const slm_linear_args& a, int64_t nb, int lane) {
-  return reinterpret_cast<const uint16_t*>(a.w) + (nb >> 2) * 64 * a.K + (nb & 3) * 1024 + lane * 8;
+__device__ __forceinline__ const bf16* stream_block(const slm_linear_args& a, int64_t nb, int lane) {
+  return reinterpret_cast<const bf16*>(a.w) + (nb >> 2) * 64 * a.K + (nb & 3) * 1024 + lane * 8;
 }
 constexpr int64_t STREAM_STEP = 64 * 64;   // elements from one step of a panel to the next
 
 // Four columns of row m, or one output: y of the epilogue.  n: column of the product, for GLU of its output
-template <typename E, int EPI>
+template <int EPI>
 __device__ __forceinline__ void stream_store(const slm_linear_args& a, int split, int64_t m, int64_t n, f32x4 v, f32x4 up) {
   if constexpr (EPI == SLM_LIN_SLABS) {
     float* y = reinterpret_cast<float*>(a.y) + ((int64_t)split * a.M + m) * a.ldy + n;
@@ -64,13 +60,13 @@ __device__ __forceinline__ void stream_store(const slm_linear_args& a, int split
 #pragma unroll
     for (int j = 0; j < 4; ++j) y[j] = a.alpha * v[j];
   } else {
-    E* y = reinterpret_cast<E*>(a.y) + m * a.ldy + n;
+    bf16* y = reinterpret_cast<bf16*>(a.y) + m * a.ldy + n;
     if constexpr (EPI == SLM_LIN_GLU) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) v[j] = clamped_glu_f32(v[j], up[j], a.limit, a.glu_alpha, a.glu_shift);
     }
 #pragma unroll
-    for (int j = 0; j < 4; ++j) y[j] = (E)v[j];
+    for (int j = 0; j < 4; ++j) y[j] = (bf16)v[j];
   }
 }
 
@@ -122,7 +118,7 @@ template <bool JOIN>
 using JoinArgs = std::conditional_t<JOIN, StreamJoin, NoJoin>;
 
 // JOIN: by stream_join, one row of tiles
-template <typename E, int MT, int NT, int D, int EPI, bool JOIN>
+template <int MT, int NT, int D, int EPI, bool JOIN>
 __global__ void __launch_bounds__(256) linear_wave_k_kernel(const slm_linear_args a, const JoinArgs<JOIN> j) {
   constexpr bool GLU = EPI == SLM_LIN_GLU;
   static_assert(!JOIN || (EPI == SLM_LIN_STORE && NT * MT == 4), "a tile a wave");
@@ -132,12 +128,12 @@ __global__ void __launch_bounds__(256) linear_wave_k_kernel(const slm_linear_arg
   const int r16 = lane & 15, g = lane >> 4;
   const int split = blockIdx.z;
   const int64_t nb0 = (int64_t)blockIdx.x * NT, m0 = (int64_t)blockIdx.y * (16 * MT), blocks = a.N >> 4;
-  const uint16_t* wp[NT];
-  const uint16_t* xp[MT];
+  const bf16* wp[NT];
+  const bf16* xp[MT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) wp[t] = stream_block(a, min(nb0 + t, blocks - 1), lane);
 #pragma unroll
-  for (int t = 0; t < MT; ++t) xp[t] = reinterpret_cast<const uint16_t*>(a.x) + min(m0 + 16 * t + r16, a.M - 1) * a.ldx + 8 * g;
+  for (int t = 0; t < MT; ++t) xp[t] = reinterpret_cast<const bf16*>(a.x) + min(m0 + 16 * t + r16, a.M - 1) * a.ldx + 8 * g;
   f32x4 acc[NT][MT];
 #pragma unroll
   for (int t = 0; t < NT; ++t)
@@ -154,17 +150,15 @@ __global__ void __launch_bounds__(256) linear_wave_k_kernel(const slm_linear_arg
     for (int t = 0; t < NT; ++t) stream_load_w(w[u][t], wp[t] + s * STREAM_STEP);
 #pragma unroll
     for (int t = 0; t < MT; ++t) {
-      x[u][t].v[0] = *reinterpret_cast<const u32x4*>(xp[t] + (s << 6));
-      x[u][t].v[1] = *reinterpret_cast<const u32x4*>(xp[t] + (s << 6) + 32);
+      x[u][t].v[0] = *reinterpret_cast<const bf16x8_t*>(xp[t] + (s << 6));
+      x[u][t].v[1] = *reinterpret_cast<const bf16x8_t*>(xp[t] + (s << 6) + 32);
     }
   };
   auto multiply = [&](int u) {
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
-      for (int v = 0; v < MT; ++v)
-#pragma unroll
-        for (int h = 0; h < 2; ++h) acc[t][v] = stream_product<E>(w[u][t].v[h], x[u][v].v[h], acc[t][v]);
+      for (int v = 0; v < MT; ++v) acc[t][v] = stream_mma(w[u][t], x[u][v], acc[t][v]);
   };
   if (cnt >= D) {
 #pragma unroll
@@ -208,7 +202,7 @@ __global__ void __launch_bounds__(256) linear_wave_k_kernel(const slm_linear_arg
     f32x4 y[1] = {total(wave)};
     if (!stream_join(y, j, split, a.n_splits, tid, reinterpret_cast<uint32_t*>(red))) return;
     const int64_t nb = nb0 + wave / MT, m = m0 + 16 * (wave % MT) + r16;
-    if (nb < blocks && m < a.M) stream_store<E, EPI>(a, 0, m, nb * 16 + 4 * g, y[0], y[0]);
+    if (nb < blocks && m < a.M) stream_store<EPI>(a, 0, m, nb * 16 + 4 * g, y[0], y[0]);
     return;
   }
   for (int i = wave; i < TILES; i += 4) {
@@ -216,11 +210,11 @@ __global__ void __launch_bounds__(256) linear_wave_k_kernel(const slm_linear_arg
     const int64_t nb = nb0 + t, m = m0 + 16 * v + r16;
     if (nb >= blocks || m >= a.M) continue;
     const f32x4 y = total(t * MT + v);
-    stream_store<E, EPI>(a, split, m, stream_column<EPI>(nb) + 4 * g, y, GLU ? total((t + 1) * MT + v) : y);
+    stream_store<EPI>(a, split, m, stream_column<EPI>(nb) + 4 * g, y, GLU ? total((t + 1) * MT + v) : y);
   }
 }
 
-template <typename E, int MT, int NT, int WK, int D, int EPI, bool JOIN>
+template <int MT, int NT, int WK, int D, int EPI, bool JOIN>
 __global__ void __launch_bounds__(256 * WK) linear_wave_n_kernel(const slm_linear_args a, const JoinArgs<JOIN> j) {
   constexpr bool GLU = EPI == SLM_LIN_GLU;
   static_assert(!JOIN || EPI == SLM_LIN_STORE, "joined products are stored");
@@ -235,19 +229,19 @@ __global__ void __launch_bounds__(256 * WK) linear_wave_n_kernel(const slm_linea
   const int r16 = lane & 15, g = lane >> 4, wn = wave & 3, kg = wave >> 2;
   const int split = blockIdx.z;
   const int64_t nb0 = (int64_t)blockIdx.x * (4 * NT) + wn * NT, m0 = (int64_t)blockIdx.y * (16 * MT), blocks = a.N >> 4;
-  const uint16_t* wp[NT];
+  const bf16* wp[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) wp[t] = stream_block(a, min(nb0 + t, blocks - 1), lane);
   const int steps = (int)(a.K >> 6), per = (steps + a.n_splits - 1) / a.n_splits;
   const int s0 = split * per, s1 = min(steps, s0 + per), cnt = s1 - s0;
   const int its = (max(cnt, 0) + WK - 1) / WK;
-  const uint16_t* xp[XU];
+  const bf16* xp[XU];
   uint32_t xd[XU];
   int xk[XU];
 #pragma unroll
   for (int i = 0; i < XU; ++i) {
     const int u = tid + 256 * WK * i, r = u / (8 * WK), c = u % (8 * WK);
-    xp[i] = reinterpret_cast<const uint16_t*>(a.x) + min(m0 + r, a.M - 1) * a.ldx;
+    xp[i] = reinterpret_cast<const bf16*>(a.x) + min(m0 + r, a.M - 1) * a.ldx;
     xk[i] = 8 * c;
     xd[i] = c / 8 * GROUP + r * 128 + ((c ^ r) & 7) * 16;
   }
@@ -273,7 +267,7 @@ __global__ void __launch_bounds__(256 * WK) linear_wave_n_kernel(const slm_linea
   const int fragment[2] = {kg * GROUP + r16 * 128 + ((g ^ r16) & 7) * 16, kg * GROUP + r16 * 128 + (((4 + g) ^ r16) & 7) * 16};
   auto fetch = [&](int v, int buf) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h) f[v % (AHEAD + 1)].v[h] = *reinterpret_cast<const u32x4*>(lds + buf * XB + v * 2048 + fragment[h]);
+    for (int h = 0; h < 2; ++h) f[v % (AHEAD + 1)].v[h] = *reinterpret_cast<const bf16x8_t*>(lds + buf * XB + v * 2048 + fragment[h]);
   };
   // step i + u: its products; between them the next step's x is written, x of D steps on and w of D - 1 steps on are asked for
   auto step = [&](int u, int i, bool mine, bool more) {
@@ -299,7 +293,7 @@ __global__ void __launch_bounds__(256 * WK) linear_wave_n_kernel(const slm_linea
 #pragma unroll
         for (int h = 0; h < 2; ++h)
 #pragma unroll
-          for (int t = 0; t < NT; ++t) acc[t][v] = stream_product<E>(w[u][t].v[h], f[v % (AHEAD + 1)].v[h], acc[t][v]);
+          for (int t = 0; t < NT; ++t) acc[t][v] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[u][t].v[h], f[v % (AHEAD + 1)].v[h], acc[t][v], 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
@@ -381,7 +375,7 @@ __global__ void __launch_bounds__(256 * WK) linear_wave_n_kernel(const slm_linea
       f32x4 up = acc[t][v];
       if constexpr (GLU && NT == 1) up = part[((wn + 1) * MT + v) * 64 + lane];
       else if constexpr (GLU) up = acc[t + 1][v];
-      if (m < a.M) stream_store<E, EPI>(a, split, m, stream_column<EPI>(nb) + 4 * g, acc[t][v], up);
+      if (m < a.M) stream_store<EPI>(a, split, m, stream_column<EPI>(nb) + 4 * g, acc[t][v], up);
     }
   }
 }
@@ -390,28 +384,28 @@ __global__ void __launch_bounds__(256 * WK) linear_wave_n_kernel(const slm_linea
 static int64_t stream_tiles(const slm_linear_args& a, int per) { return (a.N / 16 + per - 1) / per; }
 
 // (one row of tiles: M <= 128, joined products)
-template <typename E, int MT, int NT, int D, int EPI>
+template <int MT, int NT, int D, int EPI>
 static int wave_k_launch(const slm_linear_args& a, hipStream_t st, const StreamJoin* j) {
   const dim3 grid((unsigned)stream_tiles(a, NT), (unsigned)((a.M + 16 * MT - 1) / (16 * MT)), (unsigned)a.n_splits);
-  if constexpr (std::is_same<E, bf16>::value && EPI == SLM_LIN_STORE && MT == 2) {
+  if constexpr (EPI == SLM_LIN_STORE && MT == 2) {
     if (j) {
-      linear_wave_k_kernel<E, MT, NT, D, EPI, true><<<grid, dim3(256), 0, st>>>(a, *j);
+      linear_wave_k_kernel<MT, NT, D, EPI, true><<<grid, dim3(256), 0, st>>>(a, *j);
       return hip_check_launch();
     }
   }
-  linear_wave_k_kernel<E, MT, NT, D, EPI, false><<<grid, dim3(256), 0, st>>>(a, NoJoin{});
+  linear_wave_k_kernel<MT, NT, D, EPI, false><<<grid, dim3(256), 0, st>>>(a, NoJoin{});
   return hip_check_launch();
 }
-template <typename E, int MT, int NT, int WK, int D, int EPI>
+template <int MT, int NT, int WK, int D, int EPI>
 static int wave_n_launch(const slm_linear_args& a, hipStream_t st, const StreamJoin* j) {
   const dim3 grid((unsigned)stream_tiles(a, 4 * NT), (unsigned)((a.M + 16 * MT - 1) / (16 * MT)), (unsigned)a.n_splits);
-  if constexpr (std::is_same<E, bf16>::value && EPI == SLM_LIN_STORE) {
+  if constexpr (EPI == SLM_LIN_STORE) {
     if (j) {
-      linear_wave_n_kernel<E, MT, NT, WK, D, EPI, true><<<grid, dim3(256 * WK), 0, st>>>(a, *j);
+      linear_wave_n_kernel<MT, NT, WK, D, EPI, true><<<grid, dim3(256 * WK), 0, st>>>(a, *j);
       return hip_check_launch();
     }
   }
-  linear_wave_n_kernel<E, MT, NT, WK, D, EPI, false><<<grid, dim3(256 * WK), 0, st>>>(a, NoJoin{});
+  linear_wave_n_kernel<MT, NT, WK, D, EPI, false><<<grid, dim3(256 * WK), 0, st>>>(a, NoJoin{});
   return hip_check_launch();
 }
 
@@ -420,7 +414,7 @@ static int wave_n_launch(const slm_linear_args& a, hipStream_t st, const StreamJ
 // With more rows the columns of a wave weigh against the rounds they need, ties to the wider (x is read half as often):
 // 64 rows x 28672 x 4096 41 us against 48, 64 rows x 16384 x 2048 20.6 against 15.7.  Up to 32 rows and under 112 panels the chip is
 // filled by 32-column tiles (6784 columns: 15.6 us against 18.4).
-template <typename E, int EPI>
+template <int EPI>
 static int stream_shape(const slm_linear_args& a, hipStream_t st, const StreamJoin* j = nullptr) {
   constexpr bool GLU = EPI == SLM_LIN_GLU;
   const int64_t s = a.n_splits;
@@ -429,21 +423,21 @@ static int stream_shape(const slm_linear_args& a, hipStream_t st, const StreamJo
     return 4 * w >= 3 * 256 * ((w + 255) / 256);
   };
   if (a.M <= 16) {
-    if (full(4)) return wave_k_launch<E, 1, 4, 3, EPI>(a, st, j);
+    if (full(4)) return wave_k_launch<1, 4, 3, EPI>(a, st, j);
     if constexpr (!GLU) {
-      if (!full(2)) return wave_k_launch<E, 1, 1, 8, EPI>(a, st, j);
+      if (!full(2)) return wave_k_launch<1, 1, 8, EPI>(a, st, j);
     }
-    return wave_k_launch<E, 1, 2, 4, EPI>(a, st, j);
+    return wave_k_launch<1, 2, 4, EPI>(a, st, j);
   }
   const int64_t rounds1 = (stream_tiles(a, 4) * s + 255) / 256, rounds2 = (stream_tiles(a, 8) * s + 255) / 256;
   const bool wide = 2 * rounds2 <= rounds1;
   if (a.M <= 32) {
-    if (stream_tiles(a, 4) * s < 112) return wave_k_launch<E, 2, 2, 4, EPI>(a, st, j);
-    return wide ? wave_n_launch<E, 2, 2, 1, 4, EPI>(a, st, j) : wave_n_launch<E, 2, 1, 2, 4, EPI>(a, st, j);
+    if (stream_tiles(a, 4) * s < 112) return wave_k_launch<2, 2, 4, EPI>(a, st, j);
+    return wide ? wave_n_launch<2, 2, 1, 4, EPI>(a, st, j) : wave_n_launch<2, 1, 2, 4, EPI>(a, st, j);
   }
-  if (a.M <= 64) return wide ? wave_n_launch<E, 4, 2, 1, 4, EPI>(a, st, j) : wave_n_launch<E, 4, 1, 1, 4, EPI>(a, st, j);
-  if (a.M <= 96) return wide ? wave_n_launch<E, 6, 2, 1, 4, EPI>(a, st, j) : wave_n_launch<E, 6, 1, 1, 4, EPI>(a, st, j);
-  return wide ? wave_n_launch<E, 8, 2, 2, 2, EPI>(a, st, j) : wave_n_launch<E, 8, 1, 1, 4, EPI>(a, st, j);
+  if (a.M <= 64) return wide ? wave_n_launch<4, 2, 1, 4, EPI>(a, st, j) : wave_n_launch<4, 1, 1, 4, EPI>(a, st, j);
+  if (a.M <= 96) return wide ? wave_n_launch<6, 2, 1, 4, EPI>(a, st, j) : wave_n_launch<6, 1, 1, 4, EPI>(a, st, j);
+  return wide ? wave_n_launch<8, 2, 2, 2, EPI>(a, st, j) : wave_n_launch<8, 1, 1, 4, EPI>(a, st, j);
 }
 
 // A thread moves 16 bytes; a wave writes 1 KB and reads 16 half lines whose other halves the next wave reads (once per
@@ -471,35 +465,27 @@ extern "C" SLM_API int slm_stream_layout(void* out, const void* w, int64_t N, in
   return hip_check_launch();
 }
 
-static int stream_check(const slm_linear_args* a, int dtype, bool join = false) {
+static int stream_check(const slm_linear_args* a, bool join = false) {
   if (!a || !a->x || !a->w || !a->y || a->M < 0 || a->N <= 0 || a->K <= 0 || a->K % 64 || a->N % 16 || a->batch != 1 ||
       a->n_splits < 1 || a->ldx < a->K || a->epilogue < 0 || a->epilogue > SLM_LIN_GLU)
     return SLM_ERR_INVALID_ARG;
   const bool glu = a->epilogue == SLM_LIN_GLU;
   if ((glu && a->N % 64) || (a->n_splits > 1 && a->epilogue != SLM_LIN_SLABS && !join)) return SLM_ERR_INVALID_ARG;
   if (a->ldy < (glu ? a->N / 2 : a->N)) return SLM_ERR_INVALID_ARG;
-  if (a->dtype != dtype || a->K > (1 << 28) || a->N > (1 << 30) || a->M > (1 << 20) || a->n_splits > 65535) return SLM_ERR_UNSUPPORTED;
+  if (a->dtype != SLM_BF16 || a->K > (1 << 28) || a->N > (1 << 30) || a->M > (1 << 20) || a->n_splits > 65535) return SLM_ERR_UNSUPPORTED;
   return a->ldx % 8 || !aligned16(a->x) || !aligned16(a->w) ? SLM_ERR_ALIGNMENT : SLM_OK;
 }
 extern "C" SLM_API int slm_linear_stream(const slm_linear_args* a, void* stream) {
-  const int rc = stream_check(a, SLM_BF16);
+  const int rc = stream_check(a);
   if (rc != SLM_OK || a->M == 0) return rc;
   hip_clear_error();
   hipStream_t st = (hipStream_t)stream;
   switch (a->epilogue) {
-    case SLM_LIN_STORE: return stream_shape<bf16, SLM_LIN_STORE>(*a, st);
-    case SLM_LIN_F32: return stream_shape<bf16, SLM_LIN_F32>(*a, st);
-    case SLM_LIN_SLABS: return stream_shape<bf16, SLM_LIN_SLABS>(*a, st);
-    default: return stream_shape<bf16, SLM_LIN_GLU>(*a, st);
+    case SLM_LIN_STORE: return stream_shape<SLM_LIN_STORE>(*a, st);
+    case SLM_LIN_F32: return stream_shape<SLM_LIN_F32>(*a, st);
+    case SLM_LIN_SLABS: return stream_shape<SLM_LIN_SLABS>(*a, st);
+    default: return stream_shape<SLM_LIN_GLU>(*a, st);
   }
-}
-extern "C" SLM_API int slm_linear_stream_half(const slm_linear_args* a, void* stream) {
-  const int rc = stream_check(a, SLM_F16);
-  if (rc != SLM_OK) return rc;
-  if (a->epilogue != SLM_LIN_STORE) return SLM_ERR_UNSUPPORTED;
-  if (a->M == 0) return SLM_OK;
-  hip_clear_error();
-  return stream_shape<_Float16, SLM_LIN_STORE>(*a, (hipStream_t)stream);
 }
 
 // Joined products: STORE, 17 to 128 rows, at most SLM_STREAM_TICKETS tiles of 32 columns
@@ -507,17 +493,17 @@ static bool stream_join_ok(const slm_linear_args* a) {
   return a->epilogue == SLM_LIN_STORE && a->M > 16 && a->M <= 128 && a->n_splits <= 16 && stream_tiles(*a, 2) <= SLM_STREAM_TICKETS;
 }
 extern "C" SLM_API size_t slm_linear_stream_join_bytes(const slm_linear_args* a) {
-  if (stream_check(a, SLM_BF16, true) != SLM_OK || !stream_join_ok(a)) return 0;
+  if (stream_check(a, true) != SLM_OK || !stream_join_ok(a)) return 0;
   const int64_t rows = a->M <= 32 ? 32 : a->M <= 64 ? 64 : a->M <= 96 ? 96 : 128;
   return (size_t)(a->n_splits * rows * stream_tiles(*a, 8) * 128 * 4);   // (whole tiles of up to 128 columns)
 }
 extern "C" SLM_API int slm_linear_stream_join(const slm_linear_args* a, void* workspace, size_t workspace_bytes, uint32_t* tickets, void* stream) {
-  const int rc = stream_check(a, SLM_BF16, true);
+  const int rc = stream_check(a, true);
   if (rc != SLM_OK) return rc;
   if (!stream_join_ok(a)) return SLM_ERR_UNSUPPORTED;
   if (!tickets || !workspace || workspace_bytes < slm_linear_stream_join_bytes(a)) return SLM_ERR_WORKSPACE;
   if (!aligned16(workspace)) return SLM_ERR_ALIGNMENT;
   const StreamJoin j{(float*)workspace, tickets};
   hip_clear_error();
-  return stream_shape<bf16, SLM_LIN_STORE>(*a, (hipStream_t)stream, &j);
+  return stream_shape<SLM_LIN_STORE>(*a, (hipStream_t)stream, &j);
 }

@@ -2,8 +2,6 @@
 // into the layer classes of this directory or straight into the C ABI (include/slm_hip.h).
 #include "slm_llama_hip.h"
 
-#include "slm_latent.h"
-
 #include <ATen/hip/HIPEvent.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
@@ -96,7 +94,7 @@ void LlamaForCausalLMHip::load_state_dict(const StateDict& sd) {
   t = sd.get_tensor("model.norm.weight");
   if (t.defined()) { final_norm_ = t.to(options_).contiguous(); norm_loaded_ = true; }
   t = sd.get_sharded_tensor("lm_head.weight", 0, rank, world);  // [vocab, hidden] in the checkpoint
-  if (t.defined()) { lm_head_ = t.to(options_).t().contiguous(); lm_head_loaded_ = true; head_layout_ = torch::Tensor(); }
+  if (t.defined()) { lm_head_ = t.to(options_).t().contiguous(); lm_head_loaded_ = true; }
   for (size_t i = 0; i < layers_.size(); ++i) {
     const auto lsd = sd.select("model.layers." + std::to_string(i) + ".");
     if (lsd.size() == 0) continue;
@@ -194,26 +192,6 @@ void LlamaForCausalLMHip::reserve(int64_t n_tokens) {
   }
   if (lanes == 2 && !side_stream_.has_value())
     side_stream_ = c10::hip::getStreamFromPoolMasqueradingAsCUDA(false, options_.device().index());
-  if (!capturing()) lay_out_head();
-}
-
-// decode.LlamaDecodeStep._lay_out_head
-void LlamaForCausalLMHip::lay_out_head() {
-  const auto& w = lm_head_;
-  constexpr int64_t LEAST = int64_t{1} << 22, PART = 4096;   // elements; columns turned at a time
-  if (head_layout_.defined() || !lm_head_loaded_ || !w.is_cuda() || w.numel() < LEAST || w.size(0) % 64 || w.size(1) % 16 ||
-      (w.scalar_type() != torch::kBFloat16 && w.scalar_type() != torch::kHalf))
-    return;
-  const int64_t K = w.size(0), N = w.size(1), panels = (N + 63) / 64;
-  size_t free = 0, total = 0;
-  if (hipMemGetInfo(&free, &total) != hipSuccess || static_cast<size_t>(panels * 64 * K * 2) > free / 2) return;
-  auto out = torch::empty({panels, 64 * K}, w.options());
-  for (int64_t n0 = 0; n0 < N; n0 += PART) {
-    const auto part = w.slice(1, n0, std::min(n0 + PART, N)).t().contiguous();
-    const int rc = slm_stream_layout(out[n0 / 64].data_ptr(), part.data_ptr(), part.size(0), K, 0, c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream());
-    TORCH_CHECK(rc == SLM_OK, "slm_stream_layout: ", slm_latent_status_string(rc));
-  }
-  head_layout_ = out;
 }
 
 // ---- lanes -------------------------------------------------------------------------------------
@@ -559,22 +537,7 @@ torch::Tensor LlamaForCausalLMHip::forward(const torch::Tensor& tokens, const to
 torch::Tensor LlamaForCausalLMHip::logits(const torch::Tensor& hidden_states, const torch::Tensor& selected_idxes) {
   auto h = hidden_states;
   if (selected_idxes.defined()) h = h.index_select(0, selected_idxes);
-  torch::Tensor out;
-  if (head_layout_.defined() && h.dim() == 2 && h.size(0) > 0 && h.size(0) <= 128 && h.stride(1) == 1 && h.stride(0) >= h.size(1) && h.stride(0) % 8 == 0 &&
-      h.scalar_type() == lm_head_.scalar_type() && reinterpret_cast<uintptr_t>(h.data_ptr()) % 16 == 0) {   // (latent_kernels.linear_columns)
-    out = torch::empty({h.size(0), lm_head_.size(1)}, h.options());
-    slm_linear_args a{};
-    a.x = h.data_ptr(); a.w = head_layout_.data_ptr(); a.y = out.data_ptr();
-    a.M = h.size(0); a.N = lm_head_.size(1); a.K = h.size(1); a.ldx = h.stride(0); a.ldw = a.K; a.ldy = a.N;
-    a.alpha = 1.f; a.batch = 1; a.n_splits = 1; a.epilogue = SLM_LIN_STORE;
-    const bool half = h.scalar_type() == torch::kHalf;
-    a.dtype = half ? SLM_F16 : SLM_BF16;
-    void* const stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream();
-    const int rc = half ? slm_linear_stream_half(&a, stream) : slm_linear_stream(&a, stream);
-    TORCH_CHECK(rc == SLM_OK, "slm_linear_stream: ", slm_latent_status_string(rc));
-  } else {
-    out = torch::matmul(h, lm_head_);
-  }
+  auto out = torch::matmul(h, lm_head_);  // plain library GEMM (hipBLASLt)
   if (parallel_args_.world_size() > 1) {  // gather_output = true
     std::vector<torch::Tensor> parts;
     for (int r = 0; r < parallel_args_.world_size(); ++r) parts.push_back(torch::empty_like(out));

@@ -79,7 +79,7 @@ class LlamaForCausalLMHip {
   void load_state_dict(const StateDict& state_dict);
   void verify_loaded_weights() const;
 
-  // scratch of every lane + the lanes' side stream, lm_head laid out for few rows: once, before graph capture
+  // scratch of every lane + the lanes' side stream: once, before graph capture
   void reserve(int64_t n_tokens);
 
   // LlamaForCausalLMImpl::forward: final-norm hidden states [n_tokens, hidden] (static buffer view)
@@ -129,7 +129,6 @@ class LlamaForCausalLMHip {
   // (grown to `bytes`; where it may not or cannot grow and a call does without, required = 0: what there is)
   const torch::Tensor& scratch(int lane, size_t bytes, size_t required = 1);
   const torch::Tensor& deferred(int lane, int slot, size_t bytes, size_t required = 1);
-  void lay_out_head();
   const torch::Tensor& grown(torch::Tensor& t, size_t bytes, size_t required, const char* what);
 
   LlamaArgs args_;
@@ -144,7 +143,6 @@ class LlamaForCausalLMHip {
   std::unique_ptr<AttentionImpl> atten_;
   std::vector<Layer> layers_;
   torch::Tensor embed_, final_norm_, lm_head_;  // embed [vocab, hidden / tp], lm_head [hidden, vocab / tp]
-  torch::Tensor head_layout_;                   // lm_head in the order of slm_linear_stream, or undefined
   bool embed_loaded_ = false, norm_loaded_ = false, lm_head_loaded_ = false;
   // static activation buffers [max_tokens, ...]
   torch::Tensor resid_, normed_, qkv_, attn_, act_, gate_up_, o_, down_;

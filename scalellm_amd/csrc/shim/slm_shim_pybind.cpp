@@ -235,6 +235,7 @@ PYBIND11_MODULE(_slm_shim, m) {
       .def("forward",
            [](PyLlama& self, const torch::Tensor& tokens, const torch::Tensor& positions,
               const slm::InputParameters& params) { return self.model->forward(tokens, positions, self.kv, params); })
+      .def("logits", [](PyLlama& self, const torch::Tensor& hidden_states) { return self.model->logits(hidden_states, torch::Tensor()); })
       .def("last_lanes", [](PyLlama& self) { return self.model->last_lanes(); });
   py::class_<slm::W4Linear>(m, "W4Linear")
       .def(py::init<const std::string&, const torch::Tensor&, const torch::Tensor&,

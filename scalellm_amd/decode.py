@@ -267,7 +267,6 @@ class LlamaDecodeStep:
         lm_head = (torch.randn(H, shape.vocab, device=self.device, generator=gen) * 0.02).to(dtype)
         self.lm_head = lm_head[:, r * shape.vocab // tp:(r + 1) * shape.vocab // tp].contiguous()
         del embed, lm_head
-        self._head_layout: Optional[torch.Tensor] = None   # of lm_head, for steps of few rows (_lay_out_head)
         self.kv_head0 = kv_head0
         T = max_batch_tokens
         e = lambda *s: torch.empty(*s, dtype=dtype, device=self.device)  # noqa: E731
@@ -305,7 +304,7 @@ class LlamaDecodeStep:
                         seg.copy_(blk[:seg.numel()])
 
     def reserve_workspaces(self, n_tokens: int, max_kv_len: int) -> None:
-        """Grow the kernel workspace once, before graph capture, and lay weights out once more for the steps of up to n_tokens rows."""
+        """Grow the kernel workspace once, before graph capture, and make the linears' 16-bit copies for steps of many rows (_lay_out_dense)."""
         s = self.shape
 
         def need_for(rows: int) -> int:
@@ -330,7 +329,6 @@ class LlamaDecodeStep:
         if 0 < h0 < n_tokens and self._side_stream is None:
             self._side_stream = torch.cuda.Stream(device=self.device)
         if not torch.cuda.is_current_stream_capturing():
-            self._lay_out_head()
             self._lay_out_dense(n_tokens)
 
     def _lay_out_dense(self, n_tokens: int) -> None:
@@ -342,29 +340,6 @@ class LlamaDecodeStep:
         spare = lk.spare_memory(self.lm_head.device)
         for linear in linears:
             spare -= linear.lay_out_dense(spare)
-
-    # elements of a vocabulary product from which its weight is laid out once more for few rows: below, both ways are a launch of 2 to 6 us
-    HEAD_LAYOUT_MIN = 1 << 22
-
-    def _lay_out_head(self) -> None:
-        """lm_head in the order the streamed product reads it, where half of the memory that is left holds it: up to 128 rows of logits are then one linear
-        read (us, 16 bits, vendor product / streamed: 32768 x 4096 1 row 52 / 42, 32 rows 51 / 43, 128 rows 57 / 52; 128256 x 4096 190 / 157, 204 / 168,
-        244 / 231; 8192 x 1024 9.1 / 4.7, 12.0 / 6.3, 13.9 / 9.9)."""
-        w = self.lm_head
-        if self._head_layout is not None and lk.layout_is_current(self._head_layout, w):
-            return
-        self._head_layout = None
-        if not w.is_cuda or w.numel() < self.HEAD_LAYOUT_MIN or (w.size(1) + 63) // 64 * 64 * w.size(0) * w.element_size() > lk.spare_memory(w.device):
-            return
-        slm_build.ensure("latent")
-        try:
-            self._head_layout = lk.stream_layout_columns(w)
-        except torch.OutOfMemoryError:
-            pass
-
-    def weights_version(self):
-        """Changes when lm_head is changed in place or replaced while products read a copy of it (None: they read the weight itself)."""
-        return None if self._head_layout is None else (self.lm_head.data_ptr(), self._head_layout.copy_of._version)
 
     # ------------------------------------------------------------------------------------------
     # One decoder stack over a range of token rows ("lane").  A step normally has ONE lane (all rows,
@@ -771,7 +746,7 @@ class LlamaDecodeStep:
             self.last_hidden = last = kernels.last_rows(normed, q_cu)
         else:
             self.last_hidden = last = normed[(q_cu[1:] - 1).long()]
-        logits = lk.linear_columns(last, self.lm_head, self._head_layout)
+        logits = last @ self.lm_head  # plain library GEMM (hipBLASLt)
         if ar is not None and not return_logits and last.size(0) <= ar.max_tokens \
                 and 4 * pa.world_size <= s.hidden:
             return self._greedy_over_vocab_shards(logits, ar)

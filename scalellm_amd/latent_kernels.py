@@ -385,40 +385,6 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None,
     return out
 
 
-def stream_layout_columns(w: torch.Tensor) -> Optional[torch.Tensor]:
-    """stream_layout() of W^T for a contiguous W [K, N] (a column a result), in bf16 or half precision; None where the kernel has no form or W can't
-    be followed (inference tensors)."""
-    K, N = w.shape
-    if (w.dtype not in (torch.bfloat16, torch.float16) or K % 64 or N % 16 or not K or not N or not w.is_cuda or not w.is_contiguous() or
-            w.is_inference()):
-        return None
-    out = torch.empty((N + 63) // 64, K // 64, 4, 2, 64, 8, dtype=w.dtype, device=w.device)
-    with torch.cuda.device(w.device):
-        for n0 in range(0, N, 4096):   # (turned a part at a time: no second copy beside the layout)
-            part = w[:, n0:n0 + 4096].t().contiguous()
-            latent_check(_lib.latent_lib().slm_stream_layout(_p(out[n0 // 64]), _p(part), part.size(0), K, 0, _stream()), "slm_stream_layout")
-    out.copy_of, out.copy_version = w, w._version
-    return out
-
-
-def linear_columns(x: torch.Tensor, w: torch.Tensor, layout: Optional[torch.Tensor]) -> torch.Tensor:
-    """x [M, K] W [K, N] -> [M, N] of the same type: up to 128 rows from layout = stream_layout_columns(w), the vendor's otherwise."""
-    M, (K, N) = x.size(0), w.shape
-    if (layout is None or not 0 < M <= STREAM_LAYOUT_MAX_ROWS or x.dtype != w.dtype or x.dim() != 2 or x.size(1) != K or x.stride(1) != 1 or
-            x.stride(0) < K or x.stride(0) % 8 or x.data_ptr() % 16 or not layout_is_current(layout, w)):
-        return x @ w
-    out = torch.empty(M, N, dtype=x.dtype, device=x.device)
-    a = _lib.LinearArgs()
-    a.x, a.w, a.y, a.M, a.N, a.K, a.ldx, a.ldw, a.ldy = _p(x), _p(layout), _p(out), M, N, K, x.stride(0), K, N
-    a.alpha, a.batch, a.n_splits, a.epilogue, a.dtype = 1.0, 1, 1, _lib.LIN_STORE, SLM_BF16 if x.dtype == torch.bfloat16 else _lib.SLM_F16
-    L = _lib.latent_lib()
-    if x.dtype == torch.bfloat16:
-        latent_check(L.slm_linear_stream(C.byref(a), _stream()), "slm_linear_stream")
-    else:
-        latent_check(L.slm_linear_stream_half(C.byref(a), _stream()), "slm_linear_stream_half")
-    return out
-
-
 def linear_f32(x: torch.Tensor, w: torch.Tensor, alpha: float = 1.0, layout: Optional[torch.Tensor] = None) -> torch.Tensor:
     """alpha * x W^T as fp32 (logits).  layout: stream_layout(w)."""
     M, N, K = _check_xw(x, w)

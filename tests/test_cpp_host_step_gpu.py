@@ -210,3 +210,15 @@ def test_cpp_step_replicates_kv_heads_like_the_python_mirror_at_tp4(shim, rank):
         for L, (k0, v0) in zip(mine.layers, snap):
             L["kv"].key_cache.copy_(k0)
             L["kv"].value_cache.copy_(v0)
+
+
+def test_cpp_logits_refuse_other_hidden_states(shim):
+    """Rows of another width, of another type and on the host are refused, as torch's product refuses them."""
+    step, shape = _step("awq", 8, 64, 16)
+    model = cpp_model_from(shim, step, 16, 8)
+    h = torch.randn(3, shape.hidden, device=DEV).to(torch.bfloat16)
+    assert torch.equal(model.logits(h), h @ step.lm_head)
+    wide = torch.cat([h, h], 1)
+    for bad in (h[:, :192].contiguous(), h[:, :192], wide, h.cpu(), h.half()):
+        with pytest.raises(RuntimeError):
+            model.logits(bad)

@@ -296,33 +296,76 @@ def test_last_hidden_of_a_step_outlives_the_next_one():
     assert torch.equal(hidden, rows) and not torch.equal(model.last_hidden, rows)
 
 
-def test_logits_of_a_head_that_is_laid_out_once_more():
-    """Up to 128 rows from the copy, as long as lm_head is what it was: changed in place or replaced, products are its own; both hosts give the same bits.  One
-    rounding to 8 significant bits."""
-    from scalellm_amd import cpp_host
+def _wide_head(rows):
     from scalellm_amd.decode import LlamaDecodeStep, LlamaShape, make_decode_inputs
     shape = LlamaShape(hidden=512, n_heads=8, n_kv_heads=2, head_dim=64, intermediate=512, n_layers=1, vocab=8208, max_position=128)
-    tokens, positions, params, n_blocks = make_decode_inputs(130, 20, 16, torch.device(DEV), seed=3, vocab=shape.vocab)
-    model = LlamaDecodeStep(shape, 130, n_blocks, 16, dtype=torch.bfloat16, device=torch.device(DEV), kv_fill="randn", keep_checkpoint=True)
-    assert model.weights_version() is None
-    model.reserve_workspaces(130, 20)
-    assert model._head_layout is not None
+    _, _, _, n_blocks = make_decode_inputs(rows, 20, 16, torch.device(DEV), seed=3, vocab=shape.vocab)
+    model = LlamaDecodeStep(shape, rows, n_blocks, 16, dtype=torch.bfloat16, device=torch.device(DEV), kv_fill="randn", keep_checkpoint=True)
+    return model, lambda n: make_decode_inputs(n, 20, 16, torch.device(DEV), seed=3, vocab=shape.vocab)[:3]
+
+
+def _writes(model):
+    """lm_head changed in place in the ways that programs have: as a tensor, and where no version counter tells (a weight update's broadcast is such)."""
+    model.lm_head[:, 5] = 0.0
+    yield
+    model.lm_head.data.mul_(-2.0)
+    yield
+    with torch.inference_mode():
+        model.lm_head.add_(1.0)
+    yield
+
+
+def test_logits_follow_lm_head():
+    """Changed in place or replaced, before and after workspaces are reserved: the logits are those of the weight as it is; both hosts give the same bits.
+    One rounding to 8 significant bits."""
+    from scalellm_amd import cpp_host
+    model, batch = _wide_head(130)
     for n in (130, 3):
-        t, p, prm, _ = make_decode_inputs(n, 20, 16, torch.device(DEV), seed=3, vocab=shape.vocab)
+        t, p, prm = batch(n)
+        model.reserve_workspaces(130, 20)
         got = model.forward(t, p, prm, return_logits=True)
         want = model.last_hidden.double() @ model.lm_head.double()
         assert (got.double() - want).abs().max() <= 2.0 ** -8 * 1.02 * want.abs().max()
         cpp = cpp_host.from_decode_step(model, 16, 130)
         assert torch.equal(cpp.decode_step(t, p, cpp_host.cpp_params(prm), True), got)
-    version = model.weights_version()
-    model.lm_head[:, 5] = 0.0
-    assert model.weights_version() != version
-    assert not model.forward(t, p, prm, return_logits=True)[:, 5].any()
-    version, model.lm_head = model.weights_version(), model.lm_head + 1.0
-    assert model.weights_version() != version
-    got = model.forward(t, p, prm, return_logits=True)
-    assert torch.equal(got, model.last_hidden @ model.lm_head)
-    model.reserve_workspaces(130, 20)
-    again = model.forward(t, p, prm, return_logits=True)
-    want = model.last_hidden.double() @ model.lm_head.double()
-    assert model._head_layout.copy_of is model.lm_head and (again.double() - want).abs().max() <= 2.0 ** -8 * 1.02 * want.abs().max()
+    for _ in _writes(model):
+        for _ in range(2):
+            got = model.forward(t, p, prm, return_logits=True)
+            assert torch.equal(got, model.last_hidden @ model.lm_head)
+            model.reserve_workspaces(130, 20)
+    model.lm_head = model.lm_head + 1.0
+    assert torch.equal(model.forward(t, p, prm, return_logits=True), model.last_hidden @ model.lm_head)
+
+
+def test_captured_logits_follow_lm_head():
+    """A graph that the caller captured reads the weight, not a copy of what it was."""
+    model, batch = _wide_head(3)
+    t, p, prm = batch(3)
+    model.reserve_workspaces(3, 20)
+    model.forward(t, p, prm, return_logits=True)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        logits = model.forward(t, p, prm, return_logits=True)
+    for _ in _writes(model):
+        graph.replay()
+        assert torch.equal(logits, model.forward(t, p, prm, return_logits=True))
+        model.reserve_workspaces(3, 20)
+        graph.replay()
+        assert torch.equal(logits, model.last_hidden @ model.lm_head)
+
+
+def test_runner_replays_graphs_across_reservations_and_weight_updates():
+    """Graphs captured before workspaces are reserved, and before lm_head is changed in place, are replayed after it."""
+    from scalellm_amd.model_runner import ModelRunner, ModelRunnerOptions
+    model, batch = _wide_head(3)
+    t, p, prm = batch(3)
+    runner = ModelRunner(model, DEV, ModelRunnerOptions(block_size=16, cuda_graph_max_seq_len=64, cuda_graph_batch_sizes=[3]), return_logits=True)
+    runner.capture_cuda_graphs(3)
+    model.reserve_workspaces(3, 20)
+    runner.forward(t, p, prm)
+    assert (runner.num_graph_replayed, runner.num_eager) == (1, 0)
+    for i, _ in enumerate(_writes(model)):
+        got = runner.forward(t, p, prm).clone()
+        assert (runner.num_graph_replayed, runner.num_eager) == (2 + i, 0)
+        assert torch.equal(got, model.forward(t, p, prm, return_logits=True))

@@ -163,8 +163,6 @@ def _streamed_products(M, N, K):
         _close(out, ref.clamped_glu(want[:, :N // 2], want[:, N // 2:], 0.6), torch.bfloat16, b16=2e-2)
 
 
-# Weights whose columns are the results: the streamed form's edges in both 16-bit types (rows at the edges of its tiles, columns that fill no panel, parts that
-# are turned at a time, steps below and past the rings), rows with a stride.  fp32 sums of exact products, one rounding.
 @pytest.mark.parametrize("M", [17, 32, 33, 64, 65, 96, 97, 128])
 @pytest.mark.parametrize("N,K,n", [(16, 64, 3), (80, 704, 2), (3664, 1984, 3), (6752, 2112, 2), (9216, 1088, 3), (1040, 4160, 16), (16384, 192, 1)])
 def test_products_cut_in_k_and_joined(M, N, K, n):
@@ -211,23 +209,6 @@ def test_joined_products_in_a_graph():
         a = lk.linear(x, w, layout=layout, tickets=tickets)
         b = lk.linear(a[:, :K], w, layout=layout, tickets=tickets)
         assert torch.equal(first, a) and torch.equal(again, b)
-
-
-@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("M", [1, 16, 17, 33, 65, 97, 128, 129])
-@pytest.mark.parametrize("K,N", [(64, 16), (192, 4112), (2112, 8240)])
-def test_products_of_columns(M, K, N, dtype):
-    lk = _lk()
-    x = _rnd(1, M, K + 8, dtype=dtype)[:, :K]
-    w = _rnd(2, K, N, dtype=dtype, std=K ** -0.5)
-    layout = lk.stream_layout_columns(w)
-    assert torch.equal(layout, lk.stream_layout(w.t().contiguous().view(torch.bfloat16)).view(dtype))
-    got, want = lk.linear_columns(x, w, layout), x.double() @ w.double()
-    roundoff = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11   # (of 8 and 11 significant bits)
-    assert got.dtype == dtype and (got.double() - want).abs().max() <= roundoff * 1.02 * want.abs().max()
-    assert torch.equal(lk.linear_columns(x, w, None), x @ w)
-    w.mul_(-2.0)   # (the copy is not of it any more)
-    assert torch.equal(lk.linear_columns(x, w, layout), x @ w)
 
 
 # Products of many rows, in every tile: rows and columns that fill no tile, one step of 64 k and fewer than there are stages, more tiles than
