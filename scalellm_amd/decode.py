@@ -305,6 +305,11 @@ class LlamaDecodeStep:
 
     def reserve_workspaces(self, n_tokens: int, max_kv_len: int) -> None:
         """Grow the kernel workspace once, before graph capture, and make the linears' 16-bit copies for steps of many rows (_lay_out_dense)."""
+        self._reserve_scratch(n_tokens)
+        if not torch.cuda.is_current_stream_capturing():
+            self._lay_out_dense(n_tokens)
+
+    def _reserve_scratch(self, n_tokens: int) -> None:
         s = self.shape
 
         def need_for(rows: int) -> int:
@@ -328,8 +333,6 @@ class LlamaDecodeStep:
                 kernels.reserve_workspace(need_for(rows), self.device, deferred_nbytes=16 * rows * widest * 4)
         if 0 < h0 < n_tokens and self._side_stream is None:
             self._side_stream = torch.cuda.Stream(device=self.device)
-        if not torch.cuda.is_current_stream_capturing():
-            self._lay_out_dense(n_tokens)
 
     def _lay_out_dense(self, n_tokens: int) -> None:
         """16-bit copies of the linears' weights for steps of many rows, where such come and half of the memory that is left holds them."""
@@ -432,7 +435,7 @@ class LlamaDecodeStep:
         times = {}
         try:
             self.layers = all_layers[:k]
-            self.reserve_workspaces(n_tokens, kv_len)
+            self._reserve_scratch(n_tokens)   # (no copies of weights: those are of all layers, reserve_workspaces)
             o_buf, down_buf = self.buf["o"][:n_tokens], self.buf["down"][:n_tokens]
             self.buf["resid"][:n_tokens].normal_()
             import gc

@@ -217,3 +217,23 @@ def test_two_lanes_on_a_tensor_parallel_rank_equal_the_half_batches():
         assert model.last_lanes == 1
         assert torch.equal(got[r0:r1], half), (r0, r1, float((got[r0:r1].float() - half.float()).abs().max()))
         restore()
+
+
+def _many_rows(**more):
+    from scalellm_amd.decode import LlamaDecodeStep, LlamaShape
+    shape = LlamaShape(hidden=256, n_heads=8, n_kv_heads=2, head_dim=32, intermediate=640, n_layers=3, vocab=512, max_position=64)
+    model = LlamaDecodeStep(shape, 384, 800, 16, dtype=torch.bfloat16, device=DEV, **more)
+    return model, [L[name] for L in model.layers for name in ("qkv", "o", "gate_up", "down")]
+
+
+def test_probe_leaves_the_weights_as_they_are():
+    """It times some layers of a model as it stands: none gets a 16-bit copy for it that the others have not."""
+    from scalellm_amd import _lib
+    model, linears = _many_rows()
+    try:
+        assert model.probe_lanes(384, 20, n_layers=1, reps=1) is not None
+        assert all(x._dense is None for x in linears)
+        model.reserve_workspaces(384, 20)
+        assert all(x._dense is not None for x in linears)
+    finally:
+        _lib.lib().slm_decode_lane_policy_clear()   # (nothing of it for other tests)
