@@ -335,14 +335,20 @@ class LlamaDecodeStep:
             self._side_stream = torch.cuda.Stream(device=self.device)
 
     def _lay_out_dense(self, n_tokens: int) -> None:
-        """16-bit copies of the linears' weights for steps of many rows, where such come and half of the memory that is left holds them."""
+        """16-bit copies of the linears' weights for steps of many rows, where such come and half of the memory that is left holds those of all layers: a model
+        does not run on two kinds of kernels by depth."""
         linears = [L[name] for L in self.layers for name in ("qkv", "o", "gate_up", "down")]
-        if not linears or n_tokens < linears[0].dense_rows() or not self.lm_head.is_cuda:
+        if not linears or n_tokens < linears[0].dense_rows() or not self.lm_head.is_cuda or not all(x.is_loaded() for x in linears):
+            return
+        wanted = [x for x in linears if x.dense_bytes()]
+        if sum(x.dense_bytes() for x in wanted) > lk.spare_memory(self.lm_head.device):
             return
         slm_build.ensure("latent")
-        spare = lk.spare_memory(self.lm_head.device)
-        for linear in linears:
-            spare -= linear.lay_out_dense(spare)
+        for i, linear in enumerate(wanted):
+            if not linear.lay_out_dense(linear.dense_bytes()):   # (no memory all the same: those made just now, which no graph has read, go again)
+                for made in wanted[:i]:
+                    made.drop_dense()
+                return
 
     # ------------------------------------------------------------------------------------------
     # One decoder stack over a range of token rows ("lane").  A step normally has ONE lane (all rows,

@@ -291,22 +291,35 @@ class _QLinearBase:
         1069; half 210 rows 828 / 853, 290 1068 / 971."""
         return 288 if self.dtype == torch.float16 else 384
 
-    def lay_out_dense(self, spare: int) -> int:
-        """The weight in 16 bits, [N, K] row-major ([gate | up] of a merged one), the values products of many rows make of int4 for every tile: once, where
-        `spare` bytes hold it.  Returns the bytes it took.  Weights whose sums keep their order (PackedW4.any_order), act-order and 8-bit ones have none."""
+    def is_loaded(self) -> bool:
+        return self._packed is not None or all(name in self._ckpt for name in ("qweight", "qzeros", "scales") + ("bias",) * self.has_bias)
+
+    def dense_bytes(self) -> int:
+        """What lay_out_dense() would take.  0: it is made, or the weight has none, as those whose sums keep their order (PackedW4.any_order), act-order and
+        8-bit ones."""
         if self._dense is not None:
             return 0
         if self._packed is None:
             self._repack()
         p = self._packed
         groups = p.group_size in (32, 64, p.K) or (p.group_size >= 128 and p.group_size & (p.group_size - 1) == 0)   # (what the int4 products take)
-        if not groups or not p.any_order or p.perm is not None or p.k_src != p.K or p.K % 128 or p.N % 32 or 2 * p.N * p.K > spare:
+        return 0 if not groups or not p.any_order or p.perm is not None or p.k_src != p.K or p.K % 128 or p.N % 32 else 2 * p.N * p.K
+
+    def lay_out_dense(self, spare: int) -> int:
+        """The weight in 16 bits, [N, K] row-major ([gate | up] of a merged one), the values products of many rows make of int4 for every tile: once, where
+        `spare` bytes hold it.  Returns the bytes it took."""
+        need = self.dense_bytes()
+        if need > spare:
             return 0
         try:
-            self._dense = kernels.w4_dequant_rows(p)
+            if need:
+                self._dense = kernels.w4_dequant_rows(self._packed)
         except torch.OutOfMemoryError:
             return 0
-        return 2 * p.N * p.K
+        return need
+
+    def drop_dense(self) -> None:
+        self._dense = None
 
     def _gemm(self, x: torch.Tensor, bias: Optional[torch.Tensor],
               out: Optional[torch.Tensor], defer_splitk: bool = False,

@@ -237,3 +237,37 @@ def test_probe_leaves_the_weights_as_they_are():
         assert all(x._dense is not None for x in linears)
     finally:
         _lib.lib().slm_decode_lane_policy_clear()   # (nothing of it for other tests)
+
+
+def test_copies_of_all_linears_or_of_none(monkeypatch):
+    from scalellm_amd import latent_kernels as lk
+    model, linears = _many_rows()
+    need = sum(2 * x.in_features * x.out_features for x in linears)
+    assert need == 2 * 3 * 256 * (384 + 256 + 1280 + 640)
+    for spare, made in ((need - 1, False), (need, True)):
+        monkeypatch.setattr(lk, "spare_memory", lambda device: spare)
+        model.reserve_workspaces(384, 20)
+        assert [x._dense is not None for x in linears] == [made] * 12
+
+
+def test_copies_that_run_out_of_memory(monkeypatch):
+    """No memory at the last one: none is left; a later reservation makes them all.  A linear that is not loaded yet: none."""
+    from scalellm_amd import kernels
+    model, linears = _many_rows()
+    made, rows = [], kernels.w4_dequant_rows
+
+    def fail_at_last(packed):
+        if len(made) == 11:
+            raise torch.OutOfMemoryError("a full card")
+        made.append(rows(packed))
+        return made[-1]
+    monkeypatch.setattr(kernels, "w4_dequant_rows", fail_at_last)
+    model.reserve_workspaces(384, 20)
+    assert len(made) == 11 and all(x._dense is None for x in linears)
+    monkeypatch.undo()
+    packed, linears[5]._packed = linears[5]._packed, None
+    model.reserve_workspaces(384, 20)
+    assert all(x._dense is None for x in linears)
+    linears[5]._packed = packed
+    model.reserve_workspaces(384, 20)
+    assert all(x._dense is not None for x in linears)
