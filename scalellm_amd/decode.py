@@ -166,8 +166,11 @@ class LlamaDecodeStep:
                  parallel_args: Optional[ParallelArgs] = None, quant_method: str = "awq",
                  group_size: int = 128, dtype=torch.bfloat16, device="cuda", seed: int = 0,
                  kv_fill: str = "none", custom_allreduce=None, keep_checkpoint: bool = False,
-                 gptq_sym: bool = False, fuse_silu: bool = True, desc_act: bool = False, bits: int = 4):
+                 gptq_sym: bool = False, fuse_silu: bool = True, desc_act: bool = False, bits: int = 4, dense_copies: bool = True):
         pa = parallel_args or ParallelArgs()
+        # dense_copies: reserve_workspaces() may keep the AWQ linears' weights in 16 bits too (four times the packed weights: 14 GB for 32 layers of
+        # the 8b size), out of half of the memory that is left by then; False: none, for what the program allocates later
+        self.dense_copies = dense_copies
         # fuse_silu: the merged gate_up weight is packed paired and SiLU*mul runs in the GEMM
         # epilogue (identical bits; False keeps the separate kernels.silu_and_mul launch)
         fuse_silu = fuse_silu and (shape.intermediate // pa.world_size) % 32 == 0
@@ -304,7 +307,8 @@ class LlamaDecodeStep:
                         seg.copy_(blk[:seg.numel()])
 
     def reserve_workspaces(self, n_tokens: int, max_kv_len: int) -> None:
-        """Grow the kernel workspace once, before graph capture, and make the linears' 16-bit copies for steps of many rows (_lay_out_dense)."""
+        """Grow the kernel workspace once, before graph capture.  For steps of 384 rows and more (288 in half precision) it also keeps AWQ weights in 16 bits,
+        2 bytes a weight beside the half byte of the packed ones, where half of the free memory holds all of them; dense_copies = False: it doesn't."""
         self._reserve_scratch(n_tokens)
         if not torch.cuda.is_current_stream_capturing():
             self._lay_out_dense(n_tokens)
@@ -338,7 +342,7 @@ class LlamaDecodeStep:
         """16-bit copies of the linears' weights for steps of many rows, where such come and half of the memory that is left holds those of all layers: a model
         does not run on two kinds of kernels by depth."""
         linears = [L[name] for L in self.layers for name in ("qkv", "o", "gate_up", "down")]
-        if not linears or n_tokens < linears[0].dense_rows() or not self.lm_head.is_cuda or not all(x.is_loaded() for x in linears):
+        if not self.dense_copies or not linears or n_tokens < linears[0].dense_rows() or not self.lm_head.is_cuda or not all(x.is_loaded() for x in linears):
             return
         wanted = [x for x in linears if x.dense_bytes()]
         if sum(x.dense_bytes() for x in wanted) > lk.spare_memory(self.lm_head.device):

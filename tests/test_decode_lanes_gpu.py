@@ -271,3 +271,9 @@ def test_copies_that_run_out_of_memory(monkeypatch):
     linears[5]._packed = packed
     model.reserve_workspaces(384, 20)
     assert all(x._dense is not None for x in linears)
+
+
+def test_copies_are_the_programs_choice():
+    model, linears = _many_rows(dense_copies=False)
+    model.reserve_workspaces(384, 20)
+    assert all(x._dense is None for x in linears)
