@@ -79,14 +79,15 @@ SLM_API int slm_linear_stream_join(const slm_linear_args* a, void* workspace, si
 SLM_API int slm_stream_layout(void* out, const void* w, int64_t N, int64_t K, int32_t glu, void* stream);
 /* The same for many rows in bf16, batch 1, STORE or GLU, rows of x, w and y on 16 bytes, x and w below 2 GB: tiles of  */
 /* up to 256 x 256.  tile: -1 or an index of the tiles (tests); slices: 0 as many as pay, n: the tiles of the   */
-/* last round are cut in K by n.  Without the workspace (optional, content does not matter) nothing is cut.     */
+/* last round are cut in K by n.  Without the workspace (optional, content does not matter) nothing is cut.  Its size is */
+/* asked for with the arguments of any of the three calls below.                                                */
 SLM_API size_t slm_gemm_workspace_bytes(const slm_linear_args* a, int32_t tile, int32_t slices);
 SLM_API int slm_gemm(const slm_linear_args* a, void* workspace, size_t workspace_bytes, int32_t tile, int32_t slices, void* stream);
 /* The same, or in half precision (by dtype), with counters of the caller's, counters [SLM_GEMM_COUNTERS], zero before, of this */
 /* product alone: a launch less where it is cut                                                                  */
 #define SLM_GEMM_COUNTERS 256
 SLM_API int slm_gemm_counted(const slm_linear_args* a, void* workspace, size_t workspace_bytes, uint32_t* counters, int32_t tile, int32_t slices, void* stream);
-/* The same in half precision (dtype SLM_F16); its workspace is that of the call in bf16                        */
+/* The same in half precision (dtype SLM_F16)                                                                   */
 SLM_API int slm_gemm_half(const slm_linear_args* a, void* workspace, size_t workspace_bytes, int32_t tile, int32_t slices, void* stream);
 /* y = g sigmoid(alpha g) (u + shift), g = min(gate, limit), u = clamp(up, +-limit) (limit may be        */
 /* infinite: with alpha 1 and shift 0 the plain SiLU GLU); gu = [rows, 2 * half]                         */

@@ -378,7 +378,7 @@ static int gemm_check(const slm_linear_args* a, int tile, int slices, int dtype)
 using namespace slm;
 
 extern "C" SLM_API size_t slm_gemm_workspace_bytes(const slm_linear_args* a, int32_t tile, int32_t slices) {
-  return gemm_check(a, tile, slices, SLM_BF16) == SLM_OK && a->M ? gemm_plan(*a, tile, slices).bytes : 0;
+  return gemm_check(a, tile, slices, a && a->dtype == SLM_F16 ? SLM_F16 : SLM_BF16) == SLM_OK && a->M ? gemm_plan(*a, tile, slices).bytes : 0;
 }
 
 template <typename T>

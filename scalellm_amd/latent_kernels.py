@@ -338,7 +338,8 @@ def _gemm(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, glu=None, tile: i
         return False
     limit, alpha, shift = glu or (0.0, 0.0, 0.0)
     # (in the order of the fields: a third of what setting them one by one takes)
-    a = _lib.LinearArgs(_p(x), _p(w), _p(out), None, M, N, K, ldx, ldw, ldy, 0, 0, 0, 0, 1.0, limit, alpha, shift, 1, 1, _lib.LIN_GLU if glu else _lib.LIN_STORE, SLM_BF16)
+    a = _lib.LinearArgs(_p(x), _p(w), _p(out), None, M, N, K, ldx, ldw, ldy, 0, 0, 0, 0, 1.0, limit, alpha, shift, 1, 1, _lib.LIN_GLU if glu else _lib.LIN_STORE,
+                         _lib.SLM_F16 if half else SLM_BF16)
     L = _lib.latent_lib()
     need, ws = L.slm_gemm_workspace_bytes(C.byref(a), tile, slices), None
     if need:
@@ -346,8 +347,6 @@ def _gemm(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, glu=None, tile: i
             ws = torch.empty(need, dtype=torch.uint8, device=x.device)
         except torch.OutOfMemoryError:
             need = 0
-    if half:
-        a.dtype = _lib.SLM_F16
     counters = tickets.take() if need and tickets is not None else None
     if counters is not None:
         _check_counters(counters, _lib.GEMM_COUNTERS, x.device)

@@ -319,3 +319,21 @@ def test_slices_of_joined_products():
             assert L.slm_linear_stream_join(C.byref(a), 1 << 20, size, None, None) < 0
         if n > 1:
             assert K // 64 // n >= 10
+
+
+@pytest.mark.parametrize("M,N,K,tile,slices", [(2300, 4128, 320, 2, 2), (207, 4096, 2048, -1, 0), (300, 544, 704, 2, 3), (300, 544, 704, 2, 1)])
+def test_tiled_products_scratch_in_half_precision(M, N, K, tile, slices):
+    """Asked with the arguments of the call itself, the size is that of the same product in bf16; 32 bits are refused by both."""
+    import ctypes as C
+    from scalellm_amd import _lib
+    L = _lib.latent_lib()
+    a = _gemm_args(M, N, K)
+    want = L.slm_gemm_workspace_bytes(C.byref(a), tile, slices)
+    assert (want > 0) == (slices != 1)
+    a.dtype = _lib.SLM_F16
+    assert L.slm_gemm_workspace_bytes(C.byref(a), tile, slices) == want
+    assert L.slm_gemm(C.byref(a), None, 0, tile, slices, None) == -2
+    a.dtype = _lib.SLM_F32
+    assert L.slm_gemm_workspace_bytes(C.byref(a), tile, slices) == 0
+    assert L.slm_gemm_half(C.byref(a), None, 0, tile, slices, None) == -2
+    assert L.slm_gemm_counted(C.byref(a), 1 << 20, 1 << 40, 1 << 20, tile, slices, None) == -2
