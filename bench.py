@@ -615,7 +615,8 @@ def main():
     model = LlamaDecodeStep(shape, bs, n_blocks, B, pa, quant_method=quant, group_size=128,
                             dtype=torch.bfloat16, device=device, seed=0, kv_fill=args.kv_fill,
                             custom_allreduce=custom_ar, gptq_sym=gptq_sym, bits=args.bits,
-                            keep_checkpoint=args.host == "cpp")
+                            keep_checkpoint=args.host == "cpp",
+                            dense_copies=args.host != "cpp")  # (the C++ host has none: beside it, the same launches)
     if args.lanes >= 0:
         model.lanes_min = args.lanes
     model.reserve_workspaces(bs, L)

@@ -1,7 +1,8 @@
 """Python handle on the C++ HOST STEP (csrc/shim/slm_llama_hip.{h,cpp}: slm::LlamaForCausalLMHip, the
 decoder stack of src/models/meta/llama.h:123-345 composed in C++ from the layer classes of
 csrc/shim/) -- what `bench.py --host cpp` times and tests/test_cpp_host_step_gpu.py holds bit-identical to
-the Python mirror (decode.LlamaDecodeStep; its steps of many rows apart, once they run on 16-bit copies of the weights).  Nothing here computes: it loads
+the Python mirror (decode.LlamaDecodeStep).  The C++ host keeps no 16-bit copies of weights: to a mirror that has them
+(dense_copies, once reserved for 384 rows or, in half precision, 288) steps of so many rows are equal up to rounding.  Nothing here computes: it loads
 _slm_shim.so, hands it the checkpoint-format tensors under their HuggingFace names, the KV cache
 tensors and the step's integer inputs."""
 from __future__ import annotations

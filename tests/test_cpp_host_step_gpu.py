@@ -38,11 +38,11 @@ def cpp_model_from(shim, step, block_size, max_tokens, fused=True, lanes=64, qua
     return cpp_host.from_decode_step(step, block_size, max_tokens, fused=fused, lanes=lanes)
 
 
-def _step(quant, max_tokens, n_blocks, B, seed=2):
+def _step(quant, max_tokens, n_blocks, B, seed=2, **more):
     from scalellm_amd.decode import LlamaDecodeStep, LlamaShape
     shape = LlamaShape.tiny()
     step = LlamaDecodeStep(shape, max_tokens, n_blocks, B, quant_method=quant, group_size=128, dtype=torch.bfloat16,
-                           device=DEV, seed=seed, keep_checkpoint=True)
+                           device=DEV, seed=seed, keep_checkpoint=True, **more)
     # two lanes for every pure-decode batch of >= 64 tokens, on both hosts (the automatic rule wants 12 MiB of
     # K + V per sequence -- not what a tiny test model has; the rule itself: tests/test_host_logic_cpu.py)
     step.lanes_min = 64
@@ -111,6 +111,26 @@ def test_cpp_step_is_bit_identical_to_the_python_mirror(shim, quant):
         ids = fused.decode_step(tokens, positions, cpp_params(shim, params))
         assert torch.equal(ids, torch.argmax(want.float(), dim=-1).to(torch.int32)), name
         restore()
+
+
+@pytest.mark.parametrize("dense_copies", [False, True])
+def test_cpp_step_of_many_rows(shim, dense_copies):
+    """From 384 rows on the mirror multiplies by its 16-bit copies where it has them, in another order: rounding only.  Without, and below, the same bits."""
+    from scalellm_amd.decode import make_batch_inputs
+    step, shape = _step("awq", 420, 200, 16, dense_copies=dense_copies)
+    step.reserve_workspaces(420, 256)
+    linears = [L[name] for L in step.layers for name in ("qkv", "o", "gate_up", "down")]
+    assert all((x._dense is not None) == dense_copies for x in linears)
+    model = cpp_model_from(shim, step, 16, 420)
+    for lens in ([200, 183], [200, 184], [210, 17, 193]):
+        tokens, positions, params, _ = make_batch_inputs(lens, lens, 16, DEV, seed=5, vocab=shape.vocab)
+        want = step.forward(tokens, positions, params, return_logits=True).clone()
+        got = model.decode_step(tokens, positions, cpp_params(shim, params), return_logits=True)
+        if dense_copies and sum(lens) >= 384:
+            # (two layers of eight products, each rounded to 2^-9 of its value on either side)
+            assert float((got.double() - want.double()).norm() / want.double().norm()) <= 2e-2
+        else:
+            assert torch.equal(got, want), lens
 
 
 def test_cpp_step_replays_from_one_hip_graph(shim):
