@@ -370,13 +370,14 @@ void LlamaForCausalLMHip::attn(Lane& ln, size_t li, std::vector<KVCache>& kv, in
   a.total_kv_len = p.kv_total_len > 0 && p.kv_total_len < (int64_t(1) << 31) ? static_cast<int32_t>(p.kv_total_len) : 0;
   a.phase = phase;  // (1 / 2: the two lanes hand the KV-stream token on between the stream kernel and the combine pass)
   if (a.n_tokens == 0 || a.batch_size == 0) return;
-  const size_t need = slm_paged_kv_varlen_mha_workspace_bytes(&a);
-  const bool at_hand = scratch_[ln.idx].defined() && static_cast<size_t>(scratch_[ln.idx].nbytes()) >= need;
-  // (being captured: scratch that is not there only where the call cannot do without, and scratch() says so then)
-  if (need > 0 && (at_hand || !capturing() || slm_paged_kv_varlen_mha_workspace_required(&a) > 0)) {
-    const auto& ws = scratch(ln.idx, need);
-    a.workspace = ws.mutable_data_ptr();
-    a.workspace_bytes = ws.nbytes();
+  const size_t need = slm_paged_kv_varlen_mha_workspace_bytes(&a), least = slm_paged_kv_varlen_mha_workspace_required(&a);
+  if (need > 0) {
+    if (phase != 2) scratch(ln.idx, need, 0);    // as much as can be had (the combine pass takes what the pass before it wrote to)
+    if (least > 0) scratch(ln.idx, least);       // (says so where the call cannot do without)
+    if (const auto& ws = scratch_[ln.idx]; ws.defined()) {
+      a.workspace = ws.mutable_data_ptr();
+      a.workspace_bytes = ws.nbytes();
+    }
   }
   ok(slm_paged_kv_varlen_mha(&a, cur(ln.q)), "slm_paged_kv_varlen_mha");
 }

@@ -131,7 +131,9 @@ void paged_kv_varlen_mha(torch::Tensor& out, const torch::Tensor& query,
   const size_t need = slm_paged_kv_varlen_mha_workspace_bytes(&a);
   torch::Tensor ws;
   if (need > 0) {
-    ws = workspace_for(query, need, slm_paged_kv_varlen_mha_workspace_required(&a));
+    const size_t least = slm_paged_kv_varlen_mha_workspace_required(&a);
+    ws = workspace_for(query, need, least < need ? 0 : least);
+    if (!ws.defined() && least > 0) ws = workspace_for(query, least, least);   // (no more to be had: what the call cannot do without)
     a.workspace = ws.defined() ? ws.mutable_data_ptr() : nullptr;
     a.workspace_bytes = ws.defined() ? ws.nbytes() : 0;
   }

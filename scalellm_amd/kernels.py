@@ -300,11 +300,14 @@ def paged_kv_varlen_mha(
     if a.n_tokens == 0 or a.batch_size == 0:
         return
     need = L.slm_paged_kv_varlen_mha_workspace_bytes(C.byref(a))
-    if need and not _fits_or_grows(need, query.device):   # (being captured: only what the call cannot do without)
-        need = L.slm_paged_kv_varlen_mha_workspace_required(C.byref(a))
     if need:
-        ws = reserve_workspace(need, query.device)
-        a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
+        # (the combine pass reads what the pass before it wrote: its scratch as it is)
+        ws = _wanted_workspace(need, query.device) if a.phase != 2 else _workspaces.get(_dev_key(query.device))
+        if ws is None or a.phase == 2:   # no more to be had: what the call cannot do without
+            least = L.slm_paged_kv_varlen_mha_workspace_required(C.byref(a))
+            ws = reserve_workspace(least, query.device) if least else ws
+        if ws is not None:
+            a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
     check(L.slm_paged_kv_varlen_mha(C.byref(a), _stream()), "slm_paged_kv_varlen_mha")
 
 

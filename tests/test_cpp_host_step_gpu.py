@@ -242,3 +242,38 @@ def test_cpp_logits_refuse_other_hidden_states(shim):
     for bad in (h[:, :192].contiguous(), h[:, :192], wide, h.cpu(), h.half()):
         with pytest.raises(RuntimeError):
             model.logits(bad)
+
+
+def test_captured_step_with_scratch_for_the_fewest_pieces(shim, monkeypatch):
+    """Scratch as a step before the capture left it: what the attention cannot do without, but not for its many pieces."""
+    import types
+    from scalellm_amd import cpp_host, kernels
+
+    class Unreserved:
+        def __init__(self, model):
+            self.model = model
+
+        def reserve(self, n_tokens):
+            pass
+
+        def __getattr__(self, name):
+            return getattr(self.model, name)
+    step, shape = _step("awq", 40, 1600, 16)
+    made = types.SimpleNamespace(LlamaForCausalLMHip=lambda **kw: Unreserved(shim.LlamaForCausalLMHip(**kw)))
+    with monkeypatch.context() as m:
+        m.setattr(cpp_host, "load_shim", lambda: made)
+        model = cpp_host.from_decode_step(step, 16, 40)
+    rng = np.random.default_rng(3)
+    tokens, positions, params = _batch(rng, 40, 1, [int(x) for x in rng.integers(1, 480, size=40)], 16, 1600, shape.vocab)
+    prm = cpp_params(shim, params)
+    with kernels.tuning(SLM_ATTN_BAL=0):
+        want = model.decode_step(tokens, positions, prm, True).clone()
+        torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with kernels.tuning(SLM_ATTN_BAL=2):
+        with torch.cuda.graph(graph):
+            got = model.decode_step(tokens, positions, prm, True)
+    for _ in range(2):
+        graph.replay()
+        # two orders of the attention's sums; two layers of eight products, each rounded to 2^-9 of its value
+        assert float((got.double() - want.double()).norm() / want.double().norm()) <= 2e-2

@@ -451,3 +451,39 @@ def test_cpp_handler_profiling_run_with_empty_cache_only_rotates(shim):
     shim.handler_pos_emb_and_append(hc, H, HKV, D, qc, kc, v, pos, empty, prm)
     torch.cuda.synchronize()
     assert torch.equal(qc.view(5, H, D), q2) and torch.equal(kc.view(5, HKV, D), k2)
+
+
+def test_captured_attention_with_scratch_for_the_fewest_pieces(shim):
+    """The caller's scratch holds what the call cannot do without, and no more: captured, it does with that."""
+    import ctypes as C
+    from scalellm_amd import _lib, kernels
+    n, H, D, B, bound = 128, 8, 128, 16, 4096
+    lens = np.random.default_rng(3).integers(1, 200, n)
+    blocks = (lens + B - 1) // B
+    i32 = lambda v: torch.tensor(np.asarray(v), dtype=torch.int32, device=DEV)  # noqa: E731
+    cu = lambda v: i32(np.concatenate([[0], np.cumsum(v)]))                      # noqa: E731
+    g = torch.Generator().manual_seed(n)
+    q = torch.randn(n, 4 * H, D, generator=g).half().to(DEV)
+    kc, vc = ((torch.rand(int(blocks.sum()) * B, H, D, generator=g) * 2 - 1).half().to(DEV) for _ in range(2))
+    idx = (i32(np.arange(n + 1)), cu(lens), i32(np.arange(int(blocks.sum())) * B), cu(blocks))
+    out, want = torch.empty_like(q), torch.empty_like(q)
+    args = (None, B, 1, bound, D ** -0.5)
+    with kernels.tuning(SLM_ATTN_BAL=0):
+        kernels.paged_kv_varlen_mha(want, q, kc, vc, *idx, *args)
+    a = kernels._attn_args(out, q, kc, vc, *idx, *args, 0.0, -1, 0)
+    most, least = (f(C.byref(a)) for f in (_lib.lib().slm_paged_kv_varlen_mha_workspace_bytes, _lib.lib().slm_paged_kv_varlen_mha_workspace_required))
+    assert 0 < least < most
+    handler = shim.HipAttnHandler(D ** -0.5, 0.0, None)
+    handler.set_workspace(torch.empty(least, dtype=torch.uint8, device=DEV))
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    try:
+        with torch.cuda.graph(graph):
+            shim.paged_kv_varlen_mha(out, q, kc, vc, *idx, *args, 0.0, -1)
+    finally:
+        handler.set_workspace(torch.empty(most, dtype=torch.uint8, device=DEV))   # (of the process)
+    for _ in range(2):
+        out.zero_()
+        graph.replay()
+        # two orders of the same sums, rounded to half on either side
+        assert (out.float() - want.float()).abs().max().item() <= 4 * 2 ** -11
