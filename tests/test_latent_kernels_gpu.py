@@ -277,6 +277,7 @@ def test_tiled_products_with_counters_of_the_callers(M, N, K, slices, glu, dtype
         got.zero_()
         assert lk._gemm(x, w, got, tickets=tickets, **how) and torch.equal(want, got)
     assert int(words[:512].abs().max()) == 0 and bool((words.view(-1, 256)[2:] == words[512:768]).all())
+    assert int(words[512:768].max()) > 0   # (it was cut, and counted there)
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
         words.zero_()

@@ -881,7 +881,8 @@ def test_rows_of_dequantised_weights(K, N, gs, fmt, dtype):
 @pytest.mark.parametrize("paired", [False, True])
 def test_layers_of_many_rows_take_the_copy(paired, dtype):
     """From dense_rows() on, within roundings of the exact product; below, without a copy, with a bias and where sums keep their order the int4 kernels."""
-    from scalellm_amd import kernels, layers
+    import math
+    from scalellm_amd import kernels, latent_kernels as lk, layers
     from scalellm_amd.decode import _rand_int4_linear
     from scalellm_amd.model_parallel import ParallelArgs
     K, N = 640, 448
@@ -907,6 +908,10 @@ def test_layers_of_many_rows_take_the_copy(paired, dtype):
             want = torch.nn.functional.silu(want[:, :N // 2]) * want[:, N // 2:]
         # (one rounding of fp32 sums of K exact products, and of the GLU's few operations)
         assert (got.double() - want).abs().max() <= 1.02 * unit * want.abs().max()
+        tiles = torch.empty_like(got)
+        assert lk.gemm(x, lin._dense, tiles, (math.inf, 1.0, 0.0) if paired else None) and torch.equal(got, tiles)
+    lin._dense.zero_()   # (only the copy)
+    assert not lin.forward(x).any()
     with pytest.raises(kernels.SlmError):
         lin.forward(x, out=torch.empty(M, N + 8, device=DEV, dtype=dtype))
     lin.load_state_dict({})
@@ -914,3 +919,28 @@ def test_layers_of_many_rows_take_the_copy(paired, dtype):
     for other in (made("gptq"), made("awq", bias=True)):
         want = other.forward(x)
         assert (other.lay_out_dense(1 << 40) > 0) == other.has_bias and torch.equal(other.forward(x), want)
+
+
+@pytest.mark.parametrize("K,N,M", [(2048, 2048, 300), (4096, 1024, 500)])
+def test_copies_in_front_of_a_norm_round_as_deferred_sums_do(K, N, M):
+    """Half precision, rows whose int4 product leaves its sums to the residual norm: that rounds them to half before it adds, as a stored product is, so the
+    copy's result is no further from 64 bits."""
+    from scalellm_amd import kernels, layers
+    from scalellm_amd.decode import _rand_int4_linear
+    from scalellm_amd.model_parallel import ParallelArgs
+    ckpt = _rand_int4_linear(torch.Generator(device=DEV).manual_seed(5), K, N, 128, "awq", torch.float16, DEV)
+    g = torch.Generator(device=DEV).manual_seed(M)
+    x, before = (torch.randn(M, K, device=DEV, generator=g) / 8).half(), torch.randn(M, N, device=DEV, generator=g).half()
+    errors = []
+    for copy in (False, True):
+        lin = layers.RowParallelQLinear(K, N, False, layers.QuantArgs("awq", 4, 128), True, ParallelArgs(), torch.float16, DEV)
+        lin.load_state_dict(ckpt)
+        assert (lin.lay_out_dense(1 << 40 if copy else 0) > 0) == copy
+        out, resid = torch.empty(M, N, device=DEV, dtype=torch.float16), before.clone()
+        y = lin.forward(x, out=out, defer_splitk=True)
+        assert bool(lin.deferred) != copy
+        kernels.rms_norm(torch.empty_like(out), y, torch.ones(N, device=DEV, dtype=torch.float16), 1e-5, residual=resid, partials=lin.deferred)
+        want = before.double() + x.double() @ kernels.w4_dequant(lin._packed).double()
+        errors.append(((resid.double() - want).norm() / want.norm()).item())
+    # (two roundings to 2^-11 on either side; the order of the fp32 sums turns a few of them the other way)
+    assert errors[1] <= 1.005 * errors[0] and errors[0] < 2 ** -11
